@@ -1,7 +1,12 @@
 // W6 requantizer for the reference's two-plane format: a bf16 weight in its original basis -> ConvRot256 -> 6-bit codes
 // (nibble plane, then 2-bit plane), one fp8-e4m3 relative scale per 32 columns, one fp32 scale per row.  Replaces
-// gpu_w6_requant, csrc/vendor/w6a8_requant.cu: same steps and float expressions (cited by line), one workgroup per row.
-// A load-time / LoRA-bake kernel: 1.5 B read + 0.78 B written per weight, bound by its arithmetic, not by HBM.
+// gpu_w6_requant, csrc/vendor/w6a8_requant.cu: same float expressions (cited by line), bit for bit.
+//
+// A load-time / LoRA-bake kernel: 2 B read + 0.78 B written per weight, bound by its vector instructions.  A wave owns
+// chunks of 1024 values, 16 consecutive ones per lane, and keeps them in registers from the load to the packed stores: a
+// scale group is two neighbouring lanes, a row up to 16 waves that exchange one maximum.  (One thread per group over a row
+// in LDS, as the reference has it, leaves a third of the lanes idle and reads LDS at a stride of 32 words: 5376 x 5376
+// measured 170 us that way, XXX us like this; the copy rate of the part allows 16 us.)
 #include "common.hpp"
 #include "convrot.hpp"
 
@@ -37,110 +42,170 @@ __device__ __forceinline__ float e4m3_to_f(uint32_t v) {
     const float f = e == 0 ? (float)m * 0.001953125f : (e == 15 && m == 7) ? __builtin_nanf("") : u2f(((e + 120) << 23) | (m << 20));
     return (v & 0x80) ? -f : f;
 }
-__device__ __forceinline__ float level(int i, float s) {                          // :59-61
-    return fminf(127.0f, fmaxf(-127.0f, nearbyintf((float)(i - 31) * s)));
+// Level i of a group's grid, i counted from the middle (f = i - 31, a whole number in a float), :59-61.
+__device__ __forceinline__ float level(float f, float s) { return __builtin_amdgcn_fmed3f(__builtin_rintf(f * s), -127.0f, 127.0f); }
+// The other lane of an even/odd pair.
+__device__ __forceinline__ float pair_lane(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0xB1, 0xf, 0xf, false));
 }
-__device__ __forceinline__ int lower_bound(float t, float s, float inv_s) {       // :63-69
-    const float est = nearbyintf((ceilf(t) - 0.5f) * inv_s);
-    int i = (est > 2.0e9f ? 2000000000 : est < -2.0e9f ? -2000000000 : (int)est) + 31;
-    i = min(max(i, 0), 63);
-    while (i > 0 && level(i - 1, s) >= t) --i;
-    while (i < 63 && level(i, s) < t) ++i;
-    return i;
+
+// Four values of a group -> their code bytes (level index + 1), :63-80,126-148.
+// The first level at or above t: levels are whole numbers, so it is the first that reaches ceil(t), i.e. whose product
+// (i - 31) s reaches ceil(t) - 1/2 (or passes it, where that tie rounds down to an even number).  With z that quotient,
+// rint(z) is the position or the one before it, however the division's last bit falls: a whole z needs the tie looked at,
+// and any other z is farther from a whole number than the bit reaches.  One look at the level there settles it.  Outside
+// [-127, 127] every level is on one side of t and the position is an end of the grid (ENDS; a lane meets it only when
+// its group holds a value beyond the row's largest decoded one).
+// `x0` is the hash input of value 0 without its low four bits' share, kc[j] that share (see the caller).
+template <bool ENDS>
+__device__ __forceinline__ uint32_t codes4(const float* v, float inv_sc, float s, float inv_s, uint32_t x0, const uint32_t* kc) {
+    uint32_t out = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float t = v[j] * inv_sc;
+        const float f = __builtin_amdgcn_fmed3f(__builtin_rintf((__builtin_ceilf(t) - 0.5f) * inv_s), -31.f, 32.f);
+        // position minus one: f when the level there is still below t, else f - 1; the sign bit stands for the compare
+        const int below = (int)f2u(level(f, s) - t) >> 31;
+        float l = __builtin_amdgcn_fmed3f(f - u2f(~below & 0x3f800000u), -31.f, 30.f);   // the lower of the two levels, :75-80
+        if (ENDS) l = t > 127.f ? 30.f : t <= -127.f ? -31.f : l;
+        const float l0 = level(l, s), l1 = level(l + 1.f, s);
+        const uint32_t h = x0 + kc[j];                                            // x * 747796405 + 2891336453, :21-25
+        const uint32_t w = ((h >> ((h >> 28u) + 4u)) ^ h) * 277803737u;
+        const float u = (float)(((w >> 22u) ^ w) >> 8) * (1.0f / 16777216.0f);    // :27-31
+        const float d = __builtin_fmaf(u, l1 - l0, l0) - t;                       // negative where t is above the threshold
+        out = __builtin_amdgcn_cvt_pk_u8_f32(l + 32.25f - __builtin_copysignf(0.5f, d), j, out);
+    }
+    return out;
 }
-__global__ void __launch_bounds__(256) w6_requant_kernel(const uint16_t* w, uint8_t* packed, uint8_t* s_rel, float* s_channel, int K,
-                                                        uint64_t seed) {
-    extern __shared__ __attribute__((aligned(16))) float smem[];
-    __shared__ float red[4];
-    float* row = smem;                                  // [K]
-    float* gscale = smem + K;                           // [K / 32]
-    float* tiles = smem + K + K / kG;                   // four wave-private rotation tiles, 16-byte aligned (K % 256 == 0)
-    const int64_t n = blockIdx.x;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // ConvRot256 (:174-206) as the row quantizer does it: a wave per chunk of 1024 values, 16 consecutive values per
-    // lane, strides 1 and 4 inside the lane and one trip through the wave's LDS tile for strides 16 and 64; the
-    // rotated row is kept in the weight dtype (:209-217).
-    for (int c = wave; c * convrot::kChunk < K; c += 4) {
-        const int e0 = c * convrot::kChunk + lane * 16;
-        float v[16];
-        if (e0 < K) {                                   // K % 256 == 0: a lane's 16 values are all in or all out
+
+// wpr waves per row (chunks wr, wr + wpr, ...), rpb rows per workgroup.
+template <int C>
+__global__ void __launch_bounds__(1024) w6_requant_kernel(const uint16_t* w, uint8_t* packed, uint8_t* s_rel, float* s_channel, int N, int K,
+                                                         uint64_t seed, int wpr, int rpb) {
+    extern __shared__ __attribute__((aligned(16))) float tiles[];   // a rotation tile per wave
+    __shared__ float red[16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int rloc = wave / wpr, wr = wave - rloc * wpr;
+    const int64_t n = (int64_t)blockIdx.x * rpb + rloc;
+    const bool row_ok = n < N;
+    float v[C][16], gs[C], gmax[C];
+    float amax = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int e0 = (wr + c * wpr) * convrot::kChunk + lane * 16;
+        const bool act = row_ok && e0 < K;              // K % 256 == 0: a lane's 16 values are all in or all out
+        if (act) {
             const uint4* src = reinterpret_cast<const uint4*>(w + n * K + e0);
             const uint4 a = src[0], b = src[1];
             const uint32_t ww[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                v[2 * i] = u2f(ww[i] << 16);
-                v[2 * i + 1] = u2f(ww[i] & 0xffff0000u);
+                v[c][2 * i] = u2f(ww[i] << 16);
+                v[c][2 * i + 1] = u2f(ww[i] & 0xffff0000u);
             }
         } else {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) v[i] = 0.f;
+            for (int i = 0; i < 16; ++i) v[c][i] = 0.f;
         }
-        convrot::rotate_chunk<256>(v, tiles + wave * convrot::kLdsPerWave, lane);
-        if (e0 < K) {
+        // ConvRot256 (:174-206) as the row quantizer does it; the rotated row is kept in the weight dtype (:209-217)
+        convrot::rotate_chunk<256>(v[c], tiles + wave * convrot::kLdsPerWave, lane);
+        float m = 0.f;
 #pragma unroll
-            for (int i = 0; i < 16; i += 4)
-                *reinterpret_cast<float4*>(row + e0 + i) = make_float4(rnd_dt<DT_BF16>(v[i]), rnd_dt<DT_BF16>(v[i + 1]),
-                                                                       rnd_dt<DT_BF16>(v[i + 2]), rnd_dt<DT_BF16>(v[i + 3]));
+        for (int i = 0; i < 16; ++i) {
+            v[c][i] = rnd_dt<DT_BF16>(v[c][i]);
+            m = fmaxf(m, fabsf(v[c][i]));
         }
-    }
-    __syncthreads();
-
-    // phase 1: per-group step by two alternating-least-squares rounds; row maximum of the decoded weight, :94-120
-    const int groups = K / kG;
-    float amax_t = 0.f;
-    for (int g = tid; g < groups; g += 256) {
-        const float* x = row + g * kG;
-        float amax = 0.f;
-        for (int i = 0; i < kG; ++i) amax = fmaxf(amax, fabsf(x[i]));
-        float gs = fmaxf(amax / 31.0f, 1e-8f), inv = 1.0f / gs;
+        // the group's step by two alternating-least-squares rounds, :94-117.  num adds its 32 terms in index order: the odd
+        // lane of the pair goes on where the even one ends.  den sums whole numbers below 2^15: exact in any order.
+        m = fmaxf(m, pair_lane(m));
+        float step = fmaxf(m / 31.0f, 1e-8f), inv = 1.0f / step;
+        bool nan = false;
         for (int it = 0; it < 2; ++it) {
-            float num = 0.f, den = 0.f;
-            for (int i = 0; i < kG; ++i) {
-                const float q = fminf(31.0f, fmaxf(-31.0f, nearbyintf(x[i] * inv)));
-                num = __builtin_fmaf(x[i], q, num);
-                den = __builtin_fmaf(q, q, den);
+            float q[16], num = 0.f, den = 0.f;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                q[i] = __builtin_amdgcn_fmed3f(__builtin_rintf(v[c][i] * inv), -31.0f, 31.0f);
+                num = __builtin_fmaf(v[c][i], q[i], num);
+                den = __builtin_fmaf(q[i], q[i], den);
             }
-            gs = fmaxf(num / fmaxf(den, 1e-8f), 1e-8f);
-            inv = 1.0f / gs;
+            den += pair_lane(den);
+            const float head = pair_lane(num);
+            num = lane & 1 ? head : 0.f;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) num = __builtin_fmaf(v[c][i], q[i], num);
+            const float other = pair_lane(num);
+            num = lane & 1 ? num : other;
+            nan = num != num;
+            step = fmaxf(num / fmaxf(den, 1e-8f), 1e-8f);
+            inv = 1.0f / step;
         }
-        gscale[g] = gs;
-        for (int i = 0; i < kG; ++i) amax_t = fmaxf(amax_t, fabsf(fminf(31.0f, fmaxf(-31.0f, nearbyintf(x[i] * inv))) * gs));
+        // the group's largest decoded magnitude, :118-119: products and roundings are monotonic, so it is the largest
+        // value's (a NaN takes -31 in the reference's clamp)
+        amax = fmaxf(amax, (nan ? 31.0f : fminf(31.0f, __builtin_rintf(m * inv))) * step);
+        gs[c] = step;
+        gmax[c] = m;
     }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) amax_t = fmaxf(amax_t, __shfl_xor(amax_t, o, 64));
-    if ((tid & 63) == 0) red[tid >> 6] = amax_t;
-    __syncthreads();
-    const float sc = fmaxf(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])) / 127.0f, 1e-8f);   // :121
-    const float inv_sc = 1.0f / sc;
-    if (tid == 0) s_channel[n] = sc;
+    for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+    if (wpr > 1) {   // uniform over the workgroup
+        if (lane == 0) red[wave] = amax;
+        __syncthreads();
+        amax = 0.f;
+        for (int i = 0; i < wpr; ++i) amax = fmaxf(amax, red[rloc * wpr + i]);
+    }
+    const float sc = fmaxf(amax / 127.0f, 1e-8f), inv_sc = 1.0f / sc;               // :121
+    if (row_ok && wr == 0 && lane == 0) s_channel[n] = sc;
 
-    // phase 2: e4m3 relative scale, stochastic assignment between the two bracketing levels, code = level + 1, pack: :126-151
-    uint8_t* lo_plane = packed + n * (int64_t)(K * 3 / 4);
-    uint8_t* hi_plane = lo_plane + K / 2;
-    for (int g = tid; g < groups; g += 256) {
-        const uint32_t bits = f_to_e4m3(gscale[g] / sc);
-        s_rel[n * groups + g] = (uint8_t)bits;
-        const float sr = e4m3_to_f(bits), inv_sr = 1.0f / fmaxf(sr, 1e-30f);
-        const int base = g * kG;
-#pragma unroll 1
-        for (int p4 = 0; p4 < kG / 4; ++p4) {
-            uint32_t u[4];
+    // The hash multiplies index ^ seed; a lane's first index is a multiple of 16, so the product splits into one for the
+    // upper 28 bits and one for the four low bits, which is the same in all lanes.
+    const uint32_t s32 = (uint32_t)seed ^ (uint32_t)(seed >> 32);
+    uint32_t kc[16];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int e = base + 4 * p4 + j;
-                const float t = row[e] * inv_sc;
-                const int pos = lower_bound(t, sr, inv_sr);
-                const int l = min(max(pos - 1, 0), 61);                           // :75-80
-                const float l0 = level(l, sr);
-                const float thr = __builtin_fmaf(uniform01(n * K + e, seed), level(l + 1, sr) - l0, l0);
-                u[j] = (uint32_t)min(l + (t > thr ? 1 : 0), 62) + 1u;
-            }
-            lo_plane[g * (kG / 2) + 2 * p4] = (uint8_t)((u[0] & 0xF) | ((u[1] & 0xF) << 4));
-            lo_plane[g * (kG / 2) + 2 * p4 + 1] = (uint8_t)((u[2] & 0xF) | ((u[3] & 0xF) << 4));
-            hi_plane[g * (kG / 4) + p4] = (uint8_t)((u[0] >> 4) | ((u[1] >> 4) << 2) | ((u[2] >> 4) << 4) | ((u[3] >> 4) << 6));
+    for (int i = 0; i < 16; ++i) kc[i] = ((s32 ^ (uint32_t)i) & 15u) * 747796405u + 2891336453u;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int e0 = (wr + c * wpr) * convrot::kChunk + lane * 16;
+        if (!(row_ok && e0 < K)) continue;
+        const uint32_t bits = f_to_e4m3(gs[c] / sc);                                // :126-151
+        if (!(lane & 1)) s_rel[n * (K / kG) + e0 / kG] = (uint8_t)bits;
+        const float sr = e4m3_to_f(bits), inv_sr = 1.0f / fmaxf(sr, 1e-30f);
+        const uint32_t x0 = ((uint32_t)(n * K + e0) ^ (s32 & ~15u)) * 747796405u;
+        uint32_t cw[4];
+        if (__builtin_amdgcn_ballot_w64(gmax[c] * inv_sc >= 127.f) == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) cw[i] = codes4<false>(v[c] + 4 * i, inv_sc, sr, inv_sr, x0, kc + 4 * i);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) cw[i] = codes4<true>(v[c] + 4 * i, inv_sc, sr, inv_sr, x0, kc + 4 * i);
         }
+        // nibbles of codes 2j, 2j + 1 share a byte; the top bits of four codes share one (the product lines them up in
+        // its upper byte, and nothing below carries into it)
+        uint32_t lo[4], hi[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t nib = cw[i] & 0x0f0f0f0fu;
+            lo[i] = nib | (nib >> 4);                   // bytes 0 and 2
+            hi[i] = ((cw[i] >> 4) & 0x03030303u) * 0x01041040u;   // byte 3
+        }
+        uint8_t* lo_plane = packed + n * (int64_t)(K / 4 * 3);
+        *reinterpret_cast<uint2*>(lo_plane + e0 / 2) =
+            make_uint2(__builtin_amdgcn_perm(lo[1], lo[0], 0x06040200u), __builtin_amdgcn_perm(lo[3], lo[2], 0x06040200u));
+        *reinterpret_cast<uint32_t*>(lo_plane + K / 2 + e0 / 4) =
+            __builtin_amdgcn_perm(hi[1], hi[0], 0x0c0c0703u) | (__builtin_amdgcn_perm(hi[3], hi[2], 0x0c0c0703u) << 16);
     }
+}
+
+template <int C>
+int launch_requant(const void* w, void* packed, void* s_rel, void* s_channel, int N, int K, uint64_t seed, int wpr, hipStream_t st) {
+    const int rpb = wpr >= 4 ? 1 : 4 / wpr, nw = wpr * rpb;
+    const int smem = nw * convrot::kLdsPerWave * (int)sizeof(float);
+    static PerDeviceOnce once;
+    if (smem > 64 * 1024)
+        if (const int e = allow_dynamic_lds((const void*)w6_requant_kernel<C>, 16 * convrot::kLdsPerWave * (int)sizeof(float), once)) return e;
+    hipLaunchKernelGGL(w6_requant_kernel<C>, dim3((unsigned)((N + rpb - 1) / rpb)), dim3(nw * 64), smem, st, (const uint16_t*)w,
+                       (uint8_t*)packed, (uint8_t*)s_rel, (float*)s_channel, N, K, seed, wpr, rpb);
+    KCHECK();
+    return 0;
 }
 
 }  // namespace
@@ -150,14 +215,12 @@ __global__ void __launch_bounds__(256) w6_requant_kernel(const uint16_t* w, uint
 GPU_API int gpu_w6_requant(const void* weight, void* packed, void* s_rel, void* s_channel, int64_t N, int K, uint64_t seed,
                            void* stream) {
     if (K <= 0 || K % 256) return -1;
-    const size_t smem = (size_t)(K + K / kG + 4 * convrot::kLdsPerWave) * sizeof(float);
-    constexpr size_t kMaxDynamic = 160 * 1024 - 256;   // the kernel also has a few bytes of static LDS
-    if (smem > kMaxDynamic || N > 0x7fffffff) return -2;
+    if (K > 39680 || N > 0x7fffffff) return -2;
     if (N <= 0) return 0;
-    static PerDeviceOnce once;
-    if (const int e = allow_dynamic_lds((const void*)w6_requant_kernel, (int)kMaxDynamic, once)) return e;
-    hipLaunchKernelGGL(w6_requant_kernel, dim3((unsigned)N), dim3(256), smem, (hipStream_t)stream, (const uint16_t*)weight,
-                       (uint8_t*)packed, (uint8_t*)s_rel, (float*)s_channel, K, seed);
-    KCHECK();
-    return 0;
+    // a chunk per wave up to 16 waves per row; longer rows give a wave two or three
+    const int chunks = (K + convrot::kChunk - 1) / convrot::kChunk;
+    hipStream_t st = (hipStream_t)stream;
+    if (chunks <= 16) return launch_requant<1>(weight, packed, s_rel, s_channel, (int)N, K, seed, chunks, st);
+    if (chunks <= 32) return launch_requant<2>(weight, packed, s_rel, s_channel, (int)N, K, seed, (chunks + 1) / 2, st);
+    return launch_requant<3>(weight, packed, s_rel, s_channel, (int)N, K, seed, (chunks + 2) / 3, st);
 }

@@ -433,6 +433,30 @@ def test_w6_requant_bit_exact(N, K):
     assert ffi.raw("gpu_w6_requant", wd.data_ptr(), pd.data_ptr(), rd.data_ptr(), cd.data_ptr(), N, 300, 1, 0) == -1
 
 
+@pytest.mark.parametrize("N,K", [(6, 1024), (3, 1280), (2, 16384), (2, 16640), (1, 33024)])
+def test_w6_requant_row_lengths_and_grid_ends(N, K):
+    """One wave per row, ragged last chunks, sixteen waves, two and three chunks per wave; and rotated rows (the Hadamard
+    is its own inverse) whose largest value lies beyond the largest decoded one, so that codes come from the grid's ends."""
+    rot = synth.normal(90 + K, 1, N * K).reshape(N, K) * np.float32(0.02)
+    rot[:, :K // 2:32] = np.float32(3.1)            # groups of one large value among many at 15.49 steps: the step grows,
+    for i in range(1, 32):
+        rot[:, i:K // 2:32] = np.float32(1.549)     # and the largest code is 30 of 31
+    rot[:, 64:96] *= np.float32(-1)
+    H = np.array([[1, 1, 1, -1], [1, 1, -1, 1], [1, -1, 1, 1], [-1, 1, 1, 1]], np.float64) / 2
+    H256 = np.kron(np.kron(H, H), np.kron(H, H))
+    w = (rot.reshape(N, K // 256, 256).astype(np.float64) @ H256.T).reshape(N, K).astype(np.float32)
+    wb = synth.bf16_bits(w)
+    for seed in (0, 2 ** 33 + 7):
+        say("w6_requant", N, K, seed)
+        rc, packed, s_rel, s_ch = oracle.w6_requant(wb, seed)
+        pd, rd, cd = ql.w6_requant(dev_bits(wb, BF16), seed)
+        torch.cuda.synchronize()
+        assert rc == 0
+        assert np.array_equal(cd.cpu().numpy().view(np.uint32), s_ch.view(np.uint32))
+        assert np.array_equal(rd.cpu().numpy(), s_rel)
+        assert np.array_equal(pd.cpu().numpy(), packed)
+
+
 def test_checkpoint_linears_run_like_the_reference_sequence(tmp_path):
     """Weights as the reference's checkpoints store them (safetensors: int8 ConvRot with row scales, W6 triplet, dense),
     loaded and run through quantize -> GEMM; int8 and W6 outputs bit-exact against the oracle's sequence."""
