@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <type_traits>
 
 #include "../../include/gpu_api.h"
 
@@ -80,6 +81,53 @@ template <int DT> __device__ __forceinline__ void st_dt(void* p, int64_t i, floa
     else ((float*)p)[i] = v;
 }
 template <int DT> struct dt_size { static constexpr int value = DT == DT_F32 ? 4 : 2; };
+
+// Two floats -> packed f16 pair, and back.  The empty asm for the reason given at f_to_f16.
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack_f16x2(float a, float b) {
+    asm("" : "+v"(a), "+v"(b));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, f16x2));
+}
+__device__ __forceinline__ void unpack_f16x2(uint32_t u, float& a, float& b) {
+    const f16x2 h = __builtin_bit_cast(f16x2, u);
+    a = (float)h[0];
+    b = (float)h[1];
+}
+
+// Reductions over the 64 lanes of a wave, result in every lane: data-parallel-primitive moves inside rows of 16 lanes,
+// then the two row-swap instructions.  (A shuffle goes through the LDS and costs its latency six times.)
+template <int CTRL> __device__ __forceinline__ int dpp_int(int x) { return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, false); }
+__device__ __forceinline__ float wave_max_f32(float v) {
+    const auto mv = [](float x, auto ctrl) { return __builtin_bit_cast(float, dpp_int<decltype(ctrl)::value>(__builtin_bit_cast(int, x))); };
+    v = fmaxf(v, mv(v, std::integral_constant<int, 0xB1>{}));    // quad_perm [1,0,3,2]
+    v = fmaxf(v, mv(v, std::integral_constant<int, 0x4E>{}));    // quad_perm [2,3,0,1]
+    v = fmaxf(v, mv(v, std::integral_constant<int, 0x141>{}));   // row_half_mirror
+    v = fmaxf(v, mv(v, std::integral_constant<int, 0x140>{}));   // row_mirror
+    auto s = __builtin_amdgcn_permlane16_swap(f2u(v), f2u(v), false, false);
+    v = fmaxf(u2f(s[0]), u2f(s[1]));
+    s = __builtin_amdgcn_permlane32_swap(f2u(v), f2u(v), false, false);
+    return fmaxf(u2f(s[0]), u2f(s[1]));
+}
+__device__ __forceinline__ double wave_sum_f64(double v) {
+    const auto mv = [](double x, auto ctrl) {
+        const int64_t b = __builtin_bit_cast(int64_t, x);
+        constexpr int C = decltype(ctrl)::value;
+        return __builtin_bit_cast(double, ((int64_t)dpp_int<C>((int)(b >> 32)) << 32) | (uint32_t)dpp_int<C>((int)b));
+    };
+    v += mv(v, std::integral_constant<int, 0xB1>{});
+    v += mv(v, std::integral_constant<int, 0x4E>{});
+    v += mv(v, std::integral_constant<int, 0x141>{});
+    v += mv(v, std::integral_constant<int, 0x140>{});
+    const auto join = [](uint32_t hi, uint32_t lo) { return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo); };
+    uint64_t b = __builtin_bit_cast(uint64_t, v);
+    auto l = __builtin_amdgcn_permlane16_swap((uint32_t)b, (uint32_t)b, false, false);
+    auto h = __builtin_amdgcn_permlane16_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+    v = join(h[0], l[0]) + join(h[1], l[1]);
+    b = __builtin_bit_cast(uint64_t, v);
+    l = __builtin_amdgcn_permlane32_swap((uint32_t)b, (uint32_t)b, false, false);
+    h = __builtin_amdgcn_permlane32_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+    return join(h[0], l[0]) + join(h[1], l[1]);
+}
 
 // Workgroup -> tile.  Workgroups are dealt round-robin to the 8 XCDs (each with its own L2), so first renumber them
 // XCD-contiguously, then walk tiles in panels of 4 tile rows so that the 32 workgroups an XCD runs at once cover a

@@ -17,13 +17,9 @@ __device__ __forceinline__ int lds_pos(int e) {
     return (L << 4) + (((i + (L >> 1)) & 3) << 2) + j + ((e >> 8) << 4);
 }
 
-// h4_row x 4 outputs with the reference's left-to-right adds, scaled by 0.5 (csrc/common.cuh:99-106,119-122).
-// HALVE = false leaves the scaling out: the 128-wide transform, which is this library's own definition, applies its three
-// halvings together with the closing 1/sqrt(2), in one multiplication per output (bit-identical to halving per stage
-// while every intermediate stays in the normal range, and four instructions per butterfly shorter).
-template <bool HALVE = true> __device__ __forceinline__ void bfly4(float& a, float& b, float& c, float& d) {
+// h4_row x 4 outputs with the reference's left-to-right adds, times `h` (csrc/common.cuh:99-106,119-122: 0.5 per stage).
+__device__ __forceinline__ void bfly4(float& a, float& b, float& c, float& d, const float h = 1.0f) {
     const float x0 = a, x1 = b, x2 = c, x3 = d;
-    const float h = HALVE ? 0.5f : 1.0f;
     a = h * (x0 + x1 + x2 - x3);
     b = h * (x0 + x1 - x2 + x3);
     c = h * (x0 - x1 + x2 + x3);
@@ -35,13 +31,22 @@ template <bool HALVE = true> __device__ __forceinline__ void bfly4(float& a, flo
 // phases of rotate_chunk it is enough to stop the compiler from reordering them: no workgroup barrier is needed.
 #define LDS_WAVE_ORDER() asm volatile("" ::: "memory")
 
-template <int G> __device__ __forceinline__ void rotate_chunk(float* v, float* wl, int lane) {
+// ONCE: the halvings of all stages are one multiplication, in the last stage (three instead of four, or two instead of
+// three, multiplications per value saved).  A power of two moves through sums without touching a bit as long as nothing
+// overflows (the sums reach G times the largest input instead of the square root of G times) and no halved intermediate
+// would have been rounded as a subnormal; a sum is a whole multiple of its inputs' last bit, so that cannot happen when
+// every input's last bit is 2^-145 or more: any bf16 or f16 value, or int8 times a scale of 2^-100 or more.
+// The 128-wide transform, which is this library's own definition, always scales once, with the closing 1/sqrt(2).
+constexpr float kOnceLimit = 0x1p119f;   // inputs below this in magnitude cannot overflow on the way
+
+template <int G, bool ONCE = false> __device__ __forceinline__ void rotate_chunk(float* v, float* wl, int lane) {
     // strides 1 and 4: inside the lane
-    constexpr bool HV = G != 128;
+    constexpr float H = G == 128 || ONCE ? 1.0f : 0.5f;                        // a stage's factor
+    constexpr float HL = !ONCE ? 0.5f : G == 256 ? 0.0625f : 0.125f;           // the last stage's (256 and 64)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) bfly4<HV>(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+    for (int i = 0; i < 4; ++i) bfly4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3], H);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) bfly4<HV>(v[j], v[j + 4], v[j + 8], v[j + 12]);
+    for (int j = 0; j < 4; ++j) bfly4(v[j], v[j + 4], v[j + 8], v[j + 12], H);
     // to LDS in row order
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -54,9 +59,9 @@ template <int G> __device__ __forceinline__ void rotate_chunk(float* v, float* w
 #pragma unroll
         for (int a = 0; a < 16; ++a) w[a] = wl[lds_pos(base + a * 16)];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) bfly4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
+        for (int i = 0; i < 4; ++i) bfly4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3], H);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) bfly4(w[j], w[j + 4], w[j + 8], w[j + 12]);
+        for (int j = 0; j < 4; ++j) bfly4(w[j], w[j + 4], w[j + 8], w[j + 12], HL);
 #pragma unroll
         for (int a = 0; a < 16; ++a) wl[lds_pos(base + a * 16)] = w[a];
     } else if (G == 64) {
@@ -65,10 +70,10 @@ template <int G> __device__ __forceinline__ void rotate_chunk(float* v, float* w
         float4 w[4];
 #pragma unroll
         for (int d = 0; d < 4; ++d) w[d] = *reinterpret_cast<float4*>(wl + lds_pos(base + d * 16));
-        bfly4(w[0].x, w[1].x, w[2].x, w[3].x);
-        bfly4(w[0].y, w[1].y, w[2].y, w[3].y);
-        bfly4(w[0].z, w[1].z, w[2].z, w[3].z);
-        bfly4(w[0].w, w[1].w, w[2].w, w[3].w);
+        bfly4(w[0].x, w[1].x, w[2].x, w[3].x, HL);
+        bfly4(w[0].y, w[1].y, w[2].y, w[3].y, HL);
+        bfly4(w[0].z, w[1].z, w[2].z, w[3].z, HL);
+        bfly4(w[0].w, w[1].w, w[2].w, w[3].w, HL);
 #pragma unroll
         for (int d = 0; d < 4; ++d) *reinterpret_cast<float4*>(wl + lds_pos(base + d * 16)) = w[d];
     } else {
@@ -82,8 +87,8 @@ template <int G> __device__ __forceinline__ void rotate_chunk(float* v, float* w
             for (int d = 0; d < 4; ++d) w[t][d] = *reinterpret_cast<float2*>(wl + lds_pos(base + t * 64 + d * 16));
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            bfly4<false>(w[t][0].x, w[t][1].x, w[t][2].x, w[t][3].x);
-            bfly4<false>(w[t][0].y, w[t][1].y, w[t][2].y, w[t][3].y);
+            bfly4(w[t][0].x, w[t][1].x, w[t][2].x, w[t][3].x);
+            bfly4(w[t][0].y, w[t][1].y, w[t][2].y, w[t][3].y);
         }
         const float c = 0.70710678118654752f * 0.125f;
 #pragma unroll

@@ -90,22 +90,27 @@ template <int MODE> __device__ __forceinline__ void load16(const void* x, int64_
     }
 }
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
-}
-
 // Sum over the waves of one row in fp64, rounded to fp32 once (every wave of the block calls it).
 __device__ __forceinline__ float row_sum_f64(double v, double* red, int wave, int lane, int wpr, int rloc) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    v = wave_sum_f64(v);
+    if (wpr == 1) return (float)v;
     __syncthreads();
     if (lane == 0) red[wave] = v;
     __syncthreads();
     double t = 0.0;
     for (int i = 0; i < wpr; ++i) t += red[rloc * wpr + i];
     return (float)t;
+}
+
+// 1/sqrt(a) in fp64, rounded to fp32: two Newton steps on the hardware's fp32 estimate (23 bits, then 45, then the rounding
+// of fp64), a tenth of the instructions of the fp64 square root and division, which serve the ends of the range.
+__device__ __forceinline__ float rsqrt_cr(float a) {
+    if (!(a > 1e-30f && a < 1e30f)) return (float)(1.0 / sqrt((double)a));
+    const double d = (double)a;
+    double y = (double)__builtin_amdgcn_rsqf(a);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) y = __builtin_fma(0.5 * y, __builtin_fma(-d * y, y, 1.0), y);
+    return (float)y;
 }
 
 // PRO: the row prologue (csrc/kernels.cu:88-182) runs on the values as they are loaded, with the reference's rounding
@@ -192,16 +197,14 @@ __global__ void __launch_bounds__(512) quant_rows_kernel(QuantArgs p) {
             } else if (pro == PRO_GATE) {                                            // csrc/kernels.cu:95-100
                 float gg[16];
                 load16<TMODE>(p.g, m * p.g_stride + e0, gg);
-                map16(p.tab.sigmoid_bf16, gg, gg, [](float x) { return sigmoid_f(x); });
 #pragma unroll
-                for (int i = 0; i < 16; ++i) v[c][i] = R(v[c][i] * gg[i]);
+                for (int i = 0; i < 16; ++i) v[c][i] = R(v[c][i] * (MODE == MODE_BF16 ? R(sigmoid_of_bf16(gg[i])) : sigmoid_f(gg[i])));
             } else if (pro == PRO_SWIGLU || pro == PRO_SITU || pro == PRO_SITU_FAST) {  // :101-112
                 float u[16];
                 load16<TMODE>(p.x, m * p.x_stride + p.up_offset + e0, u);
                 if (pro == PRO_SWIGLU) {
-                    map16(p.tab.silu_bf16, v[c], v[c], [](float x) { return silu_f(x); });
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) v[c][i] = R(v[c][i] * u[i]);
+                    for (int i = 0; i < 16; ++i) v[c][i] = R(R(MODE == MODE_BF16 ? silu_of_bf16(v[c][i]) : silu_f(v[c][i])) * u[i]);
                 } else if (MODE == MODE_BF16 && p.tab.situ_gate_bf16) {
 #pragma unroll
                     for (int i = 0; i < 16; ++i)
@@ -211,7 +214,8 @@ __global__ void __launch_bounds__(512) quant_rows_kernel(QuantArgs p) {
                     for (int i = 0; i < 16; ++i) v[c][i] = situ_f(v[c][i], u[i]);
                 }
             } else if (pro == PRO_SILU) {
-                map16(p.tab.silu_bf16, v[c], v[c], [](float x) { return silu_f(x); });
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v[c][i] = R(MODE == MODE_BF16 ? silu_of_bf16(v[c][i]) : silu_f(v[c][i]));
             } else if (pro == PRO_GELU) {
                 map16(p.tab.gelu_bf16, v[c], v[c], [](float x) { return gelu_f(x); });
             } else if (pro == PRO_GELU_TANH) {
@@ -241,7 +245,7 @@ __global__ void __launch_bounds__(512) quant_rows_kernel(QuantArgs p) {
             }
         }
         const float ss = row_sum_f64(part, dred, wave, lane, p.wpr, rloc);
-        const float rstd = (float)(1.0 / sqrt((double)(ss / (float)p.K + p.eps)));   // :148
+        const float rstd = rsqrt_cr(ss / (float)p.K + p.eps);                        // :148
 #pragma unroll
         for (int c = 0; c < C; ++c) {
             const int e0 = (wr + c * p.wpr) * kChunk + lane * 16;
@@ -286,7 +290,18 @@ __global__ void __launch_bounds__(512) quant_rows_kernel(QuantArgs p) {
     for (int c = 0; c < C; ++c) {
         const int e0 = (wr + c * p.wpr) * kChunk + lane * 16;
         const bool act = row_ok && e0 < p.K;
-        if (G != 0) rotate_chunk<G>(v[c], wl, lane);
+        if constexpr (G != 0) {
+            // scaled once where that is exact (rotate_chunk): f16 rows always, bf16 values below the overflow limit
+            bool once = G != 128 && MODE == MODE_SD_F16;
+            if (G != 128 && MODE == MODE_BF16 && pro != PRO_SITU && pro != PRO_SITU_FAST) {
+                float big = 0.f;
+#pragma unroll
+                for (int i = 0; i < 16; i += 2) big = fmaxf(fmaxf(big, fabsf(v[c][i])), fabsf(v[c][i + 1]));
+                once = __builtin_amdgcn_ballot_w64(big >= kOnceLimit) == 0;
+            }
+            if (once) rotate_chunk<G, true>(v[c], wl, lane);
+            else rotate_chunk<G>(v[c], wl, lane);
+        }
         if (MODE == MODE_ROT_F32) {
             if (act) {
                 float4* o = reinterpret_cast<float4*>(p.out_f + m * (int64_t)p.K + e0);
@@ -294,17 +309,20 @@ __global__ void __launch_bounds__(512) quant_rows_kernel(QuantArgs p) {
                 for (int i = 0; i < 4; ++i) o[i] = make_float4(v[c][4 * i], v[c][4 * i + 1], v[c][4 * i + 2], v[c][4 * i + 3]);
             }
         } else if (MODE == MODE_SD_F16) {
-            // the maximum is taken over the half-rounded row (csrc/sd.cu:587)
+            // the maximum is taken over the half-rounded row (csrc/sd.cu:587), which is also what is divided below
 #pragma unroll
-            for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(rnd_dt<DT_F16>(v[c][i])));
+            for (int i = 0; i < 16; i += 2) {
+                unpack_f16x2(pack_f16x2(v[c][i], v[c][i + 1]), v[c][i], v[c][i + 1]);
+                amax = fmaxf(fmaxf(amax, fabsf(v[c][i])), fabsf(v[c][i + 1]));
+            }
         } else {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(v[c][i]));
+            for (int i = 0; i < 16; i += 2) amax = fmaxf(fmaxf(amax, fabsf(v[c][i])), fabsf(v[c][i + 1]));
         }
     }
     if (MODE == MODE_ROT_F32) return;
 
-    amax = wave_max(amax);
+    amax = wave_max_f32(amax);
     if (p.wpr > 1) {  // uniform over the block
         if (lane == 0) red[wave] = amax;
         __syncthreads();
@@ -313,10 +331,13 @@ __global__ void __launch_bounds__(512) quant_rows_kernel(QuantArgs p) {
     }
 
     float scale, st, rinv = 0.f;
+    bool by_rcp = true;   // f16 rows: st is a finite half
     if (MODE == MODE_SD_F16) {
         scale = fmaxf(amax, 1e-30f) / 127.f;                       // csrc/sd.cu:589
         const float sh = rnd_dt<DT_F16>(scale);
         st = sh > 0.f ? sh : scale;                                // :593
+        by_rcp = __builtin_amdgcn_ballot_w64(!(sh > 0.f && sh < __builtin_inff())) == 0;
+        rinv = __builtin_amdgcn_rcpf(st);
     } else if (MODE == MODE_BF16) {
         scale = fmaxf(fminf(amax, 3.38953139e38f) * (1.f / 127.f), 1.0e-30f);  // csrc/kernels.cu:241
         st = rnd_dt<DT_BF16>(scale);
@@ -327,48 +348,65 @@ __global__ void __launch_bounds__(512) quant_rows_kernel(QuantArgs p) {
     }
     if (row_ok && wr == 0 && lane == 0) p.scales[m] = scale;
 
+    const auto store = [&](auto rcp_tag) {
 #pragma unroll
-    for (int c = 0; c < C; ++c) {
-        const int e0 = (wr + c * p.wpr) * kChunk + lane * 16;
-        if (!(row_ok && e0 < p.K)) continue;
-        uint32_t w[4];
+        for (int c = 0; c < C; ++c) {
+            const int e0 = (wr + c * p.wpr) * kChunk + lane * 16;
+            if (!(row_ok && e0 < p.K)) continue;
+            uint32_t w[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            uint32_t acc = 0;
+            for (int i = 0; i < 4; ++i) {
+                uint32_t acc = 0;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float x = v[c][4 * i + j];
-                float t;
-                if (MODE == MODE_BF16) {
-                    // Both operands carry 8 significant bits, so their exact quotient is never closer than 2^-17
-                    // (relative) to a bf16 rounding boundary: a 1-ulp reciprocal times the numerator rounds to the
-                    // same bf16 value as the IEEE quotient does.
-                    t = rnd_dt<DT_BF16>(rnd_dt<DT_BF16>(x) * rinv);
-                } else if (MODE == MODE_SD_F16) {
-                    t = rnd_dt<DT_F16>(rnd_dt<DT_F16>(x) / st);
-                } else {
-                    t = x / st;
+                for (int j = 0; j < 4; ++j) {
+                    const float x = v[c][4 * i + j];
+                    float t;
+                    if (MODE == MODE_BF16) {
+                        // Both operands carry 8 significant bits, so their exact quotient is never closer than 2^-17
+                        // (relative) to a bf16 rounding boundary: a 1-ulp reciprocal times the numerator rounds to the
+                        // same bf16 value as the IEEE quotient does.
+                        t = rnd_dt<DT_BF16>(rnd_dt<DT_BF16>(x) * rinv);
+                    } else if (MODE == MODE_SD_F16) {
+                        // Both operands carry 11 significant bits: their quotient never equals a midpoint of two halves and
+                        // is 2^-23 (relative) away at least, more than the error left after one correction of x * rcp.
+                        float qt;
+                        if constexpr (decltype(rcp_tag)::value) {
+                            const float q0 = x * rinv;
+                            qt = __builtin_fmaf(__builtin_fmaf(-q0, st, x), rinv, q0);
+                        } else {
+                            qt = x / st;
+                        }
+                        t = rnd_dt<DT_F16>(qt);
+                    } else {
+                        t = x / st;
+                    }
+                    if (SR && (MODE == MODE_BF16 || MODE == MODE_F32)) {   // csrc/kernels.cu:1385-1388
+                        const uint64_t key = (uint64_t)(m * (int64_t)p.K + e0 + 4 * i + j) + p.seed;
+                        const float noise = (float)(pcg_hash((uint32_t)key ^ (uint32_t)(key >> 32)) >> 8) * 0x1.0p-24f;
+                        const float r = floorf(MODE == MODE_F32 ? t + noise : bf16_add_once(t, rnd_dt<DT_BF16>(noise)));
+                        const int qi = (int)fminf(127.f, fmaxf(-128.f, r));
+                        acc |= ((uint32_t)qi & 0xffu) << (8 * j);
+                    } else if (MODE == MODE_F32) {
+                        const int qi = (int)fminf(127.f, fmaxf(-128.f, nearbyintf(t)));
+                        acc |= ((uint32_t)qi & 0xffu) << (8 * j);
+                    } else {
+                        // clamp(rint(t), -128, 127) + 128 as one instruction: t is a 16-bit float, so t + 128 is exact
+                        // wherever t has a bit at 2^-16 or above set, and below that both t and t + 128 round to the
+                        // same integer; v_cvt_pk_u8_f32 rounds to nearest even, saturates to 0..255 (NaN to 0, which is
+                        // the -128 that fminf(127, fmaxf(-128, NaN)) gives) and drops the byte into place.
+                        acc = __builtin_amdgcn_cvt_pk_u8_f32(t + 128.f, j, acc);
+                    }
                 }
-                if (SR && (MODE == MODE_BF16 || MODE == MODE_F32)) {   // csrc/kernels.cu:1385-1388
-                    const uint64_t key = (uint64_t)(m * (int64_t)p.K + e0 + 4 * i + j) + p.seed;
-                    const float noise = (float)(pcg_hash((uint32_t)key ^ (uint32_t)(key >> 32)) >> 8) * 0x1.0p-24f;
-                    const float r = floorf(MODE == MODE_F32 ? t + noise : bf16_add_once(t, rnd_dt<DT_BF16>(noise)));
-                    const int qi = (int)fminf(127.f, fmaxf(-128.f, r));
-                    acc |= ((uint32_t)qi & 0xffu) << (8 * j);
-                } else if (MODE == MODE_F32) {
-                    const int qi = (int)fminf(127.f, fmaxf(-128.f, nearbyintf(t)));
-                    acc |= ((uint32_t)qi & 0xffu) << (8 * j);
-                } else {
-                    // clamp(rint(t), -128, 127) + 128 as one instruction: t is a 16-bit float, so t + 128 is exact
-                    // wherever t has a bit at 2^-16 or above set, and below that both t and t + 128 round to the
-                    // same integer; v_cvt_pk_u8_f32 rounds to nearest even, saturates to 0..255 (NaN to 0, which is
-                    // the -128 that fminf(127, fmaxf(-128, NaN)) gives) and drops the byte into place.
-                    acc = __builtin_amdgcn_cvt_pk_u8_f32(t + 128.f, j, acc);
-                }
+                w[i] = (!SR && MODE != MODE_F32) ? acc ^ 0x80808080u : acc;
             }
-            w[i] = (!SR && MODE != MODE_F32) ? acc ^ 0x80808080u : acc;
+            *reinterpret_cast<uint4*>(p.q + m * (int64_t)p.K + e0) = make_uint4(w[0], w[1], w[2], w[3]);
         }
-        *reinterpret_cast<uint4*>(p.q + m * (int64_t)p.K + e0) = make_uint4(w[0], w[1], w[2], w[3]);
+    };
+    if constexpr (MODE == MODE_SD_F16) {
+        if (by_rcp) store(std::true_type{});
+        else store(std::false_type{});
+    } else {
+        store(std::true_type{});
     }
 }
 
@@ -531,4 +569,21 @@ GPU_API int gpu_convrot_requant(int dtype, const void* x, void* q, void* s, int6
     if (K > 32768 || N > 0x7fffffff) return -2;
     QuantArgs a{x, K, (int8_t*)q, (float*)s, nullptr, (int)N, K, 1, 1, seed};
     return dtype == DT_F32 ? run_quant<MODE_F32>(a, 256, (hipStream_t)stream) : run_quant<MODE_BF16>(a, 256, (hipStream_t)stream);
+}
+
+// Test hook: out[i] = bf16 bits of sigmoid (which 0) or silu (1) of the bf16 bits in[i], as the prologues evaluate them.
+namespace {
+__global__ void __launch_bounds__(256) act_probe_kernel(int which, const uint16_t* in, uint16_t* out, int n) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const float x = bf16_to_f(in[i]);
+    out[i] = f_to_bf16(which == 0 ? sigmoid_of_bf16(x) : silu_of_bf16(x));
+}
+}  // namespace
+GPU_API int gpu_internal_act_probe(int which, const void* in, void* out, int n, void* stream) {
+    if (which < 0 || which > 1 || !in || !out || n <= 0) return -1;
+    hipLaunchKernelGGL(act_probe_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, which, (const uint16_t*)in,
+                       (uint16_t*)out, n);
+    KCHECK();
+    return 0;
 }

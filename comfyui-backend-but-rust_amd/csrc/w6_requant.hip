@@ -108,12 +108,18 @@ __global__ void __launch_bounds__(1024) w6_requant_kernel(const uint16_t* w, uin
             for (int i = 0; i < 16; ++i) v[c][i] = 0.f;
         }
         // ConvRot256 (:174-206) as the row quantizer does it; the rotated row is kept in the weight dtype (:209-217)
-        convrot::rotate_chunk<256>(v[c], tiles + wave * convrot::kLdsPerWave, lane);
         float m = 0.f;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            v[c][i] = rnd_dt<DT_BF16>(v[c][i]);
-            m = fmaxf(m, fabsf(v[c][i]));
+        for (int i = 0; i < 16; i += 2) m = fmaxf(fmaxf(m, fabsf(v[c][i])), fabsf(v[c][i + 1]));
+        if (__builtin_amdgcn_ballot_w64(m >= convrot::kOnceLimit) == 0) convrot::rotate_chunk<256, true>(v[c], tiles + wave * convrot::kLdsPerWave, lane);
+        else convrot::rotate_chunk<256>(v[c], tiles + wave * convrot::kLdsPerWave, lane);
+        m = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; i += 2) {
+            const uint32_t u = pack_bf16x2(v[c][i], v[c][i + 1]);
+            v[c][i] = u2f(u << 16);
+            v[c][i + 1] = u2f(u & 0xffff0000u);
+            m = fmaxf(fmaxf(m, fabsf(v[c][i])), fabsf(v[c][i + 1]));
         }
         // the group's step by two alternating-least-squares rounds, :94-117.  num adds its 32 terms in index order: the odd
         // lane of the pair goes on where the even one ends.  den sums whole numbers below 2^15: exact in any order.

@@ -19,8 +19,10 @@ __global__ void __launch_bounds__(256) convrot_dequant_kernel(const int8_t* q, c
     const int e0 = (int)(gid % cpr) * kChunk + lane * 16;
     const bool act = m < N && e0 < K;     // a wave past the last row still runs the (barrier-free) rotation on zeros
     float v[16];
+    bool small = true;
     if (act) {
         const float sc = s[m];
+        small = fabsf(sc) >= 0x1p-100f && fabsf(sc) < 0x1p100f;   // the product's last bit and the sums stay in range
         const uint4 u = *reinterpret_cast<const uint4*>(q + m * K + e0);
         const uint32_t w[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
@@ -29,7 +31,8 @@ __global__ void __launch_bounds__(256) convrot_dequant_kernel(const int8_t* q, c
 #pragma unroll
         for (int i = 0; i < 16; ++i) v[i] = 0.f;
     }
-    rotate_chunk<256>(v, wl, lane);
+    if (__builtin_amdgcn_ballot_w64(!small) == 0) rotate_chunk<256, true>(v, wl, lane);
+    else rotate_chunk<256>(v, wl, lane);
     if (!act) return;
     if (OUT == OUT_BF16) {
         uint32_t w[8];

@@ -112,7 +112,7 @@ int gpu_convrot_requant(int dtype, const void* x, void* q, void* s, int64_t N, i
  * for the step of every 32 columns, packed [N, 3K/4] (nibble plane then 2-bit plane, code = q + 32), s_rel fp8-e4m3
  * [N, K/32], s_channel f32 [N]; every value is rounded stochastically between its two bracketing grid levels, keyed by
  * element index and seed.  Replaces gpu_w6_requant, src/ffi.rs:132 / csrc/vendor/w6a8_requant.cu:242-252.
- * K % 256 (-1), K <= 39 680 (-2: the rotated row is held in LDS). */
+ * K % 256 (-1), K <= 39 680 (-2). */
 int gpu_w6_requant(const void* weight, void* packed, void* s_rel, void* s_channel, int64_t N, int K, uint64_t seed,
                    void* stream);
 
@@ -173,6 +173,10 @@ int gpu_int8_attn_key_bias(const void* q, const void* k, const void* v, void* o,
                            int hk, int64_t q_bs, int64_t q_rs, int64_t q_hs, int64_t k_bs, int64_t k_rs, int64_t k_hs,
                            int64_t v_bs, int64_t v_rs, int64_t v_hs, int64_t o_bs, int64_t o_rs, int64_t o_hs, float scale,
                            const float* bias, void* stream);
+
+/* Test hook, no reference counterpart: out[i] = bf16 sigmoid (which 0) or silu (1) of the bf16 bits in[i], evaluated as the
+ * quantizer's prologues evaluate it. */
+int gpu_internal_act_probe(int which, const void* in, void* out, int n, void* stream);
 
 /* Test hook, no reference counterpart: y[i] = the gfx950 float -> u8 pack conversion of x[i] (byte 0), which the attention
  * kernel's probabilities rely on being round-to-nearest-even with saturation to 0..255. */

@@ -273,6 +273,55 @@ def test_quant_rows_with_prologue_equals_prologue_then_quantizer(M, K, rotate, d
         assert np.array_equal(qd.cpu().numpy(), q), pro
 
 
+def test_sigmoid_and_silu_of_every_bf16_value():
+    """The prologues' sigmoid and SiLU come from the hardware's exp2 and reciprocal: all 65536 inputs against the oracle."""
+    bits = np.arange(65536, dtype=np.uint16).reshape(1, -1)
+    one = np.full((1, 65536), 0x3F80, np.uint16)
+    rc, silu = oracle.prologue_rows(BF16, PRO_ID["SILU"], bits, 65536)
+    rc2, gate = oracle.prologue_rows(BF16, PRO_ID["GATE"], one, 65536, g=bits)
+    assert rc == 0 and rc2 == 0
+    out = torch.zeros(65536, dtype=torch.int16, device=DEV)
+    for which, want in ((0, gate), (1, silu)):
+        say("act probe", which)
+        ffi.k("gpu_internal_act_probe", which, dev(bits.view(np.int16)).data_ptr(), out.data_ptr(), 65536, 0)
+        torch.cuda.synchronize()
+        got = out.cpu().numpy().view(np.uint16)
+        nan = (want[0] & 0x7FFF) > 0x7F80
+        assert np.array_equal(nan, (got & 0x7FFF) > 0x7F80)
+        bad = np.nonzero((got != want[0]) & ~nan)[0]
+        assert bad.size == 0, [(hex(int(b)), hex(int(got[b])), hex(int(want[0][b]))) for b in bad[:20]]
+
+
+@pytest.mark.parametrize("rotate", [64, 256])
+@pytest.mark.parametrize("M,K", [(4, 256), (3, 1280), (2, 5120)])
+def test_rotation_scaled_once_and_per_stage(M, K, rotate):
+    """Rows either side of the magnitudes up to which the rotation's halvings are one multiplication: both branches equal the
+    oracle's halving per stage, bit for bit, also beside values that overflow, subnormal ones and weight scales out of range."""
+    x = synth.normal(60 + K, rotate, M * K).reshape(M, K)
+    for gain in (1e-38, 1e-30, 1.0, 2.0 ** 117, 2.0 ** 120, 2.0 ** 126):
+        say("rotation", M, K, rotate, gain)
+        row = (x * np.float32(gain)).astype(np.float32)
+        row[:, 1::7] = np.float32(2.0 ** -131)
+        xb = synth.bf16_bits(row)
+        rc, q, s = oracle.quant_rows(BF16, xb, K, rotate)
+        qd, sd = ql.quant_rows(dev_bits(xb, BF16), rotate)
+        torch.cuda.synchronize()
+        assert rc == 0 and np.array_equal(sd.cpu().numpy().view(np.uint32), s.view(np.uint32)) and np.array_equal(qd.cpu().numpy(), q)
+    for gain in (2.0 ** -24, 2.0 ** -12, 1.0, 8000.0):   # f16: scales below the half range, subnormal halves, values near the top
+        xh = synth.f16_bits(np.clip(x * np.float32(gain), -60000, 60000))
+        rc, q, s = oracle.sd_quant_rows(xh, K, rotate)
+        qd, sd = ql.sd_quant_rows(dev_bits(xh, F16), rotate)
+        torch.cuda.synchronize()
+        assert rc == 0 and np.array_equal(sd.cpu().numpy().view(np.uint32), s.view(np.uint32)) and np.array_equal(qd.cpu().numpy(), q), gain
+    if rotate == 256:
+        qw = synth.randint(61, K, M * K, -127, 127).astype(np.int8).reshape(M, K)
+        sc = np.array([1e-3, 1e-36, 1e33, 0.0], np.float32)[:M]
+        rc, want = oracle.convrot_dequant(F32, qw, sc)
+        got = ql.convrot_dequant(dev(qw), dev(sc), torch.float32)
+        torch.cuda.synchronize()
+        assert rc == 0 and np.array_equal(got.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
 def test_quant_rows_b_and_rotate_rows_f32_with_prologues():
     M, K = 5, 1536
     c = pro_case(BF16, 801, M, K, K + 16)
