@@ -49,31 +49,36 @@ __device__ __forceinline__ float pair_lane(float x) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0xB1, 0xf, 0xf, false));
 }
 
-// Four values of a group -> their code bytes (level index + 1), :63-80,126-148.
-// The first level at or above t: levels are whole numbers, so it is the first that reaches ceil(t), i.e. whose product
-// (i - 31) s reaches ceil(t) - 1/2 (or passes it, where that tie rounds down to an even number).  With z that quotient,
-// rint(z) is the position or the one before it, however the division's last bit falls: a whole z needs the tie looked at,
-// and any other z is farther from a whole number than the bit reaches.  One look at the level there settles it.  Outside
-// [-127, 127] every level is on one side of t and the position is an end of the grid (ENDS; a lane meets it only when
-// its group holds a value beyond the row's largest decoded one).
+// Four values of a group -> their code bytes (level index + 1), :63-80,126-148.  Wanted is the pair of neighbouring levels
+// with level(l) < t <= level(l + 1), l in -31..30 (ends beyond t count as bracketing it).  Any f in -30..30 next to the
+// pair settles it by one look: l is f when level(f) is below t, else f - 1; the sign of level(f) - t stands for the compare.
+//   plain (every lane's step in [1, 4], every |t| < 127): f = rint(t / s).  f s is within s/2 of t and a level within 1/2
+//     of its product, so level(f - 1) < t <= level(f + 1) for s >= 1, whichever way t / s falls at a tie; no level
+//     reaches the clamp at +-127; and f s is a 6-bit times a 4-bit number, so adding 1.5 * 2^23 rounds it as rint does.
+//   else: levels are whole numbers, so the first level at or above t is the first that reaches ceil(t), i.e. whose product
+//     reaches ceil(t) - 1/2 (or passes it, where that tie rounds down to an even number).  With z that quotient, rint(z) is
+//     that position or the one before it: a whole z needs the tie looked at, any other is farther from a whole number
+//     than the last bit of the division reaches.  Outside [-127, 127] every level is on one side of t: an end of the grid.
 // `x0` is the hash input of value 0 without its low four bits' share, kc[j] that share (see the caller).
-template <bool ENDS>
+template <bool PLAIN>
 __device__ __forceinline__ uint32_t codes4(const float* v, float inv_sc, float s, float inv_s, uint32_t x0, const uint32_t* kc) {
+    constexpr float M = 12582912.f;
     uint32_t out = 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const float t = v[j] * inv_sc;
-        const float f = __builtin_amdgcn_fmed3f(__builtin_rintf((__builtin_ceilf(t) - 0.5f) * inv_s), -31.f, 32.f);
-        // position minus one: f when the level there is still below t, else f - 1; the sign bit stands for the compare
-        const int below = (int)f2u(level(f, s) - t) >> 31;
-        float l = __builtin_amdgcn_fmed3f(f - u2f(~below & 0x3f800000u), -31.f, 30.f);   // the lower of the two levels, :75-80
-        if (ENDS) l = t > 127.f ? 30.f : t <= -127.f ? -31.f : l;
-        const float l0 = level(l, s), l1 = level(l + 1.f, s);
+        float f, lf, lg;
+        if (PLAIN) f = __builtin_fmaf(t, inv_s, M) - M;
+        else f = t > 127.f ? 30.f : t <= -127.f ? -30.f : __builtin_rintf((__builtin_ceilf(t) - 0.5f) * inv_s);
+        f = __builtin_amdgcn_fmed3f(f, -30.f, 30.f);
+        lf = PLAIN ? __builtin_fmaf(f, s, M) - M : level(f, s);
+        const float g = f - __builtin_copysignf(1.f, lf - t);                     // the pair's other end
+        lg = PLAIN ? __builtin_fmaf(g, s, M) - M : level(g, s);
         const uint32_t h = x0 + kc[j];                                            // x * 747796405 + 2891336453, :21-25
         const uint32_t w = ((h >> ((h >> 28u) + 4u)) ^ h) * 277803737u;
         const float u = (float)(((w >> 22u) ^ w) >> 8) * (1.0f / 16777216.0f);    // :27-31
-        const float d = __builtin_fmaf(u, l1 - l0, l0) - t;                       // negative where t is above the threshold
-        out = __builtin_amdgcn_cvt_pk_u8_f32(l + 32.25f - __builtin_copysignf(0.5f, d), j, out);
+        const float d = __builtin_fmaf(u, fabsf(lg - lf), fminf(lf, lg)) - t;     // negative where t is above the threshold
+        out = __builtin_amdgcn_cvt_pk_u8_f32(fminf(f, g) - __builtin_copysignf(0.5f, d) + 32.25f, j, out);
     }
     return out;
 }
@@ -126,11 +131,13 @@ __global__ void __launch_bounds__(1024) w6_requant_kernel(const uint16_t* w, uin
         m = fmaxf(m, pair_lane(m));
         float step = fmaxf(m / 31.0f, 1e-8f), inv = 1.0f / step;
         bool nan = false;
+#pragma unroll
         for (int it = 0; it < 2; ++it) {
             float q[16], num = 0.f, den = 0.f;
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                q[i] = __builtin_amdgcn_fmed3f(__builtin_rintf(v[c][i] * inv), -31.0f, 31.0f);
+                q[i] = __builtin_rintf(v[c][i] * inv);
+                if (it > 0) q[i] = __builtin_amdgcn_fmed3f(q[i], -31.0f, 31.0f);   // the first step is the largest value's 31st part
                 num = __builtin_fmaf(v[c][i], q[i], num);
                 den = __builtin_fmaf(q[i], q[i], den);
             }
@@ -176,13 +183,27 @@ __global__ void __launch_bounds__(1024) w6_requant_kernel(const uint16_t* w, uin
         if (!(lane & 1)) s_rel[n * (K / kG) + e0 / kG] = (uint8_t)bits;
         const float sr = e4m3_to_f(bits), inv_sr = 1.0f / fmaxf(sr, 1e-30f);
         const uint32_t x0 = ((uint32_t)(n * K + e0) ^ (s32 & ~15u)) * 747796405u;
-        uint32_t cw[4];
-        if (__builtin_amdgcn_ballot_w64(gmax[c] * inv_sc >= 127.f) == 0) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) cw[i] = codes4<false>(v[c] + 4 * i, inv_sc, sr, inv_sr, x0, kc + 4 * i);
-        } else {
+        uint32_t cw[4] = {0u, 0u, 0u, 0u};
+        if (__builtin_amdgcn_ballot_w64(!(gmax[c] * inv_sc < 127.f && sr >= 1.f && sr <= 4.f)) == 0) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) cw[i] = codes4<true>(v[c] + 4 * i, inv_sc, sr, inv_sr, x0, kc + 4 * i);
+        } else {
+#pragma unroll 1
+            for (int i = 0; i < 4; ++i) {
+                // the loop stays rolled: this is the rare form
+                float x[4];
+                uint32_t k4[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    x[j] = i == 0 ? v[c][j] : i == 1 ? v[c][4 + j] : i == 2 ? v[c][8 + j] : v[c][12 + j];
+                    k4[j] = i == 0 ? kc[j] : i == 1 ? kc[4 + j] : i == 2 ? kc[8 + j] : kc[12 + j];
+                }
+                const uint32_t o = codes4<false>(x, inv_sc, sr, inv_sr, x0, k4);
+                cw[0] = i == 0 ? o : cw[0];
+                cw[1] = i == 1 ? o : cw[1];
+                cw[2] = i == 2 ? o : cw[2];
+                cw[3] = i == 3 ? o : cw[3];
+            }
         }
         // nibbles of codes 2j, 2j + 1 share a byte; the top bits of four codes share one (the product lines them up in
         // its upper byte, and nothing below carries into it)
