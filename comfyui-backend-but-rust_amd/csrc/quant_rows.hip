@@ -113,15 +113,24 @@ __device__ __forceinline__ float rsqrt_cr(float a) {
     return (float)y;
 }
 
-// PRO: the row prologue (csrc/kernels.cu:88-182) runs on the values as they are loaded, with the reference's rounding
-// points; p.pro selects it at run time.  Row sums are fp64, rounded once; the activation functions are correctly rounded.
+// CLS: the class of the row prologue (csrc/kernels.cu:88-182), which runs on the values as they are loaded, with the
+// reference's rounding points; p.pro selects the prologue within its class at run time.  Row sums are fp64, rounded once;
+// the activation functions are correctly rounded.  The classes keep what is cheap in registers apart from what calls
+// the fp64 routines: in one kernel for all, SwiGLU and the norms had the 123 registers of those calls, four waves per SIMD
+// (GEGLU 8192 x 2560 53.3 us, LayerNorm 8192 x 640 14.9 us; by class 48.8 and 13.3).
 // SR: stochastic rounding keyed by element index + p.seed (gpu_convrot_requant); a kernel variant of its own, so that the
 // plain quantizer carries neither the hash nor a branch per element.
-template <int MODE, int G, int C, bool PRO, bool SR = false>
-__global__ void __launch_bounds__(512) quant_rows_kernel(QuantArgs p) {
+enum {
+    CLS_PLAIN,
+    CLS_NORM,    // RMS, LAYERNORM, ADALN, LN_MOD, LN_AFFINE
+    CLS_GATED,   // bf16 rows: GATE, SWIGLU, SILU; f16 rows: GEGLU through its table
+    CLS_REST     // everything that may evaluate an fp64 routine, and the SD gathers
+};
+template <int MODE, int G, int C, int CLS, bool SR = false>
+__global__ void __launch_bounds__(1024) quant_rows_kernel(QuantArgs p) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    __shared__ float red[8];
-    __shared__ double dred[8];
+    __shared__ float red[16];
+    __shared__ double dred[16];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int rloc = wave / p.wpr, wr = wave - rloc * p.wpr;
     const int64_t m = (int64_t)blockIdx.x * p.rpb + rloc;
@@ -145,15 +154,15 @@ __global__ void __launch_bounds__(512) quant_rows_kernel(QuantArgs p) {
 
     float v[C][16];
     float amax = 0.f;
-    const int pro = PRO ? p.pro : PRO_PLAIN;
-    const bool ln = pro == PRO_LAYERNORM || pro == PRO_LN_MOD || pro == PRO_LN_AFFINE;
-    const bool norm = ln || pro == PRO_RMS || pro == PRO_ADALN;
+    constexpr bool NORM = CLS == CLS_NORM, GATED = CLS == CLS_GATED, REST = CLS == CLS_REST;
+    const int pro = CLS == CLS_PLAIN ? PRO_PLAIN : p.pro;
+    const bool ln = NORM && (pro == PRO_LAYERNORM || pro == PRO_LN_MOD || pro == PRO_LN_AFFINE);
     double part = 0.0;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
         const int e0 = (wr + c * p.wpr) * kChunk + lane * 16;
         const bool act = row_ok && e0 < p.K;
-        if (PRO && MODE == MODE_SD_F16 && pro == PRO_SD_UNPAD) {                     // csrc/sd.cu:650-652
+        if (REST && MODE == MODE_SD_F16 && pro == PRO_SD_UNPAD) {                     // csrc/sd.cu:650-652
             const uint16_t* r = (const uint16_t*)p.x + m * p.x_stride;
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
@@ -166,21 +175,46 @@ __global__ void __launch_bounds__(512) quant_rows_kernel(QuantArgs p) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) v[c][i] = 0.f;
         }
-        if (PRO && act) {
+        if (NORM && act) {
+            if (ln) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) part += (double)v[c][i];
+            } else {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) part += (double)v[c][i] * (double)v[c][i];
+            }
+        }
+        if (GATED && act) {
+            float u[16];
+            if (MODE == MODE_SD_F16) {                                               // GEGLU, csrc/sd.cu:642-649, row = [value | gate]
+                load16<TMODE>(p.x, m * p.x_stride + p.up_offset + e0, u);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) u[i] = f16_to_f(p.tab.gelu_f16[f_to_f16(u[i])]);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v[c][i] = R(v[c][i] * u[i]);
+            } else if (pro == PRO_GATE) {                                            // csrc/kernels.cu:95-100
+                load16<TMODE>(p.g, m * p.g_stride + e0, u);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v[c][i] = R(v[c][i] * R(sigmoid_of_bf16(u[i])));
+            } else {                                                                 // :101-106
+                const bool two = pro == PRO_SWIGLU;
+                if (two) load16<TMODE>(p.x, m * p.x_stride + p.up_offset + e0, u);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v[c][i] = R(silu_of_bf16(v[c][i]));
+                if (two) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) v[c][i] = R(v[c][i] * u[i]);
+                }
+            }
+        }
+        if (REST && act) {
             if (MODE == MODE_SD_F16) {
-                if (pro == PRO_SD_GEGLU) {                                           // :642-649, row = [value | gate]
+                if (pro == PRO_SD_GEGLU) {
                     float gg[16];
                     load16<TMODE>(p.x, m * p.x_stride + p.up_offset + e0, gg);
-                    if (p.tab.gelu_f16) {
 #pragma unroll
-                        for (int i = 0; i < 16; ++i) gg[i] = f16_to_f(p.tab.gelu_f16[f_to_f16(gg[i])]);
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < 16; ++i) gg[i] = R(gelu_f(gg[i]));
-                    }
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) v[c][i] = R(v[c][i] * gg[i]);
-                } else if (pro == PRO_SD_GN) {                                       // :653-662
+                    for (int i = 0; i < 16; ++i) v[c][i] = R(v[c][i] * R(gelu_f(gg[i])));
+                } else if (pro == PRO_SD_GN) {                                       // csrc/sd.cu:653-662
                     const float2* stats = (const float2*)p.g + (m / p.g_stride) * (int64_t)(p.K / p.per) * 2;
                     float nw[16], nb[16];
                     load16<MODE_F32>(p.norm_w, e0, nw);
@@ -190,21 +224,18 @@ __global__ void __launch_bounds__(512) quant_rows_kernel(QuantArgs p) {
                         const float2 st = stats[((e0 + i) / p.per) * 2];
                         v[c][i] = R(__builtin_fmaf((v[c][i] - st.x) * st.y, nw[i], nb[i]));
                     }
-                } else if (ln) {
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) part += (double)v[c][i];
                 }
-            } else if (pro == PRO_GATE) {                                            // csrc/kernels.cu:95-100
+            } else if (pro == PRO_GATE) {                                            // f32 rows from here: csrc/kernels.cu:95-112
                 float gg[16];
                 load16<TMODE>(p.g, m * p.g_stride + e0, gg);
 #pragma unroll
-                for (int i = 0; i < 16; ++i) v[c][i] = R(v[c][i] * (MODE == MODE_BF16 ? R(sigmoid_of_bf16(gg[i])) : sigmoid_f(gg[i])));
-            } else if (pro == PRO_SWIGLU || pro == PRO_SITU || pro == PRO_SITU_FAST) {  // :101-112
+                for (int i = 0; i < 16; ++i) v[c][i] = R(v[c][i] * R(sigmoid_f(gg[i])));
+            } else if (pro == PRO_SWIGLU || pro == PRO_SITU || pro == PRO_SITU_FAST) {
                 float u[16];
                 load16<TMODE>(p.x, m * p.x_stride + p.up_offset + e0, u);
                 if (pro == PRO_SWIGLU) {
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) v[c][i] = R(R(MODE == MODE_BF16 ? silu_of_bf16(v[c][i]) : silu_f(v[c][i])) * u[i]);
+                    for (int i = 0; i < 16; ++i) v[c][i] = R(R(silu_f(v[c][i])) * u[i]);
                 } else if (MODE == MODE_BF16 && p.tab.situ_gate_bf16) {
 #pragma unroll
                     for (int i = 0; i < 16; ++i)
@@ -215,21 +246,15 @@ __global__ void __launch_bounds__(512) quant_rows_kernel(QuantArgs p) {
                 }
             } else if (pro == PRO_SILU) {
 #pragma unroll
-                for (int i = 0; i < 16; ++i) v[c][i] = R(MODE == MODE_BF16 ? silu_of_bf16(v[c][i]) : silu_f(v[c][i]));
+                for (int i = 0; i < 16; ++i) v[c][i] = R(silu_f(v[c][i]));
             } else if (pro == PRO_GELU) {
                 map16(p.tab.gelu_bf16, v[c], v[c], [](float x) { return gelu_f(x); });
             } else if (pro == PRO_GELU_TANH) {
                 map16(p.tab.gelu_tanh_bf16, v[c], v[c], [](float x) { return gelu_tanh_f(x); });
-            } else if (ln) {
-#pragma unroll
-                for (int i = 0; i < 16; ++i) part += (double)v[c][i];
-            } else if (norm) {
-#pragma unroll
-                for (int i = 0; i < 16; ++i) part += (double)v[c][i] * (double)v[c][i];
             }
         }
     }
-    if (PRO && norm) {   // uniform over the block
+    if constexpr (NORM) {
         if (ln) {        // :133-145
             const float mean = row_sum_f64(part, dred, wave, lane, p.wpr, rloc) / (float)p.K;
             part = 0.0;
@@ -250,38 +275,44 @@ __global__ void __launch_bounds__(512) quant_rows_kernel(QuantArgs p) {
         for (int c = 0; c < C; ++c) {
             const int e0 = (wr + c * p.wpr) * kChunk + lane * 16;
             if (!(row_ok && e0 < p.K)) continue;
-            float msv[16], shv[16], nw[16], nb[16];
             const bool mod = p.mod_scale != nullptr;
-            if (mod) {
-                load16<TMODE>(p.mod_scale, e0, msv);
-                load16<TMODE>(p.mod_shift, e0, shv);
-            }
-            if (p.norm_w && (pro == PRO_RMS || pro == PRO_LAYERNORM || pro == PRO_LN_AFFINE)) load16<MODE_F32>(p.norm_w, e0, nw);
-            if (pro == PRO_LN_AFFINE) load16<MODE_F32>(p.norm_b, e0, nb);
-            // the form is chosen once per 16 values, not per value
+            // the form is chosen once per 16 values, and each loads only what it takes
+            float a[16], b[16];
+            const auto load_mod = [&]() {
+                if (mod) {
+                    load16<TMODE>(p.mod_scale, e0, a);
+                    load16<TMODE>(p.mod_shift, e0, b);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) a[i] = b[i] = 0.f;
+                }
+            };
             if (pro == PRO_ADALN) {                                                  // :163-166, one rounding
+                load_mod();
 #pragma unroll
-                for (int i = 0; i < 16; ++i) v[c][i] = R(__builtin_fmaf(v[c][i] * rstd, 1.f + (mod ? msv[i] : 0.f), mod ? shv[i] : 0.f));
+                for (int i = 0; i < 16; ++i) v[c][i] = R(__builtin_fmaf(v[c][i] * rstd, 1.f + a[i], b[i]));
             } else if (pro == PRO_LN_MOD) {                                          // ln_finish, :40-46
+                load_mod();
 #pragma unroll
-                for (int i = 0; i < 16; ++i) v[c][i] = R(__builtin_fmaf(R(v[c][i] * rstd), R(1.f + (mod ? msv[i] : 0.f)), mod ? shv[i] : 0.f));
+                for (int i = 0; i < 16; ++i) v[c][i] = R(__builtin_fmaf(R(v[c][i] * rstd), R(1.f + a[i]), b[i]));
             } else if (pro == PRO_LN_AFFINE) {
+                load16<MODE_F32>(p.norm_w, e0, a);
+                load16<MODE_F32>(p.norm_b, e0, b);
 #pragma unroll
-                for (int i = 0; i < 16; ++i) v[c][i] = R(__builtin_fmaf(v[c][i] * rstd, nw[i], nb[i]));
+                for (int i = 0; i < 16; ++i) v[c][i] = R(__builtin_fmaf(v[c][i] * rstd, a[i], b[i]));
             } else {                                                                 // RMS, LAYERNORM: :171-179
                 if (p.norm_w) {
+                    load16<MODE_F32>(p.norm_w, e0, a);
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) v[c][i] = R(v[c][i] * rstd * nw[i]);
+                    for (int i = 0; i < 16; ++i) v[c][i] = R(v[c][i] * rstd * a[i]);
                 } else {
 #pragma unroll
                     for (int i = 0; i < 16; ++i) v[c][i] = R(v[c][i] * rstd);
                 }
                 if (mod) {
+                    load_mod();
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        const float aa = R(1.f + msv[i]);
-                        v[c][i] = R(R(aa * v[c][i]) + shv[i]);
-                    }
+                    for (int i = 0; i < 16; ++i) v[c][i] = R(R(R(1.f + a[i]) * v[c][i]) + b[i]);
                 }
             }
         }
@@ -293,7 +324,7 @@ __global__ void __launch_bounds__(512) quant_rows_kernel(QuantArgs p) {
         if constexpr (G != 0) {
             // scaled once where that is exact (rotate_chunk): f16 rows always, bf16 values below the overflow limit
             bool once = G != 128 && MODE == MODE_SD_F16;
-            if (G != 128 && MODE == MODE_BF16 && pro != PRO_SITU && pro != PRO_SITU_FAST) {
+            if (G != 128 && MODE == MODE_BF16 && (!REST || (pro != PRO_SITU && pro != PRO_SITU_FAST))) {
                 float big = 0.f;
 #pragma unroll
                 for (int i = 0; i < 16; i += 2) big = fmaxf(fmaxf(big, fabsf(v[c][i])), fabsf(v[c][i + 1]));
@@ -410,44 +441,53 @@ __global__ void __launch_bounds__(512) quant_rows_kernel(QuantArgs p) {
     }
 }
 
-template <int MODE, int G, int C>
-int launch(const QuantArgs& a, int nw, hipStream_t st) {
-    const int grid = (a.M + a.rpb - 1) / a.rpb;
-    const size_t smem = G ? (size_t)nw * kLdsPerWave * sizeof(float) : 0;
-    constexpr bool CAN_PRO = true;
-    constexpr bool CAN_SR = (MODE == MODE_BF16 || MODE == MODE_F32) && G == 256;
-    if (CAN_SR && a.seed != 0 && a.pro == PRO_PLAIN)
-        hipLaunchKernelGGL((quant_rows_kernel<MODE, G, C, false, CAN_SR>), dim3(grid), dim3(nw * 64), smem, st, a);
-    else if (CAN_PRO && a.pro != PRO_PLAIN)
-        hipLaunchKernelGGL((quant_rows_kernel<MODE, G, C, CAN_PRO>), dim3(grid), dim3(nw * 64), smem, st, a);
-    else
-        hipLaunchKernelGGL((quant_rows_kernel<MODE, G, C, false>), dim3(grid), dim3(nw * 64), smem, st, a);
+template <auto KERN>
+int launch_kernel(const QuantArgs& a, int nw, int lds_per_wave, hipStream_t st) {
+    const int smem = nw * lds_per_wave;
+    if (smem > 63 * 1024) {   // the tiles of 15 or 16 waves are more than a kernel may have unasked
+        static PerDeviceOnce once;
+        if (const int e = allow_dynamic_lds(reinterpret_cast<const void*>(KERN), 16 * lds_per_wave, once)) return e;
+    }
+    hipLaunchKernelGGL(KERN, dim3((a.M + a.rpb - 1) / a.rpb), dim3(nw * 64), smem, st, a);
     KCHECK();
     return 0;
 }
 
-template <int MODE, int G>
-int launch_c(const QuantArgs& a, int nw, int C, hipStream_t st) {
-    switch (C) {
-        case 1: return launch<MODE, G, 1>(a, nw, st);
-        case 2: return launch<MODE, G, 2>(a, nw, st);
-        case 3: return launch<MODE, G, 3>(a, nw, st);
-        default: return launch<MODE, G, 4>(a, nw, st);
+template <int MODE, int G, int C>
+int launch(const QuantArgs& a, int nw, hipStream_t st) {
+    constexpr int lds = G ? kLdsPerWave * (int)sizeof(float) : 0;
+    constexpr bool CAN_SR = (MODE == MODE_BF16 || MODE == MODE_F32) && G == 256;
+    if (a.pro == PRO_PLAIN) {
+        if (CAN_SR && a.seed != 0) return launch_kernel<quant_rows_kernel<MODE, G, C, CLS_PLAIN, CAN_SR>>(a, nw, lds, st);
+        return launch_kernel<quant_rows_kernel<MODE, G, C, CLS_PLAIN>>(a, nw, lds, st);
     }
+    if (a.pro == PRO_RMS || a.pro == PRO_LAYERNORM || a.pro == PRO_ADALN || a.pro == PRO_LN_MOD || a.pro == PRO_LN_AFFINE)
+        return launch_kernel<quant_rows_kernel<MODE, G, C, CLS_NORM>>(a, nw, lds, st);
+    if constexpr (MODE == MODE_BF16 || MODE == MODE_SD_F16) {
+        const bool gated = MODE == MODE_BF16 ? a.pro == PRO_GATE || a.pro == PRO_SWIGLU || a.pro == PRO_SILU
+                                             : a.pro == PRO_SD_GEGLU && a.tab.gelu_f16;
+        if (gated) return launch_kernel<quant_rows_kernel<MODE, G, C, CLS_GATED>>(a, nw, lds, st);
+    }
+    return launch_kernel<quant_rows_kernel<MODE, G, C, CLS_REST>>(a, nw, lds, st);
 }
 
-// g: rotation group width (0, 64, 128, 256).  Picks waves per row so that a wave holds at most 4 chunks.
+template <int MODE, int G>
+int launch_c(const QuantArgs& a, int nw, int C, hipStream_t st) {
+    return C == 1 ? launch<MODE, G, 1>(a, nw, st) : launch<MODE, G, 2>(a, nw, st);
+}
+
+// g: rotation group width (0, 64, 128, 256).  A wave per chunk of 1024 values up to eight waves per row, two chunks per
+// wave beyond: short waves overlap their loads with each other's arithmetic, larger workgroups wait for their slowest wave.
+// Measured, us by the kernel trace: 4608 x 3072 one chunk per wave 14.2, two 15.8, three 16.1; GEGLU 8192 x 2560 48.8, 53.4,
+// 57.2; 2048 x 14336 fourteen waves 31.4, eight 25.9, four with four chunks each 27.7; SwiGLU 4608 x 12288 twelve waves
+// 86, eight 78.
 template <int MODE>
 int run_quant(QuantArgs a, int g, hipStream_t st) {
     if (a.M <= 0) return 0;
     const int nchunks = (a.K + kChunk - 1) / kChunk;
-    int wpr = 1;
-    while ((nchunks + wpr - 1) / wpr > 4) wpr *= 2;
-    if (wpr > 8) return -2;
-    // few rows: more waves per row (down to one chunk per wave) so that the launch has enough waves to hide latency
-    while (wpr < 8 && wpr < nchunks && (int64_t)a.M * wpr < 2048) wpr *= 2;
-    const int C = (nchunks + wpr - 1) / wpr;
-    const int nw = wpr < 2 ? 2 : wpr;   // two rows per workgroup at least: small workgroups spread evenly over the CUs
+    if (nchunks > 32) return -2;
+    const int C = nchunks > 8 ? 2 : 1, wpr = nchunks <= 8 ? nchunks : nchunks <= 16 ? 8 : (nchunks + 1) / 2;
+    const int nw = wpr < 2 ? 2 : wpr;   // two rows per workgroup at least
     a.wpr = wpr;
     a.rpb = nw / wpr;
     switch (g) {
@@ -458,11 +498,10 @@ int run_quant(QuantArgs a, int g, hipStream_t st) {
     }
 }
 
-// The activation tables, for the prologues that evaluate exp / erf / tanh on a 16-bit row.
+// The activation tables, for the prologues that evaluate erf / tanh on a 16-bit row.
 void attach_tables(QuantArgs& a, hipStream_t st) {
     const int p = a.pro;
-    if (p == PRO_GATE || p == PRO_SWIGLU || p == PRO_SITU || p == PRO_SITU_FAST || p == PRO_SILU || p == PRO_GELU || p == PRO_GELU_TANH ||
-        p == PRO_SD_GEGLU)
+    if (p == PRO_SITU || p == PRO_SITU_FAST || p == PRO_GELU || p == PRO_GELU_TANH || p == PRO_SD_GEGLU)
         if (const ActTables* t = act_tables(st)) a.tab = *t;
 }
 
