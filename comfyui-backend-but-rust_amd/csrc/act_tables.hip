@@ -20,6 +20,13 @@ __global__ void __launch_bounds__(256) fill_tables_kernel(uint16_t* h16, float* 
     h16[4 * 65536 + bits] = f_to_f16(gelu_f(h));
     f32[0 * 65536 + bits] = situ_gate_f(b);
     f32[1 * 65536 + bits] = situ_hidden_f(b);
+    if (bits <= (uint32_t)kGeluEnd) {
+        // the correctly rounded value where it satisfies both roundings, else the rounded negative side (282 of 17804: the
+        // definition's 1 + erf is an fp32 sum, coarse far out on the negative side); the GPU test goes through all of them
+        const uint16_t pos = f_to_f16(gelu_f(h)), neg = f_to_f16(gelu_f(-h));
+        const float g = (float)(-0.5 * (double)h * erfc((double)h * 0.70710678118654752440));
+        f32[2 * 65536 + bits] = f_to_f16(g) == neg && f_to_f16(h + g) == pos ? g : f16_to_f(neg);
+    }
 }
 
 constexpr int kMaxDevices = 16;
@@ -51,7 +58,7 @@ const ActTables* act_tables(hipStream_t stream) {
     uint16_t* h16 = nullptr;
     float* f32 = nullptr;
     if (hipMalloc(&h16, 5 * 65536 * sizeof(uint16_t)) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
-    if (hipMalloc(&f32, 2 * 65536 * sizeof(float)) != hipSuccess) {
+    if (hipMalloc(&f32, (2 * 65536 + kGeluEnd + 1) * sizeof(float)) != hipSuccess) {
         (void)hipGetLastError();
         (void)hipFree(h16);
         return nullptr;
@@ -71,7 +78,7 @@ const ActTables* act_tables(hipStream_t stream) {
         (void)hipFree(f32);
         return nullptr;
     }
-    g_tables[dev] = ActTables{h16, h16 + 65536, h16 + 2 * 65536, h16 + 3 * 65536, f32, f32 + 65536, h16 + 4 * 65536};
+    g_tables[dev] = ActTables{h16, h16 + 65536, h16 + 2 * 65536, h16 + 3 * 65536, f32, f32 + 65536, h16 + 4 * 65536, f32 + 2 * 65536};
     g_state[dev].store(1, std::memory_order_release);
     return &g_tables[dev];
 }

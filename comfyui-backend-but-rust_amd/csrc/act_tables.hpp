@@ -19,7 +19,12 @@ struct ActTables {
     const float* situ_hidden_bf16;
     // f16 input bits -> f16 bits of rnd(gelu(x))
     const uint16_t* gelu_f16;
+    // f16 magnitude bits a (x = the half they are) -> fp32 g with rnd(g) = rnd(gelu(-x)) and rnd(x + g) = rnd(gelu(x)), both
+    // rounded to f16: gelu(x) = x + gelu(-x), so one table of magnitudes serves both signs.  Entries 0..kGeluEnd; from
+    // kGeluEnd (5.54) on g rounds to zero and x + g to x.
+    const float* gelu_f16_g;
 };
+constexpr int kGeluEnd = 0x458b;
 
 // Tables of the current device, or nullptr if they are not built and cannot be built now (`stream` is being captured,
 // or an allocation failed: callers then evaluate per element, and a later call tries again).

@@ -40,6 +40,17 @@ inline int allow_dynamic_lds(const void* kern, int bytes, PerDeviceOnce& once) {
     return 0;
 }
 
+inline int device_cu_count() {
+    static std::atomic<int> cached[64];   // compute units per device ordinal, 0 = not asked yet
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 256;
+    const bool keep = dev >= 0 && dev < 64;
+    if (keep && (n = cached[dev].load(std::memory_order_relaxed)) > 0) return n;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 256;
+    if (keep) cached[dev].store(n, std::memory_order_relaxed);
+    return n;
+}
+
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 

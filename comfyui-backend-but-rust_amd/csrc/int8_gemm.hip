@@ -1425,17 +1425,6 @@ int launch_cfg(GemmArgs a, hipStream_t st) {
     return 0;
 }
 
-int device_cu_count() {
-    static std::atomic<int> cached[64];   // compute units per device ordinal, 0 = not asked yet
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 256;
-    const bool keep = dev >= 0 && dev < 64;
-    if (keep && (n = cached[dev].load(std::memory_order_relaxed)) > 0) return n;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 256;
-    if (keep) cached[dev].store(n, std::memory_order_relaxed);
-    return n;
-}
-
 // Launches the persistent ring kernel on `slices` K slices (1 = whole K).  With slices > 1, EPI must be EPI_ACC and
 // a.D the int32 planes.
 template <class C, int OUT_DT, int EPI>

@@ -113,6 +113,146 @@ __device__ __forceinline__ float rsqrt_cr(float a) {
     return (float)y;
 }
 
+// The rotation of a row's chunks and the maximum of their magnitudes over the lane's values.  `exact`: the values are bf16
+// or f16 numbers (rotate_chunk's condition for scaling once; bf16 ones are also checked against the overflow limit).
+template <int MODE, int G, int C>
+__device__ __forceinline__ float rotate_and_max(const QuantArgs& p, float (&v)[C][16], int64_t m, bool row_ok, int wr, int lane, float* wl, bool exact) {
+    float amax = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int e0 = (wr + c * p.wpr) * kChunk + lane * 16;
+        const bool act = row_ok && e0 < p.K;
+        if constexpr (G != 0) {
+            // scaled once where that is exact (rotate_chunk): f16 rows always, bf16 values below the overflow limit
+            bool once = G != 128 && MODE == MODE_SD_F16 && exact;
+            if (G != 128 && MODE == MODE_BF16 && exact) {
+                float big = 0.f;
+#pragma unroll
+                for (int i = 0; i < 16; i += 2) big = fmaxf(fmaxf(big, fabsf(v[c][i])), fabsf(v[c][i + 1]));
+                once = __builtin_amdgcn_ballot_w64(big >= kOnceLimit) == 0;
+            }
+            if (once) rotate_chunk<G, true>(v[c], wl, lane);
+            else rotate_chunk<G>(v[c], wl, lane);
+        }
+        if (MODE == MODE_ROT_F32) {
+            if (act) {
+                float4* o = reinterpret_cast<float4*>(p.out_f + m * (int64_t)p.K + e0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[i] = make_float4(v[c][4 * i], v[c][4 * i + 1], v[c][4 * i + 2], v[c][4 * i + 3]);
+            }
+        } else if (MODE == MODE_SD_F16) {
+            // the maximum is taken over the half-rounded row (csrc/sd.cu:587), which is also what is divided below
+#pragma unroll
+            for (int i = 0; i < 16; i += 2) {
+                unpack_f16x2(pack_f16x2(v[c][i], v[c][i + 1]), v[c][i], v[c][i + 1]);
+                amax = fmaxf(fmaxf(amax, fabsf(v[c][i])), fabsf(v[c][i + 1]));
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 16; i += 2) amax = fmaxf(fmaxf(amax, fabsf(v[c][i])), fabsf(v[c][i + 1]));
+        }
+    }
+    return amax;
+}
+
+// Scale and codes of a row whose maximum is `amax`.
+template <int MODE, int C, bool SR>
+__device__ __forceinline__ void store_codes(const QuantArgs& p, float (&v)[C][16], int64_t m, bool row_ok, int wr, int lane, float amax) {
+    float scale, st, rinv = 0.f;
+    bool by_rcp = true;   // f16 rows: st is a finite half
+    if (MODE == MODE_SD_F16) {
+        scale = fmaxf(amax, 1e-30f) / 127.f;                       // csrc/sd.cu:589
+        const float sh = rnd_dt<DT_F16>(scale);
+        st = sh > 0.f ? sh : scale;                                // :593
+        by_rcp = __builtin_amdgcn_ballot_w64(!(sh > 0.f && sh < __builtin_inff())) == 0;
+        rinv = __builtin_amdgcn_rcpf(st);
+    } else if (MODE == MODE_BF16) {
+        scale = fmaxf(fminf(amax, 3.38953139e38f) * (1.f / 127.f), 1.0e-30f);  // csrc/kernels.cu:241
+        st = rnd_dt<DT_BF16>(scale);
+        rinv = __builtin_amdgcn_rcpf(st);
+    } else {
+        scale = fmaxf(fminf(amax, 3.402823466e+38f) * (1.f / 127.f), 1.0e-30f);
+        st = scale;
+    }
+    if (row_ok && wr == 0 && lane == 0) p.scales[m] = scale;
+
+    const auto store = [&](auto rcp_tag) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int e0 = (wr + c * p.wpr) * kChunk + lane * 16;
+            if (!(row_ok && e0 < p.K)) continue;
+            uint32_t w[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if constexpr (MODE == MODE_SD_F16) {
+                    // t = half(x / st).  Both operands carry 11 significant bits: their quotient never equals a midpoint of two
+                    // halves and is 2^-23 (relative) away at least, more than the error left after one correction of x * rcp.
+                    // clamp(rint(t), -128, 127): a half around 1536 has a step of 1, so t + 1536 is 0x6600 + rint(t) and its
+                    // low byte the code; the maximum turns a NaN into the -128 that fminf(127, fmaxf(-128, NaN)) gives.
+                    float qt[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const float x = v[c][4 * i + j];
+                        if constexpr (decltype(rcp_tag)::value) {
+                            const float q0 = x * rinv;
+                            qt[j] = __builtin_fmaf(__builtin_fmaf(-q0, st, x), rinv, q0);
+                        } else {
+                            qt[j] = x / st;
+                        }
+                    }
+                    uint32_t h[2];
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        f16x2 t = __builtin_bit_cast(f16x2, pack_f16x2(qt[2 * j], qt[2 * j + 1]));
+                        t = __builtin_elementwise_min(__builtin_elementwise_max(t, f16x2{-128, -128}), f16x2{127, 127});
+                        h[j] = __builtin_bit_cast(uint32_t, t + f16x2{1536, 1536});
+                    }
+                    w[i] = __builtin_amdgcn_perm(h[1], h[0], 0x06040200u);
+                    continue;
+                }
+                uint32_t acc = 0;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float x = v[c][4 * i + j];
+                    float t;
+                    if (MODE == MODE_BF16) {
+                        // Both operands carry 8 significant bits, so their exact quotient is never closer than 2^-17
+                        // (relative) to a bf16 rounding boundary: a 1-ulp reciprocal times the numerator rounds to the
+                        // same bf16 value as the IEEE quotient does.
+                        t = rnd_dt<DT_BF16>(rnd_dt<DT_BF16>(x) * rinv);
+                    } else {
+                        t = x / st;
+                    }
+                    if (SR && (MODE == MODE_BF16 || MODE == MODE_F32)) {   // csrc/kernels.cu:1385-1388
+                        const uint64_t key = (uint64_t)(m * (int64_t)p.K + e0 + 4 * i + j) + p.seed;
+                        const float noise = (float)(pcg_hash((uint32_t)key ^ (uint32_t)(key >> 32)) >> 8) * 0x1.0p-24f;
+                        const float r = floorf(MODE == MODE_F32 ? t + noise : bf16_add_once(t, rnd_dt<DT_BF16>(noise)));
+                        const int qi = (int)fminf(127.f, fmaxf(-128.f, r));
+                        acc |= ((uint32_t)qi & 0xffu) << (8 * j);
+                    } else if (MODE == MODE_F32) {
+                        const int qi = (int)fminf(127.f, fmaxf(-128.f, nearbyintf(t)));
+                        acc |= ((uint32_t)qi & 0xffu) << (8 * j);
+                    } else {
+                        // clamp(rint(t), -128, 127) + 128 as one instruction: t is a 16-bit float, so t + 128 is exact
+                        // wherever t has a bit at 2^-16 or above set, and below that both t and t + 128 round to the
+                        // same integer; v_cvt_pk_u8_f32 rounds to nearest even, saturates to 0..255 (NaN to 0, which is
+                        // the -128 that fminf(127, fmaxf(-128, NaN)) gives) and drops the byte into place.
+                        acc = __builtin_amdgcn_cvt_pk_u8_f32(t + 128.f, j, acc);
+                    }
+                }
+                w[i] = (!SR && MODE != MODE_F32) ? acc ^ 0x80808080u : acc;
+            }
+            *reinterpret_cast<uint4*>(p.q + m * (int64_t)p.K + e0) = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+    };
+    if constexpr (MODE == MODE_SD_F16) {
+        if (by_rcp) store(std::true_type{});
+        else store(std::false_type{});
+    } else {
+        store(std::true_type{});
+    }
+}
+
 // CLS: the class of the row prologue (csrc/kernels.cu:88-182), which runs on the values as they are loaded, with the
 // reference's rounding points; p.pro selects the prologue within its class at run time.  Row sums are fp64, rounded once;
 // the activation functions are correctly rounded.  The classes keep what is cheap in registers apart from what calls
@@ -153,7 +293,6 @@ __global__ void __launch_bounds__(1024) quant_rows_kernel(QuantArgs p) {
     };
 
     float v[C][16];
-    float amax = 0.f;
     constexpr bool NORM = CLS == CLS_NORM, GATED = CLS == CLS_GATED, REST = CLS == CLS_REST;
     const int pro = CLS == CLS_PLAIN ? PRO_PLAIN : p.pro;
     const bool ln = NORM && (pro == PRO_LAYERNORM || pro == PRO_LN_MOD || pro == PRO_LN_AFFINE);
@@ -317,128 +456,133 @@ __global__ void __launch_bounds__(1024) quant_rows_kernel(QuantArgs p) {
             }
         }
     }
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-        const int e0 = (wr + c * p.wpr) * kChunk + lane * 16;
-        const bool act = row_ok && e0 < p.K;
-        if constexpr (G != 0) {
-            // scaled once where that is exact (rotate_chunk): f16 rows always, bf16 values below the overflow limit
-            bool once = G != 128 && MODE == MODE_SD_F16;
-            if (G != 128 && MODE == MODE_BF16 && (!REST || (pro != PRO_SITU && pro != PRO_SITU_FAST))) {
-                float big = 0.f;
-#pragma unroll
-                for (int i = 0; i < 16; i += 2) big = fmaxf(fmaxf(big, fabsf(v[c][i])), fabsf(v[c][i + 1]));
-                once = __builtin_amdgcn_ballot_w64(big >= kOnceLimit) == 0;
-            }
-            if (once) rotate_chunk<G, true>(v[c], wl, lane);
-            else rotate_chunk<G>(v[c], wl, lane);
+    const bool exact = !REST || (pro != PRO_SITU && pro != PRO_SITU_FAST);   // those hand on unrounded fp32 values
+    float amax = rotate_and_max<MODE, G, C>(p, v, m, row_ok, wr, lane, wl, exact);
+    if constexpr (MODE != MODE_ROT_F32) {
+        amax = wave_max_f32(amax);
+        if (p.wpr > 1) {  // uniform over the block
+            if (lane == 0) red[wave] = amax;
+            __syncthreads();
+            amax = 0.f;
+            for (int i = 0; i < p.wpr; ++i) amax = fmaxf(amax, red[rloc * p.wpr + i]);
         }
-        if (MODE == MODE_ROT_F32) {
-            if (act) {
-                float4* o = reinterpret_cast<float4*>(p.out_f + m * (int64_t)p.K + e0);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) o[i] = make_float4(v[c][4 * i], v[c][4 * i + 1], v[c][4 * i + 2], v[c][4 * i + 3]);
-            }
-        } else if (MODE == MODE_SD_F16) {
-            // the maximum is taken over the half-rounded row (csrc/sd.cu:587), which is also what is divided below
-#pragma unroll
-            for (int i = 0; i < 16; i += 2) {
-                unpack_f16x2(pack_f16x2(v[c][i], v[c][i + 1]), v[c][i], v[c][i + 1]);
-                amax = fmaxf(fmaxf(amax, fabsf(v[c][i])), fabsf(v[c][i + 1]));
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 16; i += 2) amax = fmaxf(fmaxf(amax, fabsf(v[c][i])), fabsf(v[c][i + 1]));
-        }
+        store_codes<MODE, C, SR>(p, v, m, row_ok, wr, lane, amax);
     }
-    if (MODE == MODE_ROT_F32) return;
+}
 
-    amax = wave_max_f32(amax);
-    if (p.wpr > 1) {  // uniform over the block
-        if (lane == 0) red[wave] = amax;
-        __syncthreads();
-        amax = 0.f;
-        for (int i = 0; i < p.wpr; ++i) amax = fmaxf(amax, red[rloc * p.wpr + i]);
-    }
+// GEGLU of f16 rows ahead of the quantizer (csrc/sd.cu:642-649, row = [value | gate]), one workgroup of 16 waves per CU that
+// walks the rows with the table of gelu in its LDS.  Read per lane from the 128 KB table in global memory the activation costs
+// the CU's address path a cycle per lane (8192 x 2560: 48.8 us on a GEMM's output); from the LDS the 64 lanes of a read
+// spread over the 64 banks.  71 KB of magnitudes serve both signs (act_tables.hpp).
+// C == 1: a wave per chunk, the next row's loads issued before this row's arithmetic, one barrier per row (33 us).  C == 2, 3:
+// a wave per row, no barrier, the waves' loads and arithmetic drift apart by themselves (28 us), for rows of that many
+// chunks where the rows divide well over the waves.  About 1500 cycles of vector instructions per chunk make 16 us of
+// that; the traffic alone is 20.
+// Two gates (packed f16) and their table entries -> rnd(gelu) of both, packed: max(x, 0) + g, the first as half of x + |x| so
+// that a NaN and -inf (gelu: NaN) stay what they are.
+__device__ __forceinline__ uint32_t gelu_index_x2(uint32_t gw) {   // the entries' indices, packed
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, gw & 0x7fff7fffu), u16x2{kGeluEnd, kGeluEnd}));
+}
+__device__ __forceinline__ uint32_t gelu_f16x2(uint32_t gw, float t0, float t1) {
+    float g0, g1;
+    unpack_f16x2(gw, g0, g1);
+    return pack_f16x2(__builtin_fmaf(g0 + fabsf(g0), 0.5f, t0), __builtin_fmaf(g1 + fabsf(g1), 0.5f, t1));
+}
 
-    float scale, st, rinv = 0.f;
-    bool by_rcp = true;   // f16 rows: st is a finite half
-    if (MODE == MODE_SD_F16) {
-        scale = fmaxf(amax, 1e-30f) / 127.f;                       // csrc/sd.cu:589
-        const float sh = rnd_dt<DT_F16>(scale);
-        st = sh > 0.f ? sh : scale;                                // :593
-        by_rcp = __builtin_amdgcn_ballot_w64(!(sh > 0.f && sh < __builtin_inff())) == 0;
-        rinv = __builtin_amdgcn_rcpf(st);
-    } else if (MODE == MODE_BF16) {
-        scale = fmaxf(fminf(amax, 3.38953139e38f) * (1.f / 127.f), 1.0e-30f);  // csrc/kernels.cu:241
-        st = rnd_dt<DT_BF16>(scale);
-        rinv = __builtin_amdgcn_rcpf(st);
-    } else {
-        scale = fmaxf(fminf(amax, 3.402823466e+38f) * (1.f / 127.f), 1.0e-30f);
-        st = scale;
-    }
-    if (row_ok && wr == 0 && lane == 0) p.scales[m] = scale;
-
-    const auto store = [&](auto rcp_tag) {
+constexpr int kGegluWaves = 16;
+constexpr int kGegluTable = (kGeluEnd + 4) / 4 * 4;   // floats
+template <int G, int C>
+__global__ void __launch_bounds__(kGegluWaves * 64) geglu_rows_kernel(QuantArgs p) {
+    constexpr bool PF = C == 1;
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    __shared__ float red[2][kGegluWaves];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int rloc = wave / p.wpr, wr = wave - rloc * p.wpr;
+    const int row0 = (rloc < p.rpb ? rloc : 0) * p.wpr;   // the row's first wave; waves past the last row read along
+    float* wl = lds + kGegluTable + wave * kLdsPerWave;
+    for (int i = threadIdx.x * 4; i <= kGeluEnd; i += kGegluWaves * 64 * 4)   // the table is padded to whole vectors
+        *reinterpret_cast<float4*>(lds + i) = *reinterpret_cast<const float4*>(p.tab.gelu_f16_g + i);
+    uint4 x[C][2], g[C][2];
+    const auto load = [&](int64_t m) {
 #pragma unroll
         for (int c = 0; c < C; ++c) {
             const int e0 = (wr + c * p.wpr) * kChunk + lane * 16;
-            if (!(row_ok && e0 < p.K)) continue;
-            uint32_t w[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                uint32_t acc = 0;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float x = v[c][4 * i + j];
-                    float t;
-                    if (MODE == MODE_BF16) {
-                        // Both operands carry 8 significant bits, so their exact quotient is never closer than 2^-17
-                        // (relative) to a bf16 rounding boundary: a 1-ulp reciprocal times the numerator rounds to the
-                        // same bf16 value as the IEEE quotient does.
-                        t = rnd_dt<DT_BF16>(rnd_dt<DT_BF16>(x) * rinv);
-                    } else if (MODE == MODE_SD_F16) {
-                        // Both operands carry 11 significant bits: their quotient never equals a midpoint of two halves and
-                        // is 2^-23 (relative) away at least, more than the error left after one correction of x * rcp.
-                        float qt;
-                        if constexpr (decltype(rcp_tag)::value) {
-                            const float q0 = x * rinv;
-                            qt = __builtin_fmaf(__builtin_fmaf(-q0, st, x), rinv, q0);
-                        } else {
-                            qt = x / st;
-                        }
-                        t = rnd_dt<DT_F16>(qt);
-                    } else {
-                        t = x / st;
-                    }
-                    if (SR && (MODE == MODE_BF16 || MODE == MODE_F32)) {   // csrc/kernels.cu:1385-1388
-                        const uint64_t key = (uint64_t)(m * (int64_t)p.K + e0 + 4 * i + j) + p.seed;
-                        const float noise = (float)(pcg_hash((uint32_t)key ^ (uint32_t)(key >> 32)) >> 8) * 0x1.0p-24f;
-                        const float r = floorf(MODE == MODE_F32 ? t + noise : bf16_add_once(t, rnd_dt<DT_BF16>(noise)));
-                        const int qi = (int)fminf(127.f, fmaxf(-128.f, r));
-                        acc |= ((uint32_t)qi & 0xffu) << (8 * j);
-                    } else if (MODE == MODE_F32) {
-                        const int qi = (int)fminf(127.f, fmaxf(-128.f, nearbyintf(t)));
-                        acc |= ((uint32_t)qi & 0xffu) << (8 * j);
-                    } else {
-                        // clamp(rint(t), -128, 127) + 128 as one instruction: t is a 16-bit float, so t + 128 is exact
-                        // wherever t has a bit at 2^-16 or above set, and below that both t and t + 128 round to the
-                        // same integer; v_cvt_pk_u8_f32 rounds to nearest even, saturates to 0..255 (NaN to 0, which is
-                        // the -128 that fminf(127, fmaxf(-128, NaN)) gives) and drops the byte into place.
-                        acc = __builtin_amdgcn_cvt_pk_u8_f32(t + 128.f, j, acc);
-                    }
-                }
-                w[i] = (!SR && MODE != MODE_F32) ? acc ^ 0x80808080u : acc;
+            if (rloc < p.rpb && m < p.M && e0 < p.K) {
+                const uint4* s = reinterpret_cast<const uint4*>((const uint16_t*)p.x + m * p.x_stride + e0);
+                const uint4* t = reinterpret_cast<const uint4*>((const uint16_t*)p.x + m * p.x_stride + p.up_offset + e0);
+                x[c][0] = s[0]; x[c][1] = s[1];
+                g[c][0] = t[0]; g[c][1] = t[1];
+            } else {
+                x[c][0] = x[c][1] = g[c][0] = g[c][1] = make_uint4(0u, 0u, 0u, 0u);
             }
-            *reinterpret_cast<uint4*>(p.q + m * (int64_t)p.K + e0) = make_uint4(w[0], w[1], w[2], w[3]);
         }
     };
-    if constexpr (MODE == MODE_SD_F16) {
-        if (by_rcp) store(std::true_type{});
-        else store(std::false_type{});
-    } else {
-        store(std::true_type{});
+    int64_t m = (int64_t)blockIdx.x * p.rpb + rloc;
+    if (PF) load(m);
+    __syncthreads();
+    const int64_t step = (int64_t)gridDim.x * p.rpb, first = m;
+    for (int it = 0; (int64_t)blockIdx.x * p.rpb + it * step < p.M; ++it) {   // the same count in every wave
+        m = first + it * step;
+        const bool row_ok = rloc < p.rpb && m < p.M;
+        if (!PF) load(m);
+        float v[C][16];
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const uint32_t gw[8] = {g[c][0].x, g[c][0].y, g[c][0].z, g[c][0].w, g[c][1].x, g[c][1].y, g[c][1].z, g[c][1].w};
+            const uint32_t xw[8] = {x[c][0].x, x[c][0].y, x[c][0].z, x[c][0].w, x[c][1].x, x[c][1].y, x[c][1].z, x[c][1].w};
+            float t[16];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t a = gelu_index_x2(gw[i]);
+                t[2 * i] = lds[a & 0xffffu];
+                t[2 * i + 1] = lds[a >> 16];
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t act = gelu_f16x2(gw[i], t[2 * i], t[2 * i + 1]);
+                // the product of two halves is exact in fp32, so the packed f16 product is its one rounding
+                const f16x2 pr = __builtin_bit_cast(f16x2, xw[i]) * __builtin_bit_cast(f16x2, act);
+                v[c][2 * i] = (float)pr[0];
+                v[c][2 * i + 1] = (float)pr[1];
+            }
+        }
+        if (PF) load(m + step);
+        float amax = wave_max_f32(rotate_and_max<MODE_SD_F16, G, C>(p, v, m, row_ok, wr, lane, wl, true));
+        if (p.wpr > 1) {   // uniform over the workgroup; the slots alternate, so one barrier per row is enough
+            float* r = red[it & 1];
+            if (lane == 0) r[wave] = amax;
+            __syncthreads();
+            amax = 0.f;
+            for (int i = 0; i < p.wpr; ++i) amax = fmaxf(amax, r[row0 + i]);
+        }
+        store_codes<MODE_SD_F16, C, false>(p, v, m, row_ok, wr, lane, amax);
     }
+}
+
+template <int G, int C>
+int launch_geglu(QuantArgs a, int wpr, int cus, hipStream_t st) {
+    constexpr int lds = (kGegluTable + (G ? kGegluWaves * kLdsPerWave : 0)) * (int)sizeof(float);
+    static PerDeviceOnce once;
+    if (const int e = allow_dynamic_lds(reinterpret_cast<const void*>(geglu_rows_kernel<G, C>), lds, once)) return e;
+    a.wpr = wpr;
+    a.rpb = kGegluWaves / wpr;
+    const int groups = (a.M + a.rpb - 1) / a.rpb;
+    hipLaunchKernelGGL((geglu_rows_kernel<G, C>), dim3(groups < cus ? groups : cus), dim3(kGegluWaves * 64), lds, st, a);
+    KCHECK();
+    return 0;
+}
+
+// GEGLU with the table in LDS.  A round of the wave-per-row form takes about 3.3 us per chunk of its rows and 4 us of the
+// launch's start more than the other form, whose rounds take 4.1 us.
+template <int G>
+int run_geglu(const QuantArgs& a, int nchunks, hipStream_t st) {
+    const int cus = device_cu_count();
+    if (nchunks > kGegluWaves) return launch_geglu<G, 2>(a, (nchunks + 1) / 2, cus, st);
+    const auto rounds = [&](int rpb) { return (a.M + (int64_t)rpb * cus - 1) / ((int64_t)rpb * cus); };
+    if (nchunks <= 3 && 3.3 * nchunks * rounds(kGegluWaves) + 4. < 4.1 * rounds(kGegluWaves / nchunks))
+        return nchunks == 3 ? launch_geglu<G, 3>(a, 1, cus, st) : nchunks == 2 ? launch_geglu<G, 2>(a, 1, cus, st) : launch_geglu<G, 1>(a, 1, cus, st);
+    return launch_geglu<G, 1>(a, nchunks, cus, st);
 }
 
 template <auto KERN>
@@ -466,6 +610,12 @@ int launch(const QuantArgs& a, int nw, hipStream_t st) {
     if constexpr (MODE == MODE_BF16 || MODE == MODE_SD_F16) {
         const bool gated = MODE == MODE_BF16 ? a.pro == PRO_GATE || a.pro == PRO_SWIGLU || a.pro == PRO_SILU
                                              : a.pro == PRO_SD_GEGLU && a.tab.gelu_f16;
+        if constexpr (MODE == MODE_SD_F16) {
+            // filling the table takes a workgroup 2.5 us: it pays from about 5000 chunks on (1024 x 5120: 13.0 us either way;
+            // 2048 x 5120 18.4 against 21.4, 512 x 2560 7.4 against 5.9)
+            const int nchunks = (a.K + kChunk - 1) / kChunk;
+            if (gated && (int64_t)a.M * nchunks >= 5120) return run_geglu<G>(a, nchunks, st);
+        }
         if (gated) return launch_kernel<quant_rows_kernel<MODE, G, C, CLS_GATED>>(a, nw, lds, st);
     }
     return launch_kernel<quant_rows_kernel<MODE, G, C, CLS_REST>>(a, nw, lds, st);
@@ -610,19 +760,27 @@ GPU_API int gpu_convrot_requant(int dtype, const void* x, void* q, void* s, int6
     return dtype == DT_F32 ? run_quant<MODE_F32>(a, 256, (hipStream_t)stream) : run_quant<MODE_BF16>(a, 256, (hipStream_t)stream);
 }
 
-// Test hook: out[i] = bf16 bits of sigmoid (which 0) or silu (1) of the bf16 bits in[i], as the prologues evaluate them.
+// Test hook: out[i] = bf16 bits of sigmoid (which 0) or silu (1) of the bf16 bits in[i], or f16 bits of gelu (2) of the f16
+// bits in[i], as the prologues evaluate them.
 namespace {
-__global__ void __launch_bounds__(256) act_probe_kernel(int which, const uint16_t* in, uint16_t* out, int n) {
+__global__ void __launch_bounds__(256) act_probe_kernel(int which, const uint16_t* in, uint16_t* out, int n, const float* gelu) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
+    if (which == 2) {
+        const uint32_t a = gelu_index_x2(in[i]);
+        out[i] = (uint16_t)gelu_f16x2(in[i], gelu[a & 0xffffu], 0.f);
+        return;
+    }
     const float x = bf16_to_f(in[i]);
     out[i] = f_to_bf16(which == 0 ? sigmoid_of_bf16(x) : silu_of_bf16(x));
 }
 }  // namespace
 GPU_API int gpu_internal_act_probe(int which, const void* in, void* out, int n, void* stream) {
-    if (which < 0 || which > 1 || !in || !out || n <= 0) return -1;
+    if (which < 0 || which > 2 || !in || !out || n <= 0) return -1;
+    const ActTables* t = which == 2 ? act_tables((hipStream_t)stream) : nullptr;
+    if (which == 2 && !t) return -1;
     hipLaunchKernelGGL(act_probe_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, which, (const uint16_t*)in,
-                       (uint16_t*)out, n);
+                       (uint16_t*)out, n, t ? t->gelu_f16_g : nullptr);
     KCHECK();
     return 0;
 }

@@ -174,8 +174,8 @@ int gpu_int8_attn_key_bias(const void* q, const void* k, const void* v, void* o,
                            int64_t v_bs, int64_t v_rs, int64_t v_hs, int64_t o_bs, int64_t o_rs, int64_t o_hs, float scale,
                            const float* bias, void* stream);
 
-/* Test hook, no reference counterpart: out[i] = bf16 sigmoid (which 0) or silu (1) of the bf16 bits in[i], evaluated as the
- * quantizer's prologues evaluate it. */
+/* Test hook, no reference counterpart: out[i] = bf16 sigmoid (which 0) or silu (1) of the bf16 bits in[i], or f16 gelu (2) of
+ * the f16 bits in[i], evaluated as the quantizer's prologues evaluate it. */
 int gpu_internal_act_probe(int which, const void* in, void* out, int n, void* stream);
 
 /* Test hook, no reference counterpart: y[i] = the gfx950 float -> u8 pack conversion of x[i] (byte 0), which the attention

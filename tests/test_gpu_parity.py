@@ -292,6 +292,43 @@ def test_sigmoid_and_silu_of_every_bf16_value():
         assert bad.size == 0, [(hex(int(b)), hex(int(got[b])), hex(int(want[0][b]))) for b in bad[:20]]
 
 
+def test_gelu_of_every_f16_value():
+    """GEGLU's activation through its table of magnitudes: all 65536 gates against the oracle (a value of 1 beside each)."""
+    bits = np.arange(65536, dtype=np.uint16)
+    row = np.concatenate([np.full(65536, 0x3C00, np.uint16), bits]).reshape(1, -1)
+    rc, want = oracle.sd_source_rows(oracle.SD_GEGLU, row, 1, 65536)
+    assert rc == 0
+    out = torch.zeros(65536, dtype=torch.int16, device=DEV)
+    ffi.k("gpu_internal_act_probe", 2, dev(bits.view(np.int16)).data_ptr(), out.data_ptr(), 65536, 0)
+    torch.cuda.synchronize()
+    got, want = out.cpu().numpy().view(np.uint16), want[0]
+    nan = (want & 0x7FFF) > 0x7C00
+    zero = (want & 0x7FFF) == 0
+    assert np.array_equal(nan, (got & 0x7FFF) > 0x7C00) and ((got[zero] & 0x7FFF) == 0).all()   # a zero's sign is not kept
+    bad = np.nonzero((got != want) & ~nan & ~zero)[0]
+    assert bad.size == 0, [(hex(int(b)), hex(int(got[b])), hex(int(want[b]))) for b in bad[:20]]
+
+
+@pytest.mark.parametrize("rotate", [0, 64, 256])
+@pytest.mark.parametrize("M,K", [(5121, 256), (2561, 1280), (16385, 1280), (8190, 2560), (1100, 5120), (303, 16640)])
+def test_geglu_table_kernel_forms(M, K, rotate):
+    """Row counts at which the kernel with the table in LDS runs, in each of its forms (a wave per chunk with and without idle
+    waves, a wave per row of two and three chunks, two chunks per wave): the first, last and some other rows bit-exact."""
+    say("geglu", M, K, rotate)
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    x = (torch.randn(M, 2 * K, device=DEV, generator=g) * 2).half()
+    x[0, K] = float("nan"); x[M - 1, K + 3] = float("-inf"); x[M - 1, 2 * K - 1] = float("inf")
+    rows = torch.unique(torch.cat([torch.arange(4), torch.arange(M - 4, M), torch.randint(0, M, (24,), generator=torch.Generator().manual_seed(K))])).to(DEV)
+    xb = host_bits(x[rows].contiguous())
+    rc, src = oracle.sd_source_rows(oracle.SD_GEGLU, xb, len(rows), K)
+    rc2, q, s = oracle.sd_quant_rows(src, K, rotate)
+    qd, sd = ql.sd_geglu_quant_rows(x, rotate)
+    torch.cuda.synchronize()
+    assert rc == 0 and rc2 == 0
+    assert np.array_equal(sd[rows].cpu().numpy().view(np.uint32), s.view(np.uint32))
+    assert np.array_equal(qd[rows].cpu().numpy(), q)
+
+
 @pytest.mark.parametrize("rotate", [64, 256])
 @pytest.mark.parametrize("M,K", [(4, 256), (3, 1280), (2, 5120)])
 def test_rotation_scaled_once_and_per_stage(M, K, rotate):
