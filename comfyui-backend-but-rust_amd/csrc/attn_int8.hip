@@ -37,7 +37,7 @@ struct AttnArgs {
     int b, lq, lk, h, hk, rep, qg, kb, ck, nblk;
     int64_t q_bs, q_rs, q_hs, k_bs, k_rs, k_hs, v_bs, v_rs, v_hs, o_bs, o_rs, o_hs;
     float sm, sink;
-    int vec_ok, in_vec, v_vec, use_anchor;
+    int vec_ok, in_vec, v_vec, nr_vec, use_anchor;   // nr_vec: qw, kw and rope are 16-byte aligned
     int rot4;   // lk <= 256: the rotation is only the H4 on runs of four channels, without the sign diagonal
     // per-head RMSNorm (+ weight) and RoPE ahead of the quantizers (csrc/kernels.cu:482-540 through
     // csrc/vendor/sage/quant_qk_int8.cu:160-291): q_norm / k_norm say which of Q and K take it
@@ -58,18 +58,20 @@ __device__ __forceinline__ int8_t rn_s8(float v) {
     return (int8_t)(r > 127.f ? 127.f : r < -128.f ? -128.f : r);
 }
 
-// Cross-lane moves inside a run of eight lanes, as data-parallel-primitive modifiers (no LDS traffic).
+// Cross-lane moves inside a row's lanes, as data-parallel-primitive modifiers (no LDS traffic).  A row's 16-channel blocks lie
+// on its lanes so that each move of a block bit is one such modifier: blocks 4..7 of eight run backwards, which makes
+// block ^ 4 the mirror of the eight lanes.
 template <int CTRL> __device__ __forceinline__ float dpp_mov(float x) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, false));
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
 }
-__device__ __forceinline__ float lane_xor1(float x) { return dpp_mov<0xB1>(x); }                   // quad_perm [1,0,3,2]
-__device__ __forceinline__ float lane_xor2(float x) { return dpp_mov<0x4E>(x); }                   // quad_perm [2,3,0,1]
-__device__ __forceinline__ float lane_xor4(float x) { return dpp_mov<0x1B>(dpp_mov<0x141>(x)); }   // half-row mirror (xor 7), then quad reverse (xor 3)
-
-__device__ __forceinline__ float lane_xor8(float x) { return dpp_mov<0x128>(x); }                  // row_ror:8 within a row of 16 lanes
+template <int D> __device__ __forceinline__ int block_of_lane(int lane) { return D == 64 || !(lane & 4) ? lane : lane ^ 3; }   // within the row
+__device__ __forceinline__ float block_xor1(float x) { return dpp_mov<0xB1>(x); }    // quad_perm [1,0,3,2]
+__device__ __forceinline__ float block_xor2(float x) { return dpp_mov<0x4E>(x); }    // quad_perm [2,3,0,1]
+__device__ __forceinline__ float block_xor4(float x) { return dpp_mov<0x141>(x); }   // half-row mirror
+__device__ __forceinline__ float block_xor8(float x) { return dpp_mov<0x128>(x); }   // row_ror:8 within a row of 16 lanes
 
 // Normalized Walsh-Hadamard over the 16 << LB channels of one row held by 1 << LB consecutive lanes, sixteen adjacent
-// channels per lane (ol = lane within the run), after the sign diagonal when SIGN (head dim 128 only).  Same operation
+// channels per lane (ol = the lane's block), after the sign diagonal when SIGN (head dim 128 only).  Same operation
 // order as the oracle: H4 on runs of four channels, radix-2 butterflies over the higher channel bits in ascending order
 // (two in the lane, LB across lanes), one scaling.  LB = 3: H128 (the reference's convrot128 / convrot128_plain), LB = 2:
 // H64 (convrot64).
@@ -97,22 +99,15 @@ template <int LB, bool SIGN> __device__ __forceinline__ void rot_wh(float (&v)[1
                 v[e] = lo + hi;
                 v[e | bit] = lo - hi;
             }
+    // other - v in the upper block of a pair, v + other in the lower: one fma on an exact product by -1 or 1
+    const float s1 = ol & 1 ? -1.f : 1.f, s2 = ol & 2 ? -1.f : 1.f, s4 = ol & 4 ? -1.f : 1.f;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        const float other = lane_xor1(v[e]);
-        v[e] = (ol & 1) ? other - v[e] : v[e] + other;
-    }
+    for (int e = 0; e < 16; ++e) v[e] = __builtin_fmaf(v[e], s1, block_xor1(v[e]));
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        const float other = lane_xor2(v[e]);
-        v[e] = (ol & 2) ? other - v[e] : v[e] + other;
-    }
+    for (int e = 0; e < 16; ++e) v[e] = __builtin_fmaf(v[e], s2, block_xor2(v[e]));
     if (LB == 3) {
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const float other = lane_xor4(v[e]);
-            v[e] = (ol & 4) ? other - v[e] : v[e] + other;
-        }
+        for (int e = 0; e < 16; ++e) v[e] = __builtin_fmaf(v[e], s4, block_xor4(v[e]));
     }
 #pragma unroll
     for (int e = 0; e < 16; ++e) v[e] *= LB == 3 ? 0.1767766952966369f : 0.25f;
@@ -142,17 +137,17 @@ template <int D> __device__ __forceinline__ void rotate_row(float (&v)[16], int 
 
 // Maximum over the lanes of a row.
 template <int D> __device__ __forceinline__ float max_row(float m) {
-    m = fmax_nn(m, lane_xor1(m));
-    m = fmax_nn(m, lane_xor2(m));
-    if (D >= 128) m = fmax_nn(m, lane_xor4(m));
-    if (D == 256) m = fmax_nn(m, lane_xor8(m));
+    m = fmax_nn(m, block_xor1(m));
+    m = fmax_nn(m, block_xor2(m));
+    if (D >= 128) m = fmax_nn(m, block_xor4(m));
+    if (D == 256) m = fmax_nn(m, block_xor8(m));
     return m;
 }
 
 // Sum of squares of one 128-channel row in the order of the reference's warp of 32 lanes (csrc/kernels.cu:497-513,
 // csrc/common.cuh:30-34): lane L accumulates its four channels by fma in index order, then the lanes add pairwise at
 // distances 16, 8, 4, 2, 1.  Lane L owns channels 4L..4L+3, or, with split = rope_mode 2 (with or without a table),
-// channels 2L, 2L+1, 64+2L, 65+2L.  Here eight lanes hold sixteen adjacent channels each (o8 = lane within the eight),
+// channels 2L, 2L+1, 64+2L, 65+2L.  Here eight lanes hold sixteen adjacent channels each (o8 = the lane's block),
 // so a lane carries four (eight, split) of the reference's lanes; all eight lanes get the sum.
 __device__ __forceinline__ float sumsq128(const float (&v)[16], int o8, bool split) {
     if (!split) {
@@ -165,11 +160,11 @@ __device__ __forceinline__ float sumsq128(const float (&v)[16], int o8, bool spl
             s[i] = __builtin_fmaf(v[4 * i + 3], v[4 * i + 3], s[i]);
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s[i] += lane_xor4(s[i]);   // distance 16
+        for (int i = 0; i < 4; ++i) s[i] += block_xor4(s[i]);   // distance 16
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s[i] += lane_xor2(s[i]);   // 8
+        for (int i = 0; i < 4; ++i) s[i] += block_xor2(s[i]);   // 8
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s[i] += lane_xor1(s[i]);   // 4
+        for (int i = 0; i < 4; ++i) s[i] += block_xor1(s[i]);   // 4
         return (s[0] + s[2]) + (s[1] + s[3]);                   // 2, then 1
     }
     // split: the lanes of the low half start each chain (channels 2L, 2L+1), the lanes of the high half finish it
@@ -177,15 +172,15 @@ __device__ __forceinline__ float sumsq128(const float (&v)[16], int o8, bool spl
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const float p = __builtin_fmaf(v[2 * i + 1], v[2 * i + 1], v[2 * i] * v[2 * i]);
-        const float q = lane_xor4(p);
+        const float q = block_xor4(p);
         s[i] = __builtin_fmaf(v[2 * i + 1], v[2 * i + 1], __builtin_fmaf(v[2 * i], v[2 * i], q));   // meaningful where o8 >= 4
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) s[i] += lane_xor2(s[i]);       // distance 16
+    for (int i = 0; i < 8; ++i) s[i] += block_xor2(s[i]);       // distance 16
 #pragma unroll
-    for (int i = 0; i < 8; ++i) s[i] += lane_xor1(s[i]);       // 8
+    for (int i = 0; i < 8; ++i) s[i] += block_xor1(s[i]);       // 8
     const float t = ((s[0] + s[4]) + (s[2] + s[6])) + ((s[1] + s[5]) + (s[3] + s[7]));   // 4, 2, 1
-    const float u = lane_xor4(t);
+    const float u = block_xor4(t);
     return o8 >= 4 ? t : u;
 }
 
@@ -204,6 +199,12 @@ __device__ inline float sumsq128_serial(const float* x, bool split) {
     return s[0];
 }
 
+__device__ __forceinline__ void round_bf16x2(float& x, float& y) {
+    const uint32_t u = pack_bf16x2(x, y);
+    x = u2f(u << 16);
+    y = u2f(u & 0xffff0000u);
+}
+
 // Per-head RMSNorm, weight and RoPE of one 128-channel row held by eight lanes (sixteen adjacent channels each), as the
 // reference applies them to q and k ahead of the quantizer (csrc/kernels.cu:482-540, csrc/vendor/sage/quant_qk_int8.cu:
 // 211-278): v = T((v * rstd) * w), rstd = 1/sqrt(mean(v^2) + eps) with the sum in the reference's order (sumsq128);
@@ -212,35 +213,95 @@ __device__ inline float sumsq128_serial(const float* x, bool split) {
 // 1/sqrt is correctly rounded (the reference's rsqrtf is an approximation of up to two units in the last place), and
 // c*a - s*b, s*a + c*b contract to one fma each on their first product.  w == nullptr means ones; rope_row == nullptr
 // means no rotation.  All eight lanes must call it.
-__device__ __forceinline__ void norm_rope_row(float (&v)[16], int o8, const float* w, const float* rope_row, float eps, int mode) {
-    const float ss = sumsq128(v, o8, mode == 2);
-    const float rstd = (float)(1.0 / sqrt((double)(ss / 128.f + eps)));
+// The caller has loaded the lane's weights (ones for a null w) and, unless rope_mode is 0, its pairs of (cos, sin): rope_mode 1
+// those of its own channel pairs, 2 those of channels (block & 3) * 16 .. + 15, thirty-two floats.
+__device__ __forceinline__ void norm_row(float (&v)[16], int o8, const float (&w)[16], float eps, bool split) {
+    const float rstd = rsqrt_cr(sumsq128(v, o8, split) / 128.f + eps);
 #pragma unroll
-    for (int e = 0; e < 16; ++e) v[e] = rnd_dt<DT_BF16>(v[e] * rstd * (w ? w[o8 * 16 + e] : 1.f));
-    if (!rope_row) return;
-    if (mode == 1) {
+    for (int e = 0; e < 16; e += 2) {
+        v[e] = v[e] * rstd * w[e];
+        v[e + 1] = v[e + 1] * rstd * w[e + 1];
+        round_bf16x2(v[e], v[e + 1]);
+    }
+}
+__device__ __forceinline__ void rope_pairs(float (&v)[16], const float (&cs)[16]) {
 #pragma unroll
-        for (int e = 0; e < 16; e += 2) {
-            const float c = rope_row[o8 * 16 + e], sn = rope_row[o8 * 16 + e + 1];
-            const float a = v[e], b = v[e + 1];
-            v[e] = rnd_dt<DT_BF16>(__builtin_fmaf(c, a, -(sn * b)));
-            v[e + 1] = rnd_dt<DT_BF16>(__builtin_fmaf(sn, a, c * b));
+    for (int e = 0; e < 16; e += 2) {
+        const float a = v[e], b = v[e + 1];
+        v[e] = __builtin_fmaf(cs[e], a, -(cs[e + 1] * b));
+        v[e + 1] = __builtin_fmaf(cs[e + 1], a, cs[e] * b);
+        round_bf16x2(v[e], v[e + 1]);
+    }
+}
+__device__ __forceinline__ void rope_halves(float (&v)[16], int o8, const float* r) {
+    const float sgn = o8 < 4 ? -1.f : 1.f;
+#pragma unroll
+    for (int e = 0; e < 16; e += 2) {
+        v[e] = __builtin_fmaf(v[e], r[2 * e], sgn * (block_xor4(v[e]) * r[2 * e + 1]));
+        v[e + 1] = __builtin_fmaf(v[e + 1], r[2 * e + 2], sgn * (block_xor4(v[e + 1]) * r[2 * e + 3]));
+        round_bf16x2(v[e], v[e + 1]);
+    }
+}
+__device__ __forceinline__ void load16_f32(const float* p, float (&v)[16]) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        const float4 f = reinterpret_cast<const float4*>(p)[g];
+        v[4 * g] = f.x; v[4 * g + 1] = f.y; v[4 * g + 2] = f.z; v[4 * g + 3] = f.w;
+    }
+}
+// What the quantizer kernels are instantiated for: no norm; norm with 16-byte aligned tables and rope by pairs or none; any
+// other.  The first two do without the registers of what follows them.
+enum { NORM_NONE, NORM_PAIRS, NORM_ANY };
+// N rows at once, so that their tables are all in flight before the first is used: row_of(j) is row j's position.
+template <int NM, int N, class RowOf>
+__device__ __forceinline__ void norm_rope_rows(float (&v)[N][16], int o8, const float* w, const float* rope, float eps, int mode, RowOf row_of) {
+    float wv[16];
+    if (NM == NORM_PAIRS && w) {
+        load16_f32(w + o8 * 16, wv);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) wv[e] = NM == NORM_ANY && w ? w[o8 * 16 + e] : 1.f;
+    }
+    if constexpr (NM == NORM_PAIRS) {
+        float cs[N][16];
+        if (rope) {
+#pragma unroll
+            for (int j = 0; j < N; ++j) load16_f32(rope + (int64_t)row_of(j) * 128 + o8 * 16, cs[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            norm_row(v[j], o8, wv, eps, false);
+            if (rope) rope_pairs(v[j], cs[j]);
         }
     } else {
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int j = (o8 & 3) * 16 + e;
-            const float c = rope_row[2 * j], sn = rope_row[2 * j + 1];
-            const float other = lane_xor4(v[e]);
-            v[e] = rnd_dt<DT_BF16>(o8 < 4 ? __builtin_fmaf(v[e], c, -(other * sn)) : __builtin_fmaf(v[e], c, other * sn));
+        for (int j = 0; j < N; ++j) {
+            norm_row(v[j], o8, wv, eps, mode == 2);
+            if (!rope) continue;
+            const float* r = rope + (int64_t)row_of(j) * 128;
+            if (mode == 1) {
+                float cs[16];
+#pragma unroll
+                for (int e = 0; e < 16; ++e) cs[e] = r[o8 * 16 + e];
+                rope_pairs(v[j], cs);
+            } else {
+                rope_halves(v[j], o8, r + (o8 & 3) * 32);
+            }
         }
     }
 }
 
+// Sixteen codes rn(v * inv), for |v * inv| below 2^22: around 1.5 * 2^23 a float has a step of 1, so adding that leaves the
+// rounded number in the low bits, two's complement.  No clamp: inv is the reciprocal of (largest |v|) / 127 + 1e-7.  A NaN
+// gives 0 (its payload's low byte), as the reference's conversion does.
+__device__ __forceinline__ uint32_t pack_low_bytes(float a, float b, float c, float d) {
+    return __builtin_amdgcn_perm(__builtin_amdgcn_perm(f2u(d), f2u(c), 0x0c0c0400u), __builtin_amdgcn_perm(f2u(b), f2u(a), 0x0c0c0400u), 0x05040100u);
+}
 __device__ __forceinline__ uint4 codes16(const float (&v)[16], float inv) {
-    uint32_t w[4] = {0u, 0u, 0u, 0u};
+    constexpr float M = 12582912.f;
+    uint32_t w[4];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) w[e / 4] |= (uint32_t)(uint8_t)rn_s8(v[e] * inv) << (8 * (e % 4));
+    for (int e = 0; e < 4; ++e) w[e] = pack_low_bytes(v[4 * e] * inv + M, v[4 * e + 1] * inv + M, v[4 * e + 2] * inv + M, v[4 * e + 3] * inv + M);
     return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
@@ -261,6 +322,36 @@ template <int DT> __device__ __forceinline__ void ld16_dt(const void* p, int64_t
         ld4_dt<DT>(p, i + g * 4, vec, x);
 #pragma unroll
         for (int c = 0; c < 4; ++c) v[g * 4 + c] = x[c];
+    }
+}
+
+// N rows' sixteen channels, all loads issued before the first is used.
+template <int DT, int N, class RowOf>
+__device__ __forceinline__ void load_rows(const void* p, int64_t base, int64_t rs, int vec, float (&v)[N][16], RowOf row_of) {
+    if (vec == 2) {
+        uint4 w[N][2];
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const uint4* q = reinterpret_cast<const uint4*>((const uint16_t*)p + base + (int64_t)row_of(j) * rs);
+            w[j][0] = q[0];
+            w[j][1] = q[1];
+        }
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const uint32_t u[8] = {w[j][0].x, w[j][0].y, w[j][0].z, w[j][0].w, w[j][1].x, w[j][1].y, w[j][1].z, w[j][1].w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                if (DT == DT_BF16) {
+                    v[j][2 * e] = u2f(u[e] << 16);
+                    v[j][2 * e + 1] = u2f(u[e] & 0xffff0000u);
+                } else {
+                    unpack_f16x2(u[e], v[j][2 * e], v[j][2 * e + 1]);
+                }
+            }
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < N; ++j) ld16_dt<DT>(p, base + (int64_t)row_of(j) * rs, vec, v[j]);
     }
 }
 
@@ -403,81 +494,95 @@ __device__ __forceinline__ void anchor_body(const AttnArgs& a, const int hi, con
     }
 }
 
-// Q: every run of D/16 lanes is one scale group (rows g, g+8, .. of a block of 32 rows, 16 at head dim 256), a lane
-// holding 16 channels of each of the group's rows; a wave carries 64 / (D/16) groups, a workgroup four waves.
-template <int DT, int D>
+// Q: a scale group is the rows g, g+8, .. of a block of 32 rows (16 at head dim 256), a row D/16 lanes of 16 channels each.
+// Two runs of lanes share a group's rows at head dims 64 and 128 (one run has them all at 256), so that a lane holds two
+// rows and the registers leave room for every workgroup of a usual call to be resident at once (four rows per lane, with
+// norm and rope: 158 registers, 37 us at 4608 x 24; two: 100 registers, 22 us).
+constexpr int q_runs(int D) { return D == 256 ? 1 : 2; }
+constexpr int q_groups_per_wave(int D) { return 64 / lanes_per_row(D) / q_runs(D); }
+template <int DT, int D, int NM>
 __device__ __forceinline__ void quant_q_body(const AttnArgs& a, const int hi, const int ty, const int bi) {
-    constexpr int LPR = lanes_per_row(D), GPW = 64 / LPR, WQ = q_block_rows(D), NR = WQ / 8;
-    const int lane = threadIdx.x & 63, ol = lane & (LPR - 1);
-    const int gid = (ty * 4 + (threadIdx.x >> 6)) * GPW + lane / LPR;   // scale group of the head: block * 8 + g
+    constexpr int LPR = lanes_per_row(D), NRUN = q_runs(D), GPW = q_groups_per_wave(D), WQ = q_block_rows(D), NR = WQ / 8 / NRUN;
+    const int lane = threadIdx.x & 63, ol = block_of_lane<D>(lane & (LPR - 1)), part = (lane / LPR) % NRUN;
+    const int gid = (ty * 4 + (threadIdx.x >> 6)) * GPW + lane / (LPR * NRUN);   // scale group of the head: block * 8 + g
     if (gid >= a.qg * 8) return;
     const int t = gid >> 3, g = gid & 7;
     const int64_t bh = (int64_t)bi * a.h + hi, base = bi * a.q_bs + hi * a.q_hs + ol * 16;
     float v[NR][16];
-#pragma unroll
-    for (int j = 0; j < NR; ++j) {
-        const int row = t * WQ + g + 8 * j;
-        const int rr = row < a.lq ? row : a.lq - 1;
-        ld16_dt<DT>(a.q, base + (int64_t)rr * a.q_rs, a.in_vec, v[j]);
-        if constexpr (D == 128) {
-            if (a.q_norm) norm_rope_row(v[j], ol, a.qw, a.rope ? a.rope + (int64_t)rr * D : nullptr, a.eps, a.rope_mode);
-        }
+    const auto true_row = [&](int j) { return t * WQ + g + 8 * (part * NR + j); };
+    const auto row_of = [&](int j) { return true_row(j) < a.lq ? true_row(j) : a.lq - 1; };
+    load_rows<DT, NR>(a.q, base, a.q_rs, a.in_vec, v, row_of);
+    if constexpr (NM != NORM_NONE) {
+        if (a.q_norm) norm_rope_rows<NM, NR>(v, ol, a.qw, a.rope, a.eps, a.rope_mode, row_of);
     }
     float mx = 0.f;
 #pragma unroll
     for (int j = 0; j < NR; ++j) {
         rotate_row<D>(v[j], ol, a.rot4);
-        if (t * WQ + g + 8 * j < a.lq) {
+        if (true_row(j) < a.lq) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) mx = fmax_nn(mx, fabsf(v[j][e]));
         }
     }
     mx = max_row<D>(mx);
+    if (D == 128) mx = fmax_nn(mx, block_xor8(mx));
+    if (D == 64) mx = fmax_nn(mx, block_xor4(mx));   // a lane of the other run: all of them hold its maximum
     const float sc = mx / 127.f + 1e-7f, inv = 1.f / sc;
-    if (ol == 0) a.qs[bh * a.qg * 8 + gid] = sc;
+    if (ol == 0 && part == 0) a.qs[bh * a.qg * 8 + gid] = sc;
 #pragma unroll
-    for (int j = 0; j < NR; ++j) {
-        const int row = t * WQ + g + 8 * j;
-        if (row < a.lq) *reinterpret_cast<uint4*>(a.qi + (bh * a.lq + row) * D + ol * 16) = codes16(v[j], inv);
-    }
+    for (int j = 0; j < NR; ++j)
+        if (true_row(j) < a.lq) *reinterpret_cast<uint4*>(a.qi + (bh * a.lq + true_row(j)) * D + ol * 16) = codes16(v[j], inv);
 }
 
-// K: one workgroup of 256 threads per tile of CK keys.  A scale group is the keys with (key % 8) / 2 == g; its CK/4 rows
+// K: one workgroup of NT threads per tile of CK keys.  A scale group is the keys with (key % 8) / 2 == g; its CK/4 rows
 // are shared out over the runs of D/16 lanes that serve the group, whose maxima meet in LDS.  The tile is assembled in
 // LDS in fragment order, [32-key block][channel step of 32][half of 16 channels][key][16 bytes] (the 64 lanes of the
 // attention kernel read one contiguous KB per load), and leaves as 16-byte stores over its contiguous CK * D bytes;
 // keys past lk are zeros.
-template <int DT, int CK, int D>
+constexpr int stage2_threads(int CK) { return CK == 128 ? 512 : 256; }
+template <int DT, int CK, int D, int NM>
 __device__ __forceinline__ void quant_k_body(const AttnArgs& a, const int hi, const int t, const int bi) {
-    constexpr int LPR = lanes_per_row(D), RUNS = 256 / LPR, NSUB = RUNS / 4;
+    constexpr int NT = stage2_threads(CK), LPR = lanes_per_row(D), RUNS = NT / LPR, NSUB = RUNS / 4;
     constexpr int R = (CK / 4) / NSUB;   // rows per run
     static_assert(R >= 1 && R * NSUB * 4 == CK, "rows of a group divide over its runs");
     __shared__ float omax[RUNS];
+    __shared__ __align__(16) float shift[D];
     __shared__ __align__(16) uint8_t stage[CK * D];
-    const int ol = threadIdx.x & (LPR - 1), run = threadIdx.x / LPR, g = run & 3, sub = run >> 2;
+    const int ol = block_of_lane<D>(threadIdx.x & (LPR - 1)), run = threadIdx.x / LPR, g = run & 3, sub = run >> 2;
     const int64_t bh = (int64_t)bi * a.hk + hi, base = bi * a.k_bs + hi * a.k_hs + ol * 16;
     const int anchor = a.anchors[bh];
-    float bias[16];
-#pragma unroll
-    for (int e = 0; e < 16; ++e) bias[e] = 0.f;
-    if (anchor >= 0) {
-        ld16_dt<DT>(a.k, base + (int64_t)anchor * a.k_rs, a.in_vec, bias);
-        if constexpr (D == 128) {
-            if (a.k_norm) norm_rope_row(bias, ol, a.kw, a.rope ? a.rope + (int64_t)anchor * D : nullptr, a.eps, a.rope_mode);
-        }
-    }
     float v[R][16];
+    const auto tile_row = [&](int j) { const int i = sub * R + j; return (i / 2) * 8 + g * 2 + (i % 2); };   // i: index within the group
+    const auto row_of = [&](int j) {
+        const int row = t * CK + tile_row(j);
+        return row < a.lk ? row : a.lk - 1;
+    };
+    load_rows<DT, R>(a.k, base, a.k_rs, a.in_vec, v, row_of);
+    // the anchor as the keys are seen: one run of lanes takes it through the norm, the others read it from LDS
+    if (anchor >= 0 && run == 0) {
+        float x[1][16];
+        const auto anchor_row = [&](int) { return anchor; };
+        load_rows<DT, 1>(a.k, base, a.k_rs, a.in_vec, x, anchor_row);
+        if constexpr (NM != NORM_NONE) {
+            if (a.k_norm) norm_rope_rows<NM, 1>(x, ol, a.kw, a.rope, a.eps, a.rope_mode, anchor_row);
+        }
+#pragma unroll
+        for (int e = 0; e < 16; e += 4) *reinterpret_cast<float4*>(shift + ol * 16 + e) = make_float4(x[0][e], x[0][e + 1], x[0][e + 2], x[0][e + 3]);
+    }
+    if constexpr (NM != NORM_NONE) {
+        if (a.k_norm) norm_rope_rows<NM, R>(v, ol, a.kw, a.rope, a.eps, a.rope_mode, row_of);
+    }
+    __syncthreads();
+    float bias[16];
+    if (anchor >= 0) {
+        load16_f32(shift + ol * 16, bias);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) bias[e] = 0.f;
+    }
     int rt[R];
 #pragma unroll
-    for (int j = 0; j < R; ++j) {
-        const int i = sub * R + j;                  // index within the group
-        rt[j] = (i / 2) * 8 + g * 2 + (i % 2);      // row within the tile
-        const int row = t * CK + rt[j], rr = row < a.lk ? row : a.lk - 1;
-        ld16_dt<DT>(a.k, base + (int64_t)rr * a.k_rs, a.in_vec, v[j]);
-        if constexpr (D == 128) {
-            if (a.k_norm) norm_rope_row(v[j], ol, a.kw, a.rope ? a.rope + (int64_t)rr * D : nullptr, a.eps, a.rope_mode);
-        }
-    }
+    for (int j = 0; j < R; ++j) rt[j] = tile_row(j);
     float mx = 0.f;
 #pragma unroll
     for (int j = 0; j < R; ++j) {
@@ -506,15 +611,15 @@ __device__ __forceinline__ void quant_k_body(const AttnArgs& a, const int hi, co
     __syncthreads();
     uint4* out = reinterpret_cast<uint4*>(a.ki + (bh * a.nblk + (int64_t)t * (CK / 32)) * (32 * D));
 #pragma unroll
-    for (int i = 0; i < CK * D / 16 / 256; ++i)
-        out[i * 256 + threadIdx.x] = *reinterpret_cast<const uint4*>(stage + (i * 256 + threadIdx.x) * 16);
+    for (int i = 0; i < CK * D / 16 / NT; ++i)
+        out[i * NT + threadIdx.x] = *reinterpret_cast<const uint4*>(stage + (i * NT + threadIdx.x) * 16);
 }
 
-// V abs-max per channel: 256 threads take 128 rows of one (kv head, batch), four channels per thread; non-negative
+// V abs-max per channel: NT threads take 128 rows of one (kv head, batch), four channels per thread; non-negative
 // floats order as their bits, so the workgroups combine with an integer atomic max.
-template <int DT, int D>
+template <int DT, int D, int NT>
 __device__ __forceinline__ void v_absmax_body(const AttnArgs& a, const int hi, const int chunk, const int bi) {
-    constexpr int TPR = D / 4, RL = 256 / TPR;   // threads per row, rows per pass
+    constexpr int TPR = D / 4, RL = NT / TPR;   // threads per row, rows per pass
     __shared__ float red[RL][D];
     const int c4 = threadIdx.x % TPR, rl = threadIdx.x / TPR;
     const int64_t base = bi * a.v_bs + hi * a.v_hs + c4 * 4;
@@ -544,7 +649,7 @@ __device__ __forceinline__ void v_absmax_body(const AttnArgs& a, const int hi, c
 // Two launches carry the four bodies above: work that does not depend on each other shares a launch, heads fastest so
 // that neighbouring workgroups read neighbouring memory.  Stage 1: anchors (which also clear the V accumulators) and Q.
 // Stage 2: K (needs the anchors) and the V abs-max (needs the cleared accumulators).
-template <int DT, int D>
+template <int DT, int D, int NM>
 __global__ __launch_bounds__(256) void attn_stage1_kernel(AttnArgs a) {
     int id = blockIdx.x;
     const int n_anchor = a.hk * a.b;
@@ -553,22 +658,22 @@ __global__ __launch_bounds__(256) void attn_stage1_kernel(AttnArgs a) {
         return;
     }
     id -= n_anchor;
-    constexpr int GPB = 4 * (64 / lanes_per_row(D));   // scale groups per workgroup
+    constexpr int GPB = 4 * q_groups_per_wave(D);   // scale groups per workgroup
     const int ny = (a.qg * 8 + GPB - 1) / GPB;
-    quant_q_body<DT, D>(a, id % a.h, (id / a.h) % ny, id / (a.h * ny));
+    quant_q_body<DT, D, NM>(a, id % a.h, (id / a.h) % ny, id / (a.h * ny));
 }
 
-template <int DT, int CK, int D>
-__global__ __launch_bounds__(256) void attn_stage2_kernel(AttnArgs a) {
+template <int DT, int CK, int D, int NM>
+__global__ __launch_bounds__(stage2_threads(CK)) void attn_stage2_kernel(AttnArgs a) {
     int id = blockIdx.x;
     const int n_k = a.hk * a.kb * a.b;
     if (id < n_k) {
-        quant_k_body<DT, CK, D>(a, id % a.hk, (id / a.hk) % a.kb, id / (a.hk * a.kb));
+        quant_k_body<DT, CK, D, NM>(a, id % a.hk, (id / a.hk) % a.kb, id / (a.hk * a.kb));
         return;
     }
     id -= n_k;
     const int nc = (a.lk + 127) / 128;
-    v_absmax_body<DT, D>(a, id % a.hk, (id / a.hk) % nc, id / (a.hk * nc));
+    v_absmax_body<DT, D, stage2_threads(CK)>(a, id % a.hk, (id / a.hk) % nc, id / (a.hk * nc));
 }
 
 // V codes: one workgroup per block of 32 keys.  Rows are read as they lie (a thread takes 16 channels of one key),
@@ -962,6 +1067,245 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void attn_int8_kernel(AttnAr
     }
 }
 
+// One KB global -> LDS, 16 bytes per lane, without registers; the wave's own s_waitcnt vmcnt covers it.
+__device__ __forceinline__ void dma16(uint32_t lds_dst, uint32_t lane_off, const void* base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_dst), "v"(lane_off), "s"(base) : "memory", "m0");
+}
+__device__ __forceinline__ float swap32_max(float x) {   // maximum of a lane and lane ^ 32
+    const auto r = __builtin_amdgcn_permlane32_swap(f2u(x), f2u(x), false, false);
+    return fmax_nn(u2f(r[0]), u2f(r[1]));
+}
+__device__ __forceinline__ float swap32_sum(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(f2u(x), f2u(x), false, false);
+    return u2f(r[0]) + u2f(r[1]);
+}
+
+// The attention without a key bias, head dims 64 and 128: attn_int8_kernel's arithmetic with the work of two tiles overlapped.
+// It is bound by vector instruction issue (at 4608 tokens x 24 heads of 128: 467 per wave and tile beside 32 MFMAs, which keep
+// the vector pipes waiting about 14 of their 32 cycles each) and by the last round of workgroups (864 on 512 places).
+//   * K runs a tile ahead of V through the two LDS stages: as soon as a key block's probabilities are packed, the next tile's
+//     scores go into its registers, one MFMA behind every fourth of the next block's probabilities; the products with V go
+//     an output block at a time with the fold of the block before between them.  (All scores, then all probabilities, then
+//     all products: the two waves of a SIMD want the same pipe at the same time.)
+//   * the key scales of the next tile are loaded ahead of its DMA.  Loaded where they are used, their wait is a wait for the
+//     whole tile that has just been asked for, since the counter runs in order.
+//   * numerator and denominator are relative to a base that all but never moves (below), which takes the multiplication
+//     of every output by its rescale factor out of every tile.
+//   * DMA addresses are scalar, the exchange with lane ^ 32 is a row swap.
+// 250 -> 230 us at that shape by the kernel trace, 141 -> 129 us at SDXL's 2 x 4096 x 10 x 64.  A workgroup of eight waves
+// (half the DMA per wave, one workgroup per CU) measured the same for 128 and 30 % slower for 64.
+template <int OUT_DT, int CK, int D>
+__global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
+    constexpr int NB = CK / 32, NS = D / 32, KV = CK * D, STAGE = 2 * KV + D * 4;
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l32 = lane & 31, hh = lane >> 5;
+    const int hi = blockIdx.y, bi = blockIdx.z;
+    const int row0 = blockIdx.x * 128 + wave * 32;
+    const int64_t bh = (int64_t)bi * a.h + hi, kvh = (int64_t)bi * a.hk + hi / a.rep;
+    const int r = row0 + l32, rc = r < a.lq ? r : a.lq - 1;   // rows past lq are computed on a clamped row and never stored
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)smem, lane16 = lane * 16;
+    const int8_t *kt = a.ki + kvh * a.nblk * (32 * D), *vt = a.vt + kvh * a.nblk * (32 * D);
+    const int* vst = a.vsum + kvh * a.kb * D;
+    const float* kst = a.ks + kvh * a.kb * 4 + hh * 2;
+
+    auto fetch_k = [&](int t) {
+#pragma unroll
+        for (int j = 0; j < KV / 4096; ++j) {
+            const int c = (wave + 4 * j) * 1024;
+            dma16(lds0 + (t & 1) * STAGE + c, lane16, kt + (int64_t)t * KV + c);
+        }
+    };
+    auto fetch_v = [&](int t) {
+#pragma unroll
+        for (int j = 0; j < KV / 4096; ++j) {
+            const int c = (wave + 4 * j) * 1024;
+            dma16(lds0 + (t & 1) * STAGE + KV + c, lane16, vt + (int64_t)t * KV + c);
+        }
+        if (wave == 0 && lane < D / 4) dma16(lds0 + (t & 1) * STAGE + 2 * KV, lane16, vst + (int64_t)t * D);
+    };
+    fetch_k(0);
+    fetch_v(0);
+    if (a.kb > 1) fetch_k(1);
+
+    v4i qf[NS];
+    {
+        const int8_t* qrow = a.qi + (bh * a.lq + rc) * D + hh * 16;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) qf[s] = *reinterpret_cast<const v4i*>(qrow + s * 32);
+    }
+    const float q_scale = a.qs[(bh * a.qg + r / 32) * 8 + (r & 7)];
+    float k0 = kst[0], k1 = kst[1];
+
+    float ro[NS][16];
+#pragma unroll
+    for (int x = 0; x < NS; ++x)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) ro[x][i] = 0.f;
+    float m = -50000.f, dsum = 1.f, dsum2 = 0.f;
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+    __syncthreads();
+
+    v16i S[NB];
+    auto load_kf = [&](v4i (&kf)[NS], int t, int blk) {
+        const uint8_t* st = smem + (t & 1) * STAGE + blk * (32 * D) + lane * 16;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) kf[s] = *reinterpret_cast<const v4i*>(st + s * 1024);
+    };
+#pragma unroll
+    for (int blk = 0; blk < NB; ++blk) {
+        v4i kf[NS];
+        load_kf(kf, 0, blk);
+        S[blk] = v16i{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int s = 0; s < NS; ++s) S[blk] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[s], qf[s], S[blk], 0, 0, 0);
+    }
+    __syncthreads();   // the first K stage may be fetched into
+
+    auto tile = [&](const int t, auto last_tag) {
+        constexpr bool last = decltype(last_tag)::value;
+        const uint8_t* st = smem + (t & 1) * STAGE;
+        const int key0 = t * CK;
+        float n0 = 0.f, n1 = 0.f;
+        if constexpr (!last) {
+            n0 = kst[(t + 1) * 4];
+            n1 = kst[(t + 1) * 4 + 1];
+            if (t + 2 < a.kb) fetch_k(t + 2);
+            fetch_v(t + 1);
+        }
+        const float gs0 = a.sm * (q_scale * k0), gs1 = a.sm * (q_scale * k1);
+        int i0 = last ? -50000 : INT_MIN, i1 = i0;
+#pragma unroll
+        for (int blk = 0; blk < NB; ++blk)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                int sv = S[blk][i];
+                if constexpr (last) {
+                    const int key = key0 + blk * 32 + (i / 4) * 8 + hh * 4 + (i % 4);
+                    sv = key < a.lk ? sv : INT_MIN;
+                }
+                if ((i % 4) < 2) i0 = max(i0, sv);
+                else i1 = max(i1, sv);
+            }
+        const float tile_m = swap32_max(fmax_nn(fmaf((float)i0, gs0, -kU8Offset), fmaf((float)i1, gs1, -kU8Offset)));
+        // The running base m only moves when a tile's maximum has outgrown it by 2^60 (and at the first tile): numerator and
+        // denominator are both relative to it, so any base gives the same quotient, and the outputs need no rescaling here.
+        if (__builtin_amdgcn_ballot_w64(tile_m - m > 60.f)) {
+            const float f = tile_m > m ? __builtin_amdgcn_exp2f(m - tile_m) : 1.f;
+            m = fmax_nn(m, tile_m);
+            dsum *= f;
+            dsum2 *= f;
+#pragma unroll
+            for (int x = 0; x < NS; ++x)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) ro[x][i] *= f;
+        }
+        const float t_scale = __builtin_amdgcn_exp2f(tile_m - m);
+
+        v4i pf[NB];
+        uint32_t psum = 0;
+#pragma unroll
+        for (int rg = 0; rg <= (last ? NB - 1 : NB); ++rg) {
+            // region rg: probabilities of key block rg, and under them the next tile's scores into the block before it
+            v4i kf[NS];
+            if constexpr (!last)
+                if (rg > 0) load_kf(kf, t + 1, rg - 1);
+            float e[4][4];
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+                if (rg < NB) {
+                    uint32_t packed = 0u;
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        e[g4][c] = __builtin_amdgcn_exp2f(fmaf((float)S[rg < NB ? rg : 0][g4 * 4 + c], c < 2 ? gs0 : gs1, -tile_m));
+                        if constexpr (last) {
+                            const int key = key0 + rg * 32 + g4 * 8 + hh * 4 + c;
+                            e[g4][c] = key < a.lk ? e[g4][c] : 0.f;
+                        }
+                        packed = __builtin_amdgcn_cvt_pk_u8_f32(e[g4][c], c, packed);
+                    }
+                    if constexpr (!last) psum = __builtin_amdgcn_sad_u8(packed, 0u, psum);
+                    pf[rg < NB ? rg : 0][g4] = (int)(packed ^ 0x80808080u);
+                }
+                if constexpr (!last) {
+                    if (rg > 0 && g4 % (4 / NS) == 0) {
+                        const int s = g4 / (4 / NS);
+                        if (s == 0) S[rg - 1] = v16i{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+                        S[rg - 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[s], qf[s], S[rg - 1], 0, 0, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0x100);
+                }
+            }
+            if constexpr (last) {   // the unrounded probabilities, in the reference's per-thread partials
+#pragma unroll
+                for (int fk = 0; fk < 2; ++fk) {
+                    dsum += ((e[2 * fk][0] + e[2 * fk][1]) + (e[2 * fk + 1][0] + e[2 * fk + 1][1])) * t_scale;
+                    dsum2 += ((e[2 * fk][2] + e[2 * fk][3]) + (e[2 * fk + 1][2] + e[2 * fk + 1][3])) * t_scale;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if constexpr (!last) dsum = fmaf((float)psum, t_scale, dsum);
+
+        // P.V, an output block at a time; the fold of a block rides between the products of the next
+        v16i acc[2];
+#pragma unroll
+        for (int x = 0; x <= NS; ++x) {
+            if (x < NS) {
+                const int* vsp = reinterpret_cast<const int*>(st + 2 * KV) + x * 32 + hh * 4;
+#pragma unroll
+                for (int g4 = 0; g4 < 4; ++g4) {
+                    const v4i c4 = *reinterpret_cast<const v4i*>(vsp + g4 * 8);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) acc[x & 1][g4 * 4 + c] = c4[c];
+                }
+            }
+#pragma unroll
+            for (int blk = 0; blk < NB; ++blk) {
+                if (x < NS) {
+                    const v4i vf = *reinterpret_cast<const v4i*>(st + KV + ((blk * D + x * 32 + l32) * 32 + hh * 16));
+                    acc[x & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf, pf[blk], acc[x & 1], 0, 0, 0);
+                }
+                if (x > 0) {
+#pragma unroll
+                    for (int i = blk * (16 / NB); i < (blk + 1) * (16 / NB); ++i)
+                        ro[x > 0 ? x - 1 : 0][i] = fmaf((float)acc[(x + 1) & 1][i], t_scale, ro[x > 0 ? x - 1 : 0][i]);
+                }
+                __builtin_amdgcn_sched_barrier(0x100);
+            }
+        }
+        if constexpr (!last) {
+            k0 = n0;
+            k1 = n1;
+            __builtin_amdgcn_s_waitcnt(0x0f70);   // this wave's share of the next tiles has landed
+            __syncthreads();
+        }
+    };
+    for (int t = 0; t + 1 < a.kb; ++t) tile(t, std::false_type{});
+    tile(a.kb - 1, std::true_type{});
+
+    float dtot = swap32_sum(dsum + dsum2);
+    // `sink` more keys of score zero and value zero: each adds exp2(0 - m) to the denominator, nothing to the output
+    if (a.sink != 0.f) dtot = fmaf(a.sink, __builtin_amdgcn_exp2f(-m), dtot);
+    const float rcp = 1.f / dtot;
+    if (r < a.lq) {
+        const int64_t ob = bi * a.o_bs + (int64_t)r * a.o_rs + hi * a.o_hs;
+#pragma unroll
+        for (int x = 0; x < NS; ++x)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+                const int d0 = x * 32 + g4 * 8 + hh * 4;
+                const float4 s4 = *reinterpret_cast<const float4*>(a.vs + kvh * D + d0);
+                float out[4] = {ro[x][g4 * 4] * rcp * s4.x, ro[x][g4 * 4 + 1] * rcp * s4.y, ro[x][g4 * 4 + 2] * rcp * s4.z,
+                                ro[x][g4 * 4 + 3] * rcp * s4.w};
+                if (a.vec_ok) store4<OUT_DT>(a.o, ob + d0, out);
+                else
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) st_dt<OUT_DT>(a.o, ob + d0 + c, out[c]);
+            }
+    }
+}
+
 int cta_k_for(int lk, int d) { return lk > 1024 && d != 64 ? 128 : 64; }   // csrc/attn_int8.cu:56
 
 // The caller's per-key bias, prepared once per call (csrc/vendor/sage/sage_attn_launcher.cu:343-391; attn_utils.cuh:
@@ -1017,30 +1361,43 @@ Plan plan_for(int64_t b, int64_t h, int64_t hk, int64_t lq, int64_t lk, int D) {
     return p;
 }
 
-// More than 64 KB of dynamic LDS has to be allowed once per kernel and device.
-template <class K> bool allow_lds(K kern, int bytes) {
-    static PerDeviceOnce once;
-    return allow_dynamic_lds(reinterpret_cast<const void*>(kern), bytes, once) == 0;
+template <auto KERN>
+int launch_tiles(const AttnArgs& a, int lds, hipStream_t st) {
+    if (lds > 64 * 1024) {   // has to be allowed once per kernel and device
+        static PerDeviceOnce once;
+        if (allow_dynamic_lds(reinterpret_cast<const void*>(KERN), lds, once) != 0) return -401;
+    }
+    KERN<<<dim3((a.lq + 127) / 128, a.h, a.b), 256, lds, st>>>(a);
+    return hipGetLastError() == hipSuccess ? 0 : -401;
 }
-
 template <int DT, int CK, bool MASK, bool FD, int D>
 int launch_attn(const AttnArgs& a, hipStream_t st) {
-    constexpr int kLds = 2 * (2 * CK * D + D * 4);
-    auto kern = attn_int8_kernel<DT, CK, MASK, FD, D>;
-    if (kLds > 64 * 1024 && !allow_lds(kern, kLds)) return -401;
-    kern<<<dim3((a.lq + 127) / 128, a.h, a.b), 256, kLds, st>>>(a);
-    return hipGetLastError() == hipSuccess ? 0 : -401;
+    return launch_tiles<attn_int8_kernel<DT, CK, MASK, FD, D>>(a, 2 * (2 * CK * D + D * 4), st);
+}
+template <int DT, int CK, int D>
+int launch_pipe(const AttnArgs& a, hipStream_t st) {
+    return launch_tiles<attn_int8_pipe_kernel<DT, CK, D>>(a, 2 * (2 * CK * D + D * 4), st);
 }
 
 template <int DT, int D>
 int run(AttnArgs a, hipStream_t st) {
-    constexpr int GPB = 4 * (64 / lanes_per_row(D));   // scale groups per workgroup of the Q quantizer
+    constexpr int GPB = 4 * q_groups_per_wave(D);   // scale groups per workgroup of the Q quantizer
     const int64_t n1 = (int64_t)a.hk * a.b + (int64_t)a.h * ((a.qg * 8 + GPB - 1) / GPB) * a.b;
     const int64_t n2 = (int64_t)a.hk * a.kb * a.b + (int64_t)a.hk * ((a.lk + 127) / 128) * a.b;
     if (n1 > 0x7fffffff || n2 > 0x7fffffff) return -400;
-    attn_stage1_kernel<DT, D><<<dim3((unsigned)n1), 256, 0, st>>>(a);
-    if (a.ck == 64) attn_stage2_kernel<DT, 64, D><<<dim3((unsigned)n2), 256, 0, st>>>(a);
-    else if constexpr (D != 64) attn_stage2_kernel<DT, 128, D><<<dim3((unsigned)n2), 256, 0, st>>>(a);
+    const auto stages = [&](auto nm) {
+        constexpr int NM = decltype(nm)::value;
+        attn_stage1_kernel<DT, D, NM><<<dim3((unsigned)n1), 256, 0, st>>>(a);
+        if (a.ck == 64) attn_stage2_kernel<DT, 64, D, NM><<<dim3((unsigned)n2), stage2_threads(64), 0, st>>>(a);
+        else if constexpr (D != 64) attn_stage2_kernel<DT, 128, D, NM><<<dim3((unsigned)n2), stage2_threads(128), 0, st>>>(a);
+    };
+    if constexpr (D == 128 && DT == DT_BF16) {   // the only form with a norm
+        if (!a.q_norm && !a.k_norm) stages(std::integral_constant<int, NORM_NONE>{});
+        else if (a.nr_vec && a.rope_mode != 2) stages(std::integral_constant<int, NORM_PAIRS>{});
+        else stages(std::integral_constant<int, NORM_ANY>{});
+    } else {
+        stages(std::integral_constant<int, NORM_NONE>{});
+    }
     attn_v_quant_kernel<DT, D><<<dim3(a.hk, a.nblk, a.b), 256, 0, st>>>(a);
     if (hipGetLastError() != hipSuccess) return -401;
     if constexpr (D == 128) {
@@ -1055,8 +1412,13 @@ int run(AttnArgs a, hipStream_t st) {
     }
     // f16 outputs with at most 512 keys: the reference's build takes its unfused probability path in every tile
     if (DT == DT_F16 && a.lk <= 512 && a.ck == 64) return launch_attn<DT_F16, 64, false, true, D>(a, st);
-    if (a.ck == 64) return launch_attn<DT, 64, false, false, D>(a, st);
-    if constexpr (D != 64) return launch_attn<DT, 128, false, false, D>(a, st);
+    if constexpr (D != 256) {
+        if (a.ck == 64) return launch_pipe<DT, 64, D>(a, st);
+        if constexpr (D != 64) return launch_pipe<DT, 128, D>(a, st);
+    } else {
+        if (a.ck == 64) return launch_attn<DT, 64, false, false, D>(a, st);
+        return launch_attn<DT, 128, false, false, D>(a, st);
+    }
     return -400;
 }
 
@@ -1103,7 +1465,8 @@ int int8_attn(const void* q, const void* k, const void* v, void* o, void* ws, in
     a.use_anchor = sink == 0.f ? 1 : 0;   // with a sink a zero key's score must stay zero: no shift (csrc/attn_int8.cu:134-141)
     a.vec_ok = ((o_bs | o_rs | o_hs) % 4 == 0 && ((uintptr_t)o & 7) == 0) ? 1 : 0;
     a.v_vec = ((v_bs | v_rs | v_hs) % 4 == 0 && ((uintptr_t)v & 7) == 0) ? 1 : 0;
-    a.in_vec = ((q_bs | q_rs | q_hs | k_bs | k_rs | k_hs) % 4 == 0 && (((uintptr_t)q | (uintptr_t)k) & 7) == 0) ? 1 : 0;
+    const auto vec_of = [](int64_t strides, uintptr_t base) { return strides % 8 == 0 && (base & 15) == 0 ? 2 : strides % 4 == 0 && (base & 7) == 0 ? 1 : 0; };
+    a.in_vec = vec_of(q_bs | q_rs | q_hs | k_bs | k_rs | k_hs, (uintptr_t)q | (uintptr_t)k);
     a.bias = bias;
     a.kbias = (float*)(w + p.total);   // the key-bias form's workspace is this much longer
     a.tbias = a.kbias + (int64_t)p.kb * p.ck;
@@ -1119,6 +1482,7 @@ int int8_attn(const void* q, const void* k, const void* v, void* o, void* ws, in
         a.q_norm = 1;
         a.k_norm = norm->kw ? 1 : 0;
     }
+    a.nr_vec = (((uintptr_t)a.qw | (uintptr_t)a.kw | (uintptr_t)a.rope) & 15) == 0 ? 1 : 0;
     hipStream_t st = (hipStream_t)stream;
     if (Dh == 64) return dt == DT_F16 ? run<DT_F16, 64>(a, st) : run<DT_BF16, 64>(a, st);
     if (Dh == 256) return dt == DT_F16 ? run<DT_F16, 256>(a, st) : run<DT_BF16, 256>(a, st);
@@ -1226,7 +1590,7 @@ GPU_API int gpu_internal_cvt_pk_u8_probe(const float* x, uint32_t* y, int n, voi
 // the anchor search takes it (one thread, sumsq128_serial).  out[2 * row] and out[2 * row + 1]; rows a multiple of 8.
 namespace {
 __global__ void __launch_bounds__(64) sumsq_probe_kernel(const float* x, float* out, int split) {
-    const int lane = threadIdx.x, o8 = lane & 7, row = blockIdx.x * 8 + (lane >> 3);
+    const int lane = threadIdx.x, o8 = block_of_lane<128>(lane & 7), row = blockIdx.x * 8 + (lane >> 3);
     float v[16];
 #pragma unroll
     for (int e = 0; e < 16; ++e) v[e] = x[row * 128 + o8 * 16 + e];

@@ -140,6 +140,17 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
     return join(h[0], l[0]) + join(h[1], l[1]);
 }
 
+// 1/sqrt(a) in fp64, rounded to fp32: two Newton steps on the hardware's fp32 estimate (23 bits, then 45, then the rounding
+// of fp64), a tenth of the instructions of the fp64 square root and division, which serve the ends of the range.
+__device__ __forceinline__ float rsqrt_cr(float a) {
+    if (!(a > 1e-30f && a < 1e30f)) return (float)(1.0 / sqrt((double)a));
+    const double d = (double)a;
+    double y = (double)__builtin_amdgcn_rsqf(a);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) y = __builtin_fma(0.5 * y, __builtin_fma(-d * y, y, 1.0), y);
+    return (float)y;
+}
+
 // Workgroup -> tile.  Workgroups are dealt round-robin to the 8 XCDs (each with its own L2), so first renumber them
 // XCD-contiguously, then walk tiles in panels of 4 tile rows so that the 32 workgroups an XCD runs at once cover a
 // 4 x 8 patch of tiles and share A rows / W rows in that XCD's L2.

@@ -102,17 +102,6 @@ __device__ __forceinline__ float row_sum_f64(double v, double* red, int wave, in
     return (float)t;
 }
 
-// 1/sqrt(a) in fp64, rounded to fp32: two Newton steps on the hardware's fp32 estimate (23 bits, then 45, then the rounding
-// of fp64), a tenth of the instructions of the fp64 square root and division, which serve the ends of the range.
-__device__ __forceinline__ float rsqrt_cr(float a) {
-    if (!(a > 1e-30f && a < 1e30f)) return (float)(1.0 / sqrt((double)a));
-    const double d = (double)a;
-    double y = (double)__builtin_amdgcn_rsqf(a);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) y = __builtin_fma(0.5 * y, __builtin_fma(-d * y, y, 1.0), y);
-    return (float)y;
-}
-
 // The rotation of a row's chunks and the maximum of their magnitudes over the lane's values.  `exact`: the values are bf16
 // or f16 numbers (rotate_chunk's condition for scaling once; bf16 ones are also checked against the overflow limit).
 template <int MODE, int G, int C>
