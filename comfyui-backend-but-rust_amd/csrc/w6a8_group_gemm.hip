@@ -456,10 +456,24 @@ bool shape_fits(int64_t M, int64_t N, int64_t K) {
     return ((M + BM - 1) / BM) * ((N + BN - 1) / BN) <= 0x7fffffff;
 }
 
+bool expands_first(const void* Wp, int64_t M, int64_t N, int64_t K) {
+    const int mode = g_mode.load(std::memory_order_relaxed);
+    return (mode == 1 || (mode != 0 && M >= kExpandFirstRows)) && N * K < ((int64_t)1 << 32) && ((uintptr_t)Wp & 3) == 0;
+}
+
 }  // namespace
 
-GPU_API int gpu_w6a8_group_gemm(const int8_t* A, const void* Wp, const float* xs, const float* sw, const void* bias,
-                                void* D, int32_t* partials, int64_t M, int64_t N, int64_t K, int out_dt, void* stream) {
+GPU_API int64_t gpu_w6a8_group_gemm_scratch(const void* Wp, int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K <= 0 || (K % 128) != 0 || !shape_fits(M, N, K)) return 0;
+    return expands_first(Wp, M, N, K) ? N * K : 0;
+}
+
+// `scratch`: what gpu_w6a8_group_gemm_scratch asks for, kept by the caller or taken from the allocator that the rest of its
+// tensors come from.  Without one the call makes a stream-ordered allocation of that size, which the default pool gives
+// back at every synchronization and takes again at the next call with the host waiting (M=8192, K=5120 -> N=13824 behind
+// a synchronization: 1112 us, 758 with a scratch).
+GPU_API int gpu_w6a8_group_gemm_ws(const int8_t* A, const void* Wp, const float* xs, const float* sw, const void* bias, void* D,
+                                   int32_t* partials, void* scratch, int64_t M, int64_t N, int64_t K, int out_dt, void* stream) {
     if (K < 0 || (K % 128) != 0) return -1;
     if (out_dt < DT_F32 || out_dt > DT_BF16 || M < 0 || N < 0) return -200;
     if (M == 0 || N == 0) return 0;
@@ -468,11 +482,15 @@ GPU_API int gpu_w6a8_group_gemm(const int8_t* A, const void* Wp, const float* xs
     a.tiles_m = (int)((M + BM - 1) / BM);
     a.tiles_n = (int)((N + BN - 1) / BN);
     hipStream_t st = (hipStream_t)stream;
-    const int mode = g_mode.load(std::memory_order_relaxed);
-    int8_t* w8 = nullptr;
-    if ((mode == 1 || (mode != 0 && M >= kExpandFirstRows)) && N * K < ((int64_t)1 << 32) && ((uintptr_t)Wp & 3) == 0) {
-        hipError_t e = hipMallocAsync((void**)&w8, (size_t)(N * K), st);
-        if (e != hipSuccess) return (int)e;
+    if ((uintptr_t)scratch & 15) return -1;   // stored 16 bytes at a time
+    int8_t* own = nullptr;
+    if (expands_first(Wp, M, N, K)) {
+        int8_t* w8 = (int8_t*)scratch;
+        if (!w8) {
+            hipError_t e = hipMallocAsync((void**)&own, (size_t)(N * K), st);
+            if (e != hipSuccess) return (int)e;
+            w8 = own;
+        }
         const int64_t pieces = N * K / 16;
         const unsigned grid = (unsigned)((pieces + 255) / 256 < 256 * 32 ? (pieces + 255) / 256 : 256 * 32);
         hipLaunchKernelGGL(w6_words_to_int8_kernel, dim3(grid), dim3(256), 0, st, (const uint8_t*)Wp, w8, pieces);
@@ -484,11 +502,16 @@ GPU_API int gpu_w6a8_group_gemm(const int8_t* A, const void* Wp, const float* xs
         case DT_F16: rc = launch_dt<DT_F16>(a, st); break;
         default: rc = launch_dt<DT_BF16>(a, st); break;
     }
-    if (w8) {
-        hipError_t e = hipFreeAsync(w8, st);
+    if (own) {
+        hipError_t e = hipFreeAsync(own, st);
         if (rc == 0 && e != hipSuccess) rc = (int)e;
     }
     return rc;
+}
+
+GPU_API int gpu_w6a8_group_gemm(const int8_t* A, const void* Wp, const float* xs, const float* sw, const void* bias, void* D,
+                                int32_t* partials, int64_t M, int64_t N, int64_t K, int out_dt, void* stream) {
+    return gpu_w6a8_group_gemm_ws(A, Wp, xs, sw, bias, D, partials, nullptr, M, N, K, out_dt, stream);
 }
 
 // Test hook, no reference counterpart: 0 = gpu_w6a8_group_gemm always expands the weights inside the kernel, 1 = always

@@ -39,6 +39,9 @@ SIGNATURES = {
     "gpu_int8_gemm_acc": [_P, _P, _P, _I64, _I64, _I64, _P],
     "gpu_int8_gemm_static": [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I32, _P],
     "gpu_w6a8_gemm": [_P, _P, _P, _I32, _P, _P, _P, _P, _I64, _I64, _I64, _I32, _P],
+    "gpu_w6a8_gemm_ws": [_P, _P, _P, _I32, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I32, _P],
+    "gpu_w6a8_group_gemm_ws": [_P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I32, _P],
+    "gpu_w6a8_group_gemm_scratch": [_P, _I64, _I64, _I64],
     "gpu_w6a8_group_gemm": [_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I32, _P],
     "gpu_int8_attn_d": [_P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32] + [_I64] * 12 + [_F32, _P],
     "gpu_int8_attn_f16": [_P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32] + [_I64] * 12 + [_F32, _P],
@@ -75,6 +78,7 @@ def _load():
     lib.gpu_int8_attn_workspace.restype = _I64
     lib.gpu_int8_attn_key_bias_workspace.argtypes = [_I32] * 5
     lib.gpu_int8_attn_key_bias_workspace.restype = _I64
+    lib.gpu_w6a8_group_gemm_scratch.restype = _I64
     lib.gpu_int8_gemm_static_limit.argtypes = []
     lib.gpu_int8_gemm_static_limit.restype = _I64
     lib.gpu_kernels_build_info.restype = C.c_char_p

@@ -250,7 +250,9 @@ def w6a8_gemm(A, wq, s_rel, G, xs, s_channel, bias=None, out_dtype=torch.bfloat1
     M, K = A.shape
     N = wq.shape[0]
     D = torch.empty((M, N), dtype=out_dtype, device=A.device)
-    ffi.k("gpu_w6a8_gemm", _ptr(A), _ptr(wq), _ptr(s_rel), G, _ptr(xs), _ptr(s_channel), _ptr(bias), _ptr(D), M, N, K,
+    # the expanded weights: torch's allocator orders the block by stream and keeps it between calls
+    w8 = torch.empty((N, K) if M else 0, dtype=torch.int8, device=A.device)
+    ffi.k("gpu_w6a8_gemm_ws", _ptr(A), _ptr(wq), _ptr(s_rel), G, _ptr(xs), _ptr(s_channel), _ptr(bias), _ptr(D), _ptr(w8), M, N, K,
           _TORCH_DT[out_dtype], _stream())
     return D
 
@@ -264,7 +266,8 @@ def w6a8_group_gemm(A, packed, xs, sw, bias=None, out_dtype=torch.bfloat16, want
     N = packed.shape[0]
     D = torch.empty((M, N), dtype=out_dtype, device=A.device)
     part = torch.empty((M, N, K // 128), dtype=torch.int32, device=A.device) if want_partials else None
-    ffi.k("gpu_w6a8_group_gemm", _ptr(A), _ptr(packed), _ptr(xs), _ptr(sw), _ptr(bias), _ptr(D), _ptr(part), M, N, K,
+    w8 = torch.empty((ffi.lib.gpu_w6a8_group_gemm_scratch(_ptr(packed), M, N, K),), dtype=torch.int8, device=A.device)
+    ffi.k("gpu_w6a8_group_gemm_ws", _ptr(A), _ptr(packed), _ptr(xs), _ptr(sw), _ptr(bias), _ptr(D), _ptr(part), _ptr(w8), M, N, K,
           _TORCH_DT[out_dtype], _stream())
     return (D, part) if want_partials else D
 

@@ -265,6 +265,10 @@ int64_t gpu_int8_gemm_static_limit(void);
  * gpu_int8_gemm. */
 int gpu_w6a8_gemm(const int8_t* A, const void* wq, const void* s_rel, int G, const float* xs, const float* s_channel,
                   const void* bias, void* D, int64_t M, int64_t N, int64_t K, int out_dt, void* stream);
+/* The same with the caller's scratch: N*K bytes of device memory, 16-byte aligned (-1 otherwise), in use until the work
+ * queued here has run; null allocates as above. */
+int gpu_w6a8_gemm_ws(const int8_t* A, const void* wq, const void* s_rel, int G, const float* xs, const float* s_channel,
+                     const void* bias, void* D, void* scratch, int64_t M, int64_t N, int64_t K, int out_dt, void* stream);
 
 /* W6A8 linear with fp32 scales per group of 128 along K, for this library's own packed format (no counterpart in the
  * reference, whose W6 weights are two-plane with e4m3 group factors: gpu_w6_decode / gpu_w6a8_gemm above).  Up to 4095
@@ -281,6 +285,11 @@ int gpu_w6a8_gemm(const int8_t* A, const void* wq, const void* s_rel, int G, con
  * Returns -1 for K % 128 != 0; -200 for an unknown out_dt, K == 0, or sizes beyond 32-bit byte offsets. */
 int gpu_w6a8_group_gemm(const int8_t* A, const void* Wp, const float* xs, const float* sw, const void* bias, void* D,
                         int32_t* partials, int64_t M, int64_t N, int64_t K, int out_dt, void* stream);
+/* The same with the caller's scratch, 16-byte aligned (-1 otherwise), of the bytes that gpu_w6a8_group_gemm_scratch names
+ * for the call (0: none is used), in use until the work queued here has run; null allocates as above. */
+int gpu_w6a8_group_gemm_ws(const int8_t* A, const void* Wp, const float* xs, const float* sw, const void* bias, void* D,
+                           int32_t* partials, void* scratch, int64_t M, int64_t N, int64_t K, int out_dt, void* stream);
+int64_t gpu_w6a8_group_gemm_scratch(const void* Wp, int64_t M, int64_t N, int64_t K);
 
 /* Test and tuning hook: force the GEMM kernel family.  1, 2 = 128x128 and 64x64 register-staged tiles; 6 =
  * weight-streaming kernel (256x96 tiles, two groups of waves taking turns on the K tiles, split K when N is small) for

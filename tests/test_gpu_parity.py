@@ -1094,6 +1094,34 @@ def test_linear_replays_from_a_captured_graph(M, N, K, entry):
         _ = (torch.randn(1024, device="cuda") * 2).sum().item()   # eager work between the replays
 
 
+def test_w6_scratch_of_the_caller_and_of_the_call():
+    """Both W6 linears with the caller's scratch (canaries behind it) and with one of their own: the same bits."""
+    M, N, K = 4096, 264, 512
+    A, xs = dev(rand_i8(10, 1, M, K, -127, 127)), dev(synth.uniform(10, 2, M, 0.01, 0.1))
+    wq, s_rel = dev(rand_i8(10, 3, N, K // 4 * 3, -128, 127)).view(torch.uint8), dev(synth.w6_srel_bytes(10, N, K, 32))
+    s_ch, sw = dev(synth.uniform(10, 4, N, 1e-3, 1e-2)), dev(synth.uniform(10, 5, N * (K // 128), 1e-3, 1e-2))
+    ptr, st = (lambda t: t.data_ptr()), torch.cuda.current_stream().cuda_stream
+    assert ffi.lib.gpu_w6a8_group_gemm_scratch(ptr(wq), M, N, K) == N * K
+    assert ffi.lib.gpu_w6a8_group_gemm_scratch(ptr(wq), M - 1, N, K) == 0 and ffi.lib.gpu_w6a8_group_gemm_scratch(ptr(wq), M, N, 100) == 0
+    for two_plane in (True, False):
+        outs = []
+        for own in (True, False):
+            D, w8 = torch.zeros((M, N), dtype=torch.bfloat16, device=DEV), torch.full((N * K + 64,), 77, dtype=torch.int8, device=DEV)
+            if two_plane:
+                a = (ptr(A), ptr(wq), ptr(s_rel), 32, ptr(xs), ptr(s_ch), 0, ptr(D))
+                tail = (M, N, K, BF16, st)
+                ffi.k("gpu_w6a8_gemm", *a, *tail) if own else ffi.k("gpu_w6a8_gemm_ws", *a, ptr(w8), *tail)
+            else:
+                a = (ptr(A), ptr(wq), ptr(xs), ptr(sw), 0, ptr(D), 0)
+                tail = (M, N, K, BF16, st)
+                ffi.k("gpu_w6a8_group_gemm", *a, *tail) if own else ffi.k("gpu_w6a8_group_gemm_ws", *a, ptr(w8), *tail)
+            torch.cuda.synchronize()
+            assert bool((w8[N * K:] == 77).all())
+            outs.append(D.view(torch.int16))
+        assert torch.equal(outs[0], outs[1])
+    assert ffi.raw("gpu_w6a8_gemm_ws", ptr(A), ptr(wq), ptr(s_rel), 32, ptr(xs), ptr(s_ch), 0, ptr(D), ptr(w8) + 8, M, N, K, BF16, st) == -1
+
+
 # ------------------------------------------------------------------------- W6A8, packed words + fp32 group scales
 W6G_CASES = [  # (M, N, K, out_dt, with_bias)
     (256, 128, 128, BF16, True), (100, 200, 256, BF16, False), (300, 136, 640, F32, True), (513, 260, 384, F16, True),
