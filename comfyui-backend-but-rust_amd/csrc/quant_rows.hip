@@ -648,6 +648,104 @@ int rotate_group(int rotate) { return rotate == 0 ? 0 : (rotate == 64 || rotate 
 
 bool known_prologue(int p) { return p >= PRO_PLAIN && p <= PRO_SITU_FAST && p != PRO_LN_AFFINE_SILU; }
 
+// One linear of a few rows in a launch: every workgroup quantizes the rows for itself (a wave per row, the code of the
+// quantizer above, so the codes are its codes) while its weights are on their way from HBM straight into the registers
+// that the matrix instruction reads, then multiplies them with 64 columns, 16 per wave.  Bound by latency: one trip to memory beside
+// the quantizer's chain of LDS round trips.  M=3, K=256 -> N=18432, us per linear replayed from a graph: 4.5, as a quantizer and
+// a GEMM 7.0; called from Python 12.4 and 20.5, host work.
+constexpr int kLinRows = 8, kLinK = 1024, kLinCols = 64;
+struct LinArgs {
+    const int8_t* W;
+    const float* ws;
+    const void* bias;
+    void* D;
+    int N;
+    bool vec_ok;   // four consecutive outputs, biases and scales are aligned vectors
+};
+template <int MODE, int G, int OUT_DT>
+__global__ void __launch_bounds__(256) linear_rows_kernel(QuantArgs p, LinArgs a) {
+    __shared__ __attribute__((aligned(16))) int8_t codes[kLinRows * kLinK];
+    __shared__ float xs[kLinRows];
+    __shared__ __attribute__((aligned(16))) float tiles[G ? 4 * kLdsPerWave : 1];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = lane & 15, quarter = lane >> 4;
+    const int nb = (int)blockIdx.x * kLinCols + wave * 16;
+    const int wrow = nb + row < a.N ? nb + row : a.N - 1;   // a row past the end is read as the last one and not stored
+    const v4i* src = reinterpret_cast<const v4i*>(a.W + (int64_t)wrow * p.K + quarter * 16);
+    v4i w[kLinK / 64];
+#pragma unroll
+    for (int k = 0; k < kLinK / 64; ++k)
+        if (k * 64 < p.K) w[k] = src[k * 4];
+    QuantArgs r = p;
+    r.q = codes;
+    r.scales = xs;
+    r.wpr = 1;
+    for (int m = wave; m < p.M; m += 4) {
+        float v[1][16];
+        if (lane * 16 < p.K) {
+            load16<MODE>(p.x, m * p.x_stride + lane * 16, v[0]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) v[0][i] = 0.f;
+        }
+        const float amax = wave_max_f32(rotate_and_max<MODE, G, 1>(r, v, m, true, 0, lane, tiles + (G ? wave * kLdsPerWave : 0), true));
+        store_codes<MODE, 1, false>(r, v, m, true, 0, lane, amax);
+    }
+    __syncthreads();
+    v4i acc{0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < kLinK / 64; ++k) {
+        if (k * 64 >= p.K) break;
+        v4i c{0, 0, 0, 0};
+        if (row < p.M) c = *reinterpret_cast<const v4i*>(codes + row * p.K + k * 64 + quarter * 16);
+        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[k], c, acc, 0, 0, 0);
+    }
+    // a lane holds row lane % 16 and the columns 4 * (lane / 16) + j
+    const int n = nb + 4 * quarter;
+    if (row >= p.M || n >= a.N) return;
+    const int64_t o = (int64_t)row * a.N + n;
+    float ws[4], b[4] = {0.f, 0.f, 0.f, 0.f}, out[4];
+    if (a.vec_ok) {
+        load4<DT_F32>(a.ws, n, ws);
+        if (a.bias) load4<OUT_DT>(a.bias, n, b);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            ws[j] = n + j < a.N ? a.ws[n + j] : 0.f;
+            if (a.bias && n + j < a.N) b[j] = ld_dt<OUT_DT>(a.bias, n + j);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) out[j] = __builtin_fmaf((float)acc[j] * xs[row], ws[j], b[j]);
+    if (a.vec_ok) {
+        store4<OUT_DT>(a.D, o, out);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) if (n + j < a.N) st_dt<OUT_DT>(a.D, o + j, out[j]);
+    }
+}
+
+template <int MODE, int G>
+int launch_linear_rows(const QuantArgs& q, const LinArgs& a, int out_dt, hipStream_t st) {
+    const dim3 grid((unsigned)((a.N + kLinCols - 1) / kLinCols));
+    if (out_dt == DT_F32) hipLaunchKernelGGL((linear_rows_kernel<MODE, G, DT_F32>), grid, dim3(256), 0, st, q, a);
+    else if (out_dt == DT_F16) hipLaunchKernelGGL((linear_rows_kernel<MODE, G, DT_F16>), grid, dim3(256), 0, st, q, a);
+    else hipLaunchKernelGGL((linear_rows_kernel<MODE, G, DT_BF16>), grid, dim3(256), 0, st, q, a);
+    KCHECK();
+    return 0;
+}
+template <int MODE>
+int run_linear_rows(const QuantArgs& q, const LinArgs& a, int g, int out_dt, hipStream_t st) {
+    return g == 0 ? launch_linear_rows<MODE, 0>(q, a, out_dt, st) : g == 64 ? launch_linear_rows<MODE, 64>(q, a, out_dt, st)
+         : g == 128 ? launch_linear_rows<MODE, 128>(q, a, out_dt, st) : launch_linear_rows<MODE, 256>(q, a, out_dt, st);
+}
+
+// Rows of at most one wave's chunk, few enough of them that quantizing them in every workgroup costs less than a launch: at
+// N=18432, one kernel against two, 8 rows 5.9 and 7.2 us (K=256), 9.7 and 10.9 (K=1024), 16 rows 8.9 and 7.3, 13.3 and 11.0.
+bool linear_in_one(const void* W, int dtype, int64_t M, int64_t N, int64_t K, int grp, int out_dt) {
+    return M > 0 && M <= kLinRows && K > 0 && K <= kLinK && K % (grp ? grp : 64) == 0 && N > 0 && N <= 0x7fffffff - kLinCols &&
+           (dtype == DT_BF16 || dtype == DT_F32) && out_dt >= DT_F32 && out_dt <= DT_BF16 && ((uintptr_t)W & 15) == 0;
+}
+
 }  // namespace
 
 GPU_API int gpu_quant_rows(int dtype, int prologue, const void* x, int64_t x_stride, const void* g, int64_t g_stride,
@@ -663,6 +761,25 @@ GPU_API int gpu_quant_rows(int dtype, int prologue, const void* x, int64_t x_str
                 mod_shift};
     if (dtype == DT_BF16 && M > 0) attach_tables(a, (hipStream_t)stream);
     return dtype == DT_BF16 ? run_quant<MODE_BF16>(a, grp, (hipStream_t)stream) : run_quant<MODE_F32>(a, grp, (hipStream_t)stream);
+}
+
+GPU_API int gpu_linear_w8a8(int dtype, const void* x, int64_t x_stride, const int8_t* W, const float* ws, const void* bias, void* D,
+                            void* scratch, int64_t M, int64_t N, int64_t K, int rotate, int out_dt, void* stream) {
+    const int grp = rotate_group(rotate);
+    hipStream_t st = (hipStream_t)stream;
+    if (linear_in_one(W, dtype, M, N, K, grp, out_dt)) {
+        const QuantArgs q{x, x_stride, nullptr, nullptr, nullptr, (int)M, (int)K, 1, 1, 0, PRO_PLAIN};
+        const uintptr_t size = out_dt == DT_F32 ? 4 : 2;
+        const LinArgs a{W, ws, bias, D, (int)N,
+                        N % 4 == 0 && (((uintptr_t)D | (uintptr_t)bias) & (4 * size - 1)) == 0 && ((uintptr_t)ws & 15) == 0};
+        return dtype == DT_BF16 ? run_linear_rows<MODE_BF16>(q, a, grp, out_dt, st) : run_linear_rows<MODE_F32>(q, a, grp, out_dt, st);
+    }
+    if (M < 0 || M > 0x7fffffff || K < 0 || K > 0x7fffffff) return -200;
+    int8_t* codes = (int8_t*)scratch;
+    float* xs = (float*)(codes + M * K);   // K % 64 == 0: aligned as scratch is
+    if (const int rc = gpu_quant_rows(dtype, PRO_PLAIN, x, x_stride, nullptr, 0, 0, nullptr, 0.f, nullptr, nullptr, codes, xs, (int)M, (int)K,
+                                      rotate, stream)) return rc;
+    return gpu_int8_gemm(codes, W, xs, ws, bias, D, M, N, K, out_dt, stream);
 }
 
 GPU_API int gpu_quant_rows_b(int dtype, int prologue, const void* x, int64_t x_stride, const float* norm_w,

@@ -38,6 +38,7 @@ SIGNATURES = {
     "gpu_w6_decode": [_P, _P, _P, _I64, _I32, _I32, _P],
     "gpu_int8_gemm_acc": [_P, _P, _P, _I64, _I64, _I64, _P],
     "gpu_int8_gemm_static": [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I32, _P],
+    "gpu_linear_w8a8": [_I32, _P, _I64, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I32, _I32, _P],
     "gpu_w6a8_gemm": [_P, _P, _P, _I32, _P, _P, _P, _P, _I64, _I64, _I64, _I32, _P],
     "gpu_w6a8_gemm_ws": [_P, _P, _P, _I32, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I32, _P],
     "gpu_w6a8_group_gemm_ws": [_P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I32, _P],

@@ -274,8 +274,19 @@ def w6a8_group_gemm(A, packed, xs, sw, bias=None, out_dtype=torch.bfloat16, want
 
 def linear_w8a8(x, W, ws, bias=None, rotate=0, out_dtype=None):
     """One W8A8 linear: y = dequant(quant(x) . W^T)."""
-    q, xs = quant_rows(x, rotate)
-    return int8_gemm(q, W, xs, ws, bias, x.dtype if out_dtype is None else out_dtype)
+    out_dtype = x.dtype if out_dtype is None else out_dtype
+    _rows(x)
+    _dense(W, ws, bias)
+    _want(W, torch.int8, "W"); _want(ws, torch.float32, "ws"); _want(bias, out_dtype, "bias")
+    M, K = x.shape
+    if W.dim() != 2 or W.shape[1] != K:
+        raise ValueError("x [M,K] and W [N,K] must share K, got %s and %s" % (tuple(x.shape), tuple(W.shape)))
+    N = W.shape[0]
+    D = torch.empty((M, N), dtype=out_dtype, device=x.device)
+    scratch = torch.empty((M * K + 4 * M,), dtype=torch.uint8, device=x.device)   # codes and row scales
+    ffi.k("gpu_linear_w8a8", _TORCH_DT[x.dtype], _ptr(x), x.stride(0), _ptr(W), _ptr(ws), _ptr(bias), _ptr(D), _ptr(scratch), M, N, K,
+          rotate, _TORCH_DT[out_dtype], _stream())
+    return D
 
 
 def _f32_vec(t, n, what):

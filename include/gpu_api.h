@@ -260,6 +260,12 @@ int gpu_int8_gemm_static(const int8_t* A, const int8_t* W, const float* xs, cons
                          int64_t M, int64_t N, int64_t K, int out_dt, void* stream);
 int64_t gpu_int8_gemm_static_limit(void);
 
+/* One W8A8 linear in a single call: gpu_quant_rows without a prologue, then gpu_int8_gemm, or both in one kernel for up to 8
+ * rows of K <= 1024.  Same bits.  scratch: M*K + 4*M bytes of device memory, 16-byte aligned, in use until the work queued
+ * here has run.  Return codes as the two calls'. */
+int gpu_linear_w8a8(int dtype, const void* x, int64_t x_stride, const int8_t* W, const float* ws, const void* bias, void* D,
+                    void* scratch, int64_t M, int64_t N, int64_t K, int rotate, int out_dt, void* stream);
+
 /* One W6A8 linear in a single call: gpu_w6_decode into a stream-ordered scratch buffer, then gpu_int8_gemm with
  * ws = s_channel (the call pattern of src/h3.rs:1208-1216,1251).  Returns -1 for K % 32 or G % 16, otherwise as
  * gpu_int8_gemm. */

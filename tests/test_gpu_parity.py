@@ -955,6 +955,43 @@ def test_config0_end_to_end_matches_golden_fixture():
     assert ulp_close(db.reshape(-1)[::s], nofma, BF16)
 
 
+LINEAR_ROWS = [  # (M, N, K, rotate, dtype, out_dt, with_bias): either side of 8 rows and of K = 1024, tails of the 64-column tiles
+    (1, 96, 64, 0, BF16, BF16, True), (3, 18432, 256, 256, BF16, BF16, True), (8, 8, 1024, 64, BF16, F32, False),
+    (8, 130, 768, 128, F32, BF16, True), (5, 67, 512, 256, F32, F32, True), (7, 1, 960, 0, BF16, F16, False),
+    (9, 130, 768, 128, F32, BF16, True), (8, 200, 1088, 64, BF16, F32, False), (300, 260, 1280, 256, BF16, BF16, True),
+]
+
+
+@pytest.mark.parametrize("M,N,K,rotate,dtype,out_dt,with_bias", LINEAR_ROWS)
+def test_linear_in_one_call(M, N, K, rotate, dtype, out_dt, with_bias):
+    """gpu_linear_w8a8 against the quantizer and the GEMM as two calls, bit for bit, and against the oracle: rows with a
+    stride, all-zero rows, infinities and NaN."""
+    say("linear", M, N, K, rotate, dtype, out_dt, with_bias)
+    v = synth.normal(12, 1, M * (K + 16)).reshape(M, K + 16).astype(np.float32)
+    v[0, :] = 0.0
+    if M > 2:
+        v[1, 3], v[2, 5] = np.inf, np.nan
+    x = dev(v).to(TDT[dtype])[:, :K]
+    W, ws = dev(rand_i8(12, 2, N, K, -128, 127)), dev(synth.uniform(12, 3, N, 1e-3, 1e-2))
+    bias = dev(synth.normal(12, 4, N).astype(np.float32)).to(TDT[out_dt]) if with_bias else None
+    got = ql.linear_w8a8(x, W, ws, bias, rotate, TDT[out_dt])
+    q, xs = ql.quant_rows(x, rotate, K)
+    want = ql.int8_gemm(q, W, xs, ws, bias, TDT[out_dt])
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+    xc = x.contiguous()
+    rc, ref, _ = oracle.linear_w8a8(dtype, host_bits(xc) if dtype == BF16 else xc.cpu().numpy(), rotate, W.cpu().numpy(), ws.cpu().numpy(),
+                                    None if bias is None else host_bits(bias), out_dt)
+    assert rc == 0
+    assert np.array_equal(host_bits(got).view(np.uint8), np.ascontiguousarray(ref).view(np.uint8))
+
+
+def test_linear_in_one_call_refuses_what_the_two_calls_refuse():
+    for dtype, M, N, K, rotate, out_dt, want in [(BF16, 4, 8, 100, 0, BF16, -1), (BF16, 4, 8, 128, 256, BF16, -1), (F16, 4, 8, 128, 0, BF16, -4),
+                                                 (BF16, 0, 8, 128, 0, BF16, 0), (BF16, 4, 8, 0, 0, BF16, -1), (BF16, -1, 8, 128, 0, BF16, -200)]:
+        assert ffi.raw("gpu_linear_w8a8", dtype, 0, K, 0, 0, 0, 0, 0, M, N, K, rotate, out_dt, 0) == want, (dtype, M, N, K, rotate, out_dt)
+
+
 # ------------------------------------------------------------------------------------------------ W6
 def test_w6_decode_exhaustive_and_random():
     K, G = 64, 16
