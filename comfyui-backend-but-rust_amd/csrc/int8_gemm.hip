@@ -1370,6 +1370,183 @@ __global__ void __launch_bounds__(TurnCfg::NT, 1) int8_gemm_turn_kernel(GemmArgs
     }
 }
 
+// Up to 128 rows: weights straight from HBM into the registers that the matrix instruction reads, rows of A through LDS.  The
+// kernel above moves all 256 rows of A to every CU for 96 columns of W, and what it moves bounds it; with M rows of A in
+// 16-row tiles (MT of them) the weights are most of what a CU takes in.
+//   * Eight waves; a wave owns 16 columns and one of NWK interleaved parts of K, so a workgroup covers 128 / NWK columns
+//     and walks K in panels of 512 * NWK (or 256).  The parts are added through LDS at the end.
+//   * W: a load is 16 columns x 64 bytes, an MFMA operand as it arrives.  Two panels of them are always in flight, each
+//     reissued as soon as its MFMAs have read it: 128 KB per CU (64), and no wait of one wave for another on the way.
+//   * A: the panel's rows by DMA into one of two stages, [128-byte column block][8 rows][128 bytes] with the chunk swizzle of
+//     the other kernels on the global side, a panel ahead; one barrier per panel.
+// The wait ahead of that barrier counts: the reissued W loads may stay in flight, the DMA before them may not.
+// Bound by HBM behind 5 us of launch and first trips.  us per call, weights from HBM, the better of the other kernels and this one:
+// 16 rows 1024 -> 1024 8.1 and 5.9, 4096 -> 4096 13.4 and 8.3, 12288 -> 4096 22.1 and 16.7, 4096 -> 16384 26.2 and 20.1; 64 rows
+// 8.3 and 5.2, 14.7 and 11.7, 22.9 and 20.0, 26.8 and 22.9; 128 rows 8.3 and 8.0, 16.1 and 16.4, 25.6 and 23.9, 27.4 and 24.0.
+// Eight steps of 64 per panel where two stages fit the LDS, else four: with NWK = 1 instead, 77 rows take 16.6 instead of 13.8 us
+// for 4096 -> 4096.
+template <int MT, int NWK>
+struct RowsCfg {
+    static constexpr int NT = 512, NWN = 8 / NWK, BN = 16 * NWN, RB = 2 * MT;
+    static constexpr int SP = MT * NWK <= 8 ? 8 : 4;   // steps of 64 per wave and panel; two stages have to fit the LDS
+    static constexpr int KP = 64 * SP * NWK, NLA = KP / 128 * RB / 8;
+    static constexpr int STAGE = KP / 128 * RB * 1024, SMEM = 2 * STAGE;
+};
+template <int MT, int NWK, int OUT_DT, int EPI>
+__global__ void __launch_bounds__(512, (MT * NWK <= 4 ? 4 : 2)) int8_gemm_rows_kernel(GemmArgs p, bool vec_ok) {
+    using C = RowsCfg<MT, NWK>;
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, quarter = lane >> 4;
+    const int wn = wave % C::NWN, wk = wave / C::NWN;
+    const int kb0 = (int)blockIdx.y * p.kslice;
+    const int k1 = p.kslice && kb0 + p.kslice < p.K ? kb0 + p.kslice : p.K;
+    const int nb = (int)blockIdx.x * C::BN + wn * 16;
+    const int wrow = nb + l16 < p.N ? nb + l16 : p.N - 1;   // columns past the end read the last one and are not stored
+    const uint32_t woff = (uint32_t)wrow * (uint32_t)p.K + quarter * 16;
+    const int np = (k1 - kb0 + C::KP - 1) / C::KP;
+    const uint32_t lds_base = (uint32_t)(uintptr_t)smem;
+
+    uint32_t ga[C::NLA];
+#pragma unroll
+    for (int j = 0; j < C::NLA; ++j) {
+        const int rb = (wave + 8 * j) % C::RB;
+        const int row = rb * 8 + (lane >> 3) < p.M ? rb * 8 + (lane >> 3) : p.M - 1;
+        ga[j] = (uint32_t)row * (uint32_t)p.K + (((lane & 7) ^ ((rb & 1) * 4 + (lane >> 4))) * 16);
+    }
+    const auto fetch_a = [&](int panel) {
+#pragma unroll
+        for (int j = 0; j < C::NLA; ++j) {
+            const int blk = wave + 8 * j;
+            const int k = kb0 + panel * C::KP + blk / C::RB * 128;   // a block past the end is fetched from the last one and not used
+            const int8_t* base = p.A + (k < k1 ? k : k1 - 128);
+            const uint32_t dst = lds_base + (panel & 1) * C::STAGE + blk * 1024;
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(ga[j]), "s"(base) : "memory", "m0");
+        }
+    };
+    const auto fetch_w = [&](int panel, int i) {
+        const int k = kb0 + panel * C::KP + (wk * C::SP + i) * 64;
+        return *reinterpret_cast<const v4i*>(p.W + (k < k1 ? k : k1 - 64) + (uint64_t)woff);
+    };
+    v4i w[2][C::SP], acc[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[t] = v4i{0, 0, 0, 0};
+    // the epilogue's constants first, so that their trip is over when they are used; then the longest trips
+    const int n = nb + 4 * quarter;   // a lane ends up with the columns n..n+3 of row lane % 16 of the row tiles
+    typedef uint32_t raw4 __attribute__((ext_vector_type(dt_size<OUT_DT>::value)));   // four outputs' worth, as it lies in memory
+    float4 ws4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    raw4 b4 = 0, rs4 = 0;
+    float xs[MT];
+    if (EPI != EPI_ACC) {
+        if (vec_ok && n < p.N) {
+            ws4 = *reinterpret_cast<const float4*>(p.ws + n);
+            if (p.bias) b4 = *reinterpret_cast<const raw4*>((const uint8_t*)p.bias + (int64_t)n * dt_size<OUT_DT>::value);
+            if (EPI == EPI_RESID) rs4 = *reinterpret_cast<const raw4*>((const uint8_t*)p.rscale + (int64_t)n * dt_size<OUT_DT>::value);
+        }
+#pragma unroll
+        for (int t = 0; t < MT; ++t) xs[t] = p.xs[t * 16 + l16 < p.M ? t * 16 + l16 : p.M - 1];
+    }
+    SCHED_FENCE();
+#pragma unroll
+    for (int i = 0; i < C::SP; ++i) w[0][i] = fetch_w(0, i);
+    SCHED_FENCE();
+    fetch_a(0);
+    SCHED_FENCE();
+#pragma unroll
+    for (int i = 0; i < C::SP; ++i) w[1][i] = fetch_w(1, i);
+    SCHED_FENCE();
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(C::SP) : "memory");
+
+    const auto panel_step = [&](int panel, auto set_tag, auto whole_tag) {
+        constexpr int set = decltype(set_tag)::value, whole = decltype(whole_tag)::value;
+        if (panel + 1 < np) fetch_a(panel + 1);
+        SCHED_FENCE();
+        const uint8_t* st = smem + set * C::STAGE + (l16 >> 3) * 1024 + (l16 & 7) * 128;
+#pragma unroll
+        for (int i = 0; i < C::SP; ++i) {
+            const int ks = wk * C::SP + i;
+            if (whole || kb0 + panel * C::KP + ks * 64 < k1) {
+                const uint8_t* f = st + (ks >> 1) * (C::RB * 1024) + ((((i & 1) * 4 + quarter) ^ (l16 >> 1)) * 16);
+                v4i a[MT];
+#pragma unroll
+                for (int t = 0; t < MT; ++t) a[t] = *reinterpret_cast<const v4i*>(f + t * 2048);
+                SCHED_FENCE();   // one trip to LDS for all of them
+#pragma unroll
+                for (int t = 0; t < MT; ++t) acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[set][i], a[t], acc[t], 0, 0, 0);
+            }
+            if constexpr (whole) {
+                SCHED_FENCE();
+                w[set][i] = fetch_w(panel + 2, i);
+                SCHED_FENCE();
+            }
+        }
+        if constexpr (whole) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(C::SP) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        SCHED_FENCE();
+    };
+    // whole panels in pairs without a way out between them, which would cost the compiler its count of the loads in flight
+    int panel = 0;
+    for (const int pairs_end = (k1 - kb0) / C::KP & ~1; panel < pairs_end; panel += 2) {
+        panel_step(panel, ic<0>{}, ic<1>{});
+        panel_step(panel + 1, ic<1>{}, ic<1>{});
+    }
+    if (panel < np) {
+        panel_step(panel, ic<0>{}, ic<0>{});
+        if (panel + 1 < np) panel_step(panel + 1, ic<1>{}, ic<0>{});
+    }
+
+    const auto finish = [&](const v4i& sum, int t, float x) {
+        const int m = t * 16 + l16;
+        if (m >= p.M || n >= p.N) return;
+        const int64_t o = (int64_t)m * p.N + n;
+        if (EPI == EPI_ACC) {
+            int* d = (int*)p.D + (int64_t)blockIdx.y * p.M * p.N + o;
+            if (vec_ok) *reinterpret_cast<v4i*>(d) = sum;
+            else
+#pragma unroll
+                for (int j = 0; j < 4; ++j) if (n + j < p.N) d[j] = sum[j];
+            return;
+        }
+        float ws[4] = {ws4.x, ws4.y, ws4.z, ws4.w}, b[4] = {0.f, 0.f, 0.f, 0.f}, rs[4] = {0.f, 0.f, 0.f, 0.f}, res[4] = {0.f, 0.f, 0.f, 0.f}, out[4];
+        if (vec_ok) {
+            load4<OUT_DT>(&b4, 0, b);
+            load4<OUT_DT>(&rs4, 0, rs);
+            if (EPI == EPI_RESID) load4<OUT_DT>(p.resid, o, res);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (n + j >= p.N) continue;
+                ws[j] = p.ws[n + j];
+                if (p.bias) b[j] = ld_dt<OUT_DT>(p.bias, n + j);
+                if (EPI == EPI_RESID) { rs[j] = ld_dt<OUT_DT>(p.rscale, n + j); res[j] = ld_dt<OUT_DT>(p.resid, o + j); }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) out[j] = epi_value<OUT_DT, EPI>(sum[j], x, ws[j], b[j], rs[j], res[j]);
+        if (vec_ok) store4<OUT_DT>(p.D, o, out);
+        else
+#pragma unroll
+            for (int j = 0; j < 4; ++j) if (n + j < p.N) st_dt<OUT_DT>(p.D, o + j, out[j]);
+    };
+    if constexpr (NWK == 1) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) finish(acc[t], t, EPI == EPI_ACC ? 0.f : xs[t]);
+    } else {
+        v4i* red = reinterpret_cast<v4i*>(smem) + lane;   // [part of K][16 columns][row tile][lane]
+#pragma unroll
+        for (int t = 0; t < MT; ++t) red[(wave * MT + t) * 64] = acc[t];
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            if (t % NWK != wk) continue;
+            v4i sum = red[(wn * MT + t) * 64];
+#pragma unroll
+            for (int q = 1; q < NWK; ++q) sum += red[((q * C::NWN + wn) * MT + t) * 64];
+            finish(sum, t, EPI == EPI_ACC ? 0.f : xs[t]);
+        }
+    }
+}
+
 // Sum of the int32 planes of a split-K run, then the epilogue.  planes[s][M][N]; four consecutive n per thread.
 template <int OUT_DT, int EPI>
 __global__ void __launch_bounds__(256) splitk_epilogue_kernel(GemmArgs p, const int* planes, int slices) {
@@ -1621,25 +1798,11 @@ int launch_stream(GemmArgs a, int slices, hipStream_t st) {
     return 0;
 }
 
-// M <= 256: one row of 256 x 96 tiles, the weights are read once and the run is bound by how fast they stream.  When N
-// is too small to give every CU a column slab, K is split as well: each slice writes an int32 plane (exact, so the
-// order of the sum does not matter) into the stream's scratch buffer and a second kernel adds the planes and applies
-// the epilogue.
-template <int OUT_DT, int EPI>
-int launch_skinny(GemmArgs a, hipStream_t st) {
-    bool vec_ok, aligned;
-    epilogue_alignment<OUT_DT, EPI>(a, vec_ok, aligned);
-    if (!aligned) return launch_cfg<CfgM, OUT_DT, EPI>(a, st);
+// A run on `slices` slices of kslice values of K: `body` writes the int32 planes, a second kernel adds them (exact, so the order of
+// the sum does not matter) and applies the epilogue.
+template <int OUT_DT, int EPI, class Body>
+int launch_split(const GemmArgs& a, int slices, int kslice, hipStream_t st, Body body) {
     const int num_cu = device_cu_count();
-    const int t96 = (a.N + 95) / 96, nk = a.K / 128;
-    int slices = t96 * 4 >= num_cu * 3 ? 1 : num_cu / t96;
-    if (slices > nk) slices = nk;
-    if (slices > 1) {
-        const int per = (nk + slices - 1) / slices;   // K tiles per slice
-        slices = (nk + per - 1) / per;                // no empty slice
-    }
-    if (slices <= 1) return launch_stream<OUT_DT, EPI>(a, 1, st);
-    const int per = (nk + slices - 1) / slices;
     const size_t need = (size_t)slices * a.M * a.N * sizeof(int);
     int* planes = nullptr;
     bool own = false;   // planes come from the stream-ordered pool and go back to it
@@ -1661,8 +1824,8 @@ int launch_skinny(GemmArgs a, hipStream_t st) {
     }
     GemmArgs pa = a;
     pa.D = planes;
-    pa.kslice = per * 128;
-    int rc = launch_stream<DT_F32, EPI_ACC>(pa, slices, st);
+    pa.kslice = kslice;
+    int rc = body(pa);
     if (rc == 0) {
         const int64_t nvec = (int64_t)a.M * a.N / 4;
         const unsigned grid = (unsigned)((nvec + 255) / 256 < 4096 ? (nvec + 255) / 256 : 4096);
@@ -1677,6 +1840,85 @@ int launch_skinny(GemmArgs a, hipStream_t st) {
     return rc;
 }
 
+// M <= 256: one row of 256 x 96 tiles, the weights are read once and the run is bound by how fast they stream.  When N
+// is too small to give every CU a column slab, K is split as well: each slice writes an int32 plane (exact, so the
+// order of the sum does not matter) into the stream's scratch buffer and a second kernel adds the planes and applies
+// the epilogue.
+template <int OUT_DT, int EPI>
+int launch_skinny(GemmArgs a, hipStream_t st) {
+    bool vec_ok, aligned;
+    epilogue_alignment<OUT_DT, EPI>(a, vec_ok, aligned);
+    if (!aligned) return launch_cfg<CfgM, OUT_DT, EPI>(a, st);
+    const int num_cu = device_cu_count();
+    const int t96 = (a.N + 95) / 96, nk = a.K / 128;
+    int slices = t96 * 4 >= num_cu * 3 ? 1 : num_cu / t96;
+    if (slices > nk) slices = nk;
+    if (slices > 1) {
+        const int per = (nk + slices - 1) / slices;   // K tiles per slice
+        slices = (nk + per - 1) / per;                // no empty slice
+    }
+    if (slices <= 1) return launch_stream<OUT_DT, EPI>(a, 1, st);
+    const int per = (nk + slices - 1) / slices;
+    return launch_split<OUT_DT, EPI>(a, slices, per * 128, st, [&](const GemmArgs& pa) { return launch_stream<DT_F32, EPI_ACC>(pa, slices, st); });
+}
+
+template <int MT, int NWK, int OUT_DT, int EPI>
+int launch_rows_cfg(const GemmArgs& a, bool vec_ok, int slices, hipStream_t st) {
+    using C = RowsCfg<MT, NWK>;
+    auto kern = int8_gemm_rows_kernel<MT, NWK, OUT_DT, EPI>;
+    static PerDeviceOnce once;
+    if (const int e = allow_dynamic_lds((const void*)kern, C::SMEM, once)) return e;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((a.N + C::BN - 1) / C::BN), (unsigned)slices), dim3(C::NT), C::SMEM, st, a, vec_ok);
+    KCHECK();
+    return 0;
+}
+template <int OUT_DT_, int EPI>
+int launch_rows_as(const GemmArgs& a, int mt, int nwk, bool vec_ok, int slices, hipStream_t st) {
+    constexpr int OUT_DT = EPI == EPI_ACC ? DT_F32 : OUT_DT_;   // int32 sums have no output type
+    switch (mt * 10 + nwk) {
+        case 12: return launch_rows_cfg<1, 2, OUT_DT, EPI>(a, vec_ok, slices, st);
+        case 14: return launch_rows_cfg<1, 4, OUT_DT, EPI>(a, vec_ok, slices, st);
+        case 18: return launch_rows_cfg<1, 8, OUT_DT, EPI>(a, vec_ok, slices, st);
+        case 22: return launch_rows_cfg<2, 2, OUT_DT, EPI>(a, vec_ok, slices, st);
+        case 24: return launch_rows_cfg<2, 4, OUT_DT, EPI>(a, vec_ok, slices, st);
+        case 42: return launch_rows_cfg<4, 2, OUT_DT, EPI>(a, vec_ok, slices, st);
+        case 44: return launch_rows_cfg<4, 4, OUT_DT, EPI>(a, vec_ok, slices, st);
+        case 62: return launch_rows_cfg<6, 2, OUT_DT, EPI>(a, vec_ok, slices, st);
+        default: return launch_rows_cfg<8, 2, OUT_DT, EPI>(a, vec_ok, slices, st);
+    }
+}
+
+// K that a split over workgroups has to take off each of them to be worth the planes and the second launch, about 4 us (rows
+// 77, us unsplit and split: 1536 -> 4608 9.1 and 11.2, 3072 -> 3072 15.0 and 12.1; rows 64: 3072 -> 3072 in two 9.3 and 10.9,
+// 4096 -> 4096 in two 12.3 and 11.7).
+constexpr int kSplitRowsK = 1800;
+
+// M <= 128.  The widest split of K inside the workgroup that still gives every CU at most one workgroup; where even that
+// leaves CUs without one, K is split over workgroups as well.
+template <int OUT_DT, int EPI>
+int launch_rows(GemmArgs a, hipStream_t st) {
+    bool vec_ok, aligned;
+    epilogue_alignment<OUT_DT, EPI>(a, vec_ok, aligned);
+    const int cus = device_cu_count();
+    const int mt = a.M <= 16 ? 1 : a.M <= 32 ? 2 : a.M <= 64 ? 4 : a.M <= 96 ? 6 : 8;
+    const auto tiles = [&](int nwk) { return (int)(((int64_t)a.N * nwk + 127) / 128); };
+    const int most = mt == 1 ? 8 : mt <= 4 ? 4 : 2;
+    int nwk = 2;
+    while (nwk < most && tiles(2 * nwk) <= cus) nwk *= 2;
+    if (mt == 1 && tiles(2) > cus) nwk = 4;   // several rounds: the smaller tiles fill the last one better
+    const int unit = 64 * nwk * (mt * nwk <= 8 ? 8 : 4), panels = (a.K + unit - 1) / unit;
+    int slices = vec_ok ? cus / tiles(nwk) : 1;
+    if (slices > panels) slices = panels;
+    if (slices > 1 && a.K / slices * (slices - 1) < kSplitRowsK) slices = 1;
+    if (slices <= 1) {
+        a.kslice = 0;
+        return launch_rows_as<OUT_DT, EPI>(a, mt, nwk, vec_ok, 1, st);
+    }
+    const int per = (panels + slices - 1) / slices;
+    slices = (panels + per - 1) / per;   // no empty slice
+    return launch_split<OUT_DT, EPI>(a, slices, per * unit, st, [&](const GemmArgs& pa) { return launch_rows_as<DT_F32, EPI_ACC>(pa, mt, nwk, true, slices, st); });
+}
+
 // Kernel family forced by the test hook (-1 = choose by shape).  Process-wide and only meant for tests and benchmarks:
 // relaxed atomic, so a concurrent call sees either the old or the new value, never a torn one.
 std::atomic<int> g_force_cfg{-1};
@@ -1684,8 +1926,14 @@ std::atomic<int> g_force_cfg{-1};
 int choose_cfg(int64_t M, int64_t N, int64_t K) {
     const int force = g_force_cfg.load(std::memory_order_relaxed);
     const bool dma_ok = M * K < ((int64_t)1 << 32) && N * K < ((int64_t)1 << 32);   // 32-bit lane offsets
+    if (force == 5) return dma_ok && (K % 128) == 0 && M <= 128 ? 5 : 1;
     if (force == 6 || force == 7 || force == 9) return (dma_ok && (K % 128) == 0) ? force : 1;
     if (force == 1 || force == 2) return force;
+    // Up to 128 rows: from K = 768 on (1024 for the most rows; below, the small register-staged tiles have less to start) and up
+    // to the 16384 columns that give every CU one workgroup of the tallest split.  Beyond those the streaming kernel's 96-wide
+    // tiles fill the CUs as well and its W rows come in whole lines (4096 -> 24576, us, this and that: 1 row 29.1 and 30.6, 32 rows
+    // 35.3 and 30.6, 128 rows 42.8 and 31.5; 3072 -> 18432, 16 rows 18.0 and 21.1).
+    if (M <= 128 && (K % 128) == 0 && K >= (M > 96 ? 1024 : 768) && dma_ok && (M <= 16 || N <= 16384)) return 5;
     if (M <= 256 && N >= 1024 && (K % 128) == 0 && K >= 512 && dma_ok) {
         // The weight-streaming kernel pays a fixed price per call (a prologue that waits for HBM, two launches when K
         // is split), which long K repays and short K does not.  Measured with weights from HBM, M = 16..256, K =
@@ -1715,6 +1963,7 @@ int choose_cfg(int64_t M, int64_t N, int64_t K) {
 template <int OUT_DT, int EPI>
 int dispatch_cfg(const GemmArgs& a, hipStream_t st) {
     switch (choose_cfg(a.M, a.N, a.K)) {
+        case 5: return launch_rows<OUT_DT, EPI>(a, st);
         case 6: return launch_skinny<OUT_DT, EPI>(a, st);
         case 7: return launch_ring_small<OUT_DT, EPI>(a, st);
         case 9: return launch_pp<OUT_DT, EPI>(a, st);
@@ -1916,7 +2165,7 @@ GPU_API int gpu_int8_gemm_acc(const int8_t* A, const int8_t* W, int32_t* acc, in
     return rc < 0 ? -200 : rc;
 }
 
-// Test hook: force a kernel family (1 = 128x128, 2 = 64x64 register-staged tiles; 6 = weight streaming; 7 = persistent
+// Test hook: force a kernel family (1 = 128x128, 2 = 64x64 register-staged tiles; 5 = up to 128 rows; 6 = weight streaming; 7 = persistent
 // ring, 128x192; 9 = two-group kernel; -1 or anything else = automatic).
 GPU_API int gpu_int8_gemm_force_config(int cfg) {
     g_force_cfg.store(cfg, std::memory_order_relaxed);

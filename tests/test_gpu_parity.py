@@ -773,6 +773,37 @@ def test_int8_gemm_acc_bit_exact(M, N, K, cfg):
     assert np.array_equal(got.cpu().numpy(), want)
 
 
+# Edges of the kernel for up to 128 rows: its row tiles (16, 32, 64, 96, 128), columns past the last tile and unaligned ones, K
+# shorter than a panel, panels with a remainder, an odd and an even number of them, and K split over workgroups
+ROWS_CASES = [(1, 8, 128), (15, 67, 768), (16, 1000, 4096), (17, 96, 1152), (32, 4100, 896), (33, 72, 2176), (64, 130, 1024), (65, 4096, 896),
+              (77, 1024, 3712), (96, 264, 640), (97, 96, 1280), (128, 2048, 4224), (16, 16416, 1024), (5, 4097, 2304)]
+
+
+@pytest.mark.parametrize("M,N,K", ROWS_CASES)
+def test_int8_gemm_up_to_128_rows(M, N, K):
+    say("gemm rows", M, N, K)
+    A, W = rand_i8(14, 500 + M, M, K), rand_i8(14, 600 + N, N, K)
+    A[0, :] = -128
+    W[N - 1, :] = -128
+    xs, ws = synth.uniform(14, 3, M, 0.005, 0.2), synth.uniform(14, 4, N, 1e-3, 1e-2)
+    want = oracle.int8_gemm_acc(A, W)
+    Ad, Wd, xd, wd = dev(A), dev(W), dev(xs), dev(ws)
+    for cfg in (5, -1):
+        ffi.raw("gpu_int8_gemm_force_config", cfg)
+        try:
+            assert np.array_equal(ql.int8_gemm_acc(Ad, Wd).cpu().numpy(), want), cfg
+            for dt, tob in ((BF16, oracle.bf16_bits), (F16, oracle.f16_bits), (F32, lambda a: a.astype(np.float32))):
+                bias, rs = tob(synth.normal(14, 5, N) * np.float32(0.02)), tob(synth.normal(14, 6, N))
+                resid = tob(synth.normal(14, 7, M * N).reshape(M, N))
+                for b in (None, bias):
+                    d = ql.int8_gemm(Ad, Wd, xd, wd, None if b is None else dev_bits(b, dt), TDT[dt])
+                    assert np.array_equal(host_bits(d), oracle.epilogue(want, xs, ws, b, dt, fma=1)), (cfg, dt)
+                r = ql.int8_gemm_residual(Ad, Wd, xd, wd, dev_bits(bias, dt), dev_bits(rs, dt), dev_bits(resid, dt))
+                assert np.array_equal(host_bits(r), oracle.epilogue_residual(want, xs, ws, bias, rs, resid, dt, fma=1)), (cfg, dt)
+        finally:
+            ffi.raw("gpu_int8_gemm_force_config", -1)
+
+
 # K % 16 == 8: the reference's alignment-8 configurations (csrc/vendor/cutlass_gemm_int8.cu:191,237-247)
 @pytest.mark.parametrize("M,N,K", [(5, 40, 8), (130, 264, 136), (300, 1030, 1000), (64, 2048, 4104)])
 def test_int8_gemm_k_multiple_of_8_only(M, N, K):
