@@ -1754,6 +1754,13 @@ std::mutex g_planes_mu;
 StreamPlanes g_planes[kStreamPlanes];
 int g_planes_n = 0;
 
+bool is_capturing(hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;   // not known: taken as one
+}
+
 void* stream_planes(hipStream_t st, size_t need, int num_cu) {
     if (st == hipStreamPerThread) return nullptr;   // one handle, a different stream in every thread: nothing to key on
     int dev = 0;
@@ -1763,11 +1770,7 @@ void* stream_planes(hipStream_t st, size_t need, int num_cu) {
         if (g_planes[i].dev == dev && g_planes[i].st == st) return need <= g_planes[i].bytes ? g_planes[i].ptr : nullptr;
     const size_t bytes = (size_t)num_cu * TurnCfg::BN * TurnCfg::BM * sizeof(int);
     if (g_planes_n == kStreamPlanes || need > bytes) return nullptr;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
+    if (is_capturing(st)) return nullptr;
     void* ptr = nullptr;
     if (hipMalloc(&ptr, bytes) != hipSuccess) {
         (void)hipGetLastError();
@@ -1914,6 +1917,9 @@ int launch_rows(GemmArgs a, hipStream_t st) {
         a.kslice = 0;
         return launch_rows_as<OUT_DT, EPI>(a, mt, nwk, vec_ok, 1, st);
     }
+    // Narrow outputs never split K before this kernel, so a captured graph of them held no address of the stream's planes (it may
+    // be replayed on any stream) and the static entry point left its buffer alone: both stay so.
+    if (a.N < 1024 && (tl_scratch != nullptr || is_capturing(st))) return launch_cfg<CfgS, OUT_DT, EPI>(a, st);
     const int per = (panels + slices - 1) / slices;
     slices = (panels + per - 1) / per;   // no empty slice
     return launch_split<OUT_DT, EPI>(a, slices, per * unit, st, [&](const GemmArgs& pa) { return launch_rows_as<DT_F32, EPI_ACC>(pa, mt, nwk, true, slices, st); });
@@ -1923,17 +1929,19 @@ int launch_rows(GemmArgs a, hipStream_t st) {
 // relaxed atomic, so a concurrent call sees either the old or the new value, never a torn one.
 std::atomic<int> g_force_cfg{-1};
 
-int choose_cfg(int64_t M, int64_t N, int64_t K) {
+// `whole` = A and W start at 16-byte addresses, what the kernel for up to 128 rows asks of its DMA and its weight loads; an
+// operand that starts elsewhere (a view into a larger buffer) goes to the kernels that such calls had without it.
+int choose_cfg(int64_t M, int64_t N, int64_t K, bool whole) {
     const int force = g_force_cfg.load(std::memory_order_relaxed);
     const bool dma_ok = M * K < ((int64_t)1 << 32) && N * K < ((int64_t)1 << 32);   // 32-bit lane offsets
-    if (force == 5) return dma_ok && (K % 128) == 0 && M <= 128 ? 5 : 1;
+    if (force == 5) return dma_ok && whole && (K % 128) == 0 && M <= 128 ? 5 : 1;
     if (force == 6 || force == 7 || force == 9) return (dma_ok && (K % 128) == 0) ? force : 1;
     if (force == 1 || force == 2) return force;
     // Up to 128 rows: from K = 768 on (1024 for the most rows; below, the small register-staged tiles have less to start) and up
     // to the 16384 columns that give every CU one workgroup of the tallest split.  Beyond those the streaming kernel's 96-wide
     // tiles fill the CUs as well and its W rows come in whole lines (4096 -> 24576, us, this and that: 1 row 29.1 and 30.6, 32 rows
     // 35.3 and 30.6, 128 rows 42.8 and 31.5; 3072 -> 18432, 16 rows 18.0 and 21.1).
-    if (M <= 128 && (K % 128) == 0 && K >= (M > 96 ? 1024 : 768) && dma_ok && (M <= 16 || N <= 16384)) return 5;
+    if (M <= 128 && (K % 128) == 0 && K >= (M > 96 ? 1024 : 768) && dma_ok && whole && (M <= 16 || N <= 16384)) return 5;
     if (M <= 256 && N >= 1024 && (K % 128) == 0 && K >= 512 && dma_ok) {
         // The weight-streaming kernel pays a fixed price per call (a prologue that waits for HBM, two launches when K
         // is split), which long K repays and short K does not.  Measured with weights from HBM, M = 16..256, K =
@@ -1962,7 +1970,7 @@ int choose_cfg(int64_t M, int64_t N, int64_t K) {
 
 template <int OUT_DT, int EPI>
 int dispatch_cfg(const GemmArgs& a, hipStream_t st) {
-    switch (choose_cfg(a.M, a.N, a.K)) {
+    switch (choose_cfg(a.M, a.N, a.K, (((uintptr_t)a.A | (uintptr_t)a.W) & 15) == 0)) {
         case 5: return launch_rows<OUT_DT, EPI>(a, st);
         case 6: return launch_skinny<OUT_DT, EPI>(a, st);
         case 7: return launch_ring_small<OUT_DT, EPI>(a, st);

@@ -1162,6 +1162,24 @@ def test_linear_replays_from_a_captured_graph(M, N, K, entry):
         _ = (torch.randn(1024, device="cuda") * 2).sum().item()   # eager work between the replays
 
 
+@pytest.mark.parametrize("M,N,K,entry", [(16, 512, 4096, "gpu_int8_gemm"),            # K split when run eagerly, not in a graph
+                                           (77, 4096, 1152, "gpu_int8_gemm"),           # kernel for up to 128 rows, whole K
+                                           (128, 960, 8192, "gpu_int8_gemm_static")])   # narrow: leaves the static planes alone
+def test_few_rows_replay_from_a_captured_graph(M, N, K, entry):
+    test_linear_replays_from_a_captured_graph(M, N, K, entry)
+
+
+# Up to 128 rows and operands that start inside a larger buffer: only 16-byte starts go to the kernel that asks for them
+@pytest.mark.parametrize("off_a,off_w", [(8, 0), (0, 8), (16, 16)])
+@pytest.mark.parametrize("M,N,K", [(3, 512, 1024), (128, 320, 4096)])
+def test_int8_gemm_few_rows_from_inside_a_buffer(M, N, K, off_a, off_w):
+    say("gemm rows offset", M, N, K, off_a, off_w)
+    A, W = rand_i8(15, 1, M, K), rand_i8(15, 2, N, K)
+    Ad = torch.zeros(M * K + 32, dtype=torch.int8, device="cuda")[off_a:off_a + M * K].view(M, K).copy_(dev(A))
+    Wd = torch.zeros(N * K + 32, dtype=torch.int8, device="cuda")[off_w:off_w + N * K].view(N, K).copy_(dev(W))
+    assert np.array_equal(ql.int8_gemm_acc(Ad, Wd).cpu().numpy(), oracle.int8_gemm_acc(A, W))
+
+
 def test_w6_scratch_of_the_caller_and_of_the_call():
     """Both W6 linears with the caller's scratch (canaries behind it) and with one of their own: the same bits."""
     M, N, K = 4096, 264, 512
