@@ -45,21 +45,15 @@ struct QuantArgs {
 enum { PRO_SD_GEGLU = 101, PRO_SD_UNPAD = 102, PRO_SD_GN = 103 };
 
 // csrc/kernels.cu:1355-1359
-__device__ __forceinline__ uint32_t pcg_hash(uint32_t x) {
-    const uint32_t state = x * 747796405u + 2891336453u;
+constexpr uint32_t kPcgMul = 747796405u, kPcgAdd = 2891336453u;
+__device__ __forceinline__ uint32_t pcg_hash_state(uint32_t state) {   // state: x * kPcgMul + kPcgAdd
     const uint32_t word = ((state >> ((state >> 28u) + 4u)) ^ state) * 277803737u;
     return (word >> 22u) ^ word;
 }
-// a + b of two bf16 values rounded once to bf16, what the bf16 add instruction behind __hadd gives
-// (csrc/kernels.cu:1341-1343): the exact sum fits a double, which is then cut to 8 significant bits, ties to even.
-__device__ __forceinline__ float bf16_add_once(float a, float b) {
-    const double s = (double)a + (double)b;
-    uint64_t u = __builtin_bit_cast(uint64_t, s);
-    const uint64_t rem = u & ((1ull << 45) - 1), half = 1ull << 44;
-    u >>= 45;
-    if (rem > half || (rem == half && (u & 1))) ++u;
-    return (float)__builtin_bit_cast(double, u << 45);
-}
+// a + b of two bf16 values rounded once to bf16, what the bf16 add instruction behind __hadd gives (csrc/kernels.cu:1341-1343).
+// The fp32 sum rounds first and changes nothing: it is inexact only where the smaller operand is below 2^-15 of the larger,
+// which leaves the sum 2^-10 (relative) or more away from every midpoint of two bf16 values.
+__device__ __forceinline__ float bf16_add_once(float a, float b) { return rnd_dt<DT_BF16>(a + b); }
 
 template <int MODE> __device__ __forceinline__ void load16(const void* x, int64_t off, float* v) {
     if (MODE == MODE_BF16) {
@@ -165,12 +159,18 @@ __device__ __forceinline__ void store_codes(const QuantArgs& p, float (&v)[C][16
     }
     if (row_ok && wr == 0 && lane == 0) p.scales[m] = scale;
 
-    const auto store = [&](auto rcp_tag) {
+        // Stochastic rounding: the hash of element index + seed, its halves folded, starts with a product.  Where a row's keys stay
+    // below 2^32 the fold changes nothing and a lane's 16 products differ by constants.  With that, the fp32 addition above
+    // (fp64 and 64-bit integers before) and the clamp in the pack conversion 12288 x 3072 bf16 takes 42 us instead of 53, bound
+    // by vector instructions as the plain quantizer is (38 us for as many values).
+    const uint64_t key0 = (uint64_t)(m * (int64_t)p.K) + p.seed;
+    const auto store = [&](auto fast_tag) {
 #pragma unroll
         for (int c = 0; c < C; ++c) {
             const int e0 = (wr + c * p.wpr) * kChunk + lane * 16;
             if (!(row_ok && e0 < p.K)) continue;
             uint32_t w[4];
+            const uint32_t state0 = ((uint32_t)key0 + (uint32_t)e0) * kPcgMul + kPcgAdd;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if constexpr (MODE == MODE_SD_F16) {
@@ -182,7 +182,7 @@ __device__ __forceinline__ void store_codes(const QuantArgs& p, float (&v)[C][16
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
                         const float x = v[c][4 * i + j];
-                        if constexpr (decltype(rcp_tag)::value) {
+                        if constexpr (decltype(fast_tag)::value) {
                             const float q0 = x * rinv;
                             qt[j] = __builtin_fmaf(__builtin_fmaf(-q0, st, x), rinv, q0);
                         } else {
@@ -213,11 +213,16 @@ __device__ __forceinline__ void store_codes(const QuantArgs& p, float (&v)[C][16
                         t = x / st;
                     }
                     if (SR && (MODE == MODE_BF16 || MODE == MODE_F32)) {   // csrc/kernels.cu:1385-1388
-                        const uint64_t key = (uint64_t)(m * (int64_t)p.K + e0 + 4 * i + j) + p.seed;
-                        const float noise = (float)(pcg_hash((uint32_t)key ^ (uint32_t)(key >> 32)) >> 8) * 0x1.0p-24f;
+                        uint32_t state;
+                        if constexpr (decltype(fast_tag)::value) {
+                            state = state0 + (uint32_t)(4 * i + j) * kPcgMul;
+                        } else {
+                            const uint64_t key = key0 + e0 + 4 * i + j;
+                            state = ((uint32_t)key ^ (uint32_t)(key >> 32)) * kPcgMul + kPcgAdd;
+                        }
+                        const float noise = (float)(pcg_hash_state(state) >> 8) * 0x1.0p-24f;
                         const float r = floorf(MODE == MODE_F32 ? t + noise : bf16_add_once(t, rnd_dt<DT_BF16>(noise)));
-                        const int qi = (int)fminf(127.f, fmaxf(-128.f, r));
-                        acc |= ((uint32_t)qi & 0xffu) << (8 * j);
+                        acc = __builtin_amdgcn_cvt_pk_u8_f32(r + 128.f, j, acc);   // the clamp as below; r is a whole number
                     } else if (MODE == MODE_F32) {
                         const int qi = (int)fminf(127.f, fmaxf(-128.f, nearbyintf(t)));
                         acc |= ((uint32_t)qi & 0xffu) << (8 * j);
@@ -229,13 +234,16 @@ __device__ __forceinline__ void store_codes(const QuantArgs& p, float (&v)[C][16
                         acc = __builtin_amdgcn_cvt_pk_u8_f32(t + 128.f, j, acc);
                     }
                 }
-                w[i] = (!SR && MODE != MODE_F32) ? acc ^ 0x80808080u : acc;
+                w[i] = (SR || MODE != MODE_F32) ? acc ^ 0x80808080u : acc;
             }
             *reinterpret_cast<uint4*>(p.q + m * (int64_t)p.K + e0) = make_uint4(w[0], w[1], w[2], w[3]);
         }
     };
     if constexpr (MODE == MODE_SD_F16) {
         if (by_rcp) store(std::true_type{});
+        else store(std::false_type{});
+    } else if constexpr (SR) {
+        if (key0 < ((uint64_t)1 << 32) - (uint64_t)p.K) store(std::true_type{});
         else store(std::false_type{});
     } else {
         store(std::true_type{});

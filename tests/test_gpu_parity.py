@@ -494,6 +494,24 @@ def test_convrot_requant_bit_exact(N, K, dt):
     assert ffi.raw("gpu_convrot_requant", 0, xd.data_ptr(), qd.data_ptr(), sd.data_ptr(), N, 300, 0, 0) == -1
 
 
+# Keys (element index + seed) on either side of 2^32 and of 2^64, inside a row and inside a lane's sixteen values: the hash has
+# a short form where a row's keys stay below 2^32
+@pytest.mark.parametrize("dt", [BF16, F32])
+@pytest.mark.parametrize("N,K", [(5, 256), (4, 9216)])
+def test_convrot_requant_seeds_at_the_edges(N, K, dt):
+    say("convrot_requant seeds", N, K, dt)
+    w = synth.normal(61 + K, 1, N * K).reshape(N, K) * np.float32(0.05)
+    w[1, :K // 2] *= np.float32(1e-6)   # small next to the noise
+    x = synth.bf16_bits(w) if dt == BF16 else w
+    xd = dev_bits(x, dt)
+    for seed in (2 ** 32 - 2 * K, 2 ** 32 - 2 * K - 7, 2 ** 32 - 2 * K + 1, 2 ** 32, 2 ** 64 - K - 5, 2 ** 64 - 1):
+        rc, q, s = oracle.convrot_requant(dt, x, seed)
+        qd, sd = ql.convrot_requant(xd, seed)
+        assert rc == 0
+        assert np.array_equal(sd.cpu().numpy().view(np.uint32), s.view(np.uint32)), seed
+        assert np.array_equal(qd.cpu().numpy(), q), seed
+
+
 @pytest.mark.parametrize("N,K", [(5, 256), (33, 3072), (3, 13824), (300, 512)])
 def test_w6_requant_bit_exact(N, K):
     say("w6_requant", N, K)
