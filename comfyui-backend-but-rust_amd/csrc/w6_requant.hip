@@ -51,10 +51,12 @@ __device__ __forceinline__ float pair_lane(float x) {
 
 // Four values of a group -> their code bytes (level index + 1), :63-80,126-148.  Wanted is the pair of neighbouring levels
 // with level(l) < t <= level(l + 1), l in -31..30 (ends beyond t count as bracketing it).  Any f in -30..30 next to the
-// pair settles it by one look: l is f when level(f) is below t, else f - 1; the sign of level(f) - t stands for the compare.
+// pair settles it by one look: l is f when level(f) is below t, else f - 1.
 //   plain (every lane's step in [1, 4], every |t| < 127): f = rint(t / s).  f s is within s/2 of t and a level within 1/2
 //     of its product, so level(f - 1) < t <= level(f + 1) for s >= 1, whichever way t / s falls at a tie; no level
-//     reaches the clamp at +-127; and f s is a 6-bit times a 4-bit number, so adding 1.5 * 2^23 rounds it as rint does.
+//     reaches the clamp at +-127; and f s is a 6-bit times a 4-bit number, so adding 1.5 * 2^23 rounds it as rint does.  The
+//     sign of level(f) - t stands for the compare: a level of zero is +0 here.  (Below, it can be -0, and -0 - (+0) has the sign
+//     of a smaller level: steps below 1/62 around a zero value, i.e. zero blocks in a row that is not zero.)
 //   else: levels are whole numbers, so the first level at or above t is the first that reaches ceil(t), i.e. whose product
 //     reaches ceil(t) - 1/2 (or passes it, where that tie rounds down to an even number).  With z that quotient, rint(z) is
 //     that position or the one before it: a whole z needs the tie looked at, any other is farther from a whole number
@@ -72,7 +74,7 @@ __device__ __forceinline__ uint32_t codes4(const float* v, float inv_sc, float s
         else f = t > 127.f ? 30.f : t <= -127.f ? -30.f : __builtin_rintf((__builtin_ceilf(t) - 0.5f) * inv_s);
         f = __builtin_amdgcn_fmed3f(f, -30.f, 30.f);
         lf = PLAIN ? __builtin_fmaf(f, s, M) - M : level(f, s);
-        const float g = f - __builtin_copysignf(1.f, lf - t);                     // the pair's other end
+        const float g = PLAIN ? f - __builtin_copysignf(1.f, lf - t) : lf < t ? f + 1.f : f - 1.f;   // the pair's other end
         lg = PLAIN ? __builtin_fmaf(g, s, M) - M : level(g, s);
         const uint32_t h = x0 + kc[j];                                            // x * 747796405 + 2891336453, :21-25
         const uint32_t w = ((h >> ((h >> 28u) + 4u)) ^ h) * 277803737u;

@@ -561,6 +561,27 @@ def test_w6_requant_row_lengths_and_grid_ends(N, K):
         assert np.array_equal(pd.cpu().numpy(), packed)
 
 
+@pytest.mark.parametrize("N,K", [(4, 512), (3, 1280), (2, 16640)])
+def test_w6_requant_zero_blocks_and_small_groups(N, K):
+    """Blocks of 256 zeros in rows that are not zero: their step against the row's scale rounds to 0 or to one of the smallest
+    e4m3 numbers, where every level of the grid is zero, of either sign."""
+    w = synth.normal(91 + K, 1, N * K).reshape(N, K) * np.float32(0.04)
+    w[0, :256] = 0
+    w[1, K - 256:] = -0.0
+    w[N - 1, 256:512] *= np.float32(2.0 ** -7)      # a step of about 1/30 of the row's scale
+    w[N - 1, 256:258] = 0
+    wb = synth.bf16_bits(w)
+    for seed in (0, 5, 2 ** 40 + 3):
+        say("w6_requant zeros", N, K, seed)
+        rc, packed, s_rel, s_ch = oracle.w6_requant(wb, seed)
+        pd, rd, cd = ql.w6_requant(dev_bits(wb, BF16), seed)
+        torch.cuda.synchronize()
+        assert rc == 0 and (s_rel == 0).any()
+        assert np.array_equal(cd.cpu().numpy().view(np.uint32), s_ch.view(np.uint32))
+        assert np.array_equal(rd.cpu().numpy(), s_rel)
+        assert np.array_equal(pd.cpu().numpy(), packed)
+
+
 def test_checkpoint_linears_run_like_the_reference_sequence(tmp_path):
     """Weights as the reference's checkpoints store them (safetensors: int8 ConvRot with row scales, W6 triplet, dense),
     loaded and run through quantize -> GEMM; int8 and W6 outputs bit-exact against the oracle's sequence."""
