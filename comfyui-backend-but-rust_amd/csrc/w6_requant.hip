@@ -61,6 +61,8 @@ __device__ __forceinline__ float pair_lane(float x) {
 //     reaches ceil(t) - 1/2 (or passes it, where that tie rounds down to an even number).  With z that quotient, rint(z) is
 //     that position or the one before it: a whole z needs the tie looked at, any other is farther from a whole number
 //     than the last bit of the division reaches.  Outside [-127, 127] every level is on one side of t: an end of the grid.
+//     NaN: a value's is the middle of the grid (the reference's conversion of the estimate to an integer gives 0) and above
+//     no threshold; a step's (an infinite row scale) makes every level -127, the clamp's lower end.
 // `x0` is the hash input of value 0 without its low four bits' share, kc[j] that share (see the caller).
 template <bool PLAIN>
 __device__ __forceinline__ uint32_t codes4(const float* v, float inv_sc, float s, float inv_s, uint32_t x0, const uint32_t* kc) {
@@ -71,16 +73,17 @@ __device__ __forceinline__ uint32_t codes4(const float* v, float inv_sc, float s
         const float t = v[j] * inv_sc;
         float f, lf, lg;
         if (PLAIN) f = __builtin_fmaf(t, inv_s, M) - M;
-        else f = t > 127.f ? 30.f : t <= -127.f ? -30.f : __builtin_rintf((__builtin_ceilf(t) - 0.5f) * inv_s);
-        f = __builtin_amdgcn_fmed3f(f, -30.f, 30.f);
+        else f = t > (s != s ? -127.f : 127.f) ? 30.f : t <= -127.f ? -30.f : __builtin_rintf((__builtin_ceilf(t) - 0.5f) * inv_s);
+        f = PLAIN || t == t ? __builtin_amdgcn_fmed3f(f, -30.f, 30.f) : 0.f;
         lf = PLAIN ? __builtin_fmaf(f, s, M) - M : level(f, s);
         const float g = PLAIN ? f - __builtin_copysignf(1.f, lf - t) : lf < t ? f + 1.f : f - 1.f;   // the pair's other end
         lg = PLAIN ? __builtin_fmaf(g, s, M) - M : level(g, s);
         const uint32_t h = x0 + kc[j];                                            // x * 747796405 + 2891336453, :21-25
         const uint32_t w = ((h >> ((h >> 28u) + 4u)) ^ h) * 277803737u;
         const float u = (float)(((w >> 22u) ^ w) >> 8) * (1.0f / 16777216.0f);    // :27-31
-        const float d = __builtin_fmaf(u, fabsf(lg - lf), fminf(lf, lg)) - t;     // negative where t is above the threshold
-        out = __builtin_amdgcn_cvt_pk_u8_f32(fminf(f, g) - __builtin_copysignf(0.5f, d) + 32.25f, j, out);
+        const float thr = __builtin_fmaf(u, fabsf(lg - lf), fminf(lf, lg));
+        const float half = PLAIN ? __builtin_copysignf(0.5f, thr - t) : t > thr ? -0.5f : 0.5f;   // negative where t is above the threshold
+        out = __builtin_amdgcn_cvt_pk_u8_f32(fminf(f, g) - half + 32.25f, j, out);
     }
     return out;
 }
@@ -158,7 +161,7 @@ __global__ void __launch_bounds__(1024) w6_requant_kernel(const uint16_t* w, uin
         // value's (a NaN takes -31 in the reference's clamp)
         amax = fmaxf(amax, (nan ? 31.0f : fminf(31.0f, __builtin_rintf(m * inv))) * step);
         gs[c] = step;
-        gmax[c] = m;
+        gmax[c] = nan ? __builtin_inff() : m;   // a group with a NaN is not for the plain form of codes4
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));

@@ -461,8 +461,8 @@ static inline float w6_level(int i, float s) {                                  
     return fmin_dev(127.f, fmax_dev(-127.f, nearbyintf((float)(i - 31) * s)));
 }
 static inline int w6_lower_bound(float t, float s, float inv_s) {                 /* :63-69 */
-    const float est = nearbyintf((ceilf(t) - 0.5f) * inv_s);                      /* __float2int_rn saturates */
-    int i = (est > 2.0e9f ? 2000000000 : est < -2.0e9f ? -2000000000 : (int)est) + 31;
+    const float est = nearbyintf((ceilf(t) - 0.5f) * inv_s);                      /* __float2int_rn saturates, NaN gives 0 */
+    int i = (est != est ? 0 : est > 2.0e9f ? 2000000000 : est < -2.0e9f ? -2000000000 : (int)est) + 31;
     i = i < 0 ? 0 : i > 63 ? 63 : i;
     while (i > 0 && w6_level(i - 1, s) >= t) --i;
     while (i < 63 && w6_level(i, s) < t) ++i;

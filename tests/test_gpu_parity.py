@@ -582,6 +582,28 @@ def test_w6_requant_zero_blocks_and_small_groups(N, K):
         assert np.array_equal(pd.cpu().numpy(), packed)
 
 
+@pytest.mark.parametrize("N,K", [(6, 512), (7, 1280)])
+def test_w6_requant_not_finite(N, K):
+    """NaN, infinities of one and of both signs, and finite weights whose rotation or step overflows, beside ordinary rows."""
+    w = synth.normal(92 + K, 1, N * K).reshape(N, K) * np.float32(0.04)
+    w[0, 3] = np.nan
+    w[1, K - 7] = np.inf
+    w[2, 5], w[2, 9] = np.inf, -np.inf
+    w[3, :] *= np.float32(2.0 ** 130)
+    w[4, :256] = np.float32(2.0 ** 124)
+    wb = synth.bf16_bits(w)
+    for seed in (0, 5):
+        say("w6_requant not finite", N, K, seed)
+        with np.errstate(all="ignore"):
+            rc, packed, s_rel, s_ch = oracle.w6_requant(wb, seed)
+        pd, rd, cd = ql.w6_requant(dev_bits(wb, BF16), seed)
+        torch.cuda.synchronize()
+        assert rc == 0
+        assert np.array_equal(cd.cpu().numpy().view(np.uint32), s_ch.view(np.uint32))
+        assert np.array_equal(rd.cpu().numpy() & 0x7F, s_rel & 0x7F)   # the sign of a NaN is the processor's
+        assert np.array_equal(pd.cpu().numpy(), packed)
+
+
 def test_checkpoint_linears_run_like_the_reference_sequence(tmp_path):
     """Weights as the reference's checkpoints store them (safetensors: int8 ConvRot with row scales, W6 triplet, dense),
     loaded and run through quantize -> GEMM; int8 and W6 outputs bit-exact against the oracle's sequence."""
