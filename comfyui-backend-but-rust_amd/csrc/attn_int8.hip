@@ -1200,7 +1200,8 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) ro[x][i] *= f;
         }
-        const float t_scale = __builtin_amdgcn_exp2f(tile_m - m);
+        // a NaN maximum (every key scale of the tile infinite): the tile's probabilities are 0 and its factor 1, so that it drops out
+        const float t_scale = tile_m == tile_m ? __builtin_amdgcn_exp2f(tile_m - m) : 1.f;
 
         v4i pf[NB];
         uint32_t psum = 0;

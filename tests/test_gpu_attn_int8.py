@@ -639,3 +639,24 @@ def test_attention_head_dims_64_and_256(case):
     ex = _exact(q, k, v, scale)
     cos = float((got * ex).sum() / np.sqrt((got * got).sum() * (ex * ex).sum()))
     assert cos > 0.9995, cos
+
+
+@pytest.mark.parametrize("D,lk,dtype,at", [(64, 200, torch.bfloat16, 0), (64, 1500, torch.float16, 1), (128, 400, torch.bfloat16, 1),
+                                           (128, 1300, torch.bfloat16, 0), (128, 1300, torch.float16, 1), (256, 400, torch.bfloat16, 1)])
+def test_attention_drops_a_tile_of_infinite_keys(D, lk, dtype, at):
+    """Every key scale of a tile infinite: its maximum is NaN, its probabilities are 0, and the rows are what they are without the
+    tile, bit for bit (its values are zeros, so that the scales of V agree) and against the oracle."""
+    ql, ffi = _pkg()
+    dt = oracle.BF16 if dtype == torch.bfloat16 else oracle.F16
+    q, k, v = _inputs(1, 70, lk, 2, 1, dtype, seed=D + lk + at, D=D)
+    ck = 128 if lk > 1024 and D != 64 else 64
+    drop = slice(at * ck, (at + 1) * ck)
+    k[:, drop, :, 5], v[:, drop] = float("inf"), 0
+    keep = torch.ones(lk, dtype=torch.bool)
+    keep[drop] = False
+    k2, v2 = k[:, keep].contiguous(), v[:, keep].contiguous()
+    got, want = (_bits(ql.int8_attn(q.cuda(), a.cuda(), b.cuda(), D ** -0.5)) for a, b in ((k, v), (k2, v2)))
+    assert np.array_equal(got, want)
+    ref = _to_f32(oracle.attn_int8(dt, _bits(q), _bits(k2), _bits(v2), D ** -0.5), dt)
+    tol = 2 * float(v.float().abs().max()) / 255.0 + 2 * 2.0 ** (-8 if dt == oracle.BF16 else -11) * np.abs(ref)   # as above
+    assert (np.abs(_to_f32(got, dt) - ref) <= tol).all()
