@@ -1191,14 +1191,17 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
         // The running base m only moves when a tile's maximum has outgrown it by 2^60 (and at the first tile): numerator and
         // denominator are both relative to it, so any base gives the same quotient, and the outputs need no rescaling here.
         if (__builtin_amdgcn_ballot_w64(tile_m - m > 60.f)) {
-            const float f = tile_m > m ? __builtin_amdgcn_exp2f(m - tile_m) : 1.f;
+            // in two factors (the second is 1 down to 2^-120): what the base lags behind is in the outputs, so that one factor can
+            // be below fp32's range where the product is not
+            const float step = tile_m > m ? m - tile_m : 0.f, most = fmax_nn(step, -120.f);
+            const float f = __builtin_amdgcn_exp2f(most), f2 = __builtin_amdgcn_exp2f(step - most);
             m = fmax_nn(m, tile_m);
-            dsum *= f;
-            dsum2 *= f;
+            dsum = dsum * f * f2;
+            dsum2 = dsum2 * f * f2;
 #pragma unroll
             for (int x = 0; x < NS; ++x)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) ro[x][i] *= f;
+                for (int i = 0; i < 16; ++i) ro[x][i] = ro[x][i] * f * f2;
         }
         // a NaN maximum (every key scale of the tile infinite): the tile's probabilities are 0 and its factor 1, so that it drops out
         const float t_scale = tile_m == tile_m ? __builtin_amdgcn_exp2f(tile_m - m) : 1.f;

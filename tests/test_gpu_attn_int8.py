@@ -660,3 +660,29 @@ def test_attention_drops_a_tile_of_infinite_keys(D, lk, dtype, at):
     ref = _to_f32(oracle.attn_int8(dt, _bits(q), _bits(k2), _bits(v2), D ** -0.5), dt)
     tol = 2 * float(v.float().abs().max()) / 255.0 + 2 * 2.0 ** (-8 if dt == oracle.BF16 else -11) * np.abs(ref)   # as above
     assert (np.abs(_to_f32(got, dt) - ref) <= tol).all()
+
+
+def _keys_by_level(lk, levels, seed, D=128):
+    """q near ones, keys near a multiple of ones that scores levels[i] (in powers of two) in key tile i, the last level from there
+    on, and positive values (each output has a relative error then)."""
+    g = torch.Generator().manual_seed(seed)
+    q = (1 + 0.02 * torch.randn(1, 40, 2, D, generator=g)).bfloat16()
+    unit = 1.0 / (D ** 0.5 * 1.4426950408889634)        # key level that scores 1 against a query of ones at scale D^-0.5
+    ck = 128 if lk > 1024 and D != 64 else 64
+    level = torch.tensor([levels[min(i // ck, len(levels) - 1)] for i in range(lk)])
+    k = (level[:, None, None] * unit * (1 + 0.02 * torch.randn(lk, 1, D, generator=g))).unsqueeze(0).bfloat16()
+    return q, k, (1 + torch.rand(1, lk, 1, D, generator=g)).bfloat16()
+
+
+@pytest.mark.parametrize("lk,levels", [(200, (-150.0, -100.0)), (1300, (-150.0, -100.0)), (200, (-120.0, -70.0)), (200, (-130.0, -90.0, -40.0))])
+def test_attention_scores_far_below_the_last_tiles_floor(lk, levels):
+    """The last tile's maximum starts at a raw score of -50000, which can lie far above every score there is: what the tiles
+    before gave is scaled down by that distance and counts all the same.  A sink of no weight turns the anchor off.  Tolerance:
+    four probabilities one u8 step (of 255) away at values of 1..2, and the output's rounding."""
+    ql, ffi = _pkg()
+    q, k, v = _keys_by_level(lk, levels, seed=lk)
+    scale, sink = 128 ** -0.5, 1e-38
+    ref = _to_f32(oracle.attn_int8(oracle.BF16, _bits(q), _bits(k), _bits(v), scale, use_anchor=False, sink=sink), oracle.BF16)
+    got = _to_f32(_bits(ql.int8_attn_sink(q.cuda(), k.cuda(), v.cuda(), scale, sink)), oracle.BF16)
+    assert (ref > 0.9).all()
+    assert (np.abs(got - ref) <= (2 * 4 / 255.0 + 2 * 2.0 ** -8) * ref).all()
