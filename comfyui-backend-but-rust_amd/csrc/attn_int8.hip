@@ -1289,8 +1289,20 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
     tile(a.kb - 1, std::true_type{});
 
     float dtot = swap32_sum(dsum + dsum2);
-    // `sink` more keys of score zero and value zero: each adds exp2(0 - m) to the denominator, nothing to the output
-    if (a.sink != 0.f) dtot = fmaf(a.sink, __builtin_amdgcn_exp2f(-m), dtot);
+    // `sink` more keys of score zero and value zero: each adds exp2(0 - m) to the denominator, nothing to the output.  The base can
+    // be 60 below the largest score, which would take that out of fp32's range where the score's own distance from zero does not.
+    if (a.sink != 0.f) {
+        if (m < -64.f) {
+            const float f = __builtin_amdgcn_exp2f(m + 64.f);
+            m = -64.f;
+            dtot *= f;
+#pragma unroll
+            for (int x = 0; x < NS; ++x)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) ro[x][i] *= f;
+        }
+        dtot = fmaf(a.sink, __builtin_amdgcn_exp2f(-m), dtot);
+    }
     const float rcp = 1.f / dtot;
     if (r < a.lq) {
         const int64_t ob = bi * a.o_bs + (int64_t)r * a.o_rs + hi * a.o_hs;

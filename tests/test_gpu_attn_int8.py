@@ -686,3 +686,16 @@ def test_attention_scores_far_below_the_last_tiles_floor(lk, levels):
     got = _to_f32(_bits(ql.int8_attn_sink(q.cuda(), k.cuda(), v.cuda(), scale, sink)), oracle.BF16)
     assert (ref > 0.9).all()
     assert (np.abs(got - ref) <= (2 * 4 / 255.0 + 2 * 2.0 ** -8) * ref).all()
+
+
+@pytest.mark.parametrize("lk", [200, 1300])
+@pytest.mark.parametrize("levels", [(-150.0, -100.0), (-120.0, -70.0), (-70.0, -20.0)])
+def test_attention_sink_far_above_every_key(levels, lk):
+    """All scores far below the sink's zero: each output is a tiny multiple of the values, exact to the tolerance of the test above."""
+    ql, ffi = _pkg()
+    q, k, v = _keys_by_level(lk, levels, seed=lk)
+    scale, sink = 128 ** -0.5, 3.0
+    ref = _to_f32(oracle.attn_int8(oracle.BF16, _bits(q), _bits(k), _bits(v), scale, use_anchor=False, sink=sink), oracle.BF16)
+    got = _to_f32(_bits(ql.int8_attn_sink(q.cuda(), k.cuda(), v.cuda(), scale, sink)), oracle.BF16)
+    assert (ref > 0).all() and (ref < 1e-3).all()
+    assert (np.abs(got - ref) <= (2 * 4 / 255.0 + 2 * 2.0 ** -8) * ref).all()
