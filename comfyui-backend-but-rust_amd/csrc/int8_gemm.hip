@@ -1742,7 +1742,8 @@ void retain_pool_memory() {
 // call and kept until the process ends.  Work on one stream is ordered, so its calls can share a buffer, and a
 // stream-ordered allocation per call costs about 7 us on the stream's timeline (measured: 31 against 24 us per call at
 // M=256, K=12288, N=4096).  The buffer has the one size every shape that the dispatcher splits fits into (slices *
-// column tiles <= CUs, so slices * N <= CUs * 96, times 256 rows of int32: 24 MiB on 256 CUs) and is never grown or
+// column tiles <= CUs: slices * N <= CUs * 96 times 256 rows of int32 in the streaming kernel, 24 MiB on 256 CUs, and
+// CUs * 64 times 128 rows in the kernel for up to 128) and is never grown or
 // freed, so a captured graph that holds its address stays valid.  At most kStreamPlanes streams per process are served;
 // a call on any further stream, a first call made under capture, or a shape beyond the size (a forced configuration)
 // falls back to a stream-ordered allocation, and so does hipStreamPerThread (one handle for a different stream in every
@@ -1917,9 +1918,11 @@ int launch_rows(GemmArgs a, hipStream_t st) {
         a.kslice = 0;
         return launch_rows_as<OUT_DT, EPI>(a, mt, nwk, vec_ok, 1, st);
     }
-    // Narrow outputs never split K before this kernel, so a captured graph of them held no address of the stream's planes (it may
-    // be replayed on any stream) and the static entry point left its buffer alone: both stay so.
-    if (a.N < 1024 && (tl_scratch != nullptr || is_capturing(st))) return launch_cfg<CfgS, OUT_DT, EPI>(a, st);
+    // Outputs that are narrow, or whose rows or pointers are not whole 16 bytes, do not split K in the streaming kernel either
+    // (choose_cfg, launch_skinny).  A captured graph of them holds no address of the stream's planes, so that it may be replayed on any
+    // stream, and the static entry point leaves its buffer alone: they take the register-staged tiles there.
+    if ((a.N < 1024 || !aligned) && (tl_scratch != nullptr || is_capturing(st)))
+        return a.N < 1024 ? launch_cfg<CfgS, OUT_DT, EPI>(a, st) : launch_cfg<CfgM, OUT_DT, EPI>(a, st);
     const int per = (panels + slices - 1) / slices;
     slices = (panels + per - 1) / per;   // no empty slice
     return launch_split<OUT_DT, EPI>(a, slices, per * unit, st, [&](const GemmArgs& pa) { return launch_rows_as<DT_F32, EPI_ACC>(pa, mt, nwk, true, slices, st); });

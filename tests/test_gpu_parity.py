@@ -3,6 +3,7 @@
 Bars: int8 codes, per-row scales and int32 accumulators bit-exact; bf16/f16/f32 outputs bit-exact against the oracle's
 fused-multiply-add epilogue and within one unit in the last place of the output type of its unfused form.
 """
+import ctypes as C
 import hashlib
 import json
 import os
@@ -1228,6 +1229,55 @@ def test_linear_replays_from_a_captured_graph(M, N, K, entry):
                                            (128, 960, 8192, "gpu_int8_gemm_static")])   # narrow: leaves the static planes alone
 def test_few_rows_replay_from_a_captured_graph(M, N, K, entry):
     test_linear_replays_from_a_captured_graph(M, N, K, entry)
+
+
+def _nodes_of_capture(call):
+    """Nodes of the graph that call(stream) records, which is not run."""
+    path = next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64.so" in l)   # the runtime that is loaded
+    hip, stream, graph, n = C.CDLL(path), torch.cuda.Stream(), C.c_void_p(), C.c_size_t()
+    st = C.c_void_p(stream.cuda_stream)
+    assert hip.hipStreamBeginCapture(st, 1) == 0         # thread-local
+    try:
+        call(stream.cuda_stream)
+    finally:
+        assert hip.hipStreamEndCapture(st, C.byref(graph)) == 0
+    assert hip.hipGraphGetNodes(graph, None, C.byref(n)) == 0 and hip.hipGraphDestroy(graph) == 0
+    return n.value
+
+
+@pytest.mark.parametrize("entry", ["gpu_int8_gemm", "gpu_int8_gemm_static"])
+@pytest.mark.parametrize("M,N,K,out_dt,off,split", [
+    (64, 2048, 4096, BF16, 0, True), (64, 2052, 4096, F32, 0, True),                                    # whole 16 bytes
+    (64, 1028, 4096, BF16, 0, False), (64, 2052, 4096, F16, 0, False), (16, 1036, 12288, BF16, 0, False),   # rows of whole 8 bytes
+    (64, 1024, 4096, BF16, 4, False), (128, 2048, 8192, BF16, 4, False),                                # an output 8 bytes off
+    (64, 512, 4096, BF16, 0, False)])                                                                   # narrow
+def test_captured_few_row_calls_that_share_no_planes(M, N, K, out_dt, off, split, entry):
+    """Made eagerly all of these split K.  In a graph those that are narrow or not of whole 16 bytes are one kernel node (no planes of
+    the stream or of the static array); and the eager call, the replayed one and the oracle agree."""
+    say("graph nodes", M, N, K, out_dt, off, entry)
+    A, W = rand_i8(16, 1, M, K), rand_i8(16, 2, N, K)
+    xs, ws = synth.uniform(16, 3, M, 0.005, 0.2), synth.uniform(16, 4, N, 1e-3, 1e-2)
+    Ad, Wd, xd, wd = dev(A), dev(W), dev(xs), dev(ws)
+    D = torch.zeros(M * N + off, dtype=TDT[out_dt], device=DEV)[off:].view(M, N)
+
+    def call(stream):
+        ffi.k(entry, Ad.data_ptr(), Wd.data_ptr(), xd.data_ptr(), wd.data_ptr(), 0, D.data_ptr(), M, N, K, out_dt, stream)
+
+    want = oracle.epilogue(oracle.int8_gemm_acc(A, W), xs, ws, None, out_dt, fma=1)
+    call(torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert np.array_equal(host_bits(D), want)
+    assert (_nodes_of_capture(call) > 1) == split
+    if split:
+        return
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(torch.cuda.current_stream().cuda_stream)
+    for _ in range(2):
+        D.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(host_bits(D), want)
 
 
 # Up to 128 rows and operands that start inside a larger buffer: only 16-byte starts go to the kernel that asks for them
