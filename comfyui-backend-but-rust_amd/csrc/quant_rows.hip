@@ -783,10 +783,12 @@ GPU_API int gpu_linear_w8a8(int dtype, const void* x, int64_t x_stride, const in
         return dtype == DT_BF16 ? run_linear_rows<MODE_BF16>(q, a, grp, out_dt, st) : run_linear_rows<MODE_F32>(q, a, grp, out_dt, st);
     }
     if (M < 0 || M > 0x7fffffff || K < 0 || K > 0x7fffffff) return -200;
+    const bool refuse = M > 0 && (!scratch || ((uintptr_t)scratch & 15));   // after what the quantizer refuses, of no rows
     int8_t* codes = (int8_t*)scratch;
     float* xs = (float*)(codes + M * K);   // K % 64 == 0: aligned as scratch is
-    if (const int rc = gpu_quant_rows(dtype, PRO_PLAIN, x, x_stride, nullptr, 0, 0, nullptr, 0.f, nullptr, nullptr, codes, xs, (int)M, (int)K,
-                                      rotate, stream)) return rc;
+    if (const int rc = gpu_quant_rows(dtype, PRO_PLAIN, x, x_stride, nullptr, 0, 0, nullptr, 0.f, nullptr, nullptr, codes, xs,
+                                      refuse ? 0 : (int)M, (int)K, rotate, stream)) return rc;
+    if (refuse) return -1;
     return gpu_int8_gemm(codes, W, xs, ws, bias, D, M, N, K, out_dt, stream);
 }
 

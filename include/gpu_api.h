@@ -261,8 +261,8 @@ int gpu_int8_gemm_static(const int8_t* A, const int8_t* W, const float* xs, cons
 int64_t gpu_int8_gemm_static_limit(void);
 
 /* One W8A8 linear in a single call: gpu_quant_rows without a prologue, then gpu_int8_gemm, or both in one kernel for up to 8
- * rows of K <= 1024.  Same bits.  scratch: M*K + 4*M bytes of device memory, 16-byte aligned, in use until the work queued
- * here has run.  Return codes as the two calls'. */
+ * rows of K <= 1024, which needs no scratch.  Same bits.  scratch: M*K + 4*M bytes of device memory, 16-byte aligned (-1 where it is
+ * needed and is not, or is null), in use until the work queued here has run.  Other return codes as the two calls'. */
 int gpu_linear_w8a8(int dtype, const void* x, int64_t x_stride, const int8_t* W, const float* ws, const void* bias, void* D,
                     void* scratch, int64_t M, int64_t N, int64_t K, int rotate, int out_dt, void* stream);
 

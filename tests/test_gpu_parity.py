@@ -1085,6 +1085,22 @@ def test_linear_in_one_call_refuses_what_the_two_calls_refuse():
         assert ffi.raw("gpu_linear_w8a8", dtype, 0, K, 0, 0, 0, 0, 0, M, N, K, rotate, out_dt, 0) == want, (dtype, M, N, K, rotate, out_dt)
 
 
+@pytest.mark.parametrize("M,K", [(9, 256), (8, 1088), (300, 1280)])
+def test_linear_in_one_call_refuses_a_scratch_that_is_none(M, K):
+    """Null, or 8 bytes off, where the call is two kernels: -1, and nothing is queued; the quantizer's own refusals come first."""
+    x, W, ws = torch.ones(M, K, device=DEV).bfloat16(), torch.ones(8, K, dtype=torch.int8, device=DEV), torch.ones(8, device=DEV)
+    D, scratch = torch.full((M, 8), 7.0, device=DEV), torch.full((M * K + 4 * M + 16,), 77, dtype=torch.uint8, device=DEV)
+    for s in (0, scratch.data_ptr() + 8):
+        args = (x.data_ptr(), K, W.data_ptr(), ws.data_ptr(), 0, D.data_ptr(), s, M, 8)
+        assert ffi.raw("gpu_linear_w8a8", BF16, *args, K, 0, F32, 0) == -1
+        assert ffi.raw("gpu_linear_w8a8", F16, *args, K, 0, F32, 0) == -4
+    torch.cuda.synchronize()
+    assert bool((D == 7.0).all()) and bool((scratch == 77).all())
+    assert ffi.raw("gpu_linear_w8a8", BF16, *args[:6], scratch.data_ptr(), M, 8, K, 0, F32, 0) == 0
+    torch.cuda.synchronize()
+    assert np.allclose(D.cpu().numpy(), K, rtol=1e-2)
+
+
 # ------------------------------------------------------------------------------------------------ W6
 def test_w6_decode_exhaustive_and_random():
     K, G = 64, 16
