@@ -699,3 +699,59 @@ def test_attention_sink_far_above_every_key(levels, lk):
     got = _to_f32(_bits(ql.int8_attn_sink(q.cuda(), k.cuda(), v.cuda(), scale, sink)), oracle.BF16)
     assert (ref > 0).all() and (ref < 1e-3).all()
     assert (np.abs(got - ref) <= (2 * 4 / 255.0 + 2 * 2.0 ** -8) * ref).all()
+
+
+def _base_moves(z, scale, lq, lk):
+    """Per row of head 0, the key tiles after the first at which a running base that follows a maximum more than 60 above it (in
+    powers of two) moves, and the largest distance of a maximum above it that does not move it."""
+    ck, S = z["ck"], z["qi"][0, 0].astype(np.int64) @ z["ki"][0, 0].astype(np.int64).T
+    wq, tiles = 32, (lk + ck - 1) // ck
+    qs = np.array([z["qs"][0, 0, (r // wq) * 8 + r % 8] for r in range(lq)], np.float64)[:, None]
+    moves, above, m = np.zeros((lq, tiles), bool), np.zeros(lq), np.full(lq, -50000.0)
+    for t in range(tiles):
+        key = np.arange(t * ck, min(lk, (t + 1) * ck))
+        s = S[:, key] if t + 1 < tiles else np.maximum(S[:, key], -50000)      # the last tile's floor
+        top = (s * qs * z["ks"][0, 0, t * 4 + (key % 8) // 2] * scale * 1.4426950408889634).max(1)
+        moves[:, t] = top - m > 60
+        m = np.where(moves[:, t], np.maximum(m, top), m)
+        above = np.maximum(above, top - m)
+    return moves, above
+
+
+MOVES = [  # D, lk, score level per key tile (the last from there on), dtype, sink, where the base moves besides the first tile
+    (64, 300, (0.0, 45.0, 20.0, 55.0), torch.bfloat16, 0.0, None),           # stays: factors up to 2^55
+    (128, 1300, (0.0, 0.0, 50.0, -30.0), torch.float16, 0.0, None),
+    (64, 1500, (0.0, 20.0, 100.0, 30.0), torch.float16, 0.0, 2),             # a middle tile
+    (128, 400, (-40.0, 35.0, 35.0, 120.0, 0.0), torch.bfloat16, 0.0, 1),     # and another one behind it
+    (128, 1300, (0.0,) * 10 + (90.0,), torch.bfloat16, 0.0, 10),             # the ragged last tile
+    (64, 200, (0.0, 0.0, 0.0, 100.0), torch.bfloat16, 0.0, 3),
+    (128, 400, (0.0, -30.0, 100.0, 10.0), torch.bfloat16, 200.0, 2),         # with sinks: exp2(-base) beside it
+    (128, 1300, (-55.0, 0.0), torch.bfloat16, 50.0, None),
+]
+
+
+@pytest.mark.parametrize("case", MOVES, ids=lambda c: "D%d_lk%d_%s_sink%g_tile%s" % (c[0], c[1], str(c[3])[6:], c[4], c[5]))
+def test_attention_scores_that_grow_along_the_keys(case):
+    """The base that numerators and denominators are relative to moves in a tile other than the first for some rows of a wave and not
+    for others, or lags far behind.  Values are 1..2 in even key tiles and 3..6 in odd ones, so that a tile that counts for more or
+    less than it should shows; tolerance: four probabilities one u8 step (of 255) away at values of 6, and the output's rounding."""
+    ql, ffi = _pkg()
+    D, lk, levels, dtype, sink, tile = case
+    dt = oracle.BF16 if dtype == torch.bfloat16 else oracle.F16
+    q, k, v = (t.float() for t in _keys_by_level(lk, levels, seed=D + lk, D=D))
+    q *= torch.tensor([1.0, 0.3, -0.5, 0.9])[torch.arange(40) // 3 % 4][None, :, None, None]
+    v *= torch.where(torch.arange(lk) // (128 if lk > 1024 and D != 64 else 64) % 2 == 1, 3.0, 1.0)[None, :, None, None]
+    q, k, v = q.to(dtype), k.to(dtype), v.to(dtype)
+    scale, anchor = D ** -0.5, sink == 0.0
+    z = oracle.attn_quant(dt, _bits(q), _bits(k), _bits(v), anchor)
+    moves, above = _base_moves(z, scale, 40, lk)
+    assert moves[:, 0].all()
+    if tile is None:
+        assert not moves[:, 1:].any() and above.max() > 40
+    else:
+        assert moves[:32, tile].any() and not moves[:32, tile].all()      # the rows of one wave differ
+    ref = _to_f32(oracle.attn_int8(dt, _bits(q), _bits(k), _bits(v), scale, quant=z, use_anchor=anchor, sink=sink), dt)
+    o = ql.int8_attn(q.cuda(), k.cuda(), v.cuda(), scale) if anchor else ql.int8_attn_sink(q.cuda(), k.cuda(), v.cuda(), scale, sink)
+    ulp = 2.0 ** (-8 if dt == oracle.BF16 else -11)
+    assert (ref > 1).all()
+    assert (np.abs(_to_f32(_bits(o), dt) - ref) <= 4 * 6 / 255.0 + 2 * ulp * ref).all()
