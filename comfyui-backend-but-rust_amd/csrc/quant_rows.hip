@@ -570,16 +570,18 @@ int launch_geglu(QuantArgs a, int wpr, int cus, hipStream_t st) {
     return 0;
 }
 
-// GEGLU with the table in LDS.  A round of the wave-per-row form takes about 3.3 us per chunk of its rows and 4 us of the
-// launch's start more than the other form, whose rounds take 4.1 us.
-template <int G>
-int run_geglu(const QuantArgs& a, int nchunks, hipStream_t st) {
-    const int cus = device_cu_count();
-    if (nchunks > kGegluWaves) return launch_geglu<G, 2>(a, (nchunks + 1) / 2, cus, st);
-    const auto rounds = [&](int rpb) { return (a.M + (int64_t)rpb * cus - 1) / ((int64_t)rpb * cus); };
-    if (nchunks <= 3 && 3.3 * nchunks * rounds(kGegluWaves) + 4. < 4.1 * rounds(kGegluWaves / nchunks))
-        return nchunks == 3 ? launch_geglu<G, 3>(a, 1, cus, st) : nchunks == 2 ? launch_geglu<G, 2>(a, 1, cus, st) : launch_geglu<G, 1>(a, 1, cus, st);
-    return launch_geglu<G, 1>(a, nchunks, cus, st);
+// GEGLU with the table in LDS: chunks per wave and waves per row.  Filling the table takes a workgroup 2.5 us: it pays from about
+// 5000 chunks on (1024 x 5120: 13.0 us either way; 2048 x 5120 18.4 against 21.4, 512 x 2560 7.4 against 5.9).  A round of the
+// wave-per-row form takes about 3.3 us per chunk of its rows and 4 us of the launch's start more than the other form, whose rounds
+// take 4.1 us.
+struct GegluForm { int chunks, wpr; };   // no chunks: the table stays in global memory
+GegluForm geglu_form(int M, int K, int cus) {
+    const int nchunks = (K + kChunk - 1) / kChunk;
+    if ((int64_t)M * nchunks < 5120) return {0, 0};
+    if (nchunks > kGegluWaves) return {2, (nchunks + 1) / 2};
+    const auto rounds = [&](int rpb) { return (M + (int64_t)rpb * cus - 1) / ((int64_t)rpb * cus); };
+    if (nchunks <= 3 && 3.3 * nchunks * rounds(kGegluWaves) + 4. < 4.1 * rounds(kGegluWaves / nchunks)) return {nchunks, 1};
+    return {1, nchunks};
 }
 
 template <auto KERN>
@@ -608,10 +610,13 @@ int launch(const QuantArgs& a, int nw, hipStream_t st) {
         const bool gated = MODE == MODE_BF16 ? a.pro == PRO_GATE || a.pro == PRO_SWIGLU || a.pro == PRO_SILU
                                              : a.pro == PRO_SD_GEGLU && a.tab.gelu_f16;
         if constexpr (MODE == MODE_SD_F16) {
-            // filling the table takes a workgroup 2.5 us: it pays from about 5000 chunks on (1024 x 5120: 13.0 us either way;
-            // 2048 x 5120 18.4 against 21.4, 512 x 2560 7.4 against 5.9)
-            const int nchunks = (a.K + kChunk - 1) / kChunk;
-            if (gated && (int64_t)a.M * nchunks >= 5120) return run_geglu<G>(a, nchunks, st);
+            if (gated) {
+                const int cus = device_cu_count();
+                const GegluForm f = geglu_form(a.M, a.K, cus);
+                if (f.chunks == 1) return launch_geglu<G, 1>(a, f.wpr, cus, st);
+                if (f.chunks == 2) return launch_geglu<G, 2>(a, f.wpr, cus, st);
+                if (f.chunks == 3) return launch_geglu<G, 3>(a, f.wpr, cus, st);
+            }
         }
         if (gated) return launch_kernel<quant_rows_kernel<MODE, G, C, CLS_GATED>>(a, nw, lds, st);
     }
@@ -874,6 +879,12 @@ GPU_API int gpu_convrot_requant(int dtype, const void* x, void* q, void* s, int6
     if (K > 32768 || N > 0x7fffffff) return -2;
     QuantArgs a{x, K, (int8_t*)q, (float*)s, nullptr, (int)N, K, 1, 1, seed};
     return dtype == DT_F32 ? run_quant<MODE_F32>(a, 256, (hipStream_t)stream) : run_quant<MODE_BF16>(a, 256, (hipStream_t)stream);
+}
+
+// Test hook: the form of the GEGLU quantizer that a shape takes, 100 * chunks per wave + waves per row; 0: the one for few chunks.
+GPU_API int gpu_internal_geglu_form(int M, int K) {
+    const GegluForm f = geglu_form(M, K, device_cu_count());
+    return 100 * f.chunks + f.wpr;
 }
 
 // Test hook: out[i] = bf16 bits of sigmoid (which 0) or silu (1) of the bf16 bits in[i], or f16 bits of gelu (2) of the f16

@@ -51,6 +51,7 @@ SIGNATURES = {
     "gpu_int8_attn_norm_rope": [_P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32] + [_I64] * 12 + [_F32, _P, _P, _F32, _P, _I32, _P],
     "gpu_int8_attn_key_bias": [_P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32] + [_I64] * 12 + [_F32, _P, _P],
     "gpu_internal_act_probe": [_I32, _P, _P, _I32, _P],
+    "gpu_internal_geglu_form": [_I32, _I32],
     "gpu_internal_cvt_pk_u8_probe": [_P, _P, _I32, _P],
     "gpu_internal_attn_sumsq_probe": [_P, _P, _I32, _I32, _P],
     "gpu_internal_w6a8_group_gemm_ablate": [_I32, _P, _P, _P, _P, _P, _I64, _I64, _I64, _P],

@@ -178,6 +178,10 @@ int gpu_int8_attn_key_bias(const void* q, const void* k, const void* v, void* o,
  * the f16 bits in[i], evaluated as the quantizer's prologues evaluate it. */
 int gpu_internal_act_probe(int which, const void* in, void* out, int n, void* stream);
 
+/* Test hook, no reference counterpart: the form in which gpu_sd_geglu_quant_rows runs M rows of K outputs, 100 * chunks per wave +
+ * waves per row of the kernel with its table in LDS, 0 for the kernel for few chunks. */
+int gpu_internal_geglu_form(int M, int K);
+
 /* Test hook, no reference counterpart: y[i] = the gfx950 float -> u8 pack conversion of x[i] (byte 0), which the attention
  * kernel's probabilities rely on being round-to-nearest-even with saturation to 0..255. */
 int gpu_internal_cvt_pk_u8_probe(const float* x, uint32_t* y, int n, void* stream);

@@ -311,11 +311,15 @@ def test_gelu_of_every_f16_value():
 
 
 @pytest.mark.parametrize("rotate", [0, 64, 256])
-@pytest.mark.parametrize("M,K", [(5121, 256), (2561, 1280), (16385, 1280), (8190, 2560), (1100, 5120), (303, 16640)])
-def test_geglu_table_kernel_forms(M, K, rotate):
-    """Row counts at which the kernel with the table in LDS runs, in each of its forms (a wave per chunk with and without idle
-    waves, a wave per row of two and three chunks, two chunks per wave): the first, last and some other rows bit-exact."""
-    say("geglu", M, K, rotate)
+@pytest.mark.parametrize("M,K,form", [(5121, 256, 101), (2561, 1280, 102), (16385, 1280, 102), (16383, 1280, 201), (12288, 2048, 201),
+                                      (8190, 2560, 301), (1100, 5120, 105), (303, 16640, 209), (511, 5120, 0)])
+def test_geglu_table_kernel_forms(M, K, form, rotate):
+    """Row counts at which the kernel with the table in LDS runs, in each of its forms (100 * chunks per wave + waves per row: a wave
+    per chunk with and without idle waves, a wave per row of two and three chunks, two chunks per wave), and one below: the
+    first, last and some other rows bit-exact."""
+    say("geglu", M, K, form, rotate)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:   # what the rule divides the rows by
+        assert ffi.raw("gpu_internal_geglu_form", M, K) == form
     g = torch.Generator(device=DEV).manual_seed(M + K)
     x = (torch.randn(M, 2 * K, device=DEV, generator=g) * 2).half()
     x[0, K] = float("nan"); x[M - 1, K + 3] = float("-inf"); x[M - 1, 2 * K - 1] = float("inf")
@@ -836,8 +840,9 @@ def test_int8_gemm_acc_bit_exact(M, N, K, cfg):
 
 
 # Edges of the kernel for up to 128 rows: its row tiles (16, 32, 64, 96, 128), columns past the last tile and unaligned ones, K
-# shorter than a panel, panels with a remainder, an odd and an even number of them, and K split over workgroups
-ROWS_CASES = [(1, 8, 128), (15, 67, 768), (16, 1000, 4096), (17, 96, 1152), (32, 4100, 896), (33, 72, 2176), (64, 130, 1024), (65, 4096, 896),
+# shorter than a panel, panels with a remainder, an odd and an even number of them, and K split over workgroups, with outputs of
+# whole 16 bytes and of whole 8
+ROWS_CASES = [(64, 1028, 4096), (1, 8, 128), (15, 67, 768), (16, 1000, 4096), (17, 96, 1152), (32, 4100, 896), (33, 72, 2176), (64, 130, 1024), (65, 4096, 896),
               (77, 1024, 3712), (96, 264, 640), (97, 96, 1280), (128, 2048, 4224), (16, 16416, 1024), (5, 4097, 2304)]
 
 

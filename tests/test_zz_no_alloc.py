@@ -1,5 +1,5 @@
 """gpu_int8_gemm_static, the entry point that allocates nothing, against gpu_int8_gemm: bit-equal outputs through the C ABI
-on two calls in a row, the second with a smaller input (the static split-K planes keep the first call's contents)."""
+on calls in a row, each with a smaller input (the static split-K planes keep the earlier calls' contents)."""
 import importlib
 import os
 import sys
@@ -45,8 +45,8 @@ def _run(name, A, W, xs, ws, bias):
     return D.cpu().numpy().view(np.uint16)
 
 
-# split-K shapes of the skinny path (M <= 256, N too narrow to give every CU a column slab), larger first
-SHAPES = [(256, 4096, 4096), (100, 1024, 2048)]
+# larger first: split K in the weight-streaming kernel, no split in the kernel for up to 128 rows, split K there
+SHAPES = [(256, 4096, 4096), (100, 1024, 2048), (100, 1024, 4096), (16, 1024, 8192)]
 
 
 def test_static_entry_point_matches_allocating_one_twice_in_a_row():
@@ -57,7 +57,7 @@ def test_static_entry_point_matches_allocating_one_twice_in_a_row():
         want = _run("gpu_int8_gemm", A, W, xs, ws, bias)
         got = _run("gpu_int8_gemm_static", A, W, xs, ws, bias)
         assert np.array_equal(got, want), (M, N, K)
-        if i == 1:   # and against the oracle, so that both being wrong the same way cannot pass
+        if i >= 1:   # and against the oracle, so that both being wrong the same way cannot pass
             ref = oracle.int8_gemm(A, W, xs, ws, bias, oracle.BF16, fma=1)
             assert np.array_equal(got, ref.view(np.uint16))
 
@@ -71,7 +71,8 @@ def test_static_entry_point_on_shapes_without_scratch():
 
 def test_static_entry_point_refuses_what_would_need_an_allocation():
     """K % 16 == 8 runs on padded copies that gpu_int8_gemm allocates; the entry point that may not allocate refuses it.
-    (The split-K planes of every M <= 256 shape fit the static array on a 256-CU device: slices * N <= 256 * 96.)"""
+    (The split-K planes of every M <= 256 shape fit the static array on a 256-CU device: slices * N <= 256 * 96, and 256 * 64 up to
+    128 rows.)"""
     M, N, K = 64, 128, 136
     A, W, xs, ws, bias = _inputs(60, M, N, K)
     t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
