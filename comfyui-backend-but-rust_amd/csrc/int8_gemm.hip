@@ -1385,7 +1385,7 @@ __global__ void __launch_bounds__(TurnCfg::NT, 1) int8_gemm_turn_kernel(GemmArgs
 // 8.3 and 5.2, 14.7 and 11.7, 22.9 and 20.0, 26.8 and 22.9; 128 rows 8.3 and 8.0, 16.1 and 16.4, 25.6 and 23.9, 27.4 and 24.0.
 // Eight steps of 64 per panel where two stages fit the LDS, else four: with NWK = 1 instead, 77 rows take 16.6 instead of 13.8 us
 // for 4096 -> 4096.
-template <int MT, int NWK>
+template <int MT, int NWK>   // NWK 2, 4 or 8
 struct RowsCfg {
     static constexpr int NT = 512, NWN = 8 / NWK, BN = 16 * NWN, RB = 2 * MT;
     static constexpr int SP = MT * NWK <= 8 ? 8 : 4;   // steps of 64 per wave and panel; two stages have to fit the LDS
@@ -1528,22 +1528,17 @@ __global__ void __launch_bounds__(512, (MT * NWK <= 4 ? 4 : 2)) int8_gemm_rows_k
 #pragma unroll
             for (int j = 0; j < 4; ++j) if (n + j < p.N) st_dt<OUT_DT>(p.D, o + j, out[j]);
     };
-    if constexpr (NWK == 1) {
+    v4i* red = reinterpret_cast<v4i*>(smem) + lane;   // [part of K][16 columns][row tile][lane]
 #pragma unroll
-        for (int t = 0; t < MT; ++t) finish(acc[t], t, EPI == EPI_ACC ? 0.f : xs[t]);
-    } else {
-        v4i* red = reinterpret_cast<v4i*>(smem) + lane;   // [part of K][16 columns][row tile][lane]
+    for (int t = 0; t < MT; ++t) red[(wave * MT + t) * 64] = acc[t];
+    __syncthreads();
 #pragma unroll
-        for (int t = 0; t < MT; ++t) red[(wave * MT + t) * 64] = acc[t];
-        __syncthreads();
+    for (int t = 0; t < MT; ++t) {
+        if (t % NWK != wk) continue;
+        v4i sum = red[(wn * MT + t) * 64];
 #pragma unroll
-        for (int t = 0; t < MT; ++t) {
-            if (t % NWK != wk) continue;
-            v4i sum = red[(wn * MT + t) * 64];
-#pragma unroll
-            for (int q = 1; q < NWK; ++q) sum += red[((q * C::NWN + wn) * MT + t) * 64];
-            finish(sum, t, EPI == EPI_ACC ? 0.f : xs[t]);
-        }
+        for (int q = 1; q < NWK; ++q) sum += red[((q * C::NWN + wn) * MT + t) * 64];
+        finish(sum, t, EPI == EPI_ACC ? 0.f : xs[t]);
     }
 }
 

@@ -14,14 +14,6 @@ namespace {
 
 constexpr int kG = 32;   // columns per relative scale
 
-__device__ __forceinline__ uint32_t pcg(uint32_t x) {                            // :21-25
-    x = x * 747796405u + 2891336453u;
-    const uint32_t w = ((x >> ((x >> 28u) + 4u)) ^ x) * 277803737u;
-    return (w >> 22u) ^ w;
-}
-__device__ __forceinline__ float uniform01(int64_t idx, uint64_t seed) {          // :27-31
-    return (float)(pcg((uint32_t)idx ^ (uint32_t)seed ^ (uint32_t)(seed >> 32)) >> 8) * (1.0f / 16777216.0f);
-}
 // float -> fp8 e4m3 bits, round to nearest even, saturating at 448 (finite inputs)
 __device__ __forceinline__ uint32_t f_to_e4m3(float x) {
     const uint32_t sgn = (f2u(x) >> 31) << 7;
