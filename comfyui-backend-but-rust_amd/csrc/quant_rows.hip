@@ -264,10 +264,10 @@ enum {
     CLS_REST     // everything that may evaluate an fp64 routine, and the SD gathers
 };
 template <int MODE, int G, int C, int CLS, bool SR = false>
-__global__ void __launch_bounds__(1024) quant_rows_kernel(QuantArgs p) {
+__global__ void __launch_bounds__(512, C > 3 ? 2 : 4) quant_rows_kernel(QuantArgs p) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    __shared__ float red[16];
-    __shared__ double dred[16];
+    __shared__ float red[8];
+    __shared__ double dred[8];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int rloc = wave / p.wpr, wr = wave - rloc * p.wpr;
     const int64_t m = (int64_t)blockIdx.x * p.rpb + rloc;
@@ -586,12 +586,7 @@ GegluForm geglu_form(int M, int K, int cus) {
 
 template <auto KERN>
 int launch_kernel(const QuantArgs& a, int nw, int lds_per_wave, hipStream_t st) {
-    const int smem = nw * lds_per_wave;
-    if (smem > 63 * 1024) {   // the tiles of 15 or 16 waves are more than a kernel may have unasked
-        static PerDeviceOnce once;
-        if (const int e = allow_dynamic_lds(reinterpret_cast<const void*>(KERN), 16 * lds_per_wave, once)) return e;
-    }
-    hipLaunchKernelGGL(KERN, dim3((a.M + a.rpb - 1) / a.rpb), dim3(nw * 64), smem, st, a);
+    hipLaunchKernelGGL(KERN, dim3((a.M + a.rpb - 1) / a.rpb), dim3(nw * 64), nw * lds_per_wave, st, a);   // 8 waves: 35 KB
     KCHECK();
     return 0;
 }
@@ -625,20 +620,29 @@ int launch(const QuantArgs& a, int nw, hipStream_t st) {
 
 template <int MODE, int G>
 int launch_c(const QuantArgs& a, int nw, int C, hipStream_t st) {
-    return C == 1 ? launch<MODE, G, 1>(a, nw, st) : launch<MODE, G, 2>(a, nw, st);
+    return C == 1 ? launch<MODE, G, 1>(a, nw, st) : C == 2 ? launch<MODE, G, 2>(a, nw, st) : C == 3 ? launch<MODE, G, 3>(a, nw, st) : launch<MODE, G, 4>(a, nw, st);
 }
 
-// g: rotation group width (0, 64, 128, 256).  A wave per chunk of 1024 values up to eight waves per row, two chunks per
-// wave beyond: short waves overlap their loads with each other's arithmetic, larger workgroups wait for their slowest wave.
-// Measured, us by the kernel trace: 4608 x 3072 one chunk per wave 14.2, two 15.8, three 16.1; GEGLU 8192 x 2560 48.8, 53.4,
-// 57.2; 2048 x 14336 fourteen waves 31.4, eight 25.9, four with four chunks each 27.7; SwiGLU 4608 x 12288 twelve waves
-// 86, eight 78.
+// g: rotation group width (0, 64, 128, 256).  A row goes to 1, 2, 4 or 8 waves (their number per SIMD stays even), up to three
+// chunks of 1024 values each (four beyond 24 chunks), and to more of them where the launch would have fewer than `enough` waves:
+// short waves overlap their loads with each other's arithmetic, but a row's waves wait for its slowest, and a norm's for each
+// other twice more.  us per call, a wave per chunk (two beyond 8 chunks, 8 waves) against this: bf16 rotate 128 4608 x 3072
+// 14.2 either way, 18601 x 5376 83 and 70; f32 7440 x 5376 39.9 and 36.1, with LayerNorm 90 and 52, bf16 66 and 42; f32 requantizer
+// 5376 x 5376 31.9 and 28.4.  Without a rotation (and in the f16 gathers) there is less to wait for: always as many waves as
+// chunks.  Three chunks on two waves is the worst of both (bf16 13020 x 3072: 1 wave 28.8, 2 29.1, 3 26.4).
 template <int MODE>
 int run_quant(QuantArgs a, int g, hipStream_t st) {
     if (a.M <= 0) return 0;
     const int nchunks = (a.K + kChunk - 1) / kChunk;
     if (nchunks > 32) return -2;
-    const int C = nchunks > 8 ? 2 : 1, wpr = nchunks <= 8 ? nchunks : nchunks <= 16 ? 8 : (nchunks + 1) / 2;
+    const bool norm = a.pro == PRO_RMS || a.pro == PRO_LAYERNORM || a.pro == PRO_ADALN || a.pro == PRO_LN_MOD || a.pro == PRO_LN_AFFINE;
+    const bool light = g == 0 || a.pro == PRO_SD_UNPAD || a.pro == PRO_SD_GN;
+    const int64_t enough = norm ? 2048 : light ? INT64_MAX : 12288;
+    int wpr = 1;
+    while (wpr < 8 && (nchunks + wpr - 1) / wpr > 3) wpr *= 2;
+    while (wpr < 8 && wpr < nchunks && a.M * (int64_t)wpr < enough) wpr = nchunks == 3 ? 3 : 2 * wpr;
+    wpr = wpr < nchunks ? wpr : nchunks;
+    const int C = (nchunks + wpr - 1) / wpr;
     const int nw = wpr < 2 ? 2 : wpr;   // two rows per workgroup at least
     a.wpr = wpr;
     a.rpb = nw / wpr;

@@ -364,6 +364,35 @@ def test_rotation_scaled_once_and_per_stage(M, K, rotate):
         assert rc == 0 and np.array_equal(got.cpu().numpy().view(np.uint32), want.view(np.uint32))
 
 
+# Row counts either side of those at which a row's waves take more chunks: 1, 2 and 3 chunks on one wave, 5 on two, 9 and 12 on four,
+# 17 and 25 on eight; norms from 2048 waves on
+FORMS = [(12287, 1280), (12288, 1280), (12288, 3072), (6144, 5120), (3072, 9216), (3072, 12288), (40, 17408), (40, 25600), (2048, 3072), (1024, 5376)]
+
+
+@pytest.mark.parametrize("dt", [BF16, F32])
+@pytest.mark.parametrize("M,K", FORMS)
+def test_quant_rows_in_every_split_of_a_row(M, K, dt):
+    """A row's result does not depend on how many rows there are: the whole call against the oracle on some rows, and against the same
+    rows by themselves, which take another split; plain, LayerNorm, SwiGLU and GELU prologues and the stochastic requantizer."""
+    say("splits", M, K, dt)
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    x = torch.randn(M, 2 * K, device=DEV, generator=g).to(TDT[dt])
+    rows = torch.unique(torch.cat([torch.arange(3), torch.arange(M - 3, M), torch.randint(0, M, (6,), generator=torch.Generator().manual_seed(K))])).to(DEV)
+    few = x[rows].contiguous()
+    for pro, rotate in ((ffi.PRO_PLAIN, 0), (ffi.PRO_PLAIN, 1), (ffi.PRO_LAYERNORM, 1), (ffi.PRO_SWIGLU, 1), (ffi.PRO_GELU, 1)):
+        q, s = ql.quant_rows_pro(x, pro, K, rotate, up_offset=K, eps=1e-6)
+        qf, sf = ql.quant_rows_pro(few, pro, K, rotate, up_offset=K, eps=1e-6)
+        assert torch.equal(q[rows], qf) and torch.equal(s[rows].view(torch.int32), sf.view(torch.int32)), (pro, rotate)
+        if pro == ffi.PRO_PLAIN:
+            fb = few[:, :K].contiguous()
+            rc, qo, so = oracle.quant_rows(dt, host_bits(fb) if dt == BF16 else fb.cpu().numpy(), K, rotate)
+            assert rc == 0 and np.array_equal(qf.cpu().numpy(), qo) and np.array_equal(sf.cpu().numpy().view(np.uint32), so.view(np.uint32))
+    w = x[:, :K].contiguous()
+    q, s = ql.convrot_requant(w, 7)
+    qf, sf = ql.convrot_requant(w[:3].contiguous(), 7)     # the same element indices
+    assert torch.equal(q[:3], qf) and torch.equal(s[:3].view(torch.int32), sf.view(torch.int32))
+
+
 def test_quant_rows_b_and_rotate_rows_f32_with_prologues():
     M, K = 5, 1536
     c = pro_case(BF16, 801, M, K, K + 16)
