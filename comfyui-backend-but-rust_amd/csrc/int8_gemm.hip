@@ -1894,33 +1894,56 @@ constexpr int kSplitRowsK = 1800;
 
 // M <= 128.  The widest split of K inside the workgroup that still gives every CU at most one workgroup; where even that
 // leaves CUs without one, K is split over workgroups as well.
-template <int OUT_DT, int EPI>
-int launch_rows(GemmArgs a, hipStream_t st) {
-    bool vec_ok, aligned;
-    epilogue_alignment<OUT_DT, EPI>(a, vec_ok, aligned);
-    const int cus = device_cu_count();
-    const int mt = a.M <= 16 ? 1 : a.M <= 32 ? 2 : a.M <= 64 ? 4 : a.M <= 96 ? 6 : 8;
-    const auto tiles = [&](int nwk) { return (int)(((int64_t)a.N * nwk + 127) / 128); };
+struct RowsPlan { int mt, nwk, tiles, slices, per; };   // per: K of a slice
+RowsPlan rows_plan(int64_t M, int64_t N, int64_t K, int cus, bool may_split) {
+    const int mt = M <= 16 ? 1 : M <= 32 ? 2 : M <= 64 ? 4 : M <= 96 ? 6 : 8;
+    const auto tiles = [&](int nwk) { return (int)((N * nwk + 127) / 128); };
     const int most = mt == 1 ? 8 : mt <= 4 ? 4 : 2;
     int nwk = 2;
     while (nwk < most && tiles(2 * nwk) <= cus) nwk *= 2;
     if (mt == 1 && tiles(2) > cus) nwk = 4;   // several rounds: the smaller tiles fill the last one better
-    const int unit = 64 * nwk * (mt * nwk <= 8 ? 8 : 4), panels = (a.K + unit - 1) / unit;
-    int slices = vec_ok ? cus / tiles(nwk) : 1;
+    const int unit = 64 * nwk * (mt * nwk <= 8 ? 8 : 4), panels = (int)((K + unit - 1) / unit);
+    int slices = may_split ? cus / tiles(nwk) : 1;
     if (slices > panels) slices = panels;
-    if (slices > 1 && a.K / slices * (slices - 1) < kSplitRowsK) slices = 1;
-    if (slices <= 1) {
+    if (slices > 1 && K / slices * (slices - 1) < kSplitRowsK) slices = 1;
+    if (slices <= 1) return {mt, nwk, tiles(nwk), 1, (int)K};
+    const int per = (panels + slices - 1) / slices;
+    return {mt, nwk, tiles(nwk), (panels + per - 1) / per, per * unit};   // no empty slice
+}
+
+template <int OUT_DT, int EPI>
+int launch_rows(GemmArgs a, hipStream_t st) {
+    bool vec_ok, aligned;
+    epilogue_alignment<OUT_DT, EPI>(a, vec_ok, aligned);
+    const RowsPlan p = rows_plan(a.M, a.N, a.K, device_cu_count(), vec_ok);
+    if (p.slices == 1) {
         a.kslice = 0;
-        return launch_rows_as<OUT_DT, EPI>(a, mt, nwk, vec_ok, 1, st);
+        return launch_rows_as<OUT_DT, EPI>(a, p.mt, p.nwk, vec_ok, 1, st);
     }
     // Outputs that are narrow, or whose rows or pointers are not whole 16 bytes, do not split K in the streaming kernel either
     // (choose_cfg, launch_skinny).  A captured graph of them holds no address of the stream's planes, so that it may be replayed on any
     // stream, and the static entry point leaves its buffer alone: they take the register-staged tiles there.
     if ((a.N < 1024 || !aligned) && (tl_scratch != nullptr || is_capturing(st)))
         return a.N < 1024 ? launch_cfg<CfgS, OUT_DT, EPI>(a, st) : launch_cfg<CfgM, OUT_DT, EPI>(a, st);
-    const int per = (panels + slices - 1) / slices;
-    slices = (panels + per - 1) / per;   // no empty slice
-    return launch_split<OUT_DT, EPI>(a, slices, per * unit, st, [&](const GemmArgs& pa) { return launch_rows_as<DT_F32, EPI_ACC>(pa, mt, nwk, true, slices, st); });
+    return launch_split<OUT_DT, EPI>(a, p.slices, p.per, st, [&](const GemmArgs& pa) { return launch_rows_as<DT_F32, EPI_ACC>(pa, p.mt, p.nwk, true, p.slices, st); });
+}
+
+// Where the kernels beside it are faster than the one for up to 128 rows (us, that one and the other):
+//   * short K and few columns: the small register-staged tiles have less to start (24 rows 768 -> 768 6.3 and 5.8; 128 rows 1152 -> 512
+//     8.5 and 7.5; but 48 rows 768 -> 768 4.8 and 5.8, 128 rows 1280 -> 640 8.5 and 9.2);
+//   * long K, and columns whose 96-wide tiles and K slices in the streaming kernel give a quarter more CUs a workgroup: a workgroup's
+//     own stretch of K is what the call waits for, the longer the fewer rows of A it takes in beside the weights (96 rows
+//     12288 -> 9216 36 and 28; 64 rows 14336 -> 4608 33 and 26; 32 rows 12288 -> 9216 28 and 26; but 64 rows 5120 -> 5120 13 and 15).
+// Outputs not of whole 16 bytes do not run there.
+bool rows_kernel_loses(int64_t M, int64_t N, int64_t K, bool aligned) {
+    if (K < 896) return N < 1152 && (M <= 32 || M > 64);
+    if (M > 64 && K >= 1024 && K < (M > 96 ? 1408 : 1280)) return N < (K < 1152 ? 1024 : 640);
+    if (M <= 16 || K < 5120 || N < 1024 || !aligned) return false;
+    const int cus = device_cu_count(), t96 = (int)((N + 95) / 96);
+    const RowsPlan p = rows_plan(M, N, K, cus, true);
+    const int here = p.tiles * p.slices, there = t96 * (cus / t96 > 1 ? cus / t96 : 1);
+    if (there * 4 < here * 5) return false;
+    return M > 64 ? p.per >= 5120 : M > 32 ? p.per >= 7168 : p.per >= 11264 && (p.nwk == 2 || here * 5 < cus * 3);
 }
 
 // Kernel family forced by the test hook (-1 = choose by shape).  Process-wide and only meant for tests and benchmarks:
@@ -1928,18 +1951,20 @@ int launch_rows(GemmArgs a, hipStream_t st) {
 std::atomic<int> g_force_cfg{-1};
 
 // `whole` = A and W start at 16-byte addresses, what the kernel for up to 128 rows asks of its DMA and its weight loads; an
-// operand that starts elsewhere (a view into a larger buffer) goes to the kernels that such calls had without it.
-int choose_cfg(int64_t M, int64_t N, int64_t K, bool whole) {
+// operand that starts elsewhere (a view into a larger buffer) goes to the kernels that such calls had without it.  `aligned` as
+// epilogue_alignment has it.
+int choose_cfg(int64_t M, int64_t N, int64_t K, bool whole, bool aligned) {
     const int force = g_force_cfg.load(std::memory_order_relaxed);
     const bool dma_ok = M * K < ((int64_t)1 << 32) && N * K < ((int64_t)1 << 32);   // 32-bit lane offsets
     if (force == 5) return dma_ok && whole && (K % 128) == 0 && M <= 128 ? 5 : 1;
     if (force == 6 || force == 7 || force == 9) return (dma_ok && (K % 128) == 0) ? force : 1;
     if (force == 1 || force == 2) return force;
-    // Up to 128 rows: from K = 768 on (1024 for the most rows; below, the small register-staged tiles have less to start) and up
+    // Up to 128 rows: from K = 768 on (1024 for the most rows), except where rows_kernel_loses, and up
     // to the 16384 columns that give every CU one workgroup of the tallest split.  Beyond those the streaming kernel's 96-wide
     // tiles fill the CUs as well and its W rows come in whole lines (4096 -> 24576, us, this and that: 1 row 29.1 and 30.6, 32 rows
     // 35.3 and 30.6, 128 rows 42.8 and 31.5; 3072 -> 18432, 16 rows 18.0 and 21.1).
-    if (M <= 128 && (K % 128) == 0 && K >= (M > 96 ? 1024 : 768) && dma_ok && whole && (M <= 16 || N <= 16384)) return 5;
+    if (M <= 128 && (K % 128) == 0 && K >= (M > 96 ? 1024 : 768) && dma_ok && whole && (M <= 16 || N <= 16384) &&
+        !rows_kernel_loses(M, N, K, aligned)) return 5;
     if (M <= 256 && N >= 1024 && (K % 128) == 0 && K >= 512 && dma_ok) {
         // The weight-streaming kernel pays a fixed price per call (a prologue that waits for HBM, two launches when K
         // is split), which long K repays and short K does not.  Measured with weights from HBM, M = 16..256, K =
@@ -1968,7 +1993,9 @@ int choose_cfg(int64_t M, int64_t N, int64_t K, bool whole) {
 
 template <int OUT_DT, int EPI>
 int dispatch_cfg(const GemmArgs& a, hipStream_t st) {
-    switch (choose_cfg(a.M, a.N, a.K, (((uintptr_t)a.A | (uintptr_t)a.W) & 15) == 0)) {
+    bool vec_ok, aligned;
+    epilogue_alignment<OUT_DT, EPI>(a, vec_ok, aligned);
+    switch (choose_cfg(a.M, a.N, a.K, (((uintptr_t)a.A | (uintptr_t)a.W) & 15) == 0, aligned)) {
         case 5: return launch_rows<OUT_DT, EPI>(a, st);
         case 6: return launch_skinny<OUT_DT, EPI>(a, st);
         case 7: return launch_ring_small<OUT_DT, EPI>(a, st);

@@ -627,8 +627,8 @@ int launch_c(const QuantArgs& a, int nw, int C, hipStream_t st) {
 // chunks of 1024 values each (four beyond 24 chunks), and to more of them where the launch would have fewer than `enough` waves:
 // short waves overlap their loads with each other's arithmetic, but a row's waves wait for its slowest, and a norm's for each
 // other twice more.  us per call, a wave per chunk (two beyond 8 chunks, 8 waves) against this: bf16 rotate 128 4608 x 3072
-// 14.2 either way, 18601 x 5376 83 and 70; f32 7440 x 5376 39.9 and 36.1, with LayerNorm 90 and 52, bf16 66 and 42; f32 requantizer
-// 5376 x 5376 31.9 and 28.4.  Without a rotation (and in the f16 gathers) there is less to wait for: always as many waves as
+// 14.2 either way, 18601 x 5376 76 and 62; f32 7440 x 5376 40.7 and 36.4, with LayerNorm 90 and 52, bf16 66 and 42; f32 requantizer
+// 54 and 46 there.  Without a rotation (and in the f16 gathers) there is less to wait for: always as many waves as
 // chunks.  Three chunks on two waves is the worst of both (bf16 13020 x 3072: 1 wave 28.8, 2 29.1, 3 26.4).
 template <int MODE>
 int run_quant(QuantArgs a, int g, hipStream_t st) {

@@ -870,8 +870,8 @@ def test_int8_gemm_acc_bit_exact(M, N, K, cfg):
 
 # Edges of the kernel for up to 128 rows: its row tiles (16, 32, 64, 96, 128), columns past the last tile and unaligned ones, K
 # shorter than a panel, panels with a remainder, an odd and an even number of them, and K split over workgroups, with outputs of
-# whole 16 bytes and of whole 8
-ROWS_CASES = [(64, 1028, 4096), (1, 8, 128), (15, 67, 768), (16, 1000, 4096), (17, 96, 1152), (32, 4100, 896), (33, 72, 2176), (64, 130, 1024), (65, 4096, 896),
+# whole 16 bytes and of whole 8; and calls that the automatic choice gives to the streaming kernel and the small tiles
+ROWS_CASES = [(64, 1028, 4096), (65, 9216, 5120), (33, 4612, 7296), (24, 256, 768), (100, 512, 1152), (1, 8, 128), (15, 67, 768), (16, 1000, 4096), (17, 96, 1152), (32, 4100, 896), (33, 72, 2176), (64, 130, 1024), (65, 4096, 896),
               (77, 1024, 3712), (96, 264, 640), (97, 96, 1280), (128, 2048, 4224), (16, 16416, 1024), (5, 4097, 2304)]
 
 
