@@ -623,10 +623,11 @@ int launch_c(const QuantArgs& a, int nw, int C, hipStream_t st) {
     return C == 1 ? launch<MODE, G, 1>(a, nw, st) : C == 2 ? launch<MODE, G, 2>(a, nw, st) : C == 3 ? launch<MODE, G, 3>(a, nw, st) : launch<MODE, G, 4>(a, nw, st);
 }
 
-// g: rotation group width (0, 64, 128, 256).  A row goes to 1, 2, 4 or 8 waves (their number per SIMD stays even), up to three
-// chunks of 1024 values each (four beyond 24 chunks), and to more of them where the launch would have fewer than `enough` waves:
-// short waves overlap their loads with each other's arithmetic, but a row's waves wait for its slowest, and a norm's for each
-// other twice more.  us per call, a wave per chunk (two beyond 8 chunks, 8 waves) against this: bf16 rotate 128 4608 x 3072
+// g: rotation group width (0, 64, 128, 256).  A row goes to 1, 2, 4 or 8 waves (six or seven chunks to eight: idle waves cost less
+// than uneven SIMDs, 2232 x 5376 bf16 8.7 and 8.4 us), up to three chunks of 1024 values each (four beyond 24 chunks, and in the
+// f32 requantizer), and to more of them where the launch would have fewer than `enough` waves: short waves overlap their loads
+// with each other's arithmetic, but a row's waves wait for its slowest, and a norm's for each other twice more; nine and ten chunks
+// on eight waves would leave a third of their slots empty.  us per call, a wave per chunk (two beyond 8 chunks, 8 waves) against this: bf16 rotate 128 4608 x 3072
 // 14.2 either way, 18601 x 5376 76 and 62; f32 7440 x 5376 40.7 and 36.4, with LayerNorm 90 and 52, bf16 66 and 42; f32 requantizer
 // 54 and 46 there.  Without a rotation (and in the f16 gathers) there is less to wait for: always as many waves as
 // chunks.  Three chunks on two waves is the worst of both (bf16 13020 x 3072: 1 wave 28.8, 2 29.1, 3 26.4).
@@ -637,11 +638,12 @@ int run_quant(QuantArgs a, int g, hipStream_t st) {
     if (nchunks > 32) return -2;
     const bool norm = a.pro == PRO_RMS || a.pro == PRO_LAYERNORM || a.pro == PRO_ADALN || a.pro == PRO_LN_MOD || a.pro == PRO_LN_AFFINE;
     const bool light = g == 0 || a.pro == PRO_SD_UNPAD || a.pro == PRO_SD_GN;
-    const int64_t enough = norm ? 2048 : light ? INT64_MAX : 12288;
+    const int64_t enough = norm ? 2048 : MODE == MODE_F32 && a.pro == PRO_PLAIN ? 6144 : light ? INT64_MAX : 12288;
     int wpr = 1;
-    while (wpr < 8 && (nchunks + wpr - 1) / wpr > 3) wpr *= 2;
-    while (wpr < 8 && wpr < nchunks && a.M * (int64_t)wpr < enough) wpr = nchunks == 3 ? 3 : 2 * wpr;
-    wpr = wpr < nchunks ? wpr : nchunks;
+    while (wpr < 8 && (nchunks + wpr - 1) / wpr > (MODE == MODE_F32 && a.seed ? 4 : 3)) wpr *= 2;
+    while (wpr < 8 && wpr < nchunks && a.M * (int64_t)wpr < (wpr == 4 && nchunks < 11 && nchunks > 8 ? 2048 : enough))
+        wpr = nchunks == 3 ? 3 : 2 * wpr;
+    if (nchunks < 6 && wpr > nchunks) wpr = nchunks;
     const int C = (nchunks + wpr - 1) / wpr;
     const int nw = wpr < 2 ? 2 : wpr;   // two rows per workgroup at least
     a.wpr = wpr;
