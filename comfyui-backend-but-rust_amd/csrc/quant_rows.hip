@@ -623,14 +623,16 @@ int launch_c(const QuantArgs& a, int nw, int C, hipStream_t st) {
     return C == 1 ? launch<MODE, G, 1>(a, nw, st) : C == 2 ? launch<MODE, G, 2>(a, nw, st) : C == 3 ? launch<MODE, G, 3>(a, nw, st) : launch<MODE, G, 4>(a, nw, st);
 }
 
-// g: rotation group width (0, 64, 128, 256).  A row goes to 1, 2, 4 or 8 waves (six or seven chunks to eight: idle waves cost less
-// than uneven SIMDs, 2232 x 5376 bf16 8.7 and 8.4 us), up to three chunks of 1024 values each (four beyond 24 chunks, and in the
-// f32 requantizer), and to more of them where the launch would have fewer than `enough` waves: short waves overlap their loads
-// with each other's arithmetic, but a row's waves wait for its slowest, and a norm's for each other twice more; nine and ten chunks
-// on eight waves would leave a third of their slots empty.  us per call, a wave per chunk (two beyond 8 chunks, 8 waves) against this: bf16 rotate 128 4608 x 3072
-// 14.2 either way, 18601 x 5376 76 and 62; f32 7440 x 5376 40.7 and 36.4, with LayerNorm 90 and 52, bf16 66 and 42; f32 requantizer
-// 54 and 46 there.  Without a rotation (and in the f16 gathers) there is less to wait for: always as many waves as
-// chunks.  Three chunks on two waves is the worst of both (bf16 13020 x 3072: 1 wave 28.8, 2 29.1, 3 26.4).
+// g: rotation group width (0, 64, 128, 256).  A row goes to 1, 2, 4 or 8 waves, up to three chunks of 1024 values each (four beyond
+// 24 chunks, and in the f32 requantizer), and to more of them where the launch would have fewer than `enough` waves: short
+// waves overlap their loads with each other's arithmetic, but a row's waves wait for its slowest, and a norm's for each other
+// twice more.  us per call, a wave per chunk (two beyond 8 chunks, on 8 waves) against this: bf16 rotate 128 4608 x 3072 14.2 either way,
+// 18601 x 5376 76 and 62; f32 7440 x 5376 40.7 and 36.4, with LayerNorm 90 and 52, bf16 66 and 42; f32 requantizer 54 and 46 there.
+//   * Without a rotation (and in the f16 gathers) there is less to wait for: always the most waves.
+//   * Six and seven chunks go to eight waves, not to as many: idle ones cost less than uneven SIMDs (bf16 2232 x 5376 8.4, 8.8).
+//   * Nine and ten stay on four waves: on eight, a third of the slots would be empty (bf16 rotate 128 1302 x 9216 12.5, 13.6).
+//   * Three chunks on two waves and five on four are the worst of both (bf16 13020 x 3072: 1 wave 28.8, 2 29.1, 3 26.4; f16 4882 x
+//     5120: 4 waves 23.0, 5 20.3), so those go straight to a wave per chunk.
 template <int MODE>
 int run_quant(QuantArgs a, int g, hipStream_t st) {
     if (a.M <= 0) return 0;
@@ -642,8 +644,7 @@ int run_quant(QuantArgs a, int g, hipStream_t st) {
     int wpr = 1;
     while (wpr < 8 && (nchunks + wpr - 1) / wpr > (MODE == MODE_F32 && a.seed ? 4 : 3)) wpr *= 2;
     while (wpr < 8 && wpr < nchunks && a.M * (int64_t)wpr < (wpr == 4 && nchunks < 11 && nchunks > 8 ? 2048 : enough))
-        wpr = nchunks == 3 ? 3 : 2 * wpr;
-    if (nchunks < 6 && wpr > nchunks) wpr = nchunks;
+        wpr = nchunks == 3 || nchunks == 5 ? nchunks : 2 * wpr;
     const int C = (nchunks + wpr - 1) / wpr;
     const int nw = wpr < 2 ? 2 : wpr;   // two rows per workgroup at least
     a.wpr = wpr;
