@@ -236,9 +236,9 @@ int gpu_w6_decode(const void* q, const void* s_rel, void* out, int64_t N, int K,
  * Additions with no counterpart in the reference.
  * ------------------------------------------------------------------------------------------------------------- */
 
-/* Builds, for the current device, the lookup tables that the prologues GATE / SWIGLU / SILU / GELU / GELU_TANH / SITU and
- * the SD GEGLU source use on 16-bit rows (all 65536 inputs of each activation, about 1.2 MB, held until the process
- * ends).  Optional: the first call with such a prologue builds them itself, with two device allocations, a fill kernel
+/* Builds, for the current device, the lookup tables of activations of 16-bit rows (all 65536 inputs of each, about 1.2 MB,
+ * held until the process ends): GELU / GELU_TANH / SITU and the SD GEGLU source in the quantizers, and in gpu_prologue_rows[_b]
+ * GATE / SWIGLU / SILU too, which the quantizers evaluate.  Optional: the first call with such a prologue builds them itself, with two device allocations, a fill kernel
  * on a stream of its own and a wait for it -- unless its stream is being captured, in which case that call evaluates
  * the activations per element (same bits, slower) and a later call builds the tables.  Call this once at
  * start-up to keep every quantizer call asynchronous and capturable.  Returns 0, or -1 if the tables could not be
