@@ -662,16 +662,21 @@ def test_attention_drops_a_tile_of_infinite_keys(D, lk, dtype, at):
     assert (np.abs(_to_f32(got, dt) - ref) <= tol).all()
 
 
-def _keys_by_level(lk, levels, seed, D=128):
+def _keys_by_level(lk, levels, seed, D=128, aside=0.0):
     """q near ones, keys near a multiple of ones that scores levels[i] (in powers of two) in key tile i, the last level from there
-    on, and positive values (each output has a relative error then)."""
+    on, and positive values (each output has a relative error then).  aside: q is near 2 in half of the channels and 0 in the
+    others, where the keys are that many times larger, so that raw scores are small for what they are worth."""
     g = torch.Generator().manual_seed(seed)
     q = (1 + 0.02 * torch.randn(1, 40, 2, D, generator=g)).bfloat16()
     unit = 1.0 / (D ** 0.5 * 1.4426950408889634)        # key level that scores 1 against a query of ones at scale D^-0.5
     ck = 128 if lk > 1024 and D != 64 else 64
     level = torch.tensor([levels[min(i // ck, len(levels) - 1)] for i in range(lk)])
-    k = (level[:, None, None] * unit * (1 + 0.02 * torch.randn(lk, 1, D, generator=g))).unsqueeze(0).bfloat16()
-    return q, k, (1 + torch.rand(1, lk, 1, D, generator=g)).bfloat16()
+    k = (level[:, None, None] * unit * (1 + 0.02 * torch.randn(lk, 1, D, generator=g))).unsqueeze(0)
+    if aside:
+        odd = torch.arange(D) % 2 == 1
+        q = torch.where(odd, torch.zeros(()), 2 * q.float()).bfloat16()
+        k = torch.where(odd, k * aside * torch.where(torch.rand(D, generator=g) < 0.5, -1.0, 1.0), k)
+    return q, k.bfloat16(), (1 + torch.rand(1, lk, 1, D, generator=g)).bfloat16()
 
 
 @pytest.mark.parametrize("lk,levels", [(200, (-150.0, -100.0)), (1300, (-150.0, -100.0)), (200, (-120.0, -70.0)), (200, (-130.0, -90.0, -40.0))])
@@ -689,11 +694,13 @@ def test_attention_scores_far_below_the_last_tiles_floor(lk, levels):
 
 
 @pytest.mark.parametrize("lk", [200, 1300])
-@pytest.mark.parametrize("levels", [(-150.0, -100.0), (-120.0, -70.0), (-70.0, -20.0)])
-def test_attention_sink_far_above_every_key(levels, lk):
-    """All scores far below the sink's zero: each output is a tiny multiple of the values, exact to the tolerance of the test above."""
+@pytest.mark.parametrize("levels,aside", [((-150.0, -100.0), 0.0), ((-120.0, -70.0), 0.0), ((-70.0, -20.0), 0.0),
+                                          ((-150.0, -100.0), 7.0), ((-125.0, -110.0), 7.0)])
+def test_attention_sink_far_above_every_key(levels, aside, lk):
+    """All scores far below the sink's zero: each output is a tiny multiple of the values, exact to the tolerance of the test above.
+    With raw scores above -50000 (aside) the last tile's floor is below them, and the base stays where the first tile put it."""
     ql, ffi = _pkg()
-    q, k, v = _keys_by_level(lk, levels, seed=lk)
+    q, k, v = _keys_by_level(lk, levels, seed=lk, aside=aside)
     scale, sink = 128 ** -0.5, 3.0
     ref = _to_f32(oracle.attn_int8(oracle.BF16, _bits(q), _bits(k), _bits(v), scale, use_anchor=False, sink=sink), oracle.BF16)
     got = _to_f32(_bits(ql.int8_attn_sink(q.cuda(), k.cuda(), v.cuda(), scale, sink)), oracle.BF16)
