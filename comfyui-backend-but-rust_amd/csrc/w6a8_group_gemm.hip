@@ -24,6 +24,7 @@
 // every SIMD one wave's VALU-only stretch meets the other's MFMAs.
 #include "common.hpp"
 #include <atomic>
+#include <type_traits>
 
 #define SCHED_FENCE() __builtin_amdgcn_sched_barrier(0)
 
@@ -72,6 +73,94 @@ template <int N> __device__ __forceinline__ void wait_vmcnt_n() { asm volatile("
 __device__ __forceinline__ void wait_all_dma() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 __device__ __forceinline__ void dma4(uint32_t lds_dst, uint32_t lane_off, const void* base) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_dst), "v"(lane_off), "s"(base) : "memory", "m0");
+}
+
+// Epilogue of a wave's FM x FN tiles, accf[column tile][row tile][c], whose first row is mw and first column nb; `wl` is LDS of the
+// wave's own, 32 rows of its columns.  A lane holds one m per row tile and four consecutive n per column tile, so storing straight
+// from the registers would touch 16 rows per instruction.  When the rows of D are 16-byte aligned each wave instead passes its
+// tile, 32 rows at a time, through LDS (16-byte chunks XOR-swizzled by row) and writes whole row segments, 16 bytes per lane.
+template <int OUT_DT, int FM, int FN>
+__device__ __forceinline__ void store_wave_tile(const W6Args& p, uint8_t* wl, const float (&accf)[FN][FM][4], const int mw, const int nb, const int lane) {
+    const int frow = lane & 15, fq = lane >> 4;
+    constexpr int SZ = dt_size<OUT_DT>::value;
+    const bool vec_ok = (p.N & 3) == 0 && ((uintptr_t)p.D & (4 * SZ - 1)) == 0 && ((uintptr_t)p.bias & (4 * SZ - 1)) == 0;
+    const bool rows_ok = vec_ok && (((int64_t)p.N * SZ) & 15) == 0 && ((uintptr_t)p.D & 15) == 0;
+    float bv[FN][4];
+#pragma unroll
+    for (int in = 0; in < FN; ++in) {
+        const int n = nb + 16 * in + 4 * fq;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) bv[in][c] = 0.f;
+        if (p.bias && n < p.N) {
+            if (vec_ok) {
+                load4<OUT_DT>(p.bias, n, bv[in]);
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) if (n + c < p.N) bv[in][c] = ld_dt<OUT_DT>(p.bias, n + c);
+            }
+        }
+    }
+    if (rows_ok) {
+        constexpr int ROWB = 16 * FN * SZ, CPR = ROWB / 16;     // bytes and 16-byte chunks per LDS row
+        constexpr int RPI = 64 / CPR, NI = 32 / RPI;            // rows per store instruction, instructions per piece
+#pragma unroll
+        for (int ip = 0; ip < FM / 2; ++ip) {                    // a piece: row tiles 2*ip and 2*ip + 1
+            const int mb = mw + ip * 32;
+#pragma unroll
+            for (int hm = 0; hm < 2; ++hm) {
+                const int prow = hm * 16 + frow;
+                const float xs = p.xs[mb + prow < p.M ? mb + prow : p.M - 1];
+#pragma unroll
+                for (int in = 0; in < FN; ++in) {
+                    float out[4];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) out[c] = __builtin_fmaf(accf[in][2 * ip + hm][c], xs, bv[in][c]);
+                    const int byte = (16 * in + 4 * fq) * SZ;    // columns 16*in + 4*fq .. +3 of row prow
+                    uint8_t* dst = wl + prow * ROWB + ((((byte >> 4) ^ (prow & (CPR - 1))) << 4) | (byte & 15));
+                    if (OUT_DT == DT_F32) {
+                        *reinterpret_cast<float4*>(dst) = make_float4(out[0], out[1], out[2], out[3]);
+                    } else if (OUT_DT == DT_BF16) {
+                        *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(out[0], out[1]), pack_bf16x2(out[2], out[3]));
+                    } else {
+                        *reinterpret_cast<uint2*>(dst) = make_uint2((uint32_t)f_to_f16(out[0]) | ((uint32_t)f_to_f16(out[1]) << 16),
+                                                                    (uint32_t)f_to_f16(out[2]) | ((uint32_t)f_to_f16(out[3]) << 16));
+                    }
+                }
+            }
+            asm volatile("" ::: "memory");   // the wave's own LDS writes are ordered before its reads
+#pragma unroll
+            for (int t = 0; t < NI; ++t) {
+                const int row = t * RPI + lane / CPR, ch = lane % CPR;
+                const uint4 v = *reinterpret_cast<const uint4*>(wl + row * ROWB + ((ch ^ (row & (CPR - 1))) << 4));
+                const int m = mb + row, n = nb + ch * (16 / SZ);
+                if (m < p.M && n < p.N) *reinterpret_cast<uint4*>((uint8_t*)p.D + ((int64_t)m * p.N + n) * SZ) = v;
+            }
+            asm volatile("" ::: "memory");   // ... and the reads before the next piece's writes
+        }
+        return;
+    }
+    // fallback for unaligned rows: four consecutive n per lane and tile, straight from the accumulators
+#pragma unroll
+    for (int im = 0; im < FM; ++im) {
+        const int m = mw + im * 16 + frow;
+        if (m >= p.M) continue;
+        const float xs = p.xs[m];
+#pragma unroll
+        for (int in = 0; in < FN; ++in) {
+            const int n = nb + 16 * in + 4 * fq;
+            if (n >= p.N) continue;
+            const int64_t o = (int64_t)m * p.N + n;
+            float out[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) out[c] = __builtin_fmaf(accf[in][im][c], xs, bv[in][c]);
+            if (vec_ok) {
+                store4<OUT_DT>(p.D, o, out);
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) if (n + c < p.N) st_dt<OUT_DT>(p.D, o + c, out[c]);
+            }
+        }
+    }
 }
 
 // ABL (measurement only, wrong results): bit 0 leaves out the fp32 fold, bit 1 the unpack, bit 2 the DMA of the MFMA
@@ -328,91 +417,148 @@ __global__ void __launch_bounds__(NT, 1) w6a8_group_gemm_kernel(W6Args p) {
     }
     __syncthreads();   // every wave's DMA is drained before the epilogue reuses the stages
 
-    // Epilogue.  A lane holds one m per row tile and four consecutive n per column tile, so storing straight from the
-    // registers would touch 16 rows per instruction.  When the rows of D are 16-byte aligned each wave instead passes its
-    // tile, 32 rows at a time, through a private 4 KB of LDS (16-byte chunks XOR-swizzled by row) and writes whole row
-    // segments, 16 bytes per lane.
-    constexpr int SZ = dt_size<OUT_DT>::value;
-    const bool vec_ok = (p.N & 3) == 0 && ((uintptr_t)p.D & (4 * SZ - 1)) == 0 && ((uintptr_t)p.bias & (4 * SZ - 1)) == 0;
-    const bool rows_ok = vec_ok && (((int64_t)p.N * SZ) & 15) == 0 && ((uintptr_t)p.D & 15) == 0;
-    const int nb = n0 + wn * 32;
-    float bv[FN][4];
+    store_wave_tile<OUT_DT, FM, FN>(p, smem + wave * 4096, accf, m0 + wm * 128, n0 + wn * 32, lane);   // the stages are idle
+}
+
+// The W8 form on 256 x 256 tiles: eight waves of 128 x 64, so that a group costs a wave 24 fragment reads for 64 MFMAs where the
+// 256 x 128 tile costs it 20 for 32, and a CU 64 KB of DMA where two of the smaller tiles cost 96.  256 registers hold that because a
+// lane's int32 partials live only from one row tile to the next: while the eight MFMAs of a row tile run, the fold of the one before
+// rides between them, four vector instructions to an MFMA (a probe of this mix: 24.7 cycles per MFMA and SIMD; the same MFMAs
+// and vector instructions in blocks take 31-35 from one wave and lean on the other one for the rest).  Two LDS stages of A, W and
+// scales: group g+1 travels during group g, one barrier per group.  The four lower waves issue all DMA, one instruction after
+// every other MFMA: every wave fetching its own share has both waves of a SIMD held by a DMA instruction at the same time
+// (M=8192, K=5120 -> N=13824 638 us, this way 617; K=13824 -> N=5120 646 and 630; the DMA free of charge would be 556 and 580).
+// The same tile with v_mfma_i32_32x32x32_i8, which leaves more issue slots to the fold, takes 677 us: the chip is at its power limit.
+// A persistent form with the next tile's first group under the epilogue: no change.
+// M=8192, K=5120 -> N=13824, expansion included: 256 x 128 tiles 756 us, these 617.  What is left is the fold next to the MFMAs
+// (64 MFMAs and 256 vector instructions per wave and group: 3161 cycles of a SIMD against 2048 for the MFMAs alone) at 2.0 GHz.
+constexpr int BIG_BN = 256, BIG_U = BIG_BN * BK, BIG_U_BASE = 2 * A_STAGE, BIG_S_BASE = BIG_U_BASE + 2 * BIG_U, BIG_S = BIG_BN * 4;
+constexpr int BIG_SMEM = BIG_S_BASE + 2 * BIG_S;
+
+template <int OUT_DT>
+__global__ void __launch_bounds__(NT, 1) w6a8_group_gemm_big_kernel(W6Args p) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 2, wn = wave & 3;
+    int tm, tn;
+    tile_of_block((int)blockIdx.x, (int)gridDim.x, p.tiles_m, p.tiles_n, tm, tn);
+    // The last tiles of a row or column of tiles are moved back inside the matrix, so that every row and column of a tile exists
+    // (M, N >= 256) and a wave's DMA needs one lane offset for all of them; what two tiles share, both store alike.
+    const int m0 = tm * BM < p.M - BM ? tm * BM : p.M - BM, n0 = tn * BIG_BN < p.N - BIG_BN ? tn * BIG_BN : p.N - BIG_BN, ng = p.ng;
+    const uint32_t lds_base = (uint32_t)(uintptr_t)smem;
+    constexpr int FM = 8, FN = 4;
+
+    // DMA of the lower waves: rows in blocks of 8, wave w takes blocks w + 4j of W and of A and the scales of columns 64w .. 64w+63
+    const uint32_t lrow = (uint32_t)lane >> 3;
+    const uint32_t goff = lrow * (uint32_t)p.K + ((lane & 7) ^ (((wave & 1) << 2) | (lrow >> 1))) * 16;
+    const uint32_t gs = (uint32_t)lane * (uint32_t)ng * 4u;
+    const int8_t* a_base = p.A + (int64_t)(m0 + wn * 8) * p.K;
+    const int8_t* w_base = p.W8 + (int64_t)(n0 + wn * 8) * p.K;
+    const float* s_base = p.sw + (int64_t)(n0 + wn * 64) * ng;
+    const int64_t jstep = (int64_t)32 * p.K;
+    constexpr int NDMA = 17;
+    auto dma = [&](int g, int j) {   // groups past the end re-fetch the last one, which nothing reads
+        const int gc = g < ng ? g : ng - 1, stage = g & 1;
+        if (j < 8) dma16(lds_base + BIG_U_BASE + stage * BIG_U + (wn + 4 * j) * 1024, goff, w_base + j * jstep + (int64_t)gc * BK);
+        else if (j < 16) dma16(lds_base + stage * A_STAGE + (wn + 4 * (j - 8)) * 1024, goff, a_base + (j - 8) * jstep + (int64_t)gc * BK);
+        else dma4(lds_base + BIG_S_BASE + stage * BIG_S + wn * 256, gs, s_base + gc);
+    };
+    const int frow = lane & 15, fq = lane >> 4;
+    const int fsw = (fq ^ ((frow >> 1) & 7)) << 4;
+    const int aoff = (wm * 128 + frow) * BK + fsw, woff = (wn * 64 + frow) * BK + fsw;
+
+    v4i part[2][FN];           // int32 partials of a row tile and of the one before
+    float accf[FN][FM][4];
+    float4 sv[FN];
 #pragma unroll
     for (int in = 0; in < FN; ++in) {
-        const int n = nb + 16 * in + 4 * fq;
+        part[1][in] = v4i{0, 0, 0, 0};
+        sv[in] = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) bv[in][c] = 0.f;
-        if (p.bias && n < p.N) {
-            if (vec_ok) {
-                load4<OUT_DT>(p.bias, n, bv[in]);
-            } else {
+        for (int im = 0; im < FM; ++im)
 #pragma unroll
-                for (int c = 0; c < 4; ++c) if (n + c < p.N) bv[in][c] = ld_dt<OUT_DT>(p.bias, n + c);
-            }
-        }
+            for (int r = 0; r < 4; ++r) accf[in][im][r] = 0.f;
     }
-    if (rows_ok) {
-        constexpr int ROWB = 32 * SZ, CPR = ROWB / 16;          // bytes and 16-byte chunks per LDS row (32 columns)
-        constexpr int RPI = 64 / CPR, NI = 32 / RPI;            // rows per store instruction, instructions per piece
-        uint8_t* wl = smem + wave * 4096;                        // the stages are idle: the loop ended with a barrier
+    // two of a tile's four values
+    auto fold2 = [&](int buf, int in, int im, int c0) {
+        const float s4[4] = {sv[in].x, sv[in].y, sv[in].z, sv[in].w};
 #pragma unroll
-        for (int ip = 0; ip < FM / 2; ++ip) {                    // a piece: row tiles 2*ip and 2*ip + 1
-            const int mb = m0 + wm * 128 + ip * 32;
+        for (int c = c0; c < c0 + 2; ++c) accf[in][im][c] = __builtin_fmaf((float)part[buf][in][c], s4[c], accf[in][im][c]);
+    };
+    // No branch inside: the compiler would move the folds behind it.
+    auto loop = [&](auto fetches_tag) {
+        constexpr bool fetches = decltype(fetches_tag)::value;
+        if constexpr (fetches) {
 #pragma unroll
-            for (int hm = 0; hm < 2; ++hm) {
-                const int prow = hm * 16 + frow;
-                const float xs = p.xs[mb + prow < p.M ? mb + prow : p.M - 1];
+            for (int j = 0; j < NDMA; ++j) dma(0, j);
+            wait_all_dma();
+        }
+        __syncthreads();
+        for (int g = 0; g < ng; ++g) {
+            const uint8_t* sa = smem + (g & 1) * A_STAGE;
+            const uint8_t* su = smem + BIG_U_BASE + (g & 1) * BIG_U;
+            const float* sc = reinterpret_cast<const float*>(smem + BIG_S_BASE + (g & 1) * BIG_S);
+            v4i fw[FN][2], fa[2][2];
+            auto read_a = [&](int im) {
 #pragma unroll
-                for (int in = 0; in < FN; ++in) {
-                    float out[4];
+                for (int h = 0; h < 2; ++h) fa[im & 1][h] = *reinterpret_cast<const v4i*>(sa + ((aoff + im * 16 * BK) ^ (h << 6)));
+            };
+            read_a(0);
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) out[c] = __builtin_fmaf(accf[in][2 * ip + hm][c], xs, bv[in][c]);
-                    const int byte = (16 * in + 4 * fq) * SZ;    // columns 16*in + 4*fq .. +3 of row prow
-                    uint8_t* dst = wl + prow * ROWB + ((((byte >> 4) ^ (prow & (CPR - 1))) << 4) | (byte & 15));
-                    if (OUT_DT == DT_F32) {
-                        *reinterpret_cast<float4*>(dst) = make_float4(out[0], out[1], out[2], out[3]);
-                    } else if (OUT_DT == DT_BF16) {
-                        *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(out[0], out[1]), pack_bf16x2(out[2], out[3]));
-                    } else {
-                        *reinterpret_cast<uint2*>(dst) = make_uint2((uint32_t)f_to_f16(out[0]) | ((uint32_t)f_to_f16(out[1]) << 16),
-                                                                    (uint32_t)f_to_f16(out[2]) | ((uint32_t)f_to_f16(out[3]) << 16));
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int in = 0; in < FN; ++in) fw[in][h] = *reinterpret_cast<const v4i*>(su + ((woff + in * 16 * BK) ^ (h << 6)));
+            SCHED_FENCE();
+#pragma unroll
+            for (int in = 0; in < FN; ++in) {   // the last row tile of the group before, under the first reads of this one
+                fold2(1, in, FM - 1, 0);
+                fold2(1, in, FM - 1, 2);
+            }
+            SCHED_FENCE();
+#pragma unroll
+            for (int in = 0; in < FN; ++in) sv[in] = *reinterpret_cast<const float4*>(sc + wn * 64 + 16 * in + 4 * fq);
+#pragma unroll
+            for (int im = 0; im < FM; ++im) {
+                if (im + 1 < FM) read_a(im + 1);
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int in = 0; in < FN; ++in) {
+                        const int slot = h * 4 + in, j = im * 4 + (slot >> 1);
+                        const v4i c = h == 0 ? v4i{0, 0, 0, 0} : part[im & 1][in];
+                        part[im & 1][in] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fw[in][h], fa[im & 1][h], c, 0, 0, 0);
+                        SCHED_FENCE();
+                        if (im > 0) fold2((im - 1) & 1, slot >> 1, im - 1, 2 * (slot & 1));
+                        if (fetches && (slot & 1) == 0 && j < NDMA) dma(g + 1, j);   // the stage last read before the previous barrier
+                        SCHED_FENCE();
                     }
-                }
             }
-            asm volatile("" ::: "memory");   // the wave's own LDS writes are ordered before its reads
-#pragma unroll
-            for (int t = 0; t < NI; ++t) {
-                const int row = t * RPI + lane / CPR, ch = lane % CPR;
-                const uint4 v = *reinterpret_cast<const uint4*>(wl + row * ROWB + ((ch ^ (row & (CPR - 1))) << 4));
-                const int m = mb + row, n = nb + ch * (16 / SZ);
-                if (m < p.M && n < p.N) *reinterpret_cast<uint4*>((uint8_t*)p.D + ((int64_t)m * p.N + n) * SZ) = v;
-            }
-            asm volatile("" ::: "memory");   // ... and the reads before the next piece's writes
+            if constexpr (fetches) wait_all_dma();
+            __syncthreads();
         }
-        return;
+    };
+    if (wm == 0) loop(std::true_type{});
+    else loop(std::false_type{});
+#pragma unroll
+    for (int in = 0; in < FN; ++in) {
+        fold2(1, in, FM - 1, 0);
+        fold2(1, in, FM - 1, 2);
     }
-    // fallback for unaligned rows: four consecutive n per lane and tile, straight from the accumulators
-#pragma unroll
-    for (int im = 0; im < FM; ++im) {
-        const int m = m0 + wm * 128 + im * 16 + frow;
-        if (m >= p.M) continue;
-        const float xs = p.xs[m];
-#pragma unroll
-        for (int in = 0; in < FN; ++in) {
-            const int n = nb + 16 * in + 4 * fq;
-            if (n >= p.N) continue;
-            const int64_t o = (int64_t)m * p.N + n;
-            float out[4];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) out[c] = __builtin_fmaf(accf[in][im][c], xs, bv[in][c]);
-            if (vec_ok) {
-                store4<OUT_DT>(p.D, o, out);
-            } else {
-#pragma unroll
-                for (int c = 0; c < 4; ++c) if (n + c < p.N) st_dt<OUT_DT>(p.D, o + c, out[c]);
-            }
-        }
-    }
+    // the lane number is taken anew so that the loop does not keep it
+    store_wave_tile<OUT_DT, FM, FN>(p, smem + wave * 8192, accf, m0 + wm * 128, n0 + wn * 64,
+                                    (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)));
+}
+
+template <int OUT_DT>
+int launch_big(W6Args a, hipStream_t st) {
+    auto kern = w6a8_group_gemm_big_kernel<OUT_DT>;
+    static PerDeviceOnce once;
+    if (const int e = allow_dynamic_lds((const void*)kern, BIG_SMEM, once)) return e;
+    a.tiles_n = (a.N + BIG_BN - 1) / BIG_BN;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(a.tiles_m * a.tiles_n)), dim3(NT), BIG_SMEM, st, a);
+    KCHECK();
+    return 0;
 }
 
 template <int OUT_DT, bool DUMP, int ABL = 0, bool W8 = false>
@@ -427,7 +573,8 @@ int launch(W6Args a, hipStream_t st) {
 }
 
 template <int OUT_DT>
-int launch_dt(const W6Args& a, hipStream_t st) {
+int launch_dt(const W6Args& a, bool big, hipStream_t st) {
+    if (big) return launch_big<OUT_DT>(a, st);
     if (a.W8) return a.partials ? launch<OUT_DT, true, 0, true>(a, st) : launch<OUT_DT, false, 0, true>(a, st);
     return a.partials ? launch<OUT_DT, true>(a, st) : launch<OUT_DT, false>(a, st);
 }
@@ -442,12 +589,30 @@ __global__ void __launch_bounds__(256) w6_words_to_int8_kernel(const uint8_t* Wp
     }
 }
 
-// From this many rows of A on, the weights are expanded once into a stream-ordered scratch and the kernel fetches them
-// like A; below, every workgroup expands its own 128 columns as it goes.  Each weight is used by M / 256 workgroups:
-// expanding it that many times costs the large-M shapes more vector issue slots than the int8 round trip through HBM
-// costs them time (M = 8192: 9 % faster; M = 2048: 10 % slower, the expansion being a fixed 25-30 us).
-constexpr int64_t kExpandFirstRows = 4096;
-std::atomic<int> g_mode{-1};   // test hook: 0 = always fused, 1 = always expand first, -1 = by M
+// Which form runs.  Fused, every workgroup expands its own 128 columns as it goes; the other two expand the packed weights once into
+// a scratch of N*K bytes and multiply 256 x 128 or 256 x 256 tiles of them.  A launch takes whole rounds of one tile per CU, and a
+// round takes a fixed time per group, in us on random codes: 1.42 fused (K=5120 -> N=13824: 1024 rows 115 us, 2048 228, 3072 342,
+// 8192 816), 1.26 (121, 222, 325, 745 with the expansion) and 2.05 (98, 178, 261, 611); the expansion takes about 6 us and 3.7 bytes
+// per ns.  The smallest sum runs: 512 rows of that shape fused (60 us, 71, 90), 1536 rows alike in all three (172); 4096 -> 4096
+// 2048 rows fused (54; 54, 67), 3072 on large tiles (69; 93 fused), 13824 -> 5120 1024 rows 142, 140 and 196, 2048 rows 284, 265 and 197.
+// From kExpandRows rows on the weights are always expanded (1024 -> 2048, 4096 rows: fused 20 us, expanded 22).  Below, only into a
+// scratch that the caller brings: a call without one makes no allocation there.
+constexpr int64_t kExpandRows = 4096;
+enum Form { kFused, kTiles128, kTiles256 };
+std::atomic<int> g_mode{-1};   // test hook: 0 = fused, 1 = expanded, 2 = expanded, 128 columns per tile, 3 = 256 columns, -1 = by the rule
+
+Form pick_form(const void* Wp, int64_t M, int64_t N, int64_t K, bool may_expand) {
+    const int mode = g_mode.load(std::memory_order_relaxed);
+    if (mode == 0 || N * K >= ((int64_t)1 << 32) || ((uintptr_t)Wp & 3) != 0) return kFused;
+    const int64_t cus = device_cu_count(), tm = (M + BM - 1) / BM, t128 = tm * ((N + BN - 1) / BN), t256 = tm * ((N + BIG_BN - 1) / BIG_BN);
+    const bool fits256 = M >= BM && N >= BIG_BN;
+    if (mode >= 2) return mode == 3 && fits256 ? kTiles256 : kTiles128;
+    const double ng = (double)(K / 128), expand = 6.0 + (double)N * (double)K / 3.7e6;
+    const double fused = ng * 1.42 * (double)((t128 + cus - 1) / cus), small = ng * 1.26 * (double)((t128 + cus - 1) / cus);
+    const double large = fits256 ? ng * 2.05 * (double)((t256 + cus - 1) / cus) : 1e30;
+    if (mode != 1 && M < kExpandRows && (!may_expand || fused <= expand + (small < large ? small : large))) return kFused;
+    return large < small ? kTiles256 : kTiles128;
+}
 
 // 32-bit DMA lane offsets into A, the packed weights and the scales; a tile count that fits the grid
 bool shape_fits(int64_t M, int64_t N, int64_t K) {
@@ -456,20 +621,15 @@ bool shape_fits(int64_t M, int64_t N, int64_t K) {
     return ((M + BM - 1) / BM) * ((N + BN - 1) / BN) <= 0x7fffffff;
 }
 
-bool expands_first(const void* Wp, int64_t M, int64_t N, int64_t K) {
-    const int mode = g_mode.load(std::memory_order_relaxed);
-    return (mode == 1 || (mode != 0 && M >= kExpandFirstRows)) && N * K < ((int64_t)1 << 32) && ((uintptr_t)Wp & 3) == 0;
-}
-
 }  // namespace
 
 GPU_API int64_t gpu_w6a8_group_gemm_scratch(const void* Wp, int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || (K % 128) != 0 || !shape_fits(M, N, K)) return 0;
-    return expands_first(Wp, M, N, K) ? N * K : 0;
+    return pick_form(Wp, M, N, K, true) != kFused ? N * K : 0;
 }
 
 // `scratch`: what gpu_w6a8_group_gemm_scratch asks for, kept by the caller or taken from the allocator that the rest of its
-// tensors come from.  Without one the call makes a stream-ordered allocation of that size, which the default pool gives
+// tensors come from.  Without one a call of 4096 rows or more makes a stream-ordered allocation of that size, which the default pool gives
 // back at every synchronization and takes again at the next call with the host waiting (M=8192, K=5120 -> N=13824 behind
 // a synchronization: 1112 us, 758 with a scratch).
 GPU_API int gpu_w6a8_group_gemm_ws(const int8_t* A, const void* Wp, const float* xs, const float* sw, const void* bias, void* D,
@@ -484,7 +644,8 @@ GPU_API int gpu_w6a8_group_gemm_ws(const int8_t* A, const void* Wp, const float*
     hipStream_t st = (hipStream_t)stream;
     if ((uintptr_t)scratch & 15) return -1;   // stored 16 bytes at a time
     int8_t* own = nullptr;
-    if (expands_first(Wp, M, N, K)) {
+    const Form form = pick_form(Wp, M, N, K, scratch != nullptr);
+    if (form != kFused) {
         int8_t* w8 = (int8_t*)scratch;
         if (!w8) {
             hipError_t e = hipMallocAsync((void**)&own, (size_t)(N * K), st);
@@ -496,11 +657,12 @@ GPU_API int gpu_w6a8_group_gemm_ws(const int8_t* A, const void* Wp, const float*
         hipLaunchKernelGGL(w6_words_to_int8_kernel, dim3(grid), dim3(256), 0, st, (const uint8_t*)Wp, w8, pieces);
         a.W8 = w8;
     }
+    const bool big = form == kTiles256 && !partials;   // the partials are dumped by the 128-column tiles
     int rc;
     switch (out_dt) {
-        case DT_F32: rc = launch_dt<DT_F32>(a, st); break;
-        case DT_F16: rc = launch_dt<DT_F16>(a, st); break;
-        default: rc = launch_dt<DT_BF16>(a, st); break;
+        case DT_F32: rc = launch_dt<DT_F32>(a, big, st); break;
+        case DT_F16: rc = launch_dt<DT_F16>(a, big, st); break;
+        default: rc = launch_dt<DT_BF16>(a, big, st); break;
     }
     if (own) {
         hipError_t e = hipFreeAsync(own, st);
@@ -515,7 +677,7 @@ GPU_API int gpu_w6a8_group_gemm(const int8_t* A, const void* Wp, const float* xs
 }
 
 // Test hook, no reference counterpart: 0 = gpu_w6a8_group_gemm always expands the weights inside the kernel, 1 = always
-// expands them first, -1 = chooses by M.
+// expands them first, 2 and 3 the same with tiles of 128 and 256 columns, -1 = chooses by the sizes.
 GPU_API int gpu_internal_w6a8_group_gemm_mode(int mode) {
     g_mode.store(mode, std::memory_order_relaxed);
     return 0;

@@ -195,8 +195,9 @@ int gpu_internal_w6a8_group_gemm_ablate(int ablate, const int8_t* A, const void*
                                         int64_t M, int64_t N, int64_t K, void* stream);
 
 /* Test hook, no reference counterpart: which form of gpu_w6a8_group_gemm runs.  0 = the weights are expanded to int8
- * inside the kernel, per workgroup; 1 = they are expanded once into a stream-ordered scratch (N*K bytes) and the kernel
- * fetches them like A; -1 = by M (the second form from 4096 rows on).  Both forms give the same bits. */
+ * inside the kernel, per workgroup; 1 = they are expanded once into a scratch of N*K bytes and the kernel fetches them like
+ * A, on tiles of 128 or 256 columns by the sizes; 2 and 3 = the same on tiles of 128 and (from 256 rows and columns on) 256
+ * columns; -1 = by the sizes.  All forms give the same bits. */
 int gpu_internal_w6a8_group_gemm_mode(int mode);
 
 /* Test hook, no reference counterpart: sums of squares of rows of 128 floats in the order the fused norm of
@@ -281,10 +282,10 @@ int gpu_w6a8_gemm_ws(const int8_t* A, const void* wq, const void* s_rel, int G, 
                      const void* bias, void* D, void* scratch, int64_t M, int64_t N, int64_t K, int out_dt, void* stream);
 
 /* W6A8 linear with fp32 scales per group of 128 along K, for this library's own packed format (no counterpart in the
- * reference, whose W6 weights are two-plane with e4m3 group factors: gpu_w6_decode / gpu_w6a8_gemm above).  Up to 4095
- * rows of A the weights are expanded to int8 inside the GEMM kernel, ahead of the MFMA; from 4096 rows on they are
- * expanded once into a stream-ordered scratch of N*K bytes (hipMallocAsync / hipFreeAsync on the call's stream) that
- * the same kernel then fetches like A.  Same bits either way.
+ * reference, whose W6 weights are two-plane with e4m3 group factors: gpu_w6_decode / gpu_w6a8_gemm above).  Below
+ * 4096 rows of A this call expands the weights to int8 inside the GEMM kernel, ahead of the MFMA, and allocates nothing; from
+ * 4096 rows on they are expanded once into a stream-ordered scratch of N*K bytes (hipMallocAsync / hipFreeAsync on the call's
+ * stream) that the kernel then fetches like A.  Same bits either way.
  *   Wp  uint8 [N, 3K/4]: codes u = q + 32 with q in [-32, 31]; every three bytes are the little-endian 24-bit word
  *       u0 | u1 << 6 | u2 << 12 | u3 << 18 of four consecutive k.
  *   sw  f32 [N, K/128]: one scale per output channel and group of 128 along K.
@@ -296,7 +297,8 @@ int gpu_w6a8_gemm_ws(const int8_t* A, const void* wq, const void* s_rel, int G, 
 int gpu_w6a8_group_gemm(const int8_t* A, const void* Wp, const float* xs, const float* sw, const void* bias, void* D,
                         int32_t* partials, int64_t M, int64_t N, int64_t K, int out_dt, void* stream);
 /* The same with the caller's scratch, 16-byte aligned (-1 otherwise), of the bytes that gpu_w6a8_group_gemm_scratch names
- * for the call (0: none is used), in use until the work queued here has run; null allocates as above. */
+ * for the call (0: none is used), in use until the work queued here has run; null is the call above.  With a scratch the weights
+ * are expanded first wherever that is the faster form, also below 4096 rows. */
 int gpu_w6a8_group_gemm_ws(const int8_t* A, const void* Wp, const float* xs, const float* sw, const void* bias, void* D,
                            int32_t* partials, void* scratch, int64_t M, int64_t N, int64_t K, int out_dt, void* stream);
 int64_t gpu_w6a8_group_gemm_scratch(const void* Wp, int64_t M, int64_t N, int64_t K);

@@ -1415,6 +1415,39 @@ def _w6a8_group_case(M, N, K, out_dt, with_bias):
     assert np.array_equal(host_bits(got2).view(view), want.view(view))
 
 
+@pytest.mark.parametrize("M,N,K,out_dt,with_bias", [
+    (256, 256, 128, BF16, True), (257, 300, 256, F32, True), (511, 261, 384, BF16, False), (700, 776, 640, F16, True),
+    (300, 1028, 128, F32, False), (2303, 260, 256, BF16, True),
+])
+def test_w6a8_group_gemm_large_tiles(M, N, K, out_dt, with_bias):
+    """256 x 256 tiles of expanded weights, bit for bit: whole tiles, tiles moved back inside the matrix by one row or column up to all
+    but one, rows of D that are not of whole 16 bytes."""
+    ffi.raw("gpu_internal_w6a8_group_gemm_mode", 3)
+    try:
+        _w6a8_group_case(M, N, K, out_dt, with_bias)
+    finally:
+        ffi.raw("gpu_internal_w6a8_group_gemm_mode", -1)
+
+
+def test_w6a8_group_gemm_form_needs_the_callers_scratch_below_4096_rows():
+    """2048 x 5120 -> 13824 expands its weights into a scratch that the caller brings; without one the call stays fused and allocates
+    nothing, and both give the same bits."""
+    M, N, K = 2048, 13824, 5120
+    A, xs = dev(rand_i8(11, 1, M, K, -127, 127)), dev(synth.uniform(11, 2, M, 0.01, 0.1))
+    wq, sw = dev(rand_i8(11, 3, N, K // 4 * 3, -128, 127)).view(torch.uint8), dev(synth.uniform(11, 5, N * (K // 128), 1e-3, 1e-2))
+    ptr, st = (lambda t: t.data_ptr()), torch.cuda.current_stream().cuda_stream
+    assert ffi.lib.gpu_w6a8_group_gemm_scratch(ptr(wq), M, N, K) == N * K
+    assert ffi.lib.gpu_w6a8_group_gemm_scratch(ptr(wq) + 1, M, N, K) == 0 and ffi.lib.gpu_w6a8_group_gemm_scratch(ptr(wq), 512, N, K) == 0
+    outs = []
+    for w8 in (torch.full((N * K + 64,), 77, dtype=torch.int8, device=DEV), None):
+        D = torch.zeros((M, N), dtype=torch.bfloat16, device=DEV)
+        ffi.k("gpu_w6a8_group_gemm_ws", ptr(A), ptr(wq), ptr(xs), ptr(sw), 0, ptr(D), 0, ptr(w8) if w8 is not None else 0, M, N, K, BF16, st)
+        torch.cuda.synchronize()
+        assert w8 is None or bool((w8[N * K:] == 77).all())
+        outs.append(D.view(torch.int16))
+    assert torch.equal(outs[0], outs[1])
+
+
 def test_w6a8_group_gemm_argument_checks():
     assert ffi.raw("gpu_w6a8_group_gemm", 0, 0, 0, 0, 0, 0, 0, 4, 8, 64, 2, 0) == -1      # K % 128
     assert ffi.raw("gpu_w6a8_group_gemm", 0, 0, 0, 0, 0, 0, 0, 4, 8, 128, 7, 0) == -200   # out_dt
