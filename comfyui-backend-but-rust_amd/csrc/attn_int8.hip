@@ -200,9 +200,8 @@ __device__ inline float sumsq128_serial(const float* x, bool split) {
 }
 
 __device__ __forceinline__ void round_bf16x2(float& x, float& y) {
-    const uint32_t u = pack_bf16x2(x, y);
-    x = u2f(u << 16);
-    y = u2f(u & 0xffff0000u);
+    x = rnd_bf16(x);
+    y = rnd_bf16(y);
 }
 
 // Per-head RMSNorm, weight and RoPE of one 128-channel row held by eight lanes (sixteen adjacent channels each), as the

@@ -118,9 +118,8 @@ __global__ void __launch_bounds__(1024) w6_requant_kernel(const uint16_t* w, uin
         m = 0.f;
 #pragma unroll
         for (int i = 0; i < 16; i += 2) {
-            const uint32_t u = pack_bf16x2(v[c][i], v[c][i + 1]);
-            v[c][i] = u2f(u << 16);
-            v[c][i + 1] = u2f(u & 0xffff0000u);
+            v[c][i] = rnd_bf16(v[c][i]);
+            v[c][i + 1] = rnd_bf16(v[c][i + 1]);
             m = fmaxf(fmaxf(m, fabsf(v[c][i])), fabsf(v[c][i + 1]));
         }
         // the group's step by two alternating-least-squares rounds, :94-117.  num adds its 32 terms in index order: the odd
