@@ -46,6 +46,9 @@ struct AttnArgs {
     int q_norm, k_norm, rope_mode;
     const float* bias;    // per-key logit bias of the caller, f32 [lk], or null
     float* kbias;         // prepared: bias * log2e per key of every tile (-inf: not kept / padding), then one value per tile
+    int whole, parts;     // row blocks with one workgroup each; workgroups that share the keys of every other row block
+    float* part;          // their results, and per row block how many of them are there
+    uint32_t* done;
     float* tbias;         // per tile: the bias all its keys share (times log2e), NaN when they differ, -inf when none is kept
 };
 
@@ -650,6 +653,8 @@ __device__ __forceinline__ void v_absmax_body(const AttnArgs& a, const int hi, c
 // Stage 2: K (needs the anchors) and the V abs-max (needs the cleared accumulators).
 template <int DT, int D, int NM>
 __global__ __launch_bounds__(256) void attn_stage1_kernel(AttnArgs a) {
+    if (a.parts > 1)   // finished parts, counted by the attention kernel
+        for (int i = blockIdx.x * 256 + threadIdx.x; i < (a.lq + 127) / 128 * a.h * a.b - a.whole; i += gridDim.x * 256) a.done[i] = 0u;
     int id = blockIdx.x;
     const int n_anchor = a.hk * a.b;
     if (id < n_anchor) {
@@ -1079,10 +1084,23 @@ __device__ __forceinline__ float swap32_sum(float x) {
     return u2f(r[0]) + u2f(r[1]);
 }
 
+// First key tile of part p.  The second of two halves is shorter by two tiles or three, so that it has written its result when the
+// first one ends, which then keeps its own in registers.
+__device__ __forceinline__ int part_bound(int kb, int parts, int p) { return kb * p / parts + (parts == 2 && p == 1 ? 1 : 0); }
+// Two floats to and from memory past the caches that XCDs do not share: agent-scope stores are written through and acknowledged where
+// every XCD sees them, agent-scope loads are not served from a stale line.  So a part's result needs a wait for its own stores ahead
+// of its counter, and no write-back of the whole L2 (a __threadfence per part costs more than the parts gain).
+__device__ __forceinline__ void store_agent(float* p, int i, float x, float y) {
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(p) + i, (uint64_t)f2u(x) | ((uint64_t)f2u(y) << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float2 load_agent(const float* p, int i) {
+    const uint64_t v = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p) + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return make_float2(u2f((uint32_t)v), u2f((uint32_t)(v >> 32)));
+}
+
 // The attention without a key bias, head dims 64 and 128: attn_int8_kernel's arithmetic with the work of two tiles overlapped.
 // It is bound by vector instruction issue (at 4608 tokens x 24 heads of 128: about 470 per wave and tile beside 32 MFMAs; by the
-// counters the vector pipes are busy 58 % of its cycles and the matrix pipes 25 %) and by the last round of workgroups (864 on
-// 512 places).
+// counters the vector pipes are busy 58 % of its cycles and the matrix pipes 25 %).
 //   * K runs a tile ahead of V through the two LDS stages: as soon as a key block's probabilities are packed, the next tile's
 //     scores go into its registers, one MFMA behind every fourth of the next block's probabilities; the products with V go
 //     an output block at a time with the fold of the block before between them.  (All scores, then all probabilities, then
@@ -1092,16 +1110,33 @@ __device__ __forceinline__ float swap32_sum(float x) {
 //   * numerator and denominator are relative to a base that all but never moves (below), which takes the multiplication
 //     of every output by its rescale factor out of every tile.
 //   * DMA addresses are scalar, the exchange with lane ^ 32 is a row swap.
-// 250 -> 230 us at that shape by the kernel trace, 141 -> 129 us at SDXL's 2 x 4096 x 10 x 64.  A workgroup of eight waves
+//   * SPLIT: the keys of the row blocks that do not fill the CUs once more are shared by several workgroups (key_parts, with the
+//     figures): each part has its own base, and the last to finish brings all of them to the largest.
+// 250 -> 230 us at that shape by the kernel trace, 141 -> 129 us at SDXL's 2 x 4096 x 10 x 64, before the last of these.  A workgroup of eight waves
 // (half the DMA per wave, one workgroup per CU) measured the same for 128 and 30 % slower for 64.
-template <int OUT_DT, int CK, int D>
+template <int OUT_DT, int CK, int D, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
     constexpr int NB = CK / 32, NS = D / 32, KV = CK * D, STAGE = 2 * KV + D * 4;
     extern __shared__ __align__(16) uint8_t smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l32 = lane & 31, hh = lane >> 5;
-    const int hi = blockIdx.y, bi = blockIdx.z;
-    const int row0 = blockIdx.x * 128 + wave * 32;
+    int hi = blockIdx.y, bi = blockIdx.z, rblk = blockIdx.x;
+    int parts = 1, part = 0, t0 = 0, t1 = a.kb;   // the workgroup's key tiles
+    if constexpr (SPLIT) {   // the first `whole` row blocks as they are, the others in parts
+        if (rblk >= a.whole) {
+            parts = a.parts;
+            const int i = rblk - a.whole;
+            rblk = a.whole + i / parts;
+            part = i % parts;
+            t0 = part_bound(a.kb, parts, part);
+            t1 = part_bound(a.kb, parts, part + 1);
+        }
+        const int nqb = (a.lq + 127) / 128, head = rblk / nqb;
+        bi = head / a.h;
+        hi = head - bi * a.h;
+        rblk -= head * nqb;
+    }
+    const int row0 = rblk * 128 + wave * 32;
     const int64_t bh = (int64_t)bi * a.h + hi, kvh = (int64_t)bi * a.hk + hi / a.rep;
     const int r = row0 + l32, rc = r < a.lq ? r : a.lq - 1;   // rows past lq are computed on a clamped row and never stored
     const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)smem, lane16 = lane * 16;
@@ -1124,9 +1159,9 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
         }
         if (wave == 0 && lane < D / 4) dma16(lds0 + (t & 1) * STAGE + 2 * KV, lane16, vst + (int64_t)t * D);
     };
-    fetch_k(0);
-    fetch_v(0);
-    if (a.kb > 1) fetch_k(1);
+    fetch_k(t0);
+    fetch_v(t0);
+    if (t0 + 1 < a.kb) fetch_k(t0 + 1);
 
     v4i qf[NS];
     {
@@ -1135,14 +1170,14 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
         for (int s = 0; s < NS; ++s) qf[s] = *reinterpret_cast<const v4i*>(qrow + s * 32);
     }
     const float q_scale = a.qs[(bh * a.qg + r / 32) * 8 + (r & 7)];
-    float k0 = kst[0], k1 = kst[1];
+    float k0 = kst[t0 * 4], k1 = kst[t0 * 4 + 1];
 
     float ro[NS][16];
 #pragma unroll
     for (int x = 0; x < NS; ++x)
 #pragma unroll
         for (int i = 0; i < 16; ++i) ro[x][i] = 0.f;
-    float m = -50000.f, dsum = 1.f, dsum2 = 0.f;
+    float m = -50000.f, dsum = !SPLIT || part == 0 ? 1.f : 0.f, dsum2 = 0.f;
     __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
     __syncthreads();
 
@@ -1155,7 +1190,7 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
 #pragma unroll
     for (int blk = 0; blk < NB; ++blk) {
         v4i kf[NS];
-        load_kf(kf, 0, blk);
+        load_kf(kf, t0, blk);
         S[blk] = v16i{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
         for (int s = 0; s < NS; ++s) S[blk] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[s], qf[s], S[blk], 0, 0, 0);
@@ -1285,10 +1320,70 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
             __syncthreads();
         }
     };
-    for (int t = 0; t + 1 < a.kb; ++t) tile(t, std::false_type{});
-    tile(a.kb - 1, std::true_type{});
+    if constexpr (SPLIT) {
+        // a part that ends before the last keys also multiplies the K tile behind it, which saves a third form of the tile
+        for (int t = t0; t < t1 && t + 1 < a.kb; ++t) tile(t, std::false_type{});
+        if (t1 == a.kb) tile(t1 - 1, std::true_type{});
+    } else {
+        for (int t = 0; t + 1 < a.kb; ++t) tile(t, std::false_type{});
+        tile(a.kb - 1, std::true_type{});
+    }
 
     float dtot = swap32_sum(dsum + dsum2);
+    if (SPLIT && parts > 1) {
+        // whoever finishes last of a row block's parts adds all of them, each rescaled to the largest base
+        constexpr int SLOT = 64 * (NS * 16 + 2);
+        const int64_t rb = bh * ((a.lq + 127) / 128) + rblk - a.whole;
+        float* slots = a.part + (rb * parts * 4 + wave) * SLOT;
+        uint32_t* done = a.done + rb;
+        int* verdict = reinterpret_cast<int*>(smem);
+        __syncthreads();   // the stages are read
+        if (threadIdx.x == 0) *verdict = (int)__hip_atomic_load(done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
+        __syncthreads();
+        bool mine = *verdict != 0;
+        if (!mine) {
+            float* w = slots + part * (4 * SLOT);
+#pragma unroll
+            for (int x = 0; x < NS; ++x)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) store_agent(w, (x * 8 + i) * 64 + lane, ro[x][2 * i], ro[x][2 * i + 1]);
+            store_agent(w, NS * 8 * 64 + lane, m, dtot);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the stores are where every XCD sees them
+            __syncthreads();
+            if (threadIdx.x == 0) *verdict = (int)__hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
+            __syncthreads();
+            mine = *verdict != 0;
+        }
+        if (!mine) return;
+        // in the order of the parts, whoever merges: the same bits in every call
+        const auto head = [&](int v) { return v == part ? make_float2(m, dtot) : load_agent(slots + v * (4 * SLOT), NS * 8 * 64 + lane); };
+        float base = m, d = 0.f, sum[NS][16];
+        for (int v = 0; v < parts; ++v) base = fmax_nn(base, head(v).x);
+#pragma unroll
+        for (int x = 0; x < NS; ++x)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) sum[x][i] = 0.f;
+        for (int v = 0; v < parts; ++v) {
+            const float2 md = head(v);
+            const float f = __builtin_amdgcn_exp2f(md.x - base);
+            d = fmaf(md.y, f, d);
+            const float* w = slots + v * (4 * SLOT);
+#pragma unroll
+            for (int x = 0; x < NS; ++x)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float2 o = v == part ? make_float2(ro[x][2 * i], ro[x][2 * i + 1]) : load_agent(w, (x * 8 + i) * 64 + lane);
+                    sum[x][2 * i] = fmaf(o.x, f, sum[x][2 * i]);
+                    sum[x][2 * i + 1] = fmaf(o.y, f, sum[x][2 * i + 1]);
+                }
+        }
+        m = base;
+        dtot = d;
+#pragma unroll
+        for (int x = 0; x < NS; ++x)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) ro[x][i] = sum[x][i];
+    }
     // `sink` more keys of score zero and value zero: each adds exp2(0 - m) to the denominator, nothing to the output.  The base can
     // be 60 below the largest score, which would take that out of fp32's range where the score's own distance from zero does not.
     if (a.sink != 0.f) {
@@ -1352,9 +1447,34 @@ __global__ __launch_bounds__(CK) void attn_key_bias_kernel(const float* bias, in
 }
 
 struct Plan {
-    int64_t qi, ki, qs, ks, vt, vs, anchors, vmax, vsum, total;
-    int ck, kb, qg, nblk;
+    int64_t qi, ki, qs, ks, vt, vs, anchors, vmax, vsum, done, part, whole, total;
+    int ck, kb, qg, nblk, parts;
 };
+
+// How the pipelined kernel's row blocks (128 rows of a head) go to the CUs.  What is left over a multiple of the CUs keeps some of them
+// busy for a whole row block's time, 55 us at 4608 keys, while the others idle; the keys of those row blocks are shared by P
+// workgroups each.  P is what leaves a CU the least, in row blocks: ceil(tail * P / CUs) parts of 1 / P each (a part alone on a CU
+// takes 1.3 times as long: 125 us for a row block of 8192 keys, 196 for two at once), plus about 3 us per part for writing and
+// merging it, which is 2 to 5 key tiles.  Calls in us, P = 1 and chosen: 4608 tokens x 24 heads 256 -> 231 (96 of 864 row blocks in
+// halves; in fifths 240), 2 x 4096 x 10 x 64 138 -> 115 (128 of 640 in halves), 2500 x 20 x 64 75 -> 64 (thirds; halves 71), 2048 x
+// 10 56 -> 52 (thirds; halves 55), 1024 x 10 45 -> 40.  Splitting every row block of the first costs 263: 57 MB of parts.
+// Fewer than 8 row blocks stay whole: which keys are summed together then depends on nothing but the key tiles.
+int key_parts(int64_t row_blocks, int64_t kb, int ck, int D, int64_t& whole) {
+    constexpr int64_t CUS = 256;   // not the present device's: the workspace's size and the call have to agree
+    whole = row_blocks;
+    const int64_t tail = row_blocks % CUS;
+    if (D == 256 || row_blocks < 8 || tail == 0) return 1;
+    const bool lone = row_blocks < CUS;
+    const double merge = (D == 64 ? 5.0 : ck == 64 ? 4.0 : 2.0) / (double)kb;
+    double least = (lone ? 1.3 : 1.0) - 0.05;
+    int best = 1;
+    for (int p = 2; p <= 8 && kb / p >= 4; ++p) {
+        const double n = (double)((tail * p + CUS - 1) / CUS), cost = (lone && n == 1 ? 1.3 : n) / p + n * merge;
+        if (cost < least) { least = cost - 0.05; best = p; }
+    }
+    if (best > 1) whole = row_blocks - tail;
+    return best;
+}
 
 Plan plan_for(int64_t b, int64_t h, int64_t hk, int64_t lq, int64_t lk, int D) {
     Plan p;
@@ -1373,26 +1493,31 @@ Plan plan_for(int64_t b, int64_t h, int64_t hk, int64_t lq, int64_t lk, int D) {
     p.anchors = add(b * hk * 4);
     p.vmax = add(b * hk * D * 4);
     p.vsum = add(b * hk * (int64_t)p.kb * D * 4);
+    const int64_t row_blocks = b * h * ((lq + 127) / 128);
+    p.parts = key_parts(row_blocks, p.kb, p.ck, D, p.whole);
+    p.done = add((row_blocks - p.whole) * 4);
+    p.part = add((row_blocks - p.whole) * p.parts * 4 * 64 * (D / 2 + 2) * 4);
     p.total = n;
     return p;
 }
 
 template <auto KERN>
-int launch_tiles(const AttnArgs& a, int lds, hipStream_t st) {
+int launch_tiles(const AttnArgs& a, dim3 grid, int lds, hipStream_t st) {
     if (lds > 64 * 1024) {   // has to be allowed once per kernel and device
         static PerDeviceOnce once;
         if (allow_dynamic_lds(reinterpret_cast<const void*>(KERN), lds, once) != 0) return -401;
     }
-    KERN<<<dim3((a.lq + 127) / 128, a.h, a.b), 256, lds, st>>>(a);
+    KERN<<<grid, 256, lds, st>>>(a);
     return hipGetLastError() == hipSuccess ? 0 : -401;
 }
 template <int DT, int CK, bool MASK, bool FD, int D>
 int launch_attn(const AttnArgs& a, hipStream_t st) {
-    return launch_tiles<attn_int8_kernel<DT, CK, MASK, FD, D>>(a, 2 * (2 * CK * D + D * 4), st);
+    return launch_tiles<attn_int8_kernel<DT, CK, MASK, FD, D>>(a, dim3((a.lq + 127) / 128, a.h, a.b), 2 * (2 * CK * D + D * 4), st);
 }
 template <int DT, int CK, int D>
 int launch_pipe(const AttnArgs& a, hipStream_t st) {
-    return launch_tiles<attn_int8_pipe_kernel<DT, CK, D>>(a, 2 * (2 * CK * D + D * 4), st);
+    if (a.parts > 1) return launch_tiles<attn_int8_pipe_kernel<DT, CK, D, true>>(a, dim3((unsigned)(a.whole + ((int64_t)((a.lq + 127) / 128) * a.h * a.b - a.whole) * a.parts)), 2 * (2 * CK * D + D * 4), st);
+    return launch_tiles<attn_int8_pipe_kernel<DT, CK, D, false>>(a, dim3((a.lq + 127) / 128, a.h, a.b), 2 * (2 * CK * D + D * 4), st);
 }
 
 template <int DT, int D>
@@ -1472,6 +1597,7 @@ int int8_attn(const void* q, const void* k, const void* v, void* o, void* ws, in
     a.qs = (float*)(w + p.qs); a.ks = (float*)(w + p.ks); a.vs = (float*)(w + p.vs);
     a.anchors = (int*)(w + p.anchors); a.vmax = (uint32_t*)(w + p.vmax); a.vsum = (int*)(w + p.vsum);
     a.b = b; a.lq = lq; a.lk = lk; a.h = h; a.hk = hk; a.rep = h / hk;
+    a.parts = p.parts; a.whole = (int)p.whole; a.done = (uint32_t*)(w + p.done); a.part = (float*)(w + p.part);
     a.qg = p.qg; a.kb = p.kb; a.ck = p.ck; a.nblk = p.nblk;
     a.q_bs = q_bs; a.q_rs = q_rs; a.q_hs = q_hs; a.k_bs = k_bs; a.k_rs = k_rs; a.k_hs = k_hs;
     a.v_bs = v_bs; a.v_rs = v_rs; a.v_hs = v_hs; a.o_bs = o_bs; a.o_rs = o_rs; a.o_hs = o_hs;

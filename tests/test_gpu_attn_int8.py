@@ -762,3 +762,49 @@ def test_attention_scores_that_grow_along_the_keys(case):
     ulp = 2.0 ** (-8 if dt == oracle.BF16 else -11)
     assert (ref > 1).all()
     assert (np.abs(_to_f32(_bits(o), dt) - ref) <= 4 * 6 / 255.0 + 2 * ulp * ref).all()
+
+
+SPLITS = [
+    # D, b, lq, lk, h, hk, dtype, sink, levels: row blocks (parts)
+    (128, 1, 130, 1500, 10, 2, torch.bfloat16, 0.0, None),      # 20 (3), 128-key tiles, a ragged last tile
+    (128, 2, 1, 1100, 60, 5, torch.float16, 0.0, None),         # 120 (2: five tiles and four)
+    (128, 1, 3, 520, 9, 3, torch.bfloat16, 0.0, None),          # 9 (2), 64-key tiles
+    (128, 1, 40, 1300, 264, 2, torch.bfloat16, 0.0, None),      # 264: 256 whole, 8 (2)
+    (64, 1, 1, 3000, 300, 4, torch.bfloat16, 0.0, None),        # 300: 256 whole, 44 in more than two parts
+    (128, 1, 70, 1300, 8, 1, torch.bfloat16, 30.0, None),       # a sink, added once
+    (128, 1, 33, 2600, 8, 1, torch.bfloat16, 0.0, "up"),        # every part's base differs, the last is the largest
+    (128, 1, 33, 2600, 8, 1, torch.bfloat16, 5.0, "down"),      # ... the first is
+]
+
+
+@pytest.mark.parametrize("case", SPLITS, ids=lambda c: "D%d_b%d_lq%d_lk%d_h%d_hk%d_%s_sink%g_%s" % (c[:6] + (str(c[6])[6:],) + c[7:]))
+def test_attention_with_keys_shared_by_workgroups(case):
+    """Row blocks whose keys several workgroups share: within the attention tolerance of the oracle, the same bits in every call, and
+    the workspace says that there are parts."""
+    ql, ffi = _pkg()
+    D, b, lq, lk, h, hk, dtype, sink, levels = case
+    dt = oracle.BF16 if dtype == torch.bfloat16 else oracle.F16
+    q, k, v = _inputs(b, lq, lk, h, hk, dtype, seed=D + lq + lk, D=D)
+    if levels:   # scores that grow or fall by about 90 along the keys
+        ramp = torch.linspace(-1, 1, lk) * (1 if levels == "up" else -1)
+        k[..., 0] = (ramp * 64).to(dtype)[None, :, None]
+        q[..., 0] = 8.0
+    scale = D ** -0.5
+    out = (C.c_int64 * 10)()
+    assert ffi.raw("gpu_internal_attn_layout_d", b, h, hk, lq, lk, D, C.cast(out, C.c_void_p)) == 0
+    after = ffi.lib.gpu_int8_attn_workspace_d(b, h, hk, lq, lk, D) - (out[7] + b * hk * out[9] * D * 4)   # behind the column sums
+    assert after > 8 * 2 * 4 * 64 * (D // 2 + 2) * 4, "no row block is split"
+    qd, kd, vd = q.cuda(), k.cuda(), v.cuda()
+    ws = torch.full((ffi.lib.gpu_int8_attn_workspace_d(b, h, hk, lq, lk, D) + 256,), 119, dtype=torch.uint8, device="cuda")   # counters start as rubbish
+    run = (lambda: ql.int8_attn(qd, kd, vd, scale, ws=ws)) if sink == 0.0 else (lambda: ql.int8_attn_sink(qd, kd, vd, scale, sink, ws=ws))
+    outs = [run().clone() for _ in range(3)]
+    torch.cuda.synchronize()
+    assert bool((ws[-256:] == 119).all())
+    ref = _to_f32(oracle.attn_int8(dt, _bits(q), _bits(k), _bits(v), scale, use_anchor=sink == 0.0, sink=sink), dt)
+    got = _to_f32(_bits(outs[0]), dt)
+    vmax, ulp = float(v.float().abs().max()), 2.0 ** (-8 if dt == oracle.BF16 else -11)
+    # one step of 255 of a probability on the other side of a tie, for two keys of the row's largest probability (as above), and the
+    # output's own rounding
+    assert (np.abs(got - ref) <= 2 * vmax / 255.0 + 2 * ulp * np.abs(ref)).all()
+    assert (np.abs(got - ref) <= ulp * np.abs(ref) + 1e-30).mean() > 0.97
+    assert all(torch.equal(o, outs[0]) for o in outs[1:])
