@@ -11,7 +11,9 @@ _DT_TORCH = {v: k for k, v in _TORCH_DT.items()}
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    """Handle of the current stream of the current device: torch.cuda.current_stream().cuda_stream without the Stream object made
+    for it (2.8 us of a 12.3 us call; this way 0.2, and the call 8.1 with no scratch for few rows)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t):
@@ -283,9 +285,13 @@ def linear_w8a8(x, W, ws, bias=None, rotate=0, out_dtype=None):
         raise ValueError("x [M,K] and W [N,K] must share K, got %s and %s" % (tuple(x.shape), tuple(W.shape)))
     N = W.shape[0]
     D = torch.empty((M, N), dtype=out_dtype, device=x.device)
+    args = (_TORCH_DT[x.dtype], _ptr(x), x.stride(0), _ptr(W), _ptr(ws), _ptr(bias), _ptr(D))
+    tail = (M, N, K, rotate, _TORCH_DT[out_dtype], _stream())
+    # a few short rows run as one kernel, which takes no scratch: without one the call either does that or queues nothing
+    if M <= 8 and K <= 1024 and ffi.raw("gpu_linear_w8a8", *args, 0, *tail) == 0:
+        return D
     scratch = torch.empty((M * K + 4 * M,), dtype=torch.uint8, device=x.device)   # codes and row scales
-    ffi.k("gpu_linear_w8a8", _TORCH_DT[x.dtype], _ptr(x), x.stride(0), _ptr(W), _ptr(ws), _ptr(bias), _ptr(D), _ptr(scratch), M, N, K,
-          rotate, _TORCH_DT[out_dtype], _stream())
+    ffi.k("gpu_linear_w8a8", *args, _ptr(scratch), *tail)
     return D
 
 

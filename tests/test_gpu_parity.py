@@ -1113,6 +1113,18 @@ def test_linear_in_one_call(M, N, K, rotate, dtype, out_dt, with_bias):
     assert np.array_equal(host_bits(got).view(np.uint8), np.ascontiguousarray(ref).view(np.uint8))
 
 
+def test_few_rows_with_weights_off_16_bytes_take_the_two_kernels():
+    """The Python call first asks for the one kernel, without a scratch; weights that start elsewhere than at 16 bytes refuse that and run
+    as two.  The same bits, and what neither runs is still refused."""
+    M, N, K = 3, 40, 256
+    x = dev(synth.normal(13, 1, M * K).reshape(M, K).astype(np.float32)).bfloat16()
+    W, ws = dev(rand_i8(13, 2, N, K, -128, 127)), dev(synth.uniform(13, 3, N, 1e-3, 1e-2))
+    off = torch.zeros(N * K + 16, dtype=torch.int8, device=DEV)[8:8 + N * K].view(N, K).copy_(W)
+    assert torch.equal(ql.linear_w8a8(x, off, ws, None, 256).view(torch.int16), ql.linear_w8a8(x, W, ws, None, 256).view(torch.int16))
+    with pytest.raises(ffi.KernelError):
+        ql.linear_w8a8(x[:, :100].contiguous(), W[:, :100].contiguous(), ws, None, 0)
+
+
 def test_linear_in_one_call_refuses_what_the_two_calls_refuse():
     for dtype, M, N, K, rotate, out_dt, want in [(BF16, 4, 8, 100, 0, BF16, -1), (BF16, 4, 8, 128, 256, BF16, -1), (F16, 4, 8, 128, 0, BF16, -4),
                                                  (BF16, 0, 8, 128, 0, BF16, 0), (BF16, 4, 8, 0, 0, BF16, -1), (BF16, -1, 8, 128, 0, BF16, -200)]:
