@@ -40,7 +40,7 @@ struct GemmArgs {
     int M, N, K;
     int tiles_m, tiles_n;
     uint32_t magic;   // panel_magic(tiles_m, tiles_n), for tile_of_block
-    int kslice;   // ring kernel only: K elements per split-K slice (a multiple of 128), 0 = no split
+    int kslice;   // K of a split-K slice (a multiple of 128), 0 = no split
 };
 
 template <int BM_, int BN_, int BK_, int WGM_, int WGN_, int OCC_>
@@ -139,22 +139,64 @@ __device__ __forceinline__ void epilogue_store(const GemmArgs& p, v16i (&acc)[TN
     }
 }
 
+// The constants of a wave tile's epilogue in a lane's registers: column scales and raw bias words of its runs of four columns, row
+// scales.  (runs: per 32 columns; halves: per 32 rows; see L at epilogue_shuffle)
+template <int TM, int TN, int OUT_DT, int EPI, int L>
+struct EpiConst {
+    static constexpr int SZ = (EPI == EPI_ACC || OUT_DT == DT_F32) ? 4 : 2, BW = SZ == 4 ? 4 : 2;   // 32-bit words holding 4 bias values
+    static constexpr int NRB = L == 32 ? 4 : 2, NHM = L == 32 ? 1 : 2;
+    float wsr[TN][NRB][4];
+    uint32_t braw[TN][NRB][BW];
+    float xsr[TM][NHM];
+    // In one batch, no branches between the loads, so a single wait covers them.  Columns past N read the last valid vector.
+    __device__ __forceinline__ void load_columns(const GemmArgs& p, int nb, int lane) {
+        const int fhalf = lane / L;
+#pragma unroll
+        for (int in = 0; in < TN; ++in)
+#pragma unroll
+            for (int rb = 0; rb < NRB; ++rb) {
+                int n = nb + in * 32 + (L == 32 ? rb * 8 : rb * 16) + fhalf * 4;
+                n = n < p.N ? n : p.N - 4;
+                const float4 w4 = *reinterpret_cast<const float4*>(p.ws + n);
+                wsr[in][rb][0] = w4.x; wsr[in][rb][1] = w4.y; wsr[in][rb][2] = w4.z; wsr[in][rb][3] = w4.w;
+                if (p.bias) {
+                    if (SZ == 4) {
+                        const uint4 b4 = *reinterpret_cast<const uint4*>((const uint8_t*)p.bias + (int64_t)n * 4);
+                        braw[in][rb][0] = b4.x; braw[in][rb][1] = b4.y; braw[in][rb][BW - 2] = b4.z; braw[in][rb][BW - 1] = b4.w;
+                    } else {
+                        const uint2 b2 = *reinterpret_cast<const uint2*>((const uint8_t*)p.bias + (int64_t)n * 2);
+                        braw[in][rb][0] = b2.x; braw[in][rb][1] = b2.y;
+                    }
+                } else {
+#pragma unroll
+                    for (int j = 0; j < BW; ++j) braw[in][rb][j] = 0u;
+                }
+            }
+    }
+    __device__ __forceinline__ void load_rows(const GemmArgs& p, int mb, int lane) {
+#pragma unroll
+        for (int im = 0; im < TM; ++im)
+#pragma unroll
+            for (int hm = 0; hm < NHM; ++hm) {
+                const int mrow = mb + im * 32 + hm * 16 + (lane & (L - 1));
+                xsr[im][hm] = (EPI == EPI_ACC || mrow >= p.M) ? 0.f : p.xs[mrow];
+            }
+    }
+};
+
 // Coalesced epilogue: the accumulator layout (lane = one m, four consecutive n per register group) would store 16-byte
 // pieces scattered over 32 rows per instruction.  Instead each wave rounds its values to the output type, passes a
 // 32-row piece of its tile through a private LDS region (XOR-swizzled 16-byte chunks, conflict-free both ways) and
 // writes whole rows: 16 bytes per lane, consecutive lanes on consecutive addresses.  For the residual form the LDS
 // holds z = Out(acc*xs*ws + bias), exactly the intermediate the reference rounds, and fma(z, rscale, resid) is applied
 // on the way out.  Needs row starts of D (and resid) 16-byte aligned; the caller falls back to epilogue_store otherwise.
-// STAGED: the per-column constants (ws and bias as floats, 2 x 32*TN values) are kept in the wave's LDS area `cst` and
-// read back per piece, instead of 96 registers that a persistent kernel cannot spare next to its pipeline state.  1: this
-// function loads them into `cst` first; 2: the caller has put them there (stage_columns, long before, so that their
-// trip from memory is off the epilogue's path), and `xs_lds`, when given, holds the tile's row scales the same way.
 // L: the MFMA shape the accumulators come from.  32: v16i acc[TN][TM], a lane holds row lane % 32 of a 32x32 tile and
 // the columns 8*rb + 4*(lane / 32) + j.  16: v4i acc[2*TN][2*TM] of 16x16 tiles, a lane holds row lane % 16 and the
 // columns 4*(lane / 16) + j; the 32x32 block (in, im) is then the four tiles (2*in + rb, 2*im + hm).
-template <int TM, int TN, int OUT_DT, int EPI, int PW = TN * 32, bool UNTRACKED = false, int STAGED = 0, int L = 32, class Acc>
-__device__ __forceinline__ void epilogue_shuffle(const GemmArgs& p, Acc& acc, int mb, int nb, int lane, uint8_t* wl,
-                                                 uint8_t* wl2 = nullptr, float* cst = nullptr, const float* xs_lds = nullptr) {
+// EARLY: the constants are in `own` already; else they are loaded here.
+template <int TM, int TN, int OUT_DT, int EPI, int PW, bool UNTRACKED, int L, bool EARLY, class Acc>
+__device__ __forceinline__ void epilogue_shuffle_with(const GemmArgs& p, Acc& acc, int mb, int nb, int lane, uint8_t* wl, uint8_t* wl2,
+                                                      EpiConst<TM, TN, OUT_DT, EPI, L>& own) {
     // a piece is 32 rows x PW columns of the wave tile: PW*SZ bytes per LDS row, 32*PW*SZ bytes per wave
     constexpr int SZ = (EPI == EPI_ACC || OUT_DT == DT_F32) ? 4 : 2;
     constexpr int WTN = TN * 32, NP = WTN / PW, TNP = PW / 32;
@@ -176,53 +218,9 @@ __device__ __forceinline__ void epilogue_shuffle(const GemmArgs& p, Acc& acc, in
         else return acc[2 * in + rb][2 * im + hm][j];
     };
 
-    // per-lane column constants, loaded once and in one batch (no branches between the loads, so a single wait covers
-    // them): ws and the raw bias words for the 4 n of every (in, rb).  Columns past N read the last valid vector.
-    constexpr int BW = SZ == 4 ? 4 : 2;            // 32-bit words holding 4 bias values
-    float wsr[STAGED ? 1 : TN][NRB][4];
-    uint32_t braw[STAGED ? 1 : TN][NRB][BW];
-    if (EPI != EPI_ACC && STAGED == 1) {
-        // two columns per lane and pass
-#pragma unroll
-        for (int c0 = 0; c0 < WTN; c0 += 128) {
-            const int c = c0 + lane * 2;
-            if (c < WTN) {
-                int n = nb + c;
-                n = n < p.N ? n : p.N - 2;
-                const float2 w2 = *reinterpret_cast<const float2*>(p.ws + n);
-                float2 b2 = make_float2(0.f, 0.f);
-                if (p.bias) {
-                    b2.x = ld_dt<(SZ == 4 ? DT_F32 : OUT_DT)>(p.bias, n);
-                    b2.y = ld_dt<(SZ == 4 ? DT_F32 : OUT_DT)>(p.bias, n + 1);
-                }
-                *reinterpret_cast<float2*>(cst + c) = w2;
-                *reinterpret_cast<float2*>(cst + WTN + c) = b2;
-            }
-        }
-    }
-    if (EPI != EPI_ACC && !STAGED) {
-#pragma unroll
-        for (int in = 0; in < TN; ++in)
-#pragma unroll
-            for (int rb = 0; rb < NRB; ++rb) {
-                int n = nb + in * 32 + run_col(rb);
-                n = n < p.N ? n : p.N - 4;
-                const float4 w4 = *reinterpret_cast<const float4*>(p.ws + n);
-                wsr[in][rb][0] = w4.x; wsr[in][rb][1] = w4.y; wsr[in][rb][2] = w4.z; wsr[in][rb][3] = w4.w;
-                if (p.bias) {
-                    if (SZ == 4) {
-                        const uint4 b4 = *reinterpret_cast<const uint4*>((const uint8_t*)p.bias + (int64_t)n * 4);
-                        braw[in][rb][0] = b4.x; braw[in][rb][1] = b4.y; braw[in][rb][BW - 2] = b4.z; braw[in][rb][BW - 1] = b4.w;
-                    } else {
-                        const uint2 b2 = *reinterpret_cast<const uint2*>((const uint8_t*)p.bias + (int64_t)n * 2);
-                        braw[in][rb][0] = b2.x; braw[in][rb][1] = b2.y;
-                    }
-                } else {
-#pragma unroll
-                    for (int j = 0; j < BW; ++j) braw[in][rb][j] = 0u;
-                }
-            }
-    }
+    if (EPI != EPI_ACC && !EARLY) own.load_columns(p, nb, lane);
+    const auto& wsr = own.wsr;
+    const auto& braw = own.braw;
     // bias value j of (in, rb) as float: +0.0 for a null bias
     auto bias_f = [&](int in, int rb, int j) -> float {
         if (SZ == 4) return u2f(braw[in][rb][j]);
@@ -239,15 +237,8 @@ __device__ __forceinline__ void epilogue_shuffle(const GemmArgs& p, Acc& acc, in
 
     // Every global load is issued ahead of the stores that precede its use: the memory counter retires in order, so a
     // load issued after a store cannot be waited for without also waiting for that store to reach memory.
-    float xsr[TM][NHM];
-#pragma unroll
-    for (int im = 0; im < TM; ++im)
-#pragma unroll
-        for (int hm = 0; hm < NHM; ++hm) {
-            const int mrow = mb + im * 32 + hm * 16 + frow;
-            if (xs_lds) xsr[im][hm] = EPI == EPI_ACC ? 0.f : xs_lds[im * 32 + hm * 16 + frow];
-            else xsr[im][hm] = (EPI == EPI_ACC || mrow >= p.M) ? 0.f : p.xs[mrow];
-        }
+    auto& xsr = own.xsr;
+    if (!EARLY) own.load_rows(p, mb, lane);
     float rs[NP][EPC];
     if (EPI == EPI_RESID) {
 #pragma unroll
@@ -288,17 +279,8 @@ __device__ __forceinline__ void epilogue_shuffle(const GemmArgs& p, Acc& acc, in
                         *reinterpret_cast<v4i*>(dst) = v4i{val(in, im, rb, hm, 0), val(in, im, rb, hm, 1), val(in, im, rb, hm, 2), val(in, im, rb, hm, 3)};
                     } else {
                         float o[4];
-                        if (STAGED) {
-                            const float4 w4 = *reinterpret_cast<const float4*>(cst + in * 32 + run_col(rb));
-                            const float4 b4 = *reinterpret_cast<const float4*>(cst + WTN + in * 32 + run_col(rb));
-                            o[0] = __builtin_fmaf((float)val(in, im, rb, hm, 0) * xs, w4.x, b4.x);
-                            o[1] = __builtin_fmaf((float)val(in, im, rb, hm, 1) * xs, w4.y, b4.y);
-                            o[2] = __builtin_fmaf((float)val(in, im, rb, hm, 2) * xs, w4.z, b4.z);
-                            o[3] = __builtin_fmaf((float)val(in, im, rb, hm, 3) * xs, w4.w, b4.w);
-                        } else {
 #pragma unroll
-                            for (int j = 0; j < 4; ++j) o[j] = __builtin_fmaf((float)val(in, im, rb, hm, j) * xs, wsr[in][rb][j], bias_f(in, rb, j));
-                        }
+                        for (int j = 0; j < 4; ++j) o[j] = __builtin_fmaf((float)val(in, im, rb, hm, j) * xs, wsr[in][rb][j], bias_f(in, rb, j));
                         if (OUT_DT == DT_F32) {
                             *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
                         } else if (OUT_DT == DT_BF16) {
@@ -402,6 +384,11 @@ __device__ __forceinline__ void epilogue_shuffle(const GemmArgs& p, Acc& acc, in
         }
     }
     asm volatile("" ::: "memory");
+}
+template <int TM, int TN, int OUT_DT, int EPI, int PW = TN * 32, bool UNTRACKED = false, int L = 32, class Acc>
+__device__ __forceinline__ void epilogue_shuffle(const GemmArgs& p, Acc& acc, int mb, int nb, int lane, uint8_t* wl) {
+    EpiConst<TM, TN, OUT_DT, EPI, L> own;
+    epilogue_shuffle_with<TM, TN, OUT_DT, EPI, PW, UNTRACKED, L, false>(p, acc, mb, nb, lane, wl, nullptr, own);
 }
 
 // Chooses the coalesced epilogue when row starts are 16-byte aligned.  Must be called by all waves of the workgroup:
@@ -550,7 +537,7 @@ __global__ void __launch_bounds__(C::NT, C::OCC) int8_gemm_kernel(GemmArgs p) {
     epilogue<C::TM, C::TN, OUT_DT, EPI>(p, acc, m0 + wm * C::WTM, n0 + wn * C::WTN, lane, wave, smem);
 }
 
-// 16-byte global store the compiler's wait-count bookkeeping does not see (see the ring kernel's epilogue)
+// 16-byte global store the compiler's wait-count bookkeeping does not see
 __device__ __forceinline__ void store16_untracked(void* ptr, uint4 v) {
     const v4i d = v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
     // The trailing s_nop gives the two wait states this hardware needs between a store of more than 8 bytes and a
@@ -567,274 +554,146 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_
 __device__ __forceinline__ void wg_barrier() { asm volatile("s_barrier" ::: "memory"); }
 __device__ __forceinline__ void wait_lgkmcnt0() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
-// ---------------------------------------------------------------------------------------------------------------
-// The persistent ring kernel: one workgroup per CU walks its share of the 256x256 output tiles and keeps ONE
-// global -> LDS pipeline running across all of them.  Tiles have 128-byte K rows (whole cache lines per DMA lane
-// group).  LDS holds two stages of A (2 x 32 KB) and three of W (3 x 32 KB) = 160 KB: in iteration g the DMA fetches
-// A of iteration g+1 (it must land before barrier Y of this iteration) and W of iteration g+2 (a full iteration of
-// slack), so the last-issued loads of an iteration are never the ones the next wait needs.  Iterations number
-// straight through tile boundaries: while the last K tiles of one output tile are multiplied, the first K tiles of
-// the next one are already in flight, and the stores of an epilogue drain under the next tile's K loop.
-//
-// Per iteration (64 MFMAs per wave = four 32-deep sub-steps): barrier X (every wave is done with iteration g-1, whose
-// stages are now free); sub-steps 0-2 with A DMA after MFMAs 0,3,..,21 and W DMA after MFMAs 24,28,..,52; vmcnt wait
-// that leaves only this iteration's W DMA in flight; barrier Y; sub-step 3, which prefetches the first fragments of
-// iteration g+1.  Requires K % 128 == 0 and M*K, N*K < 2^32.
-// ---------------------------------------------------------------------------------------------------------------
 template <int V> struct ic { static constexpr int value = V; };
-template <int N, int I = 0, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (I < N) {
-        f(ic<I>{});
-        static_for<N, I + 1>(f);
-    }
-}
-
-// BN: tile width; WGM x WGN: wave grid of four waves, one per SIMD (up to 512 registers each); NSA: LDS stages of A (2
-// when a 256-wide tile leaves no room for a third in 160 KB of LDS; 3 where a narrower tile does).  W always has three
-// stages.
-template <int BN_, int WGM_, int WGN_, int NSA_, int BM_ = 256>
-struct RingCfg {
-    static constexpr int BM = BM_, BN = BN_, BK = 128, WGM = WGM_, WGN = WGN_, NW = WGM * WGN, NT = 64 * NW, NSA = NSA_, NSW = 3;
-    static constexpr int WTM = BM / WGM, WTN = BN / WGN, TM = WTM / 32, TN = WTN / 32;
-    static constexpr int A_LD = BM / (8 * NW), W_LD = BN / (8 * NW);   // DMA instructions per wave per stage (8 rows each)
-    static constexpr int NDMA = A_LD + W_LD, NM = TM * TN, NF = TM + TN;
-    static constexpr int A_STAGE = BM * BK, W_STAGE = BN * BK;
-    static constexpr int W_BASE = NSA * A_STAGE;
-    static constexpr int SMEM = NSA * A_STAGE + NSW * W_STAGE;
-    static_assert(NW == 4 && BM % (32 * WGM) == 0 && BN % (32 * WGN) == 0 && BN % 32 == 0, "tile shape");
-    static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "whole DMA blocks per wave");
-    static_assert(NF <= NM && SMEM <= 160 * 1024, "fragment loads hide behind MFMAs; LDS fits");
-    // Slot of the d-th DMA instruction of an iteration (A first, then W), as the number of the MFMA it follows; an
-    // iteration has 4*NM MFMAs and barrier Y sits after MFMA 3*NM - 1.  With two A stages the A DMA is needed by this
-    // iteration's barrier Y, so it goes first and dense (inside the first one and a half sub-steps); with three,
-    // everything has an iteration of slack and is spread evenly.
-    static constexpr int slot(int d) {
-        return NSA == 2 ? (d < A_LD ? d * ((3 * NM) / (2 * A_LD)) : (3 * NM) / 2 + (d - A_LD) * ((4 * NM - (3 * NM) / 2 - 1) / W_LD))
-                        : (d * 4 * NM) / NDMA;
-    }
-    // DMA instructions of this iteration that may still be in flight at barrier Y
-    static constexpr int in_flight_at_y() {
-        int n = 0;
-        for (int d = (NSA == 2 ? A_LD : 0); d < NDMA; ++d) n += slot(d) < 3 * NM ? 1 : 0;
-        return n;
-    }
-    static constexpr bool slots_ok() {
-        for (int d = 0; d < NDMA; ++d) {
-            if (slot(d) >= 4 * NM) return false;
-            if (d > 0 && slot(d) <= slot(d - 1)) return false;
-            if (NSA == 2 && d < A_LD && slot(d) >= 2 * NM) return false;
-        }
-        return true;
-    }
-    static_assert(slots_ok(), "DMA slots must be distinct, inside the iteration, and early for a two-stage A");
-    // columns of one epilogue shuffle piece for an output element of SZ bytes: 128-byte LDS rows (four 16-byte vectors
-    // per lane in flight between the read and the store half of a piece) where the wave tile's width allows
-    static constexpr int piece_cols(int sz) { return WTN % (128 / sz) == 0 ? 128 / sz : 32; }
-    // Epilogue scratch of one wave inside a stage that was just multiplied: a shuffle piece in each of an A and a W
-    // stage; the wave's column constants (2 x WTN floats) sit behind the piece in the W stage.
-    static constexpr bool STAGED = true;
-    static constexpr int A_REGION = A_STAGE / NW, W_REGION = W_STAGE / NW;
-    static constexpr int piece_bytes(int sz) { return 32 * piece_cols(sz) * sz; }
-    static constexpr bool scratch_ok(int sz) {
-        return piece_bytes(sz) <= A_REGION && piece_bytes(sz) + (STAGED ? 2 * WTN * 4 : 0) <= W_REGION;
-    }
-    static_assert(scratch_ok(2) && scratch_ok(4), "epilogue scratch fits the stages");
+// ---------------------------------------------------------------------------------------------------------------
+// Shapes with too few 256x256 tiles for the CUs: 128 x (64 * TN) tiles, one per workgroup and CU.
+//
+// Four waves multiply (64 x (32 * TN) each, one per SIMD) and four fetch.  A DMA instruction holds the wave that issues it for about 68
+// cycles, four times a 16x16x64 MFMA, and with one wave per SIMD nothing else would run meanwhile; here the multiplying waves
+// issue none.  Their fragments are double-buffered by halves of a K step: the next half is read from LDS behind the first MFMAs of
+// this one.  One barrier per step, between its halves: step s + 1 has landed, and stage s, whose second half is in registers, may be
+// fetched into.  Four stages: a step has three to land.  The epilogue's constants are loaded ahead of the K loop and the
+// residual's lines are brought into the L2 by the waves that are done fetching.
+// Stamps at 8192 x 2560 -> 640 (256 tiles, us): 2.0 until the first MFMA, 0.53 per step (the MFMAs take 0.37), 2.1 for the epilogue,
+// 1.2 of them with constants and residual loaded where they are used.
+// Against what ran these shapes before (a ring kernel of four waves that fetched for themselves, 128 x 192 tiles; 256 x 96 tiles
+// streaming the weights for up to 256 rows), us, weights from HBM: 8192 x 2560 -> 640 20.1 and 16.2, 2048 x 2048 -> 2048 14.1 and
+// 10.2, 512 x 4096 -> 4096 21.0 and 12.1, 256 x 4096 -> 4096 18.2 and 10.8, 200 x 8192 -> 3072 23.8 and 14.8, 1024 x 4096 -> 9216
+// 41 on the two-group kernel.  The rule is at fed_plan.
+// ---------------------------------------------------------------------------------------------------------------
+template <int TN_>
+struct FedCfg {
+    static constexpr int TN = TN_, TM = 2, BM = 128, BN = 64 * TN, BK = 128, NT = 512, NS = 4;
+    static constexpr int STAGE = (BM + BN) * BK, W_BASE = BM * BK, SMEM = NS * STAGE;
+    static constexpr int A_LD = BM / 32, W_LD = BN / 32, LD = A_LD + W_LD;   // DMA instructions per fetching wave and step
+    static constexpr int piece_cols(int sz) { return TN * 32 % (128 / sz) == 0 ? 128 / sz : 32; }
+    static_assert(SMEM <= 160 * 1024, "LDS budget");
 };
-
 template <class C, int OUT_DT, int EPI>
-__global__ void __launch_bounds__(C::NT, 1) int8_gemm_ring_kernel(GemmArgs p) {
+__global__ void __launch_bounds__(512, 1) int8_gemm_fed_kernel(GemmArgs p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    constexpr int BK = C::BK, TM = C::TM, TN = C::TN, NM = C::NM, NF = C::NF, NSA = C::NSA;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave / C::WGN, wn = wave % C::WGN;
-    const int ld = p.K;                                  // row stride of A and W
-    // split K: workgroup row blockIdx.y multiplies K slice [k_lo, k_lo + nk*128) and writes its own int32 plane
-    const int k_lo = p.kslice ? (int)blockIdx.y * p.kslice : 0;
-    const int k_len = p.kslice ? (p.K - k_lo < p.kslice ? p.K - k_lo : p.kslice) : p.K;
-    const int nk = k_len / BK;
+    constexpr int NS = C::NS, LD = C::LD, FM = 2 * C::TM, FN = 2 * C::TN, BK = C::BK;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), wq = wave & 3;
+    // split K: workgroup row blockIdx.y multiplies its slice of K and writes its own int32 plane
+    const int k0 = p.kslice ? (int)blockIdx.y * p.kslice : 0;
+    const int nk = (p.kslice && k0 + p.kslice < p.K ? p.kslice : p.K - k0) / BK;
     if (p.kslice) p.D = (uint8_t*)p.D + (int64_t)blockIdx.y * p.M * p.N * 4;
-    const int8_t* Ab = p.A + k_lo;
-    const int8_t* Wb = p.W + k_lo;
-    const int G = gridDim.x, ntiles = p.tiles_m * p.tiles_n;
-    const int nt_b = (ntiles - (int)blockIdx.x + G - 1) / G;   // tiles of this workgroup: blockIdx, blockIdx + G, ...
+    int tm, tn;
+    tile_of_block((int)blockIdx.x, (int)gridDim.x, p.tiles_m, p.tiles_n, tm, tn, p.magic);
+    const int m0 = tm * C::BM, n0 = tn * C::BN;
 
-    auto tile_origin = [&](int i, int& m0, int& n0) {
-        int tm, tn;
-        tile_of_block((int)blockIdx.x + i * G, ntiles, p.tiles_m, p.tiles_n, tm, tn, p.magic);
-        m0 = tm * C::BM;
-        n0 = tn * C::BN;
-    };
-
-    // DMA streams.  Each walks (tile, K tile) pairs in the order the MFMAs will consume them and stops on the last one
-    // (re-fetching it into a stage nothing reads again keeps the loop free of branches around the DMA slots).
-    // rows come in blocks of 8 (block index wave + NW*j has the parity of wave): swz<128> of the row
-    uint32_t ga[C::A_LD], gw[C::W_LD];
-    int a_tile = 0, a_kt = 0, a_stage = 0, w_tile = 0, w_kt = 0, w_stage = 0;
-    // The row and chunk of a lane are recomputed from the hardware lane number each time a stream moves to its next
-    // tile: as loop invariants the compiler would keep sixteen of them live across the K loop, spill them, and reload
-    // them here behind full memory waits that drain the DMA pipeline (a spilled copy of the lane number does the same).
-    auto set_a = [&](int i) {
-        int m0, n0;
-        tile_origin(i, m0, n0);
-        const int l = hw_lane();
-        const int lr = l >> 3, lc = ((l & 7) ^ (((wave & 1) << 2) | (lr >> 1))) * 16;
+    if (wave >= 4) {
+        const int l = hw_lane(), lr = l >> 3, lc = ((l & 7) ^ (((wq & 1) << 2) | (lr >> 1))) * 16;
+        uint32_t ga[C::A_LD], gw[C::W_LD];
 #pragma unroll
         for (int j = 0; j < C::A_LD; ++j) {
-            const int row = (wave + C::NW * j) * 8 + lr;
-            const int gr = m0 + row < p.M ? m0 + row : p.M - 1;
-            ga[j] = (uint32_t)gr * (uint32_t)ld + lc;
+            const int row = m0 + (wq + 4 * j) * 8 + lr;
+            ga[j] = (uint32_t)(row < p.M ? row : p.M - 1) * (uint32_t)p.K + lc;
         }
-    };
-    auto set_w = [&](int i) {
-        int m0, n0;
-        tile_origin(i, m0, n0);
-        const int l = hw_lane();
-        const int lr = l >> 3, lc = ((l & 7) ^ (((wave & 1) << 2) | (lr >> 1))) * 16;
 #pragma unroll
         for (int j = 0; j < C::W_LD; ++j) {
-            const int row = (wave + C::NW * j) * 8 + lr;
-            const int gr = n0 + row < p.N ? n0 + row : p.N - 1;
-            gw[j] = (uint32_t)gr * (uint32_t)ld + lc;
+            const int row = n0 + (wq + 4 * j) * 8 + lr;
+            gw[j] = (uint32_t)(row < p.N ? row : p.N - 1) * (uint32_t)p.K + lc;
         }
-    };
-    // The DMA is written as inline assembly: through the builtin the compiler, unable to prove that a fragment read and
-    // an in-flight DMA touch different stages, puts a full vmcnt(0) wait in front of the fragment reads, which serializes
-    // the whole pipeline.  Ordering is kept by hand instead (wait_vmcnt + barriers).  scalar base + 32-bit lane offset.
-    const uint32_t lds_base = (uint32_t)(uintptr_t)smem;   // LDS byte address of the dynamic segment
-    auto dma_a = [&](int j) {
-        const int8_t* base = Ab + (int64_t)a_kt * BK;
-        const uint32_t dst = lds_base + a_stage * C::A_STAGE + (wave + C::NW * j) * 1024;
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(ga[j]), "s"(base) : "memory", "m0");
-    };
-    auto dma_w = [&](int j) {
-        const int8_t* base = Wb + (int64_t)w_kt * BK;
-        const uint32_t dst = lds_base + C::W_BASE + w_stage * C::W_STAGE + (wave + C::NW * j) * 1024;
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(gw[j]), "s"(base) : "memory", "m0");
-    };
-    auto advance_a = [&]() {
-        a_stage = a_stage == NSA - 1 ? 0 : a_stage + 1;
-        if (a_tile == nt_b - 1 && a_kt == nk - 1) return;
-        if (++a_kt == nk) { a_kt = 0; set_a(++a_tile); }
-    };
-    auto advance_w = [&]() {
-        w_stage = w_stage == C::NSW - 1 ? 0 : w_stage + 1;
-        if (w_tile == nt_b - 1 && w_kt == nk - 1) return;
-        if (++w_kt == nk) { w_kt = 0; set_w(++w_tile); }
-    };
-
-    // fragment addresses inside a stage: row r at r*128, chunk c at slot c ^ ((r>>1)&7); K sub-step kk flips bits 5 and 6
-    const int frow = lane & 31, fhalf = lane >> 5;
-    const int fsw = (fhalf ^ ((frow >> 1) & 7)) << 4;
-    int aoff[4], woff[4];
+        const uint32_t lds_base = (uint32_t)(uintptr_t)smem + wq * 1024;
+        // Weights streamed once: workgroups that all read the same columns of K of rows 4 KB apart meet in a few of the HBM's channels,
+        // so each tile column starts at a step of its own and wraps (integer sums: any order).  Cold weights, all at step 0 and
+        // staggered, us: 256 x 4096 -> 24576 34.7 and 32.0, 40 rows 26.0 and 22.6, 128 x 8192 -> 28672 55.6 and 48.5, 40 x 3072 -> 18432
+        // 17.2 and 16.6.  Slices start apart already, and with more rows tiles that share A or W do best in step (2048 x
+        // 2048 -> 2048 11.1 and 11.6).
+        const int first = p.tiles_m <= 2 && !p.kslice ? tn % nk : 0;
+        const auto fetch = [&](int step) {
+            const uint32_t dst = lds_base + (step & (NS - 1)) * C::STAGE;
+            const int at = k0 + (step + first < nk ? step + first : step + first - nk) * BK;
+            const int8_t *ab = p.A + at, *wb = p.W + at;
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-        aoff[kk] = ((wm * C::WTM + frow) * BK + fsw) ^ (kk << 5);
-        woff[kk] = ((wn * C::WTN + frow) * BK + fsw) ^ (kk << 5);
-    }
-    auto frag = [&](const uint8_t* sa, const uint8_t* sw, int kk, int j) -> v4i {
-        if (j < TM) return *reinterpret_cast<const v4i*>(sa + aoff[kk] + j * 32 * BK);
-        return *reinterpret_cast<const v4i*>(sw + woff[kk] + (j - TM) * 32 * BK);
-    };
-
-    v16i acc[TN][TM];
-    v4i f0[NF], f1[NF];
-
-    // One sub-step: NM MFMAs on `cur`; the NF fragment loads of the next sub-step ride behind the first MFMAs; DMA
-    // instructions sit in their slots (this sub-step's MFMAs are numbers BASE .. BASE + NM - 1 of the iteration).
-    auto substep = [&](auto BASE, v4i* cur, v4i* nxt, const uint8_t* sa_n, const uint8_t* sw_n, int kk_n) {
+            for (int j = 0; j < C::A_LD; ++j)
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst + j * 4096), "v"(ga[j]), "s"(ab) : "memory", "m0");
 #pragma unroll
-        for (int i = 0; i < NM; ++i) {
-            const int in = i / TM, im = i % TM;
-            acc[in][im] = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur[TM + in], cur[im], acc[in][im], 0, 0, 0);
-            SCHED_FENCE();
-#pragma unroll
-            for (int d = 0; d < C::NDMA; ++d) {
-                if (C::slot(d) == decltype(BASE)::value + i) {
-                    if (d < C::A_LD) dma_a(d);
-                    else dma_w(d - C::A_LD);
-                    SCHED_FENCE();
+            for (int j = 0; j < C::W_LD; ++j)
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst + C::W_BASE + j * 4096), "v"(gw[j]), "s"(wb) : "memory", "m0");
+        };
+        fetch(0);
+        if (nk > 1) { fetch(1); wait_vmcnt<LD>(); }
+        else wait_vmcnt<0>();
+        wg_barrier();                                        // step 0 has landed
+        for (int s = 2; s < NS && s < nk; ++s) fetch(s);
+        for (int s = 0; s < nk; ++s) {
+            if (s + NS <= nk) wait_vmcnt<(NS - 2) * LD>();   // step s + 1 has landed
+            else wait_vmcnt<0>();
+            wg_barrier();                                    // ... and nobody reads stage s any more
+            if (s + NS < nk) fetch(s + NS);
+            else if (EPI == EPI_RESID && (s + NS == nk || (nk < NS && s == 0))) {
+                // the residual's lines into this XCD's L2, which the epilogue would otherwise wait for: SZ * BN bytes of 128 rows
+                constexpr int CPR = C::BN * EpiConst<1, 1, OUT_DT, EPI, 16>::SZ / 128;
+                for (int i = wq * 64 + hw_lane(); i < 128 * CPR; i += 256) {
+                    const int row = m0 + i / CPR, col = n0 + i % CPR * (128 / EpiConst<1, 1, OUT_DT, EPI, 16>::SZ);
+                    if (row < p.M && col < p.N) {
+                        const uint32_t v = *reinterpret_cast<const volatile uint32_t*>((const uint8_t*)p.resid + ((int64_t)row * p.N + col) * EpiConst<1, 1, OUT_DT, EPI, 16>::SZ);
+                        asm volatile("" ::"v"(v));
+                    }
                 }
             }
-            if (i < NF) { nxt[i] = frag(sa_n, sw_n, kk_n, i); SCHED_FENCE(); }
         }
-    };
-
-    // prologue: A(0), W(0), [A(1),] W(1) in flight; A(0) and W(0) must land
-    set_a(0);
-    set_w(0);
-#pragma unroll
-    for (int j = 0; j < C::A_LD; ++j) dma_a(j);
-    advance_a();
-#pragma unroll
-    for (int j = 0; j < C::W_LD; ++j) dma_w(j);
-    advance_w();
-    if (NSA == 3) {
-#pragma unroll
-        for (int j = 0; j < C::A_LD; ++j) dma_a(j);
-        advance_a();
+        return;
     }
+
+    const int wm = wq >> 1, wn = wq & 1;
+    EpiConst<C::TM, C::TN, OUT_DT, EPI, 16> cst;
+    if (EPI != EPI_ACC) {
+        cst.load_columns(p, n0 + wn * C::TN * 32, hw_lane());
+        cst.load_rows(p, m0 + wm * 64, hw_lane());
+    }
+    v4i acc[FN][FM], f[2][FM + FN];
 #pragma unroll
-    for (int j = 0; j < C::W_LD; ++j) dma_w(j);
-    advance_w();
-    wait_vmcnt<(NSA == 3 ? C::A_LD : 0) + C::W_LD>();
+    for (int in = 0; in < FN; ++in)
+#pragma unroll
+        for (int im = 0; im < FM; ++im) acc[in][im] = v4i{0, 0, 0, 0};
+    const int frow = hw_lane() & 15, fq = hw_lane() >> 4;
+    const int x = frow * BK + ((fq ^ ((frow >> 1) & 7)) << 4);
+    const int ao = wm * 64 * BK + x, wo = C::W_BASE + wn * C::TN * 32 * BK + x;
+    const auto read = [&](int step, int kk, int j) {
+        const uint8_t* st = smem + (step & (NS - 1)) * C::STAGE;
+        f[kk][j] = j < FM ? *reinterpret_cast<const v4i*>(st + (ao ^ (kk << 6)) + j * 16 * BK)
+                          : *reinterpret_cast<const v4i*>(st + (wo ^ (kk << 6)) + (j - FM) * 16 * BK);
+    };
+    // the MFMAs of K half kk; the fragments of the half that follows are read behind the first of them
+    const auto half = [&](auto kk_tag, int next_step) {
+        constexpr int kk = decltype(kk_tag)::value;
+#pragma unroll
+        for (int in = 0; in < FN; ++in)
+#pragma unroll
+            for (int im = 0; im < FM; ++im) {
+                acc[in][im] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f[kk][FM + in], f[kk][im], acc[in][im], 0, 0, 0);
+                SCHED_FENCE();
+                if (in * FM + im < FM + FN) { read(next_step, 1 - kk, in * FM + im); SCHED_FENCE(); }
+            }
+    };
     wg_barrier();
 #pragma unroll
-    for (int j = 0; j < NF; ++j) f0[j] = frag(smem, smem + C::W_BASE, 0, j);
-
-    int ca = 0, cw = 0;   // stages of the iteration being multiplied
-    for (int ti = 0; ti < nt_b; ++ti) {
-#pragma unroll
-        for (int in = 0; in < TN; ++in)
-#pragma unroll
-            for (int im = 0; im < TM; ++im)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[in][im][r] = 0;
-        // The epilogue's stores are issued from inline assembly: were they visible to the compiler, it would assume
-        // them pending at the K loop's header and park a vmcnt(0) inside the loop, in front of the first fragment read,
-        // draining the DMA pipeline every iteration.  (Waits it derives for its own loads stay correct: the memory
-        // counter retires in order, so instructions it does not know about only make those waits stricter.)
-
-        int pa = 0, pw = 0;
-        for (int kt = 0; kt < nk; ++kt) {
-            const uint8_t* sa = smem + ca * C::A_STAGE;
-            const uint8_t* sw = smem + C::W_BASE + cw * C::W_STAGE;
-            const int na = ca == NSA - 1 ? 0 : ca + 1, nw = cw == C::NSW - 1 ? 0 : cw + 1;
-            wg_barrier();                                                   // X
-            substep(ic<0>{}, f0, f1, sa, sw, 1);
-            substep(ic<NM>{}, f1, f0, sa, sw, 2);
-            substep(ic<2 * NM>{}, f0, f1, sa, sw, 3);
-            wait_vmcnt<C::in_flight_at_y()>();
-            wg_barrier();                                                   // Y
-            substep(ic<3 * NM>{}, f1, f0, smem + na * C::A_STAGE, smem + C::W_BASE + nw * C::W_STAGE, 0);
-            advance_a();
-            advance_w();
-            pa = ca;
-            pw = cw;
-            ca = na;
-            cw = nw;
-        }
-
-        // epilogue of tile ti; the A stage that was just multiplied is the shuffle scratch (8 KB per wave).
-        // (The launcher only picks this kernel when the coalesced epilogue's alignment conditions hold.)
-        int m0, n0;
-        tile_origin(ti, m0, n0);
-        __syncthreads();   // every wave is done reading that stage
-        constexpr int SZ = (EPI == EPI_ACC || OUT_DT == DT_F32) ? 4 : 2;
-        constexpr int PW = C::piece_cols(SZ);
-        // Shuffle scratch, 8 KB per wave and region: the A stage and the W stage that were just multiplied (the DMA in
-        // flight fills the other stages; the next write into these two is issued inside the next iteration).
-        uint8_t* ra = smem + pa * C::A_STAGE + wave * C::A_REGION;
-        uint8_t* rw = smem + C::W_BASE + pw * C::W_STAGE + wave * C::W_REGION;
-        epilogue_shuffle<TM, TN, OUT_DT, EPI, PW, true, C::STAGED>(p, acc, m0 + wm * C::WTM, n0 + wn * C::WTN, hw_lane(), ra, rw,
-                                                               reinterpret_cast<float*>(rw + C::piece_bytes(SZ)));
-        // The first fragments of the next tile were prefetched by the last sub-step; fetching them again here instead of
-        // carrying 32 registers across the epilogue keeps the epilogue free of spills.
-#pragma unroll
-        for (int j = 0; j < NF; ++j) f0[j] = frag(smem + ca * C::A_STAGE, smem + C::W_BASE + cw * C::W_STAGE, 0, j);
+    for (int j = 0; j < FM + FN; ++j) read(0, 0, j);
+    for (int s = 0; s < nk; ++s) {
+        half(ic<0>{}, s);
+        wait_lgkmcnt0();
+        wg_barrier();
+        half(ic<1>{}, s + 1);   // past the last step: a stage of the ring, read and not used
     }
-    wait_vmcnt<0>();   // no DMA may still be writing this workgroup's LDS when it retires
+    wait_lgkmcnt0();
+    constexpr int SZ = (EPI == EPI_ACC || OUT_DT == DT_F32) ? 4 : 2;
+    constexpr int PW = C::piece_cols(SZ);
+    wg_barrier();
+    uint8_t* scratch = smem + wave * 16384;
+    epilogue_shuffle_with<C::TM, C::TN, OUT_DT, EPI, PW, true, 16, true>(p, acc, m0 + wm * 64, n0 + wn * C::TN * 32, hw_lane(), scratch, scratch + 8192, cst);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -904,7 +763,7 @@ __device__ __forceinline__ void pp_gemm_tiles(const GemmArgs& p, uint8_t* smem, 
 
     // DMA streams of this wave.  A wave fetches 8-row blocks wq, wq + 4, ... of the OTHER group's A rows and of its own
     // half of the W tile (group 0: rows 0..127, group 1: rows 128..255).
-    // Lane offsets carry the chunk swizzle (bits 1..3 of the row) on the global side, as in the ring kernel.
+    // Lane offsets carry the chunk swizzle (bits 1..3 of the row) on the global side, chunk c of row r at slot c ^ ((r >> 1) & 7).
     uint32_t ga[C::NLA], gw[C::NLW];
     // a stream's position: the (tile, k tile) it fetches next and the stage that goes to.  A stream stops on the last step
     // and keeps re-fetching it, into the stage it would have used, which nothing reads again.
@@ -1039,7 +898,7 @@ __device__ __forceinline__ void pp_gemm_tiles(const GemmArgs& p, uint8_t* smem, 
         int m0, n0;
         tile_origin(ti, m0, n0);
         uint8_t* scratch = smem + (s_last % C::NSW) * C::W_STAGE + wave * 4096;
-        epilogue_shuffle<TM, TN, OUT_DT, EPI, PW, true, false, 16>(p, acc, m0 + grp * C::GM, n0 + wq * C::WTN, hw_lane(), scratch);
+        epilogue_shuffle<TM, TN, OUT_DT, EPI, PW, true, 16>(p, acc, m0 + grp * C::GM, n0 + wq * C::WTN, hw_lane(), scratch);
     };
 
     // Both groups run the same loop; group 1 is one phase behind (the barrier in front) and multiplies its last step of a
@@ -1078,298 +937,6 @@ __global__ void __launch_bounds__(PpL::NT, 1) int8_gemm_pp_kernel(GemmArgs main,
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// Weight-streaming kernel for skinny M (M <= 256): one row of 256 x 96 tiles, every weight read from HBM exactly once.
-// Eight waves form two groups of four (one wave of each group per SIMD), and group g multiplies the K tiles
-// t = g, g + 2, ... of the workgroup's K range, all 256 x 96 outputs of them (wave tile 64 x 96, 4 x 6 tiles of
-// v_mfma_i32_16x16x64_i8), into accumulators of its own.  The groups alternate between two kinds of phase, with one
-// workgroup barrier per phase:
-//   compute: the 48 MFMAs of the group's K tile; the six W fragments of the second 64 K bytes are read behind the
-//            first MFMAs, and the wave's three DMA instructions of W follow the last one;
-//   memory:  the other 14 fragment reads of the group's next K tile with the wave's eight DMA instructions of A spread
-//            between them.
-// A group fetches only the K tiles it multiplies itself, so every wait for data is a wait of a wave on its own memory
-// counter, placed at the end of its compute phase.
-//
-// LDS: A in three stages of 32 KB, W in five of 12 KB (K tile t sits in stage t % 3 and t % 5), 2 KB of constants for the
-// epilogue.  In its memory phase before K tile t a group fetches A(t+2) into the stage of K tile t-1, whose fragments
-// the other group read a phase earlier; after multiplying K tile t it fetches W(t+4) into the W stage of K tile t-1,
-// whose second half the other group read during that earlier phase.  W, which comes from HBM, has three phases to land;
-// A, which comes from L2 behind it in the CU's in-order return path, has one and a half.
-//
-// What bounds this tile is how much a CU can keep in flight: 44 KB enter it per K tile, a third of them at HBM's
-// latency, and a kernel of any structure built on this tile (separate loader waves in lock step or free-running on LDS
-// counters, loads in registers instead of DMA) ran its K tile in the same 1350-1450 cycles.
-//
-// At the end the two groups swap halves of their accumulators through the LDS (the ring is dead by then) and each
-// finishes 32 of a wave tile's 64 rows; the tile's column constants and row scales were requested at the start and wait
-// in LDS.  Requires K % 128 == 0 and M*K, N*K < 2^32.
-// ---------------------------------------------------------------------------------------------------------------
-struct TurnCfg {
-    static constexpr int BM = 256, BN = 96, BK = 128, NSA = 3, NSW = 5, NT = 512;
-    static constexpr int TM = 2, TN = 3;                                       // wave tile 64 x 96 as 32 x 32 blocks
-    static constexpr int A_STAGE = BM * BK, W_STAGE = BN * BK, W_BASE = NSA * A_STAGE;
-    static constexpr int NLA = BM / 32, NLW = BN / 32;                         // DMA instructions (8 rows each) per wave and K tile
-    static constexpr int RING = W_BASE + NSW * W_STAGE;
-    static constexpr int CST_BASE = RING, CST_FLOATS = 2 * BN + BM, SMEM = RING + 2048;   // ws[96], bias[96], xs[256] as floats
-    static constexpr int HALF_ACC = 2 * TM * TN * 1024;                        // half of one wave's accumulators
-    static_assert(SMEM <= 160 * 1024 && CST_FLOATS * 4 <= 2048, "LDS budget");
-    static_assert(8 * HALF_ACC <= W_BASE && 8 * 4096 <= NSW * W_STAGE, "hand-over area and epilogue scratch fit the dead ring");
-};
-
-template <int OUT_DT, int EPI>
-__global__ void __launch_bounds__(TurnCfg::NT, 1) int8_gemm_turn_kernel(GemmArgs p) {
-    using C = TurnCfg;
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    constexpr int BK = C::BK, TM = C::TM, TN = C::TN, FM = 2 * TM, FN = 2 * TN;
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int grp = wave >> 2, wq = wave & 3;   // group; wave within the group = its 64-row quarter and its DMA blocks
-    const int ld = p.K;
-    // split K: workgroup row blockIdx.y multiplies K slice [k_lo, k_lo + nk*128) and writes its own int32 plane
-    const int k_lo = p.kslice ? (int)blockIdx.y * p.kslice : 0;
-    const int k_len = p.kslice ? (p.K - k_lo < p.kslice ? p.K - k_lo : p.kslice) : p.K;
-    const int nk = k_len / BK;
-    if (p.kslice) p.D = (uint8_t*)p.D + (int64_t)blockIdx.y * p.M * p.N * 4;
-    const int G = gridDim.x, ntiles = p.tiles_m * p.tiles_n;
-    const int nt_b = (ntiles - (int)blockIdx.x + G - 1) / G;   // tiles of this workgroup: blockIdx, blockIdx + G, ...
-    // The K tiles are walked from a start that differs between the workgroups of an XCD (the int32 sums do not depend
-    // on the order), so that they do not all ask that XCD's L2 for the same lines of A at the same moment.
-    const int rot = (int)(((blockIdx.x >> 3) & 31) * (unsigned)nk) >> 5;
-    auto rk = [&](int kt) { kt = kt < nk ? kt : nk - 1; return kt + rot < nk ? kt + rot : kt + rot - nk; };
-    const uint32_t lds_base = (uint32_t)(uintptr_t)smem;
-    auto dma = [&](uint32_t dst, uint32_t off, const int8_t* base) {
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory", "m0");
-    };
-
-    // DMA streams of this wave: 8-row blocks wq, wq + 4, ... of the A tile and of the W tile, of this group's K tiles.
-    // The chunk swizzle (bits 1..3 of the row) is applied on the global side; a block's parity is the wave's.
-    // (Giving W to one wave of the group and A to the other three, so that no wave's A loads queue behind its own W
-    // loads, was measured and is slower: what A waits behind is the CU's return path, not the wave's counter.)
-    uint32_t ga[C::NLA], gw[C::NLW];
-    auto set_rows = [&](int m0, int n0) {
-        const int l = hw_lane();
-        const int lr = l >> 3, lc = ((l & 7) ^ (((wq & 1) << 2) | (lr >> 1))) * 16;
-#pragma unroll
-        for (int j = 0; j < C::NLA; ++j) {
-            const int row = m0 + (wq + 4 * j) * 8 + lr;
-            ga[j] = (uint32_t)(row < p.M ? row : p.M - 1) * (uint32_t)ld + lc;
-        }
-#pragma unroll
-        for (int j = 0; j < C::NLW; ++j) {
-            const int row = n0 + (wq + 4 * j) * 8 + lr;
-            gw[j] = (uint32_t)(row < p.N ? row : p.N - 1) * (uint32_t)ld + lc;
-        }
-    };
-    // K tile and stage each stream fetches next (a stream past the last K tile re-fetches it, into a stage that nothing
-    // reads again: the number of instructions per phase, which the wait counts assume, stays fixed)
-    int a_t, a_st, w_t, w_st, r_sa, r_sw;
-    // source and destination of the A blocks a memory phase fetches
-    const int8_t* base_a;
-    uint32_t dst_a;
-    auto fetch_one = [&](auto D) { dma(dst_a + decltype(D)::value * 4096, ga[decltype(D)::value], base_a); };
-    auto fetch_w = [&]() {
-        const int8_t* base = p.W + k_lo + (int64_t)rk(w_t) * BK;
-        const uint32_t dst = lds_base + C::W_BASE + w_st * C::W_STAGE + wq * 1024;
-#pragma unroll
-        for (int j = 0; j < C::NLW; ++j) dma(dst + j * 4096, gw[j], base);
-        w_t += 2;
-        w_st = w_st >= 3 ? w_st - 3 : w_st + 2;
-    };
-    auto fetch_a = [&]() {
-        const int8_t* base = p.A + k_lo + (int64_t)rk(a_t) * BK;
-        const uint32_t dst = lds_base + a_st * C::A_STAGE + wq * 1024;
-#pragma unroll
-        for (int j = 0; j < C::NLA; ++j) dma(dst + j * 4096, ga[j], base);
-        a_t += 2;
-        a_st = a_st == 0 ? 2 : a_st - 1;
-    };
-
-    // Fragments: row r of a stage at r*128, chunk c at slot c ^ ((r>>1)&7); a lane reads row lane % 16, chunk
-    // 4*kk + lane / 16 of K half kk (which flips bit 6 of the address).
-    v4i acc[FN][FM];
-    v4i f[2][FM + FN];
-    // The memory phase: 14 fragment reads of the group's next K tile (all of A, and W for the first 64 K bytes) with the
-    // wave's 8 DMA instructions of A spread between them.  The six W fragments of the second 64 K bytes are read in the
-    // compute phase, behind the first MFMAs, and the three DMA instructions of W follow the last MFMA: a compute phase
-    // (768 cycles of MFMA) would otherwise be a third shorter than the memory phase beside it, whose reads return at the
-    // SIMD's pace of about 25 cycles each and whose DMA instructions hold the wave about 50 cycles each.  W can move
-    // because its ring has the room (a stage stays readable for one phase more), A cannot.
-    const uint8_t* sw_cur = smem;   // W stage of the K tile whose fragments are in registers (its second half still in LDS)
-    int fx = 0;
-    auto memory = [&]() {
-        constexpr int ND = C::NLA;
-        const int l = hw_lane();
-        const int frow = l & 15, fq = l >> 4;
-        const int x = frow * BK + ((fq ^ ((frow >> 1) & 7)) << 4);
-        const uint8_t* sa = smem + r_sa * C::A_STAGE + wq * 64 * BK;
-        const uint8_t* sw = smem + C::W_BASE + r_sw * C::W_STAGE;
-        sw_cur = sw;
-        fx = x ^ 64;
-        r_sa = r_sa == 0 ? 2 : r_sa - 1;
-        r_sw = r_sw >= 3 ? r_sw - 3 : r_sw + 2;
-        base_a = p.A + k_lo + (int64_t)rk(a_t) * BK;
-        dst_a = lds_base + a_st * C::A_STAGE + wq * 1024;
-        a_t += 2;
-        a_st = a_st == 0 ? 2 : a_st - 1;            // + 2 mod 3
-        constexpr int NF = 2 * FM + FN;
-        static_for<NF>([&](auto I) {
-            constexpr int i = decltype(I)::value;
-            if constexpr (i < FM) f[0][i] = *reinterpret_cast<const v4i*>(sa + x + i * 16 * BK);
-            else if constexpr (i < FM + FN) f[0][i] = *reinterpret_cast<const v4i*>(sw + x + (i - FM) * 16 * BK);
-            else f[1][i - FM - FN] = *reinterpret_cast<const v4i*>(sa + (x ^ 64) + (i - FM - FN) * 16 * BK);
-            SCHED_FENCE();
-            // DMA instruction d goes behind read (d * NF) / ND + 1
-            static_for<ND>([&](auto D) {
-                if constexpr ((decltype(D)::value * NF) / ND + 1 == i) { fetch_one(D); SCHED_FENCE(); }
-            });
-        });
-        static_for<ND>([&](auto D) {
-            if constexpr ((decltype(D)::value * NF) / ND + 1 >= NF) { fetch_one(D); SCHED_FENCE(); }
-        });
-    };
-    auto compute = [&]() {
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int in = 0; in < FN; ++in)
-#pragma unroll
-            for (int im = 0; im < FM; ++im) {
-                acc[in][im] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f[0][FM + in], f[0][im], acc[in][im], 0, 0, 0);
-                SCHED_FENCE();
-                if (im == 1) {   // one W fragment of the second half behind every fourth MFMA
-                    f[1][FM + in] = *reinterpret_cast<const v4i*>(sw_cur + fx + in * 16 * BK);
-                    SCHED_FENCE();
-                }
-            }
-#pragma unroll
-        for (int in = 0; in < FN; ++in)
-#pragma unroll
-            for (int im = 0; im < FM; ++im) {
-                acc[in][im] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f[1][FM + in], f[1][im], acc[in][im], 0, 0, 0);
-                SCHED_FENCE();
-            }
-        __builtin_amdgcn_s_setprio(0);
-        fetch_w();                                 // W(t + 4), into the stage whose second half the other group read a phase ago
-    };
-
-    for (int ti = 0; ti < nt_b; ++ti) {
-        int m0, n0;
-        {
-            int tm, tn;
-            tile_of_block((int)blockIdx.x + ti * G, ntiles, p.tiles_m, p.tiles_n, tm, tn, p.magic);
-            m0 = tm * C::BM;
-            n0 = tn * C::BN;
-        }
-        set_rows(m0, n0);
-#pragma unroll
-        for (int in = 0; in < FN; ++in)
-#pragma unroll
-            for (int im = 0; im < FM; ++im) acc[in][im] = v4i{0, 0, 0, 0};
-        // The column constants and row scales of the tile are requested now and parked in LDS at the end of the K loop, so
-        // that the epilogue finds them there instead of waiting for memory.
-        float2 c_ws = make_float2(0.f, 0.f), c_b = make_float2(0.f, 0.f);
-        float c_xs[4] = {0.f, 0.f, 0.f, 0.f};
-        const bool stager = EPI != EPI_ACC && wave == 7;
-        if (stager) {
-            const int l = hw_lane();
-            int n = n0 + 2 * l;
-            n = n < p.N ? n : p.N - 2;
-            if (2 * l < C::BN) {
-                c_ws = *reinterpret_cast<const float2*>(p.ws + n);
-                if (p.bias) {
-                    c_b.x = ld_dt<(EPI == EPI_ACC || OUT_DT == DT_F32) ? DT_F32 : OUT_DT>(p.bias, n);
-                    c_b.y = ld_dt<(EPI == EPI_ACC || OUT_DT == DT_F32) ? DT_F32 : OUT_DT>(p.bias, n + 1);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) c_xs[j] = m0 + l + 64 * j < p.M ? p.xs[m0 + l + 64 * j] : 0.f;
-        }
-        // prologue.  Group 0 asks for its first K tile (W first: it has the longer way), then group 1 for its first, so
-        // that what the first compute phase needs is at the head of the CU's return path.
-        a_t = grp; w_t = grp;
-        a_st = grp; w_st = grp;
-        r_sa = grp; r_sw = grp;
-        if (grp == 0) {
-            fetch_w();
-            fetch_a();
-            wg_barrier();
-            fetch_w();
-            wait_vmcnt<C::NLW>();              // all but the second W tile
-        } else {
-            wg_barrier();
-            fetch_w();
-            fetch_a();
-            fetch_w();
-        }
-        wg_barrier();
-        if (grp == 1) wait_vmcnt<C::NLW>();
-        // Both groups run the same loop, group 1 one phase behind.
-        if (grp == 1) wg_barrier();
-        for (int t = grp; t < nk; t += 2) {
-            memory();                          // fragments of K tile t; A(t + 2)
-            wait_lgkmcnt0();
-            wg_barrier();
-            compute();                         // K tile t; W(t + 4)
-            wait_vmcnt<C::NLW>();              // everything but the W tile fetched last has landed
-            wg_barrier();
-        }
-        if ((nk & 1) == grp) wg_barrier();     // the group with fewer K tiles sits out the last phase
-        wait_vmcnt<0>();
-        if (stager) {
-            float* cst = reinterpret_cast<float*>(smem + C::CST_BASE);
-            const int l = hw_lane();
-            if (2 * l < C::BN) {
-                *reinterpret_cast<float2*>(cst + 2 * l) = c_ws;
-                *reinterpret_cast<float2*>(cst + C::BN + 2 * l) = c_b;
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) cst[2 * C::BN + l + 64 * j] = c_xs[j];
-        }
-        __syncthreads();                       // no DMA in flight, nobody reads fragments: the LDS is free
-        // Each group finishes half of every wave tile: group 0 the 16-row tiles 0 and 1 of its waves' 64 rows, group 1
-        // tiles 2 and 3.  A wave parks the other group's half of its accumulators in LDS and adds the half it is handed.
-        v4i fin[FN][2];
-        {
-            uint8_t* mine = smem + wave * C::HALF_ACC + hw_lane() * 16;
-            const uint8_t* theirs = smem + (wave ^ 4) * C::HALF_ACC + hw_lane() * 16;
-            if (nk > 1) {
-#pragma unroll
-                for (int in = 0; in < FN; ++in)
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        *reinterpret_cast<v4i*>(mine + (in * 2 + h) * 1024) = grp == 0 ? acc[in][2 + h] : acc[in][h];
-                        fin[in][h] = grp == 0 ? acc[in][h] : acc[in][2 + h];
-                    }
-                __syncthreads();
-#pragma unroll
-                for (int in = 0; in < FN; ++in)
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) fin[in][h] += *reinterpret_cast<const v4i*>(theirs + (in * 2 + h) * 1024);
-            } else {   // one K tile: group 0 holds all of it and hands group 1 its half
-#pragma unroll
-                for (int in = 0; in < FN; ++in)
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        if (grp == 0) *reinterpret_cast<v4i*>(mine + (in * 2 + h) * 1024) = acc[in][2 + h];
-                        fin[in][h] = acc[in][h];
-                    }
-                __syncthreads();
-                if (grp == 1) {
-#pragma unroll
-                    for (int in = 0; in < FN; ++in)
-#pragma unroll
-                        for (int h = 0; h < 2; ++h) fin[in][h] = *reinterpret_cast<const v4i*>(theirs + (in * 2 + h) * 1024);
-                }
-            }
-        }
-        {
-            uint8_t* scratch = smem + C::W_BASE + wave * 4096;   // a 4 KB shuffle piece per wave
-            float* cst = reinterpret_cast<float*>(smem + C::CST_BASE);
-            const int rows = wq * 64 + grp * 32;
-            epilogue_shuffle<1, TN, OUT_DT, EPI, 32, true, 2, 16>(p, fin, m0 + rows, n0, hw_lane(), scratch, nullptr, cst, cst + 2 * C::BN + rows);
-        }
-        if (ti + 1 < nt_b) __syncthreads();    // the next tile's prologue overwrites what the epilogue reads
-    }
-}
-
 // Up to 128 rows: weights straight from HBM into the registers that the matrix instruction reads, rows of A through LDS.  The
 // kernel above moves all 256 rows of A to every CU for 96 columns of W, and what it moves bounds it; with M rows of A in
 // 16-row tiles (MT of them) the weights are most of what a CU takes in.
@@ -1597,28 +1164,6 @@ int launch_cfg(GemmArgs a, hipStream_t st) {
     return 0;
 }
 
-// Launches the persistent ring kernel on `slices` K slices (1 = whole K).  With slices > 1, EPI must be EPI_ACC and
-// a.D the int32 planes.
-template <class C, int OUT_DT, int EPI>
-int launch_ring_cfg(GemmArgs a, int slices, hipStream_t st) {
-    a.tiles_m = (a.M + C::BM - 1) / C::BM;
-    a.tiles_n = (a.N + C::BN - 1) / C::BN;
-    a.magic = panel_magic(a.tiles_m, a.tiles_n);
-    const int64_t ntiles = (int64_t)a.tiles_m * a.tiles_n;
-    if (ntiles > 0x7fffffff) return -1;
-    auto kern = int8_gemm_ring_kernel<C, OUT_DT, EPI>;
-    static PerDeviceOnce once;
-    if (const int e = allow_dynamic_lds((const void*)kern, C::SMEM, once)) return e;
-    const int num_cu = device_cu_count();
-    const int64_t per_slice = slices > 1 ? (num_cu / slices > 0 ? num_cu / slices : 1) : num_cu;
-    const unsigned grid = (unsigned)(ntiles < per_slice ? ntiles : per_slice);
-    hipLaunchKernelGGL(kern, dim3(grid, (unsigned)slices), dim3(C::NT), C::SMEM, st, a);
-    KCHECK();
-    return 0;
-}
-
-using RingS = RingCfg<192, 2, 2, 3, 128>;    // 128x192, waves 2x2 of 64x96: shapes with too few 256x256 tiles for the CUs
-
 // Rows [row0, row0 + rows) of the problem as a problem of its own.
 template <int OUT_DT, int EPI>
 GemmArgs row_band(const GemmArgs& a, int64_t row0, int64_t rows) {
@@ -1637,28 +1182,30 @@ GemmArgs row_band(const GemmArgs& a, int64_t row0, int64_t rows) {
 // idle, a sixth of the run).  The tile rows that fill whole rounds are then run as 256x256 tiles and the rows left over
 // as 128x256 tiles by further workgroups of the same launch, when that is estimated to be shorter (a small tile costs
 // about 0.6 of a large one).
+struct PpSplit { int64_t main_rows, small; double rounds; };   // tile rows of large tiles, small tiles behind them, rounds of large tiles in all
+PpSplit pp_split(int64_t M, int64_t N, int64_t cus) {
+    const int64_t tm = (M + PpL::BM - 1) / PpL::BM, tn = (N + PpL::BN - 1) / PpL::BN, full = tm * tn / cus, rem = tm * tn % cus;
+    const PpSplit whole{tm, 0, (double)(full + (rem > 0))};
+    if (full < 1 || rem == 0 || tm < 2) return whole;
+    const int64_t main_rows = full * cus / tn < tm ? full * cus / tn : tm - 1;
+    const int64_t small = ((M - main_rows * PpL::BM + PpS::BM - 1) / PpS::BM) * tn;
+    const double cost = (double)((main_rows * tn + cus - 1) / cus) + 0.6 * (double)((small + cus - 1) / cus);
+    return main_rows > 0 && cost < (double)(full + 1) - 0.1 ? PpSplit{main_rows, small, cost} : whole;
+}
+
 template <int OUT_DT, int EPI>
 int launch_pp(GemmArgs a, hipStream_t st) {
     bool vec_ok, aligned;
     epilogue_alignment<OUT_DT, EPI>(a, vec_ok, aligned);
     if (!aligned) return launch_cfg<CfgM, OUT_DT, EPI>(a, st);   // this kernel has only the coalesced epilogue
     const int64_t G = device_cu_count();
-    const int64_t tm = (a.M + PpL::BM - 1) / PpL::BM, tn = (a.N + PpL::BN - 1) / PpL::BN;
-    const int64_t full = tm * tn / G, rem = tm * tn % G;
+    const int64_t tn = (a.N + PpL::BN - 1) / PpL::BN;
+    const PpSplit sp = pp_split(a.M, a.N, G);
     GemmArgs main = a, rest = a;
-    int64_t n_main = tm * tn, n_rest = 0;
-    if (full >= 1 && rem > 0 && tm > 1) {
-        int64_t main_rows = full * G / tn;
-        if (main_rows >= tm) main_rows = tm - 1;
-        const int64_t m_main = main_rows * PpL::BM, m_rest = a.M - m_main;
-        const int64_t small = ((m_rest + PpS::BM - 1) / PpS::BM) * tn;
-        const double split_cost = (double)((main_rows * tn + G - 1) / G) + 0.6 * (double)((small + G - 1) / G);
-        if (main_rows > 0 && split_cost < (double)(full + 1) - 0.1) {
-            main = row_band<OUT_DT, EPI>(a, 0, m_main);
-            rest = row_band<OUT_DT, EPI>(a, m_main, m_rest);
-            n_main = main_rows * tn;
-            n_rest = small;
-        }
+    const int64_t n_main = sp.main_rows * tn, n_rest = sp.small;
+    if (n_rest) {
+        main = row_band<OUT_DT, EPI>(a, 0, sp.main_rows * PpL::BM);
+        rest = row_band<OUT_DT, EPI>(a, sp.main_rows * PpL::BM, a.M - sp.main_rows * PpL::BM);
     }
     if (n_main > 0x7fffffff) return -1;
     main.tiles_m = (main.M + PpL::BM - 1) / PpL::BM;
@@ -1677,21 +1224,12 @@ int launch_pp(GemmArgs a, hipStream_t st) {
 }
 
 
-// The 128x192 ring kernel on the whole problem: shapes with too few 256x256 tiles to fill the CUs.
-template <int OUT_DT, int EPI>
-int launch_ring_small(GemmArgs a, hipStream_t st) {
-    bool vec_ok, aligned;
-    epilogue_alignment<OUT_DT, EPI>(a, vec_ok, aligned);
-    if (!aligned) return launch_cfg<CfgM, OUT_DT, EPI>(a, st);
-    return launch_ring_cfg<RingS, OUT_DT, EPI>(a, 1, st);
-}
-
 // ---------------------------------------------------------------------------------------------------------------
 // Scratch of the entry point that allocates nothing (gpu_int8_gemm_static): the int32 planes of a split-K run live in
 // this file-scope device array instead of a stream-ordered allocation.  Every GPU the library runs on holds its own
 // copy at its own address until the process ends; the array's name is only a host-side handle, so the device address
-// is looked up once per device and host code uses that pointer from then on.  24 MiB covers every shape the skinny
-// path splits on a GPU with up to 256 CUs: slices * N <= 256 * 96 columns and M <= 256 rows of int32.
+// is looked up once per device and host code uses that pointer from then on.  24 MiB covers every shape that is split on a
+// GPU with up to 256 CUs: slices * tiles <= 256, and no tile of int32 is larger than 128 x 192.
 // ---------------------------------------------------------------------------------------------------------------
 constexpr size_t kStaticScratchBytes = (size_t)24 << 20;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
@@ -1736,14 +1274,14 @@ void retain_pool_memory() {
 // Split-K planes of the allocating entry points: one buffer per (device, stream), made on that stream's first split
 // call and kept until the process ends.  Work on one stream is ordered, so its calls can share a buffer, and a
 // stream-ordered allocation per call costs about 7 us on the stream's timeline (measured: 31 against 24 us per call at
-// M=256, K=12288, N=4096).  The buffer has the one size every shape that the dispatcher splits fits into (slices *
-// column tiles <= CUs: slices * N <= CUs * 96 times 256 rows of int32 in the streaming kernel, 24 MiB on 256 CUs, and
-// CUs * 64 times 128 rows in the kernel for up to 128) and is never grown or
+// M=256, K=12288, N=4096).  The buffer has the one size every shape that the dispatcher splits fits into (slices * tiles <= CUs, and
+// no tile of int32 is larger than 128 x 192: 24 MiB on 256 CUs) and is never grown or
 // freed, so a captured graph that holds its address stays valid.  At most kStreamPlanes streams per process are served;
 // a call on any further stream, a first call made under capture, or a shape beyond the size (a forced configuration)
 // falls back to a stream-ordered allocation, and so does hipStreamPerThread (one handle for a different stream in every
 // thread).  A stream handle that the runtime reuses after hipStreamDestroy inherits
 // the destroyed stream's buffer; work still queued on the destroyed stream at that moment would share it.
+constexpr size_t kPlanesPerCu = 128 * 192 * sizeof(int);
 struct StreamPlanes { int dev; hipStream_t st; void* ptr; size_t bytes; };
 constexpr int kStreamPlanes = 8;
 std::mutex g_planes_mu;
@@ -1764,7 +1302,7 @@ void* stream_planes(hipStream_t st, size_t need, int num_cu) {
     std::lock_guard<std::mutex> lock(g_planes_mu);
     for (int i = 0; i < g_planes_n; ++i)
         if (g_planes[i].dev == dev && g_planes[i].st == st) return need <= g_planes[i].bytes ? g_planes[i].ptr : nullptr;
-    const size_t bytes = (size_t)num_cu * TurnCfg::BN * TurnCfg::BM * sizeof(int);
+    const size_t bytes = (size_t)num_cu * kPlanesPerCu;
     if (g_planes_n == kStreamPlanes || need > bytes) return nullptr;
     if (is_capturing(st)) return nullptr;
     void* ptr = nullptr;
@@ -1774,27 +1312,6 @@ void* stream_planes(hipStream_t st, size_t need, int num_cu) {
     }
     g_planes[g_planes_n++] = StreamPlanes{dev, st, ptr, bytes};
     return ptr;
-}
-
-// Launches the weight-streaming kernel on `slices` K slices (1 = whole K).  With slices > 1, EPI must be EPI_ACC and a.D
-// the int32 planes.
-template <int OUT_DT, int EPI>
-int launch_stream(GemmArgs a, int slices, hipStream_t st) {
-    using C = TurnCfg;
-    a.tiles_m = (a.M + C::BM - 1) / C::BM;
-    a.tiles_n = (a.N + C::BN - 1) / C::BN;
-    a.magic = panel_magic(a.tiles_m, a.tiles_n);
-    const int64_t ntiles = (int64_t)a.tiles_m * a.tiles_n;
-    if (ntiles > 0x7fffffff) return -1;
-    auto kern = int8_gemm_turn_kernel<OUT_DT, EPI>;
-    static PerDeviceOnce once;
-    if (const int e = allow_dynamic_lds((const void*)kern, C::SMEM, once)) return e;
-    const int num_cu = device_cu_count();
-    const int64_t per_slice = slices > 1 ? (num_cu / slices > 0 ? num_cu / slices : 1) : num_cu;
-    const unsigned grid = (unsigned)(ntiles < per_slice ? ntiles : per_slice);
-    hipLaunchKernelGGL(kern, dim3(grid, (unsigned)slices), dim3(C::NT), C::SMEM, st, a);
-    KCHECK();
-    return 0;
 }
 
 // A run on `slices` slices of kslice values of K: `body` writes the int32 planes, a second kernel adds them (exact, so the order of
@@ -1839,26 +1356,85 @@ int launch_split(const GemmArgs& a, int slices, int kslice, hipStream_t st, Body
     return rc;
 }
 
-// M <= 256: one row of 256 x 96 tiles, the weights are read once and the run is bound by how fast they stream.  When N
-// is too small to give every CU a column slab, K is split as well: each slice writes an int32 plane (exact, so the
-// order of the sum does not matter) into the stream's scratch buffer and a second kernel adds the planes and applies
-// the epilogue.
+template <class C, int OUT_DT, int EPI>
+int launch_fed_cfg(GemmArgs a, int slices, hipStream_t st) {
+    a.tiles_m = (a.M + C::BM - 1) / C::BM;
+    a.tiles_n = (a.N + C::BN - 1) / C::BN;
+    a.magic = panel_magic(a.tiles_m, a.tiles_n);
+    const int64_t ntiles = (int64_t)a.tiles_m * a.tiles_n;
+    if (ntiles > 0x7fffffff) return -1;
+    auto kern = int8_gemm_fed_kernel<C, OUT_DT, EPI>;
+    static PerDeviceOnce once;
+    if (const int e = allow_dynamic_lds((const void*)kern, C::SMEM, once)) return e;
+    hipLaunchKernelGGL(kern, dim3((unsigned)ntiles, (unsigned)slices), dim3(C::NT), C::SMEM, st, a);
+    KCHECK();
+    return 0;
+}
 template <int OUT_DT, int EPI>
-int launch_skinny(GemmArgs a, hipStream_t st) {
+int launch_fed_as(const GemmArgs& a, int width, int slices, hipStream_t st) {
+    return width == 1   ? launch_fed_cfg<FedCfg<1>, OUT_DT, EPI>(a, slices, st)
+           : width == 2 ? launch_fed_cfg<FedCfg<2>, OUT_DT, EPI>(a, slices, st)
+                        : launch_fed_cfg<FedCfg<3>, OUT_DT, EPI>(a, slices, st);
+}
+
+// Tile width (of 64 columns) and K slices of the kernel with fetching waves, and its estimated time: rounds of one tile per CU, so many
+// us each and per step of 128, more per step where a CU has several tiles in a row (the clock goes down), or the weights' trip
+// from HBM, which a CU cannot take in faster than about 35 bytes per ns; a split pays for its planes and the launch that adds them.
+// The constants are fitted to 1190 shapes of 33 to 8192 rows (K 512 to 12288, N 640 to 24576, weights from HBM), where
+// the choice by these sums is 0.5 % slower than the best of all widths and slices on the average, and 1.34 times (1.55 times up to 512 rows)
+// as fast as what ran them before.
+struct FedPlan { int width, slices, per; double us; };   // per: K of a slice
+FedPlan fed_plan(int64_t M, int64_t N, int64_t K, int num_cu, bool may_split) {
+    // fixed, per round, per step of one round and of the rounds after it; a round after the first costs 0.5 more
+    static constexpr double c[3][4] = {{2.9, 1.1, 0.225, 0.25}, {1.9, 2.0, 0.29, 0.50}, {0.9, 3.55, 0.44, 0.66}};
+    const int steps = (int)(K / 128), cus = num_cu;
+    FedPlan best{3, 1, (int)K, 1e30};
+    for (int w = 1; w <= 3; ++w) {
+        const int64_t all = ((M + 127) / 128) * ((N + 64 * w - 1) / (64 * w));
+        const int tiles = all < 1 << 24 ? (int)all : 1 << 24;
+        // slices: none, two, as many as give every CU a tile, half of that
+        const int most = !may_split ? 1 : cus / tiles < steps / 3 ? cus / tiles : steps / 3;
+        const int tried[4] = {1, 2, most / 2, most};
+        for (int i = 0; i < 4; ++i) {
+            int s = tried[i];
+            if (i > 0 && (s < 2 || s > most || (i == 2 && s == 2))) continue;
+            const int per = (steps + s - 1) / s;
+            s = (steps + per - 1) / per;   // no empty slice
+            const int busy = tiles * s < cus ? tiles * s : cus;
+            const double n = (double)((tiles * s + cus - 1) / cus);
+            double us = c[w - 1][0] + n * c[w - 1][1] + (n - 1.) * 0.5 + (c[w - 1][2] + (n - 1.) * c[w - 1][3]) * per;
+            if (s > 1) us += 4.0 + (double)s * (double)M * (double)N * (8.0 / 4.2e6);
+            const double hbm = 4.0 + (double)N * (double)K / (34700. * busy);
+            if (us < hbm) us = hbm;
+            if (us < best.us) best = {w, s, per * 128, us};
+        }
+    }
+    return best;
+}
+// The two-group kernel's time on the same scale.
+double pp_us(int64_t M, int64_t N, int64_t K, int cus) {
+    const double n = pp_split(M, N, cus).rounds;
+    return -4.2 + n * (10.6 + 0.95 * (double)(K / 128));
+}
+
+// Whether a call may split K over workgroups.  Captured graphs and the static entry point do so only for the shapes that always did
+// there: elsewhere a graph holds no address of the stream's planes, so that it may be replayed on any stream, and the static
+// entry point leaves its buffer alone.
+bool fed_may_split(int64_t M, int64_t N, int64_t K, hipStream_t st) {
+    if (M <= 256 && K >= 4096 && N >= 1024 && N <= (M > 64 ? 8192 : 4096)) return true;
+    return tl_scratch == nullptr && !is_capturing(st);
+}
+
+template <int OUT_DT, int EPI>
+int launch_fed(GemmArgs a, hipStream_t st) {
     bool vec_ok, aligned;
     epilogue_alignment<OUT_DT, EPI>(a, vec_ok, aligned);
-    if (!aligned) return launch_cfg<CfgM, OUT_DT, EPI>(a, st);
-    const int num_cu = device_cu_count();
-    const int t96 = (a.N + 95) / 96, nk = a.K / 128;
-    int slices = t96 * 4 >= num_cu * 3 ? 1 : num_cu / t96;
-    if (slices > nk) slices = nk;
-    if (slices > 1) {
-        const int per = (nk + slices - 1) / slices;   // K tiles per slice
-        slices = (nk + per - 1) / per;                // no empty slice
-    }
-    if (slices <= 1) return launch_stream<OUT_DT, EPI>(a, 1, st);
-    const int per = (nk + slices - 1) / slices;
-    return launch_split<OUT_DT, EPI>(a, slices, per * 128, st, [&](const GemmArgs& pa) { return launch_stream<DT_F32, EPI_ACC>(pa, slices, st); });
+    if (!aligned) return launch_cfg<CfgM, OUT_DT, EPI>(a, st);   // only a forced family
+    FedPlan p = fed_plan(a.M, a.N, a.K, device_cu_count(), true);
+    if (p.slices > 1 && !fed_may_split(a.M, a.N, a.K, st)) p = fed_plan(a.M, a.N, a.K, device_cu_count(), false);
+    a.kslice = 0;
+    if (p.slices == 1) return launch_fed_as<OUT_DT, EPI>(a, p.width, 1, st);
+    return launch_split<OUT_DT, EPI>(a, p.slices, p.per, st, [&](const GemmArgs& pa) { return launch_fed_as<DT_F32, EPI_ACC>(pa, p.width, p.slices, st); });
 }
 
 template <int MT, int NWK, int OUT_DT, int EPI>
@@ -1920,30 +1496,26 @@ int launch_rows(GemmArgs a, hipStream_t st) {
         a.kslice = 0;
         return launch_rows_as<OUT_DT, EPI>(a, p.mt, p.nwk, vec_ok, 1, st);
     }
-    // Outputs that are narrow, or whose rows or pointers are not whole 16 bytes, do not split K in the streaming kernel either
-    // (choose_cfg, launch_skinny).  A captured graph of them holds no address of the stream's planes, so that it may be replayed on any
-    // stream, and the static entry point leaves its buffer alone: they take the register-staged tiles there.
+    // Outputs that are narrow, or whose rows or pointers are not whole 16 bytes, do not split K under capture (fed_may_split has the
+    // reason) nor in the static entry point.
     if ((a.N < 1024 || !aligned) && (tl_scratch != nullptr || is_capturing(st)))
-        return a.N < 1024 ? launch_cfg<CfgS, OUT_DT, EPI>(a, st) : launch_cfg<CfgM, OUT_DT, EPI>(a, st);
+        return aligned ? launch_fed<OUT_DT, EPI>(a, st) : a.N < 1024 ? launch_cfg<CfgS, OUT_DT, EPI>(a, st) : launch_cfg<CfgM, OUT_DT, EPI>(a, st);
     return launch_split<OUT_DT, EPI>(a, p.slices, p.per, st, [&](const GemmArgs& pa) { return launch_rows_as<DT_F32, EPI_ACC>(pa, p.mt, p.nwk, true, p.slices, st); });
 }
 
-// Where the kernels beside it are faster than the one for up to 128 rows (us, that one and the other):
-//   * short K and few columns: the small register-staged tiles have less to start (24 rows 768 -> 768 6.3 and 5.8; 128 rows 1152 -> 512
-//     8.5 and 7.5; but 48 rows 768 -> 768 4.8 and 5.8, 128 rows 1280 -> 640 8.5 and 9.2);
-//   * long K, and columns whose 96-wide tiles and K slices in the streaming kernel give a quarter more CUs a workgroup: a workgroup's
-//     own stretch of K is what the call waits for, the longer the fewer rows of A it takes in beside the weights (96 rows
-//     12288 -> 9216 36 and 28; 64 rows 14336 -> 4608 33 and 26; 32 rows 12288 -> 9216 28 and 26; but 64 rows 5120 -> 5120 13 and 15).
-// Outputs not of whole 16 bytes do not run there.
-bool rows_kernel_loses(int64_t M, int64_t N, int64_t K, bool aligned) {
-    if (K < 896) return N < 1152 && (M <= 32 || M > 64);
-    if (M > 64 && K >= 1024 && K < (M > 96 ? 1408 : 1280)) return N < (K < 1152 ? 1024 : 640);
-    if (M <= 16 || K < 5120 || N < 1024 || !aligned) return false;
-    const int cus = device_cu_count(), t96 = (int)((N + 95) / 96);
-    const RowsPlan p = rows_plan(M, N, K, cus, true);
-    const int here = p.tiles * p.slices, there = t96 * (cus / t96 > 1 ? cus / t96 : 1);
-    if (there * 4 < here * 5) return false;
-    return M > 64 ? p.per >= 5120 : M > 32 ? p.per >= 7168 : p.per >= 11264 && (p.nwk == 2 || here * 5 < cus * 3);
+// Whether the kernel for up to 128 rows runs a shape.  For outputs of whole 16 bytes: few rows, long K and few columns, where the
+// other kernel's planes and the launch that adds them cost more than the rows kernel's unevenly filled CUs.  Its time over that of
+// the kernel with fetching waves, 900 shapes with weights from HBM: up to 16 rows 0.65 to 1.0 from K = 2560 on and up to 8192 columns,
+// and 0.85 to 1.05 from K = 3584 on and 9500 to 16384 columns, but 1.0 at K = 2048, 1.1 to 1.3 just above 8192 columns (one more round) and
+// 1.1 to 1.6 above 16384; 17 to 64 rows 0.77 to 1.0 from K = 3072 on and up to 1280 columns, but 1.05 to
+// 1.15 at K = 2048 and 1.0 to 1.6 for more columns; 65 to 128 rows 1.0 to 1.7.  Other outputs have the register-staged tiles beside
+// them, which have less to start (128 rows 1152 -> 512 8.5 and 7.5 us; but 128 rows 1280 -> 640 8.5 and 9.2).
+bool rows_kernel_wins(int64_t M, int64_t N, int64_t K, bool aligned) {
+    if (aligned && M <= 16) return N <= 8192 ? K >= 2560 : K >= 3584 && N > 9500 && N <= 16384;
+    if (aligned) return M <= 64 && K >= 3072 && N <= 1280;
+    if (K < (M > 96 ? 1024 : 768) || (M > 16 && N > 16384)) return false;
+    if (K < 896) return !(N < 1152 && (M <= 32 || M > 64));
+    return !(M > 64 && K >= 1024 && K < (M > 96 ? 1408 : 1280) && N < (K < 1152 ? 1024 : 640));
 }
 
 // Kernel family forced by the test hook (-1 = choose by shape).  Process-wide and only meant for tests and benchmarks:
@@ -1955,37 +1527,21 @@ std::atomic<int> g_force_cfg{-1};
 // epilogue_alignment has it.
 int choose_cfg(int64_t M, int64_t N, int64_t K, bool whole, bool aligned) {
     const int force = g_force_cfg.load(std::memory_order_relaxed);
-    const bool dma_ok = M * K < ((int64_t)1 << 32) && N * K < ((int64_t)1 << 32);   // 32-bit lane offsets
-    if (force == 5) return dma_ok && whole && (K % 128) == 0 && M <= 128 ? 5 : 1;
-    if (force == 6 || force == 7 || force == 9) return (dma_ok && (K % 128) == 0) ? force : 1;
+    const bool tiles_ok = M * K < ((int64_t)1 << 32) && N * K < ((int64_t)1 << 32) && (K % 128) == 0;   // 32-bit lane offsets, whole steps
+    if (force == 5) return tiles_ok && whole && M <= 128 ? 5 : 1;
+    if (force == 7 || force == 9) return tiles_ok ? force : 1;
     if (force == 1 || force == 2) return force;
-    // Up to 128 rows: from K = 768 on (1024 for the most rows), except where rows_kernel_loses, and up
-    // to the 16384 columns that give every CU one workgroup of the tallest split.  Beyond those the streaming kernel's 96-wide
-    // tiles fill the CUs as well and its W rows come in whole lines (4096 -> 24576, us, this and that: 1 row 29.1 and 30.6, 32 rows
-    // 35.3 and 30.6, 128 rows 42.8 and 31.5; 3072 -> 18432, 16 rows 18.0 and 21.1).
-    if (M <= 128 && (K % 128) == 0 && K >= (M > 96 ? 1024 : 768) && dma_ok && whole && (M <= 16 || N <= 16384) &&
-        !rows_kernel_loses(M, N, K, aligned)) return 5;
-    if (M <= 256 && N >= 1024 && (K % 128) == 0 && K >= 512 && dma_ok) {
-        // The weight-streaming kernel pays a fixed price per call (a prologue that waits for HBM, two launches when K
-        // is split), which long K repays and short K does not.  Measured with weights from HBM, M = 16..256, K =
-        // 1024..12288, N = 1024..24576: it wins from K = 3072 on at M > 128 and from K = 1536 on below; under that the
-        // 128 x 192 ring tiles win for M > 128 (all N at K >= 1536, N >= 8192 below) and the small register-staged
-        // tiles for the rest.
-        if (K >= (M > 128 ? 3072 : 1536)) return 6;
-        if (M > 128 && (K >= 1536 || N >= 8192)) return 7;
-        return 2;
-    }
-    // Everything below was chosen from measured grids of shapes (weights from HBM, every family forced in turn).  A
-    // round of 128 x 192 ring tiles costs about two thirds of a round of 256 x 256 two-group tiles, so the large tiles
-    // win as soon as the small ones need a second round, i.e. more than one per CU.
+    if (tiles_ok && whole && M <= 128 && rows_kernel_wins(M, N, K, aligned)) return 5;
+    const int cus = device_cu_count();
+    // one or two steps of K and little to store: 512 threads and 96 KB of LDS to start cost more than they give (500 shapes, register-
+    // staged tiles over fetching waves: K = 128 0.93 to 1.0, K = 256 0.94 to 1.0, K = 384 0.97 to 1.1; K = 256 with 1 << 21 outputs 1.1)
+    const bool tiny = K <= 256 && M * N <= 1 << 19;
+    if (tiles_ok && aligned && !tiny) return M >= 512 && N >= 512 && pp_us(M, N, K, cus) < fed_plan(M, N, K, cus, true).us ? 9 : 7;
+    // the register-staged tiles: large ones as soon as there is work for them
+    if (M <= 256 && N >= 1024 && tiles_ok && K >= 512) return K >= 1536 || (M > 128 && N >= 8192) ? 1 : 2;
     const int64_t tiles_s = ((M + 127) / 128) * ((N + 191) / 192);
-    if (M >= 512 && N >= 512 && tiles_s > device_cu_count()) return (dma_ok && (K % 128) == 0) ? 9 : 1;
-    if (dma_ok && (K % 128) == 0) {
-        // a few hundred rows, long K, few columns: the ring tiles leave most CUs idle, the weight-streaming kernel splits
-        // K over them (not for the entry point that may not allocate: its planes are sized for 256 rows)
-        if (M <= 512 && N >= 1024 && K >= 8192 && tiles_s <= 96 && tl_scratch == nullptr) return 6;
-        if (M > 128 && N >= 192 && (tiles_s >= 96 || (tiles_s >= 40 && K >= 2048))) return 7;
-    }
+    if (M >= 512 && N >= 512 && tiles_s > cus) return 1;
+    if (tiles_ok && M > 128 && N >= 192 && (tiles_s >= 96 || (tiles_s >= 40 && K >= 2048) || (M <= 512 && N >= 1024 && K >= 8192))) return 1;
     const int64_t tiles_m = ((M + 127) / 128) * ((N + 127) / 128);
     if (M > 64 && N > 64 && tiles_m >= 256) return 1;
     return 2;
@@ -1997,8 +1553,7 @@ int dispatch_cfg(const GemmArgs& a, hipStream_t st) {
     epilogue_alignment<OUT_DT, EPI>(a, vec_ok, aligned);
     switch (choose_cfg(a.M, a.N, a.K, (((uintptr_t)a.A | (uintptr_t)a.W) & 15) == 0, aligned)) {
         case 5: return launch_rows<OUT_DT, EPI>(a, st);
-        case 6: return launch_skinny<OUT_DT, EPI>(a, st);
-        case 7: return launch_ring_small<OUT_DT, EPI>(a, st);
+        case 7: return launch_fed<OUT_DT, EPI>(a, st);
         case 9: return launch_pp<OUT_DT, EPI>(a, st);
         case 1: return launch_cfg<CfgM, OUT_DT, EPI>(a, st);
         default: return launch_cfg<CfgS, OUT_DT, EPI>(a, st);
@@ -2198,8 +1753,8 @@ GPU_API int gpu_int8_gemm_acc(const int8_t* A, const int8_t* W, int32_t* acc, in
     return rc < 0 ? -200 : rc;
 }
 
-// Test hook: force a kernel family (1 = 128x128, 2 = 64x64 register-staged tiles; 5 = up to 128 rows; 6 = weight streaming; 7 = persistent
-// ring, 128x192; 9 = two-group kernel; -1 or anything else = automatic).
+// Test hook: force a kernel family (1 = 128x128, 2 = 64x64 register-staged tiles; 5 = up to 128 rows; 7 = waves that
+// fetch for others; 9 = two-group kernel; -1 or anything else = automatic).
 GPU_API int gpu_int8_gemm_force_config(int cfg) {
     g_force_cfg.store(cfg, std::memory_order_relaxed);
     return 0;

@@ -304,11 +304,9 @@ int gpu_w6a8_group_gemm_ws(const int8_t* A, const void* Wp, const float* xs, con
 int64_t gpu_w6a8_group_gemm_scratch(const void* Wp, int64_t M, int64_t N, int64_t K);
 
 /* Test and tuning hook: force the GEMM kernel family.  1, 2 = 128x128 and 64x64 register-staged tiles; 5 = weights straight
- * into registers, for M <= 128; 6 =
- * weight-streaming kernel (256x96 tiles, two groups of waves taking turns on the K tiles, split K when N is small) for
- * M <= 256; 7 = four-wave persistent ring kernel on
- * 128x192 tiles (shapes with few tiles); 9 = two-group kernel (256x256 and 128x256 tiles, one launch), the choice for
- * large shapes; -1 = automatic.  A shape a family cannot run falls back to 1. */
+ * into registers, for M <= 128; 7 = four waves multiply what four others fetch, 128x64 to 128x192 tiles, K split where they are few;
+ * 9 = two-group kernel (256x256 and 128x256 tiles, one launch), the choice for large shapes; anything else = automatic.  A shape
+ * a family cannot run falls back to 1. */
 int gpu_int8_gemm_force_config(int cfg);
 
 /* Writes, for each of the 64 lanes and 16 accumulator registers of one v_mfma_i32_32x32x32_i8, the (row of src0,

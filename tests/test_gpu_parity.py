@@ -900,6 +900,39 @@ def test_int8_gemm_up_to_128_rows(M, N, K):
             ffi.raw("gpu_int8_gemm_force_config", -1)
 
 
+# Edges of the kernel with fetching waves: fewer steps of K than LDS stages, an odd and an even number of them, its three widths with a
+# last tile of 1, 8 or all columns and of 1, 127 or all rows, several rounds of tiles, K in equal slices and with a shorter last one
+FED_CASES = [(1, 64, 128), (128, 65, 256), (129, 136, 384), (300, 1000, 512), (255, 3008, 640), (2048, 640, 2560), (1025, 192, 896), (3000, 5000, 128), (640, 1281, 1152), (256, 1000, 3712), (200, 2048, 4096),
+             (77, 1030, 5120), (400, 136, 6016)]
+
+
+@pytest.mark.parametrize("M,N,K", FED_CASES)
+def test_int8_gemm_with_fetching_waves(M, N, K):
+    say("gemm fetching waves", M, N, K)
+    A, W = rand_i8(15, 500 + M, M, K), rand_i8(15, 600 + N, N, K)
+    A[0, :] = -128
+    W[N - 1, :] = -128
+    xs, ws = synth.uniform(15, 3, M, 0.005, 0.2), synth.uniform(15, 4, N, 1e-3, 1e-2)
+    want = oracle.int8_gemm_acc(A, W)
+    Ad, Wd, xd, wd = dev(A), dev(W), dev(xs), dev(ws)
+    for dt, tob in ((BF16, oracle.bf16_bits), (F16, oracle.f16_bits), (F32, lambda a: a.astype(np.float32))):
+        bias, rs = tob(synth.normal(15, 5, N) * np.float32(0.02)), tob(synth.normal(15, 6, N))
+        resid = tob(synth.normal(15, 7, M * N).reshape(M, N))
+        wz = [oracle.epilogue(want, xs, ws, b, dt, fma=1) for b in (None, bias)]
+        wr = oracle.epilogue_residual(want, xs, ws, bias, rs, resid, dt, fma=1)
+        for cfg in (7, -1):
+            ffi.raw("gpu_int8_gemm_force_config", cfg)
+            try:
+                assert np.array_equal(ql.int8_gemm_acc(Ad, Wd).cpu().numpy(), want), cfg
+                for b, w in zip((None, bias), wz):
+                    d = ql.int8_gemm(Ad, Wd, xd, wd, None if b is None else dev_bits(b, dt), TDT[dt])
+                    assert np.array_equal(host_bits(d), w), (cfg, dt)
+                r = ql.int8_gemm_residual(Ad, Wd, xd, wd, dev_bits(bias, dt), dev_bits(rs, dt), dev_bits(resid, dt))
+                assert np.array_equal(host_bits(r), wr), (cfg, dt)
+            finally:
+                ffi.raw("gpu_int8_gemm_force_config", -1)
+
+
 # K % 16 == 8: the reference's alignment-8 configurations (csrc/vendor/cutlass_gemm_int8.cu:191,237-247)
 @pytest.mark.parametrize("M,N,K", [(5, 40, 8), (130, 264, 136), (300, 1030, 1000), (64, 2048, 4104)])
 def test_int8_gemm_k_multiple_of_8_only(M, N, K):
