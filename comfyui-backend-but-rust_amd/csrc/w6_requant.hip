@@ -2,17 +2,20 @@
 // (nibble plane, then 2-bit plane), one fp8-e4m3 relative scale per 32 columns, one fp32 scale per row.  Replaces
 // gpu_w6_requant, csrc/vendor/w6a8_requant.cu: same float expressions (cited by line), bit for bit.
 //
-// A load-time / LoRA-bake kernel: 2 B read + 0.78 B written per weight, bound by its vector instructions.  A wave owns
-// chunks of 1024 values, 16 consecutive ones per lane, and keeps them in registers from the load to the packed stores: a
-// scale group is two neighbouring lanes, a row up to 16 waves that exchange one maximum.  (One thread per group over a row
-// in LDS, as the reference has it, leaves a third of the lanes idle and reads LDS at a stride of 32 words: 5376 x 5376
-// measured 170 us that way, 71 us like this; the copy rate of the part allows 16 us.)
+// A load-time / LoRA-bake kernel: 2 B read + 0.78 B written per weight, bound by its vector instructions (about 4000 cycles
+// of them per 1024 values).  A wave owns chunks of 1024 values, 16 consecutive ones per lane, and keeps them in registers from
+// the load to the packed stores: a scale group is two neighbouring lanes, a rotation group sixteen.  A workgroup takes as many
+// rows as fill its waves best and cuts them into chunks as if they were one, so only its last wave can have idle lanes; the rows'
+// maxima meet in LDS.  5376 x 5376, whole rows to a workgroup, the sixth
+// wave a quarter full: 69.4 us; three rows on 16 waves: 56.4.  (One thread per group over a row in LDS, as the reference has it, leaves a third of the lanes
+// idle and reads LDS at a stride of 32 words: 170 us; the copy rate of the part allows 16 us.)
 #include "common.hpp"
 #include "convrot.hpp"
 
 namespace {
 
 constexpr int kG = 32;   // columns per relative scale
+constexpr int kMaxRows = 16;   // rows of a workgroup
 
 // float -> fp8 e4m3 bits, round to nearest even, saturating at 448 (finite inputs)
 __device__ __forceinline__ uint32_t f_to_e4m3(float x) {
@@ -80,24 +83,37 @@ __device__ __forceinline__ uint32_t codes4(const float* v, float inv_sc, float s
     return out;
 }
 
-// wpr waves per row (chunks wr, wr + wpr, ...), rpb rows per workgroup.
+// The maximum over the 16 lanes of a rotation group, in all of them.
+__device__ __forceinline__ float group_max(float x) {
+    const auto step = [&](auto ctrl) {
+        x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, false)));
+    };
+    step(std::integral_constant<int, 0xB1>{});    // lane ^ 1
+    step(std::integral_constant<int, 0x4E>{});    // lane ^ 2
+    step(std::integral_constant<int, 0x141>{});   // the other half of eight
+    step(std::integral_constant<int, 0x140>{});   // the other half of sixteen
+    return x;
+}
+
+// rpb rows per workgroup, `groups` = K / 256 rotation groups each; wave w takes the chunks w, w + waves, ... of all of them.
+// group / `groups` is (group * inv_groups) >> 16.
 template <int C>
 __global__ void __launch_bounds__(1024) w6_requant_kernel(const uint16_t* w, uint8_t* packed, uint8_t* s_rel, float* s_channel, int N, int K,
-                                                         uint64_t seed, int wpr, int rpb) {
+                                                         uint64_t seed, int groups, uint32_t inv_groups, int rpb) {
     extern __shared__ __attribute__((aligned(16))) float tiles[];   // a rotation tile per wave
-    __shared__ float red[16];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int rloc = wave / wpr, wr = wave - rloc * wpr;
-    const int64_t n = (int64_t)blockIdx.x * rpb + rloc;
-    const bool row_ok = n < N;
+    __shared__ uint32_t row_max[kMaxRows];                          // the bits of a maximum that is never negative
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const int64_t n0 = (int64_t)blockIdx.x * rpb;
+    const int ngroups = (N - n0 < rpb ? (int)(N - n0) : rpb) * groups;
     float v[C][16], gs[C], gmax[C];
-    float amax = 0.f;
+    if (threadIdx.x < kMaxRows) row_max[threadIdx.x] = 0u;
+    __syncthreads();
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-        const int e0 = (wr + c * wpr) * convrot::kChunk + lane * 16;
-        const bool act = row_ok && e0 < K;              // K % 256 == 0: a lane's 16 values are all in or all out
+        const int chunk = wave + c * nw, group = chunk * 4 + (lane >> 4);
+        const bool act = group < ngroups;               // a lane's 16 values are all in or all out
         if (act) {
-            const uint4* src = reinterpret_cast<const uint4*>(w + n * K + e0);
+            const uint4* src = reinterpret_cast<const uint4*>(w + n0 * K + chunk * convrot::kChunk + lane * 16);
             const uint4 a = src[0], b = src[1];
             const uint32_t ww[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
@@ -150,20 +166,12 @@ __global__ void __launch_bounds__(1024) w6_requant_kernel(const uint16_t* w, uin
         }
         // the group's largest decoded magnitude, :118-119: products and roundings are monotonic, so it is the largest
         // value's (a NaN takes -31 in the reference's clamp)
-        amax = fmaxf(amax, (nan ? 31.0f : fminf(31.0f, __builtin_rintf(m * inv))) * step);
+        const float amax = group_max(fmaxf(0.f, (nan ? 31.0f : fminf(31.0f, __builtin_rintf(m * inv))) * step));   // 0 * inf counts for nothing
+        if (act && (lane & 15) == 0) atomicMax(row_max + (group * inv_groups >> 16), f2u(amax));
         gs[c] = step;
         gmax[c] = nan ? __builtin_inff() : m;   // a group with a NaN is not for the plain form of codes4
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
-    if (wpr > 1) {   // uniform over the workgroup
-        if (lane == 0) red[wave] = amax;
-        __syncthreads();
-        amax = 0.f;
-        for (int i = 0; i < wpr; ++i) amax = fmaxf(amax, red[rloc * wpr + i]);
-    }
-    const float sc = fmaxf(amax / 127.0f, 1e-8f), inv_sc = 1.0f / sc;               // :121
-    if (row_ok && wr == 0 && lane == 0) s_channel[n] = sc;
+    __syncthreads();
 
     // The hash multiplies index ^ seed; a lane's first index is a multiple of 16, so the product splits into one for the
     // upper 28 bits and one for the four low bits, which is the same in all lanes.
@@ -173,8 +181,12 @@ __global__ void __launch_bounds__(1024) w6_requant_kernel(const uint16_t* w, uin
     for (int i = 0; i < 16; ++i) kc[i] = ((s32 ^ (uint32_t)i) & 15u) * 747796405u + 2891336453u;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-        const int e0 = (wr + c * wpr) * convrot::kChunk + lane * 16;
-        if (!(row_ok && e0 < K)) continue;
+        const int group = (wave + c * nw) * 4 + (lane >> 4);
+        if (group >= ngroups) continue;
+        const int row = (int)(group * inv_groups >> 16), e0 = (group - row * groups) * 256 + (lane & 15) * 16;
+        const int64_t n = n0 + row;
+        const float sc = fmaxf(u2f(row_max[row]) / 127.0f, 1e-8f), inv_sc = 1.0f / sc;   // :121
+        if (e0 == 0) s_channel[n] = sc;
         const uint32_t bits = f_to_e4m3(gs[c] / sc);                                // :126-151
         if (!(lane & 1)) s_rel[n * (K / kG) + e0 / kG] = (uint8_t)bits;
         const float sr = e4m3_to_f(bits), inv_sr = 1.0f / fmaxf(sr, 1e-30f);
@@ -218,15 +230,28 @@ __global__ void __launch_bounds__(1024) w6_requant_kernel(const uint16_t* w, uin
     }
 }
 
+// Rows of a workgroup: one, or as many more as give the CUs clearly fewer waves to run: all of a workgroup's, however few lanes its
+// last has, times the workgroups of the busiest CU.  us, one row and the rows chosen: 5376 x 5376 66.6 and 56.4 (three), 4096 x 1280
+// 20.3 and 15.9 (four), 8192 x 256 19.4 and 10.9 (four), 4096 x 1536 19.1 and 16.5 (two); within 6 % the larger workgroups
+// lose by their barriers (4096 x 7680 59.7 and, two rows in 15 waves, 64.3).
+int rows_per_group(int64_t N, int groups) {
+    const int cus = device_cu_count();
+    const auto waves = [&](int r) { return (double)(((N + r - 1) / r + cus - 1) / cus) * ((r * groups + 3) / 4); };
+    int best = 1;
+    for (int r = 2; r <= kMaxRows && r * groups <= 64; ++r)
+        if (waves(r) < 0.92 * waves(best)) best = r;
+    return best;
+}
+
 template <int C>
-int launch_requant(const void* w, void* packed, void* s_rel, void* s_channel, int N, int K, uint64_t seed, int wpr, hipStream_t st) {
-    const int rpb = wpr >= 4 ? 1 : 4 / wpr, nw = wpr * rpb;
+int launch_requant(const void* w, void* packed, void* s_rel, void* s_channel, int N, int K, uint64_t seed, int rpb, hipStream_t st) {
+    const int groups = K / 256, chunks = (rpb * groups + 3) / 4, nw = (chunks + C - 1) / C;
     const int smem = nw * convrot::kLdsPerWave * (int)sizeof(float);
     static PerDeviceOnce once;
     if (smem > 64 * 1024)
         if (const int e = allow_dynamic_lds((const void*)w6_requant_kernel<C>, 16 * convrot::kLdsPerWave * (int)sizeof(float), once)) return e;
     hipLaunchKernelGGL(w6_requant_kernel<C>, dim3((unsigned)((N + rpb - 1) / rpb)), dim3(nw * 64), smem, st, (const uint16_t*)w,
-                       (uint8_t*)packed, (uint8_t*)s_rel, (float*)s_channel, N, K, seed, wpr, rpb);
+                       (uint8_t*)packed, (uint8_t*)s_rel, (float*)s_channel, N, K, seed, groups, (65536u + groups - 1) / groups, rpb);
     KCHECK();
     return 0;
 }
@@ -241,9 +266,9 @@ GPU_API int gpu_w6_requant(const void* weight, void* packed, void* s_rel, void* 
     if (K > 39680 || N > 0x7fffffff) return -2;
     if (N <= 0) return 0;
     // a chunk per wave up to 16 waves per row; longer rows give a wave two or three
-    const int chunks = (K + convrot::kChunk - 1) / convrot::kChunk;
+    const int groups = K / 256, chunks = (groups + 3) / 4;
     hipStream_t st = (hipStream_t)stream;
-    if (chunks <= 16) return launch_requant<1>(weight, packed, s_rel, s_channel, (int)N, K, seed, chunks, st);
-    if (chunks <= 32) return launch_requant<2>(weight, packed, s_rel, s_channel, (int)N, K, seed, (chunks + 1) / 2, st);
-    return launch_requant<3>(weight, packed, s_rel, s_channel, (int)N, K, seed, (chunks + 2) / 3, st);
+    if (chunks > 32) return launch_requant<3>(weight, packed, s_rel, s_channel, (int)N, K, seed, 1, st);
+    if (chunks > 16) return launch_requant<2>(weight, packed, s_rel, s_channel, (int)N, K, seed, 1, st);
+    return launch_requant<1>(weight, packed, s_rel, s_channel, (int)N, K, seed, rows_per_group(N, groups), st);
 }

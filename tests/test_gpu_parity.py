@@ -616,6 +616,28 @@ def test_w6_requant_zero_blocks_and_small_groups(N, K):
         assert np.array_equal(pd.cpu().numpy(), packed)
 
 
+@pytest.mark.parametrize("N,K", [(1030, 256), (1301, 768), (1101, 1280), (700, 5376)])
+def test_w6_requant_several_rows_per_workgroup(N, K):
+    """Enough rows that a workgroup takes several, in chunks across their ends, with a last workgroup of fewer: rows of very different
+    scales, of zeros and with a NaN or an infinity next to one another."""
+    w = synth.normal(93 + K, 1, N * K).reshape(N, K) * np.float32(0.04)
+    w *= np.float32(2.0) ** (np.arange(N) % 7 - 3).astype(np.float32)[:, None]
+    w[4::11] = 0
+    w[6, 3], w[7, K - 1] = np.nan, np.inf
+    w[N - 1, :16] = np.float32(3.0)
+    wb = synth.bf16_bits(w)
+    for seed in (0, 2 ** 40 + 3):
+        say("w6_requant rows", N, K, seed)
+        with np.errstate(all="ignore"):
+            rc, packed, s_rel, s_ch = oracle.w6_requant(wb, seed)
+        pd, rd, cd = ql.w6_requant(dev_bits(wb, BF16), seed)
+        torch.cuda.synchronize()
+        assert rc == 0
+        assert np.array_equal(cd.cpu().numpy().view(np.uint32), s_ch.view(np.uint32))
+        assert np.array_equal(rd.cpu().numpy(), s_rel)
+        assert np.array_equal(pd.cpu().numpy(), packed)
+
+
 @pytest.mark.parametrize("N,K", [(6, 512), (7, 1280)])
 def test_w6_requant_not_finite(N, K):
     """NaN, infinities of one and of both signs, and finite weights whose rotation or step overflows, beside ordinary rows."""
