@@ -46,15 +46,13 @@ enum { PRO_SD_GEGLU = 101, PRO_SD_UNPAD = 102, PRO_SD_GN = 103 };
 
 // csrc/kernels.cu:1355-1359
 constexpr uint32_t kPcgMul = 747796405u, kPcgAdd = 2891336453u;
-__device__ __forceinline__ uint32_t pcg_hash_state(uint32_t state) {   // state: x * kPcgMul + kPcgAdd
+// The hash's upper 24 bits in place, as a float: 2^32 times the noise in [0, 1).  In place they take one three-operand bit operation
+// where a shift down to whole numbers takes a second instruction, and the power of two rides in the addition that follows
+// (12288 x 3072 bf16 39.7 -> 37.4 us).
+__device__ __forceinline__ float pcg_noise_state(uint32_t state) {   // state: x * kPcgMul + kPcgAdd
     const uint32_t word = ((state >> ((state >> 28u) + 4u)) ^ state) * 277803737u;
-    return (word >> 22u) ^ word;
+    return (float)(((word >> 22u) ^ word) & 0xffffff00u);
 }
-// a + b of two bf16 values rounded once to bf16, what the bf16 add instruction behind __hadd gives (csrc/kernels.cu:1341-1343).
-// The fp32 sum rounds first and changes nothing: it is inexact only where the smaller operand is below 2^-15 of the larger,
-// which leaves the sum 2^-10 (relative) or more away from every midpoint of two bf16 values.
-__device__ __forceinline__ float bf16_add_once(float a, float b) { return rnd_dt<DT_BF16>(a + b); }
-
 template <int MODE> __device__ __forceinline__ void load16(const void* x, int64_t off, float* v) {
     if (MODE == MODE_BF16) {
         const uint4* p = reinterpret_cast<const uint4*>((const uint16_t*)x + off);
@@ -161,8 +159,8 @@ __device__ __forceinline__ void store_codes(const QuantArgs& p, float (&v)[C][16
 
     // Stochastic rounding: the hash of element index + seed, its halves folded, starts with a product.  Where a row's keys stay
     // below 2^32 the fold changes nothing and a lane's 16 products differ by constants.  With that, the fp32 addition above
-    // (fp64 and 64-bit integers before) and the clamp in the pack conversion 12288 x 3072 bf16 takes 42 us instead of 53 (45
-    // where the keys pass 2^32), bound by vector instructions: the same rows rounded to nearest take 28 to 32.
+    // (fp64 and 64-bit integers before) and the clamp in the pack conversion 12288 x 3072 bf16 took 42 us instead of 53 (45
+    // where the keys pass 2^32), now 37, bound by vector instructions: the same rows rounded to nearest take 26.
     const uint64_t key0 = (uint64_t)(m * (int64_t)p.K) + p.seed;
     const auto store = [&](auto fast_tag) {
 #pragma unroll
@@ -220,8 +218,12 @@ __device__ __forceinline__ void store_codes(const QuantArgs& p, float (&v)[C][16
                             const uint64_t key = key0 + e0 + 4 * i + j;
                             state = ((uint32_t)key ^ (uint32_t)(key >> 32)) * kPcgMul + kPcgAdd;
                         }
-                        const float noise = (float)(pcg_hash_state(state) >> 8) * 0x1.0p-24f;
-                        const float r = floorf(MODE == MODE_F32 ? t + noise : bf16_add_once(t, rnd_dt<DT_BF16>(noise)));
+                        // bf16: t plus the rounded noise, rounded once to bf16 as __hadd's instruction does (csrc/kernels.cu:1341-1343).
+                        // The fp32 sum rounds first and changes nothing: it is inexact only where the smaller operand is below
+                        // 2^-15 of the larger, which leaves the sum 2^-10 (relative) or more away from every midpoint of two bf16 values.
+                        const float noise = pcg_noise_state(state);
+                        const float r = floorf(MODE == MODE_F32 ? __builtin_fmaf(noise, 0x1.0p-32f, t)
+                                                                : rnd_dt<DT_BF16>(__builtin_fmaf(rnd_dt<DT_BF16>(noise), 0x1.0p-32f, t)));
                         acc = __builtin_amdgcn_cvt_pk_u8_f32(r + 128.f, j, acc);   // the clamp as below; r is a whole number
                     } else if (MODE == MODE_F32) {
                         const int qi = (int)fminf(127.f, fmaxf(-128.f, nearbyintf(t)));

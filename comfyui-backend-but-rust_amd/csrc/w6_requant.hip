@@ -7,8 +7,8 @@
 // the load to the packed stores: a scale group is two neighbouring lanes, a rotation group sixteen.  A workgroup takes as many
 // rows as fill its waves best and cuts them into chunks as if they were one, so only its last wave can have idle lanes; the rows'
 // maxima meet in LDS.  5376 x 5376, whole rows to a workgroup, the sixth
-// wave a quarter full: 69.4 us; three rows on 16 waves: 56.4.  (One thread per group over a row in LDS, as the reference has it, leaves a third of the lanes
-// idle and reads LDS at a stride of 32 words: 170 us; the copy rate of the part allows 16 us.)
+// wave a quarter full: 69.4 us; three rows on 16 waves: 55.  (One thread per group over a row in LDS, as the reference has it,
+// leaves a third of the lanes idle and reads LDS at a stride of 32 words: 170 us; the copy rate of the part allows 16 us.)
 #include "common.hpp"
 #include "convrot.hpp"
 
@@ -75,7 +75,7 @@ __device__ __forceinline__ uint32_t codes4(const float* v, float inv_sc, float s
         lg = PLAIN ? __builtin_fmaf(g, s, M) - M : level(g, s);
         const uint32_t h = x0 + kc[j];                                            // x * 747796405 + 2891336453, :21-25
         const uint32_t w = ((h >> ((h >> 28u) + 4u)) ^ h) * 277803737u;
-        const float u = (float)(((w >> 22u) ^ w) >> 8) * (1.0f / 16777216.0f);    // :27-31
+        const float u = (float)(((w >> 22u) ^ w) & 0xffffff00u) * 0x1.0p-32f;     // :27-31, the 24 bits left where they are
         const float thr = __builtin_fmaf(u, fabsf(lg - lf), fminf(lf, lg));
         const float half = PLAIN ? __builtin_copysignf(0.5f, thr - t) : t > thr ? -0.5f : 0.5f;   // negative where t is above the threshold
         out = __builtin_amdgcn_cvt_pk_u8_f32(fminf(f, g) - half + 32.25f, j, out);
