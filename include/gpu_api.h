@@ -258,7 +258,7 @@ int gpu_int8_gemm_acc(const int8_t* A, const int8_t* W, int32_t* acc, int64_t M,
  * is written before it is read).  The first call on a device looks up the array's address and sets kernel attributes:
  * make it once before capturing a graph that contains this call.  The array occupies its 24 MiB on every device the
  * process uses, from the moment the library is loaded.  A shape whose planes would not fit returns -210 with a message on
- * stderr (every shape the automatic choice splits fits; with gpu_int8_gemm_force_config(6), M > 256 can exceed it);
+ * stderr (every shape that is split fits);
  * gpu_int8_gemm_static_limit() returns the array's size in bytes.  K % 16 == 8, which gpu_int8_gemm serves from
  * padded copies that it allocates, is refused here (-200).  Other return codes as gpu_int8_gemm. */
 int gpu_int8_gemm_static(const int8_t* A, const int8_t* W, const float* xs, const float* ws, const void* bias, void* D,
