@@ -8,9 +8,9 @@
 // stores 8-byte (bf16/f16) or 16-byte (f32) vectors straight from the accumulators.
 #include <atomic>
 #include <cstdio>
-#include <mutex>
 
 #include "common.hpp"
+#include "kept_buffers.hpp"
 
 // Nothing is scheduled across this point: it pins hand-interleaved instruction orders and keeps live ranges short.
 #define SCHED_FENCE() __builtin_amdgcn_sched_barrier(0)
@@ -1272,21 +1272,18 @@ void retain_pool_memory() {
 }
 
 // Split-K planes of the allocating entry points: one buffer per (device, stream), made on that stream's first split
-// call and kept until the process ends.  Work on one stream is ordered, so its calls can share a buffer, and a
-// stream-ordered allocation per call costs about 7 us on the stream's timeline (measured: 31 against 24 us per call at
+// call and kept until the process ends.  Work on one stream is ordered, so its calls can share a buffer (kept_buffers.hpp: also
+// those of several host threads, since a call queues both its launches under the buffer's lock), and a stream-ordered
+// allocation per call costs about 7 us on the stream's timeline (measured: 31 against 24 us per call at
 // M=256, K=12288, N=4096).  The buffer has the one size every shape that the dispatcher splits fits into (slices * tiles <= CUs, and
 // no tile of int32 is larger than 128 x 192: 24 MiB on 256 CUs) and is never grown or
-// freed, so a captured graph that holds its address stays valid.  At most kStreamPlanes streams per process are served;
+// freed, so a captured graph that holds its address stays valid.  At most eight streams per process are served;
 // a call on any further stream, a first call made under capture, or a shape beyond the size (a forced configuration)
 // falls back to a stream-ordered allocation, and so does hipStreamPerThread (one handle for a different stream in every
 // thread).  A stream handle that the runtime reuses after hipStreamDestroy inherits
 // the destroyed stream's buffer; work still queued on the destroyed stream at that moment would share it.
 constexpr size_t kPlanesPerCu = 128 * 192 * sizeof(int);
-struct StreamPlanes { int dev; hipStream_t st; void* ptr; size_t bytes; };
-constexpr int kStreamPlanes = 8;
-std::mutex g_planes_mu;
-StreamPlanes g_planes[kStreamPlanes];
-int g_planes_n = 0;
+KeptBuffers<8> g_planes;
 
 bool is_capturing(hipStream_t st) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -1295,65 +1292,48 @@ bool is_capturing(hipStream_t st) {
     return true;   // not known: taken as one
 }
 
-void* stream_planes(hipStream_t st, size_t need, int num_cu) {
-    if (st == hipStreamPerThread) return nullptr;   // one handle, a different stream in every thread: nothing to key on
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-    std::lock_guard<std::mutex> lock(g_planes_mu);
-    for (int i = 0; i < g_planes_n; ++i)
-        if (g_planes[i].dev == dev && g_planes[i].st == st) return need <= g_planes[i].bytes ? g_planes[i].ptr : nullptr;
-    const size_t bytes = (size_t)num_cu * kPlanesPerCu;
-    if (g_planes_n == kStreamPlanes || need > bytes) return nullptr;
-    if (is_capturing(st)) return nullptr;
-    void* ptr = nullptr;
-    if (hipMalloc(&ptr, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    g_planes[g_planes_n++] = StreamPlanes{dev, st, ptr, bytes};
-    return ptr;
-}
-
 // A run on `slices` slices of kslice values of K: `body` writes the int32 planes, a second kernel adds them (exact, so the order of
 // the sum does not matter) and applies the epilogue.
 template <int OUT_DT, int EPI, class Body>
 int launch_split(const GemmArgs& a, int slices, int kslice, hipStream_t st, Body body) {
-    const int num_cu = device_cu_count();
     const size_t need = (size_t)slices * a.M * a.N * sizeof(int);
-    int* planes = nullptr;
-    bool own = false;   // planes come from the stream-ordered pool and go back to it
-    if (tl_scratch == nullptr) {
-        planes = (int*)stream_planes(st, need, num_cu);
-        if (!planes) {
-            own = true;
-            retain_pool_memory();
-            hipError_t e = hipMallocAsync((void**)&planes, need, st);
-            if (e != hipSuccess) return (int)e;
-        }
-    } else {
+    const auto queue = [&](void* planes) -> int {   // every plane element is written before it is read: nothing to clear
+        GemmArgs pa = a;
+        pa.D = planes;
+        pa.kslice = kslice;
+        if (const int rc = body(pa)) return rc;
+        const int64_t nvec = (int64_t)a.M * a.N / 4;
+        const unsigned grid = (unsigned)((nvec + 255) / 256 < 4096 ? (nvec + 255) / 256 : 4096);
+        hipLaunchKernelGGL((splitk_epilogue_kernel<OUT_DT, EPI>), dim3(grid), dim3(256), 0, st, a, (const int*)planes, slices);
+        return (int)hipGetLastError();
+    };
+    if (tl_scratch != nullptr) {
         if (need > tl_scratch_bytes) {
             fprintf(stderr, "gpu_int8_gemm_static: M=%d N=%d K=%d needs %zu bytes of split-K scratch, the static buffer has %zu\n",
                     a.M, a.N, a.K, need, tl_scratch_bytes);
             return -210;
         }
-        planes = (int*)tl_scratch;   // every plane element is written before it is read: nothing to clear
+        return queue(tl_scratch);
     }
-    GemmArgs pa = a;
-    pa.D = planes;
-    pa.kslice = kslice;
-    int rc = body(pa);
-    if (rc == 0) {
-        const int64_t nvec = (int64_t)a.M * a.N / 4;
-        const unsigned grid = (unsigned)((nvec + 255) / 256 < 4096 ? (nvec + 255) / 256 : 4096);
-        hipLaunchKernelGGL((splitk_epilogue_kernel<OUT_DT, EPI>), dim3(grid), dim3(256), 0, st, a, (const int*)planes, slices);
-        hipError_t le = hipGetLastError();
-        if (le != hipSuccess) rc = (int)le;
-    }
-    if (own) {
-        hipError_t e = hipFreeAsync(planes, st);
-        if (rc == 0 && e != hipSuccess) rc = (int)e;
-    }
-    return rc;
+    int rc = 0, dev = 0;
+    const auto make = [&](size_t bytes) -> void* {
+        void* ptr = nullptr;
+        if (is_capturing(st)) return nullptr;
+        if (hipMalloc(&ptr, bytes) == hipSuccess) return ptr;
+        (void)hipGetLastError();
+        return nullptr;
+    };
+    // hipStreamPerThread: one handle, a different stream in every thread: nothing to key on
+    if (st != hipStreamPerThread && hipGetDevice(&dev) == hipSuccess &&
+        g_planes.with(dev, st, need, (size_t)device_cu_count() * kPlanesPerCu, make, [&](void* planes) { rc = queue(planes); }))
+        return rc;
+    void* planes = nullptr;   // from the stream-ordered pool, and back to it
+    retain_pool_memory();
+    hipError_t e = hipMallocAsync(&planes, need, st);
+    if (e != hipSuccess) return (int)e;
+    rc = queue(planes);
+    e = hipFreeAsync(planes, st);
+    return rc == 0 ? (int)e : rc;
 }
 
 template <class C, int OUT_DT, int EPI>

@@ -7,6 +7,7 @@ import ctypes as C
 import hashlib
 import json
 import os
+import threading
 
 import numpy as np
 import pytest
@@ -953,6 +954,39 @@ def test_int8_gemm_with_fetching_waves(M, N, K):
                 assert np.array_equal(host_bits(r), wr), (cfg, dt)
             finally:
                 ffi.raw("gpu_int8_gemm_force_config", -1)
+
+
+def test_split_k_calls_of_two_threads_on_one_stream():
+    """Both launches of a call that splits K go through its stream's planes: calls that two threads make on the same stream, each with
+    operands of its own, give each thread its own sums."""
+    shapes = [(64, 1024, 8192), (300, 512, 4096)]
+    stream = torch.cuda.current_stream().cuda_stream
+    work = []
+    for t, (M, N, K) in enumerate(shapes):
+        say("gemm threads", M, N, K)
+        A, W = rand_i8(16, 10 + t, M, K), rand_i8(16, 20 + t, N, K)
+        xs, ws = synth.uniform(16, 30 + t, M, 0.005, 0.2), synth.uniform(16, 40 + t, N, 1e-3, 1e-2)
+        want = torch.from_numpy(oracle.epilogue(oracle.int8_gemm_acc(A, W), xs, ws, None, F32, fma=1)).to(DEV)
+        work.append((M, N, K, dev(A), dev(W), dev(xs), dev(ws), want, torch.empty((100, M, N), device=DEV)))
+    for M, N, K, A, W, xs, ws, want, out in work:   # the stream's buffer is there before the threads start
+        assert ffi.raw("gpu_int8_gemm", A.data_ptr(), W.data_ptr(), xs.data_ptr(), ws.data_ptr(), 0, out.data_ptr(), M, N, K, F32, stream) == 0
+    torch.cuda.synchronize()
+    codes = [[], []]
+
+    def calls(t):
+        M, N, K, A, W, xs, ws, want, out = work[t]
+        for i in range(out.shape[0]):
+            codes[t].append(ffi.raw("gpu_int8_gemm", A.data_ptr(), W.data_ptr(), xs.data_ptr(), ws.data_ptr(), 0, out[i].data_ptr(), M, N, K, F32, stream))
+
+    threads = [threading.Thread(target=calls, args=(t,)) for t in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for t in range(2):
+        assert not any(codes[t])
+        assert bool((work[t][8].view(torch.int32) == work[t][7].view(torch.int32)).all())
 
 
 # K % 16 == 8: the reference's alignment-8 configurations (csrc/vendor/cutlass_gemm_int8.cu:191,237-247)

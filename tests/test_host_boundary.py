@@ -4,6 +4,7 @@ import ctypes
 import json
 import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -227,3 +228,57 @@ def test_rust_host_crate_follows_the_headers_and_the_build_script():
             assert '"%s"' % flag in rs, flag
     for src, extra in build.EXTRA.items():
         assert src in rs and all('"%s"' % e in rs for e in extra)
+
+
+KEPT_BUFFERS = r"""
+#include "kept_buffers.hpp"
+#include <chrono>
+#include <cstdio>
+#include <thread>
+#include <vector>
+static KeptBuffers<2> kept;
+static std::mutex queue_mu;
+static std::vector<int> queue_;   // thread * 2 + launch
+static char memory[4][64];
+static int made = 0;
+int main() {
+    const auto make = [](size_t) -> void* { return memory[made++]; };
+    const auto call = [&](int thread) {
+        for (int i = 0; i < 20; ++i)
+            kept.with(0, nullptr, 8, 64, make, [&](void*) {
+                for (int launch = 0; launch < 2; ++launch) {
+                    { std::lock_guard<std::mutex> lock(queue_mu); queue_.push_back(thread * 2 + launch); }
+                    std::this_thread::sleep_for(std::chrono::microseconds(300));
+                }
+            });
+    };
+    std::thread a(call, 0), b(call, 1);
+    a.join();
+    b.join();
+    if (queue_.size() != 80 || made != 1) return 1;
+    for (size_t i = 0; i < queue_.size(); i += 2)
+        if (queue_[i] % 2 != 0 || queue_[i + 1] != queue_[i] + 1) return 2;   // a call's launches stand together
+    // one buffer per (device, stream); none where the call needs more than it holds, where it cannot be made, or beyond the last
+    int other = 0;
+    void *p0 = nullptr, *p1 = nullptr;
+    const auto none = [](size_t) -> void* { return nullptr; };
+    const auto ignore = [](void*) {};
+    if (kept.with(0, nullptr, 65, 64, make, ignore) || kept.with(0, &other, 65, 64, make, ignore)) return 3;
+    if (kept.with(0, &other, 8, 64, none, ignore) || made != 1) return 4;
+    if (!kept.with(0, nullptr, 64, 64, make, [&](void* p) { p0 = p; }) || !kept.with(0, &other, 8, 64, make, [&](void* p) { p1 = p; })) return 5;
+    if (p0 != memory[0] || p1 != memory[1] || made != 2) return 6;
+    if (kept.with(1, nullptr, 8, 64, make, ignore) || made != 2) return 7;
+    std::puts("ok");
+    return 0;
+}
+"""
+
+
+def test_calls_of_two_threads_on_one_stream_keep_their_launches_together(tmp_path):
+    """The buffer that a split-K GEMM's two launches share: what a second thread queues on the same stream comes before or behind
+    both of them, never between."""
+    src, exe = tmp_path / "kept.cpp", str(tmp_path / "kept")
+    src.write_text(KEPT_BUFFERS)
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-pthread", "-I", os.path.join(ROOT, "comfyui-backend-but-rust_amd", "csrc"), str(src), "-o", exe])
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout == "ok\n", (r.returncode, r.stdout)
