@@ -1405,13 +1405,25 @@ bool fed_may_split(int64_t M, int64_t N, int64_t K, hipStream_t st) {
     return tl_scratch == nullptr && !is_capturing(st);
 }
 
+// Kernel family forced by the test hook (-1 = choose by shape), or 7000 + 100 * width + slices: the kernel with fetching waves on
+// tiles of 64 * width columns and so many slices of K.  Process-wide and only meant for tests and benchmarks:
+// relaxed atomic, so a concurrent call sees either the old or the new value, never a torn one.
+std::atomic<int> g_force_cfg{-1};
+
+FedPlan fed_plan_or_forced(int64_t M, int64_t N, int64_t K, bool may_split) {
+    const int force = g_force_cfg.load(std::memory_order_relaxed) - 7000, width = force / 100;
+    if (force < 0 || width < 1 || width > 3) return fed_plan(M, N, K, device_cu_count(), may_split);
+    const int steps = (int)(K / 128), asked = !may_split || force % 100 < 1 ? 1 : force % 100 < steps ? force % 100 : steps, per = (steps + asked - 1) / asked;
+    return {width, (steps + per - 1) / per, per * 128, 0.};
+}
+
 template <int OUT_DT, int EPI>
 int launch_fed(GemmArgs a, hipStream_t st) {
     bool vec_ok, aligned;
     epilogue_alignment<OUT_DT, EPI>(a, vec_ok, aligned);
     if (!aligned) return launch_cfg<CfgM, OUT_DT, EPI>(a, st);   // only a forced family
-    FedPlan p = fed_plan(a.M, a.N, a.K, device_cu_count(), true);
-    if (p.slices > 1 && !fed_may_split(a.M, a.N, a.K, st)) p = fed_plan(a.M, a.N, a.K, device_cu_count(), false);
+    FedPlan p = fed_plan_or_forced(a.M, a.N, a.K, true);
+    if (p.slices > 1 && !fed_may_split(a.M, a.N, a.K, st)) p = fed_plan_or_forced(a.M, a.N, a.K, false);
     a.kslice = 0;
     if (p.slices == 1) return launch_fed_as<OUT_DT, EPI>(a, p.width, 1, st);
     return launch_split<OUT_DT, EPI>(a, p.slices, p.per, st, [&](const GemmArgs& pa) { return launch_fed_as<DT_F32, EPI_ACC>(pa, p.width, p.slices, st); });
@@ -1498,30 +1510,31 @@ bool rows_kernel_wins(int64_t M, int64_t N, int64_t K, bool aligned) {
     return !(M > 64 && K >= 1024 && K < (M > 96 ? 1408 : 1280) && N < (K < 1152 ? 1024 : 640));
 }
 
-// Kernel family forced by the test hook (-1 = choose by shape).  Process-wide and only meant for tests and benchmarks:
-// relaxed atomic, so a concurrent call sees either the old or the new value, never a torn one.
-std::atomic<int> g_force_cfg{-1};
-
-// `whole` = A and W start at 16-byte addresses, what the kernel for up to 128 rows asks of its DMA and its weight loads; an
-// operand that starts elsewhere (a view into a larger buffer) goes to the kernels that such calls had without it.  `aligned` as
-// epilogue_alignment has it.
-int choose_cfg(int64_t M, int64_t N, int64_t K, bool whole, bool aligned) {
+// `start`: the low four bits of A's and W's addresses together.  The kernel for up to 128 rows asks for 16-byte starts (its weight
+// loads and its DMA).  The other DMA kernels take operands from any 4-byte address, the alignment that a DMA of several
+// dwords needs; an operand that starts there but not at 16 bytes (a view into a larger buffer) goes to them from the sizes on from which
+// such calls always did, and to the register-staged tiles below.  Other starts always take the register-staged tiles, whose
+// ordinary loads may be unaligned.  `aligned` as epilogue_alignment has it.
+int choose_cfg(int64_t M, int64_t N, int64_t K, int start, bool aligned) {
     const int force = g_force_cfg.load(std::memory_order_relaxed);
     const bool tiles_ok = M * K < ((int64_t)1 << 32) && N * K < ((int64_t)1 << 32) && (K % 128) == 0;   // 32-bit lane offsets, whole steps
-    if (force == 5) return tiles_ok && whole && M <= 128 ? 5 : 1;
-    if (force == 7 || force == 9) return tiles_ok ? force : 1;
+    const bool dma_ok = tiles_ok && (start & 3) == 0;
+    if (force == 5) return tiles_ok && start == 0 && M <= 128 ? 5 : 1;
+    if (force == 7 || force / 1000 == 7) return dma_ok ? 7 : 1;
+    if (force == 9) return dma_ok ? 9 : 1;
     if (force == 1 || force == 2) return force;
-    if (tiles_ok && whole && M <= 128 && rows_kernel_wins(M, N, K, aligned)) return 5;
+    if (tiles_ok && start == 0 && M <= 128 && rows_kernel_wins(M, N, K, aligned)) return 5;
     const int cus = device_cu_count();
     // one or two steps of K and little to store: 512 threads and 96 KB of LDS to start cost more than they give (500 shapes, register-
     // staged tiles over fetching waves: K = 128 0.93 to 1.0, K = 256 0.94 to 1.0, K = 384 0.97 to 1.1; K = 256 with 1 << 21 outputs 1.1)
     const bool tiny = K <= 256 && M * N <= 1 << 19;
-    if (tiles_ok && aligned && !tiny) return M >= 512 && N >= 512 && pp_us(M, N, K, cus) < fed_plan(M, N, K, cus, true).us ? 9 : 7;
-    // the register-staged tiles: large ones as soon as there is work for them
-    if (M <= 256 && N >= 1024 && tiles_ok && K >= 512) return K >= 1536 || (M > 128 && N >= 8192) ? 1 : 2;
+    const int large = !dma_ok || !aligned ? 1 : M >= 512 && N >= 512 && pp_us(M, N, K, cus) < fed_plan(M, N, K, cus, true).us ? 9 : 7;
+    if (dma_ok && aligned && start == 0 && !tiny) return large;
+    // the register-staged tiles: large ones, or for operands off 16 bytes the DMA kernels, as soon as there is work for them
+    if (M <= 256 && N >= 1024 && tiles_ok && K >= 512) return K >= 1536 || (M > 128 && N >= 8192) ? large : 2;
     const int64_t tiles_s = ((M + 127) / 128) * ((N + 191) / 192);
-    if (M >= 512 && N >= 512 && tiles_s > cus) return 1;
-    if (tiles_ok && M > 128 && N >= 192 && (tiles_s >= 96 || (tiles_s >= 40 && K >= 2048) || (M <= 512 && N >= 1024 && K >= 8192))) return 1;
+    if (M >= 512 && N >= 512 && tiles_s > cus) return large;
+    if (tiles_ok && M > 128 && N >= 192 && (tiles_s >= 96 || (tiles_s >= 40 && K >= 2048) || (M <= 512 && N >= 1024 && K >= 8192))) return large;
     const int64_t tiles_m = ((M + 127) / 128) * ((N + 127) / 128);
     if (M > 64 && N > 64 && tiles_m >= 256) return 1;
     return 2;
@@ -1531,7 +1544,7 @@ template <int OUT_DT, int EPI>
 int dispatch_cfg(const GemmArgs& a, hipStream_t st) {
     bool vec_ok, aligned;
     epilogue_alignment<OUT_DT, EPI>(a, vec_ok, aligned);
-    switch (choose_cfg(a.M, a.N, a.K, (((uintptr_t)a.A | (uintptr_t)a.W) & 15) == 0, aligned)) {
+    switch (choose_cfg(a.M, a.N, a.K, (int)(((uintptr_t)a.A | (uintptr_t)a.W) & 15), aligned)) {
         case 5: return launch_rows<OUT_DT, EPI>(a, st);
         case 7: return launch_fed<OUT_DT, EPI>(a, st);
         case 9: return launch_pp<OUT_DT, EPI>(a, st);
@@ -1734,9 +1747,29 @@ GPU_API int gpu_int8_gemm_acc(const int8_t* A, const int8_t* W, int32_t* acc, in
 }
 
 // Test hook: force a kernel family (1 = 128x128, 2 = 64x64 register-staged tiles; 5 = up to 128 rows; 7 = waves that
-// fetch for others; 9 = two-group kernel; -1 or anything else = automatic).
+// fetch for others, 7000 + 100 * width + slices = those with that tile width (of 64 columns) and split; 9 = two-group
+// kernel; -1 or anything else = automatic).
 GPU_API int gpu_int8_gemm_force_config(int cfg) {
     g_force_cfg.store(cfg, std::memory_order_relaxed);
+    return 0;
+}
+
+// Test hook: what a call outside capture runs, for operands that start `start` bytes behind 16-byte addresses and outputs of whole 16
+// bytes or not.  out[0] = family as above, out[1] = tile width (family 7; of 64 columns) or 16-row tiles (5), out[2] = slices of K.
+GPU_API int gpu_internal_int8_gemm_plan(int64_t M, int64_t N, int64_t K, int start, int aligned, int32_t* out) {
+    if (M <= 0 || N <= 0 || K <= 0 || !shape_ok(M, N, K) || !out) return -200;
+    out[0] = choose_cfg(M, N, K, start & 15, aligned != 0);
+    out[1] = 0;
+    out[2] = 1;
+    if (out[0] == 7 && aligned) {
+        const FedPlan p = fed_plan_or_forced(M, N, K, true);
+        out[1] = p.width;
+        out[2] = p.slices;
+    } else if (out[0] == 5) {
+        const RowsPlan p = rows_plan(M, N, K, device_cu_count(), (N & 3) == 0);
+        out[1] = p.mt;
+        out[2] = p.slices;
+    }
     return 0;
 }
 

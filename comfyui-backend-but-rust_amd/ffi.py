@@ -59,6 +59,7 @@ SIGNATURES = {
     "gpu_internal_attn_layout": [_I32, _I32, _I32, _I32, _I32, _P],
     "gpu_internal_attn_layout_d": [_I32, _I32, _I32, _I32, _I32, _I32, _P],
     "gpu_int8_gemm_force_config": [_I32],
+    "gpu_internal_int8_gemm_plan": [_I64, _I64, _I64, _I32, _I32, _P],
     "gpu_act_tables_init": [],
     "gpu_mfma_layout_probe": [_P, _P],
     "gpu_mfma_ceiling_probe": [_I32, _I32, _P, _P, _P],

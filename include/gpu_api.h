@@ -305,9 +305,16 @@ int64_t gpu_w6a8_group_gemm_scratch(const void* Wp, int64_t M, int64_t N, int64_
 
 /* Test and tuning hook: force the GEMM kernel family.  1, 2 = 128x128 and 64x64 register-staged tiles; 5 = weights straight
  * into registers, for M <= 128; 7 = four waves multiply what four others fetch, 128x64 to 128x192 tiles, K split where they are few;
+ * 7000 + 100 * width + slices = 7 with tiles of 64 * width columns (width 1 to 3) and K in that many slices;
  * 9 = two-group kernel (256x256 and 128x256 tiles, one launch), the choice for large shapes; anything else = automatic.  A shape
  * a family cannot run falls back to 1. */
 int gpu_int8_gemm_force_config(int cfg);
+
+/* Test hook, no reference counterpart: which kernel a gpu_int8_gemm call outside capture takes for A and W that start `start` bytes
+ * behind 16-byte addresses, and outputs whose pointers and rows are of whole 16 bytes (aligned != 0) or not.  out[0] = family
+ * (numbers as above), out[1] = tile width of family 7 or row tiles of family 5, out[2] = slices of K.  Without a device it
+ * answers for 256 CUs. */
+int gpu_internal_int8_gemm_plan(int64_t M, int64_t N, int64_t K, int start, int aligned, int32_t* out);
 
 /* Writes, for each of the 64 lanes and 16 accumulator registers of one v_mfma_i32_32x32x32_i8, the (row of src0,
  * row of src1) pair that the register holds, as out[lane*16 + r] = i*32 + j.  A start-up self check of the operand

@@ -956,6 +956,23 @@ def test_int8_gemm_with_fetching_waves(M, N, K):
                 ffi.raw("gpu_int8_gemm_force_config", -1)
 
 
+@pytest.mark.parametrize("start", [1, 2, 4, 8, 12])
+@pytest.mark.parametrize("M,N,K", [(64, 136, 384), (3, 512, 1024), (200, 2056, 1536), (520, 25088, 128)])
+def test_int8_gemm_operands_off_16_bytes(M, N, K, start):
+    """A and W as views into larger buffers: the register-staged tiles at any address and, for the two larger shapes at a multiple of 4
+    bytes, the kernels with DMA."""
+    say("gemm start", M, N, K, start)
+    A, W = rand_i8(17, 500 + M, M, K), rand_i8(17, 600 + N, N, K)
+    xs, ws = synth.uniform(17, 3, M, 0.005, 0.2), synth.uniform(17, 4, N, 1e-3, 1e-2)
+    off = lambda a: torch.zeros(a.size + 16, dtype=torch.int8, device=DEV)[start:start + a.size].view(a.shape).copy_(dev(a))
+    plan = (C.c_int32 * 3)()
+    assert ffi.raw("gpu_internal_int8_gemm_plan", M, N, K, start, 1, C.cast(plan, C.c_void_p)) == 0
+    assert (plan[0] in (7, 9)) == (M >= 200 and start % 4 == 0)
+    want = oracle.epilogue(oracle.int8_gemm_acc(A, W), xs, ws, None, BF16, fma=1)
+    for a, w in ((off(A), off(W)), (off(A), dev(W)), (dev(A), off(W))):
+        assert np.array_equal(host_bits(ql.int8_gemm(a, w, dev(xs), dev(ws), None, torch.bfloat16)), want)
+
+
 def test_split_k_calls_of_two_threads_on_one_stream():
     """Both launches of a call that splits K go through its stream's planes: calls that two threads make on the same stream, each with
     operands of its own, give each thread its own sums."""

@@ -282,3 +282,37 @@ def test_calls_of_two_threads_on_one_stream_keep_their_launches_together(tmp_pat
     subprocess.check_call(["g++", "-std=c++17", "-O1", "-pthread", "-I", os.path.join(ROOT, "comfyui-backend-but-rust_amd", "csrc"), str(src), "-o", exe])
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout == "ok\n", (r.returncode, r.stdout)
+
+
+def gemm_plan(M, N, K, start=0, aligned=1):
+    out = (ctypes.c_int32 * 3)()
+    assert ffi.raw("gpu_internal_int8_gemm_plan", M, N, K, start, aligned, ctypes.cast(out, ctypes.c_void_p)) == 0
+    return tuple(out)
+
+
+def test_gemm_operands_off_16_bytes_keep_the_kernels_that_take_them():
+    """The kernel for up to 128 rows takes operands from 16-byte addresses only, the other two with DMA from 4-byte ones; and off 16
+    bytes those run the sizes from which they always did, the register-staged tiles what is smaller."""
+    def fetches(M, N, K):   # off 16 bytes, a multiple of 4
+        tiles = -(-M // 128) * -(-N // 192)
+        if K % 128:
+            return False
+        if M <= 256 and N >= 1024 and K >= 512:
+            return K >= 1536 or (M > 128 and N >= 8192)
+        if M >= 512 and N >= 512 and tiles > 256:
+            return True
+        return M > 128 and N >= 192 and (tiles >= 96 or (tiles >= 40 and K >= 2048) or (M <= 512 and N >= 1024 and K >= 8192))
+
+    assert gemm_plan(64, 136, 384)[0] == 7 and gemm_plan(4608, 12288, 3072)[0] == 9   # 16-byte starts: everything but the smallest
+    taken = set()
+    for M in (1, 3, 64, 128, 129, 256, 300, 512, 2048, 8192):
+        for N in (8, 136, 192, 512, 640, 1024, 4096, 8192, 12288):
+            for K in (64, 128, 384, 512, 1024, 1536, 2048, 8192):
+                for start in range(1, 16):
+                    family = gemm_plan(M, N, K, start)[0]
+                    if start % 4 == 0 and fetches(M, N, K):
+                        assert family in (7, 9), (M, N, K, start)
+                    else:
+                        assert family in (1, 2), (M, N, K, start, family)
+                    taken.add(family)
+    assert taken == {1, 2, 7, 9}
