@@ -1358,33 +1358,35 @@ int launch_fed_as(const GemmArgs& a, int width, int slices, hipStream_t st) {
 }
 
 // Tile width (of 64 columns) and K slices of the kernel with fetching waves, and its estimated time: rounds of one tile per CU, so many
-// us each and per step of 128, more per step where a CU has several tiles in a row (the clock goes down), or the weights' trip
-// from HBM, which a CU cannot take in faster than about 35 bytes per ns; a split pays for its planes and the launch that adds them.
-// The constants are fitted to 1190 shapes of 33 to 8192 rows (K 512 to 12288, N 640 to 24576, weights from HBM), where
-// the choice by these sums is 0.5 % slower than the best of all widths and slices on the average, and 1.34 times (1.55 times up to 512 rows)
-// as fast as what ran them before.
+// us each and per step of 128, more per step where tiles have all their 128 rows of A to fetch and where a CU has several tiles in
+// a row (the clock goes down), or the weights' trip from HBM, which a CU cannot take in faster than about 32 bytes per ns.  A split
+// pays for its planes and the launch that adds them, and some more where the slices start whole KB apart: their rows then meet in the
+// same of HBM's channels (24 x 3072 -> 2048 in eight 9.5 us, in five 8.2).  Tiles of 192 columns share 128-byte lines of outputs
+// whose rows are not whole ones (3490 x 512 -> 6536 43.6 us on them, 31.6 on 128 columns).
+// The constants are fitted to 3000 shapes of 1 to 8192 rows (K 256 to 14208, N 256 to 28000), calls in a row with weights that come
+// from HBM and not from the last-level cache (3 GiB of them in turn).  The choice is 1.1 % slower than the best of all
+// widths and slices on the average; constants fitted to weights that had stayed in that cache split K too rarely: 2.7 %, and 128 x 5120
+// -> 3072 in one slice 22.9 us, in five 13.4.
 struct FedPlan { int width, slices, per; double us; };   // per: K of a slice
 FedPlan fed_plan(int64_t M, int64_t N, int64_t K, int num_cu, bool may_split) {
-    // fixed, per round, per step of one round and of the rounds after it; a round after the first costs 0.5 more
-    static constexpr double c[3][4] = {{2.9, 1.1, 0.225, 0.25}, {1.9, 2.0, 0.29, 0.50}, {0.9, 3.55, 0.44, 0.66}};
+    // fixed, per round, per step, per step with 128 rows, per step and round after the first
+    static constexpr double c[3][5] = {{0.89, 2.20, 0.30, 0.07, 0.35}, {1.02, 3.12, 0.50, 0.01, 0.43}, {-0.69, 4.99, 0.89, -0.20, 0.63}};
     const int steps = (int)(K / 128), cus = num_cu;
+    const double rows = M < 128 ? (double)M / 128. : 1.;
     FedPlan best{3, 1, (int)K, 1e30};
     for (int w = 1; w <= 3; ++w) {
         const int64_t all = ((M + 127) / 128) * ((N + 64 * w - 1) / (64 * w));
         const int tiles = all < 1 << 24 ? (int)all : 1 << 24;
-        // slices: none, two, as many as give every CU a tile, half of that
         const int most = !may_split ? 1 : cus / tiles < steps / 3 ? cus / tiles : steps / 3;
-        const int tried[4] = {1, 2, most / 2, most};
-        for (int i = 0; i < 4; ++i) {
-            int s = tried[i];
-            if (i > 0 && (s < 2 || s > most || (i == 2 && s == 2))) continue;
-            const int per = (steps + s - 1) / s;
-            s = (steps + per - 1) / per;   // no empty slice
+        for (const int asked : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24}) {
+            if (asked > 1 && asked > most) break;
+            const int per = (steps + asked - 1) / asked, s = (steps + per - 1) / per;   // no empty slice
             const int busy = tiles * s < cus ? tiles * s : cus;
             const double n = (double)((tiles * s + cus - 1) / cus);
-            double us = c[w - 1][0] + n * c[w - 1][1] + (n - 1.) * 0.5 + (c[w - 1][2] + (n - 1.) * c[w - 1][3]) * per;
-            if (s > 1) us += 4.0 + (double)s * (double)M * (double)N * (8.0 / 4.2e6);
-            const double hbm = 4.0 + (double)N * (double)K / (34700. * busy);
+            double us = c[w - 1][0] + n * c[w - 1][1] + (c[w - 1][2] + rows * c[w - 1][3] + (n - 1.) * c[w - 1][4]) * per;
+            if (w == 3 && N % 64 != 0) us += 1.6 * n;
+            if (s > 1) us += 3.4 + (double)s * (0.05 + (double)M * (double)N * 1.69e-6) + (per % 8 == 0 ? 0.29 : 0.);
+            const double hbm = 3.86 + (double)N * (double)K / (32490. * busy);
             if (us < hbm) us = hbm;
             if (us < best.us) best = {w, s, per * 128, us};
         }
@@ -1394,7 +1396,7 @@ FedPlan fed_plan(int64_t M, int64_t N, int64_t K, int num_cu, bool may_split) {
 // The two-group kernel's time on the same scale.
 double pp_us(int64_t M, int64_t N, int64_t K, int cus) {
     const double n = pp_split(M, N, cus).rounds;
-    return -4.2 + n * (10.6 + 0.95 * (double)(K / 128));
+    return -3.0 + n * (12.0 + (double)(K / 128));
 }
 
 // Whether a call may split K over workgroups.  Captured graphs and the static entry point do so only for the shapes that always did
@@ -1488,23 +1490,33 @@ int launch_rows(GemmArgs a, hipStream_t st) {
         a.kslice = 0;
         return launch_rows_as<OUT_DT, EPI>(a, p.mt, p.nwk, vec_ok, 1, st);
     }
-    // Outputs that are narrow, or whose rows or pointers are not whole 16 bytes, do not split K under capture (fed_may_split has the
-    // reason) nor in the static entry point.
-    if ((a.N < 1024 || !aligned) && (tl_scratch != nullptr || is_capturing(st)))
+    // Under capture (fed_may_split has the reason) and in the static entry point outputs that are narrow, or whose rows or pointers are
+    // not whole 16 bytes, do not split K, nor do more rows with shorter K.
+    if ((a.N < 1024 || !aligned || (a.M <= 16 ? a.K < 2560 : a.K < 3072 || a.N > 1280)) && (tl_scratch != nullptr || is_capturing(st)))
         return aligned ? launch_fed<OUT_DT, EPI>(a, st) : a.N < 1024 ? launch_cfg<CfgS, OUT_DT, EPI>(a, st) : launch_cfg<CfgM, OUT_DT, EPI>(a, st);
     return launch_split<OUT_DT, EPI>(a, p.slices, p.per, st, [&](const GemmArgs& pa) { return launch_rows_as<DT_F32, EPI_ACC>(pa, p.mt, p.nwk, true, p.slices, st); });
 }
 
-// Whether the kernel for up to 128 rows runs a shape.  For outputs of whole 16 bytes: few rows, long K and few columns, where the
-// other kernel's planes and the launch that adds them cost more than the rows kernel's unevenly filled CUs.  Its time over that of
-// the kernel with fetching waves, 900 shapes with weights from HBM: up to 16 rows 0.65 to 1.0 from K = 2560 on and up to 8192 columns,
-// and 0.85 to 1.05 from K = 3584 on and 9500 to 16384 columns, but 1.0 at K = 2048, 1.1 to 1.3 just above 8192 columns (one more round) and
-// 1.1 to 1.6 above 16384; 17 to 64 rows 0.77 to 1.0 from K = 3072 on and up to 1280 columns, but 1.05 to
-// 1.15 at K = 2048 and 1.0 to 1.6 for more columns; 65 to 128 rows 1.0 to 1.7.  Other outputs have the register-staged tiles beside
-// them, which have less to start (128 rows 1152 -> 512 8.5 and 7.5 us; but 128 rows 1280 -> 640 8.5 and 9.2).
+// Whether the kernel for up to 128 rows runs a shape.  For outputs of whole 16 bytes: up to 64 rows and 8192 columns, from the K on
+// from which it is faster than the kernel with fetching waves up to where that one splits K better.  Its time over the other's by
+// 1500 shapes with weights from HBM, calls in a row:
+//   1 to 16 rows: 0.73 to 0.96 from K = 1408 to 4600, 0.85 to 1.1 above, 1.04 and more below.  Beyond 8192 columns, where it takes one more
+//     round: 0.91 up to K = 1920, 1.06 to 1.13 up to 3300, 0.81 to 1.07 above (from 9 rows on only up to 10240), but 1.03 to 1.25 there
+//     where weight rows are whole 4 KB (from 9 rows on: whole KB), which the other kernel's staggered starts suit.
+//   17 to 32: 0.77 to 0.99 from K = 1920 to 4096; above, 0.81 to 1.04 with few columns and 1.0 to 1.3 with many.
+//   33 to 64: 0.88 to 1.0 from K = 1024 to 2304 and 0.84 to 0.93 above 2816, but 1.0 to 1.16 between with few columns (its panels of 1024 end half empty).
+//   65 to 128: 1.0 to 1.6.
+// Other outputs have the register-staged tiles beside them, which have less to start (128 rows 1152 -> 512 8.5 and 7.5 us; but 128
+// rows 1280 -> 640 8.5 and 9.2).
 bool rows_kernel_wins(int64_t M, int64_t N, int64_t K, bool aligned) {
-    if (aligned && M <= 16) return N <= 8192 ? K >= 2560 : K >= 3584 && N > 9500 && N <= 16384;
-    if (aligned) return M <= 64 && K >= 3072 && N <= 1280;
+    if (aligned && M <= 16) {
+        if (N <= 8192) return K >= 1408;
+        return N <= 16384 && K >= 1408 && (K <= 1920 || (K >= 3328 && (M <= 8 ? K % 4096 != 0 : K <= 10240 && K % 1024 != 0)));
+    }
+    if (aligned && M <= 32) return N <= 8192 && ((K >= 1920 && K <= 4096) || (K > 4096 && N <= 1280));
+    if (aligned && M <= 64)
+        return N <= 8192 && ((K >= 1024 && K <= 2304) || (K > 2816 && K <= 3584) || (K > 2304 && K <= 2816 && N > 3072) || (K > 3584 && N <= (K <= 4608 ? 3072 : 1280)));
+    if (aligned) return false;
     if (K < (M > 96 ? 1024 : 768) || (M > 16 && N > 16384)) return false;
     if (K < 896) return !(N < 1152 && (M <= 32 || M > 64));
     return !(M > 64 && K >= 1024 && K < (M > 96 ? 1408 : 1280) && N < (K < 1152 ? 1024 : 640));
@@ -1526,9 +1538,12 @@ int choose_cfg(int64_t M, int64_t N, int64_t K, int start, bool aligned) {
     if (tiles_ok && start == 0 && M <= 128 && rows_kernel_wins(M, N, K, aligned)) return 5;
     const int cus = device_cu_count();
     // one or two steps of K and little to store: 512 threads and 96 KB of LDS to start cost more than they give (500 shapes, register-
-    // staged tiles over fetching waves: K = 128 0.93 to 1.0, K = 256 0.94 to 1.0, K = 384 0.97 to 1.1; K = 256 with 1 << 21 outputs 1.1)
-    const bool tiny = K <= 256 && M * N <= 1 << 19;
-    const int large = !dma_ok || !aligned ? 1 : M >= 512 && N >= 512 && pp_us(M, N, K, cus) < fed_plan(M, N, K, cus, true).us ? 9 : 7;
+    // staged tiles over fetching waves: K = 128 0.93 to 1.0, K = 256 0.94 to 1.0, K = 384 0.97 to 1.1; K = 256 with 1 << 21 outputs 1.1; one step
+    // and more columns than the CUs take at once in tiles of 64, 25 x 24784 4.4 us and 5.1, but 73 x 10368 4.4 and 3.8)
+    const bool tiny = K <= 256 && (M * N <= 1 << 19 || (K <= 128 && M * N <= 1 << 20 && N > 64 * cus));
+    // (with one or two steps of K in several rounds the fetching waves' tiles take a fifth longer than the sums say: K = 128, 5366 x 3144
+    // 28.1 and 20.9 us on the two-group kernel, 536 x 22792 17.0 and 13.7)
+    const int large = !dma_ok || !aligned ? 1 : M >= 512 && N >= 512 && pp_us(M, N, K, cus) < fed_plan(M, N, K, cus, true).us * (K <= 256 ? 1.2 : 1.) ? 9 : 7;
     if (dma_ok && aligned && start == 0 && !tiny) return large;
     // the register-staged tiles: large ones, or for operands off 16 bytes the DMA kernels, as soon as there is work for them
     if (M <= 256 && N >= 1024 && tiles_ok && K >= 512) return K >= 1536 || (M > 128 && N >= 8192) ? large : 2;
