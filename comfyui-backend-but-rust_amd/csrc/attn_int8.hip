@@ -1087,8 +1087,8 @@ __device__ __forceinline__ float swap32_sum(float x) {
     return u2f(r[0]) + u2f(r[1]);
 }
 
-// First key tile of part p.  The second of two halves is shorter by two tiles or three, so that it has written its result when the
-// first one ends, which then keeps its own in registers.
+// First key tile of part p.  The second of two halves is shorter by two tiles, or by one where their number is odd, so that it has
+// mostly written its result when the first one ends, which then keeps its own in registers.
 __device__ __forceinline__ int part_bound(int kb, int parts, int p) { return kb * p / parts + (parts == 2 && p == 1 ? 1 : 0); }
 // Two floats to and from memory past the caches that XCDs do not share: agent-scope stores are written through and acknowledged where
 // every XCD sees them, agent-scope loads are not served from a stale line.  So a part's result needs a wait for its own stores ahead
@@ -1149,20 +1149,20 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
     const int* vst = a.vsum + kvh * a.kb * D;
     const float* kst = a.ks + kvh * a.kb * 4 + hh * 2;
 
-    // The DMA of a wave's share of K tile tk (j < NF), V tile tv and its column sums (j = 2 NF).  Tiles past the end re-fetch the last
-    // one, which nothing reads, and every wave fetches column sums (two waves the same ones): no branch in the tile loop.
+    // The DMA of a wave's share of K tile tk (j < NF), V tile tv and its column sums (j = 2 NF).  A K tile past the end fetches the last
+    // one, into the stage that a tile tk would have: nothing reads that stage any more, while the last tile's own stage is being read.
+    // Every wave fetches column sums (two waves the same ones): no branch in the tile loop.
     constexpr int NF = KV / 4096;
     auto dma = [&](int j, int tk, int tv) {
         const int c = (wave + 4 * (j % NF)) * 1024, cs = D == 128 ? (wave & 1) * 256 : 0;
-        if (j < NF) dma16(lds0 + (tk & 1) * STAGE + c, lane16, kt + (int64_t)tk * KV + c);
+        if (j < NF) dma16(lds0 + (tk & 1) * STAGE + c, lane16, kt + (int64_t)(tk < a.kb ? tk : a.kb - 1) * KV + c);
         else if (j < 2 * NF) dma16(lds0 + (tv & 1) * STAGE + KV + c, lane16, vt + (int64_t)tv * KV + c);
         else dma4(lds0 + (tv & 1) * STAGE + 2 * KV + cs, lane16 >> 2, (const uint8_t*)(vst + (int64_t)tv * D) + cs);
     };
-    auto or_last = [&](int t) { return t < a.kb ? t : a.kb - 1; };
 #pragma unroll
     for (int j = 0; j <= 2 * NF; ++j) dma(j, t0, t0);
 #pragma unroll
-    for (int j = 0; j < NF; ++j) dma(j, or_last(t0 + 1), 0);
+    for (int j = 0; j < NF; ++j) dma(j, t0 + 1, 0);
 
     v4i qf[NS];
     {
@@ -1266,7 +1266,7 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
                     pf[rg < NB ? rg : 0][g4] = (int)(packed ^ 0x80808080u);
                 }
                 if constexpr (!last) {
-                    if (rg * 4 + g4 >= 1 && rg * 4 + g4 <= 2 * NF + 1) dma(rg * 4 + g4 - 1, or_last(t + 2), t + 1);
+                    if (rg * 4 + g4 >= 1 && rg * 4 + g4 <= 2 * NF + 1) dma(rg * 4 + g4 - 1, t + 2, t + 1);
                     if (rg > 0 && g4 % (4 / NS) == 0) {
                         const int s = g4 / (4 / NS);
                         if (s == 0) S[rg - 1] = v16i{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
