@@ -1476,8 +1476,7 @@ int key_parts(int64_t row_blocks, int64_t kb, int ck, int D, int64_t& whole) {
     return best;
 }
 
-// `piped`: the pipelined kernel runs; the other one shares no keys.
-Plan plan_for(int64_t b, int64_t h, int64_t hk, int64_t lq, int64_t lk, int D, bool piped) {
+Plan plan_for(int64_t b, int64_t h, int64_t hk, int64_t lq, int64_t lk, int D) {
     Plan p;
     p.ck = cta_k_for((int)lk, D);
     p.kb = (int)((lk + p.ck - 1) / p.ck);
@@ -1495,8 +1494,7 @@ Plan plan_for(int64_t b, int64_t h, int64_t hk, int64_t lq, int64_t lk, int D, b
     p.vmax = add(b * hk * D * 4);
     p.vsum = add(b * hk * (int64_t)p.kb * D * 4);
     const int64_t row_blocks = b * h * ((lq + 127) / 128);
-    p.whole = row_blocks;
-    p.parts = piped ? key_parts(row_blocks, p.kb, p.ck, D, p.whole) : 1;
+    p.parts = key_parts(row_blocks, p.kb, p.ck, D, p.whole);
     p.done = add((row_blocks - p.whole) * 4);
     p.part = add((row_blocks - p.whole) * p.parts * 4 * 64 * (D / 2 + 2) * 4);
     p.total = n;
@@ -1591,8 +1589,7 @@ int int8_attn(const void* q, const void* k, const void* v, void* o, void* ws, in
         fprintf(stderr, "int8 attention: %s\n", why);
         return -400;
     }
-    const bool unfused = dt == DT_F16 && lk <= 512;   // see run(); its workspace function knows no type and reserves for bf16
-    const Plan p = plan_for(b, h, hk, lq, lk, Dh, !bias && !unfused);
+    const Plan p = plan_for(b, h, hk, lq, lk, Dh);
     char* w = (char*)ws;
     AttnArgs a;
     a.q = q; a.k = k; a.v = v; a.o = o;
@@ -1639,7 +1636,7 @@ int int8_attn(const void* q, const void* k, const void* v, void* o, void* ws, in
 GPU_API int64_t gpu_int8_attn_workspace_d(int b, int h, int hk, int lq, int lk, int head_dim) {
     if (head_dim != 64 && head_dim != 128 && head_dim != 256) return 0;
     if (b <= 0 || h <= 0 || hk <= 0 || lq <= 0 || lk <= 0) return 0;
-    return plan_for(b, h, hk, lq, lk, head_dim, true).total;
+    return plan_for(b, h, hk, lq, lk, head_dim).total;
 }
 
 GPU_API int64_t gpu_int8_attn_workspace(int b, int h, int hk, int lq, int lk) {
@@ -1700,7 +1697,7 @@ static int64_t key_mask_width(int lk) {
 
 GPU_API int64_t gpu_int8_attn_key_bias_workspace(int b, int h, int hk, int lq, int lk) {
     if (b <= 0 || h <= 0 || hk <= 0 || lq <= 0 || lk <= 0) return 0;
-    return plan_for(b, h, hk, lq, lk, 128, false).total + (key_mask_width(lk) * 4 + 255) / 256 * 256;
+    return gpu_int8_attn_workspace_d(b, h, hk, lq, lk, 128) + (key_mask_width(lk) * 4 + 255) / 256 * 256;
 }
 
 // gpu_int8_attn with bias (f32 [lk], the same for every batch item, query and head) added to each key's logits, as an
@@ -1754,7 +1751,7 @@ GPU_API int gpu_internal_attn_sumsq_probe(const float* x, float* out, int rows, 
 // anchors, vsum, key tile length, key tiles.
 GPU_API int gpu_internal_attn_layout_d(int b, int h, int hk, int lq, int lk, int head_dim, int64_t* out) {
     if (b <= 0 || h <= 0 || hk <= 0 || lq <= 0 || lk <= 0 || !out || (head_dim != 64 && head_dim != 128 && head_dim != 256)) return -400;
-    const Plan p = plan_for(b, h, hk, lq, lk, head_dim, true);
+    const Plan p = plan_for(b, h, hk, lq, lk, head_dim);
     const int64_t v[10] = {p.qi, p.ki, p.qs, p.ks, p.vt, p.vs, p.anchors, p.vsum, p.ck, p.kb};
     for (int i = 0; i < 10; ++i) out[i] = v[i];
     return 0;

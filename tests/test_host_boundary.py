@@ -332,17 +332,3 @@ def test_gemm_choice_where_it_was_measured():
         assert family == 7 and slices == 1, (M, N, K, slices)
     for M, N, K in [(4608, 3072, 3072), (8192, 5120, 640), (1024, 9216, 4096), (5366, 3144, 128)]:
         assert gemm_plan(M, N, K)[0] == 9, (M, N, K)
-
-
-@pytest.mark.parametrize("b,h,hk,lq,lk", [(1, 205, 205, 128, 8192), (1, 10, 2, 130, 1500), (2, 24, 24, 4608, 4608), (1, 1, 1, 5, 7)])
-def test_key_bias_workspace_holds_no_parts_of_shared_keys(b, h, hk, lq, lk):
-    """The key-bias form never shares a row block's keys between workgroups: its workspace ends with the column sums and the prepared
-    bias, while the form without a bias has the parts behind them where there are any."""
-    out = (ctypes.c_int64 * 10)()
-    assert ffi.raw("gpu_internal_attn_layout", b, h, hk, lq, lk, ctypes.cast(out, ctypes.c_void_p)) == 0
-    up = lambda n: -(-n // 256) * 256
-    sums = out[7] + up(b * hk * out[9] * 128 * 4)
-    bias = up((-(-lk // 128) * 129 + 3) // 4 * 4 * 4)
-    assert ffi.lib.gpu_int8_attn_key_bias_workspace(b, h, hk, lq, lk) == sums + bias
-    blocks = b * h * -(-lq // 128)
-    assert (ffi.lib.gpu_int8_attn_workspace(b, h, hk, lq, lk) > sums) == (blocks >= 8)
