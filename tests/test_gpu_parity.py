@@ -30,6 +30,13 @@ def say(*a):
     print(*a, flush=True)
 
 
+def gemm_plan(M, N, K, start=0, aligned=1):
+    """(family, tile width or row tiles, slices of K) of a gpu_int8_gemm call outside capture."""
+    out = (C.c_int32 * 3)()
+    assert ffi.raw("gpu_internal_int8_gemm_plan", M, N, K, start, aligned, C.cast(out, C.c_void_p)) == 0
+    return tuple(out)
+
+
 def dev_bits(bits, dt):
     """numpy array (uint16 bits for bf16/f16, float32 for f32) -> CUDA tensor of that dtype."""
     if dt == F32:
@@ -873,7 +880,7 @@ ACC_CASES = [(1, 96, 256), (3, 32, 16), (64, 64, 64), (65, 72, 48), (100, 104, 3
              (77, 4096, 1280), (250, 25000, 128)]
 
 
-@pytest.mark.parametrize("cfg", [2, 1, 6, 7, 9])
+@pytest.mark.parametrize("cfg", [2, 1, 7302, 7, 9])   # 7302: tiles of 192 columns, K in two slices
 @pytest.mark.parametrize("M,N,K", ACC_CASES)
 def test_int8_gemm_acc_bit_exact(M, N, K, cfg):
     say("gemm_acc", M, N, K, "cfg", cfg)
@@ -893,7 +900,7 @@ def test_int8_gemm_acc_bit_exact(M, N, K, cfg):
 
 # Edges of the kernel for up to 128 rows: its row tiles (16, 32, 64, 96, 128), columns past the last tile and unaligned ones, K
 # shorter than a panel, panels with a remainder, an odd and an even number of them, and K split over workgroups, with outputs of
-# whole 16 bytes and of whole 8; and calls that the automatic choice gives to the streaming kernel and the small tiles
+# whole 16 bytes and of whole 8; and calls that the automatic choice gives to the kernel with fetching waves and the small tiles
 ROWS_CASES = [(64, 1028, 4096), (65, 9216, 5120), (33, 4612, 7296), (24, 256, 768), (100, 512, 1152), (1, 8, 128), (15, 67, 768), (16, 1000, 4096), (17, 96, 1152), (32, 4100, 896), (33, 72, 2176), (64, 130, 1024), (65, 4096, 896),
               (77, 1024, 3712), (96, 264, 640), (97, 96, 1280), (128, 2048, 4224), (16, 16416, 1024), (5, 4097, 2304)]
 
@@ -923,8 +930,10 @@ def test_int8_gemm_up_to_128_rows(M, N, K):
             ffi.raw("gpu_int8_gemm_force_config", -1)
 
 
-# Edges of the kernel with fetching waves: fewer steps of K than LDS stages, an odd and an even number of them, its three widths with a
-# last tile of 1, 8 or all columns and of 1, 127 or all rows, several rounds of tiles, K in equal slices and with a shorter last one
+# The kernel with fetching waves as the dispatch plans it (every width and split is
+# forced below): fewer steps of K than LDS stages, an odd and an even number of them, last tiles of 8 or all columns and of 1,
+# 127 or all rows, several rounds of tiles, K in slices.  Outputs whose rows are not of whole 16 bytes (65, 1281, 1030) take the
+# register-staged tiles when this kernel is forced
 FED_CASES = [(1, 64, 128), (128, 65, 256), (129, 136, 384), (300, 1000, 512), (255, 3008, 640), (2048, 640, 2560), (1025, 192, 896), (3000, 5000, 128), (640, 1281, 1152), (256, 1000, 3712), (200, 2048, 4096),
              (77, 1030, 5120), (400, 136, 6016)]
 
@@ -956,6 +965,42 @@ def test_int8_gemm_with_fetching_waves(M, N, K):
                 ffi.raw("gpu_int8_gemm_force_config", -1)
 
 
+# (steps of K, slices): one step, fewer than, as many as and more than the four LDS stages, a long run; slices of equal length and with a
+# shorter last one
+FED_STEPS = [(1, 1), (3, 1), (4, 1), (5, 1), (20, 1), (5, 2), (20, 3), (8, 4)]
+
+
+@pytest.mark.parametrize("M,cols", [(129, 8), (200, -8), (128, 0)])   # last tiles of 1, 72 and all rows; of 8, all but 8 and all columns
+@pytest.mark.parametrize("steps,slices", FED_STEPS)
+@pytest.mark.parametrize("width", [1, 2, 3])
+def test_int8_gemm_fetching_waves_every_width_and_split(width, steps, slices, M, cols):
+    K, N = 128 * steps, 64 * width * 2 + cols
+    say("gemm fetching waves", width, steps, slices, M, N)
+    A, W = rand_i8(18, 500 + M, M, K), rand_i8(18, 600 + N, N, K)
+    A[0, :] = -128
+    W[N - 1, :] = -128
+    xs, ws = synth.uniform(18, 3, M, 0.005, 0.2), synth.uniform(18, 4, N, 1e-3, 1e-2)
+    want = oracle.int8_gemm_acc(A, W)
+    Ad, Wd, xd, wd = dev(A), dev(W), dev(xs), dev(ws)
+    ffi.raw("gpu_int8_gemm_force_config", 7000 + 100 * width + slices)
+    try:
+        assert gemm_plan(M, N, K) == (7, width, slices)
+        assert np.array_equal(ql.int8_gemm_acc(Ad, Wd).cpu().numpy(), want)
+        for dt, tob in ((BF16, oracle.bf16_bits), (F16, oracle.f16_bits), (F32, lambda a: a.astype(np.float32))):
+            bias, rs = tob(synth.normal(18, 5, N) * np.float32(0.02)), tob(synth.normal(18, 6, N))
+            resid = tob(synth.normal(18, 7, M * N).reshape(M, N))
+            for b in (None, bias):
+                d = ql.int8_gemm(Ad, Wd, xd, wd, None if b is None else dev_bits(b, dt), TDT[dt])
+                assert np.array_equal(host_bits(d), oracle.epilogue(want, xs, ws, b, dt, fma=1)), dt
+            wr = oracle.epilogue_residual(want, xs, ws, bias, rs, resid, dt, fma=1)
+            rd = dev_bits(resid, dt)
+            assert np.array_equal(host_bits(ql.int8_gemm_residual(Ad, Wd, xd, wd, dev_bits(bias, dt), dev_bits(rs, dt), rd)), wr), dt
+            ql.int8_gemm_residual(Ad, Wd, xd, wd, dev_bits(bias, dt), dev_bits(rs, dt), rd, D=rd)   # in place
+            assert np.array_equal(host_bits(rd), wr), dt
+    finally:
+        ffi.raw("gpu_int8_gemm_force_config", -1)
+
+
 @pytest.mark.parametrize("start", [1, 2, 4, 8, 12])
 @pytest.mark.parametrize("M,N,K", [(64, 136, 384), (3, 512, 1024), (200, 2056, 1536), (520, 25088, 128)])
 def test_int8_gemm_operands_off_16_bytes(M, N, K, start):
@@ -965,12 +1010,30 @@ def test_int8_gemm_operands_off_16_bytes(M, N, K, start):
     A, W = rand_i8(17, 500 + M, M, K), rand_i8(17, 600 + N, N, K)
     xs, ws = synth.uniform(17, 3, M, 0.005, 0.2), synth.uniform(17, 4, N, 1e-3, 1e-2)
     off = lambda a: torch.zeros(a.size + 16, dtype=torch.int8, device=DEV)[start:start + a.size].view(a.shape).copy_(dev(a))
-    plan = (C.c_int32 * 3)()
-    assert ffi.raw("gpu_internal_int8_gemm_plan", M, N, K, start, 1, C.cast(plan, C.c_void_p)) == 0
-    assert (plan[0] in (7, 9)) == (M >= 200 and start % 4 == 0)
+    assert (gemm_plan(M, N, K, start)[0] in (7, 9)) == (M >= 200 and start % 4 == 0)
     want = oracle.epilogue(oracle.int8_gemm_acc(A, W), xs, ws, None, BF16, fma=1)
     for a, w in ((off(A), off(W)), (off(A), dev(W)), (dev(A), off(W))):
         assert np.array_equal(host_bits(ql.int8_gemm(a, w, dev(xs), dev(ws), None, torch.bfloat16)), want)
+
+
+def test_split_k_planes_beyond_the_streams_buffer():
+    """No planned split needs more planes than the buffer holds; a forced one that does allocates for itself and gives the same bits, and
+    the entry point that may not allocate refuses it."""
+    M, N, K = 256, 4096, 4096
+    A, W = rand_i8(19, 1, M, K), rand_i8(19, 2, N, K)
+    xs, ws = dev(synth.uniform(19, 3, M, 0.005, 0.2)), dev(synth.uniform(19, 4, N, 1e-3, 1e-2))
+    Ad, Wd, D = dev(A), dev(W), torch.empty((M, N), device=DEV)
+    assert ffi.lib.gpu_int8_gemm_static_limit() < 16 * M * N * 4
+    want = ql.int8_gemm(Ad, Wd, xs, ws, None, torch.float32)
+    ffi.raw("gpu_int8_gemm_force_config", 7116)
+    try:
+        assert gemm_plan(M, N, K) == (7, 1, 16)
+        assert np.array_equal(ql.int8_gemm_acc(Ad, Wd).cpu().numpy(), oracle.int8_gemm_acc(A, W))
+        assert torch.equal(ql.int8_gemm(Ad, Wd, xs, ws, None, torch.float32).view(torch.int32), want.view(torch.int32))
+        assert ffi.raw("gpu_int8_gemm_static", Ad.data_ptr(), Wd.data_ptr(), xs.data_ptr(), ws.data_ptr(), 0, D.data_ptr(), M, N, K, F32,
+                       torch.cuda.current_stream().cuda_stream) == -210
+    finally:
+        ffi.raw("gpu_int8_gemm_force_config", -1)
 
 
 def test_split_k_calls_of_two_threads_on_one_stream():
@@ -1033,10 +1096,7 @@ def test_int8_gemm_k_multiple_of_8_only(M, N, K):
 # More 256x256 tiles than CUs, and not a multiple of the CU count: the persistent kernel's workgroups then own unequal
 # numbers of tiles, and every output form runs through its coalesced epilogue.
 MANY_TILE_CASES = [(4352, 4096, 256), (4100, 4400, 384), (2304, 8200, 640),
-                   # either side of the dispatcher's thresholds: two row tiles of the weight-streaming kernel with K split
-                   # (planes beyond the per-stream buffer), ring tiles for few tiles and long K, short K at M <= 256 on
-                   # the register-staged and ring tiles, M <= 128 with K = 1536 on the weight-streaming kernel, and a
-                   # shape where the two-group tiles cover half of the CUs
+                   # the kernel with fetching waves: K split and whole, tiles of 64 and 128 columns, one, two and more row tiles
                    (384, 1056, 8192), (512, 4096, 2048), (256, 1024, 1024), (256, 12288, 1024), (200, 2048, 2048),
                    (100, 3008, 1536), (2048, 2048, 512)]
 
@@ -1085,7 +1145,7 @@ def test_int8_gemm_epilogue(M, N, K, with_bias, out_dt):
     bias = tob(synth.normal(2, 5, N) * np.float32(0.02)) if with_bias else None
     want = oracle.int8_gemm(A, W, xs, ws, bias, out_dt, fma=1)
     loose = oracle.int8_gemm(A, W, xs, ws, bias, out_dt, fma=0)
-    for cfg in (-1, 1, 2, 6, 7, 9):
+    for cfg in (-1, 1, 2, 7302, 7, 9):
         ffi.raw("gpu_int8_gemm_force_config", cfg)
         try:
             got = ql.int8_gemm(dev(A), dev(W), dev(xs), dev(ws), None if bias is None else dev_bits(bias, out_dt), TDT[out_dt])
@@ -1129,9 +1189,9 @@ def test_int8_gemm_residual_in_place(out_dt):
 
 
 RESID_CASES = [  # (M, N, K, kernel families that can run the shape)
-    (200, 1024, 4096, (-1, 6, 1, 2)),          # skinny: split K, planes summed by the reduce kernel
-    (256, 2400, 1024, (-1, 6, 1)),             # skinny: one K slice, the streaming kernel's own epilogue
-    (600, 768, 512, (-1, 1, 2, 7, 9)),         # tile kernels and the persistent kernels
+    (200, 1024, 4096, (-1, 7302, 1, 2)),       # split K, planes summed by the reduce kernel
+    (256, 2400, 1024, (-1, 7301, 1)),          # one K slice, the kernel's own epilogue
+    (600, 768, 512, (-1, 1, 2, 7, 9)),         # every family for more than 128 rows
 ]
 
 
@@ -1139,8 +1199,8 @@ RESID_CASES = [  # (M, N, K, kernel families that can run the shape)
 @pytest.mark.parametrize("M,N,K,cfgs", RESID_CASES)
 def test_int8_gemm_residual_in_place_every_kernel_family(M, N, K, cfgs, out_dt):
     """gpu_int8_gemm_residual with D aliasing resid (the down-projection pattern of src/dit.rs:592) through every kernel
-    family: the streaming kernel's residual epilogue, the split-K reduce kernel's, the persistent kernels' and the
-    tile kernels', bit-exact against the oracle."""
+    family: the residual epilogue of the kernel with fetching waves, the split-K reduce kernel's, the two-group kernel's and the
+    register-staged tiles', bit-exact against the oracle."""
     say("gemm_residual", M, N, K, out_dt)
     A = rand_i8(13, 1, M, K, -127, 127)
     W = rand_i8(13, 2, N, K, -127, 127)
@@ -1352,16 +1412,21 @@ def test_quant_rows_with_more_than_2_to_the_31_elements(rotate):
 
 
 # ------------------------------------------------------------------------------------------------ graph capture
-@pytest.mark.parametrize("M,N,K,entry", [(4096, 4096, 256, "gpu_int8_gemm"),          # two-group kernel
-                                           (1024, 2304, 256, "gpu_int8_gemm"),          # ring kernel on 128x192 tiles
-                                           (256, 24576, 3072, "gpu_int8_gemm"),         # weight-streaming kernel, whole K
-                                           (640, 1536, 512, "gpu_int8_gemm"),           # register-staged tiles
-                                           (256, 2048, 4096, "gpu_int8_gemm_static")])  # weight-streaming kernel, split K, static planes
-def test_linear_replays_from_a_captured_graph(M, N, K, entry):
+@pytest.mark.parametrize("M,N,K,entry,plan", [(4096, 4096, 256, "gpu_int8_gemm", (9, 1)),          # two-group kernel
+                                               (1024, 2304, 256, "gpu_int8_gemm", (7, 1)),          # fetching waves
+                                               (256, 24576, 3072, "gpu_int8_gemm", (7, 1)),
+                                               (640, 1536, 512, "gpu_int8_gemm", (7, 1)),
+                                               (640, 768, 256, "gpu_int8_gemm", (2, 1)),            # register-staged tiles
+                                               (256, 2048, 4096, "gpu_int8_gemm_static", (7, 2)),   # split K, static planes
+                                               (256, 4096, 8192, "gpu_int8_gemm_static", (7, 2)),
+                                               (64, 1024, 8192, "gpu_int8_gemm_static", (5, 2))])
+def test_linear_replays_from_a_captured_graph(M, N, K, entry, plan):
     """The quantizer and the GEMM allocate nothing on these routes (the split-K shape through the entry point with the
     static planes), so one linear can be captured.  Three replays with new activations and eager work between them,
     each against the oracle's linear on the same inputs."""
     say("graph", M, N, K, entry)
+    family, _, slices = gemm_plan(M, N, K)
+    assert (family, min(slices, 2)) == plan   # 2: split
     W, ws, bias = synth.w8_weights(21, N, K)
     bias = oracle.bf16_bits(bias)
     Wd, wsd, bd = dev(W), dev(ws), dev_bits(bias, BF16)
@@ -1392,11 +1457,12 @@ def test_linear_replays_from_a_captured_graph(M, N, K, entry):
         _ = (torch.randn(1024, device="cuda") * 2).sum().item()   # eager work between the replays
 
 
-@pytest.mark.parametrize("M,N,K,entry", [(16, 512, 4096, "gpu_int8_gemm"),            # K split when run eagerly, not in a graph
-                                           (77, 4096, 1152, "gpu_int8_gemm"),           # kernel for up to 128 rows, whole K
-                                           (128, 960, 8192, "gpu_int8_gemm_static")])   # narrow: leaves the static planes alone
-def test_few_rows_replay_from_a_captured_graph(M, N, K, entry):
-    test_linear_replays_from_a_captured_graph(M, N, K, entry)
+@pytest.mark.parametrize("M,N,K,entry,plan", [(16, 512, 8192, "gpu_int8_gemm", (5, 2)),            # K split when run eagerly, not in a graph
+                                               (16, 4096, 1536, "gpu_int8_gemm", (5, 1)),           # kernel for up to 128 rows, whole K
+                                               (77, 4096, 1152, "gpu_int8_gemm", (7, 1)),
+                                               (128, 960, 8192, "gpu_int8_gemm_static", (7, 2))])   # narrow: leaves the static planes alone
+def test_few_rows_replay_from_a_captured_graph(M, N, K, entry, plan):
+    test_linear_replays_from_a_captured_graph(M, N, K, entry, plan)
 
 
 def _nodes_of_capture(call):
@@ -1614,7 +1680,7 @@ def test_full_size_linear_rows_against_oracle(name, M, K, N, rotate, kind):
     got_rowsum = acc.to(torch.int64).sum(dim=1).cpu().numpy()
     assert np.array_equal(got_rowsum, want_rowsum)
     # every kernel family that can run the shape gives the same bits
-    for cfg in (1, 7, 9) if M > 256 and M * N < 8192 * 5120 else (1,) if M > 256 else (6, 1):
+    for cfg in (1, 7, 9) if M > 256 and M * N < 8192 * 5120 else (1,) if M > 256 else (7, 7302, 7201, 1):
         ffi.raw("gpu_int8_gemm_force_config", cfg)
         try:
             d2 = ql.int8_gemm(qd, Wd, xsd, wsd, bd, torch.bfloat16)

@@ -1,5 +1,6 @@
 """gpu_int8_gemm_static, the entry point that allocates nothing, against gpu_int8_gemm: bit-equal outputs through the C ABI
 on calls in a row, each with a smaller input (the static split-K planes keep the earlier calls' contents)."""
+import ctypes
 import importlib
 import os
 import sys
@@ -45,14 +46,18 @@ def _run(name, A, W, xs, ws, bias):
     return D.cpu().numpy().view(np.uint16)
 
 
-# larger first: split K in the weight-streaming kernel, no split in the kernel for up to 128 rows, split K there
-SHAPES = [(256, 4096, 4096), (100, 1024, 2048), (100, 1024, 4096), (16, 1024, 8192)]
+# larger planes first, so that the later calls find stale ones: (M, N, K, family, K split).  7: the kernel with fetching waves, 5: the one
+# for up to 128 rows
+SHAPES = [(256, 4096, 12288, 7, True), (64, 1024, 8192, 5, True), (100, 1024, 2048, 7, False), (100, 1024, 4096, 7, True), (16, 1024, 8192, 5, True)]
 
 
 def test_static_entry_point_matches_allocating_one_twice_in_a_row():
     assert ffi.lib.gpu_int8_gemm_static_limit() == 24 << 20
-    for i, (M, N, K) in enumerate(SHAPES):
+    for i, (M, N, K, family, split) in enumerate(SHAPES):
         print("no-alloc case", i, M, N, K, flush=True)
+        plan = (ctypes.c_int32 * 3)()
+        ffi.k("gpu_internal_int8_gemm_plan", M, N, K, 0, 1, ctypes.cast(plan, ctypes.c_void_p))
+        assert plan[0] == family and (plan[2] > 1) == split, (M, N, K, tuple(plan))
         A, W, xs, ws, bias = _inputs(40 + i, M, N, K)
         want = _run("gpu_int8_gemm", A, W, xs, ws, bias)
         got = _run("gpu_int8_gemm_static", A, W, xs, ws, bias)
@@ -71,8 +76,8 @@ def test_static_entry_point_on_shapes_without_scratch():
 
 def test_static_entry_point_refuses_what_would_need_an_allocation():
     """K % 16 == 8 runs on padded copies that gpu_int8_gemm allocates; the entry point that may not allocate refuses it.
-    (The split-K planes of every M <= 256 shape fit the static array on a 256-CU device: slices * N <= 256 * 96, and 256 * 64 up to
-    128 rows.)"""
+    (The split-K planes of every shape that is split fit the static array on a 256-CU device: slices * tiles <= 256, and no tile
+    is larger than 128 x 192.)"""
     M, N, K = 64, 128, 136
     A, W, xs, ws, bias = _inputs(60, M, N, K)
     t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
