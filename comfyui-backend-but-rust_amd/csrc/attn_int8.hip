@@ -1103,7 +1103,7 @@ __device__ __forceinline__ float2 load_agent(const float* p, int i) {
 
 // The attention without a key bias, head dims 64 and 128: attn_int8_kernel's arithmetic with the work of two tiles overlapped.
 // It is bound by vector instruction issue (at 4608 tokens x 24 heads of 128: about 470 per wave and tile beside 32 MFMAs; by the
-// counters the vector pipes are busy 58 % of its cycles and the matrix pipes 25 %).
+// counters the vector pipes are busy 69 % of its cycles and the matrix pipes 29 %).
 //   * K runs a tile ahead of V through the two LDS stages: as soon as a key block's probabilities are packed, the next tile's
 //     scores go into its registers, one MFMA behind every fourth of the next block's probabilities; the products with V go
 //     an output block at a time with the fold of the block before between them.  (All scores, then all probabilities, then
@@ -1458,7 +1458,8 @@ struct Plan {
 // merging it, which is 2 to 5 key tiles.  Calls in us, P = 1 and chosen: 4608 tokens x 24 heads 256 -> 231 (96 of 864 row blocks in
 // halves; in fifths 240), 2 x 4096 x 10 x 64 138 -> 115 (128 of 640 in halves), 2500 x 20 x 64 75 -> 64 (thirds; halves 71), 2048 x
 // 10 56 -> 52 (thirds; halves 55), 1024 x 10 45 -> 40.  Splitting every row block of the first costs 263: 57 MB of parts.
-// Fewer than 8 row blocks stay whole: which keys are summed together then depends on nothing but the key tiles.
+// Fewer than 8 row blocks stay whole: which keys are summed together then depends on nothing but the key tiles.  From 8 on it depends on
+// the number of row blocks, so a row's last bits can change with the batch and the head count (its error does not).
 int key_parts(int64_t row_blocks, int64_t kb, int ck, int D, int64_t& whole) {
     constexpr int64_t CUS = 256;   // not the present device's: the workspace's size and the call have to agree
     whole = row_blocks;

@@ -567,9 +567,9 @@ template <int V> struct ic { static constexpr int value = V; };
 // Stamps at 8192 x 2560 -> 640 (256 tiles, us): 2.0 until the first MFMA, 0.53 per step (the MFMAs take 0.37), 2.1 for the epilogue,
 // 1.2 of them with constants and residual loaded where they are used.
 // Against what ran these shapes before (a ring kernel of four waves that fetched for themselves, 128 x 192 tiles; 256 x 96 tiles
-// streaming the weights for up to 256 rows), us, weights from HBM: 8192 x 2560 -> 640 20.1 and 16.2, 2048 x 2048 -> 2048 14.1 and
-// 10.2, 512 x 4096 -> 4096 21.0 and 12.1, 256 x 4096 -> 4096 18.2 and 10.8, 200 x 8192 -> 3072 23.8 and 14.8, 1024 x 4096 -> 9216
-// 41 on the two-group kernel.  The rule is at fed_plan.
+// streaming the weights for up to 256 rows), us, weights from HBM: 8192 x 2560 -> 640 20.5 and 19.0, 2048 x 2048 -> 2048 16.7 and
+// 12.6, 512 x 4096 -> 4096 27.3 and 15.4, 256 x 4096 -> 4096 19.3 and 15.3, 200 x 8192 -> 3072 24.7 and 16.6, 40 x 4096 -> 24576 32.7 and
+// 22.3.  The rule is at fed_plan.
 // ---------------------------------------------------------------------------------------------------------------
 template <int TN_>
 struct FedCfg {
@@ -938,8 +938,8 @@ __global__ void __launch_bounds__(PpL::NT, 1) int8_gemm_pp_kernel(GemmArgs main,
 
 // ---------------------------------------------------------------------------------------------------------------
 // Up to 128 rows: weights straight from HBM into the registers that the matrix instruction reads, rows of A through LDS.  The
-// kernel above moves all 256 rows of A to every CU for 96 columns of W, and what it moves bounds it; with M rows of A in
-// 16-row tiles (MT of them) the weights are most of what a CU takes in.
+// kernel with fetching waves takes weights and A into a CU's LDS through one load path, in tiles of 128 rows; here only the M
+// rows there are, in 16-row tiles (MT of them), go that way, and the weights are most of what a CU takes in.
 //   * Eight waves; a wave owns 16 columns and one of NWK interleaved parts of K, so a workgroup covers 128 / NWK columns
 //     and walks K in panels of 512 * NWK (or 256).  The parts are added through LDS at the end.
 //   * W: a load is 16 columns x 64 bytes, an MFMA operand as it arrives.  Two panels of them are always in flight, each
@@ -947,9 +947,9 @@ __global__ void __launch_bounds__(PpL::NT, 1) int8_gemm_pp_kernel(GemmArgs main,
 //   * A: the panel's rows by DMA into one of two stages, [128-byte column block][8 rows][128 bytes] with the chunk swizzle of
 //     the other kernels on the global side, a panel ahead; one barrier per panel.
 // The wait ahead of that barrier counts: the reissued W loads may stay in flight, the DMA before them may not.
-// Bound by HBM behind 5 us of launch and first trips.  us per call, weights from HBM, the better of the other kernels and this one:
-// 16 rows 1024 -> 1024 8.1 and 5.9, 4096 -> 4096 13.4 and 8.3, 12288 -> 4096 22.1 and 16.7, 4096 -> 16384 26.2 and 20.1; 64 rows
-// 8.3 and 5.2, 14.7 and 11.7, 22.9 and 20.0, 26.8 and 22.9; 128 rows 8.3 and 8.0, 16.1 and 16.4, 25.6 and 23.9, 27.4 and 24.0.
+// Bound by HBM behind 5 us of launch and first trips.  us per call, weights from HBM, the kernel with fetching waves and this one:
+// 16 rows 1024 -> 1024 5.9 and 6.5, 2048 -> 5120 8.1 and 6.6, 4096 -> 4096 10.4 and 8.8, 12288 -> 4096 16.5 and 16.3; 64 rows 2048 -> 4096
+// 8.4 and 8.0, 3072 -> 4096 10.7 and 9.5, 5120 -> 640 9.2 and 8.1; 40 rows 4096 -> 24576 22.3 and 36.3.  The rule is at rows_kernel_wins.
 // Eight steps of 64 per panel where two stages fit the LDS, else four: with NWK = 1 instead, 77 rows take 16.6 instead of 13.8 us
 // for 4096 -> 4096.
 template <int MT, int NWK>   // NWK 2, 4 or 8

@@ -123,7 +123,9 @@ int gpu_w6_requant(const void* weight, void* packed, void* s_rel, void* s_channe
  * keys H4 on runs of four channels only; beyond, H64 at head dim 64, sign diagonal + H128 at 128, H128 on each half at
  * 256.  q/k/v/o: [b, seq, heads, head_dim] through element strides (batch, row, head), bf16 (gpu_int8_attn,
  * gpu_int8_attn_d) or f16 (gpu_int8_attn_f16); h % hk == 0 (grouped-query heads); ws: 256-byte aligned device scratch of
- * gpu_int8_attn_workspace[_d] bytes, layout private to the library.
+ * gpu_int8_attn_workspace[_d] bytes, layout private to the library.  A call gives the same bits every time.  Where the row blocks (128
+ * query rows of a head) of a call are 8 or more, some of them may have their keys summed in parts, by how many there are: the last
+ * bits of a row can then differ between calls of another batch, head count or query length, its error does not.
  * Replaces gpu_int8_attn_workspace_d / gpu_int8_attn_workspace (csrc/attn_int8.cu:62-82), gpu_int8_attn_d (:101-108),
  * gpu_int8_attn_f16 (:111-118), gpu_int8_attn (:225-231); src/ffi.rs binds them under the same names.
  * Returns 0, -400 (argument the library refuses: message on stderr; gpu_int8_attn_workspace_d returns 0 bytes for a
@@ -216,10 +218,13 @@ int gpu_internal_attn_layout_d(int b, int h, int hk, int lq, int lk, int head_di
  * K % 16 == 0 is the fast path; K % 16 == 8 (the reference's alignment-8 tile configurations,
  * csrc/vendor/cutlass_gemm_int8.cu:191,237-247) runs on zero-padded copies of A and W in a stream-ordered allocation
  * (A and W 8-byte aligned); any other K is refused.
- * M <= 256 with long K and few output columns splits K; the int32 planes of the slices go to a 24 MiB buffer that the
- * first such call on a stream allocates (hipMalloc) and the library keeps for that stream.  That first call should be
- * made outside graph capture; under capture, on a ninth stream or on hipStreamPerThread the call uses hipMallocAsync /
- * hipFreeAsync on `stream` instead, as does a shape whose planes exceed the buffer (more than 256 rows). */
+ * A shape whose tiles leave CUs idle while K is long splits K, at any M (16 x 8192 -> 1024, 256 x 8192 -> 4096, 1024 x 5120 -> 320);
+ * gpu_internal_int8_gemm_plan tells which do.  The int32 planes of the slices go to a 24 MiB buffer that the
+ * first such call on a stream allocates (hipMalloc) and the library keeps for that stream; two threads may make such calls on one
+ * stream.  That first call should be made outside graph capture; if it comes under capture, on a ninth stream or on
+ * hipStreamPerThread the call uses hipMallocAsync / hipFreeAsync on `stream` instead.  Under capture K is split only up to 256
+ * rows and for K >= 4096 and 1024 columns or more (up to 16 rows K >= 2560, up to 64 rows and 1280 columns K >= 3072); a graph that
+ * holds such a call holds the buffer of its stream, so replay it there, and not while another thread queues split calls on it. */
 int gpu_int8_gemm(const int8_t* A, const int8_t* W, const float* xs, const float* ws, const void* bias, void* D,
                   int64_t M, int64_t N, int64_t K, int out_dt, void* stream);
 
@@ -251,7 +256,7 @@ int gpu_int8_gemm_acc(const int8_t* A, const int8_t* W, int32_t* acc, int64_t M,
 
 /* gpu_int8_gemm for callers that cannot allocate device memory (code under HIP graph capture, serving loops and
  * harnesses that forbid hipMalloc): same arguments, same results bit for bit, but the int32 planes of a split-K run
- * (M <= 256 with a narrow N) live in a fixed 24 MiB device array inside the library instead of a buffer allocated
+ * (the shapes that split under capture) live in a fixed 24 MiB device array inside the library instead of a buffer allocated
  * for the stream, and the call makes no hipMalloc / hipFree of any kind, first call included.  No counterpart in the reference.
  * Every call on one GPU shares that GPU's array: calls that overlap in time on one GPU (two streams, two threads) race
  * on it and must be serialized by the caller.  Nothing in the array needs clearing between calls (every plane element
