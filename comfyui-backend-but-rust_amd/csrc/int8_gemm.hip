@@ -1499,23 +1499,31 @@ int launch_rows(GemmArgs a, hipStream_t st) {
 
 // Whether the kernel for up to 128 rows runs a shape.  For outputs of whole 16 bytes: up to 64 rows and 8192 columns, from the K on
 // from which it is faster than the kernel with fetching waves up to where that one splits K better.  Its time over the other's by
-// 1500 shapes with weights from HBM, calls in a row:
-//   1 to 16 rows: 0.73 to 0.96 from K = 1408 to 4600, 0.85 to 1.1 above, 1.04 and more below.  Beyond 8192 columns, where it takes one more
-//     round: 0.91 up to K = 1920, 1.06 to 1.13 up to 3300, 0.81 to 1.07 above (from 9 rows on only up to 10240), but 1.03 to 1.25 there
-//     where weight rows are whole 4 KB (from 9 rows on: whole KB), which the other kernel's staggered starts suit.
-//   17 to 32: 0.77 to 0.99 from K = 1920 to 4096; above, 0.81 to 1.04 with few columns and 1.0 to 1.3 with many.
-//   33 to 64: 0.88 to 1.0 from K = 1024 to 2304 and 0.84 to 0.93 above 2816, but 1.0 to 1.16 between with few columns (its panels of 1024 end half empty).
+// 6000 shapes with weights from HBM, calls in a row:
+//   1 to 16 rows: 0.6 to 0.98 from K = 1408 to 4000, 0.6 to 1.1 above (1.05 to 1.3 for 1280 to 2048 columns from K = 8192 on), 1.0 and
+//     more below.  Beyond 8192 columns, where it takes one more round: 0.91 up to K = 1920, 1.06 to 1.13 up to 3300, 0.8 to 1.07 above (from
+//     9 rows on also 1.04 to 1.11 up to 9500 columns from K = 10240 on), but 0.9 to 1.2 there where weight rows are whole 4 KB (from 9 rows
+//     on: whole 2 KB), which the other kernel's staggered starts suit.
+//   17 to 32: 0.77 to 1.0 from K = 1920 to 4096.  Above, 0.81 to 1.15 up to 1280 columns; 1.0 to 1.45 from there to 5120, where this kernel
+//     splits K over workgroups too or leaves CUs without one; 0.76 to 1.05 beyond (from K = 8192 on: beyond 6144), where its 160 to 256
+//     workgroups take all of K and the other kernel has planes to add.
+//   33 to 64: 0.88 to 1.0 from K = 1024 to 2304 and 0.84 to 1.0 from 2816 to 4096, but 1.0 to 1.16 between with few columns (its panels of
+//     1024 end half empty) and from 3072 to 4096 columns above K = 3584.  From K = 4096 on 0.8 to 1.0 up to 1280 columns, 1.0 to 1.38 from
+//     there to 6144, 0.85 to 1.08 beyond, up to K = 10240.
 //   65 to 128: 1.0 to 1.6.
 // Other outputs have the register-staged tiles beside them, which have less to start (128 rows 1152 -> 512 8.5 and 7.5 us; but 128
 // rows 1280 -> 640 8.5 and 9.2).
 bool rows_kernel_wins(int64_t M, int64_t N, int64_t K, bool aligned) {
     if (aligned && M <= 16) {
         if (N <= 8192) return K >= 1408;
-        return N <= 16384 && K >= 1408 && (K <= 1920 || (K >= 3328 && (M <= 8 ? K % 4096 != 0 : K <= 10240 && K % 1024 != 0)));
+        return N <= 16384 && K >= 1408 && (K <= 1920 || (K >= 3328 && (M <= 8 ? K % 4096 != 0 : K % 2048 != 0 && (K <= 10240 || N > 9500))));
     }
-    if (aligned && M <= 32) return N <= 8192 && ((K >= 1920 && K <= 4096) || (K > 4096 && N <= 1280));
-    if (aligned && M <= 64)
-        return N <= 8192 && ((K >= 1024 && K <= 2304) || (K > 2816 && K <= 3584) || (K > 2304 && K <= 2816 && N > 3072) || (K > 3584 && N <= (K <= 4608 ? 3072 : 1280)));
+    if (aligned && M <= 32) return N <= 8192 && K >= 1920 && (K <= 4096 || N <= 1280 || N > (K < 8192 ? 5120 : 6144));
+    if (aligned && M <= 64) {
+        if (N > 8192 || K < 1024) return false;
+        if (K <= 3584) return K <= 2304 || K > 2816 || N > 3072;
+        return K < 4096 ? N <= 3072 || N > 4096 : N <= 1280 || (N > 6144 && K <= 10240);
+    }
     if (aligned) return false;
     if (K < (M > 96 ? 1024 : 768) || (M > 16 && N > 16384)) return false;
     if (K < 896) return !(N < 1152 && (M <= 32 || M > 64));

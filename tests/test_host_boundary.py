@@ -320,9 +320,10 @@ def test_gemm_operands_off_16_bytes_keep_the_kernels_that_take_them():
 
 def test_gemm_choice_where_it_was_measured():
     """Shapes at which one kernel, or another number of slices of K, was timed at least 8 % faster than the others with weights from HBM."""
-    for M, N, K in [(1, 5120, 2048), (16, 8192, 2048), (4, 1280, 4096), (17, 3072, 3072), (32, 2048, 3072), (64, 2048, 2048), (48, 5120, 3072), (64, 640, 5120), (1, 12552, 3968), (1, 10240, 5120)]:
+    for M, N, K in [(1, 5120, 2048), (16, 8192, 2048), (4, 1280, 4096), (17, 3072, 3072), (32, 2048, 3072), (64, 2048, 2048), (48, 5120, 3072), (64, 640, 5120), (1, 12552, 3968), (1, 10240, 5120), (20, 7520, 6144), (17, 7304, 13312), (21, 5384, 7808),
+                    (41, 7376, 3712), (44, 5184, 3840), (56, 7816, 4992), (35, 7880, 9216), (11, 15688, 13312)]:
         assert gemm_plan(M, N, K)[0] == 5, (M, N, K)
-    for M, N, K in [(8, 4096, 640), (16, 24576, 4096), (17, 9216, 2048), (32, 6144, 8192), (64, 1280, 2560), (65, 1280, 2048), (128, 4096, 3072)]:
+    for M, N, K in [(8, 4096, 640), (16, 24576, 4096), (17, 9216, 2048), (22, 3072, 6144), (35, 2952, 4224), (41, 1760, 4224), (60, 4096, 8192), (64, 1280, 2560), (65, 1280, 2048), (128, 4096, 3072)]:
         assert gemm_plan(M, N, K)[0] == 7, (M, N, K)
     for M, N, K in [(128, 3072, 5120), (96, 640, 2560), (256, 1280, 5120), (256, 8448, 12288), (512, 640, 5120), (1024, 320, 5120)]:
         family, _, slices = gemm_plan(M, N, K)
