@@ -1451,11 +1451,29 @@ struct Plan {
     int ck, kb, qg, nblk, parts;
 };
 
+// What `parts` workgroups per row block of the tail take off a call, in us: the key tiles that a CU has less to go through, minus a fixed
+// cost, one per part and one for the CUs that write parts at the same time.  Fitted to 1300 calls of 256 to 5000 keys against the same
+// calls unshared, within about 1 us; of 800 others 77 took more than 3 % longer shared by the relative costs alone, with this 3.  It leaves few keys unshared, where the relative costs of key_parts see a gain:
+// 2 x 492 x 9 x 128 31.8 us unshared and 37.0 in halves, 516 x 20 x 128 35.0 and 38.4, 602 x 19 x 64 27.0 and 28.8.  1849 queries, 877
+// keys x 2 x 128 stay in thirds (36.6 and 33.5), 2 x 300 queries, 1859 keys x 15 x 64 in fifths (51.9 and 45.4).
+double parts_gain_us(int64_t tail, int64_t kb, int ck, int D, bool lone, int parts) {
+    struct Cost { double tile, fixed, part, busy; };
+    static constexpr Cost c[3][2] = {{{1.06, -0.3, 2.2, 4.0}, {0.77, 2.35, 0.47, 0.54}},    // head dim 64; [1]: behind whole row blocks
+                                     {{1.75, -2.4, 4.85, 5.5}, {1.4, 0.4, 2.8, 1.7}},       // 128 with tiles of 64 keys
+                                     {{1.66, 0.83, 1.73, 3.1}, {1.34, -2.0, 1.32, 5.0}}};   // and of 128
+    const Cost& k = c[D == 64 ? 0 : ck == 64 ? 1 : 2][lone ? 0 : 1];
+    const double busy = (double)(tail * parts) / 256.;
+    const int n = (int)((tail * parts + 255) / 256);   // parts of the busiest CU
+    // their time, of a part that has a CU for itself: two at once 1.6 to 1.7; of head dim 128 only two fit, and a third gains nothing
+    const double time = !lone ? n : n == 1 ? 1. : D == 64 ? n - 0.43 : n == 2 ? 1.7 : n + 1.;
+    return k.tile * (double)kb * (1. - time / parts) - (k.fixed + k.part * parts + k.busy * (lone && busy > 1. ? 1. : busy));
+}
+
 // How the pipelined kernel's row blocks (128 rows of a head) go to the CUs.  What is left over a multiple of the CUs keeps some of them
 // busy for a whole row block's time, 55 us at 4608 keys, while the others idle; the keys of those row blocks are shared by P
 // workgroups each.  P is what leaves a CU the least, in row blocks: ceil(tail * P / CUs) parts of 1 / P each (a part alone on a CU
 // takes 1.3 times as long: 125 us for a row block of 8192 keys, 196 for two at once), plus about 3 us per part for writing and
-// merging it, which is 2 to 5 key tiles.  Calls in us, P = 1 and chosen: 4608 tokens x 24 heads 256 -> 231 (96 of 864 row blocks in
+// merging it, which is 2 to 5 key tiles; and parts_gain_us has to see a gain.  Calls in us, P = 1 and chosen: 4608 tokens x 24 heads 256 -> 231 (96 of 864 row blocks in
 // halves; in fifths 240), 2 x 4096 x 10 x 64 138 -> 115 (128 of 640 in halves), 2500 x 20 x 64 75 -> 64 (thirds; halves 71), 2048 x
 // 10 56 -> 52 (thirds; halves 55), 1024 x 10 45 -> 40.  Splitting every row block of the first costs 263: 57 MB of parts.
 // Fewer than 8 row blocks stay whole: which keys are summed together then depends on nothing but the key tiles.  From 8 on it depends on
@@ -1473,7 +1491,8 @@ int key_parts(int64_t row_blocks, int64_t kb, int ck, int D, int64_t& whole) {
         const double n = (double)((tail * p + CUS - 1) / CUS), cost = (lone && n == 1 ? 1.3 : n) / p + n * merge;
         if (cost < least) { least = cost - 0.05; best = p; }
     }
-    if (best > 1) whole = row_blocks - tail;
+    if (best == 1 || parts_gain_us(tail, kb, ck, D, lone, best) < 0.15) return 1;
+    whole = row_blocks - tail;
     return best;
 }
 

@@ -333,3 +333,16 @@ def test_gemm_choice_where_it_was_measured():
         assert family == 7 and slices == 1, (M, N, K, slices)
     for M, N, K in [(4608, 3072, 3072), (8192, 5120, 640), (1024, 9216, 4096), (5366, 3144, 128)]:
         assert gemm_plan(M, N, K)[0] == 9, (M, N, K)
+
+
+@pytest.mark.parametrize("b,h,lq,lk,d,shared", [(2, 9, 492, 492, 128, False), (1, 20, 516, 516, 128, False), (1, 19, 602, 602, 64, False), (2, 11, 356, 560, 128, False),
+                                                (1, 21, 686, 686, 64, False), (1, 11, 640, 640, 128, False), (2, 6, 1029, 539, 64, False), (1, 2, 1849, 877, 128, True),
+                                                (2, 15, 300, 1859, 64, True), (1, 10, 1024, 1024, 128, True), (1, 24, 4608, 4608, 128, True), (2, 10, 4096, 4096, 64, True)])
+def test_attention_shares_keys_where_that_was_measured_faster(b, h, lq, lk, d, shared):
+    """A workspace that ends with the column sums of V has no room for parts: no row block's keys are shared."""
+    out = (ctypes.c_int64 * 10)()
+    assert ffi.raw("gpu_internal_attn_layout_d", b, h, h, lq, lk, d, ctypes.cast(out, ctypes.c_void_p)) == 0
+    vsum, kb = out[7], out[9]
+    plain = vsum + (b * h * kb * d * 4 + 255) // 256 * 256
+    total = ffi.lib.gpu_int8_attn_workspace_d(b, h, h, lq, lk, d)
+    assert (total > plain) == shared and total >= plain
