@@ -233,13 +233,19 @@ __global__ void __launch_bounds__(1024) w6_requant_kernel(const uint16_t* w, uin
 // Rows of a workgroup: one, or as many more as give the CUs clearly fewer waves to run: all of a workgroup's, however few lanes its
 // last has, times the workgroups of the busiest CU.  us, one row and the rows chosen: 5376 x 5376 66.6 and 56.4 (three), 4096 x 1280
 // 20.3 and 15.9 (four), 8192 x 256 19.4 and 10.9 (four), 4096 x 1536 19.1 and 16.5 (two); within 6 % the larger workgroups
-// lose by their barriers (4096 x 7680 59.7 and, two rows in 15 waves, 64.3).
+// lose by their barriers (4096 x 7680 59.7 and, two rows in 15 waves, 64.3).  With up to three workgroups per CU a SIMD waits for its
+// own waves: a workgroup's go to the four SIMDs from the first on, so that two workgroups of two waves meet on the same two SIMDs and
+// one of four does not (448 x 2048 8.1 and 6.9, 453 x 5120 10.9 and 9.9; 1400 shapes: 19 more than 4 % slower than with fixed rows, with this 5).
 int rows_per_group(int64_t N, int groups) {
-    const int cus = device_cu_count();
-    const auto waves = [&](int r) { return (double)(((N + r - 1) / r + cus - 1) / cus) * ((r * groups + 3) / 4); };
+    const int64_t cus = device_cu_count();
+    const auto wgs = [&](int r) { return ((N + r - 1) / r + cus - 1) / cus; };   // of the busiest CU
+    const auto waves = [&](int r) { return (double)wgs(r) * ((r * groups + 3) / 4); };
+    const auto on_simd = [&](int r) { return wgs(r) * ((r * groups + 15) / 16); };
     int best = 1;
     for (int r = 2; r <= kMaxRows && r * groups <= 64; ++r)
         if (waves(r) < 0.92 * waves(best)) best = r;
+    for (int r = 2; r <= kMaxRows && r * groups <= 64; ++r)
+        if (wgs(best) <= 3 && waves(r) <= waves(best) && on_simd(r) < on_simd(best)) best = r;
     return best;
 }
 
@@ -271,4 +277,10 @@ GPU_API int gpu_w6_requant(const void* weight, void* packed, void* s_rel, void* 
     if (chunks > 32) return launch_requant<3>(weight, packed, s_rel, s_channel, (int)N, K, seed, 1, st);
     if (chunks > 16) return launch_requant<2>(weight, packed, s_rel, s_channel, (int)N, K, seed, 1, st);
     return launch_requant<1>(weight, packed, s_rel, s_channel, (int)N, K, seed, rows_per_group(N, groups), st);
+}
+
+// Test hook: rows of a workgroup of gpu_w6_requant.
+GPU_API int gpu_internal_w6_requant_rows(int64_t N, int K) {
+    if (N <= 0 || K <= 0 || (K % 256) != 0 || K > 39680) return -1;
+    return K > 16 * convrot::kChunk ? 1 : rows_per_group(N, K / 256);
 }

@@ -115,6 +115,9 @@ int gpu_convrot_requant(int dtype, const void* x, void* q, void* s, int64_t N, i
  * K % 256 (-1), K <= 39 680 (-2). */
 int gpu_w6_requant(const void* weight, void* packed, void* s_rel, void* s_channel, int64_t N, int K, uint64_t seed,
                    void* stream);
+/* Test hook, no reference counterpart: how many rows share a workgroup of that call; -1 for sizes it refuses.  Without a
+ * device it answers for 256 CUs. */
+int gpu_internal_w6_requant_rows(int64_t N, int K);
 
 /* INT8 attention, head dims 64, 128 and 256: o = softmax(q . k^T * scale) . v with q and k rotated and quantized per
  * scale group (eight groups per block of 32 query rows, 16 at head dim 256; four per key tile), an optional K anchor

@@ -346,3 +346,14 @@ def test_attention_shares_keys_where_that_was_measured_faster(b, h, lq, lk, d, s
     plain = vsum + (b * h * kb * d * 4 + 255) // 256 * 256
     total = ffi.lib.gpu_int8_attn_workspace_d(b, h, h, lq, lk, d)
     assert (total > plain) == shared and total >= plain
+
+
+def test_w6_requant_rows_of_a_workgroup_where_they_were_measured():
+    """Row counts that took 5 % and more off the other choices."""
+    for N, K, rows in [(448, 2048, 2), (318, 2048, 2), (405, 1792, 2), (299, 4864, 2), (453, 5120, 2), (5376, 5376, 3), (4096, 1280, 4), (8192, 256, 4), (4096, 1536, 2), (4096, 7680, 1)]:
+        assert ffi.raw("gpu_internal_w6_requant_rows", N, K) == rows, (N, K)
+    for N in (1, 64, 300, 1000, 2276, 3127, 12288, 24576):
+        for K in range(256, 39680 + 1, 256):
+            rows = ffi.raw("gpu_internal_w6_requant_rows", N, K)
+            assert 1 <= rows <= 16 and (rows == 1 or rows * K <= 16384), (N, K, rows)   # what its LDS array and 16 waves hold
+    assert ffi.raw("gpu_internal_w6_requant_rows", 4, 300) == -1
