@@ -1453,9 +1453,10 @@ struct Plan {
 
 // What `parts` workgroups per row block of the tail take off a call, in us: the key tiles that a CU has less to go through, minus a fixed
 // cost, one per part and one for the CUs that write parts at the same time.  Fitted to 1300 calls of 256 to 5000 keys against the same
-// calls unshared, within about 1 us; of 800 others 77 took more than 3 % longer shared by the relative costs alone, with this 3.  It leaves few keys unshared, where the relative costs of key_parts see a gain:
-// 2 x 492 x 9 x 128 31.8 us unshared and 37.0 in halves, 516 x 20 x 128 35.0 and 38.4, 602 x 19 x 64 27.0 and 28.8.  1849 queries, 877
-// keys x 2 x 128 stay in thirds (36.6 and 33.5), 2 x 300 queries, 1859 keys x 15 x 64 in fifths (51.9 and 45.4).
+// calls unshared, within about 1 us; of 800 others 77 took more than 3 % longer shared by the relative costs of key_parts alone, with
+// this 3.  It leaves few keys unshared where those see a gain: 2 x 492 x 9 x 128 31.8 us unshared and 37.0 in halves, 516 x 20 x 128 35.0
+// and 38.4, 602 x 19 x 64 27.0 and 28.8.  1849 queries, 877 keys x 2 x 128 stay in thirds (36.6 and 33.5), 2 x 300 queries, 1859 keys x
+// 15 x 64 in fifths (51.9 and 45.4).
 double parts_gain_us(int64_t tail, int64_t kb, int ck, int D, bool lone, int parts) {
     struct Cost { double tile, fixed, part, busy; };
     static constexpr Cost c[3][2] = {{{1.06, -0.3, 2.2, 4.0}, {0.77, 2.35, 0.47, 0.54}},    // head dim 64; [1]: behind whole row blocks
