@@ -1372,22 +1372,34 @@ FedPlan fed_plan(int64_t M, int64_t N, int64_t K, int num_cu, bool may_split) {
     // fixed, per round, per step, per step with 128 rows, per step and round after the first
     static constexpr double c[3][5] = {{0.89, 2.20, 0.30, 0.07, 0.35}, {1.02, 3.12, 0.50, 0.01, 0.43}, {-0.69, 4.99, 0.89, -0.20, 0.63}};
     const int steps = (int)(K / 128), cus = num_cu;
-    const double rows = M < 128 ? (double)M / 128. : 1.;
+    const double rows = M < 128 ? (double)M / 128. : 1., hbm = (double)N * (double)K / 32490., plane = 0.05 + (double)M * (double)N * 1.69e-6;
     FedPlan best{3, 1, (int)K, 1e30};
     for (int w = 1; w <= 3; ++w) {
-        const int64_t all = ((M + 127) / 128) * ((N + 64 * w - 1) / (64 * w));
+        const int64_t all = (M + 127) / 128 * ((N + 64 * w - 1) / (64 * w));
         const int tiles = all < 1 << 24 ? (int)all : 1 << 24;
-        const int most = !may_split ? 1 : cus / tiles < steps / 3 ? cus / tiles : steps / 3;
+        const double* k = c[w - 1];
+        const double step = k[2] + rows * k[3];
+        if (tiles * 2 > cus || !may_split || steps < 6) {   // nothing to split
+            const double n = (double)((tiles + cus - 1) / cus), trip = 3.86 + hbm / (tiles < cus ? tiles : cus);
+            double us = k[0] + n * k[1] + (step + (n - 1.) * k[4]) * steps + (w == 3 && N % 64 != 0 ? 1.6 * n : 0.);
+            if (us < trip) us = trip;
+            if (us < best.us) best = {w, 1, steps * 128, us};
+            continue;
+        }
+        // no more tiles than CUs: one round, however K is split
+        const int most = cus / tiles < steps / 3 ? cus / tiles : steps / 3;
+        const double fixed = k[0] + k[1] + (w == 3 && N % 64 != 0 ? 1.6 : 0.), per_tile = hbm / tiles;
+        int before = 0;
         for (const int asked : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24}) {
-            if (asked > 1 && asked > most) break;
-            const int per = (steps + asked - 1) / asked, s = (steps + per - 1) / per;   // no empty slice
-            const int busy = tiles * s < cus ? tiles * s : cus;
-            const double n = (double)((tiles * s + cus - 1) / cus);
-            double us = c[w - 1][0] + n * c[w - 1][1] + (c[w - 1][2] + rows * c[w - 1][3] + (n - 1.) * c[w - 1][4]) * per;
-            if (w == 3 && N % 64 != 0) us += 1.6 * n;
-            if (s > 1) us += 3.4 + (double)s * (0.05 + (double)M * (double)N * 1.69e-6) + (per % 8 == 0 ? 0.29 : 0.);
-            const double hbm = 3.86 + (double)N * (double)K / (32490. * busy);
-            if (us < hbm) us = hbm;
+            if (asked > most) break;
+            const int per = (steps + asked - 1) / asked;
+            if (per == before) continue;
+            before = per;
+            const int s = per * (asked - 1) < steps ? asked : (steps + per - 1) / per;   // no empty slice
+            const double trip = 3.86 + per_tile / s;
+            double us = fixed + step * per;
+            if (s > 1) us += 3.4 + s * plane + (per % 8 == 0 ? 0.29 : 0.);
+            if (us < trip) us = trip;
             if (us < best.us) best = {w, s, per * 128, us};
         }
     }

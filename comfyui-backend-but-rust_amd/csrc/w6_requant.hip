@@ -237,16 +237,23 @@ __global__ void __launch_bounds__(1024) w6_requant_kernel(const uint16_t* w, uin
 // own waves: a workgroup's go to the four SIMDs from the first on, so that two workgroups of two waves meet on the same two SIMDs and
 // one of four does not (448 x 2048 8.1 and 6.9, 453 x 5120 10.9 and 9.9; 1400 shapes: 19 more than 4 % slower than with fixed rows, with this 5).
 int rows_per_group(int64_t N, int groups) {
-    const int64_t cus = device_cu_count();
-    const auto wgs = [&](int r) { return ((N + r - 1) / r + cus - 1) / cus; };   // of the busiest CU
-    const auto waves = [&](int r) { return (double)wgs(r) * ((r * groups + 3) / 4); };
-    const auto on_simd = [&](int r) { return wgs(r) * ((r * groups + 15) / 16); };
-    int best = 1;
-    for (int r = 2; r <= kMaxRows && r * groups <= 64; ++r)
-        if (waves(r) < 0.92 * waves(best)) best = r;
-    for (int r = 2; r <= kMaxRows && r * groups <= 64; ++r)
-        if (wgs(best) <= 3 && waves(r) <= waves(best) && on_simd(r) < on_simd(best)) best = r;
-    return best;
+    const uint32_t cus = (uint32_t)device_cu_count(), rows = (uint32_t)N;
+    struct Choice { int r; uint32_t wgs; double waves; uint32_t on_simd; };   // wgs: of the busiest CU
+    const auto choice = [&](int r) {
+        const uint32_t wgs = ((rows + r - 1) / r + cus - 1) / cus;
+        return Choice{r, wgs, (double)wgs * ((r * groups + 3) / 4), wgs * ((r * groups + 15) / 16)};
+    };
+    const int most = 64 / groups < kMaxRows ? 64 / groups : kMaxRows;
+    Choice best = choice(1);
+    for (int r = 2; r <= most; ++r) {
+        const Choice c = choice(r);
+        if (c.waves < 0.92 * best.waves) best = c;
+    }
+    for (int r = 2; r <= most && best.wgs <= 3; ++r) {
+        const Choice c = choice(r);
+        if (c.waves <= best.waves && c.on_simd < best.on_simd) best = c;
+    }
+    return best.r;
 }
 
 template <int C>
@@ -281,6 +288,6 @@ GPU_API int gpu_w6_requant(const void* weight, void* packed, void* s_rel, void* 
 
 // Test hook: rows of a workgroup of gpu_w6_requant.
 GPU_API int gpu_internal_w6_requant_rows(int64_t N, int K) {
-    if (N <= 0 || K <= 0 || (K % 256) != 0 || K > 39680) return -1;
+    if (N <= 0 || N > 0x7fffffff || K <= 0 || (K % 256) != 0 || K > 39680) return -1;
     return K > 16 * convrot::kChunk ? 1 : rows_per_group(N, K / 256);
 }
