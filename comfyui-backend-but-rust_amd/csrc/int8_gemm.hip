@@ -41,6 +41,7 @@ struct GemmArgs {
     int tiles_m, tiles_n;
     uint32_t magic;   // panel_magic(tiles_m, tiles_n), for tile_of_block
     int kslice;   // K of a split-K slice (a multiple of 128), 0 = no split
+    int n_first;  // two-group kernel: the first column of these tiles
 };
 
 template <int BM_, int BN_, int BK_, int WGM_, int WGN_, int OCC_>
@@ -722,9 +723,9 @@ __global__ void __launch_bounds__(512, 1) int8_gemm_fed_kernel(GemmArgs p) {
 // with group 0 multiplying.
 // Requires K % 128 == 0, M*K and N*K < 2^32, and the coalesced epilogue's alignment.
 // ---------------------------------------------------------------------------------------------------------------
-// GM: rows of a group.  128 gives the 256x256 tile (wave tiles 128x64); 64 gives a 128x256 tile (wave tiles 64x64) for
-// the rows a whole number of rounds of the large tile leaves over: half the work per tile, so the last, partly filled
-// round costs half as much, at a step that is bound by its 6 DMA instructions per wave rather than by its 16 MFMAs.
+// GM: rows of a group.  128 gives the 256x256 tile (wave tiles 128x64), 96 a 192x256 tile, 64 a 128x256 tile (wave tiles 64x64):
+// half the work per tile, at a step that is bound by its 6 DMA instructions per wave rather than by its 32 MFMAs.  pp_split
+// says which run.
 template <int GM_>
 struct PpCfg {
     static constexpr int GM = GM_, BM = 2 * GM, BN = 256, BK = 128, NT = 512;
@@ -737,6 +738,7 @@ struct PpCfg {
     static constexpr int piece_cols(int sz) { return sz == 2 ? 64 : 32; }           // 4 KB shuffle pieces
 };
 using PpL = PpCfg<128>;
+using PpM = PpCfg<96>;
 using PpS = PpCfg<64>;
 
 // The work of workgroup `bid` of `G` on problem p.
@@ -754,7 +756,7 @@ __device__ __forceinline__ void pp_gemm_tiles(const GemmArgs& p, uint8_t* smem, 
         int tm, tn;
         tile_of_block(bid + i * G, ntiles, p.tiles_m, p.tiles_n, tm, tn, p.magic);
         m0 = tm * C::BM;
-        n0 = tn * C::BN;
+        n0 = p.n_first + tn * C::BN;
     };
     const uint32_t lds_base = (uint32_t)(uintptr_t)smem;
     auto dma = [&](uint32_t dst, uint32_t off, const int8_t* base) {
@@ -925,14 +927,14 @@ __device__ __forceinline__ void pp_gemm_tiles(const GemmArgs& p, uint8_t* smem, 
     wait_vmcnt<0>();   // no DMA may still be writing this workgroup's LDS when it retires
 }
 
-// Workgroups 0 .. g_main-1 walk the 256x256 tiles of `main`; the rest walk the 128x256 tiles of `rest` (the rows that
-// whole rounds of large tiles leave over, or nothing).  One launch: the hardware starts a workgroup of the second kind
+// Workgroups 0 .. g_main-1 walk the tiles of `main`; the others walk the 128x256 tiles of `rest` (the rows or columns that
+// whole rounds of large tiles leave over, everything, or nothing).  One launch: the hardware starts a workgroup of the second kind
 // on each CU as its workgroup of the first kind retires, with no gap between two launches.
-template <int OUT_DT, int EPI>
+template <class Main, int OUT_DT, int EPI>
 __global__ void __launch_bounds__(PpL::NT, 1) int8_gemm_pp_kernel(GemmArgs main, GemmArgs rest, int g_main) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int bid = (int)blockIdx.x;
-    if (bid < g_main) pp_gemm_tiles<PpL, OUT_DT, EPI>(main, smem, bid, g_main);
+    if (bid < g_main) pp_gemm_tiles<Main, OUT_DT, EPI>(main, smem, bid, g_main);
     else pp_gemm_tiles<PpS, OUT_DT, EPI>(rest, smem, bid - g_main, (int)gridDim.x - g_main);
 }
 
@@ -1147,6 +1149,12 @@ __global__ void __launch_bounds__(256) splitk_epilogue_kernel(GemmArgs p, const 
 using CfgM = Cfg<128, 128, 64, 2, 2, 2>;
 using CfgS = Cfg<64, 64, 64, 2, 2, 4>;
 
+// Kernel family forced by the test hook (-1 = choose by shape), or 7000 + 100 * width + slices: the kernel with fetching waves on
+// tiles of 64 * width columns and so many slices of K, or 9000 + 10 * kind + split: the two-group kernel (kind: 256, 192 or 128
+// rows; split: none, rows, columns).  Process-wide and only meant for tests and benchmarks:
+// relaxed atomic, so a concurrent call sees either the old or the new value, never a torn one.
+std::atomic<int> g_force_cfg{-1};
+
 template <class C, int OUT_DT, int EPI>
 int launch_cfg(GemmArgs a, hipStream_t st) {
     a.tiles_m = (a.M + C::BM - 1) / C::BM;
@@ -1177,52 +1185,84 @@ GemmArgs row_band(const GemmArgs& a, int64_t row0, int64_t rows) {
     return b;
 }
 
-// Large shapes on the two-group kernel.  Every CU gets whole 256x256 tiles; when the tile count is not a multiple of the
-// CU count, the last round would keep only some CUs busy for a full tile's time (864 tiles on 256 CUs: 96 busy, 160
-// idle, a sixth of the run).  The tile rows that fill whole rounds are then run as 256x256 tiles and the rows left over
-// as 128x256 tiles by further workgroups of the same launch, when that is estimated to be shorter (a small tile costs
-// about 0.6 of a large one).
-struct PpSplit { int64_t main_rows, small; double rounds; };   // tile rows of large tiles, small tiles behind them, rounds of large tiles in all
+// Large shapes on the two-group kernel.  A launch takes whole rounds of one tile per CU, and what counts is how little of the last
+// round is idle: tiles of 256, 192 or 128 rows by 256 columns, and where the tiles of 256 or 192 rows fill whole rounds and some
+// more, the tile rows or tile columns that fill the whole ones, with the rest as 128 x 256 tiles by further workgroups of the same
+// launch.  The smallest sum of rounds runs, a round of the smaller tiles counted as 0.78 and 0.67 of one of 256 rows: three
+// quarters and half of the work, but a step of theirs is bound by its DMA instructions.  (kCost is what chose best over 260 shapes of 512 to
+// 8192 rows timed in all seven forms, 0.8 % slower than the best of them; 256-row tiles with rows left over alone 7.1 %.)  us, those and
+// the present choice: 2048 x 14336 -> 5376 145 and 125 (192 rows: 231 tiles instead of 168), 3000 x 2048 -> 7168 46 and 42,
+// 6000 x 1024 -> 3072 29 and 25, 8192 x 640 -> 5120 38.7 and 38.1 (columns left over; bound by the chip's writes beside the MFMAs).
+struct PpSplit {
+    int rows;                          // of a tile of the first kind: 256 or 192; 128: there are only tiles of the second
+    int64_t main_tm, main_tn, small;   // the grid of those tiles, and how many of the second kind
+    bool columns;                      // the second kind takes the columns that are left, not the rows
+    double rounds;                     // rounds of 256 x 256 tiles in all
+};
 PpSplit pp_split(int64_t M, int64_t N, int64_t cus) {
-    const int64_t tm = (M + PpL::BM - 1) / PpL::BM, tn = (N + PpL::BN - 1) / PpL::BN, full = tm * tn / cus, rem = tm * tn % cus;
-    const PpSplit whole{tm, 0, (double)(full + (rem > 0))};
-    if (full < 1 || rem == 0 || tm < 2) return whole;
-    const int64_t main_rows = full * cus / tn < tm ? full * cus / tn : tm - 1;
-    const int64_t small = ((M - main_rows * PpL::BM + PpS::BM - 1) / PpS::BM) * tn;
-    const double cost = (double)((main_rows * tn + cus - 1) / cus) + 0.6 * (double)((small + cus - 1) / cus);
-    return main_rows > 0 && cost < (double)(full + 1) - 0.1 ? PpSplit{main_rows, small, cost} : whole;
+    static constexpr double kCost[3] = {1.0, 0.78, 0.67};
+    const int64_t tn = (N + 255) / 256;
+    const auto rounds = [&](int64_t tiles) { return (double)((tiles + cus - 1) / cus); };
+    const int force = g_force_cfg.load(std::memory_order_relaxed) - 9000;
+    PpSplit best{256, 0, 0, 0, false, 1e30};
+    for (int kind = 0; kind < 3; ++kind) {
+        if (force >= 0 && force < 30 && kind != force / 10) continue;
+        const int bm = 256 - 64 * kind;
+        const int64_t tm = (M + bm - 1) / bm, full = tm * tn / cus;
+        const double whole = kCost[kind] * rounds(tm * tn);
+        PpSplit form[3] = {kind == 2 ? PpSplit{bm, 0, 0, tm * tn, false, whole} : PpSplit{bm, tm, tn, 0, false, whole}, best, best};
+        int forms = 1;
+        if (kind < 2 && full >= 1 && tm > 1 && tn > 1 && tm * tn % cus != 0) {
+            const int64_t rows = full * cus / tn < tm ? full * cus / tn : tm - 1, cols = full * cus / tm < tn ? full * cus / tm : tn - 1;
+            const int64_t by_rows = (M - rows * bm + 127) / 128 * tn, by_cols = (M + 127) / 128 * (tn - cols);
+            form[1] = {bm, rows, tn, by_rows, false, rows > 0 ? kCost[kind] * rounds(rows * tn) + kCost[2] * rounds(by_rows) : 1e30};
+            form[2] = {bm, tm, cols, by_cols, true, cols > 0 ? kCost[kind] * rounds(tm * cols) + kCost[2] * rounds(by_cols) : 1e30};
+            forms = 3;
+        }
+        if (force >= 0 && force < 30) return form[force % 10 < forms ? force % 10 : 0];
+        for (int i = 0; i < forms; ++i)
+            if (form[i].rounds < best.rounds - 0.005) best = form[i];
+    }
+    return best;
 }
 
-template <int OUT_DT, int EPI>
-int launch_pp(GemmArgs a, hipStream_t st) {
-    bool vec_ok, aligned;
-    epilogue_alignment<OUT_DT, EPI>(a, vec_ok, aligned);
-    if (!aligned) return launch_cfg<CfgM, OUT_DT, EPI>(a, st);   // this kernel has only the coalesced epilogue
-    const int64_t G = device_cu_count();
-    const int64_t tn = (a.N + PpL::BN - 1) / PpL::BN;
-    const PpSplit sp = pp_split(a.M, a.N, G);
-    GemmArgs main = a, rest = a;
-    const int64_t n_main = sp.main_rows * tn, n_rest = sp.small;
-    if (n_rest) {
-        main = row_band<OUT_DT, EPI>(a, 0, sp.main_rows * PpL::BM);
-        rest = row_band<OUT_DT, EPI>(a, sp.main_rows * PpL::BM, a.M - sp.main_rows * PpL::BM);
-    }
-    if (n_main > 0x7fffffff) return -1;
-    main.tiles_m = (main.M + PpL::BM - 1) / PpL::BM;
-    main.tiles_n = (int)tn;
-    rest.tiles_m = (rest.M + PpS::BM - 1) / PpS::BM;
-    rest.tiles_n = (int)tn;
-    main.magic = panel_magic(main.tiles_m, main.tiles_n);
-    rest.magic = panel_magic(rest.tiles_m, rest.tiles_n);
-    const int g_main = (int)(n_main < G ? n_main : G), g_rest = (int)(n_rest < G ? n_rest : G);
-    auto kern = int8_gemm_pp_kernel<OUT_DT, EPI>;
+template <class Main, int OUT_DT, int EPI>
+int launch_pp_as(const GemmArgs& main, const GemmArgs& rest, int g_main, int g_rest, hipStream_t st) {
+    auto kern = int8_gemm_pp_kernel<Main, OUT_DT, EPI>;
     static PerDeviceOnce once;
     if (const int e = allow_dynamic_lds((const void*)kern, PpL::SMEM, once)) return e;
     hipLaunchKernelGGL(kern, dim3((unsigned)(g_main + g_rest)), dim3(PpL::NT), PpL::SMEM, st, main, rest, g_main);
     KCHECK();
     return 0;
 }
-
+template <int OUT_DT, int EPI>
+int launch_pp(GemmArgs a, hipStream_t st) {
+    bool vec_ok, aligned;
+    epilogue_alignment<OUT_DT, EPI>(a, vec_ok, aligned);
+    if (!aligned) return launch_cfg<CfgM, OUT_DT, EPI>(a, st);   // this kernel has only the coalesced epilogue
+    const int64_t G = device_cu_count();
+    const PpSplit sp = pp_split(a.M, a.N, G);
+    GemmArgs main = a, rest = a;
+    const int64_t n_main = sp.main_tm * sp.main_tn, n_rest = sp.small, tn = (a.N + 255) / 256;
+    if (n_main > 0x7fffffff || n_rest > 0x7fffffff) return -1;
+    if (n_main && n_rest) {
+        if (sp.columns) {
+            rest.n_first = (int)sp.main_tn * 256;
+        } else {
+            main = row_band<OUT_DT, EPI>(a, 0, sp.main_tm * sp.rows);
+            rest = row_band<OUT_DT, EPI>(a, sp.main_tm * sp.rows, a.M - sp.main_tm * sp.rows);
+        }
+    }
+    main.tiles_m = (int)sp.main_tm;
+    main.tiles_n = (int)sp.main_tn;
+    rest.tiles_m = (rest.M + PpS::BM - 1) / PpS::BM;
+    rest.tiles_n = (int)(sp.columns ? tn - sp.main_tn : tn);
+    main.magic = n_main ? panel_magic(main.tiles_m, main.tiles_n) : 0;
+    rest.magic = panel_magic(rest.tiles_m, rest.tiles_n);
+    const int g_main = (int)(n_main < G ? n_main : G), g_rest = (int)(n_rest < G ? n_rest : G);
+    return sp.rows == PpM::BM ? launch_pp_as<PpM, OUT_DT, EPI>(main, rest, g_main, g_rest, st)
+                              : launch_pp_as<PpL, OUT_DT, EPI>(main, rest, g_main, g_rest, st);
+}
 
 // ---------------------------------------------------------------------------------------------------------------
 // Scratch of the entry point that allocates nothing (gpu_int8_gemm_static): the int32 planes of a split-K run live in
@@ -1405,10 +1445,11 @@ FedPlan fed_plan(int64_t M, int64_t N, int64_t K, int num_cu, bool may_split) {
     }
     return best;
 }
-// The two-group kernel's time on the same scale.
+// The two-group kernel's time on the same scale, fitted to 260 shapes (8.5 % rms).  With it the choice between the two kernels is 0.2 % slower
+// than the faster of them over 1000 shapes of 512 to 8192 rows, one in a hundred by more than 1 %.
 double pp_us(int64_t M, int64_t N, int64_t K, int cus) {
     const double n = pp_split(M, N, cus).rounds;
-    return -3.0 + n * (12.0 + (double)(K / 128));
+    return 1.1 + n * (7.2 + 1.25 * (double)(K / 128));
 }
 
 // Whether a call may split K over workgroups.  Captured graphs and the static entry point do so only for the shapes that always did
@@ -1419,10 +1460,6 @@ bool fed_may_split(int64_t M, int64_t N, int64_t K, hipStream_t st) {
     return tl_scratch == nullptr && !is_capturing(st);
 }
 
-// Kernel family forced by the test hook (-1 = choose by shape), or 7000 + 100 * width + slices: the kernel with fetching waves on
-// tiles of 64 * width columns and so many slices of K.  Process-wide and only meant for tests and benchmarks:
-// relaxed atomic, so a concurrent call sees either the old or the new value, never a torn one.
-std::atomic<int> g_force_cfg{-1};
 
 FedPlan fed_plan_or_forced(int64_t M, int64_t N, int64_t K, bool may_split) {
     const int force = g_force_cfg.load(std::memory_order_relaxed) - 7000, width = force / 100;
@@ -1553,7 +1590,7 @@ int choose_cfg(int64_t M, int64_t N, int64_t K, int start, bool aligned) {
     const bool dma_ok = tiles_ok && (start & 3) == 0;
     if (force == 5) return tiles_ok && start == 0 && M <= 128 ? 5 : 1;
     if (force == 7 || force / 1000 == 7) return dma_ok ? 7 : 1;
-    if (force == 9) return dma_ok ? 9 : 1;
+    if (force == 9 || force / 1000 == 9) return dma_ok ? 9 : 1;
     if (force == 1 || force == 2) return force;
     if (tiles_ok && start == 0 && M <= 128 && rows_kernel_wins(M, N, K, aligned)) return 5;
     const int cus = device_cu_count();
@@ -1561,9 +1598,7 @@ int choose_cfg(int64_t M, int64_t N, int64_t K, int start, bool aligned) {
     // staged tiles over fetching waves: K = 128 0.93 to 1.0, K = 256 0.94 to 1.0, K = 384 0.97 to 1.1; K = 256 with 1 << 21 outputs 1.1; one step
     // and more columns than the CUs take at once in tiles of 64, 25 x 24784 4.4 us and 5.1, but 73 x 10368 4.4 and 3.8)
     const bool tiny = K <= 256 && (M * N <= 1 << 19 || (K <= 128 && M * N <= 1 << 20 && N > 64 * cus));
-    // (with one or two steps of K in several rounds the fetching waves' tiles take a fifth longer than the sums say: K = 128, 5366 x 3144
-    // 28.1 and 20.9 us on the two-group kernel, 536 x 22792 17.0 and 13.7)
-    const int large = !dma_ok || !aligned ? 1 : M >= 512 && N >= 512 && pp_us(M, N, K, cus) < fed_plan(M, N, K, cus, true).us * (K <= 256 ? 1.2 : 1.) ? 9 : 7;
+    const int large = !dma_ok || !aligned ? 1 : M >= 512 && N >= 512 && pp_us(M, N, K, cus) < fed_plan(M, N, K, cus, true).us ? 9 : 7;
     if (dma_ok && aligned && start == 0 && !tiny) return large;
     // the register-staged tiles: large ones, or for operands off 16 bytes the DMA kernels, as soon as there is work for them
     if (M <= 256 && N >= 1024 && tiles_ok && K >= 512) return K >= 1536 || (M > 128 && N >= 8192) ? large : 2;
@@ -1734,7 +1769,7 @@ GPU_API int gpu_int8_gemm(const int8_t* A, const int8_t* W, const float* xs, con
     if (out_dt < DT_F32 || out_dt > DT_BF16 || M < 0 || N < 0 || K < 0 || !shape_ok(M, N, K)) return -200;
     PaddedK pad(A, W, M, N, K, (hipStream_t)stream);
     if (pad.rc != 0) return pad.rc < 0 ? -200 : pad.rc;
-    GemmArgs a{A, W, xs, ws, bias, nullptr, nullptr, D, (int)M, (int)N, (int)K, 0, 0, 0};
+    GemmArgs a{A, W, xs, ws, bias, nullptr, nullptr, D, (int)M, (int)N, (int)K, 0, 0, 0, 0, 0};
     const int rc = dispatch_dt<EPI_PLAIN>(a, out_dt, (hipStream_t)stream);
     return rc < 0 ? -200 : rc;
 }
@@ -1747,7 +1782,7 @@ GPU_API int gpu_int8_gemm_residual(const int8_t* A, const int8_t* W, const float
     if (out_dt < DT_F32 || out_dt > DT_BF16 || M < 0 || N < 0 || K < 0 || !shape_ok(M, N, K)) return -201;
     PaddedK pad(A, W, M, N, K, (hipStream_t)stream);
     if (pad.rc != 0) return pad.rc < 0 ? -201 : pad.rc;
-    GemmArgs a{A, W, xs, ws, bias, rscale, resid, D, (int)M, (int)N, (int)K, 0, 0, 0};
+    GemmArgs a{A, W, xs, ws, bias, rscale, resid, D, (int)M, (int)N, (int)K, 0, 0, 0, 0, 0};
     const int rc = dispatch_dt<EPI_RESID>(a, out_dt, (hipStream_t)stream);
     return rc < 0 ? -201 : rc;
 }
@@ -1760,7 +1795,7 @@ GPU_API int gpu_int8_gemm_static(const int8_t* A, const int8_t* W, const float* 
     int rc = 0;
     void* ptr = static_scratch(&rc);
     if (!ptr) return rc;
-    GemmArgs a{A, W, xs, ws, bias, nullptr, nullptr, D, (int)M, (int)N, (int)K, 0, 0, 0};
+    GemmArgs a{A, W, xs, ws, bias, nullptr, nullptr, D, (int)M, (int)N, (int)K, 0, 0, 0, 0, 0};
     tl_scratch = ptr;
     tl_scratch_bytes = kStaticScratchBytes;
     rc = dispatch_dt<EPI_PLAIN>(a, out_dt, (hipStream_t)stream);
@@ -1776,14 +1811,14 @@ GPU_API int gpu_int8_gemm_acc(const int8_t* A, const int8_t* W, int32_t* acc, in
     if (M < 0 || N < 0 || K < 0 || !shape_ok(M, N, K)) return -200;
     PaddedK pad(A, W, M, N, K, (hipStream_t)stream);
     if (pad.rc != 0) return pad.rc < 0 ? -200 : pad.rc;
-    GemmArgs a{A, W, nullptr, nullptr, nullptr, nullptr, nullptr, acc, (int)M, (int)N, (int)K, 0, 0, 0};
+    GemmArgs a{A, W, nullptr, nullptr, nullptr, nullptr, nullptr, acc, (int)M, (int)N, (int)K, 0, 0, 0, 0, 0};
     const int rc = dispatch_cfg<DT_F32, EPI_ACC>(a, (hipStream_t)stream);
     return rc < 0 ? -200 : rc;
 }
 
 // Test hook: force a kernel family (1 = 128x128, 2 = 64x64 register-staged tiles; 5 = up to 128 rows; 7 = waves that
 // fetch for others, 7000 + 100 * width + slices = those with that tile width (of 64 columns) and split; 9 = two-group
-// kernel; -1 or anything else = automatic).
+// kernel, 9000 + 10 * kind + split = that with one of its tile grids; -1 or anything else = automatic).
 GPU_API int gpu_int8_gemm_force_config(int cfg) {
     g_force_cfg.store(cfg, std::memory_order_relaxed);
     return 0;

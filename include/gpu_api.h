@@ -314,8 +314,9 @@ int64_t gpu_w6a8_group_gemm_scratch(const void* Wp, int64_t M, int64_t N, int64_
 /* Test and tuning hook: force the GEMM kernel family.  1, 2 = 128x128 and 64x64 register-staged tiles; 5 = weights straight
  * into registers, for M <= 128; 7 = four waves multiply what four others fetch, 128x64 to 128x192 tiles, K split where they are few;
  * 7000 + 100 * width + slices = 7 with tiles of 64 * width columns (width 1 to 3) and K in that many slices;
- * 9 = two-group kernel (256x256 and 128x256 tiles, one launch), the choice for large shapes; anything else = automatic.  A shape
- * a family cannot run falls back to 1. */
+ * 9 = two-group kernel (tiles of 256, 192 and 128 rows by 256 columns, one launch), the choice for large shapes; 9000 + 10 * kind + split
+ * = 9 with tiles of 256, 192 or 128 rows (kind 0 to 2) and nothing, the rows or the columns that whole rounds leave over as
+ * 128-row tiles (split 0 to 2); anything else = automatic.  A shape a family cannot run falls back to 1. */
 int gpu_int8_gemm_force_config(int cfg);
 
 /* Test hook, no reference counterpart: which kernel a gpu_int8_gemm call outside capture takes for A and W that start `start` bytes

@@ -1001,6 +1001,34 @@ def test_int8_gemm_fetching_waves_every_width_and_split(width, steps, slices, M,
         ffi.raw("gpu_int8_gemm_force_config", -1)
 
 
+# The two-group kernel's tile grids (9000 + 10 * kind + split; kind: tiles of 256, 192 or 128 rows, split: none, the rows that whole
+# rounds of 256 tiles leave over as 128-row tiles, or the columns).  More tiles than CUs with last tiles of few rows and columns,
+# one to five steps of K, and shapes of less than one tile
+@pytest.mark.parametrize("cfg", [9000, 9001, 9002, 9010, 9011, 9012, 9020])
+@pytest.mark.parametrize("M,N,K", [(2100, 7704, 128), (2113, 7688, 384), (193, 264, 256), (385, 520, 640), (100, 72, 128)])
+def test_int8_gemm_tile_grids(M, N, K, cfg):
+    say("gemm tile grid", M, N, K, cfg)
+    A, W = rand_i8(19, 500 + M, M, K), rand_i8(19, 600 + N, N, K)
+    A[0, :] = -128
+    W[N - 1, :] = -128
+    xs, ws = synth.uniform(19, 3, M, 0.005, 0.2), synth.uniform(19, 4, N, 1e-3, 1e-2)
+    want = oracle.int8_gemm_acc(A, W)
+    Ad, Wd, xd, wd = dev(A), dev(W), dev(xs), dev(ws)
+    ffi.raw("gpu_int8_gemm_force_config", cfg)
+    try:
+        assert gemm_plan(M, N, K)[0] == 9
+        assert np.array_equal(ql.int8_gemm_acc(Ad, Wd).cpu().numpy(), want)
+        for dt, tob in ((BF16, oracle.bf16_bits), (F16, oracle.f16_bits), (F32, lambda a: a.astype(np.float32))):
+            bias, rs = tob(synth.normal(19, 5, N) * np.float32(0.02)), tob(synth.normal(19, 6, N))
+            resid = tob(synth.normal(19, 7, M * N).reshape(M, N))
+            d = ql.int8_gemm(Ad, Wd, xd, wd, dev_bits(bias, dt), TDT[dt])
+            assert np.array_equal(host_bits(d), oracle.epilogue(want, xs, ws, bias, dt, fma=1)), dt
+            r = ql.int8_gemm_residual(Ad, Wd, xd, wd, dev_bits(bias, dt), dev_bits(rs, dt), dev_bits(resid, dt))
+            assert np.array_equal(host_bits(r), oracle.epilogue_residual(want, xs, ws, bias, rs, resid, dt, fma=1)), dt
+    finally:
+        ffi.raw("gpu_int8_gemm_force_config", -1)
+
+
 @pytest.mark.parametrize("start", [1, 2, 4, 8, 12])
 @pytest.mark.parametrize("M,N,K", [(64, 136, 384), (3, 512, 1024), (200, 2056, 1536), (520, 25088, 128)])
 def test_int8_gemm_operands_off_16_bytes(M, N, K, start):
