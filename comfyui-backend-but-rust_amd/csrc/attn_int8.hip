@@ -1075,9 +1075,6 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void attn_int8_kernel(AttnAr
 __device__ __forceinline__ void dma16(uint32_t lds_dst, uint32_t lane_off, const void* base) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_dst), "v"(lane_off), "s"(base) : "memory", "m0");
 }
-__device__ __forceinline__ void dma4(uint32_t lds_dst, uint32_t lane_off, const void* base) {   // 256 bytes, 4 per lane
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_dst), "v"(lane_off), "s"(base) : "memory", "m0");
-}
 __device__ __forceinline__ float swap32_max(float x) {   // maximum of a lane and lane ^ 32
     const auto r = __builtin_amdgcn_permlane32_swap(f2u(x), f2u(x), false, false);
     return fmax_nn(u2f(r[0]), u2f(r[1]));
@@ -1101,6 +1098,18 @@ __device__ __forceinline__ float2 load_agent(const float* p, int i) {
     return make_float2(u2f((uint32_t)v), u2f((uint32_t)(v >> 32)));
 }
 
+// Integer sums become floats without v_cvt_f32_i32: the accumulator starts at the bits of 1.5 * 2^23 (the products with V at that plus
+// 128 x the column sums), where floats have a step of 1 and room for +-2^22, so that its bits are a float all the way, and an exact
+// subtraction takes the start off again.  A score is at most 128^3 (head dim 128), a product 255 * 128 * 128.  With two waves on
+// a SIMD a conversion takes 4 cycles, as do maxima, shifts, permutes and anything with a scalar operand; fp32 additions,
+// multiplications and fma on registers of two waves go side by side, 2.2 cycles each.
+constexpr int kSumOne = 0x4B400000;
+__device__ __forceinline__ v16i sum_one() {
+    constexpr int z = kSumOne;
+    return v16i{z, z, z, z, z, z, z, z, z, z, z, z, z, z, z, z};
+}
+__device__ __forceinline__ float sum_value(int bits) { return __builtin_bit_cast(float, bits) - 12582912.f; }
+
 // The attention without a key bias, head dims 64 and 128: attn_int8_kernel's arithmetic with the work of two tiles overlapped.
 // It is bound by vector instruction issue (at 4608 tokens x 24 heads of 128: about 470 per wave and tile beside 32 MFMAs; by the
 // counters the vector pipes are busy 69 % of its cycles and the matrix pipes 29 %).
@@ -1115,6 +1124,10 @@ __device__ __forceinline__ float2 load_agent(const float* p, int i) {
 //   * numerator and denominator are relative to a base that all but never moves (below), which takes the multiplication
 //     of every output by its rescale factor out of every tile.
 //   * DMA addresses are scalar, the exchange with lane ^ 32 is a row swap.
+//   * the first output block's V fragments and column sums are read under the last probabilities, the others' under the products of the
+//     block before; the last key block's scores go between the first block's products; integer sums become floats by a subtraction
+//     (sum_value); V lies in LDS a half of its 32 bytes at a time (2-way bank conflicts, a fifth of the LDS cycles, before).
+//     Together 4608 x 24 x 128 255.4 -> 250.0 us a call, 2 x 4096 x 10 x 64 117.1 -> 116.4.
 //   * SPLIT: the keys of the row blocks that do not fill the CUs once more are shared by several workgroups (key_parts, with the
 //     figures): each part has its own base, and the last to finish brings all of them to the largest.
 // 250 -> 230 us at that shape by the kernel trace, 141 -> 129 us at SDXL's 2 x 4096 x 10 x 64, before the last of these.  A workgroup of eight waves
@@ -1145,22 +1158,26 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
     const int64_t bh = (int64_t)bi * a.h + hi, kvh = (int64_t)bi * a.hk + hi / a.rep;
     const int r = row0 + l32, rc = r < a.lq ? r : a.lq - 1;   // rows past lq are computed on a clamped row and never stored
     const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)smem, lane16 = lane * 16;
+    const uint32_t v_lane = l32 * 32 + hh * 16;   // V: a KB of 32 channels, both halves' 16 bytes side by side; in LDS a half at a time
     const int8_t *kt = a.ki + kvh * a.nblk * (32 * D), *vt = a.vt + kvh * a.nblk * (32 * D);
     const int* vst = a.vsum + kvh * a.kb * D;
     const float* kst = a.ks + kvh * a.kb * 4 + hh * 2;
 
-    // The DMA of a wave's share of K tile tk (j < NF), V tile tv and its column sums (j = 2 NF).  A K tile past the end fetches the last
-    // one, into the stage that a tile tk would have: nothing reads that stage any more, while the last tile's own stage is being read.
-    // Every wave fetches column sums (two waves the same ones): no branch in the tile loop.
+    // The DMA of a wave's share of K tile tk (j < NF) and V tile tv.  A K tile past the end fetches the last one, into the stage that
+    // a tile tk would have: nothing reads that stage any more, while the last tile's own stage is being read.
     constexpr int NF = KV / 4096;
     auto dma = [&](int j, int tk, int tv) {
-        const int c = (wave + 4 * (j % NF)) * 1024, cs = D == 128 ? (wave & 1) * 256 : 0;
+        const int c = (wave + 4 * (j % NF)) * 1024;
         if (j < NF) dma16(lds0 + (tk & 1) * STAGE + c, lane16, kt + (int64_t)(tk < a.kb ? tk : a.kb - 1) * KV + c);
-        else if (j < 2 * NF) dma16(lds0 + (tv & 1) * STAGE + KV + c, lane16, vt + (int64_t)tv * KV + c);
-        else dma4(lds0 + (tv & 1) * STAGE + 2 * KV + cs, lane16 >> 2, (const uint8_t*)(vst + (int64_t)tv * D) + cs);
+        else dma16(lds0 + (tv & 1) * STAGE + KV + c, v_lane, vt + (int64_t)tv * KV + c);
     };
+    // The column sums go through a register, where they get the bias kSumOne.  Every wave takes 64 of them (at 128 two waves the same
+    // ones, at 64 all): no branch in the tile loop.
+    const int vcol = (D == 128 ? (wave & 1) * 64 : 0) + lane;
+    auto put_sums = [&](int tv, int sum) { reinterpret_cast<int*>(smem + (tv & 1) * STAGE + 2 * KV)[vcol] = sum + kSumOne; };
+    const int sum0 = vst[t0 * D + vcol];
 #pragma unroll
-    for (int j = 0; j <= 2 * NF; ++j) dma(j, t0, t0);
+    for (int j = 0; j < 2 * NF; ++j) dma(j, t0, t0);
 #pragma unroll
     for (int j = 0; j < NF; ++j) dma(j, t0 + 1, 0);
 
@@ -1180,6 +1197,7 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
         for (int i = 0; i < 16; ++i) ro[x][i] = 0.f;
     float m = -50000.f, dsum = !SPLIT || part == 0 ? 1.f : 0.f, dsum2 = 0.f;
     __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+    put_sums(t0, sum0);
     __syncthreads();
 
     v16i S[NB];
@@ -1192,7 +1210,7 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
     for (int blk = 0; blk < NB; ++blk) {
         v4i kf[NS];
         load_kf(kf, t0, blk);
-        S[blk] = v16i{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+        S[blk] = sum_one();
 #pragma unroll
         for (int s = 0; s < NS; ++s) S[blk] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[s], qf[s], S[blk], 0, 0, 0);
     }
@@ -1203,12 +1221,14 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
         const uint8_t* st = smem + (t & 1) * STAGE;
         const int key0 = t * CK;
         float n0 = 0.f, n1 = 0.f;
+        int next_sum = 0;
         if constexpr (!last) {
             n0 = kst[(t + 1) * 4];
             n1 = kst[(t + 1) * 4 + 1];
+            next_sum = vst[(t + 1) * D + vcol];
         }
         const float gs0 = a.sm * (q_scale * k0), gs1 = a.sm * (q_scale * k1);
-        int i0 = last ? -50000 : INT_MIN, i1 = i0;
+        int i0 = last ? kSumOne - 50000 : INT_MIN, i1 = i0;
 #pragma unroll
         for (int blk = 0; blk < NB; ++blk)
 #pragma unroll
@@ -1221,7 +1241,7 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
                 if ((i % 4) < 2) i0 = max(i0, sv);
                 else i1 = max(i1, sv);
             }
-        const float tile_m = swap32_max(fmax_nn(fmaf((float)i0, gs0, -kU8Offset), fmaf((float)i1, gs1, -kU8Offset)));
+        const float tile_m = swap32_max(fmax_nn(fmaf((float)(i0 - kSumOne), gs0, -kU8Offset), fmaf((float)(i1 - kSumOne), gs1, -kU8Offset)));
         // The running base m only moves when a tile's maximum has outgrown it by 2^60 (and at the first tile): numerator and
         // denominator are both relative to it, so any base gives the same quotient, and the outputs need no rescaling here.
         if (__builtin_amdgcn_ballot_w64(tile_m - m > 60.f)) {
@@ -1240,10 +1260,24 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
         // a NaN maximum (every key scale of the tile infinite): the tile's probabilities are 0 and its factor 1, so that it drops out
         const float t_scale = tile_m == tile_m ? __builtin_amdgcn_exp2f(tile_m - m) : 1.f;
 
-        v4i pf[NB];
+        v4i pf[NB], vf[2][NB];
+        v16i acc[2];
+        // the fragments of V for output block x, and the column sums that its products start from
+        auto load_vf = [&](int x, int blk) {
+            vf[x & 1][blk] = *reinterpret_cast<const v4i*>(st + KV + (blk * D + x * 32) * 32 + lane16);
+        };
+        auto load_sums = [&](int x) {
+            const int* vsp = reinterpret_cast<const int*>(st + 2 * KV) + x * 32 + hh * 4;
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+                const v4i c4 = *reinterpret_cast<const v4i*>(vsp + g4 * 8);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) acc[x & 1][g4 * 4 + c] = c4[c];
+            }
+        };
         uint32_t psum = 0;
 #pragma unroll
-        for (int rg = 0; rg <= (last ? NB - 1 : NB); ++rg) {
+        for (int rg = 0; rg < NB; ++rg) {
             // region rg: probabilities of key block rg, and under them the next tile's scores into the block before it
             v4i kf[NS];
             if constexpr (!last)
@@ -1251,29 +1285,33 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
             float e[4][4];
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4) {
-                if (rg < NB) {
-                    uint32_t packed = 0u;
+                uint32_t packed = 0u;
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        e[g4][c] = __builtin_amdgcn_exp2f(fmaf((float)S[rg < NB ? rg : 0][g4 * 4 + c], c < 2 ? gs0 : gs1, -tile_m));
-                        if constexpr (last) {
-                            const int key = key0 + rg * 32 + g4 * 8 + hh * 4 + c;
-                            e[g4][c] = key < a.lk ? e[g4][c] : 0.f;
-                        }
-                        packed = __builtin_amdgcn_cvt_pk_u8_f32(e[g4][c], c, packed);
+                for (int c = 0; c < 4; ++c) {
+                    e[g4][c] = __builtin_amdgcn_exp2f(fmaf(sum_value(S[rg][g4 * 4 + c]), c < 2 ? gs0 : gs1, -tile_m));
+                    if constexpr (last) {
+                        const int key = key0 + rg * 32 + g4 * 8 + hh * 4 + c;
+                        e[g4][c] = key < a.lk ? e[g4][c] : 0.f;
                     }
-                    if constexpr (!last) psum = __builtin_amdgcn_sad_u8(packed, 0u, psum);
-                    pf[rg < NB ? rg : 0][g4] = (int)(packed ^ 0x80808080u);
+                    packed = __builtin_amdgcn_cvt_pk_u8_f32(e[g4][c], c, packed);
                 }
+                if constexpr (!last) psum = __builtin_amdgcn_sad_u8(packed, 0u, psum);
+                pf[rg][g4] = (int)(packed ^ 0x80808080u);
                 if constexpr (!last) {
-                    if (rg * 4 + g4 >= 1 && rg * 4 + g4 <= 2 * NF + 1) dma(rg * 4 + g4 - 1, t + 2, t + 1);
+                    if (rg * 4 + g4 >= 1 && rg * 4 + g4 <= 2 * NF) dma(rg * 4 + g4 - 1, t + 2, t + 1);
                     if (rg > 0 && g4 % (4 / NS) == 0) {
                         const int s = g4 / (4 / NS);
-                        if (s == 0) S[rg - 1] = v16i{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+                        if (s == 0) S[rg - 1] = sum_one();
                         S[rg - 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[s], qf[s], S[rg - 1], 0, 0, 0);
                     }
-                    __builtin_amdgcn_sched_barrier(0x100);
                 }
+                if (rg == NB - 1) {   // what the products begin with
+                    if (g4 == 1) load_sums(0);
+                    if (g4 >= 2)
+#pragma unroll
+                        for (int blk = (g4 - 2) * NB / 2; blk < (g4 - 1) * NB / 2; ++blk) load_vf(0, blk);
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
             if constexpr (last) {   // the unrounded probabilities, in the reference's per-thread partials
 #pragma unroll
@@ -1286,37 +1324,38 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
         }
         if constexpr (!last) dsum = fmaf((float)psum, t_scale, dsum);
 
-        // P.V, an output block at a time; the fold of a block rides between the products of the next
-        v16i acc[2];
+        // P.V, an output block at a time; the fold of a block rides between the products of the next, the fragments of the block after
+        // that are read under them, and the last key block's scores go between the first block's products
+        v4i kf[NS];
+        if constexpr (!last) load_kf(kf, t + 1, NB - 1);
+        if constexpr (!last) S[NB - 1] = sum_one();
 #pragma unroll
         for (int x = 0; x <= NS; ++x) {
-            if (x < NS) {
-                const int* vsp = reinterpret_cast<const int*>(st + 2 * KV) + x * 32 + hh * 4;
-#pragma unroll
-                for (int g4 = 0; g4 < 4; ++g4) {
-                    const v4i c4 = *reinterpret_cast<const v4i*>(vsp + g4 * 8);
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) acc[x & 1][g4 * 4 + c] = c4[c];
-                }
-            }
 #pragma unroll
             for (int blk = 0; blk < NB; ++blk) {
-                if (x < NS) {
-                    const v4i vf = *reinterpret_cast<const v4i*>(st + KV + ((blk * D + x * 32 + l32) * 32 + hh * 16));
-                    acc[x & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf, pf[blk], acc[x & 1], 0, 0, 0);
-                }
+                if (x < NS) acc[x & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(vf[x & 1][blk], pf[blk], acc[x & 1], 0, 0, 0);
+                if constexpr (!last)
+                    if (x == 0)
+#pragma unroll
+                        for (int s = blk * NS / NB; s < (blk + 1) * NS / NB; ++s)
+                            S[NB - 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[s], qf[s], S[NB - 1], 0, 0, 0);
                 if (x > 0) {
 #pragma unroll
                     for (int i = blk * (16 / NB); i < (blk + 1) * (16 / NB); ++i)
-                        ro[x > 0 ? x - 1 : 0][i] = fmaf((float)acc[(x + 1) & 1][i], t_scale, ro[x > 0 ? x - 1 : 0][i]);
+                        ro[x > 0 ? x - 1 : 0][i] = fmaf(sum_value(acc[(x + 1) & 1][i]), t_scale, ro[x > 0 ? x - 1 : 0][i]);
                 }
-                __builtin_amdgcn_sched_barrier(0x100);
+                if (x + 1 < NS) {
+                    load_vf(x + 1, blk);
+                    if (blk == NB - 1) load_sums(x + 1);
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
         if constexpr (!last) {
             k0 = n0;
             k1 = n1;
             __builtin_amdgcn_s_waitcnt(0x0f70);   // this wave's share of the next tiles has landed
+            put_sums(t + 1, next_sum);
             __syncthreads();
         }
     };

@@ -808,3 +808,29 @@ def test_attention_with_keys_shared_by_workgroups(case):
     assert (np.abs(got - ref) <= 2 * vmax / 255.0 + 2 * ulp * np.abs(ref)).all()
     assert (np.abs(got - ref) <= ulp * np.abs(ref) + 1e-30).mean() > 0.97
     assert all(torch.equal(o, outs[0]) for o in outs[1:])
+
+
+@pytest.mark.parametrize("D,lk,keys", [(128, 1300, "same"), (128, 1300, "both"), (128, 200, "both"), (64, 200, "same"), (64, 1500, "both")])
+def test_attention_integer_sums_at_their_limits(D, lk, keys):
+    """Rows with one channel: rotated they have codes of +-127 only, so that scores are +-127 * 127 * D, and equal keys with values of one
+    sign per channel make products of 255 * 127 * (keys of a tile), the largest that the accumulators' start has to leave room for."""
+    ql, ffi = _pkg()
+    lq, h = 70, 2
+    q, k, v = torch.zeros(1, lq, h, D), torch.zeros(1, lk, h, D), torch.ones(1, lk, h, D)
+    q[..., 5] = 2.0
+    k[..., 5] = 1.0
+    v[..., ::2] = -1.0
+    if keys == "both":
+        k[:, ::3, :, 5] = -1.0
+    q, k, v = q.bfloat16(), k.bfloat16(), v.bfloat16()
+    scale = 0.25
+    if D == 128:   # without the anchor, which would take the keys' common part off
+        ref = _to_f32(oracle.attn_int8(oracle.BF16, _bits(q), _bits(k), _bits(v), scale, use_anchor=False, sink=1.0), oracle.BF16)
+        got = _to_f32(_bits(ql.int8_attn_sink(q.cuda(), k.cuda(), v.cuda(), scale, 1.0)), oracle.BF16)
+    else:
+        ref = _to_f32(oracle.attn_int8(oracle.BF16, _bits(q), _bits(k), _bits(v), scale), oracle.BF16)
+        got = _to_f32(_bits(ql.int8_attn(q.cuda(), k.cuda(), v.cuda(), scale)), oracle.BF16)
+    # one u8 step of every key (all land on the same side of a boundary) moves numerator and denominator alike, by 1 / 255 of the
+    # smallest probability's share at most
+    assert (np.abs(got - ref) <= 2.0 / 255.0 * np.abs(ref)).all()
+    assert np.abs(ref).min() > 0.5
