@@ -1098,17 +1098,11 @@ __device__ __forceinline__ float2 load_agent(const float* p, int i) {
     return make_float2(u2f((uint32_t)v), u2f((uint32_t)(v >> 32)));
 }
 
-// Integer sums become floats without v_cvt_f32_i32: the accumulator starts at the bits of 1.5 * 2^23 (the products with V at that plus
-// 128 x the column sums), where floats have a step of 1 and room for +-2^22, so that its bits are a float all the way, and an exact
-// subtraction takes the start off again.  A score is at most 128^3 (head dim 128), a product 255 * 128 * 128.  With two waves on
-// a SIMD a conversion takes 4 cycles, as do maxima, shifts, permutes and anything with a scalar operand; fp32 additions,
-// multiplications and fma on registers of two waves go side by side, 2.2 cycles each.
-constexpr int kSumOne = 0x4B400000;
+// A score is at most 128^3 (head dim 128), a product with V 255 * 128 * 128: both fit sum_value.
 __device__ __forceinline__ v16i sum_one() {
     constexpr int z = kSumOne;
     return v16i{z, z, z, z, z, z, z, z, z, z, z, z, z, z, z, z};
 }
-__device__ __forceinline__ float sum_value(int bits) { return __builtin_bit_cast(float, bits) - 12582912.f; }
 
 // The attention without a key bias, head dims 64 and 128: attn_int8_kernel's arithmetic with the work of two tiles overlapped.
 // It is bound by vector instruction issue (at 4608 tokens x 24 heads of 128: about 470 per wave and tile beside 32 MFMAs; by the

@@ -422,16 +422,18 @@ __global__ void __launch_bounds__(NT, 1) w6a8_group_gemm_kernel(W6Args p) {
 
 // The W8 form on 256 x 256 tiles: eight waves of 128 x 64, so that a group costs a wave 24 fragment reads for 64 MFMAs where the
 // 256 x 128 tile costs it 20 for 32, and a CU 64 KB of DMA where two of the smaller tiles cost 96.  256 registers hold that because a
-// lane's int32 partials live only from one row tile to the next: while the eight MFMAs of a row tile run, the fold of the one before
-// rides between them, four vector instructions to an MFMA (a probe of this mix: 24.7 cycles per MFMA and SIMD; the same MFMAs
-// and vector instructions in blocks take 31-35 from one wave and lean on the other one for the rest).  Two LDS stages of A, W and
-// scales: group g+1 travels during group g, one barrier per group.  The four lower waves issue all DMA, one instruction after
-// every other MFMA: every wave fetching its own share has both waves of a SIMD held by a DMA instruction at the same time
-// (M=8192, K=5120 -> N=13824 638 us, this way 617; K=13824 -> N=5120 646 and 630; the DMA free of charge would be 556 and 580).
+// lane's int32 partials live only from one row tile to the next: behind the eight MFMAs of a row tile comes the fold of the one before,
+// 32 additions (sum_value) and 32 fma in a row.  A vector instruction behind every MFMA does not overlap with the other wave's: a probe of
+// this mix, four to an MFMA and two waves, takes 25.0 cycles per MFMA and SIMD with any kind of vector instruction; in runs of 8 and
+// 32 23.3 with conversions, 23.2 with additions (of 64 and 256 21.9 and 20.6, for which there are no registers).  In the kernel 614 us one by one with
+// conversions, 610 with additions, 605 in runs with conversions, 597 in runs with additions; runs of 4 and 16 603.
+// Two LDS stages of A, W and scales: group g+1 travels during group g, one barrier per group.  The four lower waves issue all DMA, one
+// instruction after every eight of the fold: every wave fetching its own share has both waves of a SIMD held by a DMA instruction at the
+// same time (608); between the MFMAs 598, twice as dense 600, spread over all of the group 630 (they land too late).
 // The same tile with v_mfma_i32_32x32x32_i8, which leaves more issue slots to the fold, takes 677 us: the chip is at its power limit.
 // A persistent form with the next tile's first group under the epilogue: no change.
-// M=8192, K=5120 -> N=13824, expansion included: 256 x 128 tiles 756 us, these 617.  What is left is the fold next to the MFMAs
-// (64 MFMAs and 256 vector instructions per wave and group: 3161 cycles of a SIMD against 2048 for the MFMAs alone) at 2.0 GHz.
+// M=8192, K=5120 -> N=13824, expansion included: 256 x 128 tiles 756 us, these 597.  What is left is the fold next to the MFMAs
+// (64 MFMAs and 256 vector instructions per wave and group), near the power limit.
 constexpr int BIG_BN = 256, BIG_U = BIG_BN * BK, BIG_U_BASE = 2 * A_STAGE, BIG_S_BASE = BIG_U_BASE + 2 * BIG_U, BIG_S = BIG_BN * 4;
 constexpr int BIG_SMEM = BIG_S_BASE + 2 * BIG_S;
 
@@ -473,7 +475,7 @@ __global__ void __launch_bounds__(NT, 1) w6a8_group_gemm_big_kernel(W6Args p) {
     float4 sv[FN];
 #pragma unroll
     for (int in = 0; in < FN; ++in) {
-        part[1][in] = v4i{0, 0, 0, 0};
+        part[1][in] = v4i{kSumOne, kSumOne, kSumOne, kSumOne};
         sv[in] = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int im = 0; im < FM; ++im)
@@ -484,7 +486,7 @@ __global__ void __launch_bounds__(NT, 1) w6a8_group_gemm_big_kernel(W6Args p) {
     auto fold2 = [&](int buf, int in, int im, int c0) {
         const float s4[4] = {sv[in].x, sv[in].y, sv[in].z, sv[in].w};
 #pragma unroll
-        for (int c = c0; c < c0 + 2; ++c) accf[in][im][c] = __builtin_fmaf((float)part[buf][in][c], s4[c], accf[in][im][c]);
+        for (int c = c0; c < c0 + 2; ++c) accf[in][im][c] = __builtin_fmaf(sum_value(part[buf][in][c]), s4[c], accf[in][im][c]);
     };
     // No branch inside: the compiler would move the folds behind it.
     auto loop = [&](auto fetches_tag) {
@@ -522,17 +524,20 @@ __global__ void __launch_bounds__(NT, 1) w6a8_group_gemm_big_kernel(W6Args p) {
             for (int im = 0; im < FM; ++im) {
                 if (im + 1 < FM) read_a(im + 1);
 #pragma unroll
-                for (int h = 0; h < 2; ++h)
+                for (int slot = 0; slot < 8; ++slot) {
+                    const int h = slot >> 2, in = slot & 3;
+                    const v4i c = h == 0 ? v4i{kSumOne, kSumOne, kSumOne, kSumOne} : part[im & 1][in];
+                    part[im & 1][in] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fw[in][h], fa[im & 1][h], c, 0, 0, 0);
+                }
+                SCHED_FENCE();
 #pragma unroll
-                    for (int in = 0; in < FN; ++in) {
-                        const int slot = h * 4 + in, j = im * 4 + (slot >> 1);
-                        const v4i c = h == 0 ? v4i{0, 0, 0, 0} : part[im & 1][in];
-                        part[im & 1][in] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fw[in][h], fa[im & 1][h], c, 0, 0, 0);
-                        SCHED_FENCE();
-                        if (im > 0) fold2((im - 1) & 1, slot >> 1, im - 1, 2 * (slot & 1));
-                        if (fetches && (slot & 1) == 0 && j < NDMA) dma(g + 1, j);   // the stage last read before the previous barrier
-                        SCHED_FENCE();
-                    }
+                for (int slot = 0; slot < 8; ++slot) {
+                    const int j = im * 4 + (slot >> 1);
+                    if (im > 0) fold2((im - 1) & 1, slot >> 1, im - 1, 2 * (slot & 1));
+                    SCHED_FENCE();
+                    if (fetches && (slot & 1) == 0 && j < NDMA) dma(g + 1, j);   // the stage last read before the previous barrier
+                    SCHED_FENCE();
+                }
             }
             if constexpr (fetches) wait_all_dma();
             __syncthreads();
@@ -592,7 +597,7 @@ __global__ void __launch_bounds__(256) w6_words_to_int8_kernel(const uint8_t* Wp
 // Which form runs.  Fused, every workgroup expands its own 128 columns as it goes; the other two expand the packed weights once into
 // a scratch of N*K bytes and multiply 256 x 128 or 256 x 256 tiles of them.  A launch takes whole rounds of one tile per CU, and a
 // round takes a fixed time per group, in us on random codes: 1.42 fused (K=5120 -> N=13824: 1024 rows 115 us, 2048 228, 3072 342,
-// 8192 816), 1.26 (121, 222, 325, 745 with the expansion) and 2.05 (98, 178, 261, 611); the expansion takes about 6 us and 3.7 bytes
+// 8192 816), 1.26 (121, 222, 325, 745 with the expansion) and 2.0 (98, 176, 255, 597); the expansion takes about 6 us and 3.7 bytes
 // per ns.  The smallest sum runs: 512 rows of that shape fused (60 us, 71, 90), 1536 rows alike in all three (172); 4096 -> 4096
 // 2048 rows fused (54; 54, 67), 3072 on large tiles (69; 93 fused), 13824 -> 5120 1024 rows 142, 140 and 196, 2048 rows 284, 265 and 197.
 // From kExpandRows rows on the weights are always expanded (1024 -> 2048, 4096 rows: fused 20 us, expanded 22).  Below, only into a
@@ -609,7 +614,7 @@ Form pick_form(const void* Wp, int64_t M, int64_t N, int64_t K, bool may_expand)
     if (mode >= 2) return mode == 3 && fits256 ? kTiles256 : kTiles128;
     const double ng = (double)(K / 128), expand = 6.0 + (double)N * (double)K / 3.7e6;
     const double fused = ng * 1.42 * (double)((t128 + cus - 1) / cus), small = ng * 1.26 * (double)((t128 + cus - 1) / cus);
-    const double large = fits256 ? ng * 2.05 * (double)((t256 + cus - 1) / cus) : 1e30;
+    const double large = fits256 ? ng * 2.0 * (double)((t256 + cus - 1) / cus) : 1e30;
     if (mode != 1 && M < kExpandRows && (!may_expand || fused <= expand + (small < large ? small : large))) return kFused;
     return large < small ? kTiles256 : kTiles128;
 }
