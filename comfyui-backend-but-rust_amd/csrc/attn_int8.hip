@@ -55,12 +55,6 @@ struct AttnArgs {
 // fmaxf as the reference's device code uses it: a NaN operand is dropped.
 __device__ __forceinline__ float fmax_nn(float a, float b) { return __builtin_fmaxf(a, b); }
 
-__device__ __forceinline__ int8_t rn_s8(float v) {
-    if (v != v) return 0;
-    const float r = __builtin_rintf(v);
-    return (int8_t)(r > 127.f ? 127.f : r < -128.f ? -128.f : r);
-}
-
 // Cross-lane moves inside a row's lanes, as data-parallel-primitive modifiers (no LDS traffic).  A row's 16-channel blocks lie
 // on its lanes so that each move of a block bit is one such modifier: blocks 4..7 of eight run backwards, which makes
 // block ^ 4 the mirror of the eight lanes.
@@ -368,11 +362,7 @@ __device__ __forceinline__ void anchor_body(const AttnArgs& a, const int hi, con
     __shared__ int chosen;
     const int tid = threadIdx.x, c = tid & (D - 1);
     const int64_t base = bi * a.k_bs + hi * a.k_hs;
-    if (tid < D) {   // the V quantizer's accumulators for this (kv head, batch) start at zero
-        const int64_t bh = (int64_t)bi * a.hk + hi;
-        a.vmax[bh * D + c] = 0u;
-        for (int t = 0; t < a.kb; ++t) a.vsum[(bh * a.kb + t) * D + c] = 0;
-    }
+    if (tid < D) a.vmax[((int64_t)bi * a.hk + hi) * D + c] = 0u;   // the V maxima of this (kv head, batch) start at zero
     bool normed = false;
     if constexpr (D == 128) {
         if (a.k_norm) {
@@ -649,8 +639,8 @@ __device__ __forceinline__ void v_absmax_body(const AttnArgs& a, const int hi, c
 }
 
 // Two launches carry the four bodies above: work that does not depend on each other shares a launch, heads fastest so
-// that neighbouring workgroups read neighbouring memory.  Stage 1: anchors (which also clear the V accumulators) and Q.
-// Stage 2: K (needs the anchors) and the V abs-max (needs the cleared accumulators).
+// that neighbouring workgroups read neighbouring memory.  Stage 1: anchors (which also clear the V maxima) and Q.
+// Stage 2: K (needs the anchors) and the V abs-max (needs them cleared).
 template <int DT, int D, int NM>
 __global__ __launch_bounds__(256) void attn_stage1_kernel(AttnArgs a) {
     if (a.parts > 1)   // finished parts, counted by the attention kernel
@@ -680,58 +670,92 @@ __global__ __launch_bounds__(stage2_threads(CK)) void attn_stage2_kernel(AttnArg
     v_absmax_body<DT, D, stage2_threads(CK)>(a, id % a.hk, (id / a.hk) % nc, id / (a.hk * nc));
 }
 
-// V codes: one workgroup per block of 32 keys.  Rows are read as they lie (a thread takes 16 channels of one key),
-// quantized and turned through LDS.  vt[(kv head, block)][d][32]: position h*16 + j of a row holds key
-// (j/4)*8 + h*4 + j%4 of the block, which is the order a lane of the attention kernel holds its 16 scores in.  Keys past
-// lk are zeros.  128 x the column sums go to vsum[(kv head, key tile)][d] by integer atomics.
-template <int DT, int D>
-__global__ __launch_bounds__(256) void attn_v_quant_kernel(AttnArgs a) {
-    constexpr int LPR = lanes_per_row(D), KPP = 256 / LPR;   // keys per pass of the read phase
+// V codes: one workgroup per key tile.  A thread takes eight channels of four keys, so that four codes of a channel are a dword of the
+// order vt[(kv head, block of 32 keys)][d][32], where position h*16 + j of a row holds key (j/4)*8 + h*4 + j%4 of the block: the
+// order a lane of the attention kernel holds its 16 scores in.  The tile is assembled in LDS (eight channels 272 bytes apart: writes of a
+// wave meet in pairs instead of sixteens) and leaves as 16-byte stores.  Keys past lk are zeros.  128 x the column sums of the tile
+// go to vsum[(kv head, key tile)][d].  Bound by the chain of loads: the rows are asked for ahead of the channels' maxima.  A workgroup per 32
+// keys with 16 byte reads and two atomics per output row, rows loaded behind the maxima: 4608 x 24 x 128 13.0 us, this 7.4;
+// 2 x 4096 x 10 x 64 7.8 and 5.5.
+constexpr int v_threads(int CK, int D) { return CK * D / 32; }
+template <int DT, int CK, int D>
+__global__ __launch_bounds__(v_threads(CK, D)) void attn_v_quant_kernel(AttnArgs a) {
+    constexpr int NT = v_threads(CK, D), CPR = D / 8, GROUP = 272, BLOCK = CPR * GROUP;   // bytes of eight channels, of 32 keys
     __shared__ float inv_s[D];
-    __shared__ __align__(16) int8_t tile[32][D];
-    const int hi = blockIdx.x, s = blockIdx.y, bi = blockIdx.z;
+    __shared__ int sums[D];
+    __shared__ __align__(16) uint8_t stage[CK / 32 * BLOCK];
+    const int hi = blockIdx.x, t = blockIdx.y, bi = blockIdx.z;
     const int64_t bh = (int64_t)bi * a.hk + hi;
-    if (threadIdx.x < D) {
-        const float sc = fmax_nn(u2f(a.vmax[bh * D + threadIdx.x]) * (1.f / 127.f), 1e-12f);
-        if (s == 0) a.vs[bh * D + threadIdx.x] = sc;
-        inv_s[threadIdx.x] = 1.f / sc;
-    }
-    __syncthreads();
+    const int c8 = threadIdx.x % CPR, kg = threadIdx.x / CPR, key0 = t * CK + kg * 4;
+    float v[4][8];
+    {
+        const int64_t base = bi * a.v_bs + hi * a.v_hs + c8 * 8;
+        uint4 u[4];
+        if (a.v_vec == 2) {
 #pragma unroll
-    for (int pass = 0; pass < (32 + KPP - 1) / KPP; ++pass) {
-        const int key = pass * KPP + threadIdx.x / LPR, seg = threadIdx.x % LPR;
-        if (key >= 32) break;
-        const int row = s * 32 + key;
-        uint32_t w[4] = {0u, 0u, 0u, 0u};
-        if (row < a.lk) {
-            const int64_t at = bi * a.v_bs + hi * a.v_hs + (int64_t)row * a.v_rs + seg * 16;
+            for (int j = 0; j < 4; ++j)   // rows past the end read the last one
+                u[j] = *reinterpret_cast<const uint4*>((const uint16_t*)a.v + base + (int64_t)(key0 + j < a.lk ? key0 + j : a.lk - 1) * a.v_rs);
 #pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-                float x[4];
-                ld4_dt<DT>(a.v, at + g4 * 4, a.v_vec, x);
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t w[4] = {u[j].x, u[j].y, u[j].z, u[j].w};
 #pragma unroll
-                for (int c = 0; c < 4; ++c) w[g4] |= (uint32_t)(uint8_t)rn_s8(x[c] * inv_s[seg * 16 + g4 * 4 + c]) << (8 * c);
+                for (int e = 0; e < 4; ++e) {
+                    if (DT == DT_BF16) {
+                        v[j][2 * e] = u2f(w[e] << 16);
+                        v[j][2 * e + 1] = u2f(w[e] & 0xffff0000u);
+                    } else {
+                        unpack_f16x2(w[e], v[j][2 * e], v[j][2 * e + 1]);
+                    }
+                }
             }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int e = 0; e < 8; e += 4) {
+                    float x[4];
+                    ld4_dt<DT>(a.v, base + (int64_t)(key0 + j < a.lk ? key0 + j : a.lk - 1) * a.v_rs + e, a.v_vec, x);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) v[j][e + c] = x[c];
+                }
         }
-        *reinterpret_cast<uint4*>(&tile[key][seg * 16]) = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+    for (int d = threadIdx.x; d < D; d += NT) {
+        const float sc = fmax_nn(u2f(a.vmax[bh * D + d]) * (1.f / 127.f), 1e-12f);
+        if (t == 0) a.vs[bh * D + d] = sc;
+        inv_s[d] = 1.f / sc;
+        sums[d] = 0;
     }
     __syncthreads();
+    float inv[8];
 #pragma unroll
-    for (int pass = 0; pass < (2 * D + 255) / 256; ++pass) {
-        const int id = pass * 256 + threadIdx.x;
-        if (id >= 2 * D) break;
-        const int d = id % D, hh = id / D;
-        uint32_t w[4] = {0u, 0u, 0u, 0u};
-        int sum = 0;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int q = tile[(j / 4) * 8 + hh * 4 + (j % 4)][d];
-            sum += q;
-            w[j / 4] |= (uint32_t)(uint8_t)q << (8 * (j % 4));
-        }
-        *reinterpret_cast<uint4*>(a.vt + ((bh * a.nblk + s) * D + d) * 32 + hh * 16) = make_uint4(w[0], w[1], w[2], w[3]);
-        atomicAdd(&a.vsum[(bh * a.kb + s / (a.ck / 32)) * D + d], 128 * sum);
+    for (int e = 0; e < 8; e += 4) {
+        const float4 f = *reinterpret_cast<const float4*>(inv_s + c8 * 8 + e);
+        inv[e] = f.x; inv[e + 1] = f.y; inv[e + 2] = f.z; inv[e + 3] = f.w;
     }
+    // Codes as codes16 makes them: |v| <= 127 scales.  Bytes of keys past lk are cleared.
+    const int left = a.lk - key0;
+    const uint32_t keep = left >= 4 ? 0xffffffffu : left <= 0 ? 0u : (1u << (8 * left)) - 1u;
+    uint8_t* dst = stage + (kg >> 3) * BLOCK + c8 * GROUP + (kg & 1) * 16 + ((kg & 7) >> 1) * 4;
+    constexpr float M = 12582912.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+        *reinterpret_cast<uint32_t*>(dst + e * 32) =
+            pack_low_bytes(v[0][e] * inv[e] + M, v[1][e] * inv[e] + M, v[2][e] * inv[e] + M, v[3][e] * inv[e] + M) & keep;
+    __syncthreads();
+    uint4* out = reinterpret_cast<uint4*>(a.vt + (bh * a.nblk + (int64_t)t * (CK / 32)) * (32 * D));
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int id = i * NT + threadIdx.x, blk = id / (2 * D), d = id / 2 % D;
+        const uint4 w = *reinterpret_cast<const uint4*>(stage + blk * BLOCK + (d / 8) * GROUP + (d % 8) * 32 + (id & 1) * 16);
+        out[id] = w;
+        int sum = 0;
+        for (const uint32_t x : {w.x, w.y, w.z, w.w}) sum = __builtin_amdgcn_sdot4((int)x, 0x01010101, sum, false);
+        sum += dpp_int<0xB1>(sum);   // the row's other half
+        if (!(id & 1)) atomicAdd(&sums[d], sum);
+    }
+    __syncthreads();
+    for (int d = threadIdx.x; d < D; d += NT) a.vsum[(bh * a.kb + t) * D + d] = 128 * sums[d];
 }
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
@@ -1593,7 +1617,8 @@ int run(AttnArgs a, hipStream_t st) {
     } else {
         stages(std::integral_constant<int, NORM_NONE>{});
     }
-    attn_v_quant_kernel<DT, D><<<dim3(a.hk, a.nblk, a.b), 256, 0, st>>>(a);
+    if (a.ck == 64) attn_v_quant_kernel<DT, 64, D><<<dim3(a.hk, a.kb, a.b), v_threads(64, D), 0, st>>>(a);
+    else if constexpr (D != 64) attn_v_quant_kernel<DT, 128, D><<<dim3(a.hk, a.kb, a.b), v_threads(128, D), 0, st>>>(a);
     if (hipGetLastError() != hipSuccess) return -401;
     if constexpr (D == 128) {
         if (a.bias) {
@@ -1660,8 +1685,8 @@ int int8_attn(const void* q, const void* k, const void* v, void* o, void* ws, in
     a.sink = sink;
     a.use_anchor = sink == 0.f ? 1 : 0;   // with a sink a zero key's score must stay zero: no shift (csrc/attn_int8.cu:134-141)
     a.vec_ok = ((o_bs | o_rs | o_hs) % 4 == 0 && ((uintptr_t)o & 7) == 0) ? 1 : 0;
-    a.v_vec = ((v_bs | v_rs | v_hs) % 4 == 0 && ((uintptr_t)v & 7) == 0) ? 1 : 0;
     const auto vec_of = [](int64_t strides, uintptr_t base) { return strides % 8 == 0 && (base & 15) == 0 ? 2 : strides % 4 == 0 && (base & 7) == 0 ? 1 : 0; };
+    a.v_vec = vec_of(v_bs | v_rs | v_hs, (uintptr_t)v);
     a.in_vec = vec_of(q_bs | q_rs | q_hs | k_bs | k_rs | k_hs, (uintptr_t)q | (uintptr_t)k);
     a.bias = bias;
     a.kbias = (float*)(w + p.total);   // the key-bias form's workspace is this much longer
