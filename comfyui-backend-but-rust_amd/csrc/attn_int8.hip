@@ -32,7 +32,7 @@ struct AttnArgs {
     int8_t *qi, *ki, *vt;
     float *qs, *ks, *vs;
     int* anchors;
-    uint32_t* vmax;
+    float* vmax;   // [kv head][v_chunks][D]: largest |v| of each chunk of keys
     int* vsum;
     int b, lq, lk, h, hk, rep, qg, kb, ck, nblk;
     int64_t q_bs, q_rs, q_hs, k_bs, k_rs, k_hs, v_bs, v_rs, v_hs, o_bs, o_rs, o_hs;
@@ -362,7 +362,6 @@ __device__ __forceinline__ void anchor_body(const AttnArgs& a, const int hi, con
     __shared__ int chosen;
     const int tid = threadIdx.x, c = tid & (D - 1);
     const int64_t base = bi * a.k_bs + hi * a.k_hs;
-    if (tid < D) a.vmax[((int64_t)bi * a.hk + hi) * D + c] = 0u;   // the V maxima of this (kv head, batch) start at zero
     bool normed = false;
     if constexpr (D == 128) {
         if (a.k_norm) {
@@ -533,13 +532,12 @@ __device__ __forceinline__ void quant_q_body(const AttnArgs& a, const int hi, co
 // keys past lk are zeros.
 constexpr int stage2_threads(int CK) { return CK == 128 ? 512 : 256; }
 template <int DT, int CK, int D, int NM>
-__device__ __forceinline__ void quant_k_body(const AttnArgs& a, const int hi, const int t, const int bi) {
+__device__ __forceinline__ void quant_k_body(const AttnArgs& a, const int hi, const int t, const int bi, uint8_t* stage) {
     constexpr int NT = stage2_threads(CK), LPR = lanes_per_row(D), RUNS = NT / LPR, NSUB = RUNS / 4;
     constexpr int R = (CK / 4) / NSUB;   // rows per run
     static_assert(R >= 1 && R * NSUB * 4 == CK, "rows of a group divide over its runs");
     __shared__ float omax[RUNS];
     __shared__ __align__(16) float shift[D];
-    __shared__ __align__(16) uint8_t stage[CK * D];
     const int ol = block_of_lane<D>(threadIdx.x & (LPR - 1)), run = threadIdx.x / LPR, g = run & 3, sub = run >> 2;
     const int64_t bh = (int64_t)bi * a.hk + hi, base = bi * a.k_bs + hi * a.k_hs + ol * 16;
     const int anchor = a.anchors[bh];
@@ -607,25 +605,23 @@ __device__ __forceinline__ void quant_k_body(const AttnArgs& a, const int hi, co
         out[i * NT + threadIdx.x] = *reinterpret_cast<const uint4*>(stage + (i * NT + threadIdx.x) * 16);
 }
 
-// V abs-max per channel: NT threads take 128 rows of one (kv head, batch), four channels per thread; non-negative
-// floats order as their bits, so the workgroups combine with an integer atomic max.
-template <int DT, int D, int NT>
+// V abs-max per channel over a chunk of the keys of one (kv head, batch), four channels per thread.  The chunks' maxima are
+// stored side by side and folded by every workgroup that needs them: 32 chunks at most, which a fold reads in one trip.
+__host__ __device__ constexpr int v_chunks(int lk) { return lk >= 32 * 128 ? 32 : (lk + 127) / 128; }
+template <int DT, int D>
 __device__ __forceinline__ void v_absmax_body(const AttnArgs& a, const int hi, const int chunk, const int bi) {
-    constexpr int TPR = D / 4, RL = NT / TPR;   // threads per row, rows per pass
+    constexpr int TPR = D / 4, RL = 256 / TPR;   // threads per row, rows per pass
     __shared__ float red[RL][D];
-    const int c4 = threadIdx.x % TPR, rl = threadIdx.x / TPR;
+    const int c4 = threadIdx.x % TPR, rl = threadIdx.x / TPR, chunks = v_chunks(a.lk);
     const int64_t base = bi * a.v_bs + hi * a.v_hs + c4 * 4;
     float mx[4] = {0.f, 0.f, 0.f, 0.f};
-    const int r0 = chunk * 128;
-#pragma unroll 4
-    for (int i = 0; i < 128 / RL; ++i) {
-        const int r = r0 + rl + RL * i;
-        if (r < a.lk) {
-            float x[4];
-            ld4_dt<DT>(a.v, base + (int64_t)r * a.v_rs, a.v_vec, x);
+    const int rows = (a.lk + chunks - 1) / chunks, r0 = chunk * rows, r1 = r0 + rows < a.lk ? r0 + rows : a.lk;
+#pragma unroll 8
+    for (int r = r0 + rl; r < r1; r += RL) {
+        float x[4];
+        ld4_dt<DT>(a.v, base + (int64_t)r * a.v_rs, a.v_vec, x);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) mx[c] = fmax_nn(mx[c], fabsf(x[c]));
-        }
+        for (int c = 0; c < 4; ++c) mx[c] = fmax_nn(mx[c], fabsf(x[c]));
     }
 #pragma unroll
     for (int c = 0; c < 4; ++c) red[rl][c4 * 4 + c] = mx[c];
@@ -634,13 +630,133 @@ __device__ __forceinline__ void v_absmax_body(const AttnArgs& a, const int hi, c
         float m = 0.f;
 #pragma unroll
         for (int i = 0; i < RL; ++i) m = fmax_nn(m, red[i][threadIdx.x]);
-        atomicMax(&a.vmax[((int64_t)bi * a.hk + hi) * D + threadIdx.x], f2u(m));
+        a.vmax[(((int64_t)bi * a.hk + hi) * chunks + chunk) * D + threadIdx.x] = m;
+    }
+}
+
+// V codes: a workgroup per key tile (two tiles of 64 keys at head dim 64).  A thread takes eight channels of four keys, so that four codes
+// of a channel are a dword of the order vt[(kv head, block of 32 keys)][d][32], where position h*16 + j of a row holds key
+// (j/4)*8 + h*4 + j%4 of the block: the order a lane of the attention kernel holds its 16 scores in.  The tile is assembled in LDS
+// (eight channels 272 bytes apart: writes of a wave meet in pairs instead of sixteens) and leaves as 16-byte stores.  Keys past lk
+// are zeros.  128 x the column sums of a tile go to vsum[(kv head, key tile)][d].  Bound by the chain of loads: the rows are asked for
+// ahead of the channels' maxima.  A workgroup per 32 keys with 16 byte reads and two atomics per output row, rows loaded behind the
+// maxima, as a launch of its own: 4608 x 24 x 128 13.0 us, this, as a launch of its own, 7.4; 2 x 4096 x 10 x 64 7.8 and 5.5.
+constexpr int v_tiles(int CK, int D) { return stage2_threads(CK) * 32 / D > CK ? 2 : 1; }
+constexpr int v_stage_bytes(int CK, int D) { return v_tiles(CK, D) * CK / 32 * (D / 8) * 272; }
+template <int DT, int CK, int D>
+__device__ __forceinline__ void quant_v_body(const AttnArgs& a, const int hi, const int unit, const int bi, uint8_t* stage) {
+    constexpr int NT = stage2_threads(CK), CPR = D / 8, GROUP = 272, BLOCK = CPR * GROUP;   // bytes of eight channels, of 32 keys
+    constexpr int TILES = v_tiles(CK, D), KEYS = TILES * CK, KPP = NT / CPR * 4, PASSES = KEYS / KPP, PARTS = NT / D;
+    static_assert(PASSES * KPP == KEYS && PARTS >= 1 && PARTS * D == NT, "threads divide over keys and channels");
+    __shared__ float part_max[PARTS][D];
+    __shared__ __align__(16) float inv_s[D];
+    __shared__ int sums[TILES][D];
+    const int64_t bh = (int64_t)bi * a.hk + hi;
+    const int c8 = threadIdx.x % CPR, kg = threadIdx.x / CPR, key0 = unit * KEYS + kg * 4;
+    const int64_t base = bi * a.v_bs + hi * a.v_hs + c8 * 8;
+    float v[PASSES][4][8];
+    const auto row_at = [&](int p, int j) {   // rows past the end read the last one
+        const int key = key0 + p * KPP + j;
+        return base + (int64_t)(key < a.lk ? key : a.lk - 1) * a.v_rs;
+    };
+    if (a.v_vec == 2) {
+        uint4 u[PASSES][4];
+#pragma unroll
+        for (int p = 0; p < PASSES; ++p)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) u[p][j] = *reinterpret_cast<const uint4*>((const uint16_t*)a.v + row_at(p, j));
+#pragma unroll
+        for (int p = 0; p < PASSES; ++p)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t w[4] = {u[p][j].x, u[p][j].y, u[p][j].z, u[p][j].w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (DT == DT_BF16) {
+                        v[p][j][2 * e] = u2f(w[e] << 16);
+                        v[p][j][2 * e + 1] = u2f(w[e] & 0xffff0000u);
+                    } else {
+                        unpack_f16x2(w[e], v[p][j][2 * e], v[p][j][2 * e + 1]);
+                    }
+                }
+            }
+    } else {
+#pragma unroll
+        for (int p = 0; p < PASSES; ++p)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int e = 0; e < 8; e += 4) {
+                    float x[4];
+                    ld4_dt<DT>(a.v, row_at(p, j) + e, a.v_vec, x);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) v[p][j][e + c] = x[c];
+                }
+    }
+    {
+        const int d = threadIdx.x % D, part = threadIdx.x / D, chunks = v_chunks(a.lk);
+        const float* src = a.vmax + bh * chunks * D + d;
+        float m = 0.f;
+#pragma unroll
+        for (int i = 0; i < 32 / PARTS; ++i) {   // a chunk twice changes nothing
+            const int c = i * PARTS + part;
+            m = fmax_nn(m, src[(c < chunks ? c : chunks - 1) * D]);
+        }
+        part_max[part][d] = m;
+        __syncthreads();
+        if (threadIdx.x < D) {
+            m = 0.f;
+#pragma unroll
+            for (int i = 0; i < PARTS; ++i) m = fmax_nn(m, part_max[i][d]);
+            const float sc = fmax_nn(m * (1.f / 127.f), 1e-12f);
+            if (unit == 0) a.vs[bh * D + d] = sc;
+            inv_s[d] = 1.f / sc;
+#pragma unroll
+            for (int i = 0; i < TILES; ++i) sums[i][d] = 0;
+        }
+    }
+    __syncthreads();
+    float inv[8];
+#pragma unroll
+    for (int e = 0; e < 8; e += 4) {
+        const float4 f = *reinterpret_cast<const float4*>(inv_s + c8 * 8 + e);
+        inv[e] = f.x; inv[e + 1] = f.y; inv[e + 2] = f.z; inv[e + 3] = f.w;
+    }
+    // Codes as codes16 makes them: |v| <= 127 scales.  Bytes of keys past lk are cleared.
+    constexpr float M = 12582912.f;
+#pragma unroll
+    for (int p = 0; p < PASSES; ++p) {
+        const int left = a.lk - (key0 + p * KPP), k4 = kg + p * (KPP / 4);
+        const uint32_t keep = left >= 4 ? 0xffffffffu : left <= 0 ? 0u : (1u << (8 * left)) - 1u;
+        uint8_t* dst = stage + (k4 >> 3) * BLOCK + c8 * GROUP + (k4 & 1) * 16 + ((k4 & 7) >> 1) * 4;
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            *reinterpret_cast<uint32_t*>(dst + e * 32) =
+                pack_low_bytes(v[p][0][e] * inv[e] + M, v[p][1][e] * inv[e] + M, v[p][2][e] * inv[e] + M, v[p][3][e] * inv[e] + M) & keep;
+    }
+    __syncthreads();
+    uint4* out = reinterpret_cast<uint4*>(a.vt + (bh * a.nblk + (int64_t)unit * (KEYS / 32)) * (32 * D));
+#pragma unroll
+    for (int i = 0; i < 2 * PASSES; ++i) {
+        const int id = i * NT + threadIdx.x, blk = id / (2 * D), d = id / 2 % D;
+        const uint4 w = *reinterpret_cast<const uint4*>(stage + blk * BLOCK + (d / 8) * GROUP + (d % 8) * 32 + (id & 1) * 16);
+        if (TILES == 1 || unit * TILES + blk / (CK / 32) < a.kb) out[id] = w;
+        int sum = 0;
+        for (const uint32_t x : {w.x, w.y, w.z, w.w}) sum = __builtin_amdgcn_sdot4((int)x, 0x01010101, sum, false);
+        sum += dpp_int<0xB1>(sum);   // the row's other half
+        if (!(id & 1)) atomicAdd(&sums[blk / (CK / 32)][d], sum);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < TILES * D; i += NT) {
+        const int t = unit * TILES + i / D;
+        if (t < a.kb) a.vsum[(bh * a.kb + t) * D + i % D] = 128 * sums[i / D][i % D];
     }
 }
 
 // Two launches carry the four bodies above: work that does not depend on each other shares a launch, heads fastest so
-// that neighbouring workgroups read neighbouring memory.  Stage 1: anchors (which also clear the V maxima) and Q.
-// Stage 2: K (needs the anchors) and the V abs-max (needs them cleared).
+// that neighbouring workgroups read neighbouring memory.  Stage 1: anchors, the V maxima and Q.  Stage 2: K (needs the anchors) and V
+// (needs the maxima).  Three launches, the maxima beside K and combined by atomics on memory that stage 1 cleared: 4608 x 24 x 128
+// with norm and rope 245.3 us a call, this way 236.3; 2 x 4096 x 10 x 64 112.8 and 108.7.
 template <int DT, int D, int NM>
 __global__ __launch_bounds__(256) void attn_stage1_kernel(AttnArgs a) {
     if (a.parts > 1)   // finished parts, counted by the attention kernel
@@ -652,6 +768,12 @@ __global__ __launch_bounds__(256) void attn_stage1_kernel(AttnArgs a) {
         return;
     }
     id -= n_anchor;
+    const int chunks = v_chunks(a.lk), n_v = a.hk * chunks * a.b;
+    if (id < n_v) {
+        v_absmax_body<DT, D>(a, id % a.hk, (id / a.hk) % chunks, id / (a.hk * chunks));
+        return;
+    }
+    id -= n_v;
     constexpr int GPB = 4 * q_groups_per_wave(D);   // scale groups per workgroup
     const int ny = (a.qg * 8 + GPB - 1) / GPB;
     quant_q_body<DT, D, NM>(a, id % a.h, (id / a.h) % ny, id / (a.h * ny));
@@ -659,103 +781,16 @@ __global__ __launch_bounds__(256) void attn_stage1_kernel(AttnArgs a) {
 
 template <int DT, int CK, int D, int NM>
 __global__ __launch_bounds__(stage2_threads(CK)) void attn_stage2_kernel(AttnArgs a) {
+    __shared__ __align__(16) uint8_t stage[v_stage_bytes(CK, D) > CK * D ? v_stage_bytes(CK, D) : CK * D];
     int id = blockIdx.x;
     const int n_k = a.hk * a.kb * a.b;
     if (id < n_k) {
-        quant_k_body<DT, CK, D, NM>(a, id % a.hk, (id / a.hk) % a.kb, id / (a.hk * a.kb));
+        quant_k_body<DT, CK, D, NM>(a, id % a.hk, (id / a.hk) % a.kb, id / (a.hk * a.kb), stage);
         return;
     }
     id -= n_k;
-    const int nc = (a.lk + 127) / 128;
-    v_absmax_body<DT, D, stage2_threads(CK)>(a, id % a.hk, (id / a.hk) % nc, id / (a.hk * nc));
-}
-
-// V codes: one workgroup per key tile.  A thread takes eight channels of four keys, so that four codes of a channel are a dword of the
-// order vt[(kv head, block of 32 keys)][d][32], where position h*16 + j of a row holds key (j/4)*8 + h*4 + j%4 of the block: the
-// order a lane of the attention kernel holds its 16 scores in.  The tile is assembled in LDS (eight channels 272 bytes apart: writes of a
-// wave meet in pairs instead of sixteens) and leaves as 16-byte stores.  Keys past lk are zeros.  128 x the column sums of the tile
-// go to vsum[(kv head, key tile)][d].  Bound by the chain of loads: the rows are asked for ahead of the channels' maxima.  A workgroup per 32
-// keys with 16 byte reads and two atomics per output row, rows loaded behind the maxima: 4608 x 24 x 128 13.0 us, this 7.4;
-// 2 x 4096 x 10 x 64 7.8 and 5.5.
-constexpr int v_threads(int CK, int D) { return CK * D / 32; }
-template <int DT, int CK, int D>
-__global__ __launch_bounds__(v_threads(CK, D)) void attn_v_quant_kernel(AttnArgs a) {
-    constexpr int NT = v_threads(CK, D), CPR = D / 8, GROUP = 272, BLOCK = CPR * GROUP;   // bytes of eight channels, of 32 keys
-    __shared__ float inv_s[D];
-    __shared__ int sums[D];
-    __shared__ __align__(16) uint8_t stage[CK / 32 * BLOCK];
-    const int hi = blockIdx.x, t = blockIdx.y, bi = blockIdx.z;
-    const int64_t bh = (int64_t)bi * a.hk + hi;
-    const int c8 = threadIdx.x % CPR, kg = threadIdx.x / CPR, key0 = t * CK + kg * 4;
-    float v[4][8];
-    {
-        const int64_t base = bi * a.v_bs + hi * a.v_hs + c8 * 8;
-        uint4 u[4];
-        if (a.v_vec == 2) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)   // rows past the end read the last one
-                u[j] = *reinterpret_cast<const uint4*>((const uint16_t*)a.v + base + (int64_t)(key0 + j < a.lk ? key0 + j : a.lk - 1) * a.v_rs);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t w[4] = {u[j].x, u[j].y, u[j].z, u[j].w};
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    if (DT == DT_BF16) {
-                        v[j][2 * e] = u2f(w[e] << 16);
-                        v[j][2 * e + 1] = u2f(w[e] & 0xffff0000u);
-                    } else {
-                        unpack_f16x2(w[e], v[j][2 * e], v[j][2 * e + 1]);
-                    }
-                }
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int e = 0; e < 8; e += 4) {
-                    float x[4];
-                    ld4_dt<DT>(a.v, base + (int64_t)(key0 + j < a.lk ? key0 + j : a.lk - 1) * a.v_rs + e, a.v_vec, x);
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) v[j][e + c] = x[c];
-                }
-        }
-    }
-    for (int d = threadIdx.x; d < D; d += NT) {
-        const float sc = fmax_nn(u2f(a.vmax[bh * D + d]) * (1.f / 127.f), 1e-12f);
-        if (t == 0) a.vs[bh * D + d] = sc;
-        inv_s[d] = 1.f / sc;
-        sums[d] = 0;
-    }
-    __syncthreads();
-    float inv[8];
-#pragma unroll
-    for (int e = 0; e < 8; e += 4) {
-        const float4 f = *reinterpret_cast<const float4*>(inv_s + c8 * 8 + e);
-        inv[e] = f.x; inv[e + 1] = f.y; inv[e + 2] = f.z; inv[e + 3] = f.w;
-    }
-    // Codes as codes16 makes them: |v| <= 127 scales.  Bytes of keys past lk are cleared.
-    const int left = a.lk - key0;
-    const uint32_t keep = left >= 4 ? 0xffffffffu : left <= 0 ? 0u : (1u << (8 * left)) - 1u;
-    uint8_t* dst = stage + (kg >> 3) * BLOCK + c8 * GROUP + (kg & 1) * 16 + ((kg & 7) >> 1) * 4;
-    constexpr float M = 12582912.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-        *reinterpret_cast<uint32_t*>(dst + e * 32) =
-            pack_low_bytes(v[0][e] * inv[e] + M, v[1][e] * inv[e] + M, v[2][e] * inv[e] + M, v[3][e] * inv[e] + M) & keep;
-    __syncthreads();
-    uint4* out = reinterpret_cast<uint4*>(a.vt + (bh * a.nblk + (int64_t)t * (CK / 32)) * (32 * D));
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int id = i * NT + threadIdx.x, blk = id / (2 * D), d = id / 2 % D;
-        const uint4 w = *reinterpret_cast<const uint4*>(stage + blk * BLOCK + (d / 8) * GROUP + (d % 8) * 32 + (id & 1) * 16);
-        out[id] = w;
-        int sum = 0;
-        for (const uint32_t x : {w.x, w.y, w.z, w.w}) sum = __builtin_amdgcn_sdot4((int)x, 0x01010101, sum, false);
-        sum += dpp_int<0xB1>(sum);   // the row's other half
-        if (!(id & 1)) atomicAdd(&sums[d], sum);
-    }
-    __syncthreads();
-    for (int d = threadIdx.x; d < D; d += NT) a.vsum[(bh * a.kb + t) * D + d] = 128 * sums[d];
+    const int units = (a.kb + v_tiles(CK, D) - 1) / v_tiles(CK, D);
+    quant_v_body<DT, CK, D>(a, id % a.hk, (id / a.hk) % units, id / (a.hk * units), stage);
 }
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
@@ -1569,7 +1604,7 @@ Plan plan_for(int64_t b, int64_t h, int64_t hk, int64_t lq, int64_t lk, int D) {
     p.vt = add(b * hk * (int64_t)p.nblk * D * 32);
     p.vs = add(b * hk * D * 4);
     p.anchors = add(b * hk * 4);
-    p.vmax = add(b * hk * D * 4);
+    p.vmax = add(b * hk * v_chunks((int)lk) * D * 4);
     p.vsum = add(b * hk * (int64_t)p.kb * D * 4);
     const int64_t row_blocks = b * h * ((lq + 127) / 128);
     p.parts = key_parts(row_blocks, p.kb, p.ck, D, p.whole);
@@ -1601,8 +1636,9 @@ int launch_pipe(const AttnArgs& a, hipStream_t st) {
 template <int DT, int D>
 int run(AttnArgs a, hipStream_t st) {
     constexpr int GPB = 4 * q_groups_per_wave(D);   // scale groups per workgroup of the Q quantizer
-    const int64_t n1 = (int64_t)a.hk * a.b + (int64_t)a.h * ((a.qg * 8 + GPB - 1) / GPB) * a.b;
-    const int64_t n2 = (int64_t)a.hk * a.kb * a.b + (int64_t)a.hk * ((a.lk + 127) / 128) * a.b;
+    const int tiles = v_tiles(a.ck, D);
+    const int64_t n1 = (int64_t)a.hk * a.b * (1 + v_chunks(a.lk)) + (int64_t)a.h * ((a.qg * 8 + GPB - 1) / GPB) * a.b;
+    const int64_t n2 = (int64_t)a.hk * a.b * (a.kb + (a.kb + tiles - 1) / tiles);
     if (n1 > 0x7fffffff || n2 > 0x7fffffff) return -400;
     const auto stages = [&](auto nm) {
         constexpr int NM = decltype(nm)::value;
@@ -1617,8 +1653,6 @@ int run(AttnArgs a, hipStream_t st) {
     } else {
         stages(std::integral_constant<int, NORM_NONE>{});
     }
-    if (a.ck == 64) attn_v_quant_kernel<DT, 64, D><<<dim3(a.hk, a.kb, a.b), v_threads(64, D), 0, st>>>(a);
-    else if constexpr (D != 64) attn_v_quant_kernel<DT, 128, D><<<dim3(a.hk, a.kb, a.b), v_threads(128, D), 0, st>>>(a);
     if (hipGetLastError() != hipSuccess) return -401;
     if constexpr (D == 128) {
         if (a.bias) {
@@ -1674,7 +1708,7 @@ int int8_attn(const void* q, const void* k, const void* v, void* o, void* ws, in
     a.q = q; a.k = k; a.v = v; a.o = o;
     a.qi = (int8_t*)(w + p.qi); a.ki = (int8_t*)(w + p.ki); a.vt = (int8_t*)(w + p.vt);
     a.qs = (float*)(w + p.qs); a.ks = (float*)(w + p.ks); a.vs = (float*)(w + p.vs);
-    a.anchors = (int*)(w + p.anchors); a.vmax = (uint32_t*)(w + p.vmax); a.vsum = (int*)(w + p.vsum);
+    a.anchors = (int*)(w + p.anchors); a.vmax = (float*)(w + p.vmax); a.vsum = (int*)(w + p.vsum);
     a.b = b; a.lq = lq; a.lk = lk; a.h = h; a.hk = hk; a.rep = h / hk;
     a.parts = p.parts; a.whole = (int)p.whole; a.done = (uint32_t*)(w + p.done); a.part = (float*)(w + p.part);
     a.qg = p.qg; a.kb = p.kb; a.ck = p.ck; a.nblk = p.nblk;

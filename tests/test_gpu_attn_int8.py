@@ -834,3 +834,26 @@ def test_attention_integer_sums_at_their_limits(D, lk, keys):
     # smallest probability's share at most
     assert (np.abs(got - ref) <= 2.0 / 255.0 * np.abs(ref)).all()
     assert np.abs(ref).min() > 0.5
+
+
+@pytest.mark.parametrize("case", [
+    # an odd number of 64-key tiles (two to a workgroup), chunks of the maxima that do not divide the keys, 32 chunks and more keys
+    # than 32 x 128, two passes of a workgroup over a tile of head dim 256
+    (64, 1, 40, 65, 1, 1, torch.bfloat16, 0.0), (64, 2, 33, 130, 2, 1, torch.float16, 0.0), (64, 1, 20, 4225, 1, 1, torch.bfloat16, 0.0),
+    (128, 1, 20, 4100, 2, 1, torch.bfloat16, 0.0), (128, 1, 20, 5000, 1, 1, torch.float16, 0.0), (256, 1, 20, 1027, 1, 1, torch.bfloat16, 0.0),
+    (256, 1, 20, 300, 2, 1, torch.float16, 0.0),
+], ids=lambda c: "D%d_lk%d" % (c[0], c[3]))
+def test_attention_value_codes_tile_by_tile(case):
+    test_attention_head_dims_64_and_256(case)
+
+
+@pytest.mark.parametrize("D,at", [(64, 1), (64, 4), (128, 4), (256, 1)])
+def test_attention_values_off_16_bytes(D, at):
+    """V that starts on 2 and on 8 bytes takes narrower loads; the same bits."""
+    ql, ffi = _pkg()
+    lq, lk, h = 40, 331, 2
+    q, k, v = (t.cuda() for t in _inputs(1, lq, lk, h, h, torch.bfloat16, seed=D + at, D=D))
+    wide = torch.zeros(1, lk, h, D + 8, dtype=torch.bfloat16, device="cuda")
+    moved = wide[..., at:at + D]
+    moved.copy_(v)
+    assert torch.equal(ql.int8_attn(q, k, moved, 0.1), ql.int8_attn(q, k, v, 0.1))
