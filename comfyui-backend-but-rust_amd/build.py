@@ -50,11 +50,27 @@ def build_blas():
     return BLAS_OUT
 
 
+CALLS_OUT = os.path.join(HERE, "_pycalls.so")
+
+
+def build_calls():
+    """The Python calls that are native code (csrc/py_linear.cpp): host code only, against torch's headers and libgpu_kernels.so."""
+    import sysconfig
+    import torch
+    t, rocm = os.path.dirname(torch.__file__), os.environ.get("ROCM_PATH", "/opt/rocm")
+    subprocess.check_call(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+                           "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI), "-isystem", os.path.join(t, "include"),
+                           "-isystem", os.path.join(rocm, "include"), "-isystem", sysconfig.get_paths()["include"],
+                           os.path.join(CSRC, "py_linear.cpp"), "-o", CALLS_OUT, "-L" + os.path.join(t, "lib"), "-L" + HERE, "-lgpu_kernels",
+                           "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", "-Wl,-rpath,$ORIGIN"])
+    return CALLS_OUT
+
+
 def stale():
     if not os.path.exists(OUT):
         return True
     t = os.path.getmtime(OUT)
-    if not os.path.exists(BLAS_OUT):
+    if not os.path.exists(BLAS_OUT) or not os.path.exists(CALLS_OUT):
         return True
     deps = [os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith((".hip", ".hpp", ".cpp"))]
     deps.append(os.path.join(os.path.dirname(HERE), "include", "gpu_api.h"))
@@ -68,6 +84,7 @@ def build(force=True):
         objs = list(ex.map(_compile, SOURCES))
     subprocess.check_call(["hipcc", "--offload-arch=" + ARCH, "-shared", "-fPIC", "-o", OUT, *objs])
     build_blas()
+    build_calls()
     return OUT
 
 

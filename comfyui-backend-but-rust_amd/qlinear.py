@@ -5,6 +5,7 @@ the stream; all arithmetic happens in libgpu_kernels.so.
 import torch
 
 from . import ffi
+from . import _pycalls   # csrc/py_linear.cpp, built beside libgpu_kernels.so
 
 _TORCH_DT = {torch.float32: ffi.DT_F32, torch.float16: ffi.DT_F16, torch.bfloat16: ffi.DT_BF16}
 _DT_TORCH = {v: k for k, v in _TORCH_DT.items()}
@@ -276,6 +277,12 @@ def w6a8_group_gemm(A, packed, xs, sw, bias=None, out_dtype=torch.bfloat16, want
 
 def linear_w8a8(x, W, ws, bias=None, rotate=0, out_dtype=None):
     """One W8A8 linear: y = dequant(quant(x) . W^T)."""
+    y = _pycalls.linear_w8a8(x, W, ws, bias, rotate, out_dtype)
+    return _linear_w8a8(x, W, ws, bias, rotate, out_dtype) if y is None else y
+
+
+def _linear_w8a8(x, W, ws, bias, rotate, out_dtype):
+    """The call in Python: what the native one leaves to it, and every refusal."""
     out_dtype = x.dtype if out_dtype is None else out_dtype
     _rows(x)
     _dense(W, ws, bias)

@@ -1889,3 +1889,48 @@ def test_quant_rows_random_shapes_and_data_bit_exact(seed):
         assert rc == 0
         assert np.array_equal(sd.cpu().numpy().view(np.uint32), s.view(np.uint32)), (which, M, K, stride, rotate)
         assert np.array_equal(qd.cpu().numpy(), q), (which, M, K, stride, rotate)
+
+
+@pytest.mark.parametrize("M,K,N,rotate,dtype,bias,out", [(1, 256, 96, 256, torch.bfloat16, True, None), (8, 1024, 200, 0, torch.float32, False, None),
+                                                         (9, 1024, 200, 128, torch.bfloat16, True, None), (3, 1088, 136, 64, torch.bfloat16, False, torch.float32),
+                                                         (200, 512, 384, 256, torch.bfloat16, True, torch.float16)])
+def test_linear_call_native_and_in_python(M, K, N, rotate, dtype, bias, out):
+    """The native call and the Python one behind it: the same outputs, on a row stride of its own too, and under a dispatch mode,
+    which the native one leaves to Python."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Seen(TorchDispatchMode):
+        names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    g = torch.Generator().manual_seed(M + K)
+    wide = torch.randn(M, K + 8, generator=g).to(dtype).to(DEV)
+    W, ws = torch.randint(-127, 128, (N, K), dtype=torch.int8, generator=g).to(DEV), torch.rand(N, generator=g).to(DEV)
+    b = torch.randn(N, generator=g).to(out or dtype).to(DEV) if bias else None
+    for x in (wide[:, :K], wide[:, :K].contiguous()):
+        native = ql._pycalls.linear_w8a8(x, W, ws, b, rotate, out)
+        assert native is not None and native.dtype == (out or dtype) and not native.requires_grad
+        want = ql._linear_w8a8(x, W, ws, b, rotate, out)
+        with Seen():
+            assert ql._pycalls.linear_w8a8(x, W, ws, b, rotate, out) is None
+            seen = ql.linear_w8a8(x, W, ws, b, rotate, out)
+        assert any("empty" in n for n in Seen.names)
+        assert torch.equal(native, want) and torch.equal(seen, want)
+
+
+def test_linear_call_refuses_in_python_what_the_native_one_does_not_take():
+    x, W, ws = torch.zeros(3, 256, dtype=torch.bfloat16, device=DEV), torch.zeros(64, 256, dtype=torch.int8, device=DEV), torch.ones(64, device=DEV)
+    class Sub(torch.Tensor):
+        pass
+    assert ql._pycalls.linear_w8a8(x.as_subclass(Sub), W, ws, None, 256, None) is None
+    assert torch.equal(ql.linear_w8a8(x.as_subclass(Sub), W, ws, None, 256), ql.linear_w8a8(x, W, ws, None, 256))
+    assert ql.linear_w8a8(x[:0], W, ws).shape == (0, 64)
+    for bad in ((x.cpu(), W, ws), (x.t(), W, ws), (x, W.t(), ws), (x, W.float(), ws), (x, W, ws.double()), (x, W[:, :128].contiguous(), ws),
+                (x, W, ws, torch.zeros(64, device=DEV))):
+        with pytest.raises(ValueError):
+            ql.linear_w8a8(*bad)
+    with pytest.raises(ffi.KernelError):
+        ql.linear_w8a8(x[:, :200].contiguous(), W[:, :200].contiguous(), ws)   # K % 64
