@@ -103,7 +103,7 @@ template <int DT> __device__ __forceinline__ void st_dt(void* p, int64_t i, floa
 }
 template <int DT> struct dt_size { static constexpr int value = DT == DT_F32 ? 4 : 2; };
 
-// Two floats -> packed f16 pair, and back.  The empty asm for the reason given at f_to_f16.
+// Two floats -> packed f16 pair as one v_cvt_pk_f16_f32, and back.  The empty asm for the reason given at f_to_f16.
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack_f16x2(float a, float b) {
     asm("" : "+v"(a), "+v"(b));
@@ -227,8 +227,8 @@ template <int OUT_DT> __device__ __forceinline__ void store4(void* p, int64_t i,
         *reinterpret_cast<uint2*>((uint16_t*)p + i) = u;
     } else {
         uint2 u;
-        u.x = (uint32_t)f_to_f16(v[0]) | ((uint32_t)f_to_f16(v[1]) << 16);
-        u.y = (uint32_t)f_to_f16(v[2]) | ((uint32_t)f_to_f16(v[3]) << 16);
+        u.x = pack_f16x2(v[0], v[1]);
+        u.y = pack_f16x2(v[2], v[3]);
         *reinterpret_cast<uint2*>((uint16_t*)p + i) = u;
     }
 }

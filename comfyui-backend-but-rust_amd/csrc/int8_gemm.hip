@@ -19,6 +19,7 @@ namespace {
 
 __device__ __forceinline__ void store16_untracked(void* ptr, uint4 v);
 __device__ __forceinline__ void store16_untracked_at(const void* base, uint32_t off, uint4 v);
+__device__ __forceinline__ void store16_cached_at(const void* base, uint32_t off, uint4 v);
 // A 64-bit value that is the same in every lane, moved to scalar registers.
 __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
     const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
@@ -42,6 +43,7 @@ struct GemmArgs {
     uint32_t magic;   // panel_magic(tiles_m, tiles_n), for tile_of_block
     int kslice;   // K of a split-K slice (a multiple of 128), 0 = no split
     int n_first;  // two-group kernel: the first column of these tiles
+    bool cached;  // two-group kernel: whole wave tiles are stored with the caches' default policy (launch_pp)
 };
 
 template <int BM_, int BN_, int BK_, int WGM_, int WGN_, int OCC_>
@@ -287,8 +289,7 @@ __device__ __forceinline__ void epilogue_shuffle_with(const GemmArgs& p, Acc& ac
                         } else if (OUT_DT == DT_BF16) {
                             *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
                         } else {
-                            *reinterpret_cast<uint2*>(dst) = make_uint2((uint32_t)f_to_f16(o[0]) | ((uint32_t)f_to_f16(o[1]) << 16),
-                                                                        (uint32_t)f_to_f16(o[2]) | ((uint32_t)f_to_f16(o[3]) << 16));
+                            *reinterpret_cast<uint2*>(dst) = make_uint2(pack_f16x2(o[0], o[1]), pack_f16x2(o[2], o[3]));
                         }
                     }
                 }
@@ -320,9 +321,9 @@ __device__ __forceinline__ void epilogue_shuffle_with(const GemmArgs& p, Acc& ac
                     z0 = u2f(zw[j] << 16); z1 = u2f(zw[j] & 0xffff0000u); r0 = u2f(rw[j] << 16); r1 = u2f(rw[j] & 0xffff0000u);
                     ow[j] = pack_bf16x2(__builtin_fmaf(z0, rs[np][2 * j], r0), __builtin_fmaf(z1, rs[np][2 * j + 1], r1));
                 } else {
-                    z0 = f16_to_f((uint16_t)(zw[j] & 0xffffu)); z1 = f16_to_f((uint16_t)(zw[j] >> 16));
-                    r0 = f16_to_f((uint16_t)(rw[j] & 0xffffu)); r1 = f16_to_f((uint16_t)(rw[j] >> 16));
-                    ow[j] = (uint32_t)f_to_f16(__builtin_fmaf(z0, rs[np][2 * j], r0)) | ((uint32_t)f_to_f16(__builtin_fmaf(z1, rs[np][2 * j + 1], r1)) << 16);
+                    unpack_f16x2(zw[j], z0, z1);
+                    unpack_f16x2(rw[j], r0, r1);
+                    ow[j] = pack_f16x2(__builtin_fmaf(z0, rs[np][2 * j], r0), __builtin_fmaf(z1, rs[np][2 * j + 1], r1));
                 }
             }
         }
@@ -331,13 +332,13 @@ __device__ __forceinline__ void epilogue_shuffle_with(const GemmArgs& p, Acc& ac
     auto store_piece = [&](int im, int np, const uint4* v, const uint4* rv) {
         if (full) {
             const uint64_t piece = tile_base + (uint64_t)(im * 32) * row_bytes + (uint64_t)(np * PW * SZ);
+            const auto each = [&](auto store) {
 #pragma unroll
-            for (int t = 0; t < PASSES; ++t) {
-                const uint64_t pass = piece + (uint64_t)(t * RPI) * row_bytes;
-                const uint4 o = finish(np, v[t], rv[t]);
-                if (UNTRACKED) store16_untracked_at((const void*)pass, lane_off, o);
-                else *reinterpret_cast<uint4*>((uint8_t*)pass + lane_off) = o;
-            }
+                for (int t = 0; t < PASSES; ++t) store((const void*)(piece + (uint64_t)(t * RPI) * row_bytes), finish(np, v[t], rv[t]));
+            };
+            if (!UNTRACKED) each([&](const void* at, const uint4& x) { *reinterpret_cast<uint4*>((uint8_t*)at + lane_off) = x; });
+            else if (EPI != EPI_RESID && p.cached) each([&](const void* at, const uint4& x) { store16_cached_at(at, lane_off, x); });
+            else each([&](const void* at, const uint4& x) { store16_untracked_at(at, lane_off, x); });
             return;
         }
         int l = lane;
@@ -549,6 +550,11 @@ __device__ __forceinline__ void store16_untracked(void* ptr, uint4 v) {
 __device__ __forceinline__ void store16_untracked_at(const void* base, uint32_t off, uint4 v) {
     const v4i d = v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
     asm volatile("global_store_dwordx4 %0, %1, %2 nt\n\ts_nop 1" ::"v"(off), "v"(d), "s"(base) : "memory");
+}
+// The same with the caches' default policy.
+__device__ __forceinline__ void store16_cached_at(const void* base, uint32_t off, uint4 v) {
+    const v4i d = v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
+    asm volatile("global_store_dwordx4 %0, %1, %2\n\ts_nop 1" ::"v"(off), "v"(d), "s"(base) : "memory");
 }
 
 template <int N> __device__ __forceinline__ void wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
@@ -1242,6 +1248,12 @@ int launch_pp(GemmArgs a, hipStream_t st) {
     if (!aligned) return launch_cfg<CfgM, OUT_DT, EPI>(a, st);   // this kernel has only the coalesced epilogue
     const int64_t G = device_cu_count();
     const PpSplit sp = pp_split(a.M, a.N, G);
+    // Outputs that the last-level cache (256 MB) holds beside the operands stay there for whoever reads them next; larger ones pass by it.
+    // GEMM, and with the quantizer that reads its output, us, non-temporal and cached: 84 MB 8192 x 640 -> 5120 38.2 / 71.7 and 36.4 / 68.5,
+    // 4096 x 1280 -> 10240 55.5 / 88.7 and 53.6 / 84.9; 85 MB 4608 x 3072 -> 9216 107.6 / 139.6 and 107.0 / 137.8; 34 MB 2048 x 2048 -> 8192
+    // 30.9 / 43.8 and 30.5 / 42.0; 113 MB 4608 x 3072 -> 12288 137.9 / 176.4 and 136.3 / 177.5.  The residual form has no gain (4608 x 12288 ->
+    // 3072 127.3 / 139.3 and 127.5 / 138.7) and keeps the one way.
+    a.cached = (double)a.M * a.N * (EPI == EPI_ACC || OUT_DT == DT_F32 ? 4 : 2) <= 100e6;
     GemmArgs main = a, rest = a;
     const int64_t n_main = sp.main_tm * sp.main_tn, n_rest = sp.small, tn = (a.N + 255) / 256;
     if (n_main > 0x7fffffff || n_rest > 0x7fffffff) return -1;

@@ -122,8 +122,7 @@ __device__ __forceinline__ void store_wave_tile(const W6Args& p, uint8_t* wl, co
                     } else if (OUT_DT == DT_BF16) {
                         *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(out[0], out[1]), pack_bf16x2(out[2], out[3]));
                     } else {
-                        *reinterpret_cast<uint2*>(dst) = make_uint2((uint32_t)f_to_f16(out[0]) | ((uint32_t)f_to_f16(out[1]) << 16),
-                                                                    (uint32_t)f_to_f16(out[2]) | ((uint32_t)f_to_f16(out[3]) << 16));
+                        *reinterpret_cast<uint2*>(dst) = make_uint2(pack_f16x2(out[0], out[1]), pack_f16x2(out[2], out[3]));
                     }
                 }
             }
