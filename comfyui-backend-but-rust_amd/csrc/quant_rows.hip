@@ -136,9 +136,9 @@ __device__ __forceinline__ float rotate_and_max(const QuantArgs& p, float (&v)[C
     return amax;
 }
 
-// Scale and codes of a row whose maximum is `amax`.
+// Scale and codes of a row whose maximum is `amax`; a lane's values start at column first + c * step of it.
 template <int MODE, int C, bool SR>
-__device__ __forceinline__ void store_codes(const QuantArgs& p, float (&v)[C][16], int64_t m, bool row_ok, int wr, int lane, float amax) {
+__device__ __forceinline__ void store_codes(const QuantArgs& p, float (&v)[C][16], int64_t m, bool row_ok, int first, int step, float amax) {
     float scale, st, rinv = 0.f;
     bool by_rcp = true;   // f16 rows: st is a finite half
     if (MODE == MODE_SD_F16) {
@@ -155,7 +155,7 @@ __device__ __forceinline__ void store_codes(const QuantArgs& p, float (&v)[C][16
         scale = fmaxf(fminf(amax, 3.402823466e+38f) * (1.f / 127.f), 1.0e-30f);
         st = scale;
     }
-    if (row_ok && wr == 0 && lane == 0) p.scales[m] = scale;
+    if (row_ok && first == 0) p.scales[m] = scale;
 
     // Stochastic rounding: the hash of element index + seed, its halves folded, starts with a product.  Where a row's keys stay
     // below 2^32 the fold changes nothing and a lane's 16 products differ by constants.  With that, the fp32 addition above
@@ -165,7 +165,7 @@ __device__ __forceinline__ void store_codes(const QuantArgs& p, float (&v)[C][16
     const auto store = [&](auto fast_tag) {
 #pragma unroll
         for (int c = 0; c < C; ++c) {
-            const int e0 = (wr + c * p.wpr) * kChunk + lane * 16;
+            const int e0 = first + c * step;
             if (!(row_ok && e0 < p.K)) continue;
             uint32_t w[4];
             const uint32_t state0 = ((uint32_t)key0 + (uint32_t)e0) * kPcgMul + kPcgAdd;
@@ -465,7 +465,7 @@ __global__ void __launch_bounds__(512, C > 3 ? 2 : 4) quant_rows_kernel(QuantArg
             amax = 0.f;
             for (int i = 0; i < p.wpr; ++i) amax = fmaxf(amax, red[rloc * p.wpr + i]);
         }
-        store_codes<MODE, C, SR>(p, v, m, row_ok, wr, lane, amax);
+        store_codes<MODE, C, SR>(p, v, m, row_ok, wr * kChunk + lane * 16, p.wpr * kChunk, amax);
     }
 }
 
@@ -555,7 +555,7 @@ __global__ void __launch_bounds__(kGegluWaves * 64) geglu_rows_kernel(QuantArgs 
             amax = 0.f;
             for (int i = 0; i < p.wpr; ++i) amax = fmaxf(amax, r[row0 + i]);
         }
-        store_codes<MODE_SD_F16, C, false>(p, v, m, row_ok, wr, lane, amax);
+        store_codes<MODE_SD_F16, C, false>(p, v, m, row_ok, wr * kChunk + lane * 16, p.wpr * kChunk, amax);
     }
 }
 
@@ -586,6 +586,100 @@ GegluForm geglu_form(int M, int K, int cus) {
     return {1, nchunks};
 }
 
+// LayerNorm of f16 rows ahead of the quantizer (csrc/sd.cu:633-640) for widths that leave a wave per row many idle lanes: a workgroup takes as
+// many rows as fill its waves and cuts them into chunks as if they were one.  A rotation group of 64 is four lanes of one row;
+// their sums and maxima meet in LDS, and every lane adds those of its row.  Bound by vector instructions (about 700 per wave: the fp64
+// sums, the rotation, the divisions), of which idle lanes take as many as busy ones.
+// us, a wave per row and this: 8192 x 640 11.7 and 9.5, 8192 x 320 10.9 and 6.3, 16384 x 768 20.1 and 17.0, 2048 x 512 4.8 and 4.35, 256 x 320
+// 4.0 and 3.7.  Beyond 768 columns the longer sums and barriers cost what the lanes give (8192 x 832 12.3 and 12.7, 8192 x 1280 18.5 and
+// 20.3), as more than four waves do (8192 x 448 in seven 7.6, in four 7.4; 1024 x 448 4.9 and 4.2); below 1024 rows only
+// whole rows of one wave pay (256 x 448, nine rows on four waves, 4.1; a wave per row 4.0).
+constexpr int kLnWaves = 4;
+struct LnForm { int rows, waves; };   // of a workgroup; no rows: a wave per chunk of a row
+LnForm ln_form(int M, int K) {
+    LnForm best{0, 0};
+    if (K % 64 != 0 || K > 768) return best;
+    double busy = 1.2 * K / kChunk;   // share of the lanes with values
+    for (int waves = 1; waves <= (M < 1024 ? 1 : kLnWaves); ++waves) {
+        const int rows = waves * kChunk / K < 16 ? waves * kChunk / K : 16;
+        const double b = (double)rows * K / (waves * kChunk);
+        if (b > (best.rows ? 1.06 : 1.) * busy) {
+            best = {rows, waves};
+            busy = b;
+        }
+    }
+    return best;
+}
+template <int G, int NQ>   // NQ: a quarter of a row's groups at least
+__global__ void __launch_bounds__(kLnWaves * 64) ln_rows_f16_kernel(QuantArgs p, int gpr, uint32_t inv_gpr) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    __shared__ double sums[2][kLnWaves * 16];
+    __shared__ float maxima[kLnWaves * 16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int group = wave * 16 + (lane >> 2);   // of 64 columns; row = group / gpr
+    const int rloc = (int)(group * inv_gpr >> 16), e0 = (int)threadIdx.x * 16 - rloc * p.K;
+    const int64_t m = (int64_t)blockIdx.x * p.rpb + rloc;
+    const bool act = rloc < p.rpb && m < p.M;
+    int at[NQ];   // a group past the row's (or of no row) is read from its first, and not counted
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) at[i] = act ? rloc * gpr + (i * 4 + (lane & 3) < gpr ? i * 4 + (lane & 3) : 0) : 0;
+    const auto row_sum = [&](double part, double* meet) {
+        const auto mv = [](double x, auto ctrl) {
+            const int64_t b = __builtin_bit_cast(int64_t, x);
+            constexpr int C = decltype(ctrl)::value;
+            return __builtin_bit_cast(double, ((int64_t)dpp_int<C>((int)(b >> 32)) << 32) | (uint32_t)dpp_int<C>((int)b));
+        };
+        const auto quad = [&](double x) {
+            x += mv(x, std::integral_constant<int, 0xB1>{});
+            return x + mv(x, std::integral_constant<int, 0x4E>{});
+        };
+        part = quad(part);
+        if ((lane & 3) == 0) meet[group] = part;
+        __syncthreads();
+        double t = 0.0;   // every fourth of the row's, the other three from the neighbours
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) {
+            const double x = meet[at[i]];
+            t += i * 4 + (lane & 3) < gpr ? x : 0.0;
+        }
+        return (float)quad(t);
+    };
+    float v[1][16], a[16], b[16];
+    if (act) {
+        load16<MODE_SD_F16>(p.x, m * p.x_stride + e0, v[0]);
+        load16<MODE_F32>(p.norm_w, e0, a);
+        load16<MODE_F32>(p.norm_b, e0, b);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[0][i] = a[i] = b[i] = 0.f;
+    }
+    double part = 0.0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) part += (double)v[0][i];
+    const float mean = row_sum(part, sums[0]) / (float)p.K;
+    part = 0.0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        v[0][i] -= mean;
+        part += (double)v[0][i] * (double)v[0][i];
+    }
+    const float rstd = rsqrt_cr(row_sum(part, sums[1]) / (float)p.K + p.eps);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[0][i] = act ? rnd_dt<DT_F16>(__builtin_fmaf(v[0][i] * rstd, a[i], b[i])) : 0.f;
+    float amax = rotate_and_max<MODE_SD_F16, G, 1>(p, v, m, act, 0, lane, lds + wave * kLdsPerWave, true);
+    const auto quad_max = [](float x) {
+        x = fmaxf(x, __builtin_bit_cast(float, dpp_int<0xB1>(__builtin_bit_cast(int, x))));
+        return fmaxf(x, __builtin_bit_cast(float, dpp_int<0x4E>(__builtin_bit_cast(int, x))));
+    };
+    amax = quad_max(amax);
+    if ((lane & 3) == 0) maxima[group] = amax;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) amax = fmaxf(amax, maxima[at[i]]);
+    amax = quad_max(amax);
+    store_codes<MODE_SD_F16, 1, false>(p, v, m, act, e0, 0, amax);
+}
+
 template <auto KERN>
 int launch_kernel(const QuantArgs& a, int nw, int lds_per_wave, hipStream_t st) {
     hipLaunchKernelGGL(KERN, dim3((a.M + a.rpb - 1) / a.rpb), dim3(nw * 64), nw * lds_per_wave, st, a);   // 8 waves: 35 KB
@@ -600,6 +694,17 @@ int launch(const QuantArgs& a, int nw, hipStream_t st) {
     if (a.pro == PRO_PLAIN) {
         if (CAN_SR && a.seed != 0) return launch_kernel<quant_rows_kernel<MODE, G, C, CLS_PLAIN, CAN_SR>>(a, nw, lds, st);
         return launch_kernel<quant_rows_kernel<MODE, G, C, CLS_PLAIN>>(a, nw, lds, st);
+    }
+    if constexpr (MODE == MODE_SD_F16) {
+        if (const LnForm f = ln_form(a.M, a.K); a.pro == PRO_LN_AFFINE && f.rows) {
+            QuantArgs r = a;
+            r.rpb = f.rows;
+            const int gpr = a.K / 64;
+            const auto kern = gpr <= 8 ? ln_rows_f16_kernel<G, 2> : ln_rows_f16_kernel<G, 3>;
+            hipLaunchKernelGGL(kern, dim3((a.M + f.rows - 1) / f.rows), dim3(f.waves * 64), f.waves * lds, st, r, gpr, (65536u + gpr - 1) / gpr);
+            KCHECK();
+            return 0;
+        }
     }
     if (a.pro == PRO_RMS || a.pro == PRO_LAYERNORM || a.pro == PRO_ADALN || a.pro == PRO_LN_MOD || a.pro == PRO_LN_AFFINE)
         return launch_kernel<quant_rows_kernel<MODE, G, C, CLS_NORM>>(a, nw, lds, st);
@@ -710,7 +815,7 @@ __global__ void __launch_bounds__(256) linear_rows_kernel(QuantArgs p, LinArgs a
             for (int i = 0; i < 16; ++i) v[0][i] = 0.f;
         }
         const float amax = wave_max_f32(rotate_and_max<MODE, G, 1>(r, v, m, true, 0, lane, tiles + (G ? wave * kLdsPerWave : 0), true));
-        store_codes<MODE, 1, false>(r, v, m, true, 0, lane, amax);
+        store_codes<MODE, 1, false>(r, v, m, true, lane * 16, 0, amax);
     }
     __syncthreads();
     v4i acc{0, 0, 0, 0};

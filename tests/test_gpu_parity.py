@@ -1666,6 +1666,26 @@ def test_w6a8_group_gemm_argument_checks():
     assert ffi.raw("gpu_w6a8_group_gemm", 0, 0, 0, 0, 0, 0, 0, 0, 8, 128, 2, 0) == 0      # empty
 
 
+@pytest.mark.parametrize("K", [64, 192, 320, 448, 512, 576, 640, 704, 768, 832])
+@pytest.mark.parametrize("M", [1, 7, 1030])
+def test_layer_norm_quantizer_with_rows_that_share_waves(M, K):
+    """Narrow f16 rows: several to a wave or to four waves, the last workgroup short, rows of zeros and of infinities among them."""
+    x = synth.f16_bits(synth.normal(911, K, M * (K + 64)).reshape(M, K + 64) * np.float32(1.5))
+    x[M // 2, :] = 0
+    if M > 5:
+        x[3, :] = 0x7c00
+    w, b = (1 + 0.2 * synth.normal(912, 1, K)).astype(np.float32), (0.1 * synth.normal(912, 2, K)).astype(np.float32)
+    rc, row = oracle.sd_source_rows(oracle.SD_LN, x, M, K, x_stride=K + 64, w=w, b=b, eps=1e-5)
+    assert rc == 0
+    keep = np.arange(M) != 3 if M > 5 else np.ones(M, bool)   # what becomes of infinities is their row's own affair
+    for rotate in (0, 64) + ((256,) if K % 256 == 0 else ()):
+        rc, q, s = oracle.sd_quant_rows(row, K, rotate)
+        got, sc = ql.sd_ln_quant_rows(dev_bits(x, F16), dev(w), dev(b), 1e-5, rotate, K=K)
+        torch.cuda.synchronize()
+        assert np.array_equal(sc.cpu().numpy().view(np.uint32)[keep], s.view(np.uint32)[keep])
+        assert np.array_equal(got.cpu().numpy()[keep], q[keep])
+
+
 # ------------------------------------------------------------------------------------------------ full-size shapes
 FULL = [  # (name, M, K, N, rotate, kind)
     ("dit mlp up", 4608, 3072, 12288, 128, "t3"),
