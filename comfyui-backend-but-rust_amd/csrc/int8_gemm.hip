@@ -1248,12 +1248,15 @@ int launch_pp(GemmArgs a, hipStream_t st) {
     if (!aligned) return launch_cfg<CfgM, OUT_DT, EPI>(a, st);   // this kernel has only the coalesced epilogue
     const int64_t G = device_cu_count();
     const PpSplit sp = pp_split(a.M, a.N, G);
-    // Outputs that the last-level cache (256 MB) holds beside the operands stay there for whoever reads them next; larger ones pass by it.
-    // GEMM, and with the quantizer that reads its output, us, non-temporal and cached: 84 MB 8192 x 640 -> 5120 38.2 / 71.7 and 36.4 / 68.5,
-    // 4096 x 1280 -> 10240 55.5 / 88.7 and 53.6 / 84.9; 85 MB 4608 x 3072 -> 9216 107.6 / 139.6 and 107.0 / 137.8; 34 MB 2048 x 2048 -> 8192
-    // 30.9 / 43.8 and 30.5 / 42.0; 113 MB 4608 x 3072 -> 12288 137.9 / 176.4 and 136.3 / 177.5.  The residual form has no gain (4608 x 12288 ->
-    // 3072 127.3 / 139.3 and 127.5 / 138.7) and keeps the one way.
-    a.cached = (double)a.M * a.N * (EPI == EPI_ACC || OUT_DT == DT_F32 ? 4 : 2) <= 100e6;
+    // Outputs of 40 to 100 MB are stored with the caches' default policy: the last-level cache (256 MB) holds them beside the operands for
+    // whoever reads them next.  Smaller ones would lie in the L2 (32 MB) until the kernel's end writes them back, larger ones gain nothing.
+    // us, non-temporal and cached (behind the stroke with the quantizer that reads the output): 84 MB 8192 x 640 -> 5120 38.2 / 71.7 and
+    // 36.4 / 68.5, 4096 x 1280 -> 10240 55.5 / 88.7 and 53.6 / 84.9; 67 MB of floats 2048 x 512 -> 8192 20.4 and 18.9; 50 MB 1024 x 1024 -> 12288
+    // 21.1 and 20.7; 42 MB 2048 x 1280 -> 10240 30.5 / 50.5 and 30.5 / 50.1; 25 MB 1024 x 1024 -> 12288 17.0 and 17.6; 14 MB 520 x 256 -> 13088
+    // 8.6 and 9.7; 113 MB 4608 x 3072 -> 12288 137.9 / 176.4 and 136.3 / 177.5.  The residual form has no gain (4608 x 12288 -> 3072
+    // 127.3 / 139.3 and 127.5 / 138.7) and keeps the one way.
+    const double out_bytes = (double)a.M * a.N * (EPI == EPI_ACC || OUT_DT == DT_F32 ? 4 : 2);
+    a.cached = out_bytes >= 40e6 && out_bytes <= 100e6;
     GemmArgs main = a, rest = a;
     const int64_t n_main = sp.main_tm * sp.main_tn, n_rest = sp.small, tn = (a.N + 255) / 256;
     if (n_main > 0x7fffffff || n_rest > 0x7fffffff) return -1;
