@@ -1214,7 +1214,10 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
     const uint32_t v_lane = l32 * 32 + hh * 16;   // V: a KB of 32 channels, both halves' 16 bytes side by side; in LDS a half at a time
     const int8_t *kt = a.ki + kvh * a.nblk * (32 * D), *vt = a.vt + kvh * a.nblk * (32 * D);
     const int* vst = a.vsum + kvh * a.kb * D;
-    const float* kst = a.ks + kvh * a.kb * 4 + hh * 2;
+    // scalar bases and 32-bit lane offsets
+    const uint8_t *kst = (const uint8_t*)(a.ks + kvh * a.kb * 4), *vs8 = (const uint8_t*)vst;
+    const uint32_t k_lane = hh * 8;
+    const auto key_scales = [&](int t) { return *reinterpret_cast<const float2*>(kst + (int64_t)t * 16 + k_lane); };
 
     // The DMA of a wave's share of K tile tk (j < NF) and V tile tv.  A K tile past the end fetches the last one, into the stage that
     // a tile tk would have: nothing reads that stage any more, while the last tile's own stage is being read.
@@ -1228,7 +1231,8 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
     // ones, at 64 all): no branch in the tile loop.
     const int vcol = (D == 128 ? (wave & 1) * 64 : 0) + lane;
     auto put_sums = [&](int tv, int sum) { reinterpret_cast<int*>(smem + (tv & 1) * STAGE + 2 * KV)[vcol] = sum + kSumOne; };
-    const int sum0 = vst[t0 * D + vcol];
+    const auto get_sums = [&](int tv) { return *reinterpret_cast<const int*>(vs8 + (int64_t)tv * (D * 4) + (uint32_t)(vcol * 4)); };
+    const int sum0 = get_sums(t0);
 #pragma unroll
     for (int j = 0; j < 2 * NF; ++j) dma(j, t0, t0);
 #pragma unroll
@@ -1241,7 +1245,7 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
         for (int s = 0; s < NS; ++s) qf[s] = *reinterpret_cast<const v4i*>(qrow + s * 32);
     }
     const float q_scale = a.qs[(bh * a.qg + r / 32) * 8 + (r & 7)];
-    float k0 = kst[t0 * 4], k1 = kst[t0 * 4 + 1];
+    float k0 = key_scales(t0).x, k1 = key_scales(t0).y;
 
     float ro[NS][16];
 #pragma unroll
@@ -1253,7 +1257,8 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
     put_sums(t0, sum0);
     __syncthreads();
 
-    v16i S[NB];
+    v16i S[NB], one = sum_one();
+    if constexpr (D == 64) asm("" : "+v"(one));   // kept in registers: made anew, it is eight instructions of a tile's 280
     auto load_kf = [&](v4i (&kf)[NS], int t, int blk) {
         const uint8_t* st = smem + (t & 1) * STAGE + blk * (32 * D) + lane * 16;
 #pragma unroll
@@ -1263,7 +1268,7 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
     for (int blk = 0; blk < NB; ++blk) {
         v4i kf[NS];
         load_kf(kf, t0, blk);
-        S[blk] = sum_one();
+        S[blk] = one;
 #pragma unroll
         for (int s = 0; s < NS; ++s) S[blk] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[s], qf[s], S[blk], 0, 0, 0);
     }
@@ -1276,9 +1281,10 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
         float n0 = 0.f, n1 = 0.f;
         int next_sum = 0;
         if constexpr (!last) {
-            n0 = kst[(t + 1) * 4];
-            n1 = kst[(t + 1) * 4 + 1];
-            next_sum = vst[(t + 1) * D + vcol];
+            const float2 n = key_scales(t + 1);
+            n0 = n.x;
+            n1 = n.y;
+            next_sum = get_sums(t + 1);
         }
         const float gs0 = a.sm * (q_scale * k0), gs1 = a.sm * (q_scale * k1);
         int i0 = last ? kSumOne - 50000 : INT_MIN, i1 = i0;
@@ -1294,7 +1300,7 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
                 if ((i % 4) < 2) i0 = max(i0, sv);
                 else i1 = max(i1, sv);
             }
-        const float tile_m = swap32_max(fmax_nn(fmaf((float)(i0 - kSumOne), gs0, -kU8Offset), fmaf((float)(i1 - kSumOne), gs1, -kU8Offset)));
+        const float tile_m = swap32_max(fmax_nn(fmaf(sum_value(i0), gs0, -kU8Offset), fmaf(sum_value(i1), gs1, -kU8Offset)));
         // The running base m only moves when a tile's maximum has outgrown it by 2^60 (and at the first tile): numerator and
         // denominator are both relative to it, so any base gives the same quotient, and the outputs need no rescaling here.
         if (__builtin_amdgcn_ballot_w64(tile_m - m > 60.f)) {
@@ -1354,7 +1360,7 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
                     if (rg * 4 + g4 >= 1 && rg * 4 + g4 <= 2 * NF) dma(rg * 4 + g4 - 1, t + 2, t + 1);
                     if (rg > 0 && g4 % (4 / NS) == 0) {
                         const int s = g4 / (4 / NS);
-                        if (s == 0) S[rg - 1] = sum_one();
+                        if (s == 0) S[rg - 1] = one;
                         S[rg - 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[s], qf[s], S[rg - 1], 0, 0, 0);
                     }
                 }
@@ -1381,7 +1387,7 @@ __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
         // that are read under them, and the last key block's scores go between the first block's products
         v4i kf[NS];
         if constexpr (!last) load_kf(kf, t + 1, NB - 1);
-        if constexpr (!last) S[NB - 1] = sum_one();
+        if constexpr (!last) S[NB - 1] = one;
 #pragma unroll
         for (int x = 0; x <= NS; ++x) {
 #pragma unroll
