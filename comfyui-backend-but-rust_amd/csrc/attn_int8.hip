@@ -354,13 +354,18 @@ __device__ __forceinline__ void load_rows(const void* p, int64_t base, int64_t r
 // The K anchor of one (kv head, batch).  The nine sampled keys go to LDS (a thread per channel); the sums then follow the
 // reference's block of 128 threads in four warps: thread t walks channels t and t + 128 with one set of accumulators
 // (head dim 256), threads past the head dim hold zeros (64), warps add by a shuffle-down tree and the four warps in
-// order (csrc/vendor/sage/quant_qk_int8.cu:640-756).
+// order (csrc/vendor/sage/quant_qk_int8.cu:640-756).  A chain of LDS trips by few threads, which short calls wait for: rows and parts of
+// sums lie so that their readers meet in different banks, maxima go over lanes instead of 128 reads of one thread, and every thread picks the
+// candidate itself.  us a call, with rows 128 floats apart, one thread's maxima and the candidate through LDS, and this: with norm and rope
+// 300 x 24 x 128 27.2 and 26.1, 1024 x 24 x 128 44.9 and 43.9; 256 x 10 x 64 16.6 and 16.3, 2 x 1600 x 7 x 64 33.6 and 33.3; 4608 x 24 x 128 and
+// 2 x 4096 x 10 x 64 the same.  (cos and sin asked for beside the keys: 26.8 and 45.3, registers of the whole launch.)
 template <int DT, int D>
 __device__ __forceinline__ void anchor_body(const AttnArgs& a, const int hi, const int bi) {
-    __shared__ float s[9][D];
-    __shared__ float energy[128], best_energy[128], amax[128], bmax[128], dist[9][128];
-    __shared__ int chosen;
-    const int tid = threadIdx.x, c = tid & (D - 1);
+    __shared__ __align__(16) float s[9][D + 4];
+    constexpr int PART = 36;   // floats from one 32-thread part of a sum to the next: the parts' readers meet in other banks
+    __shared__ __align__(16) float dist[10][4 * PART], best_energy[4 * PART];   // nine candidates, then the energy
+    __shared__ float amax[2], bmax[2];
+    const int tid = threadIdx.x, c = tid & (D - 1), slot = (tid >> 5) * PART + (tid & 31);
     const int64_t base = bi * a.k_bs + hi * a.k_hs;
     bool normed = false;
     if constexpr (D == 128) {
@@ -426,10 +431,11 @@ __device__ __forceinline__ void anchor_body(const AttnArgs& a, const int hi, con
                 d9[i] = fmaf(d, d, d9[i]);
             }
         }
-        energy[tid] = e;
-        amax[tid] = m;
+        dist[9][slot] = e;
+        m = wave_max_f32(m);
+        if ((tid & 63) == 0) amax[tid >> 6] = m;
 #pragma unroll
-        for (int i = 0; i < 9; ++i) dist[i][tid] = d9[i];
+        for (int i = 0; i < 9; ++i) dist[i][slot] = d9[i];
     }
     __syncthreads();
     auto tree = [](const float* x) {
@@ -440,21 +446,17 @@ __device__ __forceinline__ void anchor_body(const AttnArgs& a, const int hi, con
         return t[0];
     };
     __shared__ float warp_sum[11][4];   // nine candidate distances, then the two energies
-    if (tid < 36) warp_sum[tid / 4][tid % 4] = tree(&dist[tid / 4][(tid % 4) * 32]);
-    else if (tid < 40) warp_sum[9][tid - 36] = tree(&energy[(tid - 36) * 32]);
+    if (tid < 40) warp_sum[tid / 4][tid % 4] = tree(&dist[tid / 4][(tid % 4) * PART]);
     __syncthreads();
-    if (tid == 0) {
-        int best = 0;
-        float best_d = 3.402823466e+38F;
-        for (int i = 0; i < 9; ++i) {
-            float d = 0.f;
-            for (int w = 0; w < 4; ++w) d += warp_sum[i][w];
-            if (d < best_d) { best = i; best_d = d; }
-        }
-        chosen = best;
+    int best = 0;   // every thread for itself: broadcasts cost less than a barrier
+    float best_d = 3.402823466e+38F;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+        float d = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) d += warp_sum[i][w];
+        if (d < best_d) { best = i; best_d = d; }
     }
-    __syncthreads();
-    const int best = chosen;
     if (tid < 128) {
         float be = 0.f, bm = 0.f;
         for (int ch = tid; ch < D; ch += 128) {
@@ -465,22 +467,20 @@ __device__ __forceinline__ void anchor_body(const AttnArgs& a, const int hi, con
                 bm = fmax_nn(bm, fabsf(r));
             }
         }
-        best_energy[tid] = be;
-        bmax[tid] = bm;
+        best_energy[slot] = be;
+        bm = wave_max_f32(bm);
+        if ((tid & 63) == 0) bmax[tid >> 6] = bm;
     }
     __syncthreads();
-    if (tid < 4) warp_sum[10][tid] = tree(&best_energy[tid * 32]);
+    if (tid < 4) warp_sum[10][tid] = tree(&best_energy[tid * PART]);
     __syncthreads();
     if (tid == 0) {
-        float e0 = 0.f, e1 = 0.f, m0 = 0.f, m1 = 0.f;
+        float e0 = 0.f, e1 = 0.f;
         for (int w = 0; w < 4; ++w) {
             e0 += warp_sum[9][w];
             e1 += warp_sum[10][w];
         }
-        for (int i = 0; i < 128; ++i) {
-            m0 = fmax_nn(m0, amax[i]);
-            m1 = fmax_nn(m1, bmax[i]);
-        }
+        const float m0 = fmax_nn(amax[0], amax[1]), m1 = fmax_nn(bmax[0], bmax[1]);
         a.anchors[bi * a.hk + hi] = (a.use_anchor && e1 < e0 && m1 <= m0 * 1.125f) ? (int)((int64_t)best * (a.lk - 1) / 8) : -1;
     }
 }
