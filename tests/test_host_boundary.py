@@ -200,6 +200,13 @@ def test_makefile_and_build_script_list_the_same_units_and_flags():
         assert line and line.group(1).split() == extra
 
 
+def test_make_builds_the_libraries_without_python():
+    """The default target is for hosts that link the kernels natively: nothing in it runs Python or needs torch."""
+    out = subprocess.check_output(["make", "-n", "-B", "-C", os.path.join(ROOT, "comfyui-backend-but-rust_amd")], text=True)
+    assert "libgpu_kernels.a" in out and "libgpu_kernels.so" in out and "libgpu_blas.so" in out
+    assert "python" not in out and "py_linear" not in out
+
+
 def test_rust_host_crate_follows_the_headers_and_the_build_script():
     """rust/src/sys.rs is generated from the headers (same names, arity and scalar types as the ctypes table), and
     rust/build.rs compiles the units and flags that build.py does.  No Rust toolchain is needed for either check."""
