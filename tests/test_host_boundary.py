@@ -207,6 +207,22 @@ def test_make_builds_the_libraries_without_python():
     assert "python" not in out and "py_linear" not in out
 
 
+@pytest.mark.parametrize("torch", ["absent", "not for ROCm"])
+def test_build_script_without_torch(torch, monkeypatch, capsys):
+    """ctypes callers need no torch: without it the build script makes the libraries, and leaves out what only torch's users import."""
+    import sys
+    import types
+    build = pkg("build")
+    made = []
+    other = types.SimpleNamespace(version=types.SimpleNamespace(hip=None), __file__="torch/__init__.py", _C=types.SimpleNamespace(_GLIBCXX_USE_CXX11_ABI=True))
+    monkeypatch.setitem(sys.modules, "torch", None if torch == "absent" else other)   # None: import torch raises ImportError
+    monkeypatch.setattr(build, "_compile", lambda src: made.append(src) or src[:-4] + ".o")
+    monkeypatch.setattr(build.subprocess, "check_call", lambda cmd: made.append(cmd[cmd.index("-o") + 1]))
+    assert build.build() == build.OUT
+    assert made[-2:] == [build.OUT, build.BLAS_OUT] and sorted(made[:-2]) == sorted(build.SOURCES)
+    assert "torch" in capsys.readouterr().err
+
+
 def test_rust_host_crate_follows_the_headers_and_the_build_script():
     """rust/src/sys.rs is generated from the headers (same names, arity and scalar types as the ctypes table), and
     rust/build.rs compiles the units and flags that build.py does.  No Rust toolchain is needed for either check."""
