@@ -2,10 +2,30 @@
 src/unet.rs:436-456, src/h3.rs:1208-1251): quantize rows, then the fused int8 GEMM.  torch supplies device memory and
 the stream; all arithmetic happens in libgpu_kernels.so.
 """
+import importlib.machinery
+import importlib.util
+import os
+
 import torch
 
-from . import ffi
-from . import _pycalls   # csrc/py_linear.cpp, built beside libgpu_kernels.so
+from . import build, ffi
+
+
+def _native_calls():
+    """csrc/py_linear.cpp as build.py made it, or None where it was not made: what it does can be done in Python too, with more host time."""
+    path = build.CALLS_OUT
+    if not os.path.exists(path):
+        return None
+    loader = importlib.machinery.ExtensionFileLoader(__package__ + "._pycalls", path)
+    try:
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader(loader.name, loader))
+        loader.exec_module(module)
+    except ImportError as e:
+        raise ImportError("%s cannot be loaded (%s); run `python __graft_entry__.py` or the package's build.py" % (path, e)) from e
+    return module
+
+
+_pycalls = _native_calls()
 
 _TORCH_DT = {torch.float32: ffi.DT_F32, torch.float16: ffi.DT_F16, torch.bfloat16: ffi.DT_BF16}
 _DT_TORCH = {v: k for k, v in _TORCH_DT.items()}
@@ -277,7 +297,7 @@ def w6a8_group_gemm(A, packed, xs, sw, bias=None, out_dtype=torch.bfloat16, want
 
 def linear_w8a8(x, W, ws, bias=None, rotate=0, out_dtype=None):
     """One W8A8 linear: y = dequant(quant(x) . W^T)."""
-    y = _pycalls.linear_w8a8(x, W, ws, bias, rotate, out_dtype)
+    y = None if _pycalls is None else _pycalls.linear_w8a8(x, W, ws, bias, rotate, out_dtype)
     return _linear_w8a8(x, W, ws, bias, rotate, out_dtype) if y is None else y
 
 

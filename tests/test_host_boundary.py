@@ -223,6 +223,39 @@ def test_build_script_without_torch(torch, monkeypatch, capsys):
     assert "torch" in capsys.readouterr().err
 
 
+def _package_with(tmp_path, native):
+    """The package beside its kernel library in a folder of its own, its native calls as `native` makes them; what a process that imports
+    qlinear from there prints or fails with."""
+    import sys
+    src = os.path.join(ROOT, "comfyui-backend-but-rust_amd")
+    dst = tmp_path / "comfyui-backend-but-rust_amd"
+    dst.mkdir()
+    for f in os.listdir(src):
+        if f.endswith(".py") or f in ("libgpu_kernels.so", "libgpu_blas.so"):
+            os.symlink(os.path.join(src, f), dst / f)
+    native(dst)
+    code = """if True:
+        import importlib
+        ql = importlib.import_module("comfyui-backend-but-rust_amd.qlinear")
+        ql._linear_w8a8 = lambda *args: args
+        print(ql._pycalls, ql.linear_w8a8(1, 2, 3, rotate=64))
+    """
+    return subprocess.run([sys.executable, "-c", code], cwd=tmp_path, capture_output=True, text=True, timeout=300)
+
+
+def test_qlinear_without_the_native_calls(tmp_path):
+    """A tree with the kernel library alone: qlinear is there, and its calls are made in Python."""
+    r = _package_with(tmp_path, lambda d: None)
+    assert r.returncode == 0 and r.stdout.split("\n")[0] == "None (1, 2, 3, None, 64, None)", r.stderr[-500:]
+
+
+def test_qlinear_names_the_build_where_the_native_calls_do_not_load(tmp_path):
+    """A file that is there and cannot be loaded is an error that says what to run, not a reason to run slower."""
+    name = os.path.basename(pkg("build").CALLS_OUT)
+    r = _package_with(tmp_path, lambda d: (d / name).write_bytes(b"no library"))
+    assert r.returncode != 0 and "ImportError" in r.stderr and "build.py" in r.stderr and name in r.stderr, r.stderr[-500:]
+
+
 def test_rust_host_crate_follows_the_headers_and_the_build_script():
     """rust/src/sys.rs is generated from the headers (same names, arity and scalar types as the ctypes table), and
     rust/build.rs compiles the units and flags that build.py does.  No Rust toolchain is needed for either check."""
