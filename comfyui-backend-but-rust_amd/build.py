@@ -3,9 +3,11 @@
 hipcc cross-compiles for gfx950 without a GPU.  Objects are built in parallel, one per .hip file, then linked.
 """
 import concurrent.futures
+import glob
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -50,9 +52,6 @@ def build_blas():
     return BLAS_OUT
 
 
-CALLS_OUT = os.path.join(HERE, "_pycalls.so")
-
-
 def _torch():
     """torch for ROCm, or None: the libraries and ffi.py do without it."""
     try:
@@ -62,31 +61,47 @@ def _torch():
     return torch if torch.version.hip else None
 
 
+def calls_out():
+    """The file of the native calls.  Its name carries the Python and the torch that it is compiled against: others look for another."""
+    import torch
+    return os.path.join(HERE, "_pycalls-torch" + torch.__version__ + sysconfig.get_config_var("EXT_SUFFIX"))
+
+
+def drop_calls():
+    """Native calls of any torch: compiled against a kernel library and header that are about to change."""
+    for f in glob.glob(os.path.join(glob.escape(HERE), "_pycalls*.so")):
+        os.remove(f)
+
+
 def build_calls():
     """The Python calls that are native code (csrc/py_linear.cpp): host code only, against torch's headers and libgpu_kernels.so."""
-    import sysconfig
+    drop_calls()
     torch = _torch()
     if torch is None:
         sys.stderr.write("torch for ROCm cannot be imported: the native calls of the Python side (csrc/py_linear.cpp) are left out\n")
         return None
+    out = calls_out()
+    part = os.path.join(HERE, "_pycalls-unfinished.so")
     t, rocm = os.path.dirname(torch.__file__), os.environ.get("ROCM_PATH", "/opt/rocm")
     subprocess.check_call(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
                            "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI), "-isystem", os.path.join(t, "include"),
                            "-isystem", os.path.join(rocm, "include"), "-isystem", sysconfig.get_paths()["include"],
-                           os.path.join(CSRC, "py_linear.cpp"), "-o", CALLS_OUT, "-L" + os.path.join(t, "lib"), "-L" + HERE, "-lgpu_kernels",
+                           os.path.join(CSRC, "py_linear.cpp"), "-o", part, "-L" + os.path.join(t, "lib"), "-L" + HERE, "-lgpu_kernels",
                            "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", "-Wl,-rpath,$ORIGIN"])
-    return CALLS_OUT
+    os.replace(part, out)
+    return out
+
+
+def _older(out, deps):
+    return not os.path.exists(out) or any(os.path.getmtime(d) > os.path.getmtime(out) for d in deps)
 
 
 def stale():
-    if not os.path.exists(OUT):
-        return True
-    t = os.path.getmtime(OUT)
-    if not os.path.exists(BLAS_OUT) or (not os.path.exists(CALLS_OUT) and _torch() is not None):
-        return True
-    deps = [os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith((".hip", ".hpp", ".cpp"))]
-    deps.append(os.path.join(os.path.dirname(HERE), "include", "gpu_api.h"))
-    return any(os.path.getmtime(d) > t for d in deps)
+    """Whether an output is missing or older than what it is made from: each by its own time, since a later one's compilation may have failed."""
+    include = os.path.join(os.path.dirname(HERE), "include")
+    kernels = [os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith((".hip", ".hpp"))] + [os.path.join(include, "gpu_api.h")]
+    return (_older(OUT, kernels) or _older(BLAS_OUT, [os.path.join(CSRC, "blas_gemm.cpp"), os.path.join(include, "gpu_blas_api.h")]) or
+            (_torch() is not None and _older(calls_out(), [os.path.join(CSRC, "py_linear.cpp"), os.path.join(include, "gpu_api.h"), OUT])))
 
 
 def build(force=True):
@@ -94,6 +109,7 @@ def build(force=True):
         return OUT
     with concurrent.futures.ThreadPoolExecutor(max_workers=len(SOURCES)) as ex:
         objs = list(ex.map(_compile, SOURCES))
+    drop_calls()
     subprocess.check_call(["hipcc", "--offload-arch=" + ARCH, "-shared", "-fPIC", "-o", OUT, *objs])
     build_blas()
     build_calls()

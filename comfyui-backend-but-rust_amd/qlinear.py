@@ -13,7 +13,7 @@ from . import build, ffi
 
 def _native_calls():
     """csrc/py_linear.cpp as build.py made it, or None where it was not made: what it does can be done in Python too, with more host time."""
-    path = build.CALLS_OUT
+    path = build.calls_out()
     if not os.path.exists(path):
         return None
     loader = importlib.machinery.ExtensionFileLoader(__package__ + "._pycalls", path)

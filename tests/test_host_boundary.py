@@ -208,7 +208,7 @@ def test_make_builds_the_libraries_without_python():
 
 
 @pytest.mark.parametrize("torch", ["absent", "not for ROCm"])
-def test_build_script_without_torch(torch, monkeypatch, capsys):
+def test_build_script_without_torch(torch, tmp_path, monkeypatch, capsys):
     """ctypes callers need no torch: without it the build script makes the libraries, and leaves out what only torch's users import."""
     import sys
     import types
@@ -216,11 +216,72 @@ def test_build_script_without_torch(torch, monkeypatch, capsys):
     made = []
     other = types.SimpleNamespace(version=types.SimpleNamespace(hip=None), __file__="torch/__init__.py", _C=types.SimpleNamespace(_GLIBCXX_USE_CXX11_ABI=True))
     monkeypatch.setitem(sys.modules, "torch", None if torch == "absent" else other)   # None: import torch raises ImportError
+    monkeypatch.setattr(build, "HERE", str(tmp_path))
     monkeypatch.setattr(build, "_compile", lambda src: made.append(src) or src[:-4] + ".o")
     monkeypatch.setattr(build.subprocess, "check_call", lambda cmd: made.append(cmd[cmd.index("-o") + 1]))
     assert build.build() == build.OUT
     assert made[-2:] == [build.OUT, build.BLAS_OUT] and sorted(made[:-2]) == sorted(build.SOURCES)
     assert "torch" in capsys.readouterr().err
+
+
+def test_build_script_knows_which_outputs_are_older_than_their_sources(tmp_path, monkeypatch):
+    """Every output against its own sources: a compilation that failed behind the kernel library's leaves an old file that is not
+    taken for a new one, nor is one that was compiled against another torch or Python."""
+    build = pkg("build")
+    csrc, include = tmp_path / "pkg" / "csrc", tmp_path / "include"
+    csrc.mkdir(parents=True)
+    include.mkdir()
+    monkeypatch.setattr(build, "HERE", str(tmp_path / "pkg"))
+    monkeypatch.setattr(build, "CSRC", str(csrc))
+    for name in ("OUT", "BLAS_OUT"):
+        monkeypatch.setattr(build, name, str(tmp_path / "pkg" / os.path.basename(getattr(build, name))))
+    calls = build.calls_out()
+    sources = [csrc / "quant_rows.hip", csrc / "common.hpp", csrc / "blas_gemm.cpp", csrc / "py_linear.cpp", include / "gpu_api.h", include / "gpu_blas_api.h"]
+
+    def touch(path, when):
+        open(path, "a").close()
+        os.utime(path, (when, when))
+
+    def tree(**later):   # sources at 100, the libraries at 200, the native calls, linked against the first of them, at 210
+        for p in sources:
+            touch(p, later.get(p.name.replace(".", "_"), 100))
+        touch(build.OUT, later.get("out", 200))
+        touch(build.BLAS_OUT, later.get("blas", 200))
+        touch(calls, later.get("calls", 210))
+        return build.stale()
+
+    assert not tree()
+    assert tree(py_linear_cpp=220) and tree(blas_gemm_cpp=220) and tree(common_hpp=220) and tree(quant_rows_hip=220) and tree(gpu_api_h=220)
+    # the kernel library was linked anew, and then the other compilation failed
+    assert tree(py_linear_cpp=220, out=230, blas=230) and tree(gpu_api_h=220, out=230, blas=230)
+    assert tree(blas_gemm_cpp=220, out=230, calls=240) and tree(out=230, blas=230)
+    assert not tree(py_linear_cpp=220, out=230, blas=230, calls=240)
+    import torch
+    monkeypatch.setattr(torch, "__version__", "0.0.1")
+    assert build.stale()
+
+
+def test_build_script_leaves_no_old_native_calls_behind_a_failure(tmp_path, monkeypatch):
+    """What was compiled against the former kernel library is gone before the new one is there, and a file appears whole."""
+    build = pkg("build")
+    monkeypatch.setattr(build, "HERE", str(tmp_path))
+    for name in ("OUT", "BLAS_OUT"):
+        monkeypatch.setattr(build, name, str(tmp_path / os.path.basename(getattr(build, name))))
+    calls = build.calls_out()
+    open(calls, "w").close()
+    monkeypatch.setattr(build, "_compile", lambda src: src[:-4] + ".o")
+
+    def run(cmd):
+        out = cmd[cmd.index("-o") + 1]
+        assert out != calls and not os.path.exists(calls)
+        if cmd[0] == "g++":
+            open(out, "w").close()
+            raise subprocess.CalledProcessError(1, cmd)
+
+    monkeypatch.setattr(build.subprocess, "check_call", run)
+    with pytest.raises(subprocess.CalledProcessError):
+        build.build()
+    assert not os.path.exists(calls)
 
 
 def _package_with(tmp_path, native):
@@ -251,7 +312,7 @@ def test_qlinear_without_the_native_calls(tmp_path):
 
 def test_qlinear_names_the_build_where_the_native_calls_do_not_load(tmp_path):
     """A file that is there and cannot be loaded is an error that says what to run, not a reason to run slower."""
-    name = os.path.basename(pkg("build").CALLS_OUT)
+    name = os.path.basename(pkg("build").calls_out())
     r = _package_with(tmp_path, lambda d: (d / name).write_bytes(b"no library"))
     assert r.returncode != 0 and "ImportError" in r.stderr and "build.py" in r.stderr and name in r.stderr, r.stderr[-500:]
 
