@@ -1215,6 +1215,7 @@ __device__ __forceinline__ v16i sum_one() {
 template <int OUT_DT, int CK, int D, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void attn_int8_pipe_kernel(AttnArgs a) {
     constexpr int NB = CK / 32, NS = D / 32, KV = CK * D, STAGE = 2 * KV + D * 4;
+    static_assert(128 * 128 * D < kSumRoom && 255 * 128 * CK < kSumRoom, "scores and products with V stay within sum_value's range");
     extern __shared__ __align__(16) uint8_t smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l32 = lane & 31, hh = lane >> 5;

@@ -199,7 +199,8 @@ __device__ __forceinline__ void tile_of_block(int b, int nblocks, int tiles_m, i
 // have a step of 1 and room for +-2^22, so that its bits are a float all the way, and an exact subtraction takes the start off again.
 // Two waves of a SIMD issue fp32 additions, multiplications and fma on registers side by side, 1.05 ns each (2.2 cycles), also beside
 // another wave's slower instruction; conversions, maxima, packing, left shifts and anything with a scalar operand take 1.85 ns, one at a time.
-constexpr int kSumOne = 0x4B400000;
+// A kernel that starts its sums there holds their largest magnitude below kSumRoom by a static_assert.
+constexpr int kSumOne = 0x4B400000, kSumRoom = 1 << 22;
 __device__ __forceinline__ float sum_value(int bits) { return __builtin_bit_cast(float, bits) - 12582912.f; }
 
 // Four consecutive elements of a dtype-coded array <-> four floats (8- or 16-byte vector access).

@@ -449,6 +449,7 @@ __global__ void __launch_bounds__(NT, 1) w6a8_group_gemm_big_kernel(W6Args p) {
     const int m0 = tm * BM < p.M - BM ? tm * BM : p.M - BM, n0 = tn * BIG_BN < p.N - BIG_BN ? tn * BIG_BN : p.N - BIG_BN, ng = p.ng;
     const uint32_t lds_base = (uint32_t)(uintptr_t)smem;
     constexpr int FM = 8, FN = 4;
+    static_assert(128 * 32 * BK < kSumRoom, "a group's sums of int8 rows and 6-bit codes stay within sum_value's range");
 
     // DMA of the lower waves: rows in blocks of 8, wave w takes blocks w + 4j of W and of A and the scales of columns 64w .. 64w+63
     const uint32_t lrow = (uint32_t)lane >> 3;
