@@ -19,6 +19,7 @@ namespace {
 
 __device__ __forceinline__ void store16_untracked(void* ptr, uint4 v);
 __device__ __forceinline__ void store16_untracked_at(const void* base, uint32_t off, uint4 v);
+__device__ __forceinline__ void store16_through_at(const void* base, uint32_t off, uint4 v);
 __device__ __forceinline__ void store16_cached_at(const void* base, uint32_t off, uint4 v);
 // A 64-bit value that is the same in every lane, moved to scalar registers.
 __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
@@ -29,6 +30,7 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
 
 enum { EPI_PLAIN = 0, EPI_RESID = 1, EPI_ACC = 2 };
 
+enum { STORE_PAST, STORE_THROUGH, STORE_CACHED };   // past the caches, through the L2, by the default policy
 struct GemmArgs {
     const int8_t* A;
     const int8_t* W;
@@ -43,7 +45,7 @@ struct GemmArgs {
     uint32_t magic;   // panel_magic(tiles_m, tiles_n), for tile_of_block
     int kslice;   // K of a split-K slice (a multiple of 128), 0 = no split
     int n_first;  // two-group kernel: the first column of these tiles
-    bool cached;  // two-group kernel: whole wave tiles are stored with the caches' default policy (launch_pp)
+    int policy;   // two-group kernel: how whole wave tiles are stored (store_policy)
 };
 
 template <int BM_, int BN_, int BK_, int WGM_, int WGN_, int OCC_>
@@ -337,7 +339,8 @@ __device__ __forceinline__ void epilogue_shuffle_with(const GemmArgs& p, Acc& ac
                 for (int t = 0; t < PASSES; ++t) store((const void*)(piece + (uint64_t)(t * RPI) * row_bytes), finish(np, v[t], rv[t]));
             };
             if (!UNTRACKED) each([&](const void* at, const uint4& x) { *reinterpret_cast<uint4*>((uint8_t*)at + lane_off) = x; });
-            else if (EPI != EPI_RESID && p.cached) each([&](const void* at, const uint4& x) { store16_cached_at(at, lane_off, x); });
+            else if (EPI != EPI_RESID && p.policy == STORE_THROUGH) each([&](const void* at, const uint4& x) { store16_through_at(at, lane_off, x); });
+            else if (EPI != EPI_RESID && p.policy == STORE_CACHED) each([&](const void* at, const uint4& x) { store16_cached_at(at, lane_off, x); });
             else each([&](const void* at, const uint4& x) { store16_untracked_at(at, lane_off, x); });
             return;
         }
@@ -550,6 +553,11 @@ __device__ __forceinline__ void store16_untracked(void* ptr, uint4 v) {
 __device__ __forceinline__ void store16_untracked_at(const void* base, uint32_t off, uint4 v) {
     const v4i d = v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
     asm volatile("global_store_dwordx4 %0, %1, %2 nt\n\ts_nop 1" ::"v"(off), "v"(d), "s"(base) : "memory");
+}
+// The same, written through to the last-level cache (device scope), which keeps it: the L2 does not.
+__device__ __forceinline__ void store16_through_at(const void* base, uint32_t off, uint4 v) {
+    const v4i d = v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
+    asm volatile("global_store_dwordx4 %0, %1, %2 sc1\n\ts_nop 1" ::"v"(off), "v"(d), "s"(base) : "memory");
 }
 // The same with the caches' default policy.
 __device__ __forceinline__ void store16_cached_at(const void* base, uint32_t off, uint4 v) {
@@ -1232,6 +1240,26 @@ PpSplit pp_split(int64_t M, int64_t N, int64_t cus) {
     return best;
 }
 
+// How the two-group kernel stores outputs of 40 to 100 MB, which the last-level cache (256 MB) can hold beside the operands for whoever reads
+// them next; all others go past the caches.  us with weights from HBM and outputs in turn in 0.6 to 0.9 GB.
+//   * Rows of whole 64 bytes are written through to that cache, the L2 (32 MB) keeps nothing.  Past the caches and this way, alone and with the
+//     quantizer that reads the output behind it: 84 MB 8192 x 640 -> 5120 35.0 and 37.3, 66.9 and 64.6; 4096 x 1280 -> 10240 53.7 and 54.4, 88.1 and
+//     86.2; 67 MB of floats 2048 x 512 -> 8192 19.7 and 19.5, 46.9 and 41.2; 43 MB 4420 x 1024 -> 4864 25.7 and 26.7, 43.0 and 42.2.  51 such shapes:
+//     alone 0.973 where the same output buffer comes again and 1.018 where it does not (1.06 at most), with the reader 0.976 and 0.973 (1.015 at
+//     most, 47 MB 1034 x 5376 -> 22528).  By the caches' default policy the L2 keeps such lines until the kernel's end writes them back: 39.5
+//     and 60.2 alone in the first two, and nothing gained with the reader (67.6 and 90.5; 42 MB 2048 x 1280 -> 10240 50.3 and 54.7).
+//   * Other rows end in the middle of 64 bytes, which memory writes with a read ahead of it unless the L2 has brought the two rows' parts
+//     together: the default policy.  0.85 of the time past the caches (45 shapes, 16-bit; 0.78 in floats), written through 1.15 (bf16 5114 x 256 -> 4976
+//     24.1 past the caches, 34.5 through; 6385 x 256 -> 7000, one output buffer, with the quantizer of its rows 56 past them, 31 this way).
+//   * The range ends where the default policy had been seen to lose.  60 shapes of 20 to 40 MB written through have 1.008 alone and 0.978 with
+//     the reader, 19 of 100 to 150 MB 1.011 and 0.961, but 14 MB 520 x 256 -> 13312 8.3 and 8.8 alone, 134 MB 8192 x 512 -> 8192 45.8 and 59.9: left as it
+//     was.  The residual form has no gain (4608 x 12288 -> 3072 127.3 and 127.5, by the default policy) and keeps the one way.
+int store_policy(int64_t M, int64_t row_bytes, uintptr_t D) {
+    const double bytes = (double)M * (double)row_bytes;
+    if (bytes < 40e6 || bytes > 100e6) return STORE_PAST;
+    return (((uintptr_t)row_bytes | D) & 63) == 0 ? STORE_THROUGH : STORE_CACHED;
+}
+
 template <class Main, int OUT_DT, int EPI>
 int launch_pp_as(const GemmArgs& main, const GemmArgs& rest, int g_main, int g_rest, hipStream_t st) {
     auto kern = int8_gemm_pp_kernel<Main, OUT_DT, EPI>;
@@ -1248,15 +1276,8 @@ int launch_pp(GemmArgs a, hipStream_t st) {
     if (!aligned) return launch_cfg<CfgM, OUT_DT, EPI>(a, st);   // this kernel has only the coalesced epilogue
     const int64_t G = device_cu_count();
     const PpSplit sp = pp_split(a.M, a.N, G);
-    // Outputs of 40 to 100 MB are stored with the caches' default policy: the last-level cache (256 MB) holds them beside the operands for
-    // whoever reads them next.  Smaller ones would lie in the L2 (32 MB) until the kernel's end writes them back, larger ones gain nothing.
-    // us, non-temporal and cached (behind the stroke with the quantizer that reads the output): 84 MB 8192 x 640 -> 5120 38.2 / 71.7 and
-    // 36.4 / 68.5, 4096 x 1280 -> 10240 55.5 / 88.7 and 53.6 / 84.9; 67 MB of floats 2048 x 512 -> 8192 20.4 and 18.9; 50 MB 1024 x 1024 -> 12288
-    // 21.1 and 20.7; 42 MB 2048 x 1280 -> 10240 30.5 / 50.5 and 30.5 / 50.1; 25 MB 1024 x 1024 -> 12288 17.0 and 17.6; 14 MB 520 x 256 -> 13088
-    // 8.6 and 9.7; 113 MB 4608 x 3072 -> 12288 137.9 / 176.4 and 136.3 / 177.5.  The residual form has no gain (4608 x 12288 -> 3072
-    // 127.3 / 139.3 and 127.5 / 138.7) and keeps the one way.
-    const double out_bytes = (double)a.M * a.N * (EPI == EPI_ACC || OUT_DT == DT_F32 ? 4 : 2);
-    a.cached = out_bytes >= 40e6 && out_bytes <= 100e6;
+    constexpr int SZ = EPI == EPI_ACC || OUT_DT == DT_F32 ? 4 : 2;
+    a.policy = store_policy(a.M, (int64_t)a.N * SZ, (uintptr_t)a.D);
     GemmArgs main = a, rest = a;
     const int64_t n_main = sp.main_tm * sp.main_tn, n_rest = sp.small, tn = (a.N + 255) / 256;
     if (n_main > 0x7fffffff || n_rest > 0x7fffffff) return -1;
@@ -1840,7 +1861,8 @@ GPU_API int gpu_int8_gemm_force_config(int cfg) {
 }
 
 // Test hook: what a call outside capture runs, for operands that start `start` bytes behind 16-byte addresses and outputs of whole 16
-// bytes or not.  out[0] = family as above, out[1] = tile width (family 7; of 64 columns) or 16-row tiles (5), out[2] = slices of K.
+// bytes or not.  out[0] = family as above, out[1] = tile width (family 7; of 64 columns), 16-row tiles (5) or store policy of 16-bit outputs
+// from a whole line on (9); out[2] = slices of K.
 GPU_API int gpu_internal_int8_gemm_plan(int64_t M, int64_t N, int64_t K, int start, int aligned, int32_t* out) {
     if (M <= 0 || N <= 0 || K <= 0 || !shape_ok(M, N, K) || !out) return -200;
     out[0] = choose_cfg(M, N, K, start & 15, aligned != 0);
@@ -1854,6 +1876,8 @@ GPU_API int gpu_internal_int8_gemm_plan(int64_t M, int64_t N, int64_t K, int sta
         const RowsPlan p = rows_plan(M, N, K, device_cu_count(), (N & 3) == 0);
         out[1] = p.mt;
         out[2] = p.slices;
+    } else if (out[0] == 9) {
+        out[1] = store_policy(M, N * 2, 0);
     }
     return 0;
 }

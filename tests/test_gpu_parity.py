@@ -1029,6 +1029,29 @@ def test_int8_gemm_tile_grids(M, N, K, cfg):
         ffi.raw("gpu_int8_gemm_force_config", -1)
 
 
+# Outputs of the two-group kernel in the range where the last-level cache keeps them: rows of whole lines, of half ones and of 16 bytes, from
+# a whole line on and 16 bytes behind one, with a last row and a last column of tiles that are not whole
+@pytest.mark.parametrize("dt,M,N,off", [(BF16, 4161, 4992, 0), (BF16, 4161, 4960, 0), (F16, 4161, 4984, 0), (BF16, 4161, 4992, 8), (F32, 2113, 4992, 0), (F32, 2113, 4996, 0)])
+def test_int8_gemm_store_policies(dt, M, N, off):
+    say("gemm store policy", dt, M, N, off)
+    K = 128
+    A, W = rand_i8(23, 1, M, K), rand_i8(23, 2, N, K)
+    xs, ws = synth.uniform(23, 3, M, 0.005, 0.2), synth.uniform(23, 4, N, 1e-3, 1e-2)
+    Ad, Wd, xd, wd = dev(A), dev(W), dev(xs), dev(ws)
+    D = torch.zeros(M * N + 64, dtype=TDT[dt], device=DEV)
+    ffi.raw("gpu_int8_gemm_force_config", 9)
+    try:
+        ffi.k("gpu_int8_gemm", Ad.data_ptr(), Wd.data_ptr(), xd.data_ptr(), wd.data_ptr(), 0, D[off:].data_ptr(), M, N, K, dt,
+              torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+    finally:
+        ffi.raw("gpu_int8_gemm_force_config", -1)
+    got = host_bits(D)
+    want = oracle.epilogue(oracle.int8_gemm_acc(A, W), xs, ws, None, dt, fma=1)
+    assert np.array_equal(got[off:off + M * N].reshape(M, N), want)
+    assert not got[:off].any() and not got[off + M * N:].any()
+
+
 @pytest.mark.parametrize("start", [1, 2, 4, 8, 12])
 @pytest.mark.parametrize("M,N,K", [(64, 136, 384), (3, 512, 1024), (200, 2056, 1536), (520, 25088, 128)])
 def test_int8_gemm_operands_off_16_bytes(M, N, K, start):

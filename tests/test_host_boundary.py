@@ -452,6 +452,15 @@ def test_gemm_choice_where_it_was_measured():
         assert gemm_plan(M, N, K)[0] == 9, (M, N, K)
 
 
+def test_gemm_store_policy_where_it_was_measured():
+    """16-bit outputs of 40 to 100 MB: rows of whole 64 bytes are written through the L2 (by the default policy up to 1.13 times as long), others by
+    the default policy (past the caches up to 1.8 times as long, written through 1.4)."""
+    for M, N, K, policy in [(8192, 5120, 640, 1), (4096, 10240, 1280, 1), (4420, 4864, 1024, 1), (4160, 6144, 256, 1), (6154, 4896, 256, 1),
+                            (5114, 4976, 256, 2), (8192, 5128, 640, 2), (7807, 3088, 256, 2), (6385, 7000, 256, 2),
+                            (3655, 5376, 768, 0), (4608, 12288, 3072, 0), (8192, 8192, 512, 0), (3000, 5000, 768, 0)]:   # too small, too large
+        assert gemm_plan(M, N, K)[:2] == (9, policy), (M, N, K)
+
+
 @pytest.mark.parametrize("b,h,lq,lk,d,shared", [(2, 9, 492, 492, 128, False), (1, 20, 516, 516, 128, False), (1, 19, 602, 602, 64, False), (2, 11, 356, 560, 128, False),
                                                 (1, 21, 686, 686, 64, False), (1, 11, 640, 640, 128, False), (2, 6, 1029, 539, 64, False), (1, 2, 1849, 877, 128, True),
                                                 (2, 15, 300, 1859, 64, True), (1, 10, 1024, 1024, 128, True), (1, 24, 4608, 4608, 128, True), (2, 10, 4096, 4096, 64, True)])
