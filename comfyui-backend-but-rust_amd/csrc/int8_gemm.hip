@@ -1481,11 +1481,15 @@ FedPlan fed_plan(int64_t M, int64_t N, int64_t K, int num_cu, bool may_split) {
     }
     return best;
 }
-// The two-group kernel's time on the same scale, fitted to 260 shapes (8.5 % rms).  With it the choice between the two kernels is 0.2 % slower
-// than the faster of them over 1000 shapes of 512 to 8192 rows, one in a hundred by more than 1 %.
-double pp_us(int64_t M, int64_t N, int64_t K, int cus) {
-    const double n = pp_split(M, N, cus).rounds;
-    return 1.1 + n * (7.2 + 1.25 * (double)(K / 128));
+// Whether the two-group kernel is estimated to be faster than that.  Its time on the same scale is fitted to 260 shapes (8.5 % rms).  `wide`:
+// outputs of 32 bits.  In one round of 128-row tiles a CU's epilogue has nothing beside it, and with 32 bits it writes twice as much there as in
+// the smaller tiles of the other kernel: up to K = 1024 1.05 times as long as that (93 shapes; 5377 x 768 -> 1112 17.8 us and 15.6,
+// 2433 x 768 -> 2648 18.9 and 16.8), from there on 0.97 (45).  Weights from HBM, outputs in turn: the choice is 0.6 % slower than the faster
+// of the two kernels over 790 shapes with 16-bit outputs, 0.45 % over 1490 with 32-bit ones (0.75 % without that line).
+bool pp_wins(int64_t M, int64_t N, int64_t K, int cus, bool wide) {
+    const PpSplit sp = pp_split(M, N, cus);
+    if (wide && sp.rows == PpS::BM && sp.small <= cus && K <= 1024) return false;
+    return 1.1 + sp.rounds * (7.2 + 1.25 * (double)(K / 128)) < fed_plan(M, N, K, cus, true).us;
 }
 
 // Whether a call may split K over workgroups.  Captured graphs and the static entry point do so only for the shapes that always did
@@ -1619,8 +1623,8 @@ bool rows_kernel_wins(int64_t M, int64_t N, int64_t K, bool aligned) {
 // loads and its DMA).  The other DMA kernels take operands from any 4-byte address, the alignment that a DMA of several
 // dwords needs; an operand that starts there but not at 16 bytes (a view into a larger buffer) goes to them from the sizes on from which
 // such calls always did, and to the register-staged tiles below.  Other starts always take the register-staged tiles, whose
-// ordinary loads may be unaligned.  `aligned` as epilogue_alignment has it.
-int choose_cfg(int64_t M, int64_t N, int64_t K, int start, bool aligned) {
+// ordinary loads may be unaligned.  `aligned` as epilogue_alignment has it, `wide` as pp_wins.
+int choose_cfg(int64_t M, int64_t N, int64_t K, int start, bool aligned, bool wide) {
     const int force = g_force_cfg.load(std::memory_order_relaxed);
     const bool tiles_ok = M * K < ((int64_t)1 << 32) && N * K < ((int64_t)1 << 32) && (K % 128) == 0;   // 32-bit lane offsets, whole steps
     const bool dma_ok = tiles_ok && (start & 3) == 0;
@@ -1634,7 +1638,7 @@ int choose_cfg(int64_t M, int64_t N, int64_t K, int start, bool aligned) {
     // staged tiles over fetching waves: K = 128 0.93 to 1.0, K = 256 0.94 to 1.0, K = 384 0.97 to 1.1; K = 256 with 1 << 21 outputs 1.1; one step
     // and more columns than the CUs take at once in tiles of 64, 25 x 24784 4.4 us and 5.1, but 73 x 10368 4.4 and 3.8)
     const bool tiny = K <= 256 && (M * N <= 1 << 19 || (K <= 128 && M * N <= 1 << 20 && N > 64 * cus));
-    const int large = !dma_ok || !aligned ? 1 : M >= 512 && N >= 512 && pp_us(M, N, K, cus) < fed_plan(M, N, K, cus, true).us ? 9 : 7;
+    const int large = !dma_ok || !aligned ? 1 : M >= 512 && N >= 512 && pp_wins(M, N, K, cus, wide) ? 9 : 7;
     if (dma_ok && aligned && start == 0 && !tiny) return large;
     // the register-staged tiles: large ones, or for operands off 16 bytes the DMA kernels, as soon as there is work for them
     if (M <= 256 && N >= 1024 && tiles_ok && K >= 512) return K >= 1536 || (M > 128 && N >= 8192) ? large : 2;
@@ -1650,7 +1654,7 @@ template <int OUT_DT, int EPI>
 int dispatch_cfg(const GemmArgs& a, hipStream_t st) {
     bool vec_ok, aligned;
     epilogue_alignment<OUT_DT, EPI>(a, vec_ok, aligned);
-    switch (choose_cfg(a.M, a.N, a.K, (int)(((uintptr_t)a.A | (uintptr_t)a.W) & 15), aligned)) {
+    switch (choose_cfg(a.M, a.N, a.K, (int)(((uintptr_t)a.A | (uintptr_t)a.W) & 15), aligned, EPI == EPI_ACC || OUT_DT == DT_F32)) {
         case 5: return launch_rows<OUT_DT, EPI>(a, st);
         case 7: return launch_fed<OUT_DT, EPI>(a, st);
         case 9: return launch_pp<OUT_DT, EPI>(a, st);
@@ -1861,11 +1865,12 @@ GPU_API int gpu_int8_gemm_force_config(int cfg) {
 }
 
 // Test hook: what a call outside capture runs, for operands that start `start` bytes behind 16-byte addresses and outputs of whole 16
-// bytes or not.  out[0] = family as above, out[1] = tile width (family 7; of 64 columns), 16-row tiles (5) or store policy of 16-bit outputs
-// from a whole line on (9); out[2] = slices of K.
+// bytes or not.  out[0] = family as above, out[1] = tile width (family 7; of 64 columns), 16-row tiles (5) or store policy of outputs from
+// a whole line on (9); out[2] = slices of K.  Outputs are 16-bit ones, with aligned = 3 32-bit ones.
 GPU_API int gpu_internal_int8_gemm_plan(int64_t M, int64_t N, int64_t K, int start, int aligned, int32_t* out) {
     if (M <= 0 || N <= 0 || K <= 0 || !shape_ok(M, N, K) || !out) return -200;
-    out[0] = choose_cfg(M, N, K, start & 15, aligned != 0);
+    const bool wide = aligned == 3;
+    out[0] = choose_cfg(M, N, K, start & 15, aligned != 0, wide);
     out[1] = 0;
     out[2] = 1;
     if (out[0] == 7 && aligned) {
@@ -1877,7 +1882,7 @@ GPU_API int gpu_internal_int8_gemm_plan(int64_t M, int64_t N, int64_t K, int sta
         out[1] = p.mt;
         out[2] = p.slices;
     } else if (out[0] == 9) {
-        out[1] = store_policy(M, N * 2, 0);
+        out[1] = store_policy(M, N * (wide ? 4 : 2), 0);
     }
     return 0;
 }

@@ -320,8 +320,8 @@ int64_t gpu_w6a8_group_gemm_scratch(const void* Wp, int64_t M, int64_t N, int64_
 int gpu_int8_gemm_force_config(int cfg);
 
 /* Test hook, no reference counterpart: which kernel a gpu_int8_gemm call outside capture takes for A and W that start `start` bytes
- * behind 16-byte addresses, and outputs whose pointers and rows are of whole 16 bytes (aligned != 0) or not.  out[0] = family
- * (numbers as above), out[1] = tile width of family 7, row tiles of family 5 or, of family 9, how 16-bit outputs from a 128-byte address on
+ * behind 16-byte addresses, and outputs whose pointers and rows are of whole 16 bytes (aligned 1: 16-bit outputs, 3: 32-bit ones) or not (0).  out[0] = family
+ * (numbers as above), out[1] = tile width of family 7, row tiles of family 5 or, of family 9, how outputs from a 128-byte address on
  * are stored (0 past the caches, 1 through the L2, 2 by the default policy); out[2] = slices of K.  Without a device it answers for
  * 256 CUs. */
 int gpu_internal_int8_gemm_plan(int64_t M, int64_t N, int64_t K, int start, int aligned, int32_t* out);

@@ -461,6 +461,21 @@ def test_gemm_store_policy_where_it_was_measured():
         assert gemm_plan(M, N, K)[:2] == (9, policy), (M, N, K)
 
 
+def test_gemm_choice_for_32_bit_outputs():
+    """Shapes of which the other kernel took 8 % and more longer: with 32-bit outputs, one round of 128-row tiles and short K, the one with
+    fetching waves is the faster one; with longer K or several rounds it is not."""
+    for M, N, K in [(5377, 1112, 768), (7465, 840, 384), (2433, 2648, 768), (2482, 2360, 256), (3159, 2104, 256), (5599, 1128, 768)]:
+        assert gemm_plan(M, N, K, aligned=3)[0] == 7, (M, N, K)
+    for M, N, K in [(4608, 12288, 3072), (817, 9176, 8704), (1423, 4240, 1792), (8192, 5120, 640)]:
+        assert gemm_plan(M, N, K, aligned=3)[0] == 9, (M, N, K)
+    for M in (512, 1030, 2433, 5377, 8192):   # 32-bit outputs change nothing else
+        for N in (512, 840, 1112, 2648, 5120, 12288):
+            for K in (256, 768, 1024, 1152, 4096):
+                narrow, wide = gemm_plan(M, N, K), gemm_plan(M, N, K, aligned=3)
+                tiles = -(-M // 128) * -(-N // 256)
+                assert narrow[0] == wide[0] or (tiles <= 256 and K <= 1024 and (narrow[0], wide[0]) == (9, 7)), (M, N, K)
+
+
 @pytest.mark.parametrize("b,h,lq,lk,d,shared", [(2, 9, 492, 492, 128, False), (1, 20, 516, 516, 128, False), (1, 19, 602, 602, 64, False), (2, 11, 356, 560, 128, False),
                                                 (1, 21, 686, 686, 64, False), (1, 11, 640, 640, 128, False), (2, 6, 1029, 539, 64, False), (1, 2, 1849, 877, 128, True),
                                                 (2, 15, 300, 1859, 64, True), (1, 10, 1024, 1024, 128, True), (1, 24, 4608, 4608, 128, True), (2, 10, 4096, 4096, 64, True)])
