@@ -30,7 +30,9 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
 
 enum { EPI_PLAIN = 0, EPI_RESID = 1, EPI_ACC = 2 };
 
-enum { STORE_PAST, STORE_THROUGH, STORE_CACHED };   // past the caches, through the L2, by the default policy
+// How whole wave tiles are stored: as the compiler does it; or by stores that it does not count, past the caches, through the L2, by the
+// caches' default policy.  A kernel of its own for each: a choice in the store loop costs scalar registers, up to 1.8 % of a short call.
+enum { STORE_TRACKED = -1, STORE_PAST, STORE_THROUGH, STORE_CACHED };
 struct GemmArgs {
     const int8_t* A;
     const int8_t* W;
@@ -45,7 +47,6 @@ struct GemmArgs {
     uint32_t magic;   // panel_magic(tiles_m, tiles_n), for tile_of_block
     int kslice;   // K of a split-K slice (a multiple of 128), 0 = no split
     int n_first;  // two-group kernel: the first column of these tiles
-    int policy;   // two-group kernel: how whole wave tiles are stored (store_policy)
 };
 
 template <int BM_, int BN_, int BK_, int WGM_, int WGN_, int OCC_>
@@ -199,7 +200,7 @@ struct EpiConst {
 // the columns 8*rb + 4*(lane / 32) + j.  16: v4i acc[2*TN][2*TM] of 16x16 tiles, a lane holds row lane % 16 and the
 // columns 4*(lane / 16) + j; the 32x32 block (in, im) is then the four tiles (2*in + rb, 2*im + hm).
 // EARLY: the constants are in `own` already; else they are loaded here.
-template <int TM, int TN, int OUT_DT, int EPI, int PW, bool UNTRACKED, int L, bool EARLY, class Acc>
+template <int TM, int TN, int OUT_DT, int EPI, int PW, int STORE, int L, bool EARLY, class Acc>
 __device__ __forceinline__ void epilogue_shuffle_with(const GemmArgs& p, Acc& acc, int mb, int nb, int lane, uint8_t* wl, uint8_t* wl2,
                                                       EpiConst<TM, TN, OUT_DT, EPI, L>& own) {
     // a piece is 32 rows x PW columns of the wave tile: PW*SZ bytes per LDS row, 32*PW*SZ bytes per wave
@@ -334,14 +335,15 @@ __device__ __forceinline__ void epilogue_shuffle_with(const GemmArgs& p, Acc& ac
     auto store_piece = [&](int im, int np, const uint4* v, const uint4* rv) {
         if (full) {
             const uint64_t piece = tile_base + (uint64_t)(im * 32) * row_bytes + (uint64_t)(np * PW * SZ);
-            const auto each = [&](auto store) {
 #pragma unroll
-                for (int t = 0; t < PASSES; ++t) store((const void*)(piece + (uint64_t)(t * RPI) * row_bytes), finish(np, v[t], rv[t]));
-            };
-            if (!UNTRACKED) each([&](const void* at, const uint4& x) { *reinterpret_cast<uint4*>((uint8_t*)at + lane_off) = x; });
-            else if (EPI != EPI_RESID && p.policy == STORE_THROUGH) each([&](const void* at, const uint4& x) { store16_through_at(at, lane_off, x); });
-            else if (EPI != EPI_RESID && p.policy == STORE_CACHED) each([&](const void* at, const uint4& x) { store16_cached_at(at, lane_off, x); });
-            else each([&](const void* at, const uint4& x) { store16_untracked_at(at, lane_off, x); });
+            for (int t = 0; t < PASSES; ++t) {
+                const uint64_t pass = piece + (uint64_t)(t * RPI) * row_bytes;
+                const uint4 o = finish(np, v[t], rv[t]);
+                if (STORE == STORE_TRACKED) *reinterpret_cast<uint4*>((uint8_t*)pass + lane_off) = o;
+                else if (STORE == STORE_THROUGH) store16_through_at((const void*)pass, lane_off, o);
+                else if (STORE == STORE_CACHED) store16_cached_at((const void*)pass, lane_off, o);
+                else store16_untracked_at((const void*)pass, lane_off, o);
+            }
             return;
         }
         int l = lane;
@@ -355,7 +357,7 @@ __device__ __forceinline__ void epilogue_shuffle_with(const GemmArgs& p, Acc& ac
             if (m >= p.M || ncol >= p.N) continue;
             uint8_t* out = base + t * step;
             const uint4 o = finish(np, v[t], rv[t]);
-            if (UNTRACKED) store16_untracked(out, o);
+            if (STORE != STORE_TRACKED) store16_untracked(out, o);
             else *reinterpret_cast<uint4*>(out) = o;
         }
     };
@@ -390,10 +392,10 @@ __device__ __forceinline__ void epilogue_shuffle_with(const GemmArgs& p, Acc& ac
     }
     asm volatile("" ::: "memory");
 }
-template <int TM, int TN, int OUT_DT, int EPI, int PW = TN * 32, bool UNTRACKED = false, int L = 32, class Acc>
+template <int TM, int TN, int OUT_DT, int EPI, int PW = TN * 32, int STORE = STORE_TRACKED, int L = 32, class Acc>
 __device__ __forceinline__ void epilogue_shuffle(const GemmArgs& p, Acc& acc, int mb, int nb, int lane, uint8_t* wl) {
     EpiConst<TM, TN, OUT_DT, EPI, L> own;
-    epilogue_shuffle_with<TM, TN, OUT_DT, EPI, PW, UNTRACKED, L, false>(p, acc, mb, nb, lane, wl, nullptr, own);
+    epilogue_shuffle_with<TM, TN, OUT_DT, EPI, PW, STORE, L, false>(p, acc, mb, nb, lane, wl, nullptr, own);
 }
 
 // Chooses the coalesced epilogue when row starts are 16-byte aligned.  Must be called by all waves of the workgroup:
@@ -708,7 +710,7 @@ __global__ void __launch_bounds__(512, 1) int8_gemm_fed_kernel(GemmArgs p) {
     constexpr int PW = C::piece_cols(SZ);
     wg_barrier();
     uint8_t* scratch = smem + wave * 16384;
-    epilogue_shuffle_with<C::TM, C::TN, OUT_DT, EPI, PW, true, 16, true>(p, acc, m0 + wm * 64, n0 + wn * C::TN * 32, hw_lane(), scratch, scratch + 8192, cst);
+    epilogue_shuffle_with<C::TM, C::TN, OUT_DT, EPI, PW, STORE_PAST, 16, true>(p, acc, m0 + wm * 64, n0 + wn * C::TN * 32, hw_lane(), scratch, scratch + 8192, cst);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -756,7 +758,7 @@ using PpM = PpCfg<96>;
 using PpS = PpCfg<64>;
 
 // The work of workgroup `bid` of `G` on problem p.
-template <class C, int OUT_DT, int EPI>
+template <class C, int OUT_DT, int EPI, int STORE>
 __device__ __forceinline__ void pp_gemm_tiles(const GemmArgs& p, uint8_t* smem, const int bid, const int G) {
     constexpr int BK = C::BK, TM = C::TM, TN = C::TN;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -914,7 +916,7 @@ __device__ __forceinline__ void pp_gemm_tiles(const GemmArgs& p, uint8_t* smem, 
         int m0, n0;
         tile_origin(ti, m0, n0);
         uint8_t* scratch = smem + (s_last % C::NSW) * C::W_STAGE + wave * 4096;
-        epilogue_shuffle<TM, TN, OUT_DT, EPI, PW, true, 16>(p, acc, m0 + grp * C::GM, n0 + wq * C::WTN, hw_lane(), scratch);
+        epilogue_shuffle<TM, TN, OUT_DT, EPI, PW, STORE, 16>(p, acc, m0 + grp * C::GM, n0 + wq * C::WTN, hw_lane(), scratch);
     };
 
     // Both groups run the same loop; group 1 is one phase behind (the barrier in front) and multiplies its last step of a
@@ -944,12 +946,12 @@ __device__ __forceinline__ void pp_gemm_tiles(const GemmArgs& p, uint8_t* smem, 
 // Workgroups 0 .. g_main-1 walk the tiles of `main`; the others walk the 128x256 tiles of `rest` (the rows or columns that
 // whole rounds of large tiles leave over, everything, or nothing).  One launch: the hardware starts a workgroup of the second kind
 // on each CU as its workgroup of the first kind retires, with no gap between two launches.
-template <class Main, int OUT_DT, int EPI>
+template <class Main, int OUT_DT, int EPI, int STORE>
 __global__ void __launch_bounds__(PpL::NT, 1) int8_gemm_pp_kernel(GemmArgs main, GemmArgs rest, int g_main) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int bid = (int)blockIdx.x;
-    if (bid < g_main) pp_gemm_tiles<Main, OUT_DT, EPI>(main, smem, bid, g_main);
-    else pp_gemm_tiles<PpS, OUT_DT, EPI>(rest, smem, bid - g_main, (int)gridDim.x - g_main);
+    if (bid < g_main) pp_gemm_tiles<Main, OUT_DT, EPI, STORE>(main, smem, bid, g_main);
+    else pp_gemm_tiles<PpS, OUT_DT, EPI, STORE>(rest, smem, bid - g_main, (int)gridDim.x - g_main);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1260,9 +1262,9 @@ int store_policy(int64_t M, int64_t row_bytes, uintptr_t D) {
     return (((uintptr_t)row_bytes | D) & 63) == 0 ? STORE_THROUGH : STORE_CACHED;
 }
 
-template <class Main, int OUT_DT, int EPI>
+template <class Main, int OUT_DT, int EPI, int STORE>
 int launch_pp_as(const GemmArgs& main, const GemmArgs& rest, int g_main, int g_rest, hipStream_t st) {
-    auto kern = int8_gemm_pp_kernel<Main, OUT_DT, EPI>;
+    auto kern = int8_gemm_pp_kernel<Main, OUT_DT, EPI, STORE>;
     static PerDeviceOnce once;
     if (const int e = allow_dynamic_lds((const void*)kern, PpL::SMEM, once)) return e;
     hipLaunchKernelGGL(kern, dim3((unsigned)(g_main + g_rest)), dim3(PpL::NT), PpL::SMEM, st, main, rest, g_main);
@@ -1277,7 +1279,7 @@ int launch_pp(GemmArgs a, hipStream_t st) {
     const int64_t G = device_cu_count();
     const PpSplit sp = pp_split(a.M, a.N, G);
     constexpr int SZ = EPI == EPI_ACC || OUT_DT == DT_F32 ? 4 : 2;
-    a.policy = store_policy(a.M, (int64_t)a.N * SZ, (uintptr_t)a.D);
+    const int policy = EPI == EPI_RESID ? (int)STORE_PAST : store_policy(a.M, (int64_t)a.N * SZ, (uintptr_t)a.D);
     GemmArgs main = a, rest = a;
     const int64_t n_main = sp.main_tm * sp.main_tn, n_rest = sp.small, tn = (a.N + 255) / 256;
     if (n_main > 0x7fffffff || n_rest > 0x7fffffff) return -1;
@@ -1296,8 +1298,16 @@ int launch_pp(GemmArgs a, hipStream_t st) {
     main.magic = n_main ? panel_magic(main.tiles_m, main.tiles_n) : 0;
     rest.magic = panel_magic(rest.tiles_m, rest.tiles_n);
     const int g_main = (int)(n_main < G ? n_main : G), g_rest = (int)(n_rest < G ? n_rest : G);
-    return sp.rows == PpM::BM ? launch_pp_as<PpM, OUT_DT, EPI>(main, rest, g_main, g_rest, st)
-                              : launch_pp_as<PpL, OUT_DT, EPI>(main, rest, g_main, g_rest, st);
+    const auto as = [&](auto store) {
+        constexpr int S = decltype(store)::value;
+        return sp.rows == PpM::BM ? launch_pp_as<PpM, OUT_DT, EPI, S>(main, rest, g_main, g_rest, st)
+                                  : launch_pp_as<PpL, OUT_DT, EPI, S>(main, rest, g_main, g_rest, st);
+    };
+    if constexpr (EPI != EPI_RESID) {
+        if (policy == STORE_THROUGH) return as(ic<STORE_THROUGH>{});
+        if (policy == STORE_CACHED) return as(ic<STORE_CACHED>{});
+    }
+    return as(ic<STORE_PAST>{});
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1809,7 +1819,7 @@ GPU_API int gpu_int8_gemm(const int8_t* A, const int8_t* W, const float* xs, con
     if (out_dt < DT_F32 || out_dt > DT_BF16 || M < 0 || N < 0 || K < 0 || !shape_ok(M, N, K)) return -200;
     PaddedK pad(A, W, M, N, K, (hipStream_t)stream);
     if (pad.rc != 0) return pad.rc < 0 ? -200 : pad.rc;
-    GemmArgs a{A, W, xs, ws, bias, nullptr, nullptr, D, (int)M, (int)N, (int)K, 0, 0, 0, 0, 0};
+    GemmArgs a{A, W, xs, ws, bias, nullptr, nullptr, D, (int)M, (int)N, (int)K, 0, 0, 0, 0};
     const int rc = dispatch_dt<EPI_PLAIN>(a, out_dt, (hipStream_t)stream);
     return rc < 0 ? -200 : rc;
 }
@@ -1822,7 +1832,7 @@ GPU_API int gpu_int8_gemm_residual(const int8_t* A, const int8_t* W, const float
     if (out_dt < DT_F32 || out_dt > DT_BF16 || M < 0 || N < 0 || K < 0 || !shape_ok(M, N, K)) return -201;
     PaddedK pad(A, W, M, N, K, (hipStream_t)stream);
     if (pad.rc != 0) return pad.rc < 0 ? -201 : pad.rc;
-    GemmArgs a{A, W, xs, ws, bias, rscale, resid, D, (int)M, (int)N, (int)K, 0, 0, 0, 0, 0};
+    GemmArgs a{A, W, xs, ws, bias, rscale, resid, D, (int)M, (int)N, (int)K, 0, 0, 0, 0};
     const int rc = dispatch_dt<EPI_RESID>(a, out_dt, (hipStream_t)stream);
     return rc < 0 ? -201 : rc;
 }
@@ -1835,7 +1845,7 @@ GPU_API int gpu_int8_gemm_static(const int8_t* A, const int8_t* W, const float* 
     int rc = 0;
     void* ptr = static_scratch(&rc);
     if (!ptr) return rc;
-    GemmArgs a{A, W, xs, ws, bias, nullptr, nullptr, D, (int)M, (int)N, (int)K, 0, 0, 0, 0, 0};
+    GemmArgs a{A, W, xs, ws, bias, nullptr, nullptr, D, (int)M, (int)N, (int)K, 0, 0, 0, 0};
     tl_scratch = ptr;
     tl_scratch_bytes = kStaticScratchBytes;
     rc = dispatch_dt<EPI_PLAIN>(a, out_dt, (hipStream_t)stream);
@@ -1851,7 +1861,7 @@ GPU_API int gpu_int8_gemm_acc(const int8_t* A, const int8_t* W, int32_t* acc, in
     if (M < 0 || N < 0 || K < 0 || !shape_ok(M, N, K)) return -200;
     PaddedK pad(A, W, M, N, K, (hipStream_t)stream);
     if (pad.rc != 0) return pad.rc < 0 ? -200 : pad.rc;
-    GemmArgs a{A, W, nullptr, nullptr, nullptr, nullptr, nullptr, acc, (int)M, (int)N, (int)K, 0, 0, 0, 0, 0};
+    GemmArgs a{A, W, nullptr, nullptr, nullptr, nullptr, nullptr, acc, (int)M, (int)N, (int)K, 0, 0, 0, 0};
     const int rc = dispatch_cfg<DT_F32, EPI_ACC>(a, (hipStream_t)stream);
     return rc < 0 ? -200 : rc;
 }
