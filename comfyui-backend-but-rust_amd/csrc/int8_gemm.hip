@@ -722,14 +722,14 @@ __global__ void __launch_bounds__(512, 1) int8_gemm_fed_kernel(GemmArgs p) {
 // workgroup barrier between phases:
 //   compute: the 64 MFMAs (16x16x64, 16 cycles each) of one 128-deep K step, on fragments already in registers, and
 //            nothing else;
-//   memory:  the 24 fragment reads of the group's next K step and 8 DMA instructions per wave.
+//   memory:  the 24 fragment reads of the group's next K step and NLA + NLW = 8 DMA instructions per wave.
 // While one wave of a SIMD is in its memory phase the other is in its compute phase, so the matrix pipe always has an
 // MFMA to run and no MFMA waits behind a DMA.
 //
 // LDS (160 KB): three 32 KB stages of W (both groups read them) and two 16 KB stages of A for each group.  With global
 // step s = tile * nk + k tile, group 0 computes step s in phase 2s and group 1 in phase 2s + 1.  Group 0's memory phase
 // before step s fetches A of group 1 for step s + 1 and rows 0..127 of W for step s + 2; group 1's fetches A of group 0
-// and rows 128..255 of W, both for step s + 2.  Every memory phase ends with a wait that leaves only its own 8 DMA
+// and rows 128..255 of W, both for step s + 2.  Every memory phase ends with a wait that leaves only its own NLA + NLW DMA
 // instructions in flight, so what a phase fetches is visible to everybody two phases later, and each stage is refilled
 // only after the barrier that follows its last reader.  Steps run straight through tile boundaries.
 //
@@ -740,8 +740,8 @@ __global__ void __launch_bounds__(512, 1) int8_gemm_fed_kernel(GemmArgs p) {
 // Requires K % 128 == 0, M*K and N*K < 2^32, and the coalesced epilogue's alignment.
 // ---------------------------------------------------------------------------------------------------------------
 // GM: rows of a group.  128 gives the 256x256 tile (wave tiles 128x64), 96 a 192x256 tile, 64 a 128x256 tile (wave tiles 64x64):
-// half the work per tile, at a step that is bound by its 6 DMA instructions per wave rather than by its 32 MFMAs.  pp_split
-// says which run.
+// half the work per tile, at a step that is bound by its 6 DMA instructions per wave (7 with 96 rows) rather than by its 32 MFMAs.
+// pp_split says which run.
 template <int GM_>
 struct PpCfg {
     static constexpr int GM = GM_, BM = 2 * GM, BN = 256, BK = 128, NT = 512;
@@ -1205,10 +1205,11 @@ GemmArgs row_band(const GemmArgs& a, int64_t row0, int64_t rows) {
 // round is idle: tiles of 256, 192 or 128 rows by 256 columns, and where the tiles of 256 or 192 rows fill whole rounds and some
 // more, the tile rows or tile columns that fill the whole ones, with the rest as 128 x 256 tiles by further workgroups of the same
 // launch.  The smallest sum of rounds runs, a round of the smaller tiles counted as 0.78 and 0.67 of one of 256 rows: three
-// quarters and half of the work, but a step of theirs is bound by its DMA instructions.  (kCost is what chose best over 260 shapes of 512 to
-// 8192 rows timed in all seven forms, 0.8 % slower than the best of them; 256-row tiles with rows left over alone 7.1 %.)  us, those and
-// the present choice: 2048 x 14336 -> 5376 145 and 125 (192 rows: 231 tiles instead of 168), 3000 x 2048 -> 7168 46 and 42,
-// 6000 x 1024 -> 3072 29 and 25, 8192 x 640 -> 5120 38.7 and 38.1 (columns left over; bound by the chip's writes beside the MFMAs).
+// quarters and half of the work, but a step of theirs is bound by its DMA instructions.  kCost is what chose best over 260 shapes of 512 to
+// 8192 rows timed in all seven forms; over 720 others, weights from HBM and outputs in turn, it is 0.8 % slower than the best of them, 256-row
+// tiles with rows left over alone 10 %.  us, those and the present choice, weights from HBM (from the last-level cache): 2048 x 14336 -> 5376
+// 134.4 and 123.8 (125.2 and 122.2; 192 rows: 231 tiles instead of 168), 3000 x 2048 -> 7168 46.7 and 43.7 (45.2 and 42.3), 6000 x 1024 -> 3072
+// 28.6 and 26.3 (28.4 and 26.0), 8192 x 640 -> 5120 39.2 and 39.5 (35.3 and 35.1; columns left over; bound by the chip's writes beside the MFMAs).
 struct PpSplit {
     int rows;                          // of a tile of the first kind: 256 or 192; 128: there are only tiles of the second
     int64_t main_tm, main_tn, small;   // the grid of those tiles, and how many of the second kind

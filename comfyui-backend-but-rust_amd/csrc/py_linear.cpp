@@ -1,6 +1,7 @@
 // qlinear.linear_w8a8's call as native code: the checks, the output's allocation and the launch of gpu_linear_w8a8 behind one call from
-// Python.  A few rows take 5 us on the GPU; checked, allocated and called from Python they took 8.1 us of host time (a tensor
-// 1.5, the call through ctypes with its 13 arguments about 2, attribute reads and checks the rest), this way 4.1 (3 x 256 -> 18432 8.1 -> 4.6 us a call in a row of them).
+// Python.  3 x 256 -> 18432 takes 4.1 us on the GPU with weights that it has just read and 4.7 with 20 of them in turn (replayed from a
+// graph); checked, allocated and called from Python it took 8.7 us of host time (a tensor 1.5, the call through ctypes with its 13 arguments
+// about 2, attribute reads and checks the rest), this way 4.7.  A call in a row of them 8.1 and 4.9 us, bound by both sides alike.
 //
 // It answers None for whatever it does not take (a check that fails, tensor subclasses, modes and transforms that want to see the
 // calls, return codes other than 0), and the caller then does the whole call in Python, which raises what there is to raise.

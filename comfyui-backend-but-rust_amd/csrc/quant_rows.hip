@@ -779,7 +779,7 @@ bool known_prologue(int p) { return p >= PRO_PLAIN && p <= PRO_SITU_FAST && p !=
 // quantizer above, so the codes are its codes) while its weights are on their way from HBM straight into the registers
 // that the matrix instruction reads, then multiplies them with 64 columns, 16 per wave.  Bound by latency: one trip to memory beside
 // the quantizer's chain of LDS round trips.  M=3, K=256 -> N=18432, us per linear replayed from a graph: 4.5, as a quantizer and
-// a GEMM 7.0; called from Python 12.4 and 20.5, host work.
+// a GEMM 7.0; a call from Python 4.9 where it is native code, 8.1 without, host work.
 constexpr int kLinRows = 8, kLinK = 1024, kLinCols = 64;
 struct LinArgs {
     const int8_t* W;

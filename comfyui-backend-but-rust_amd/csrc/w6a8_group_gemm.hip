@@ -422,17 +422,18 @@ __global__ void __launch_bounds__(NT, 1) w6a8_group_gemm_kernel(W6Args p) {
 // The W8 form on 256 x 256 tiles: eight waves of 128 x 64, so that a group costs a wave 24 fragment reads for 64 MFMAs where the
 // 256 x 128 tile costs it 20 for 32, and a CU 64 KB of DMA where two of the smaller tiles cost 96.  256 registers hold that because a
 // lane's int32 partials live only from one row tile to the next: behind the eight MFMAs of a row tile comes the fold of the one before,
-// 32 additions (sum_value) and 32 fma in a row.  A vector instruction behind every MFMA does not overlap with the other wave's: a probe of
-// this mix, four to an MFMA and two waves, takes 25.0 cycles per MFMA and SIMD with any kind of vector instruction; in runs of 8 and
-// 32 23.3 with conversions, 23.2 with additions (of 64 and 256 21.9 and 20.6, for which there are no registers).  In the kernel 614 us one by one with
-// conversions, 610 with additions, 605 in runs with conversions, 597 in runs with additions; runs of 4 and 16 603.
+// 16 additions (sum_value) and 16 fma in a row.  A vector instruction behind every MFMA does not overlap with the other wave's: a probe of
+// this mix, four to an MFMA and two waves, takes 25.0 cycles per MFMA and SIMD with any kind of vector instruction; eight MFMAs and then 32 of
+// them 23.3 with conversions, 23.2 with additions (64 and then 256 21.9 and 20.6, for which there are no registers).  In the kernel 614 us one by
+// one with conversions, 610 with additions, 605 in such runs with conversions, 597 with additions; four MFMAs and then 16 603.
 // Two LDS stages of A, W and scales: group g+1 travels during group g, one barrier per group.  The four lower waves issue all DMA, one
 // instruction after every eight of the fold: every wave fetching its own share has both waves of a SIMD held by a DMA instruction at the
 // same time (608); between the MFMAs 598, twice as dense 600, spread over all of the group 630 (they land too late).
 // The same tile with v_mfma_i32_32x32x32_i8, which leaves more issue slots to the fold, takes 677 us: the chip is at its power limit.
 // A persistent form with the next tile's first group under the epilogue: no change.
-// M=8192, K=5120 -> N=13824, expansion included: 256 x 128 tiles 756 us, these 597.  What is left is the fold next to the MFMAs
-// (64 MFMAs and 256 vector instructions per wave and group), near the power limit.
+// M=8192, K=5120 -> N=13824, expansion (23 us) included: 256 x 128 tiles 756 us, these 597.  Beside the fold next to the MFMAs (64 MFMAs and 256
+// vector instructions per wave and group) the issue of DMA and of fragment reads counts: with the DMA of the first two groups only 556 us,
+// with the first group's fragments kept 561, with neither 515; K=13824 -> N=5120 602, 547, 563 and 500.
 constexpr int BIG_BN = 256, BIG_U = BIG_BN * BK, BIG_U_BASE = 2 * A_STAGE, BIG_S_BASE = BIG_U_BASE + 2 * BIG_U, BIG_S = BIG_BN * 4;
 constexpr int BIG_SMEM = BIG_S_BASE + 2 * BIG_S;
 

@@ -33,7 +33,7 @@ _DT_TORCH = {v: k for k, v in _TORCH_DT.items()}
 
 def _stream():
     """Handle of the current stream of the current device: torch.cuda.current_stream().cuda_stream without the Stream object made
-    for it (2.8 us of a 12.3 us call; this way 0.2, and the call 8.1 with no scratch for few rows)."""
+    for it, which took 2.8 us of a call's host time; this way 0.2."""
     return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
